@@ -131,6 +131,13 @@ __device__ __forceinline__ uint64_t philox_bounded(PhiloxKey key, uint64_t pos,
   return __umul64hi(r, n);
 }
 
+// A value stored where the host looks for it (pinned host memory, polled while
+// the kernel may still be running): written through to the system at once, not
+// when the kernel ends.  Also right for device memory.
+__device__ __forceinline__ void store_for_host(int64_t* p, int64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------------- wave helpers
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
@@ -323,7 +330,8 @@ struct SliceView {
       const int64_t c = r.span.lo + (lane_id() < r.count ? lane_id() : r.count - 1);
       const int64_t start = sub_indptr[c];
       r.lane_start = start > first_u ? (int32_t)(start - first_u) : 0;
-      r.lane_shift = indptr[cols[c]] - start;
+      // (an id outside the matrix is an empty column: its pointer is not read)
+      r.lane_shift = sub_indptr[c + 1] > start ? indptr[cols[c]] - start : 0;
       if (key_offset) r.lane_offset = key_offset[c];
     }
     return r;

@@ -193,8 +193,8 @@ __global__ __launch_bounds__(kBlock) void scan_down_kernel(
     else if (i < n)
       out[i] = result.v[0];
     if (last_mirror) {
-      if (i == n - 1) *last_mirror = result.v[0];
-      if (i + 1 == n - 1) *last_mirror = result.v[1];
+      if (i == n - 1) store_for_host(last_mirror, result.v[0]);
+      if (i + 1 == n - 1) store_for_host(last_mirror, result.v[1]);
     }
   }
 }
@@ -259,7 +259,7 @@ int exclusive_scan_i64(const int64_t* in, int64_t* out, int64_t n, void* ws,
 __global__ __launch_bounds__(kBlock) void copy_i64_kernel(const int64_t* __restrict__ src,
                                                           int64_t n, int64_t* __restrict__ dst) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) dst[i] = src[i];
+  if (i < n) store_for_host(dst + i, src[i]);
 }
 
 }  // namespace gs

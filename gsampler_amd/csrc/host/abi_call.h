@@ -8,6 +8,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <atomic>
+#include <limits>
 #include <torch/torch.h>
 
 #include <vector>
@@ -97,28 +98,47 @@ inline torch::Tensor new_workspace(size_t bytes, const torch::Tensor& like) {
                       device_options(like).dtype(torch::kUInt8));
 }
 
-// Last element of a device prefix array (one blocking 8-byte copy).
-inline int64_t read_last(const torch::Tensor& prefix) {
-  return prefix[prefix.numel() - 1].item<int64_t>();
+// ---------------------------------------------------- values for the host
+// A word of pinned host memory that a kernel on its way will store to.  The host
+// marks it, hands its address to the kernel and, when it needs the value, looks
+// at the word itself until the value is there: it arrives while the kernel is
+// still running, about a microsecond after the store.  (An event behind the
+// kernel costs the device a gap of 5-8 us in front of whatever comes next, and
+// the host another 10 us to be woken.)
+constexpr int64_t kNotYet = std::numeric_limits<int64_t>::min();
+
+// Waits until words[0 .. n) have all been stored to by work queued on `stream`.
+// Every now and then the stream itself is asked, so that a failed kernel ends
+// the wait; once the stream is idle the words hold whatever they will hold.
+inline void await_words(const int64_t* words, size_t n, hipStream_t stream) {
+  constexpr int kPollsPerQuery = 1 << 13;
+  for (size_t i = 0; i < n; ++i) {
+    int polls = 0;
+    while (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) == kNotYet) {
+      if (++polls < kPollsPerQuery) {
+        __builtin_ia32_pause();
+        continue;
+      }
+      polls = 0;
+      const hipError_t e = hipStreamQuery(stream);
+      if (e == hipErrorNotReady) continue;
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+      TORCH_CHECK(hipDeviceSynchronize() == hipSuccess && __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != kNotYet,
+                  "the kernel that was to report a count never did");
+    }
+  }
 }
 
-// The same value without stalling the GPU: the copy into pinned host memory is
-// queued on the current stream at once, get() waits for it.  Work launched in
-// between (into buffers sized by an upper bound) keeps the GPU busy while the
-// value travels.  Slots come from a small per-thread ring of pinned words that
-// lives until the process ends; a slot is reused after kSlots later reads.
+// One such word.  Slots come from a small per-thread ring that lives until the
+// process ends; a slot is reused after kSlots later requests.
 class AsyncCount {
  public:
   AsyncCount() = default;
   explicit AsyncCount(const torch::Tensor& prefix) {
-    Ring& r = ring();
-    ticket_ = r.next++;
-    slot_ = (int)(ticket_ % kSlots);
-    hipStream_t s = (hipStream_t)cur_stream();
+    *this = mirrored();
     const int64_t* src = prefix.data_ptr<int64_t>() + prefix.numel() - 1;
-    GS_CALL(gs_copy_i64(src, 1, r.words + slot_, (gs_stream_t)s));
-    check(hipEventRecord(r.events[slot_], s));
-    pending_ = true;
+    GS_CALL(gs_copy_i64(src, 1, mirror(), cur_stream()));
+    arm();
   }
   // For a kernel that stores the value to the host itself: hand it mirror(),
   // then arm() once it is queued.
@@ -127,22 +147,28 @@ class AsyncCount {
     Ring& r = ring();
     c.ticket_ = r.next++;
     c.slot_ = (int)(c.ticket_ % kSlots);
+    // a request that nobody asked for: its kernel must not store later
+    if (r.armed[c.slot_]) await_words(r.words + c.slot_, 1, r.stream[c.slot_]);
+    r.armed[c.slot_] = false;
+    r.words[c.slot_] = kNotYet;
     return c;
   }
   bool requested() const { return slot_ >= 0; }
   int64_t* mirror() const { return ring().words + slot_; }
   void arm() {
-    check(hipEventRecord(ring().events[slot_], (hipStream_t)cur_stream()));
+    Ring& r = ring();
+    r.stream[slot_] = (hipStream_t)cur_stream();
+    r.armed[slot_] = true;
     pending_ = true;
   }
   int64_t get() {
     TORCH_CHECK(slot_ >= 0, "AsyncCount: nothing was requested");
-    Ring& r = ring();
     if (pending_) {
+      Ring& r = ring();
       // every operator reads its counts before it returns; one left waiting
       // while kSlots later requests went by would read another request's word
       TORCH_CHECK(r.next - ticket_ <= (unsigned)kSlots, "AsyncCount: the slot was reused");
-      check(hipEventSynchronize(r.events[slot_]));
+      await_words(r.words + slot_, 1, r.stream[slot_]);
       value_ = r.words[slot_];
       pending_ = false;
     }
@@ -153,18 +179,16 @@ class AsyncCount {
   static constexpr int kSlots = 64;
   struct Ring {
     int64_t* words = nullptr;
-    hipEvent_t events[kSlots];
+    hipStream_t stream[kSlots] = {};
+    bool armed[kSlots] = {};
     unsigned next = 0;
   };
-  static void check(hipError_t e) {
-    TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
-  }
   static Ring& ring() {
     static thread_local Ring* r = [] {
       Ring* x = new Ring();
-      check(hipHostMalloc((void**)&x->words, kSlots * sizeof(int64_t), hipHostMallocDefault));
-      for (int i = 0; i < kSlots; ++i)
-        check(hipEventCreateWithFlags(&x->events[i], hipEventDisableTiming));
+      const hipError_t e =
+          hipHostMalloc((void**)&x->words, kSlots * sizeof(int64_t), hipHostMallocDefault);
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
       return x;
     }();
     return *r;
@@ -174,6 +198,12 @@ class AsyncCount {
   bool pending_ = false;
   int64_t value_ = 0;
 };
+
+// Last element of a device prefix array.
+inline int64_t read_last(const torch::Tensor& prefix) {
+  if (!prefix.is_cuda()) return prefix[prefix.numel() - 1].item<int64_t>();
+  return AsyncCount(prefix).get();
+}
 
 // Host copies of small offset arrays (batch pointers).  Splitting results per
 // batch needs them on the host; a blocking copy at that point waits for
@@ -194,13 +224,13 @@ class OffsetMirror {
   }
   static void arm(const torch::Tensor& offsets) {
     Entry& e = entry_for(offsets, false);
-    check(hipEventRecord(e.event, (hipStream_t)cur_stream()));
+    e.stream = (hipStream_t)cur_stream();
     e.pending = true;
   }
   static const std::vector<int64_t>& values(const torch::Tensor& offsets) {
     Entry& e = entry_for(offsets);
     if (e.pending) {
-      check(hipEventSynchronize(e.event));
+      await_words(e.pinned, e.count, e.stream);
       e.host.assign(e.pinned, e.pinned + e.count);
       e.pending = false;
     }
@@ -213,7 +243,7 @@ class OffsetMirror {
     int64_t version = -1, epoch = -1;
     int64_t* pinned = nullptr;
     size_t capacity = 0, count = 0;
-    hipEvent_t event = nullptr;
+    hipStream_t stream = nullptr;
     bool pending = false;
     std::vector<int64_t> host;
   };
@@ -234,7 +264,7 @@ class OffsetMirror {
           e.version == (int64_t)offsets._version() && e.epoch == cache_epoch())
         return e;
     Entry& e = ring[next++ % kEntries];
-    if (e.pending) check(hipEventSynchronize(e.event));  // its copy must not land later
+    if (e.pending) await_words(e.pinned, e.count, e.stream);  // its copy must not land later
     e.tensor = offsets;
     e.version = offsets._version();
     e.epoch = cache_epoch();
@@ -250,13 +280,13 @@ class OffsetMirror {
       e.capacity = e.count < 1024 ? 1024 : e.count;
       check(hipHostMalloc((void**)&e.pinned, e.capacity * sizeof(int64_t), hipHostMallocDefault));
     }
-    if (!e.event) check(hipEventCreateWithFlags(&e.event, hipEventDisableTiming));
+    for (size_t i = 0; i < e.count; ++i) e.pinned[i] = kNotYet;
     if (!copy) return e;
     torch::Tensor c = offsets.contiguous();
     hipStream_t s = (hipStream_t)cur_stream();
     if (e.count > 0)
       GS_CALL(gs_copy_i64(c.data_ptr<int64_t>(), (int64_t)e.count, e.pinned, (gs_stream_t)s));
-    check(hipEventRecord(e.event, s));
+    e.stream = s;
     e.pending = true;
     return e;
   }

@@ -36,10 +36,12 @@ GraphAndIndex Graph::SamplingProbs(int64_t axis, torch::Tensor edge_probs,
   MajorResult r;
   r.indptr = new_ids(n + 1, m.indptr);
   torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
+  AsyncCount count = AsyncCount::mirrored();
   GS_CALL(gs_csc_col_count(cptr(m.indptr), n, nullptr, n, fanout, replace ? 1 : 0,
-                           mptr(r.indptr), nullptr, nullptr, ws.data_ptr(), ws.numel(),
+                           mptr(r.indptr), count.mirror(), nullptr, ws.data_ptr(), ws.numel(),
                            cur_stream()));
-  const int64_t nnz = read_last(r.indptr);
+  count.arm();
+  const int64_t nnz = count.get();
   r.minor_ids = new_ids(nnz, m.indptr);
   r.select = new_ids(nnz, m.indptr);
   if (with_coo) r.major_ids = new_ids(nnz, m.indptr);

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kLabelThreads) void list_labels_kernel(
   }
   if (t == 0) {
     if (out_count) *out_count = total;
-    if (out_count_mirror) *out_count_mirror = total;
+    if (out_count_mirror) store_for_host(out_count_mirror, total);
   }
   __syncthreads();
 

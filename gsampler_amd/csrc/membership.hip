@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
     int64_t nnz, int64_t* __restrict__ out_indptr, int64_t* __restrict__ out_total) {
   const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
-  if (c == 0 && out_total) *out_total = nnz > 0 ? chunk_off[num_chunks] : 0;
+  if (c == 0 && out_total) store_for_host(out_total, nnz > 0 ? chunk_off[num_chunks] : 0);
   if (indptr == nullptr || c > num_major) return;
   const int64_t e = indptr[c];
   out_indptr[c] = nnz == 0 ? 0

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kCountThreads) void col_count_small_kernel(
     if (i <= num_items) sub_indptr[i] = run;
     run += cnt[k];
   }
-  if (threadIdx.x == 0 && total_mirror) *total_mirror = total;
+  if (threadIdx.x == 0 && total_mirror) store_for_host(total_mirror, total);
 }
 
 // Edge-parallel slice: thread e owns output edge e, finds its column by binary

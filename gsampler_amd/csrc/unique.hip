@@ -1047,7 +1047,7 @@ __global__ __launch_bounds__(kOffsetsThreads) void unique_offsets_kernel(
     }
     unique_ptr[b] = r;
     unique_ptr_ws[b] = r;
-    if (unique_ptr_mirror) unique_ptr_mirror[b] = r;
+    if (unique_ptr_mirror) store_for_host(unique_ptr_mirror + b, r);
   }
 }
 
@@ -1332,7 +1332,7 @@ __global__ __launch_bounds__(kBlock) void unique_empty_kernel(
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   unique_ptr[i] = 0;
-  if (unique_ptr_mirror) unique_ptr_mirror[i] = 0;
+  if (unique_ptr_mirror) store_for_host(unique_ptr_mirror + i, 0);
 }
 
 static int check_unique_args(const int64_t* seeds, const int64_t* seeds_ptr,
