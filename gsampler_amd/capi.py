@@ -66,6 +66,11 @@ SIGNATURES = {
     "gs_decode_batch_ids": (_int, [_p, _i64, _i64, _p, _p, _p]),
     "gs_split_indptr": (_int, [_p, _p, _i64, _i64, _p, _p]),
     "gs_batch_seeds_distinct": (_int, [_p, _p, _p, _p, _i64, _p, _p]),
+    "gs_slice_compact_workspace_bytes": (_sz, [_i64, _i64]),
+    "gs_slice_compact_count": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p,
+                                      _p, _sz, _p]),
+    "gs_slice_compact_fill": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p,
+                                     _p, _p, _sz, _p]),
     "gs_first_position": (_int, [_p, _i64, _i64, _p, _p]),
     "gs_csc_col_slice_values": (_int, [_p, _p, _i64, _p, _i64, _p, _i64, _p, _p]),
     "gs_list_labels": (_int, [_p, _i64, _p, _p, _i64, _p, _p, _p, _p, _p, _p]),

@@ -78,6 +78,51 @@ static std::tuple<torch::Tensor, torch::Tensor> batch_offsets(
   return {ptr, orig};
 }
 
+// The rows of an encoded slice are numbered through one flag byte per
+// (batch, row) while those bytes are cheap next to the edges: clearing and
+// reading them back streams at several TB/s, a sort of the edges' keys costs
+// about 50 ps per key and pass, ten passes, and a dozen launches.
+static bool compact_by_flags(int64_t num_batches, int64_t stride, int64_t nnz) {
+  constexpr int64_t kAlways = int64_t(1) << 24, kNever = int64_t(1) << 30;
+  if (stride == 0 || num_batches > kNever / stride) return false;
+  const int64_t keys = num_batches * stride;
+  return keys <= kAlways || keys / 256 <= nnz;
+}
+
+// The encoded slice with its rows numbered anew, and those rows: which ids, and
+// where every batch's begin (compact.hip).
+static MajorResult compact_slice(const Compressed& m, const torch::Tensor& cols,
+                                 const torch::Tensor& offsets, int64_t nnz,
+                                 const torch::Tensor& col_bptr, int64_t stride,
+                                 torch::Tensor* row_bptr, torch::Tensor* rows) {
+  const int64_t B = col_bptr.numel() - 1, n = cols.numel();
+  MajorResult r;
+  r.indptr = offsets;
+  torch::Tensor key_offset = new_ids(n, m.indptr);
+  *row_bptr = new_ids(B + 1, m.indptr);
+  torch::Tensor ws = new_workspace(gs_slice_compact_workspace_bytes(B, stride), m.indptr);
+  const torch::Tensor& narrow = m.narrow_indices();
+  const int32_t* ids32 = narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr;
+  int64_t* mirror = OffsetMirror::reserve(*row_bptr);
+  GS_CALL(gs_slice_compact_count(cptr(m.indptr), cptr(m.indices), ids32, cptr(cols), n,
+                                 cptr(offsets), nnz, cptr(col_bptr), B, stride, mptr(key_offset),
+                                 mptr(*row_bptr), mirror, ws.data_ptr(), ws.numel(),
+                                 cur_stream()));
+  OffsetMirror::arm(*row_bptr);
+  torch::Tensor bound = new_ids(std::min(nnz, B * stride), m.indptr);
+  r.minor_ids = new_ids(nnz, m.indptr);
+  r.select = new_ids(nnz, m.indptr);
+  r.major_ids = new_ids(nnz, m.indptr);
+  GS_CALL(gs_slice_compact_fill(cptr(m.indptr), cptr(m.indices), ids32, cptr(cols), n,
+                                cptr(offsets), nnz, cptr(key_offset), B, stride, mptr(bound),
+                                mptr(r.major_ids), mptr(r.minor_ids), mptr(r.select),
+                                ws.data_ptr(), ws.numel(), cur_stream()));
+  const int64_t total = OffsetMirror::values(*row_bptr).back();
+  BatchOffsets::trust(*row_bptr, total);
+  *rows = trim_to(bound, total);
+  return r;
+}
+
 GraphAndIndex Graph::BatchColSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
                                      bool encoding) {
   seeds = ids(seeds, "seeds");
@@ -87,15 +132,24 @@ GraphAndIndex Graph::BatchColSlicing(torch::Tensor seeds, torch::Tensor col_bptr
   BatchOffsets::check(col_bptr, seeds.numel(), "BatchColSlicing");
   const Compressed& m = compressed(kCSC);
   const int64_t stride = num_rows_;
-  MajorResult r = major_slice(m, seeds, true, col_bptr, encoding ? stride : 0);
+  MajorResult r;
   torch::Tensor row_bptr, orig_rows;
-  if (encoding) {
-    // compact the encoded row ids: sorted unique + rank of every edge's row
-    auto uniq = torch::_unique2(r.minor_ids, /*sorted=*/true,
-                                /*return_inverse=*/true, /*return_counts=*/false);
-    r.minor_ids = std::get<1>(uniq);
-    std::tie(row_bptr, orig_rows) = batch_offsets(std::get<0>(uniq), B, stride);
-    BatchOffsets::trust(row_bptr);
+  if (!encoding) {
+    r = major_slice(m, seeds, true, col_bptr, 0);
+  } else {
+    int64_t nnz = 0;
+    torch::Tensor offsets = slice_offsets(m, seeds, &nnz);
+    if (compact_by_flags(B, stride, nnz)) {
+      r = compact_slice(m, seeds, offsets, nnz, col_bptr, stride, &row_bptr, &orig_rows);
+    } else {
+      // few edges of a huge range of keys: sorted unique + rank of every edge's row
+      r = major_slice(m, seeds, true, col_bptr, stride);
+      auto uniq = torch::_unique2(r.minor_ids, /*sorted=*/true,
+                                  /*return_inverse=*/true, /*return_counts=*/false);
+      r.minor_ids = std::get<1>(uniq);
+      std::tie(row_bptr, orig_rows) = batch_offsets(std::get<0>(uniq), B, stride);
+      BatchOffsets::trust(row_bptr);
+    }
   }
   const int64_t new_rows = encoding ? orig_rows.numel() : num_rows_ * B;
   GraphPtr g = derive(kCSC, kCSC | kCOO, r, new_rows, seeds.numel());

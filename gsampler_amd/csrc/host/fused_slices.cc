@@ -21,19 +21,11 @@ const Graph::SliceOffsets& Graph::slice_offsets_for(const torch::Tensor& cols) {
       slice_offsets_->epoch == cache_epoch())
     return *slice_offsets_;
   auto so = std::make_unique<SliceOffsets>();
-  const int64_t num_major = m.indptr.numel() - 1, n = cols.numel();
   so->cols = cols;
   so->version = cols._version();
   so->indptr_version = m.indptr._version();
   so->epoch = cache_epoch();
-  so->sub_indptr = new_ids(n + 1, m.indptr);
-  torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
-  AsyncCount count = AsyncCount::mirrored();
-  GS_CALL(gs_csc_col_count(cptr(m.indptr), num_major, cptr(cols), n, -1, 0,
-                           mptr(so->sub_indptr), count.mirror(), nullptr, ws.data_ptr(), ws.numel(),
-                           cur_stream()));
-  count.arm();
-  so->nnz = count.get();
+  so->sub_indptr = slice_offsets(m, cols, &so->nnz);
   slice_offsets_ = std::move(so);
   return *slice_offsets_;
 }

@@ -189,18 +189,27 @@ const Compressed& Graph::compressed(int64_t format) {
 }
 
 // ---------------------------------------------------- operators, major axis
+torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, int64_t* nnz) {
+  const int64_t n = picked.numel();
+  torch::Tensor offsets = new_ids(n + 1, m.indptr);
+  torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
+  AsyncCount count = AsyncCount::mirrored();
+  GS_CALL(gs_csc_col_count(cptr(m.indptr), m.indptr.numel() - 1, cptr(picked), n, -1, 0,
+                           mptr(offsets), count.mirror(), nullptr, ws.data_ptr(), ws.numel(),
+                           cur_stream()));
+  count.arm();
+  *nnz = count.get();
+  return offsets;
+}
+
 MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
                                bool with_coo, const torch::Tensor& batch_ptr,
                                int64_t encode_stride) {
   const int64_t num_major = m.indptr.numel() - 1;
   const int64_t n = picked.numel();
   MajorResult r;
-  r.indptr = new_ids(n + 1, m.indptr);
-  torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
-  GS_CALL(gs_csc_col_count(cptr(m.indptr), num_major, cptr(picked), n, -1, 0,
-                           mptr(r.indptr), nullptr, nullptr, ws.data_ptr(), ws.numel(),
-                           cur_stream()));
-  const int64_t nnz = read_last(r.indptr);
+  int64_t nnz = 0;
+  r.indptr = slice_offsets(m, picked, &nnz);
   r.minor_ids = new_ids(nnz, m.indptr);
   r.select = new_ids(nnz, m.indptr);
   if (with_coo) r.major_ids = new_ids(nnz, m.indptr);

@@ -368,6 +368,8 @@ class Graph : public torch::CustomClassHolder {
   ListLabels& list_labels_for(const torch::Tensor& col_seeds, const torch::Tensor& row_ids);
 };
 
+// Offsets of the slice along the compressed axis by `picked`, and its size.
+torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, int64_t* nnz);
 // Operators along the compressed axis (graph.cc) and across it (slicing.cc).
 MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo, const torch::Tensor& batch_ptr,

@@ -400,6 +400,41 @@ int gs_unique_fill_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
                            gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * Column slice of a super-batch with its rows numbered anew: batch b's rows are
+ * the ids that some edge of its columns has, in increasing order, and batch b's
+ * numbers follow batch b - 1's (what the reference gets from ids encoded as
+ * id + batch * num_rows and a sorted unique with inverse,
+ * src/cuda/batch/slicing.cu:25-27, src/cuda/batch/encoding_decoding.cu:99).
+ * A key  id + batch * stride  is a value of a dense range (stride = number of
+ * rows of the matrix), so one flag byte per key takes the place of the sort;
+ * workspace: gs_slice_compact_workspace_bytes, about 1.25 bytes per key.
+ *   cols, sub_indptr, nnz   the columns and the offsets gs_csc_col_count gave
+ *   indices / indices32     row ids, either width (indices32 wins when given)
+ *   batch_ptr[num_batches + 1]  offsets into cols
+ * count: writes out_key_offset[num_cols_picked] (stride times the batch of a
+ *   column), row_ptr[num_batches + 1] (rows before each batch, last = total) and
+ *   the same to row_ptr_mirror when given (pinned host memory).
+ * fill: same arguments, workspace untouched in between; out_rows[total] = the row
+ *   id of every number; the slice itself unless out_indices is NULL: out_indices
+ *   = number of the edge's row, out_select = edge position in the matrix,
+ *   out_coo_col (nullable) = position of its column in cols.
+ * ---------------------------------------------------------------------- */
+size_t gs_slice_compact_workspace_bytes(int64_t num_batches, int64_t stride);
+int gs_slice_compact_count(const int64_t* indptr, const int64_t* indices,
+                           const int32_t* indices32, const int64_t* cols,
+                           int64_t num_cols_picked, const int64_t* sub_indptr, int64_t nnz,
+                           const int64_t* batch_ptr, int64_t num_batches, int64_t stride,
+                           int64_t* out_key_offset, int64_t* row_ptr, int64_t* row_ptr_mirror,
+                           void* workspace, size_t workspace_bytes, gs_stream_t stream);
+int gs_slice_compact_fill(const int64_t* indptr, const int64_t* indices,
+                          const int32_t* indices32, const int64_t* cols,
+                          int64_t num_cols_picked, const int64_t* sub_indptr, int64_t nnz,
+                          const int64_t* key_offset, int64_t num_batches, int64_t stride,
+                          int64_t* out_rows, int64_t* out_coo_col, int64_t* out_indices,
+                          int64_t* out_select, void* workspace, size_t workspace_bytes,
+                          gs_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * out_first[r] = smallest position e with ids[e] == r, INT64_MAX when r does
  * not occur, for ids of a small dense range [0, num_ids) (ids outside it are
  * ignored).  The relabel step of a row-sliced matrix uses it: its rows are
