@@ -42,6 +42,7 @@ SIGNATURES = {
     "gs_profile_get": (_int, [_int, C.c_char_p, _sz, C.POINTER(C.c_longlong),
                               C.POINTER(C.c_double)]),
     "gs_copy_i64": (_int, [_p, _i64, _p, _p]),
+    "gs_take_i64": (_int, [_p, _p, _i64, _p, _p, _p]),
     "gs_scan_workspace_bytes": (_sz, [_i64]),
     "gs_exclusive_scan_i64": (_int, [_p, _p, _i64, _p, _sz, _p]),
     "gs_csc_col_count": (_int, [_p, _i64, _p, _i64, _i64, _int, _p, _p, _p, _p, _sz, _p]),
@@ -66,6 +67,13 @@ SIGNATURES = {
     "gs_decode_batch_ids": (_int, [_p, _i64, _i64, _p, _p, _p]),
     "gs_split_indptr": (_int, [_p, _p, _i64, _i64, _p, _p]),
     "gs_batch_seeds_distinct": (_int, [_p, _p, _p, _p, _i64, _p, _p]),
+    "gs_unique_count_distinct": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _sz,
+                                        _p]),
+    "gs_layer_max_positions": (_i64, []),
+    "gs_layer_workspace_bytes": (_sz, [_i64, _int]),
+    "gs_layer_begin": (_int, [_i64, _int, _p, _sz, _p]),
+    "gs_sample_layer": (_int, [_p, _i64, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _int, _u64,
+                               _u64, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _sz, _p]),
     "gs_slice_compact_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_slice_compact_count": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p,
                                       _p, _sz, _p]),

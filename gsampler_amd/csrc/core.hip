@@ -262,9 +262,34 @@ __global__ __launch_bounds__(kBlock) void copy_i64_kernel(const int64_t* __restr
   if (i < n) store_for_host(dst + i, src[i]);
 }
 
+// out[i] = src[index[i]], for the host as well when mirror is given.
+__global__ __launch_bounds__(kBlock) void take_i64_kernel(const int64_t* __restrict__ src,
+                                                          const int64_t* __restrict__ index,
+                                                          int64_t n, int64_t* __restrict__ out,
+                                                          int64_t* mirror) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int64_t v = src[index[i]];
+  out[i] = v;
+  if (mirror) store_for_host(mirror + i, v);
+}
+
 }  // namespace gs
 
 extern "C" {
+
+int gs_take_i64(const int64_t* src, const int64_t* index, int64_t n, int64_t* out,
+                int64_t* out_mirror, gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(n >= 0, "take_i64: negative length %lld", (long long)n);
+  if (n == 0) return GS_OK;
+  GS_REQUIRE(src && index && out, "take_i64: null pointer");
+  hipStream_t s = as_stream(stream);
+  GS_LAUNCH("take_i64", s,
+            take_i64_kernel<<<dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, s>>>(
+                src, index, n, out, out_mirror));
+  return GS_OK;
+}
 
 int gs_copy_i64(const int64_t* src, int64_t n, int64_t* dst, gs_stream_t stream) {
   using namespace gs;

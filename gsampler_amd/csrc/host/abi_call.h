@@ -308,13 +308,15 @@ class EdgeCount {
     // batch, which is the column's label in the batch's block while the batch's
     // seeds are distinct (the relabel pass then has nothing to do on that side)
     torch::Tensor col_labels;
+    bool no_select = false;  // set by a caller that has no use for the edges' positions
   };
   static Hint& hint() {
     static thread_local Hint h;
     return h;
   }
   struct HintScope {
-    explicit HintScope(const torch::Tensor& col_bptr) {
+    explicit HintScope(const torch::Tensor& col_bptr, bool no_select = false) {
+      hint().no_select = no_select;
       hint().col_bptr = col_bptr;
       hint().edge_bptr = torch::Tensor();
       hint().col_labels = torch::Tensor();
@@ -331,8 +333,11 @@ class EdgeCount {
   void arm(const torch::Tensor& prefix) {
     Hint& h = hint();
     if (h.col_bptr.defined()) {
-      edge_bptr_ = prefix.index_select(0, h.col_bptr);
-      OffsetMirror::prefetch(edge_bptr_);
+      edge_bptr_ = new_ids(h.col_bptr.numel(), prefix);
+      int64_t* mirror = OffsetMirror::reserve(edge_bptr_);
+      GS_CALL(gs_take_i64(cptr(prefix), cptr(h.col_bptr), h.col_bptr.numel(), mptr(edge_bptr_),
+                          mirror, cur_stream()));
+      OffsetMirror::arm(edge_bptr_);
       h.edge_bptr = edge_bptr_;
     } else {
       count_.arm();
@@ -405,6 +410,43 @@ class BatchOffsets {
           k.epoch == cache_epoch())
         return &k;
     return nullptr;
+  }
+};
+
+// `n` elements of a fresh buffer of this library's own from `offset` on, as a
+// tensor: what at::narrow gives, without the dispatcher and the view bookkeeping
+// of autograd (ids carry no gradient; a step cuts a few hundred such pieces).
+// `shared`: whether writes in place to the piece count as writes to the buffer.
+inline torch::Tensor piece_of(const torch::Tensor& buffer, int64_t offset, int64_t n,
+                              bool shared = true) {
+  auto impl = c10::make_intrusive<c10::TensorImpl>(
+      c10::TensorImpl::VIEW, c10::Storage(buffer.storage()), buffer.key_set(), buffer.dtype());
+  impl->set_storage_offset(buffer.storage_offset() + offset);
+  impl->set_sizes_contiguous(c10::IntArrayRef(&n, 1));
+  if (shared && !buffer.is_inference())
+    impl->set_version_counter(buffer.unsafeGetTensorImpl()->version_counter());
+  return torch::Tensor(std::move(impl));
+}
+
+// Pinned host words that live until the process ends, one run per thread: what a
+// kernel reports to an operator that waits for it before it returns.
+class PinnedWords {
+ public:
+  // n words, all marked as not yet there; valid until the thread's next take()
+  static int64_t* take(size_t n) {
+    static thread_local int64_t* words = nullptr;
+    static thread_local size_t capacity = 0;
+    if (capacity < n) {
+      if (words) (void)hipHostFree(words);
+      words = nullptr;
+      capacity = 0;
+      const size_t want = n < 4096 ? 4096 : n;
+      const hipError_t e = hipHostMalloc((void**)&words, want * sizeof(int64_t), hipHostMallocDefault);
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+      capacity = want;
+    }
+    for (size_t i = 0; i < n; ++i) words[i] = kNotYet;
+    return words;
   }
 };
 

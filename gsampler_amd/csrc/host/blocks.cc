@@ -20,8 +20,17 @@ int64_t BlockBatch::NumSrcOf(int64_t b) {
   return f_off_[(size_t)b + 1] - f_off_[(size_t)b];
 }
 
+void BlockBatch::set_host_offsets(std::vector<int64_t> f, std::vector<int64_t> e,
+                                  std::vector<int64_t> c, std::vector<uint8_t> grouped) {
+  f_off_ = std::move(f);
+  e_off_ = std::move(e);
+  c_off_ = std::move(c);
+  grouped_ = std::move(grouped);
+  have_host_ = true;
+}
+
 void BlockBatch::fetch() {
-  if (have_host_) return;
+  if (have_host_ && indptr.defined()) return;
   // Offsets by destination of every block: the columns of the sampled matrix
   // are the destinations, so its indptr, cut at the batch boundaries and
   // rebased, is the blocks' indptr (the relabelled edges keep their order).
@@ -31,6 +40,7 @@ void BlockBatch::fetch() {
   indptr = new_ids(total, sampled_indptr);
   GS_CALL(gs_split_indptr(cptr(sampled_indptr), cptr(col_bptr), num_batches, total, mptr(indptr),
                           cur_stream()));
+  if (have_host_) return;
   distinct = new_ids(num_batches, sampled_indptr);
   GS_CALL(gs_batch_seeds_distinct(cptr(frontier), cptr(frontier_ptr), cptr(col_seeds),
                                   cptr(col_bptr), num_batches, mptr(distinct), cur_stream()));
@@ -76,8 +86,7 @@ BlockViews BlockBatch::Block(int64_t b) {
           nf, nc};
 }
 
-// All blocks at once, one list per field (the per-batch splits are made by
-// torch's split, which is far cheaper than a view at a time).
+// All blocks at once, one list per field.
 BlockParts BlockBatch::Blocks() {
   fetch();
   auto sizes = [](const std::vector<int64_t>& off) {
@@ -86,19 +95,17 @@ BlockParts BlockBatch::Blocks() {
     return s;
   };
   const std::vector<int64_t> ne = sizes(e_off_), nf = sizes(f_off_), nc = sizes(c_off_);
-  std::vector<torch::Tensor> rows = torch::split_with_sizes(row, ne);
-  std::vector<torch::Tensor> cols = torch::split_with_sizes(col, ne);
-  std::vector<torch::Tensor> fronts = torch::split_with_sizes(frontier, nf);
-  std::vector<c10::optional<torch::Tensor>> eids((size_t)num_batches), offs((size_t)num_batches);
-  if (e_ids.has_value()) {
-    std::vector<torch::Tensor> parts = torch::split_with_sizes(e_ids.value(), ne);
-    for (size_t i = 0; i < parts.size(); ++i) eids[i] = parts[i];
+  const size_t B = (size_t)num_batches;
+  std::vector<torch::Tensor> rows(B), cols(B), fronts(B);
+  std::vector<c10::optional<torch::Tensor>> eids(B), offs(B);
+  for (size_t i = 0; i < B; ++i) {
+    rows[i] = piece_of(row, e_off_[i], ne[i]);
+    cols[i] = piece_of(col, e_off_[i], ne[i]);
+    fronts[i] = piece_of(frontier, f_off_[i], nf[i]);
+    if (e_ids.has_value()) eids[i] = piece_of(e_ids.value(), e_off_[i], ne[i]);
+    // block i's offsets sit at [c_off + i, c_off + i + nc] of the split array
+    if (grouped_[i]) offs[i] = piece_of(indptr, c_off_[i] + (int64_t)i, nc[i] + 1);
   }
-  std::vector<int64_t> with_end(nc);
-  for (int64_t& n : with_end) n += 1;  // a block's offsets have one entry more than it has columns
-  std::vector<torch::Tensor> pieces = torch::split_with_sizes(indptr, with_end);
-  for (size_t i = 0; i < pieces.size(); ++i)
-    if (grouped_[i]) offs[i] = pieces[i];
   return {rows, cols, offs, fronts, eids, nf, nc};
 }
 

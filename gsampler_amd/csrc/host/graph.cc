@@ -16,7 +16,7 @@ RandomState& random_state() {
   return state;
 }
 
-static uint64_t next_call_id() { return random_state().next_call++; }
+uint64_t next_call_id() { return random_state().next_call++; }
 
 // ------------------------------------------------------------------ loading
 // A loaded matrix is checked once (a few reductions and one read-back): every
@@ -271,7 +271,10 @@ MajorResult major_sample_uniform(const Compressed& m,
   const int64_t bound = n * fanout;
   const int64_t size = bound <= kBoundLimit ? bound : count.get();
   r.minor_ids = new_ids(size, m.indptr);
-  r.select = new_ids(size, m.indptr);
+  // (the reservoir algorithm keeps its slots in the array of positions)
+  const RandomState& rs = random_state();
+  const bool no_select = EdgeCount::hint().no_select && fanout <= 64 && (replace || rs.algo != GS_ALGO_RESERVOIR);
+  if (!no_select) r.select = new_ids(size, m.indptr);
   if (with_coo) r.major_ids = new_ids(size, m.indptr);
   // a super-batched caller that asked for no coordinate form gets the columns'
   // places inside their batches instead (EdgeCount::Hint)
@@ -281,7 +284,6 @@ MajorResult major_sample_uniform(const Compressed& m,
   int64_t* out_col = with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr;
   const int64_t* col_batch_ptr = label_cols ? cptr(hint.col_bptr) : nullptr;
   const int64_t col_batches = label_cols ? hint.col_bptr.numel() - 1 : 0;
-  const RandomState& rs = random_state();
   const torch::Tensor& narrow = m.narrow_indices();
   if (narrow.defined()) {
     GS_CALL(gs_csc_col_sample_uniform_fill_i32(
@@ -301,7 +303,7 @@ MajorResult major_sample_uniform(const Compressed& m,
   const int64_t nnz = count.get();
   if (label_cols) hint.col_labels = col_labels.narrow(0, 0, nnz);
   r.minor_ids = r.minor_ids.narrow(0, 0, nnz);
-  r.select = r.select.narrow(0, 0, nnz);
+  if (!no_select) r.select = r.select.narrow(0, 0, nnz);
   if (with_coo) r.major_ids = r.major_ids.narrow(0, 0, nnz);
   return r;
 }

@@ -66,6 +66,7 @@ struct RandomState {
   int64_t algo = 0;      // GS_ALGO_AUTO
 };
 RandomState& random_state();
+uint64_t next_call_id();  // takes one
 
 // Views of one mini-batch block: (row, col, indptr by destination -- absent for
 // a mini-batch whose seeds repeat --, source ids, edge ids if the matrix carries
@@ -111,6 +112,10 @@ class BlockBatch : public torch::CustomClassHolder {
   torch::Tensor EdgePtr() { return coo_ptr; }
   torch::Tensor ColPtr() { return col_bptr; }
   c10::optional<torch::Tensor> EdgeIds() { return e_ids; }
+  // For a producer that has the offsets on the host already: of the frontier, the
+  // edges and the columns, and per batch whether its seeds are distinct.
+  void set_host_offsets(std::vector<int64_t> f, std::vector<int64_t> e, std::vector<int64_t> c,
+                        std::vector<uint8_t> grouped);
 
  private:
   void fetch();
@@ -250,8 +255,25 @@ class Graph : public torch::CustomClassHolder {
   // Not in the reference: relabel + all mini-batch blocks of the layer (edge
   // list and compressed form) in one call; see blocks.cc.
   c10::intrusive_ptr<BlockBatch> BatchBlocks(torch::Tensor col_seeds, torch::Tensor row_ids);
+  // Not in the reference: all layers of a node-wise sampler in one call
+  // (layers.cc) -- what gs.jit.compile runs for a chain of slice + sample +
+  // relabel.  Per layer: frontier, row and column labels, edge ids (none) ...
+  std::vector<c10::optional<torch::Tensor>> SampleLayers(
+      torch::Tensor seeds, std::vector<int64_t> fanouts, bool replace,
+      c10::optional<torch::Tensor> edge_probs);
+  // ... or, for a super-batch, the layer's blocks.
+  std::vector<c10::intrusive_ptr<BlockBatch>> BatchSampleLayers(
+      torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
+      c10::optional<torch::Tensor> edge_probs);
 
  private:
+  struct Layer;
+  std::vector<Layer> sample_layers(const torch::Tensor& seeds, const torch::Tensor& col_bptr,
+                                   const std::vector<int64_t>& fanouts, bool replace,
+                                   const c10::optional<torch::Tensor>& edge_probs, bool blocks);
+  Layer large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr, int64_t fanout,
+                    bool replace, const torch::Tensor& cdf);
+
   // Unique/relabel state shared by all_nodes() and to_dgl_block(): the
   // frontier is computed once, the relabel pass reuses the hash tables.
   struct Frontier {
@@ -376,6 +398,10 @@ MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
                         int64_t encode_stride);
 MajorResult major_sample_uniform(const Compressed& m, const torch::Tensor& picked,
                                  int64_t fanout, bool replace, bool with_coo);
+MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
+                                  const torch::Tensor& picked, int64_t fanout, bool replace,
+                                  bool with_coo);
+void check_weighted_fanout(int64_t fanout, bool replace, const char* who);
 MajorResult minor_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo);
 // First n entries of a buffer sized by an upper bound: a view, or a copy when

@@ -1,0 +1,289 @@
+// layers.cc -- all layers of a node-wise sampler (slice columns, sample, unique,
+// relabel; the frontier is the next layer's columns) in one operator call, for a
+// single mini-batch and for a super-batch.
+//
+// Small layers are three launches each (layers.hip), read the number of their
+// columns from the device and are queued one behind the other: the host waits
+// once, at the end, for all offsets.  A layer whose bound has grown too large for
+// that waits for the one before it first; large layers run on the count / fill /
+// unique kernels, with the edges' positions in the matrix left out (nobody asked
+// for them) and the columns' labels left by the sampler.
+#include "abi_call.h"
+#include "graph.h"
+
+namespace gs {
+
+struct Graph::Layer {
+  torch::Tensor frontier, frontier_ptr, row, col, edge_ptr;
+  torch::Tensor block_indptr;    // offsets per block, or
+  torch::Tensor sampled_indptr;  // the offsets over all columns they come from
+  torch::Tensor cols, col_bptr;
+  std::vector<int64_t> f_off, e_off;
+  std::vector<uint8_t> distinct;
+};
+
+namespace {
+
+// Positions (fanout + 1 per column) up to which a layer takes the three launches:
+// beyond, hashing into one table in global memory is slower than partitioning the
+// keys first.  And up to which it may be queued on a bound alone, without the host
+// knowing the number of its columns: outputs are sized by the bound.
+constexpr int64_t kSmallPositions = int64_t(1) << 20;
+constexpr int64_t kQueuedPositions = int64_t(1) << 19;
+
+// A small layer on its way: outputs in one buffer, cut up when the sizes are in.
+struct Queued {
+  torch::Tensor buffer;
+  int64_t bound = 0, fanout = 0;
+  int64_t at_ptr = 0, at_edge_ptr = 0, at_indptr = 0, at_row = 0, at_col = 0;
+  const int64_t* mirror = nullptr;
+};
+
+}  // namespace
+
+// One layer on the kernels for large layers; waits for its edge and key counts.
+Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr,
+                                int64_t fanout, bool replace, const torch::Tensor& cdf) {
+  const Compressed& m = compressed(kCSC);
+  const int64_t B = col_bptr.numel() - 1, S = cols.numel();
+  Layer l;
+  EdgeCount::HintScope batch(col_bptr, /*no_select=*/true);
+  MajorResult r = cdf.defined() ? major_sample_weighted(m, cdf, cols, fanout, replace, false)
+                                : major_sample_uniform(m, cols, fanout, replace, false);
+  l.sampled_indptr = r.indptr;
+  l.edge_ptr = EdgeCount::hint().edge_bptr;
+  if (!l.edge_ptr.defined()) l.edge_ptr = r.indptr.index_select(0, col_bptr);
+  const torch::Tensor& rows = r.minor_ids;
+  const int64_t E = rows.numel();
+  l.row = new_ids(E, rows);
+  const torch::Tensor labels = EdgeCount::hint().col_labels;
+  const bool prefilled = labels.defined() && labels.numel() == E && E > 0;
+  l.col = prefilled ? labels : new_ids(E, rows);
+  torch::Tensor ws = new_workspace(gs_unique_workspace_bytes(S, E, B), rows);
+  l.frontier_ptr = new_ids(B + 1, rows);
+  int64_t* distinct = PinnedWords::take((size_t)B);
+  int64_t* mirror = OffsetMirror::reserve(l.frontier_ptr);
+  GS_CALL(gs_unique_count_distinct(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E,
+                                   B, mptr(l.frontier_ptr), mirror, distinct, ws.data_ptr(),
+                                   ws.numel(), cur_stream()));
+  OffsetMirror::arm(l.frontier_ptr);
+  const int64_t bound = S + E <= kBoundLimit ? S + E : OffsetMirror::values(l.frontier_ptr).back();
+  torch::Tensor frontier = new_ids(bound, rows);
+  GS_CALL(gs_unique_fill_relabel(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E, B,
+                                 cptr(l.frontier_ptr), mptr(frontier), nullptr, cptr(r.indptr),
+                                 mptr(l.row), mptr(l.col), prefilled ? 1 : 0, ws.data_ptr(),
+                                 ws.numel(), cur_stream()));
+  l.e_off = OffsetMirror::values(l.edge_ptr);
+  l.f_off = OffsetMirror::values(l.frontier_ptr);
+  await_words(distinct, (size_t)B, (hipStream_t)cur_stream());
+  l.distinct.assign((size_t)B, 1);
+  for (int64_t b = 0; b < B; ++b) l.distinct[(size_t)b] = distinct[b] != 0;
+  l.frontier = frontier.narrow(0, 0, l.f_off.back());
+  return l;
+}
+
+std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
+                                               const torch::Tensor& col_bptr,
+                                               const std::vector<int64_t>& fanouts, bool replace,
+                                               const c10::optional<torch::Tensor>& edge_probs,
+                                               bool blocks) {
+  const Compressed& m = compressed(kCSC);
+  const bool weighted = edge_probs.has_value();
+  const torch::Tensor cdf = weighted ? weight_cdf_for(edge_probs.value(), kCSC) : torch::Tensor();
+  const int64_t B = col_bptr.defined() ? col_bptr.numel() - 1 : 1;
+  const int64_t num_cols = m.indptr.numel() - 1;
+  const int64_t stride = std::max<int64_t>(std::max(num_cols, num_rows_), 1);
+  const RandomState& rs = random_state();
+  const uint64_t first_call = rs.next_call;
+  // (rows of a matrix that was loaded or converted are known to lie below num_rows)
+  bool small_ok = m.num_minor >= 0 && m.num_minor <= stride && B <= (int64_t)0xFFFFFFFEll / stride &&
+                  (weighted || replace || rs.algo != GS_ALGO_RESERVOIR);
+  auto fits = [&](int64_t columns, int64_t fanout, int64_t most) {
+    return small_ok && columns > 0 && fanout >= 1 && fanout < 64 && columns <= most / (fanout + 1);
+  };
+  const torch::Tensor& narrow = m.narrow_indices();
+  const size_t L = fanouts.size();
+  for (;;) {
+    std::vector<Layer> out(L);
+    std::vector<Queued> queued(L);
+    const size_t words = (size_t)(3 * B + 3);
+    torch::Tensor ws;
+    int64_t ws_positions = 0;
+    int64_t* mirrors = nullptr;
+    bool retry = false;
+    // the layer's columns: exact on the host, or a bound while `known` is false
+    torch::Tensor cols = seeds, ptr = col_bptr;
+    int64_t n = seeds.numel();
+    bool known = true;
+    size_t settled = 0;  // layers whose sizes are on the host
+    auto settle = [&](size_t upto) {
+      for (; settled < upto; ++settled) {
+        Queued& q = queued[settled];
+        if (!q.buffer.defined()) continue;
+        Layer& l = out[settled];
+        await_words(q.mirror, words, (hipStream_t)cur_stream());
+        const int64_t* w = q.mirror;
+        l.f_off.assign(w, w + B + 1);
+        l.e_off.assign(w + B + 1, w + 2 * (B + 1));
+        l.distinct.resize((size_t)B);
+        for (int64_t b = 0; b < B; ++b) l.distinct[(size_t)b] = w[2 * (B + 1) + b] != 0;
+        retry = retry || w[3 * B + 2] != 0;
+        l.frontier = piece_of(q.buffer, 0, l.f_off.back(), false);
+        l.row = piece_of(q.buffer, q.at_row, l.e_off.back(), false);
+        l.col = piece_of(q.buffer, q.at_col, l.e_off.back(), false);
+        l.frontier_ptr = piece_of(q.buffer, q.at_ptr, B + 1, false);
+        l.edge_ptr = piece_of(q.buffer, q.at_edge_ptr, B + 1, false);
+        const int64_t columns = settled ? out[settled - 1].f_off.back() : seeds.numel();
+        if (blocks) l.block_indptr = piece_of(q.buffer, q.at_indptr, columns + B, false);
+      }
+    };
+    for (size_t i = 0; i < L && !retry; ++i) {
+      const int64_t K = fanouts[i];
+      if (!known && !fits(n, K, kQueuedPositions)) {
+        settle(i);
+        if (retry) break;
+        n = out[i - 1].f_off.back();
+        cols = out[i - 1].frontier;
+        ptr = out[i - 1].frontier_ptr;
+        known = true;
+      }
+      Layer& l = out[i];
+      l.cols = cols;
+      l.col_bptr = ptr;
+      if (!fits(n, K, known ? kSmallPositions : kQueuedPositions)) {
+        if (!ptr.defined()) {  // a single batch: offsets 0, n
+          ptr = torch::arange(0, 2, device_options(m.indptr).dtype(torch::kInt64)) * n;
+          BatchOffsets::trust(ptr, n);
+        }
+        l = large_layer(cols, ptr, K, replace, cdf);
+        mirrors = nullptr;  // it has used the thread's pinned words
+        l.cols = cols;
+        l.col_bptr = ptr;
+        cols = l.frontier;
+        ptr = l.frontier_ptr;
+        n = cols.numel();
+        settled = i + 1;
+        continue;
+      }
+      const int64_t positions = n * (K + 1);
+      if (ws_positions < positions) {
+        // room for the layers that can be queued behind this one as well
+        int64_t most = positions, bound = positions;
+        for (size_t j = i + 1; j < L && fits(bound, fanouts[j], kQueuedPositions); ++j) {
+          bound *= fanouts[j] + 1;
+          most = std::max(most, bound);
+        }
+        ws = new_workspace(gs_layer_workspace_bytes(most, weighted ? 1 : 0), m.indptr);
+        ws_positions = most;
+        GS_CALL(gs_layer_begin(most, weighted ? 1 : 0, ws.data_ptr(), (size_t)ws.numel(),
+                               cur_stream()));
+      }
+      if (!mirrors) mirrors = PinnedWords::take(words * L);
+      Queued& q = queued[i];
+      auto even = [](int64_t x) { return (x + 1) & ~int64_t(1); };
+      int64_t at = even(positions);
+      q.at_row = at;
+      at += even(n * K);
+      q.at_col = at;
+      at += even(n * K);
+      q.at_ptr = at;
+      at += even(B + 1);
+      q.at_edge_ptr = at;
+      at += even(B + 1);
+      q.at_indptr = at;
+      at += blocks ? n + B : 0;
+      q.buffer = new_ids(at, m.indptr);
+      q.mirror = mirrors + words * i;
+      int64_t* base = mptr(q.buffer);
+      GS_CALL(gs_sample_layer(
+          cptr(m.indptr), num_cols, cptr(m.indices),
+          narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(cdf), stride, cptr(cols), n,
+          cptr(ptr), B, K, replace ? 1 : 0, rs.seed, next_call_id(), base, base + q.at_ptr,
+          base + q.at_row, base + q.at_col, base + q.at_edge_ptr,
+          blocks ? base + q.at_indptr : nullptr, mirrors + words * i, ws_positions, ws.data_ptr(),
+          (size_t)ws.numel(), cur_stream()));
+      // the next layer's columns, as far as they are known
+      cols = piece_of(q.buffer, 0, positions, false);
+      ptr = piece_of(q.buffer, q.at_ptr, B + 1, false);
+      n = positions;
+      known = false;
+    }
+    if (!retry) settle(L);
+    if (!retry) {
+      for (size_t i = 1; i < L; ++i)
+        if (queued[i - 1].buffer.defined()) {  // the pieces, in place of the bounds
+          out[i].cols = out[i - 1].frontier;
+          out[i].col_bptr = out[i - 1].frontier_ptr;
+        }
+      for (const Layer& l : out) {
+        BatchOffsets::trust(l.frontier_ptr, l.f_off.back());
+        BatchOffsets::trust(l.edge_ptr, l.e_off.back());
+      }
+      return out;
+    }
+    // a seed that is no id of this matrix: its keys do not fit the small layers' table
+    GS_CALL(hipStreamSynchronize((hipStream_t)cur_stream()) == hipSuccess ? GS_OK : GS_ERR_HIP);
+    random_state().next_call = first_call;
+    small_ok = false;
+  }
+}
+
+static void check_layers(const std::vector<int64_t>& fanouts, bool replace, bool weighted) {
+  TORCH_CHECK(!fanouts.empty(), "SampleLayers: no layers");
+  for (int64_t k : fanouts) {
+    TORCH_CHECK(k >= 0, "fanout must be non-negative, got ", k);
+    if (weighted) check_weighted_fanout(k, replace, "SampleLayers");
+  }
+}
+
+std::vector<c10::optional<torch::Tensor>> Graph::SampleLayers(
+    torch::Tensor seeds, std::vector<int64_t> fanouts, bool replace,
+    c10::optional<torch::Tensor> edge_probs) {
+  check_layers(fanouts, replace, edge_probs.has_value());
+  seeds = ids(seeds, "seeds");
+  std::vector<c10::optional<torch::Tensor>> out;
+  if (seeds.numel() == 0) {  // no columns, no edges: layer after layer
+    for (size_t i = 0; i < fanouts.size(); ++i) {
+      next_call_id();
+      const torch::Tensor none = new_ids(0, compressed(kCSC).indptr);
+      out.insert(out.end(), {none, none.clone(), none.clone(), c10::nullopt});
+    }
+    return out;
+  }
+  for (Layer& l : sample_layers(seeds, {}, fanouts, replace, edge_probs, false))
+    out.insert(out.end(), {l.frontier, l.row, l.col, c10::nullopt});
+  return out;
+}
+
+std::vector<c10::intrusive_ptr<BlockBatch>> Graph::BatchSampleLayers(
+    torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
+    c10::optional<torch::Tensor> edge_probs) {
+  check_layers(fanouts, replace, edge_probs.has_value());
+  seeds = ids(seeds, "seeds");
+  col_bptr = ids(col_bptr, "col_bptr");
+  BatchOffsets::check(col_bptr, seeds.numel(), "BatchSampleLayers");
+  std::vector<int64_t> c_off = OffsetMirror::values(col_bptr);
+  std::vector<c10::intrusive_ptr<BlockBatch>> out;
+  for (Layer& l : sample_layers(seeds, col_bptr, fanouts, replace, edge_probs, true)) {
+    auto b = c10::make_intrusive<BlockBatch>();
+    b->num_batches = col_bptr.numel() - 1;
+    b->num_dst_total = l.cols.numel();
+    b->frontier = l.frontier;
+    b->frontier_ptr = l.frontier_ptr;
+    b->row = l.row;
+    b->col = l.col;
+    b->coo_ptr = l.edge_ptr;
+    b->col_bptr = l.col_bptr;
+    b->col_seeds = l.cols;
+    b->sampled_indptr = l.sampled_indptr;
+    b->indptr = l.block_indptr;
+    std::vector<int64_t> f_off = l.f_off;
+    b->set_host_offsets(std::move(l.f_off), std::move(l.e_off), std::move(c_off),
+                        std::move(l.distinct));
+    c_off = std::move(f_off);
+    out.push_back(std::move(b));
+  }
+  return out;
+}
+
+}  // namespace gs

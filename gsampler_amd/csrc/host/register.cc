@@ -114,7 +114,9 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_BatchGetCOOEids", &Graph::BatchGetCOOEids)
       .def("_CAPI_BatchGetColCounts", &Graph::BatchGetColCounts)
       .def("_CAPI_BatchGetValidNodes", &Graph::BatchGetValidNodes)
-      .def("_CAPI_BatchBlocks", &Graph::BatchBlocks);
+      .def("_CAPI_BatchBlocks", &Graph::BatchBlocks)
+      .def("_CAPI_SampleLayers", &Graph::SampleLayers)
+      .def("_CAPI_BatchSampleLayers", &Graph::BatchSampleLayers);
 }
 
 TORCH_LIBRARY(gs_ops, m) {

@@ -5,8 +5,6 @@
 
 namespace gs {
 
-static uint64_t take_call_id() { return random_state().next_call++; }
-
 // Traces are stored step-major ([walk_length + 1][num_seeds] in memory) and
 // returned with shape [num_seeds, walk_length + 1] exactly as the reference
 // does (src/cuda/fusion/random_walk.cu:34,67): callers obtain per-step rows
@@ -19,7 +17,7 @@ torch::Tensor Graph::RandomWalk(torch::Tensor seeds, int64_t walk_length) {
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
   GS_CALL(gs_random_walk(cptr(csc_->indptr), cptr(csc_->indices), num_cols_,
-                         cptr(seeds), n, walk_length, rs.seed, take_call_id(),
+                         cptr(seeds), n, walk_length, rs.seed, next_call_id(),
                          mptr(out), cur_stream()));
   return out.reshape({n, -1});
 }
@@ -50,7 +48,7 @@ torch::Tensor Graph::Node2Vec(torch::Tensor seeds, int64_t walk_length, double p
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
   GS_CALL(gs_node2vec(cptr(csc_->indptr), cptr(csc_->indices), num_cols_,
-                      cptr(seeds), n, walk_length, p, q, rs.seed, take_call_id(),
+                      cptr(seeds), n, walk_length, p, q, rs.seed, next_call_id(),
                       mptr(out), cur_stream()));
   return out.reshape({n, -1});
 }

@@ -5,8 +5,6 @@
 
 namespace gs {
 
-static uint64_t take_call_id() { return random_state().next_call++; }
-
 static torch::Tensor f32(const torch::Tensor& t, const char* name) {
   TORCH_CHECK(t.defined() && t.is_cuda(), name, " must live on the GPU");
   TORCH_CHECK(t.scalar_type() == torch::kFloat32, name, " must be float32 (got ",
@@ -50,7 +48,7 @@ GraphAndIndex Graph::SamplingProbs(int64_t axis, torch::Tensor edge_probs,
   const RandomState& rs = random_state();
   GS_CALL(gs_csc_col_sample_weighted_fill(
       cptr(m.indptr), n, cptr(m.indices), probs.data_ptr<float>(), nullptr,
-      nullptr, n, fanout, replace ? 1 : 0, rs.seed, take_call_id(), cptr(r.indptr),
+      nullptr, n, fanout, replace ? 1 : 0, rs.seed, next_call_id(), cptr(r.indptr),
       nullptr, nullptr,
       replace ? scratch.data_ptr() : nullptr,
       with_coo ? mptr(r.major_ids) : nullptr, mptr(r.minor_ids), mptr(r.select),
@@ -85,6 +83,52 @@ torch::Tensor Graph::weight_cdf_for(const torch::Tensor& edge_probs, int64_t for
   return cdf_;
 }
 
+// Slice + sample through the CDF; the twin of major_sample_uniform.
+MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
+                                  const torch::Tensor& picked, int64_t fanout, bool replace,
+                                  bool with_coo) {
+  const int64_t num_major = m.indptr.numel() - 1, n = picked.numel();
+  MajorResult r;
+  r.indptr = new_ids(n + 1, m.indptr);
+  torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
+  EdgeCount count;
+  torch::Tensor col_span = new_ids(n, m.indptr);  // the columns' starts and degrees, for the fill pass
+  GS_CALL(gs_csc_col_count(cptr(m.indptr), num_major, cptr(picked), n, fanout,
+                           replace ? 1 : 0, mptr(r.indptr), count.mirror(), mptr(col_span),
+                           ws.data_ptr(), ws.numel(), cur_stream()));
+  count.arm(r.indptr);
+  const int64_t bound = n * fanout;
+  const int64_t size = bound <= kBoundLimit ? bound : count.get();
+  r.minor_ids = new_ids(size, m.indptr);
+  EdgeCount::Hint& hint = EdgeCount::hint();
+  const bool no_select = hint.no_select;
+  if (!no_select) r.select = new_ids(size, m.indptr);
+  if (with_coo) r.major_ids = new_ids(size, m.indptr);
+  // (as in the uniform sampler: a super-batched caller without a coordinate form
+  // gets the columns' places inside their batches)
+  const bool label_cols = !with_coo && hint.col_bptr.defined();
+  torch::Tensor col_labels = label_cols ? new_ids(size, m.indptr) : torch::Tensor();
+  const RandomState& rs = random_state();
+  GS_CALL(gs_csc_col_sample_weighted_fill(
+      cptr(m.indptr), num_major, cptr(m.indices), nullptr, cptr(cdf), cptr(picked), n,
+      fanout, replace ? 1 : 0, rs.seed, next_call_id(), cptr(r.indptr), cptr(col_span),
+      nullptr, nullptr,
+      with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr,
+      mptr(r.minor_ids), mptr(r.select), label_cols ? cptr(hint.col_bptr) : nullptr,
+      label_cols ? hint.col_bptr.numel() - 1 : 0, cur_stream()));
+  const int64_t nnz = count.get();
+  if (label_cols) hint.col_labels = col_labels.narrow(0, 0, nnz);
+  r.minor_ids = r.minor_ids.narrow(0, 0, nnz);
+  if (!no_select) r.select = r.select.narrow(0, 0, nnz);
+  if (with_coo) r.major_ids = r.major_ids.narrow(0, 0, nnz);
+  return r;
+}
+
+void check_weighted_fanout(int64_t fanout, bool replace, const char* who) {
+  TORCH_CHECK(fanout >= 0, "fanout must be non-negative, got ", fanout);
+  TORCH_CHECK(replace || fanout <= 64, who, ": fanout above 64 needs replace=True");
+}
+
 GraphAndIndex Graph::FusedSlicingSamplingProbs(int64_t axis, torch::Tensor seeds,
                                                torch::Tensor edge_probs,
                                                int64_t fanout, bool replace,
@@ -96,46 +140,12 @@ GraphAndIndex Graph::FusedSlicingSamplingProbs(int64_t axis, torch::Tensor seeds
   const int64_t other = on_format == kCSC ? kCSR : kCSC;
   TORCH_CHECK(output_format != other, "FusedSlicingSamplingProbs: on_format ", on_format,
               " cannot produce output_format ", output_format);
-  TORCH_CHECK(fanout >= 0, "fanout must be non-negative, got ", fanout);
-  TORCH_CHECK(replace || fanout <= 64,
-              "FusedSlicingSamplingProbs: fanout above 64 needs replace=True");
+  check_weighted_fanout(fanout, replace, "FusedSlicingSamplingProbs");
   seeds = ids(seeds, "seeds");
   const Compressed& m = compressed(on_format);
   torch::Tensor cdf = weight_cdf_for(edge_probs, on_format);
-  const bool with_coo = output_format & kCOO;
-  const int64_t num_major = m.indptr.numel() - 1, n = seeds.numel();
-  MajorResult r;
-  r.indptr = new_ids(n + 1, m.indptr);
-  torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
-  EdgeCount count;
-  torch::Tensor col_span = new_ids(n, m.indptr);  // the columns' starts and degrees, for the fill pass
-  GS_CALL(gs_csc_col_count(cptr(m.indptr), num_major, cptr(seeds), n, fanout,
-                           replace ? 1 : 0, mptr(r.indptr), count.mirror(), mptr(col_span),
-                           ws.data_ptr(), ws.numel(), cur_stream()));
-  count.arm(r.indptr);
-  const int64_t bound = n * fanout;
-  const int64_t size = bound <= kBoundLimit ? bound : count.get();
-  r.minor_ids = new_ids(size, m.indptr);
-  r.select = new_ids(size, m.indptr);
-  if (with_coo) r.major_ids = new_ids(size, m.indptr);
-  // (as in the uniform sampler: a super-batched caller without a coordinate form
-  // gets the columns' places inside their batches)
-  EdgeCount::Hint& hint = EdgeCount::hint();
-  const bool label_cols = !with_coo && hint.col_bptr.defined();
-  torch::Tensor col_labels = label_cols ? new_ids(size, m.indptr) : torch::Tensor();
-  const RandomState& rs = random_state();
-  GS_CALL(gs_csc_col_sample_weighted_fill(
-      cptr(m.indptr), num_major, cptr(m.indices), nullptr, cptr(cdf), cptr(seeds), n,
-      fanout, replace ? 1 : 0, rs.seed, take_call_id(), cptr(r.indptr), cptr(col_span),
-      nullptr, nullptr,
-      with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr,
-      mptr(r.minor_ids), mptr(r.select), label_cols ? cptr(hint.col_bptr) : nullptr,
-      label_cols ? hint.col_bptr.numel() - 1 : 0, cur_stream()));
-  const int64_t nnz = count.get();
-  if (label_cols) hint.col_labels = col_labels.narrow(0, 0, nnz);
-  r.minor_ids = r.minor_ids.narrow(0, 0, nnz);
-  r.select = r.select.narrow(0, 0, nnz);
-  if (with_coo) r.major_ids = r.major_ids.narrow(0, 0, nnz);
+  MajorResult r = major_sample_weighted(m, cdf, seeds, fanout, replace, output_format & kCOO);
+  const int64_t n = seeds.numel();
   const int64_t new_rows = axis == 0 ? n : num_rows_;
   const int64_t new_cols = axis == 0 ? num_cols_ : n;
   GraphPtr g = derive(on_format, output_format, r, new_rows, new_cols);
@@ -171,7 +181,7 @@ torch::Tensor ListSampling(int64_t num_items, int64_t num_picks, bool replace) {
       {count}, torch::TensorOptions().dtype(torch::kInt64).device(torch::kCUDA));
   const RandomState& rs = random_state();
   GS_CALL(gs_list_sample_uniform(num_items, num_picks, replace ? 1 : 0,
-                                 (int)rs.algo, rs.seed, take_call_id(), mptr(out),
+                                 (int)rs.algo, rs.seed, next_call_id(), mptr(out),
                                  cur_stream()));
   return out;
 }
@@ -209,7 +219,7 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
   const RandomState& rs = random_state();
   GS_CALL(gs_list_sample_weighted_fill(
       probs.data_ptr<float>(), cptr(range), n, nseg, num_picks, replace ? 1 : 0,
-      rs.seed, take_call_id(), cptr(out_range), total, mptr(out), ws.data_ptr(),
+      rs.seed, next_call_id(), cptr(out_range), total, mptr(out), ws.data_ptr(),
       ws.numel(), cur_stream()));
   return {out, out_range};
 }

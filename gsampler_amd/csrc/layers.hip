@@ -1,0 +1,540 @@
+// layers.hip -- one layer of node-wise sampling (column slice + sample + unique +
+// relabel) in three launches, for layers small enough that launches and the
+// host's waits cost more than the work.
+//
+// The layer's keys are laid out with a fixed number of places per column, so that
+// nothing has to be counted before it can be sampled: batch b, whose columns are
+// [s_lo, s_lo + ns), owns (fanout + 1) ns positions from (fanout + 1) s_lo on -- its
+// seeds first, then fanout places per column, of which a short column leaves some
+// empty.  Order of positions = order of the keys of the layer (seeds of a batch,
+// then its edges), so first occurrences, ranks and labels come out as they do from
+// the packed layout.
+//   pick    a column on fanout + 1 neighbouring lanes (its seed and its picks).
+//           Keys are first made distinct inside the work-group in LDS -- a hub that
+//           every column picks would otherwise be thousands of atomics on one
+//           word -- and then go into one table in global memory, smallest position
+//           first.  Every position keeps the slot its key landed in.
+//   flag    every position reads the first position of its key from that slot; per
+//           64 positions a word of which are first occurrences and one of which
+//           are edges; counts per tile of 1024 positions
+//   label   every work-group adds up the tiles' counts for itself (at most 1024),
+//           then writes frontier, labels and offsets of its tile, and empties its
+//           share of the table for the next layer.  Work-group 0 reports the
+//           offsets of all batches to the host.
+// The number of columns is read from the device (the last entry of the previous
+// layer's frontier offsets), launches are sized by its bound, and nothing is waited
+// for between layers.
+// GraphSAGE [25,10], 1024 seeds, 100 K nodes: 16 launches and four waits, 128 us,
+// before; seven launches and one wait now.
+#include "common.h"
+#include "hashtable.h"
+
+namespace gs {
+
+constexpr int kPickThreads = 512;
+constexpr int kPickSlots = 1024;  // LDS table of a work-group's keys, at most half full
+constexpr int kPickShift = 22;    // 32 - log2(kPickSlots)
+constexpr int kLayerTile = 1024;  // positions per work-group of flag and label
+constexpr int kLayerWords = kLayerTile / kWave;
+constexpr int kLayerWordsPerWave = kLayerWords / (kBlock / kWave);
+constexpr int kLayerMaxTiles = 1024;
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
+static_assert(kPickThreads * 2 <= kPickSlots, "the LDS table is at most half full");
+
+// 64 positions: which are first occurrences / edges, and how many of either their
+// tile has before them.
+struct alignas(16) LayerWord {
+  uint64_t first, edge;
+  uint32_t first_before, edge_before;
+  uint64_t unused;
+};
+
+struct LayerWs {
+  uint64_t* table;     // [slots] key << 32 | first position, empty between layers
+  uint32_t* slot;      // [positions] slot of the position's key, kNoSlot: no key here
+  uint32_t* first;     // [positions] first position of the key
+  uint32_t* key;       // [positions] the key, written where it occurs first
+  LayerWord* words;    // [tiles * kLayerWords]
+  uint2* tile_cnt;     // [tiles] first occurrences, edges
+  int64_t* picked;     // [columns * fanout] rows of a weighted layer
+  int32_t* wide;       // [1] raised by a seed that is no id of the matrix
+  int64_t slots, tiles;
+  size_t total;
+};
+
+static int64_t layer_table_slots(int64_t positions) {
+  int64_t slots = 4096;
+  while (slots < 2 * positions) slots <<= 1;
+  return slots;
+}
+
+static LayerWs carve_layer(void* ws, int64_t positions, int weighted) {
+  Carver c(ws);
+  LayerWs w;
+  const int64_t n = positions > 0 ? positions : 1;
+  w.slots = layer_table_slots(n);
+  w.tiles = ceil_div(n, kLayerTile);
+  w.table = c.take<uint64_t>((size_t)w.slots);  // first, so that its place does not depend on the rest
+  w.wide = c.take<int32_t>(1);
+  w.slot = c.take<uint32_t>((size_t)n);
+  w.first = c.take<uint32_t>((size_t)n);
+  w.key = c.take<uint32_t>((size_t)n);
+  w.words = c.take<LayerWord>((size_t)w.tiles * kLayerWords);
+  w.tile_cnt = c.take<uint2>((size_t)w.tiles);
+  w.picked = c.take<int64_t>(weighted ? (size_t)n : 1);
+  w.total = c.total();
+  return w;
+}
+
+// The layer's columns: ids, how many (on the device), and their batches.
+struct LayerColumns {
+  const int64_t* ids;
+  const int64_t* ptr;  // [B + 1] offsets of the batches, null: one batch of `count`
+  int64_t B, count;    // count: bound of the number of columns when ptr is given
+  __device__ __forceinline__ int64_t num() const { return ptr ? ptr[B] : count; }
+  __device__ __forceinline__ int64_t lo(int64_t b) const { return ptr ? ptr[b] : 0; }
+  __device__ __forceinline__ int64_t hi(int64_t b) const { return ptr ? ptr[b + 1] : count; }
+  // batch of a column, at or after batch b0
+  __device__ __forceinline__ int64_t batch_of(int64_t c, int64_t b0) const {
+    if (!ptr) return 0;
+    int64_t b = b0;
+    while (b + 1 < B && ptr[b + 1] <= c) ++b;
+    return b;
+  }
+};
+
+// The slot of a key in the global table after (key, position) went in.
+__device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask, uint32_t key,
+                                                 uint32_t position) {
+  const uint64_t mine = ((uint64_t)key << 32) | position;
+  uint32_t slot = hash32(key) & mask;
+  for (uint32_t probes = 0; probes <= mask; ++probes) {  // at most half full: ends early
+    uint64_t cur = table[slot];
+    if (cur == kEmptySlot) {
+      cur = atomicCAS((unsigned long long*)(table + slot), (unsigned long long)kEmptySlot,
+                      (unsigned long long)mine);
+      if (cur == kEmptySlot) return slot;
+    }
+    if ((uint32_t)(cur >> 32) == key) {
+      // a stale read can only cost an atomic: positions of a slot only decrease
+      if (cur > mine) atomicMin((unsigned long long*)(table + slot), (unsigned long long)mine);
+      return slot;
+    }
+    slot = (slot + 1) & mask;
+  }
+  return 0;
+}
+
+// Floyd's rule among the lanes of one column (sampling.hip): lane `lane` of the
+// `K` from wavefront lane gbase on.
+__device__ __forceinline__ int64_t floyd_pick(int lane, int gbase, int K, int64_t deg,
+                                              PhiloxKey key, uint64_t pos) {
+  const int64_t base = deg - K;
+  const int64_t j = base + lane;
+  const int64_t t = (int64_t)philox_bounded(key, pos, (uint64_t)lane, (uint64_t)j + 1);
+  bool dup = false;
+  for (int m = 0; m < K; ++m) {
+    const int64_t tm = __shfl(t, gbase + m, kWave);
+    dup |= (m < lane) & (tm == t);
+  }
+  const int64_t mi = t - base;
+  for (int m = 0; m < K; ++m) {
+    const int dm = __shfl((int)dup, gbase + m, kWave);
+    if (mi == m && m < lane) dup |= (dm != 0);
+  }
+  return dup ? j : t;
+}
+
+// picked: rows drawn by another kernel, fanout places per column; null: uniform.
+template <typename IdT>
+__global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_cols, const IdT* __restrict__ indices,
+    LayerColumns cols, int fanout, int cols_per_wave, int replace, PhiloxKey key, uint32_t stride,
+    const int64_t* __restrict__ picked, uint64_t* table, uint32_t mask,
+    uint32_t* __restrict__ slot_of, int32_t* wide) {
+  __shared__ uint32_t tags[kPickSlots], mins[kPickSlots], global_slot[kPickSlots];
+  const int64_t n = cols.num();
+  constexpr int kWaves = kPickThreads / kWave;
+  const int64_t first_col = (int64_t)blockIdx.x * (kWaves * cols_per_wave);
+  if (first_col >= n) return;  // uniform per work-group
+  for (int i = threadIdx.x; i < kPickSlots; i += kPickThreads) {
+    tags[i] = kNoSlot;
+    mins[i] = 0xFFFFFFFFu;
+  }
+  const int wave_lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int width = fanout + 1;
+  const int group = wave_lane / width;
+  const int lane = wave_lane - group * width;  // 0: the seed, j + 1: pick j
+  const int64_t c = first_col + wave * cols_per_wave + group;
+  const bool live = group < cols_per_wave && c < n;
+  uint32_t my_key = kNoSlot, position = 0;
+  if (live) {
+    const int64_t id = cols.ids[c];
+    const int64_t b0 = cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(first_col)) : 0;
+    const int64_t b = cols.batch_of(c, b0);
+    const int64_t s_lo = cols.lo(b), ns = cols.hi(b) - s_lo;
+    const int64_t fb = s_lo * width;
+    int64_t start;
+    const int64_t deg = column_degree(indptr, num_cols, id, &start);
+    int64_t row = -1;
+    if (lane == 0) {
+      row = id;
+      if ((uint64_t)id >= (uint64_t)stride) {  // no id of this matrix: the caller takes another path
+        *wide = 1;
+        row = 0;
+      }
+      position = (uint32_t)(fb + (c - s_lo));
+    } else {
+      position = (uint32_t)(fb + ns + (c - s_lo) * fanout + (lane - 1));
+      const int64_t j = lane - 1;
+      if (picked) {
+        const int64_t have = replace ? (deg > 0 ? fanout : 0) : (deg < fanout ? deg : fanout);
+        if (j < have) row = picked[c * fanout + j];
+      } else if (replace) {
+        if (deg > 0)
+          row = (int64_t)indices[start + (int64_t)philox_bounded(key, (uint64_t)c, (uint64_t)j,
+                                                                 (uint64_t)deg)];
+      } else if (deg <= fanout) {
+        if (j < deg) row = (int64_t)indices[start + j];
+      } else {
+        row = (int64_t)indices[start + floyd_pick((int)j, group * width + 1, fanout, deg, key,
+                                                  (uint64_t)c)];
+      }
+    }
+    if (row >= 0) my_key = (uint32_t)b * stride + (uint32_t)row;
+  }
+  __syncthreads();
+  uint32_t at = 0;
+  if (my_key != kNoSlot) {
+    at = (my_key * 0x85EBCA6Bu) >> kPickShift;
+    for (;;) {
+      uint32_t cur = tags[at];
+      if (cur == kNoSlot) cur = atomicCAS(&tags[at], kNoSlot, my_key);
+      if (cur == kNoSlot || cur == my_key) break;
+      at = (at + 1) & (kPickSlots - 1);
+    }
+    if (mins[at] > position) atomicMin(&mins[at], position);
+  }
+  __syncthreads();
+  if (my_key != kNoSlot && mins[at] == position)
+    global_slot[at] = layer_insert(table, mask, my_key, position);
+  __syncthreads();
+  if (live) slot_of[position] = my_key != kNoSlot ? global_slot[at] : kNoSlot;
+}
+
+// What the work-groups of a tile know about the batches in it.
+struct TileBatches {
+  int64_t b_lo, b_hi;  // batches of the tile's first and last position
+  __device__ __forceinline__ int64_t of(const LayerColumns& cols, int width, int64_t p) const {
+    int64_t b = b_lo;
+    while (b < b_hi && cols.ptr[b + 1] * width <= p) ++b;
+    return b;
+  }
+};
+__device__ __forceinline__ TileBatches tile_batches(const LayerColumns& cols, int width,
+                                                    int64_t p0, int64_t p_last) {
+  if (!cols.ptr) return TileBatches{0, 0};
+  return TileBatches{segment_of(cols.ptr, cols.B, wave_uniform_first(p0 / width)),
+                     segment_of(cols.ptr, cols.B, wave_uniform_first(p_last / width))};
+}
+
+__global__ __launch_bounds__(kBlock) void layer_flag_kernel(
+    LayerColumns cols, int fanout, const uint64_t* __restrict__ table,
+    const uint32_t* __restrict__ slot_of, uint32_t* __restrict__ first,
+    uint32_t* __restrict__ keys, LayerWord* __restrict__ words, uint2* __restrict__ tile_cnt) {
+  __shared__ uint32_t wave_first[kBlock / kWave], wave_edge[kBlock / kWave];
+  const int width = fanout + 1;
+  const int64_t N = cols.num() * width;
+  const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
+  if (p0 >= N) return;
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  const int64_t wave_p0 = p0 + (int64_t)wave * kLayerWordsPerWave * kWave;
+  uint32_t s[kLayerWordsPerWave];
+  uint64_t e[kLayerWordsPerWave];
+#pragma unroll
+  for (int j = 0; j < kLayerWordsPerWave; ++j) {
+    const int64_t p = wave_p0 + j * kWave + lane;
+    s[j] = p < N ? slot_of[p] : kNoSlot;
+  }
+#pragma unroll
+  for (int j = 0; j < kLayerWordsPerWave; ++j) e[j] = s[j] != kNoSlot ? table[s[j]] : 0ull;
+  const TileBatches batches =
+      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
+  LayerWord mine{0ull, 0ull, 0u, 0u, 0ull};
+  uint32_t firsts = 0, edges = 0;
+#pragma unroll
+  for (int j = 0; j < kLayerWordsPerWave; ++j) {
+    const int64_t p = wave_p0 + j * kWave + lane;
+    bool is_first = false, is_edge = false;
+    if (s[j] != kNoSlot) {
+      const uint32_t f = (uint32_t)e[j];
+      first[p] = f;
+      is_first = f == (uint32_t)p;
+      if (is_first) keys[p] = (uint32_t)(e[j] >> 32);
+      const int64_t b = batches.of(cols, width, p);
+      const int64_t s_lo = cols.lo(b);
+      is_edge = p - s_lo * width >= cols.hi(b) - s_lo;
+    }
+    const uint64_t fw = __ballot(is_first), ew = __ballot(is_edge);
+    if (lane == j) mine = LayerWord{fw, ew, firsts, edges, 0ull};
+    firsts += (uint32_t)__popcll(fw);
+    edges += (uint32_t)__popcll(ew);
+  }
+  if (lane == 0) {
+    wave_first[wave] = firsts;
+    wave_edge[wave] = edges;
+  }
+  __syncthreads();
+  uint32_t fb = 0, eb = 0, fa = 0, ea = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / kWave; ++w) {
+    if (w < wave) {
+      fb += wave_first[w];
+      eb += wave_edge[w];
+    }
+    fa += wave_first[w];
+    ea += wave_edge[w];
+  }
+  if (lane < kLayerWordsPerWave) {
+    mine.first_before += fb;
+    mine.edge_before += eb;
+    words[(int64_t)blockIdx.x * kLayerWords + wave * kLayerWordsPerWave + lane] = mine;
+  }
+  if (threadIdx.x == 0) tile_cnt[blockIdx.x] = make_uint2(fa, ea);
+}
+
+struct LayerOut {
+  int64_t *frontier, *frontier_ptr, *row, *col, *edge_ptr, *block_indptr;  // block_indptr may be null
+  // for the host: frontier_ptr[B + 1], edge_ptr[B + 1], seeds distinct[B], wide seeds[1]
+  int64_t* mirror;
+};
+
+__global__ __launch_bounds__(kBlock) void layer_label_kernel(
+    LayerColumns cols, int fanout, uint32_t stride, const uint32_t* __restrict__ first,
+    const uint32_t* __restrict__ keys, const LayerWord* __restrict__ words,
+    const uint2* __restrict__ tile_cnt, uint64_t* __restrict__ table, int64_t table_slots,
+    const int32_t* __restrict__ wide, LayerOut out) {
+  __shared__ uint2 before[kLayerMaxTiles];  // first occurrences and edges before a tile
+  __shared__ uint64_t smem[kBlock / kWave + 1];
+  // the table is done with: its share emptied by every work-group of the launch
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < table_slots;
+       i += (int64_t)gridDim.x * kBlock)
+    table[i] = kEmptySlot;
+  const int width = fanout + 1;
+  const int64_t n = cols.num(), N = n * width;
+  const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
+  if (blockIdx.x != 0 && (int64_t)blockIdx.x >= tiles) return;
+  constexpr int kPer = kLayerMaxTiles / kBlock;
+  uint2 cnt[kPer];
+  uint64_t sum = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int64_t t = (int64_t)threadIdx.x * kPer + j;
+    cnt[j] = t < tiles ? tile_cnt[t] : make_uint2(0u, 0u);
+    sum += ((uint64_t)cnt[j].y << 32) | cnt[j].x;
+  }
+  uint64_t total;
+  uint64_t run = block_exclusive_sum<uint64_t>(sum, smem, &total);
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    before[threadIdx.x * kPer + j] = make_uint2((uint32_t)run, (uint32_t)(run >> 32));
+    run += ((uint64_t)cnt[j].y << 32) | cnt[j].x;
+  }
+  __syncthreads();
+  const uint32_t all_first = (uint32_t)total, all_edges = (uint32_t)(total >> 32);
+  auto ranks = [&](int64_t p, uint32_t* f, uint32_t* e) {  // counts before position p <= N
+    if (p >= N) {
+      *f = all_first;
+      *e = all_edges;
+      return;
+    }
+    const LayerWord w = words[p / kWave];
+    const uint2 t = before[p / kLayerTile];
+    const uint64_t below = (1ull << (int)(p % kWave)) - 1ull;
+    *f = t.x + w.first_before + (uint32_t)__popcll(w.first & below);
+    *e = t.y + w.edge_before + (uint32_t)__popcll(w.edge & below);
+  };
+  auto rank_first = [&](uint32_t p) {
+    const LayerWord w = words[p / kWave];
+    return before[p / kLayerTile].x + w.first_before +
+           (uint32_t)__popcll(w.first & ((1ull << (int)(p % kWave)) - 1ull));
+  };
+  auto seeds_distinct = [&](int64_t fb, int64_t ns, uint32_t f0) {
+    if (ns == 0) return true;
+    const int64_t q = fb + ns - 1;
+    return ((words[q / kWave].first >> (int)(q % kWave)) & 1ull) &&
+           rank_first((uint32_t)q) - f0 == (uint32_t)(ns - 1);
+  };
+  if (blockIdx.x == 0) {
+    for (int64_t b = threadIdx.x; b <= cols.B; b += kBlock) {
+      const int64_t s_lo = b < cols.B ? cols.lo(b) : n;
+      uint32_t f, e;
+      ranks(s_lo * width, &f, &e);
+      out.frontier_ptr[b] = f;
+      out.edge_ptr[b] = e;
+      store_for_host(out.mirror + b, f);
+      store_for_host(out.mirror + (cols.B + 1) + b, e);
+      if (b < cols.B) {
+        const int64_t s_hi = cols.hi(b);
+        if (out.block_indptr) {
+          uint32_t f1, e1;
+          ranks(s_hi * width, &f1, &e1);
+          out.block_indptr[s_hi + b] = e1 - e;  // the last offset of the block
+        }
+        store_for_host(out.mirror + 2 * (cols.B + 1) + b,
+                       seeds_distinct(s_lo * width, s_hi - s_lo, f) ? 1 : 0);
+      } else {
+        store_for_host(out.mirror + 3 * cols.B + 2, *wide);
+      }
+    }
+  }
+  const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
+  if (p0 >= N) return;
+  const TileBatches batches =
+      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
+  int64_t b = -1, s_lo = 0, ns = 0, fb = 0;
+  uint32_t f0 = 0, e0 = 0;
+  bool distinct = true;
+#pragma unroll
+  for (int i = 0; i < kLayerTile / kBlock; ++i) {
+    const int64_t p = p0 + i * kBlock + threadIdx.x;
+    if (p >= N) break;
+    const int64_t b_now = batches.of(cols, width, p);
+    if (b_now != b) {
+      b = b_now;
+      s_lo = cols.lo(b);
+      ns = cols.hi(b) - s_lo;
+      fb = s_lo * width;
+      ranks(fb, &f0, &e0);
+      distinct = seeds_distinct(fb, ns, f0);
+    }
+    const LayerWord w = words[p / kWave];
+    const int bit = (int)(p % kWave);
+    const uint64_t below = (1ull << bit) - 1ull;
+    const uint2 t = before[blockIdx.x];
+    if ((w.first >> bit) & 1ull)
+      out.frontier[t.x + w.first_before + (uint32_t)__popcll(w.first & below)] =
+          (int64_t)(keys[p] - (uint32_t)b * stride);
+    const uint32_t local = (uint32_t)(p - fb);
+    if (local < (uint32_t)ns) continue;
+    const uint32_t slot = local - (uint32_t)ns;
+    const uint32_t c = slot / (uint32_t)fanout;  // the column, counted in its batch
+    const uint32_t e = t.y + w.edge_before + (uint32_t)__popcll(w.edge & below);
+    if (out.block_indptr && slot - c * (uint32_t)fanout == 0)
+      out.block_indptr[s_lo + c + b] = e - e0;
+    if ((w.edge >> bit) & 1ull) {
+      out.row[e] = rank_first(first[p]) - f0;
+      out.col[e] = distinct ? c : rank_first(first[fb + c]) - f0;
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void layer_clear_kernel(uint64_t* table, int64_t slots,
+                                                             int32_t* wide) {
+  int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i == 0) *wide = 0;
+  for (; i < slots; i += (int64_t)gridDim.x * kBlock) table[i] = kEmptySlot;
+}
+
+// weighted.hip: draws of a weighted layer into fanout places per column, the number
+// of columns read from the device.
+int launch_weighted_places(const int64_t* indptr, int64_t num_cols, const int64_t* indices,
+                           const int64_t* cdf, const int64_t* column_ids, const int64_t* num_dev,
+                           int64_t bound, int64_t fanout, int replace, PhiloxKey key,
+                           int64_t* out_rows, hipStream_t s);
+
+}  // namespace gs
+
+extern "C" {
+
+int64_t gs_layer_max_positions(void) { return (int64_t)gs::kLayerMaxTiles * gs::kLayerTile; }
+
+size_t gs_layer_workspace_bytes(int64_t max_positions, int weighted) {
+  if (max_positions < 0 || max_positions > gs_layer_max_positions()) return 0;
+  return gs::carve_layer(nullptr, max_positions, weighted).total;
+}
+
+int gs_layer_begin(int64_t max_positions, int weighted, void* workspace, size_t workspace_bytes,
+                   gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(max_positions >= 0 && max_positions <= gs_layer_max_positions(),
+             "layer_begin: %lld positions", (long long)max_positions);
+  const LayerWs w = carve_layer(workspace, max_positions, weighted);
+  if (workspace == nullptr || workspace_bytes < w.total) {
+    set_error("layer workspace too small: %zu < %zu", workspace_bytes, w.total);
+    return GS_ERR_WORKSPACE;
+  }
+  int64_t blocks = ceil_div(w.slots, kBlock * 4);
+  if (blocks > 2048) blocks = 2048;
+  hipStream_t s = as_stream(stream);
+  GS_LAUNCH("layer_clear", s,
+            layer_clear_kernel<<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(w.table, w.slots,
+                                                                               w.wide));
+  return GS_OK;
+}
+
+int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indices,
+                    const int32_t* indices32, const int64_t* cdf, int64_t id_stride,
+                    const int64_t* columns, int64_t num_columns, const int64_t* col_ptr,
+                    int64_t num_batches, int64_t fanout, int replace, uint64_t seed,
+                    uint64_t call_id, int64_t* out_frontier, int64_t* out_frontier_ptr,
+                    int64_t* out_row, int64_t* out_col, int64_t* out_edge_ptr,
+                    int64_t* out_block_indptr, int64_t* mirror,
+                    int64_t max_positions, void* workspace, size_t workspace_bytes,
+                    gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(num_cols >= 0 && num_columns >= 1, "sample_layer: no columns");
+  GS_REQUIRE(num_batches >= 1 && (col_ptr || num_batches == 1),
+             "sample_layer: %lld batches need col_ptr", (long long)num_batches);
+  GS_REQUIRE(fanout >= 1 && fanout < kWave, "sample_layer: fanout %lld", (long long)fanout);
+  GS_REQUIRE(id_stride >= 1 && id_stride >= num_cols &&
+                 num_batches <= (int64_t)0xFFFFFFFEll / id_stride,
+             "sample_layer: %lld batches of ids below %lld", (long long)num_batches,
+             (long long)id_stride);
+  const int64_t positions = num_columns * (fanout + 1);
+  GS_REQUIRE(positions <= max_positions && max_positions <= gs_layer_max_positions(),
+             "sample_layer: %lld positions", (long long)positions);
+  GS_REQUIRE(indptr && columns && out_frontier && out_frontier_ptr && out_row && out_col &&
+                 out_edge_ptr && mirror,
+             "sample_layer: null pointer");
+  const LayerWs w = carve_layer(workspace, max_positions, cdf != nullptr);
+  if (workspace == nullptr || workspace_bytes < w.total) {
+    set_error("layer workspace too small: %zu < %zu", workspace_bytes, w.total);
+    return GS_ERR_WORKSPACE;
+  }
+  const int64_t slots = layer_table_slots(positions);  // of the table, what this layer uses
+  hipStream_t s = as_stream(stream);
+  const PhiloxKey key = make_key(seed, call_id);
+  const LayerColumns cols{columns, col_ptr, num_batches, num_columns};
+  const int cols_per_wave = kWave / ((int)fanout + 1);
+  const unsigned pick_grid =
+      (unsigned)ceil_div(num_columns, (kPickThreads / kWave) * cols_per_wave);
+  const unsigned tile_grid = (unsigned)ceil_div(positions, kLayerTile);
+  if (cdf) {
+    int rc = launch_weighted_places(indptr, num_cols, indices, cdf, columns,
+                                    col_ptr ? col_ptr + num_batches : nullptr, num_columns, fanout,
+                                    replace, key, w.picked, s);
+    if (rc != GS_OK) return rc;
+  }
+#define GS_PICK(T, IDS)                                                                       \
+  GS_LAUNCH("layer_pick", s,                                                                  \
+            layer_pick_kernel<T><<<dim3(pick_grid), dim3(kPickThreads), 0, s>>>(              \
+                indptr, num_cols, IDS, cols, (int)fanout, cols_per_wave, replace, key,        \
+                (uint32_t)id_stride, cdf ? w.picked : nullptr, w.table, (uint32_t)(slots - 1), \
+                w.slot, w.wide))
+  if (indices32) GS_PICK(int32_t, indices32);
+  else GS_PICK(int64_t, indices);
+#undef GS_PICK
+  GS_LAUNCH("layer_flag", s,
+            layer_flag_kernel<<<dim3(tile_grid), dim3(kBlock), 0, s>>>(
+                cols, (int)fanout, w.table, w.slot, w.first, w.key, w.words, w.tile_cnt));
+  const LayerOut out{out_frontier, out_frontier_ptr, out_row, out_col,
+                     out_edge_ptr, out_block_indptr, mirror};
+  GS_LAUNCH("layer_label", s,
+            layer_label_kernel<<<dim3(tile_grid), dim3(kBlock), 0, s>>>(
+                cols, (int)fanout, (uint32_t)id_stride, w.first, w.key, w.words, w.tile_cnt,
+                w.table, slots, w.wide, out));
+  return GS_OK;
+}
+
+}  // extern "C"

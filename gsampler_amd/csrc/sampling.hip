@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kBlock) void sample_uniform_packed_kernel(
   }
   out_indices[out_start + lane] = v;
   if (kProbe & kProbeOneStore) return;
-  out_select[out_start + lane] = p;
+  if (out_select) out_select[out_start + lane] = p;
   if (out_coo_col) out_coo_col[out_start + lane] = col_label;
 }
 
@@ -252,8 +252,7 @@ static int sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const Id
              "sample_uniform: Floyd sampling needs fanout <= 64, got %lld",
              (long long)fanout);
   if (num_items == 0 || fanout == 0) return GS_OK;
-  GS_REQUIRE(indptr && sub_indptr && out_indices && out_select,
-             "sample_uniform: null pointer");
+  GS_REQUIRE(indptr && sub_indptr && out_indices, "sample_uniform: null pointer");
   GS_REQUIRE(column_ids != nullptr || num_items <= num_cols,
              "sample_uniform: %lld items but the matrix has %lld columns",
              (long long)num_items, (long long)num_cols);
@@ -272,6 +271,8 @@ static int sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const Id
                   col_span));
     return GS_OK;
   }
+  // (the reservoir keeps its slots there)
+  GS_REQUIRE(out_select, "sample_uniform: this algorithm and fanout need out_select");
 #define GS_SAMPLE_ARGS                                                          \
   indptr, num_cols, indices, column_ids, num_items, fanout, replace, key, sub_indptr, \
       out_coo_col, out_indices, out_select, labels, col_span, s

@@ -1011,7 +1011,8 @@ __global__ __launch_bounds__(kOffsetsThreads) void unique_offsets_kernel(
     const int64_t* __restrict__ flat_ptr, int64_t B, int64_t N, int64_t groups,
     const int64_t* __restrict__ group_cnt, int64_t* group_off,
     const RankWord* __restrict__ words, int64_t* __restrict__ unique_ptr,
-    int64_t* __restrict__ unique_ptr_ws, int64_t* unique_ptr_mirror) {
+    int64_t* __restrict__ unique_ptr_ws, int64_t* unique_ptr_mirror,
+    const BatchInfo* __restrict__ batch, int64_t* distinct_mirror) {
   __shared__ int64_t smem[kOffsetsThreads / kWave + 1];
   int64_t carry = 0;
   constexpr int kPer = 8;
@@ -1034,16 +1035,26 @@ __global__ __launch_bounds__(kOffsetsThreads) void unique_offsets_kernel(
   }
   if (threadIdx.x == 0) group_off[groups] = carry;
   __syncthreads();
+  auto rank_at = [&](int64_t p, bool* is_first) {  // p < N
+    const RankWord w = words[p / kWave];
+    // written above by other threads of this work-group: read past the
+    // compute unit's own cache
+    const int64_t off = __hip_atomic_load(group_off + p / kGroup, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+    *is_first = (w.bits >> (int)(p % kWave)) & 1ull;
+    return off + (int64_t)w.before + __popcll(w.bits & ((1ull << (int)(p % kWave)) - 1ull));
+  };
   for (int64_t b = threadIdx.x; b <= B; b += kOffsetsThreads) {
     const int64_t p = flat_ptr[b];
-    int64_t r = carry;
-    if (p < N) {
-      const RankWord w = words[p / kWave];
-      // written above by other threads of this work-group: read past the
-      // compute unit's own cache
-      const int64_t off = __hip_atomic_load(group_off + p / kGroup, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT);
-      r = off + w.before + __popcll(w.bits & ((1ull << (int)(p % kWave)) - 1ull));
+    bool first;
+    const int64_t r = p < N ? rank_at(p, &first) : carry;
+    if (distinct_mirror && b < B) {
+      // the last seed of distinct seeds is a first occurrence with as many
+      // first occurrences of its batch before it as there are other seeds
+      const int64_t ns = batch[b].ns;
+      int64_t ok = 1;
+      if (ns > 0) ok = rank_at(p + ns - 1, &first) - r == ns - 1 && first;
+      store_for_host(distinct_mirror + b, ok);
     }
     unique_ptr[b] = r;
     unique_ptr_ws[b] = r;
@@ -1328,9 +1339,11 @@ __global__ __launch_bounds__(kBlock) void unique_fill_relabel_kernel(
 
 // No keys at all: every batch is empty.
 __global__ __launch_bounds__(kBlock) void unique_empty_kernel(
-    int64_t* __restrict__ unique_ptr, int64_t* unique_ptr_mirror, int64_t n) {
+    int64_t* __restrict__ unique_ptr, int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+    int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
+  if (distinct_mirror && i < n - 1) store_for_host(distinct_mirror + i, 1);
   unique_ptr[i] = 0;
   if (unique_ptr_mirror) store_for_host(unique_ptr_mirror + i, 0);
 }
@@ -1377,6 +1390,17 @@ int gs_unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
                     int64_t num_batches, int64_t* unique_ptr,
                     int64_t* unique_ptr_mirror, void* workspace,
                     size_t workspace_bytes, gs_stream_t stream) {
+  return gs_unique_count_distinct(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+                                  num_batches, unique_ptr, unique_ptr_mirror, nullptr, workspace,
+                                  workspace_bytes, stream);
+}
+
+int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
+                             int64_t num_seeds, const int64_t* rows,
+                             const int64_t* rows_ptr, int64_t num_rows_keys,
+                             int64_t num_batches, int64_t* unique_ptr,
+                             int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+                             void* workspace, size_t workspace_bytes, gs_stream_t stream) {
   using namespace gs;
   const int64_t S = num_seeds, E = num_rows_keys, B = num_batches;
   int rc = check_unique_args(seeds, seeds_ptr, S, rows, rows_ptr, E, B);
@@ -1391,7 +1415,8 @@ int gs_unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
     GS_LAUNCH("unique_plan", s,
               unique_empty_kernel<<<dim3((unsigned)ceil_div(B + 1, kBlock)),
                                     dim3(kBlock), 0, s>>>(unique_ptr,
-                                                          unique_ptr_mirror, B + 1));
+                                                          unique_ptr_mirror, distinct_mirror,
+                                                          B + 1));
     return GS_OK;
   }
   const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
@@ -1433,7 +1458,7 @@ int gs_unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
   GS_LAUNCH("unique_offsets", s,
             unique_offsets_kernel<<<dim3(1), dim3(kOffsetsThreads), 0, s>>>(
                 w.flat_ptr, B, N, w.groups, w.group_cnt, w.group_off, w.words,
-                unique_ptr, w.unique_ptr, unique_ptr_mirror));
+                unique_ptr, w.unique_ptr, unique_ptr_mirror, w.batch, distinct_mirror));
   return GS_OK;
 }
 

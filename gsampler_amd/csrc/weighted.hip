@@ -484,9 +484,9 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
     int replace, PhiloxKey key, const int64_t* __restrict__ sub_indptr,
     int64_t* __restrict__ out_coo_col, int64_t* __restrict__ out_indices,
     int64_t* __restrict__ out_select, ColumnLabels labels,
-    const int64_t* __restrict__ col_span) {
+    const int64_t* __restrict__ col_span, const int64_t* __restrict__ num_dev) {
   const int64_t item = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (item >= num_items) return;
+  if (item >= (num_dev ? *num_dev : num_items)) return;
   // (asked for here, so that its loads travel with the ones below)
   const int64_t col_label =
       out_coo_col ? labels.of_near(item, item - lane_id()) : item;
@@ -495,7 +495,8 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
   int64_t in_start;
   const int64_t deg = column_span(col_span, column_ids, indptr, num_cols, item, &in_start);
   if (deg == 0) return;
-  const int64_t out_start = sub_indptr[item];
+  // (without offsets every column has `fanout` places of its own)
+  const int64_t out_start = sub_indptr ? sub_indptr[item] : item * fanout;
   const uint64_t* col = cdf + in_start;  // col[j], 1 <= j <= deg: entry of item j - 1
   // A column's shares add up to 2^cb - 1, or to 0 when it has no positive weight.
   // Which of the two is in the column's last entry, one more random line that a
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
     if (!hold) {
       const int64_t p = in_start + off;
       out_indices[out_start + taken] = row_of(off, entry);
-      out_select[out_start + taken] = p;
+      if (out_select) out_select[out_start + taken] = p;
       if (out_coo_col) out_coo_col[out_start + taken] = col_label;
     }
 #pragma unroll
@@ -609,9 +610,11 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
     for (int i = 0; i < KMAX; ++i)
       if (i < taken) out_indices[out_start + i] = (int64_t)held_row[i];
   }
+  if (out_select) {
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i)
-    if (i < taken) out_select[out_start + i] = in_start + held[i];
+    for (int i = 0; i < KMAX; ++i)
+      if (i < taken) out_select[out_start + i] = in_start + held[i];
+  }
   if (out_coo_col) {
 #pragma unroll
     for (int i = 0; i < KMAX; ++i)
@@ -626,14 +629,50 @@ static int launch_weighted_cdf(const int64_t* indptr, int64_t num_cols,
                                int fanout, int replace, PhiloxKey key,
                                const int64_t* sub_indptr, int64_t* out_coo_col,
                                int64_t* out_indices, int64_t* out_select,
-                               ColumnLabels labels, const int64_t* col_span, hipStream_t s) {
+                               ColumnLabels labels, const int64_t* col_span,
+                               const int64_t* num_dev, hipStream_t s) {
   GS_LAUNCH("sample_weighted_cdf", s,
             sample_weighted_cdf_kernel<KMAX><<<dim3((unsigned)ceil_div(num_items, kBlock)),
                                                dim3(kBlock), 0, s>>>(
                 indptr, num_cols, indices, (const uint64_t*)cdf, column_ids, num_items,
                 fanout, replace, key, sub_indptr, out_coo_col, out_indices, out_select, labels,
-                col_span));
+                col_span, num_dev));
   return GS_OK;
+}
+
+// (every slot of the register arrays costs instructions in every draw whether it is
+// used or not: the common fan-outs get arrays of their own size)
+static int launch_weighted_cdf_any(const int64_t* indptr, int64_t num_cols,
+                                   const int64_t* indices, const int64_t* cdf,
+                                   const int64_t* column_ids, int64_t num_items, int fanout,
+                                   int replace, PhiloxKey key, const int64_t* sub_indptr,
+                                   int64_t* out_coo_col, int64_t* out_indices,
+                                   int64_t* out_select, ColumnLabels labels,
+                                   const int64_t* col_span, const int64_t* num_dev,
+                                   hipStream_t s) {
+#define GS_CDF_ARGS                                                              \
+  indptr, num_cols, indices, cdf, column_ids, num_items, fanout, replace, key, sub_indptr, \
+      out_coo_col, out_indices, out_select, labels, col_span, num_dev, s
+  if (fanout <= 4) return launch_weighted_cdf<4>(GS_CDF_ARGS);
+  if (fanout == 5) return launch_weighted_cdf<5>(GS_CDF_ARGS);
+  if (fanout <= 8) return launch_weighted_cdf<8>(GS_CDF_ARGS);
+  if (fanout <= 10) return launch_weighted_cdf<10>(GS_CDF_ARGS);
+  if (fanout <= 12) return launch_weighted_cdf<12>(GS_CDF_ARGS);
+  if (fanout <= 15) return launch_weighted_cdf<15>(GS_CDF_ARGS);
+  if (fanout <= 16) return launch_weighted_cdf<16>(GS_CDF_ARGS);
+  if (fanout <= 24) return launch_weighted_cdf<24>(GS_CDF_ARGS);
+  if (fanout <= 32) return launch_weighted_cdf<32>(GS_CDF_ARGS);
+  return launch_weighted_cdf<64>(GS_CDF_ARGS);
+#undef GS_CDF_ARGS
+}
+
+int launch_weighted_places(const int64_t* indptr, int64_t num_cols, const int64_t* indices,
+                           const int64_t* cdf, const int64_t* column_ids, const int64_t* num_dev,
+                           int64_t bound, int64_t fanout, int replace, PhiloxKey key,
+                           int64_t* out_rows, hipStream_t s) {
+  return launch_weighted_cdf_any(indptr, num_cols, indices, cdf, column_ids, bound, (int)fanout,
+                                 replace, key, nullptr, nullptr, out_rows, nullptr,
+                                 ColumnLabels{nullptr, 0}, nullptr, num_dev, s);
 }
 
 // ------------------------------------------------------------ list sampling
@@ -1235,7 +1274,7 @@ int gs_csc_col_sample_weighted_fill(
   const ColumnLabels labels{col_batch_ptr, num_col_batches};
   GS_REQUIRE(fanout >= 0, "sample_weighted: negative fanout %lld", (long long)fanout);
   if (num_items == 0 || fanout == 0) return GS_OK;
-  GS_REQUIRE(indptr && (probs || cdf) && sub_indptr && out_indices && out_select,
+  GS_REQUIRE(indptr && (probs || cdf) && sub_indptr && out_indices && (out_select || cdf),
              "sample_weighted: null pointer");
   GS_REQUIRE(column_ids != nullptr || num_items <= num_cols,
              "sample_weighted: %lld items but the matrix has %lld columns",
@@ -1247,23 +1286,9 @@ int gs_csc_col_sample_weighted_fill(
                "sample_weighted: fanout %lld > %d is not supported without replacement",
                (long long)fanout, kMaxCdfFanout);
     GS_REQUIRE(fanout <= INT32_MAX, "sample_weighted: fanout too large");
-#define GS_CDF_ARGS                                                              \
-  indptr, num_cols, indices, cdf, column_ids, num_items, (int)fanout, replace, \
-      key, sub_indptr, out_coo_col, out_indices, out_select, labels, col_span, s
-    // (every slot of the register arrays costs instructions in every draw whether it is
-    // used or not: the common fan-outs get arrays of their own size)
-    if (fanout <= 4) return launch_weighted_cdf<4>(GS_CDF_ARGS);
-    if (fanout == 5) return launch_weighted_cdf<5>(GS_CDF_ARGS);
-    if (fanout <= 8) return launch_weighted_cdf<8>(GS_CDF_ARGS);
-    if (fanout <= 10) return launch_weighted_cdf<10>(GS_CDF_ARGS);
-    if (fanout <= 12) return launch_weighted_cdf<12>(GS_CDF_ARGS);
-    if (fanout <= 15) return launch_weighted_cdf<15>(GS_CDF_ARGS);
-    if (fanout <= 16) return launch_weighted_cdf<16>(GS_CDF_ARGS);
-    if (fanout <= 24) return launch_weighted_cdf<24>(GS_CDF_ARGS);
-    if (fanout <= 32) return launch_weighted_cdf<32>(GS_CDF_ARGS);
-    return launch_weighted_cdf<64>(GS_CDF_ARGS);
-#undef GS_CDF_ARGS
-    return GS_OK;
+    return launch_weighted_cdf_any(indptr, num_cols, indices, cdf, column_ids, num_items,
+                                   (int)fanout, replace, key, sub_indptr, out_coo_col, out_indices,
+                                   out_select, labels, col_span, nullptr, s);
   }
   if (replace) {
     GS_REQUIRE(cdf_scratch, "sample_weighted: sampling with replacement needs the CDF scratch");

@@ -9,6 +9,7 @@ the reference's python/gs/jit/module.py:191-259."""
 from typing import Any, List, Sequence, Tuple
 
 import torch
+from torch import fx
 from torch.fx import PH
 from torch.utils import _pytree as pytree
 
@@ -61,6 +62,9 @@ class compile:  # noqa: N801 -- the reference's public name
         self._format_select = format_select
         self.compact = bool(must_compact) and not self.use_batchmatrix
         self.try_compact = bool(try_compact)
+        # where the run-time inputs that are matrix data come from: (matrix, which dict, key)
+        self._data_keys = [(i, j, key) for i, parts in enumerate(matrix_parts(args, self.kinds)[1])
+                           for j, part in enumerate(parts) for key in part]
         self.gm = self._build(args, self.compact)
         self.compact_search_ms = None
         if self.try_compact and not self.compact and not self.use_batchmatrix:
@@ -69,6 +73,7 @@ class compile:  # noqa: N801 -- the reference's public name
             self.compact_search_ms = (plain_ms, compact_ms)
             if compact_ms < plain_ms:
                 self.gm, self.compact = other, True
+        self._run = self._executable(self.gm)
 
     def _time(self, gm, args, runs=3):
         """Milliseconds per call of one variant on the example arguments."""
@@ -139,10 +144,35 @@ class compile:  # noqa: N801 -- the reference's public name
         return gm
 
     # -------------------------------------------------------------------- run
+    def _executable(self, gm):
+        """What a call runs: a copy of the operator graph whose sampling layers are
+        chained into one operator and whose generated code takes flat inputs and
+        builds the result in place (the pytree machinery of a traced module costs
+        more than the operators of a small sampler).  None when the graph's inputs
+        or result have no such form: the module itself is called then."""
+        codegen = gm.graph._codegen
+        info = getattr(codegen, "pytree_info", None)
+        if info is None:
+            return None
+        graph, copied = fx.Graph(), {}
+        flat = graph.graph_copy(gm.graph, copied)
+        inputs = [n for n in graph.nodes if n.op == "placeholder"]
+        if len(inputs) != 2 + len(self._data_keys):
+            return None
+        try:
+            graph.output(pytree.tree_unflatten(list(flat), info.out_spec)
+                         if info.out_spec is not None else flat)
+            run = passes.chain_layers(fx.GraphModule(gm, graph))
+        except (TypeError, ValueError):
+            return None
+        return run.forward
+
     def __call__(self, *args):
         graphs, data = matrix_parts(args, self.kinds)
         # matrix arguments are rebuilt inside the graph; their slots only keep
         # the positions of the other run-time inputs
         passthrough = tuple(None if k in (MATRIX, BATCH_MATRIX, STATIC) else a
                             for a, k in zip(args, self.kinds))
+        if self._run is not None:
+            return self._run(passthrough, graphs, *(data[i][j][key] for i, j, key in self._data_keys))
         return self.gm(passthrough, graphs, data)

@@ -25,6 +25,9 @@ hoisting of tensor constants.  Operator rewrites (observable in
                                                   -> _CAPI_SlicedESquareSum,
                                                      _CAPI_ColRowSlicing on the
                                                      parent matrix
+  chain_layers                  layers of slice + sample -> relabel
+                                                  -> _CAPI_SampleLayers,
+                                                     _CAPI_BatchSampleLayers
   select_formats                deterministic on_format / output_format choice
 """
 import operator
@@ -565,6 +568,97 @@ def sink_block_construction(gm: fx.GraphModule) -> fx.GraphModule:
     for n in [n for n in gm.graph.nodes if n in moving]:
         output.prepend(n)
     return _finish(gm)
+
+
+def _is_empty_constant(gm: fx.GraphModule, node) -> bool:
+    """The null tensor that stands for "no id mapping"."""
+    return (isinstance(node, fx.Node) and node.op == "get_attr"
+            and getattr(getattr(gm, node.target, None), "numel", lambda: -1)() == 0)
+
+
+def chain_layers(gm: fx.GraphModule) -> fx.GraphModule:
+    """Layer after layer of  slice + sample -> relabel,  each layer's frontier the
+    next one's seeds and the sampled matrix and its edge index used for nothing
+    else, becomes one operator call:
+        _CAPI_SlicingSampling[Probs] -> _CAPI_GraphRelabel          (one mini-batch)
+            => _CAPI_SampleLayers(seeds, fanouts, replace, weights)
+        _CAPI_BatchFusedSlicingSampling[Probs] -> _CAPI_BatchBlocks  (a super-batch)
+            => _CAPI_BatchSampleLayers(seeds, ptr, fanouts, replace, weights)
+    The operator draws the same samples.  Run on the executed copy of the graph:
+    the operator graph that a compiled sampler shows keeps its layers."""
+    single = {"_CAPI_SlicingSampling": (2, None, 3, 4, 5), "_CAPI_SlicingSamplingProbs": (2, 3, 4, 5, 6)}
+    batch = {"_CAPI_BatchFusedSlicingSampling": (1, None, 3, 4), "_CAPI_BatchFusedSlicingSamplingProbs": (1, 3, 4, 5)}
+    order = {n: i for i, n in enumerate(gm.graph.nodes)}
+    draws = [n for n in gm.graph.nodes if _draws_random_numbers(n)]
+
+    def layer_of(node):
+        """(matrix, seeds, ptr, weights, fanout, replace, relabel) of one layer, or None."""
+        if node.op != "call_method" or (node.target not in single and node.target not in batch):
+            return None
+        is_batch = node.target in batch
+        at = (batch if is_batch else single)[node.target]
+        args = node.args
+        if not is_batch and (args[1] != 1 or args[at[4]] != _CSC):
+            return None
+        sampled = _getitem_users(node, 0)
+        if len(sampled) != 1 or len(node.users) != 1 or len(sampled[0].users) != 1:
+            return None
+        relabel = next(iter(sampled[0].users))
+        if not _is_method(relabel, "_CAPI_BatchBlocks" if is_batch else "_CAPI_GraphRelabel"):
+            return None
+        seeds, fanout, replace = args[at[0]], args[at[2]], args[at[3]]
+        if (relabel.args[0] is not sampled[0] or relabel.args[1] is not seeds
+                or not _is_empty_constant(gm, relabel.args[2])
+                or type(fanout) is not int or type(replace) is not bool):
+            return None
+        return (args[0], seeds, args[2] if is_batch else None,
+                args[at[1]] if at[1] is not None else None, fanout, replace, relabel)
+
+    chains, current = [], []
+    for node in draws:
+        layer = layer_of(node)
+        if layer is None:
+            current = []
+            continue
+        if current:
+            (graph, _, _, weights, _, replace, prev) = current[-1][1]
+            follows = (layer[0] is graph and layer[3] is weights and layer[5] == replace
+                       and (layer[2] is None) == (current[-1][1][2] is None))
+            if follows and layer[2] is None:
+                follows = layer[1] in _getitem_users(prev, 0)
+            elif follows:
+                follows = (_is_method(layer[1], "frontier") and layer[1].args[0] is prev
+                           and _is_method(layer[2], "frontier_ptr") and layer[2].args[0] is prev)
+            if follows:
+                current.append((node, layer))
+                continue
+        current = [(node, layer)]
+        chains.append(current)
+    for chain in chains:
+        first, (graph, seeds, ptr, weights, _, replace, _) = chain[0]
+        if any(a is not None and order[a] > order[first] for a in (graph, seeds, ptr, weights)):
+            continue
+        fanouts = [layer[4] for _, layer in chain]
+        with gm.graph.inserting_before(first):
+            if ptr is None:
+                out = gm.graph.call_method("_CAPI_SampleLayers",
+                                           args=(graph, seeds, fanouts, replace, weights))
+            else:
+                out = gm.graph.call_method("_CAPI_BatchSampleLayers",
+                                           args=(graph, seeds, ptr, fanouts, replace, weights))
+            for i, (_, layer) in enumerate(chain):
+                relabel = layer[6]
+                if ptr is not None:
+                    blocks = gm.graph.call_function(operator.getitem, args=(out, i))
+                    relabel.replace_all_uses_with(blocks)
+                    continue
+                for j in range(4):
+                    users = _getitem_users(relabel, j)
+                    if users:
+                        item = gm.graph.call_function(operator.getitem, args=(out, 4 * i + j))
+                        for u in users:
+                            u.replace_all_uses_with(item)
+    return dce(gm)
 
 
 # --------------------------------------------------------------- formats

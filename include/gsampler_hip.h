@@ -87,11 +87,17 @@ int gs_profile_get(int index, char* name, size_t name_bytes, long long* calls,
  * dst[0..n) = src[0..n).  dst may be pinned host memory that the device can
  * address: counts and batch pointer arrays that the host needs (to size the next
  * launch, to split results per batch) are sent this way, by a kernel in stream
- * order whose completion an event marks, instead of a memcpy call per array
- * (the reference reads them with blocking copies, e.g.
- * src/cuda/slicing.cu:146, src/cuda/batch/batch_split.cu:107-119).
+ * order, instead of a memcpy call per array (the reference reads them with
+ * blocking copies, e.g. src/cuda/slicing.cu:146,
+ * src/cuda/batch/batch_split.cu:107-119).  The values are written through to the
+ * host as they are stored: a host that marked the words first may look at them
+ * while the stream is still running.
+ * gs_take_i64: out[i] = src[index[i]], also stored to out_mirror[i] (nullable) in
+ * that way.
  * ---------------------------------------------------------------------- */
 int gs_copy_i64(const int64_t* src, int64_t n, int64_t* dst, gs_stream_t stream);
+int gs_take_i64(const int64_t* src, const int64_t* index, int64_t n, int64_t* out,
+                int64_t* out_mirror, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Exclusive prefix sum of n int64 values, in place allowed (in == out).
@@ -398,6 +404,56 @@ int gs_unique_fill_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
                            const int64_t* col_indptr, int64_t* out_row, int64_t* out_col,
                            int out_col_prefilled, void* workspace, size_t workspace_bytes,
                            gs_stream_t stream);
+
+/* ------------------------------------------------------------------------
+ * gs_unique_count that also reports, per batch, whether its seeds are pairwise
+ * different (1 or 0) to distinct_mirror[num_batches] (pinned host memory): what
+ * gs_batch_seeds_distinct finds out from the frontier, before that is written.
+ * ---------------------------------------------------------------------- */
+int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr, int64_t num_seeds,
+                             const int64_t* rows, const int64_t* rows_ptr,
+                             int64_t num_rows_keys, int64_t num_batches, int64_t* unique_ptr,
+                             int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+                             void* workspace, size_t workspace_bytes, gs_stream_t stream);
+
+/* ------------------------------------------------------------------------
+ * One whole layer of node-wise sampling in three launches, for small layers:
+ * column slice + sampling + unique + relabel, i.e. gs_csc_col_count, a sampler
+ * fill and gs_unique_count / gs_unique_fill_relabel with the same picks, frontier
+ * and labels, but without a value that the host has to wait for in between -- the
+ * number of columns is read from the device, and the layers of a sampler can be
+ * queued one behind the other (examples/graphsage/graphsage.py:7-17).
+ *   columns[num_columns], col_ptr[num_batches + 1]  the layer's columns and their
+ *       batches; with col_ptr, num_columns is a bound and col_ptr[num_batches] the
+ *       number.  A previous layer's out_frontier / out_frontier_ptr fit as they are.
+ *       col_ptr NULL: one batch of num_columns columns.
+ *   indices / indices32   row ids, either width; cdf (nullable): neighbours by
+ *       weight through gs_weight_cdf_build's array, else uniform
+ *   id_stride             exceeds every id (rows and columns); num_batches times it
+ *       stays below 2^32 - 1
+ *   outputs, sized by the bound n = num_columns: out_frontier[n (fanout + 1)],
+ *       out_frontier_ptr[num_batches + 1], out_row / out_col[n fanout] (labels),
+ *       out_edge_ptr[num_batches + 1], out_block_indptr[n + num_batches] (nullable;
+ *       as gs_split_indptr lays it out)
+ *   mirror[3 num_batches + 3]  pinned host memory: frontier_ptr, edge_ptr, per
+ *       batch whether its seeds are distinct, and a word that is not 0 when some
+ *       column is no id below id_stride (the outputs are then not to be used)
+ * fanout in [1, 63]; n (fanout + 1) <= max_positions <= gs_layer_max_positions().
+ * The workspace is prepared once by gs_layer_begin and serves any number of
+ * layers of at most max_positions (and with the same `weighted`) after that.
+ * ---------------------------------------------------------------------- */
+int64_t gs_layer_max_positions(void);
+size_t gs_layer_workspace_bytes(int64_t max_positions, int weighted);
+int gs_layer_begin(int64_t max_positions, int weighted, void* workspace, size_t workspace_bytes,
+                   gs_stream_t stream);
+int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indices,
+                    const int32_t* indices32, const int64_t* cdf, int64_t id_stride,
+                    const int64_t* columns, int64_t num_columns, const int64_t* col_ptr,
+                    int64_t num_batches, int64_t fanout, int replace, uint64_t seed,
+                    uint64_t call_id, int64_t* out_frontier, int64_t* out_frontier_ptr,
+                    int64_t* out_row, int64_t* out_col, int64_t* out_edge_ptr,
+                    int64_t* out_block_indptr, int64_t* mirror, int64_t max_positions,
+                    void* workspace, size_t workspace_bytes, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Column slice of a super-batch with its rows numbered anew: batch b's rows are

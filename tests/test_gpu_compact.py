@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import gsampler_amd as gs
-from conftest import random_csc
+from tests.conftest import random_csc
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -16,7 +16,7 @@ DEV = "cuda:0"
     (63, 40, 6, 0, 2, False),           # batch border inside a rank word
     (4096, 900, 9, 0, 7, False),        # batches of exactly one group, many short columns a run
     (5001, 700, 40, 30000, 4, False),   # columns longer than a run of edges
-    (5001, 3000, 700, 0, 5, True),      # above 2^20 edges: the int32 copy of the ids
+    (5001, 4000, 800, 0, 5, True),      # above 2^20 edges: the int32 copy of the ids
 ])
 def test_rows_numbered_anew(rng, rows, cols, max_deg, hub, batches, narrow):
     indptr, indices = random_csc(rng, cols, rows, max_deg, hub_deg=hub)

@@ -1,0 +1,116 @@
+"""All layers of a node-wise sampler in one call (small layers: three launches each, queued
+without waits) against the layers operator by operator, at sizes where the short path begins,
+ends or has remainders."""
+import numpy as np
+import pytest
+import torch
+
+import gsampler_amd as gs
+from tests.conftest import random_csc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def single(A, seeds, fanouts, replace):
+    out = []
+    for k in fanouts:
+        sub = A[:, seeds]
+        sub = sub.individual_sampling(k, sub.edata["w"] if "w" in A.edata else None, replace)
+        seeds = sub.all_nodes()
+        out.append(sub.to_dgl_block())
+    return seeds, out
+
+
+def batched(A, seeds, ptr, fanouts, replace):
+    out = []
+    for k in fanouts:
+        sub = A[:, seeds::ptr]
+        sub = sub.individual_sampling(k, sub.edata["w"] if "w" in A.edata else None, replace)
+        seeds, ptr = sub.all_nodes()
+        out.append(sub.to_dgl_block())
+    return out
+
+
+def both(func, m, args, layers):
+    compiled = gs.jit.compile(func=func, args=(m, *args))
+    called = [n.target for n in compiled._run.__self__.graph.nodes if n.op == "call_method"]
+    assert sum("SampleLayers" in t for t in called) == 1 and "_CAPI_GraphRelabel" not in called
+    gs.manual_seed(5)
+    got = compiled(m, *args)
+    assert gs.random_state() == (5, layers)
+    gs.manual_seed(5)
+    graph, data = [m._graph], [[m.row_ndata, m.col_ndata, m.edata]]
+    run_time = tuple(a if isinstance(a, torch.Tensor) else None for a in (None, *args))
+    return got, compiled.gm(run_time, graph, data)
+
+
+def same(a, b):
+    assert a.num_src == b.num_src and a.num_dst == b.num_dst
+    assert torch.equal(a.row, b.row) and torch.equal(a.col, b.col)
+    assert torch.equal(a.srcdata["_ID"], b.srcdata["_ID"])
+    for x, y in zip(a.csc(), b.csc()):
+        assert (x is None) == (y is None) and (x is None or torch.equal(x, y))
+
+
+def matrix(rng, nodes, max_deg, hub, weighted):
+    indptr, indices = random_csc(rng, nodes, nodes, max_deg, hub_deg=hub)
+    indices[rng.random(indices.size) < 0.2] = nodes // 3        # a hub on the other side
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    if weighted:
+        m.edata["w"] = torch.from_numpy(rng.random(indices.size).astype(np.float32)).to(DEV)
+    return m
+
+
+@pytest.mark.parametrize("nodes,count,fanouts,replace,weighted", [
+    (50, 1, [1], False, False),
+    (3000, 73, [15, 10, 5], False, False),       # queued layers
+    (3000, 1024, [63], True, False),             # the widest column of the short path
+    (3000, 200, [64, 3], False, False),          # one fanout too many for it, then short again
+    (9000, 5000, [31, 31], False, False),        # second layer above the bound of queued layers
+    (40000, 33000, [40, 2], False, False),       # first layer above the bound of short ones
+    (3000, 65, [10, 5], False, True),
+    (3000, 300, [7, 7], True, True),
+])
+def test_one_batch(rng, nodes, count, fanouts, replace, weighted):
+    m = matrix(rng, nodes, 60, 2500, weighted)
+    seeds = torch.from_numpy(rng.integers(0, nodes, count)).to(DEV)      # some repeat
+    (n0, b0), (n1, b1) = both(single, m, (seeds, fanouts, replace), len(fanouts))
+    assert torch.equal(n0, n1) and len(b0) == len(b1) == len(fanouts)
+    for x, y in zip(b0, b1):
+        same(x, y)
+
+
+@pytest.mark.parametrize("cuts,fanouts,replace,weighted", [
+    ([0, 64], [5], False, False),
+    ([0, 0, 7, 7, 1000, 1001], [15, 10, 5], False, False),       # empty batches, one of one seed
+    ([0, 300, 300, 512], [4, 4], True, False),
+    (list(range(0, 6001, 60)), [15, 10], False, False),          # second layer large
+    ([0, 100, 250], [10, 5], False, True),
+])
+def test_super_batch(rng, cuts, fanouts, replace, weighted):
+    nodes = 7000
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(matrix(rng, nodes, 40, 3000, weighted), False)
+    seeds = torch.cat([torch.from_numpy(rng.permutation(nodes)[:hi - lo])
+                       for lo, hi in zip(cuts, cuts[1:])])
+    if len(cuts) == 4:
+        seeds[3] = seeds[0]                                      # a batch whose seeds repeat
+    ptr = torch.tensor(cuts, device=DEV)
+    got, want = both(batched, bm, (seeds.to(DEV), ptr, fanouts, replace), len(fanouts))
+    for layer, other in zip(got, want):
+        assert layer.totals() == other.totals() and len(layer) == len(other) == len(cuts) - 1
+        for name in ("frontier", "frontier_ptr", "row", "col", "edge_ptr", "indptr", "col_ptr"):
+            assert torch.equal(getattr(layer.batch, name)(), getattr(other.batch, name)()), name
+        for x, y in zip(layer, other):
+            same(x, y)
+
+
+def test_seeds_outside_the_matrix_take_the_other_path(rng):
+    m = matrix(rng, 500, 20, 0, False)
+    seeds = torch.tensor([3, -1, 499, 500, 1 << 40, 7], device=DEV)
+    (n0, b0), (n1, b1) = both(single, m, (seeds, [4, 3], False), 2)
+    assert torch.equal(n0, n1)
+    for x, y in zip(b0, b1):
+        same(x, y)
