@@ -1,12 +1,14 @@
 #!/usr/bin/env python3
 """Builds gsampler_amd/lib/libgs.so: the C++ operator library that registers
 gs_classes.Graph and gs_ops with PyTorch-ROCm and calls the C ABI of
-libgsampler_hip.so (built first by ../Makefile).  Host code only: compiled with
+libgsampler_hip.so (built first by ../Makefile), and gsampler_amd/lib/_gs_python.so,
+the Python binding that fills Block objects.  Host code only: compiled with
 g++ against the torch headers, no device code in this library."""
 import glob
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -51,6 +53,21 @@ def main() -> None:
            "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"]
     print("+ link", out, flush=True)
     subprocess.check_call(cmd)
+
+    # the Python binding of the block hand-off, on top of libgs.so
+    src = os.path.join(HERE, "python", "binding.cpp")
+    obj = os.path.join(BUILD, "binding.o")
+    if (force or not os.path.exists(obj)
+            or os.path.getmtime(obj) <= max(os.path.getmtime(src), newest_hdr)):
+        print("+ g++", os.path.basename(src), flush=True)
+        subprocess.check_call(["g++", *flags, *inc, f"-I{sysconfig.get_paths()['include']}",
+                               "-fvisibility-inlines-hidden", "-c", src, "-o", obj])
+    out = os.path.join(LIB_DIR, "_gs_python.so")
+    print("+ link", out, flush=True)
+    subprocess.check_call(["g++", "-shared", "-o", out, obj, f"-L{LIB_DIR}", "-l:libgs.so",
+                           "-lgsampler_hip", f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10",
+                           "-lc10_hip", "-ltorch_hip", "-ltorch_python", "-L/opt/rocm/lib",
+                           "-lamdhip64", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"])
 
 
 if __name__ == "__main__":

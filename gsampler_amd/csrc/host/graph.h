@@ -11,7 +11,9 @@
 
 #include "abi_call.h"
 
+#include <functional>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -101,6 +103,7 @@ class BlockBatch : public torch::CustomClassHolder {
   BlockViews Block(int64_t b);
   BlockParts Blocks();
   int64_t NumSrcOf(int64_t b);
+  bool grouped(int64_t b) const { return grouped_[(size_t)b] != 0; }  // after Offsets()
   torch::Tensor Frontier() { return frontier; }
   torch::Tensor FrontierPtr() { return frontier_ptr; }
   torch::Tensor Row() { return row; }
@@ -265,14 +268,36 @@ class Graph : public torch::CustomClassHolder {
   std::vector<c10::intrusive_ptr<BlockBatch>> BatchSampleLayers(
       torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
       c10::optional<torch::Tensor> edge_probs);
+  // The same; `done` takes the finished layers one by one where the host would
+  // otherwise only wait for the next one.  Returns the layers it was not called for.
+  using LayerDone = std::function<void(c10::intrusive_ptr<BlockBatch>)>;
+  std::vector<c10::intrusive_ptr<BlockBatch>> BatchSampleLayersWhile(
+      torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
+      c10::optional<torch::Tensor> edge_probs, const LayerDone& done);
 
  private:
   struct Layer;
+  // `idle(layers)` runs while the device works on layer layers.size()
+  using LayersIdle = std::function<void(std::vector<Layer>& layers, size_t complete)>;
   std::vector<Layer> sample_layers(const torch::Tensor& seeds, const torch::Tensor& col_bptr,
                                    const std::vector<int64_t>& fanouts, bool replace,
-                                   const c10::optional<torch::Tensor>& edge_probs, bool blocks);
+                                   const c10::optional<torch::Tensor>& edge_probs, bool blocks,
+                                   const LayersIdle& idle);
   Layer large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr, int64_t fanout,
-                    bool replace, const torch::Tensor& cdf);
+                    bool replace, const torch::Tensor& cdf, const std::function<void()>& idle);
+  // Workspace of the small layers, kept between calls (one per matrix, at most
+  // 2^20 positions, about 40 MB): its table is empty whenever a call has been
+  // queued, so the next call on the same stream starts without clearing it.  A call
+  // takes it out and puts it back; one that finds none (another thread has it, or it
+  // belongs to another stream) makes its own.
+  struct LayerWorkspace {
+    torch::Tensor ws;
+    int64_t positions = 0;
+    bool weighted = false;
+    gs_stream_t stream = nullptr;
+  };
+  LayerWorkspace layer_ws_;
+  std::mutex layer_ws_guard_;
 
   // Unique/relabel state shared by all_nodes() and to_dgl_block(): the
   // frontier is computed once, the relabel pass reuses the hash tables.

@@ -28,7 +28,7 @@ namespace {
 // beyond, hashing into one table in global memory is slower than partitioning the
 // keys first.  And up to which it may be queued on a bound alone, without the host
 // knowing the number of its columns: outputs are sized by the bound.
-constexpr int64_t kSmallPositions = int64_t(1) << 20;
+constexpr int64_t kSmallPositions = int64_t(1) << 19;
 constexpr int64_t kQueuedPositions = int64_t(1) << 19;
 
 // A small layer on its way: outputs in one buffer, cut up when the sizes are in.
@@ -43,7 +43,8 @@ struct Queued {
 
 // One layer on the kernels for large layers; waits for its edge and key counts.
 Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr,
-                                int64_t fanout, bool replace, const torch::Tensor& cdf) {
+                                int64_t fanout, bool replace, const torch::Tensor& cdf,
+                                const std::function<void()>& idle) {
   const Compressed& m = compressed(kCSC);
   const int64_t B = col_bptr.numel() - 1, S = cols.numel();
   Layer l;
@@ -73,6 +74,7 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
                                  cptr(l.frontier_ptr), mptr(frontier), nullptr, cptr(r.indptr),
                                  mptr(l.row), mptr(l.col), prefilled ? 1 : 0, ws.data_ptr(),
                                  ws.numel(), cur_stream()));
+  idle();
   l.e_off = OffsetMirror::values(l.edge_ptr);
   l.f_off = OffsetMirror::values(l.frontier_ptr);
   await_words(distinct, (size_t)B, (hipStream_t)cur_stream());
@@ -86,7 +88,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
                                                const torch::Tensor& col_bptr,
                                                const std::vector<int64_t>& fanouts, bool replace,
                                                const c10::optional<torch::Tensor>& edge_probs,
-                                               bool blocks) {
+                                               bool blocks, const LayersIdle& idle) {
   const Compressed& m = compressed(kCSC);
   const bool weighted = edge_probs.has_value();
   const torch::Tensor cdf = weighted ? weight_cdf_for(edge_probs.value(), kCSC) : torch::Tensor();
@@ -107,8 +109,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
     std::vector<Layer> out(L);
     std::vector<Queued> queued(L);
     const size_t words = (size_t)(3 * B + 3);
-    torch::Tensor ws;
-    int64_t ws_positions = 0;
+    LayerWorkspace lw;
     int64_t* mirrors = nullptr;
     bool retry = false;
     // the layer's columns: exact on the host, or a bound while `known` is false
@@ -155,7 +156,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           ptr = torch::arange(0, 2, device_options(m.indptr).dtype(torch::kInt64)) * n;
           BatchOffsets::trust(ptr, n);
         }
-        l = large_layer(cols, ptr, K, replace, cdf);
+        l = large_layer(cols, ptr, K, replace, cdf, [&] { idle(out, i); });
         mirrors = nullptr;  // it has used the thread's pinned words
         l.cols = cols;
         l.col_bptr = ptr;
@@ -166,16 +167,24 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
         continue;
       }
       const int64_t positions = n * (K + 1);
-      if (ws_positions < positions) {
+      if (!lw.ws.defined()) {
+        std::lock_guard<std::mutex> lock(layer_ws_guard_);
+        if (layer_ws_.ws.defined() && layer_ws_.stream == cur_stream() &&
+            layer_ws_.weighted == weighted)
+          std::swap(lw, layer_ws_);
+      }
+      if (lw.positions < positions) {
         // room for the layers that can be queued behind this one as well
         int64_t most = positions, bound = positions;
         for (size_t j = i + 1; j < L && fits(bound, fanouts[j], kQueuedPositions); ++j) {
           bound *= fanouts[j] + 1;
           most = std::max(most, bound);
         }
-        ws = new_workspace(gs_layer_workspace_bytes(most, weighted ? 1 : 0), m.indptr);
-        ws_positions = most;
-        GS_CALL(gs_layer_begin(most, weighted ? 1 : 0, ws.data_ptr(), (size_t)ws.numel(),
+        lw.ws = new_workspace(gs_layer_workspace_bytes(most, weighted ? 1 : 0), m.indptr);
+        lw.positions = most;
+        lw.weighted = weighted;
+        lw.stream = cur_stream();
+        GS_CALL(gs_layer_begin(most, weighted ? 1 : 0, lw.ws.data_ptr(), (size_t)lw.ws.numel(),
                                cur_stream()));
       }
       if (!mirrors) mirrors = PinnedWords::take(words * L);
@@ -200,8 +209,8 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(cdf), stride, cptr(cols), n,
           cptr(ptr), B, K, replace ? 1 : 0, rs.seed, next_call_id(), base, base + q.at_ptr,
           base + q.at_row, base + q.at_col, base + q.at_edge_ptr,
-          blocks ? base + q.at_indptr : nullptr, mirrors + words * i, ws_positions, ws.data_ptr(),
-          (size_t)ws.numel(), cur_stream()));
+          blocks ? base + q.at_indptr : nullptr, mirrors + words * i, lw.positions, lw.ws.data_ptr(),
+          (size_t)lw.ws.numel(), cur_stream()));
       // the next layer's columns, as far as they are known
       cols = piece_of(q.buffer, 0, positions, false);
       ptr = piece_of(q.buffer, q.at_ptr, B + 1, false);
@@ -215,6 +224,12 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           out[i].cols = out[i - 1].frontier;
           out[i].col_bptr = out[i - 1].frontier_ptr;
         }
+      if (lw.ws.defined()) {
+        std::lock_guard<std::mutex> lock(layer_ws_guard_);
+        if (!layer_ws_.ws.defined() || layer_ws_.stream != lw.stream ||
+            layer_ws_.positions <= lw.positions)
+          std::swap(lw, layer_ws_);
+      }
       for (const Layer& l : out) {
         BatchOffsets::trust(l.frontier_ptr, l.f_off.back());
         BatchOffsets::trust(l.edge_ptr, l.e_off.back());
@@ -250,21 +265,21 @@ std::vector<c10::optional<torch::Tensor>> Graph::SampleLayers(
     }
     return out;
   }
-  for (Layer& l : sample_layers(seeds, {}, fanouts, replace, edge_probs, false))
+  for (Layer& l : sample_layers(seeds, {}, fanouts, replace, edge_probs, false,
+                                [](std::vector<Layer>&, size_t) {}))
     out.insert(out.end(), {l.frontier, l.row, l.col, c10::nullopt});
   return out;
 }
 
-std::vector<c10::intrusive_ptr<BlockBatch>> Graph::BatchSampleLayers(
+std::vector<c10::intrusive_ptr<BlockBatch>> Graph::BatchSampleLayersWhile(
     torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
-    c10::optional<torch::Tensor> edge_probs) {
+    c10::optional<torch::Tensor> edge_probs, const LayerDone& done) {
   check_layers(fanouts, replace, edge_probs.has_value());
   seeds = ids(seeds, "seeds");
   col_bptr = ids(col_bptr, "col_bptr");
   BatchOffsets::check(col_bptr, seeds.numel(), "BatchSampleLayers");
   std::vector<int64_t> c_off = OffsetMirror::values(col_bptr);
-  std::vector<c10::intrusive_ptr<BlockBatch>> out;
-  for (Layer& l : sample_layers(seeds, col_bptr, fanouts, replace, edge_probs, true)) {
+  auto batch_of = [&](Layer& l) {
     auto b = c10::make_intrusive<BlockBatch>();
     b->num_batches = col_bptr.numel() - 1;
     b->num_dst_total = l.cols.numel();
@@ -278,12 +293,26 @@ std::vector<c10::intrusive_ptr<BlockBatch>> Graph::BatchSampleLayers(
     b->sampled_indptr = l.sampled_indptr;
     b->indptr = l.block_indptr;
     std::vector<int64_t> f_off = l.f_off;
-    b->set_host_offsets(std::move(l.f_off), std::move(l.e_off), std::move(c_off),
-                        std::move(l.distinct));
+    b->set_host_offsets(l.f_off, l.e_off, std::move(c_off), l.distinct);
     c_off = std::move(f_off);
-    out.push_back(std::move(b));
-  }
+    return b;
+  };
+  size_t handed = 0;
+  auto idle = [&](std::vector<Layer>& layers, size_t complete) {
+    if (!done) return;
+    for (; handed < complete; ++handed) done(batch_of(layers[handed]));
+  };
+  std::vector<Layer> layers =
+      sample_layers(seeds, col_bptr, fanouts, replace, edge_probs, true, idle);
+  std::vector<c10::intrusive_ptr<BlockBatch>> out;
+  for (; handed < layers.size(); ++handed) out.push_back(batch_of(layers[handed]));
   return out;
+}
+
+std::vector<c10::intrusive_ptr<BlockBatch>> Graph::BatchSampleLayers(
+    torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
+    c10::optional<torch::Tensor> edge_probs) {
+  return BatchSampleLayersWhile(seeds, col_bptr, fanouts, replace, edge_probs, LayerDone());
 }
 
 }  // namespace gs

@@ -35,6 +35,7 @@ from typing import Dict, Iterable, List, Optional
 
 import torch.fx as fx
 
+from .. import _library
 from ..format import _COO, _CSC, _CSR
 
 # Operators that write into a caller-allocated tensor: they have no users in the
@@ -584,6 +585,7 @@ def chain_layers(gm: fx.GraphModule) -> fx.GraphModule:
             => _CAPI_SampleLayers(seeds, fanouts, replace, weights)
         _CAPI_BatchFusedSlicingSampling[Probs] -> _CAPI_BatchBlocks  (a super-batch)
             => _CAPI_BatchSampleLayers(seeds, ptr, fanouts, replace, weights)
+    (both called through the native binding, which makes the block objects).
     The operator draws the same samples.  Run on the executed copy of the graph:
     the operator graph that a compiled sampler shows keeps its layers."""
     single = {"_CAPI_SlicingSampling": (2, None, 3, 4, 5), "_CAPI_SlicingSamplingProbs": (2, 3, 4, 5, 6)}
@@ -641,11 +643,11 @@ def chain_layers(gm: fx.GraphModule) -> fx.GraphModule:
         fanouts = [layer[4] for _, layer in chain]
         with gm.graph.inserting_before(first):
             if ptr is None:
-                out = gm.graph.call_method("_CAPI_SampleLayers",
-                                           args=(graph, seeds, fanouts, replace, weights))
+                out = gm.graph.call_function(_library.native.sample_layers,
+                                             args=(graph, seeds, fanouts, replace, weights))
             else:
-                out = gm.graph.call_method("_CAPI_BatchSampleLayers",
-                                           args=(graph, seeds, ptr, fanouts, replace, weights))
+                out = gm.graph.call_function(_library.native.batch_sample_layers,
+                                             args=(graph, seeds, ptr, fanouts, replace, weights))
             for i, (_, layer) in enumerate(chain):
                 relabel = layer[6]
                 if ptr is not None:

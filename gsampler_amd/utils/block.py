@@ -13,6 +13,8 @@ from typing import Dict, List, Optional
 
 import torch
 
+from .. import _library
+
 
 class Block:
     # A super-batched sampler hands out hundreds of these per step: fixed slots
@@ -99,6 +101,10 @@ def create_block_from_csc(indptr, indices, e_ids, num_src, num_dst) -> Block:
     return block
 
 
+_native = _library.native
+_native.set_block_class(Block)
+
+
 class BlockList(Sequence):
     """The blocks of one layer of a super-batched sampler, one per mini-batch.
 
@@ -109,7 +115,9 @@ class BlockList(Sequence):
     when it is asked for; `materialize()` makes all of them from one call."""
 
     def __init__(self, batch, edata: Optional[Dict[str, torch.Tensor]] = None):
-        self._batch = batch
+        # the native view of the operator library's object (a batch that came out of a
+        # torch operator is wrapped; compiled samplers hand over native ones)
+        self._batch = batch if isinstance(batch, _native.BlockBatch) else _native.wrap(batch)
         self._edata = dict(edata) if edata else {}
         self._blocks: Optional[List[Optional[Block]]] = None
         self._edge_offsets = None
@@ -141,34 +149,22 @@ class BlockList(Sequence):
         return block
 
     def materialize(self) -> List[Block]:
-        """Every block of the layer, from one call that cuts the layer's arrays into
-        per-batch views.  The objects are filled slot by slot (no constructor call,
-        no per-block conversions): a step hands out a few hundred of them."""
-        if self._blocks is not None and all(b is not None for b in self._blocks):
-            return self._blocks
-        rows, cols, indptrs, fronts, eids, num_src, num_dst = self._batch.blocks()
-        have = self._blocks or [None] * len(rows)
-        edata = self._edata
-        if edata and self._edge_offsets is None:
-            self._edge_offsets = self._batch.offsets()[2]
-        off = self._edge_offsets
-        new = Block.__new__
-        blocks = []
-        for i in range(len(rows)):
-            b = have[i]
-            if b is None:
-                b = new(Block)
-                b.row, b.col, b.indptr = rows[i], cols[i], indptrs[i]
-                b.num_src, b.num_dst = num_src[i], num_dst[i]
-                b.srcdata = {"_ID": fronts[i]}
-                b.dstdata = {}
-                e = eids[i]
-                b.edata = {} if e is None else {"_ID": e}
-                if edata:
-                    lo, hi = off[i], off[i + 1]
-                    for key, value in edata.items():
-                        b.edata[key] = value[lo:hi]
-            blocks.append(b)
+        """Every block of the layer: the objects are filled natively, edge data that
+        was asked for is added here."""
+        have = self._blocks
+        if have is not None and all(b is not None for b in have):
+            return have
+        blocks = self._batch.make_blocks()
+        if self._edata:
+            if self._edge_offsets is None:
+                self._edge_offsets = self._batch.offsets()[2]
+            off = self._edge_offsets
+            for key, value in self._edata.items():
+                sizes = [hi - lo for lo, hi in zip(off, off[1:])]
+                for block, part in zip(blocks, torch.split(value, sizes)):
+                    block.edata[key] = part
+        if have is not None:       # blocks handed out before stay the ones handed out
+            blocks = [new if old is None else old for new, old in zip(blocks, have)]
         self._blocks = blocks
         return blocks
 
