@@ -39,9 +39,18 @@ struct Compressed {
   mutable int64_t indices32_epoch = -1;    // and the cache epoch (invalidate_caches)
   mutable const void* indices32_source = nullptr;  // and its address
   const torch::Tensor& narrow_indices() const;
+  // Where the column behind every edge lies (gs_hop_table), for walks over a
+  // square matrix; made at the second walk over the same matrix.
+  mutable torch::Tensor hops;
+  mutable int64_t hops_versions[2] = {-1, -1}, hops_epoch = -1, hops_asked = 0;
+  mutable const void* hops_source = nullptr;
+  mutable gs_stream_t hops_stream = nullptr;
+  const torch::Tensor& hop_table() const;
   // Call after assigning another `indices` or `indptr` to a matrix that was used.
   void forget_derived() {
     indices32 = torch::Tensor();
+    hops = torch::Tensor();
+    hops_asked = 0;
   }
 };
 

@@ -9,35 +9,94 @@
 
 namespace gs {
 
+// Work-groups of one wavefront while there are fewer walks than fill the machine.
+constexpr int64_t kFewWalks = int64_t(1) << 16;
+
+// Where the column behind an edge lies: what a step needs to know about the node it
+// arrives at.  hops[e] belongs to row id indices[e]; with the table a step is one
+// load in the chain (the hop of the edge it draws) where it is two without (the id,
+// then that column's offsets), and the id itself is only written out.
+struct alignas(8) Hop {
+  uint32_t start, degree;
+};
+
+__global__ __launch_bounds__(kBlock) void hop_table_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_cols, const int64_t* __restrict__ indices,
+    int64_t nnz, Hop* __restrict__ hops) {
+  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (e >= nnz) return;
+  int64_t start;
+  const int64_t deg = column_degree(indptr, num_cols, indices[e], &start);
+  hops[e] = Hop{(uint32_t)start, (uint32_t)deg};
+}
+
+// The random words of a step depend on none of its loads and are drawn while one is
+// on its way; the picks of kHeldSteps steps wait in registers and leave together
+// (loads and stores count down one in-order counter: a store in between is waited
+// for by the next load).
+constexpr int kHeldSteps = 8;
+template <typename IdT, bool kHops>
 __global__ __launch_bounds__(kBlock) void random_walk_kernel(
-    const int64_t* __restrict__ indptr, const int64_t* __restrict__ indices,
-    int64_t num_cols, const int64_t* __restrict__ seeds, int64_t num_seeds,
-    int64_t walk_length, PhiloxKey key, int64_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t* __restrict__ indptr, const IdT* __restrict__ indices,
+    const Hop* __restrict__ hops, int64_t num_cols, const int64_t* __restrict__ seeds,
+    int64_t num_seeds, int64_t walk_length, PhiloxKey key, int64_t* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= num_seeds) return;
   int64_t curr = seeds[i];
   out[i] = curr;
-  for (int64_t step = 1; step <= walk_length; ++step) {
-    int64_t pick = -1;
-    if (curr >= 0 && curr < num_cols) {
-      const int64_t start = indptr[curr];
-      const int64_t deg = indptr[curr + 1] - start;
-      if (deg > 0)
-        pick = indices[start + (int64_t)philox_bounded(key, (uint64_t)i, (uint64_t)step,
-                                                        (uint64_t)deg)];
+  int64_t start = 0, deg = 0;
+  if (kHops) deg = column_degree(indptr, num_cols, curr, &start);
+  Words4 w = philox(key, (uint64_t)i, 1);
+  for (int64_t step0 = 1; step0 <= walk_length; step0 += kHeldSteps) {
+    int64_t held[kHeldSteps];
+#pragma unroll
+    for (int h = 0; h < kHeldSteps; ++h) {
+      held[h] = -1;
+      if (step0 + h <= walk_length) {
+        const uint64_t r = ((uint64_t)w.y << 32) | w.x;
+        if (!kHops) deg = column_degree(indptr, num_cols, curr, &start);
+        if (deg > 0) {
+          const int64_t e = start + (int64_t)__umul64hi(r, (uint64_t)deg);
+          if (kHops) {
+            const Hop next = hops[e];
+            start = next.start;
+            deg = next.degree;
+          }
+          held[h] = (int64_t)indices[e];
+        }
+        w = philox(key, (uint64_t)i, (uint64_t)(step0 + h + 1));
+        curr = held[h];
+      }
     }
-    curr = pick;
-    out[step * num_seeds + i] = pick;
+#pragma unroll
+    for (int h = 0; h < kHeldSteps; ++h)
+      if (step0 + h <= walk_length) out[(step0 + h) * num_seeds + i] = held[h];
   }
 }
 
-// Is `target` among the sorted ids ptr[0, n)?
-__device__ __forceinline__ bool sorted_contains(const int64_t* ptr, int64_t n,
-                                                int64_t target) {
-  int64_t lo = 0, hi = n;
+// Is `target` among the sorted ids ptr[0, n)?  kWide: three probes a round, in
+// flight together -- half the dependent round trips of a bisection for half as many
+// loads again, which pays while the machine is not full.
+template <bool kWide, typename IdT>
+__device__ __forceinline__ bool sorted_contains(const IdT* ptr, int64_t n, int64_t target) {
+  int64_t lo = 0, hi = n;  // ids before lo are smaller, ids from hi on are not
+  if (kWide)
+    while (hi - lo > 3) {
+      const int64_t quarter = (hi - lo) >> 2;
+      const int64_t m0 = lo + quarter, m1 = m0 + quarter, m2 = m1 + quarter;
+      const int64_t v0 = (int64_t)ptr[m0], v1 = (int64_t)ptr[m1], v2 = (int64_t)ptr[m2];
+      if (v0 == target || v1 == target || v2 == target) return true;
+      if (v1 < target) {
+        lo = (v2 < target ? m2 : m1) + 1;
+        if (v2 >= target) hi = m2;
+      } else {
+        hi = v0 < target ? m1 : m0;
+        if (v0 < target) lo = m0 + 1;
+      }
+    }
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
-    const int64_t v = ptr[mid];
+    const int64_t v = (int64_t)ptr[mid];
     if (v == target) return true;
     if (v < target)
       lo = mid + 1;
@@ -54,98 +113,233 @@ constexpr uint32_t kMaxAttempts = 1u << 16;
 // candidate; the candidate is accepted outright when y < min(p, q, 1), else when
 // y < h with h = p for a return to the previous node, q for a neighbour of the
 // previous node, 1 otherwise.
+//
+// G lanes walk one walk: lane g of a group looks at attempts g, g + G, ... of a
+// step, and the lowest accepted attempt is the one that counts, so a step takes one
+// round of loads where one lane takes as many as the slowest of 64 walks has
+// attempts.  Worth it while the machine is not full: a candidate that a group looks
+// at in vain costs a line.  (30 000 walks of 40 steps on 9 M edges: 173 us with one
+// lane a walk, 76 with four at p = 2, q = 0.5; 1318 and 374 with eight at p = 0.25,
+// q = 4, where a candidate in sixteen is accepted for sure.  1 M walks on 124 M
+// edges are bound by lines: 3.3 ms with one lane, 3.9 with two.)
+// (A loop in which every lane goes on to its own next step, instead of waiting for
+// its wavefront at every step, was 28 % slower there: the lanes' stores of a step no
+// longer meet in a line.)
+template <typename IdT, int G, bool kHops>
 __global__ __launch_bounds__(kBlock) void node2vec_kernel(
-    const int64_t* __restrict__ indptr, const int64_t* __restrict__ indices,
-    int64_t num_cols, const int64_t* __restrict__ seeds, int64_t num_seeds,
+    const int64_t* __restrict__ indptr, const IdT* __restrict__ indices,
+    const Hop* __restrict__ hops, int64_t num_cols, const int64_t* __restrict__ seeds, int64_t num_seeds,
     int64_t walk_length, double p, double q, PhiloxKey key,
     int64_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= num_seeds) return;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = t / G;
+  const uint32_t g = (uint32_t)(t % G);
+  if (i >= num_seeds) return;  // whole groups leave together
+  const int group0 = lane_id() - (int)g;
   const double max_scale = p > q ? p : q;
   const double reject_from = max_scale > 1.0 ? max_scale : 1.0;
   double accept_below = p < q ? p : q;
   if (accept_below > 1.0) accept_below = 1.0;
   int64_t curr = seeds[i];
   int64_t last = -1;  // no previous node before the first step
-  out[i] = curr;
+  int64_t last_start = 0, last_deg = 0;
+  if (g == 0) out[i] = curr;
+  int64_t held = -1;  // the pick of step s waits in lane s % G of the group
+  int64_t next_start, next_deg = column_degree(indptr, num_cols, curr, &next_start);
   for (int64_t step = 1; step <= walk_length; ++step) {
-    int64_t pick = -1;
-    if (curr >= 0 && curr < num_cols) {
-      const int64_t start = indptr[curr];
-      const int64_t deg = indptr[curr + 1] - start;
+    int64_t pick = -1, start = next_start, deg = next_deg;
+    if (!kHops && step > 1) deg = column_degree(indptr, num_cols, curr, &start);
+    next_deg = 0;
+    if (deg > 0) {
       if (deg == 1) {
-        pick = indices[start];
-      } else if (deg > 1) {
-        for (uint32_t attempt = 0;; ++attempt) {
+        pick = (int64_t)indices[start];
+        if (kHops) {
+          const Hop n = hops[start];
+          next_start = n.start;
+          next_deg = n.degree;
+        }
+      } else {
+        for (uint32_t attempt = g;; attempt += G) {
           const Words4 w = philox(key, (uint64_t)i, ((uint64_t)step << 32) | attempt);
           const double u = (double)((w.z >> 8) + 1u) * 0x1p-24;  // (0, 1]
           const int y = (int)floor(u * max_scale);
           const uint64_t r = ((uint64_t)w.y << 32) | w.x;
-          const int64_t cand = indices[start + (int64_t)__umul64hi(r, (uint64_t)deg)];
-          pick = cand;
-          if (attempt + 1 >= kMaxAttempts) break;
-          if ((double)y >= reject_from) continue;
-          if ((double)y < accept_below) break;
-          double h = 1.0;
-          if (cand == last) {
-            h = p;
-          } else if (((double)y < q) != ((double)y < 1.0) && last >= 0 &&
-                     last < num_cols) {
-            // the verdict differs between a neighbour of the previous node
-            // (h = q) and any other node (h = 1) only for levels between q and
-            // 1; everywhere else the adjacency search would change nothing
-            const int64_t ls = indptr[last];
-            if (sorted_contains(indices + ls, indptr[last + 1] - ls, cand)) h = q;
+          const int64_t e = start + (int64_t)__umul64hi(r, (uint64_t)deg);
+          Hop hop{0, 0};
+          if (kHops) hop = hops[e];
+          const int64_t cand = (int64_t)indices[e];
+          bool taken = attempt + 1 >= kMaxAttempts || (double)y < accept_below;
+          if (!taken && (double)y < reject_from) {
+            double h = 1.0;
+            if (cand == last) {
+              h = p;
+            } else if (((double)y < q) != ((double)y < 1.0) && last_deg > 0) {
+              // the verdict differs between a neighbour of the previous node
+              // (h = q) and any other node (h = 1) only for levels between q and
+              // 1; everywhere else the adjacency search would change nothing
+              if (sorted_contains<kHops>(indices + last_start, last_deg, cand)) h = q;
+            }
+            taken = (double)y < h;
           }
-          if ((double)y < h) break;
+          pick = cand;
+          if (G == 1) {
+            next_start = hop.start;
+            next_deg = hop.degree;
+            if (taken) break;
+          } else {
+            const uint64_t hits = (__ballot(taken) >> group0) & ((1ull << G) - 1ull);
+            if (hits) {
+              const int winner = group0 + __ffsll((unsigned long long)hits) - 1;
+              pick = __shfl(cand, winner, kWave);
+              if (kHops) {
+                next_start = (uint32_t)__shfl((int)hop.start, winner, kWave);
+                next_deg = (uint32_t)__shfl((int)hop.degree, winner, kWave);
+              }
+              break;
+            }
+          }
         }
       }
     }
     last = curr;
+    last_start = start;
+    last_deg = deg;
     curr = pick;
-    out[step * num_seeds + i] = pick;
+    if (G == 1) {
+      out[step * num_seeds + i] = pick;
+    } else {
+      if ((uint32_t)(step % G) == g) held = pick;
+      if (step % G == G - 1 || step == walk_length) {
+        const int64_t s = step - step % G + g;  // what this lane holds, if of this round
+        if (s >= 1 && s <= step) out[s * num_seeds + i] = held;
+      }
+    }
   }
 }
 
-}  // namespace gs
+// Up to this many walks a call is bound by the latency of its chains of loads: the
+// hop table shortens them.  More walks are bound by lines, of which the table costs
+// as many as it saves, and the column pointer's are the better cached ones.
+constexpr int64_t kHopWalks = int64_t(1) << 15;
 
-extern "C" {
-
-int gs_random_walk(const int64_t* indptr, const int64_t* indices, int64_t num_cols,
-                   const int64_t* seeds, int64_t num_seeds, int64_t walk_length,
-                   uint64_t seed, uint64_t call_id, int64_t* out_traces,
-                   gs_stream_t stream) {
-  using namespace gs;
+template <typename IdT>
+static int random_walk(const int64_t* indptr, const IdT* indices, const Hop* hops,
+                       int64_t num_cols, const int64_t* seeds, int64_t num_seeds,
+                       int64_t walk_length, uint64_t seed, uint64_t call_id, int64_t* out_traces,
+                       gs_stream_t stream) {
   GS_REQUIRE(num_seeds >= 0 && walk_length >= 0 && num_cols >= 0,
              "random_walk: negative size");
   if (num_seeds == 0) return GS_OK;
   GS_REQUIRE(indptr && seeds && out_traces, "random_walk: null pointer");
   hipStream_t s = as_stream(stream);
-  GS_LAUNCH("random_walk", s,
-            random_walk_kernel<<<dim3((unsigned)ceil_div(num_seeds, kBlock)),
-                                 dim3(kBlock), 0, s>>>(
-                indptr, indices, num_cols, seeds, num_seeds, walk_length,
-                make_key(seed, call_id), out_traces));
+  const int threads = num_seeds < kFewWalks ? kWave : kBlock;
+#define GS_RANDOM_WALK(HOPS)                                                                     \
+  GS_LAUNCH("random_walk", s,                                                                    \
+            (random_walk_kernel<IdT, HOPS>)<<<dim3((unsigned)ceil_div(num_seeds, threads)),      \
+                                              dim3(threads), 0, s>>>(                            \
+                indptr, indices, hops, num_cols, seeds, num_seeds, walk_length,                  \
+                make_key(seed, call_id), out_traces))
+  if (hops && num_seeds <= kHopWalks) GS_RANDOM_WALK(true);
+  else GS_RANDOM_WALK(false);
+#undef GS_RANDOM_WALK
   return GS_OK;
 }
 
-int gs_node2vec(const int64_t* indptr, const int64_t* indices, int64_t num_cols,
-                const int64_t* seeds, int64_t num_seeds, int64_t walk_length,
-                double p, double q, uint64_t seed, uint64_t call_id,
-                int64_t* out_traces, gs_stream_t stream) {
-  using namespace gs;
+template <typename IdT>
+static int node2vec(const int64_t* indptr, const IdT* indices, const Hop* hops, int64_t num_cols,
+                    const int64_t* seeds, int64_t num_seeds, int64_t walk_length, double p,
+                    double q, uint64_t seed, uint64_t call_id, int64_t* out_traces,
+                    gs_stream_t stream) {
   GS_REQUIRE(num_seeds >= 0 && walk_length >= 0 && num_cols >= 0,
              "node2vec: negative size");
   GS_REQUIRE(p > 0.0 && q > 0.0, "node2vec: p and q must be positive");
   if (num_seeds == 0) return GS_OK;
   GS_REQUIRE(indptr && seeds && out_traces, "node2vec: null pointer");
   hipStream_t s = as_stream(stream);
-  GS_LAUNCH("node2vec", s,
-            node2vec_kernel<<<dim3((unsigned)ceil_div(num_seeds, kBlock)),
-                              dim3(kBlock), 0, s>>>(
-                indptr, indices, num_cols, seeds, num_seeds, walk_length, p, q,
-                make_key(seed, call_id), out_traces));
+  // As many lanes a walk as keep the call's lanes below what fills the machine:
+  // 200 K where most candidates are accepted, 400 K where an accepted one is rare
+  // (the best of 1, 2, 4, 8, 16 lanes at 1 K to 1 M walks).
+  const double most = p > q ? p : q, least = p < q ? p : q;
+  const int64_t lanes = (least < 1.0 ? least : 1.0) * 4.0 < most ? 400000 : 200000;
+  int group = 16;
+  while (group > 1 && num_seeds * group > lanes) group >>= 1;
+  const int threads = num_seeds * group < kFewWalks ? kWave : kBlock;
+#define GS_NODE2VEC(G, HOPS)                                                                    \
+  GS_LAUNCH("node2vec", s,                                                                      \
+            (node2vec_kernel<IdT, G, HOPS>)<<<dim3((unsigned)ceil_div(num_seeds * (G), threads)), \
+                                              dim3(threads), 0, s>>>(                           \
+                indptr, indices, hops, num_cols, seeds, num_seeds, walk_length, p, q,           \
+                make_key(seed, call_id), out_traces))
+  const bool use_hops = hops && num_seeds <= kHopWalks;
+  if (group == 16) {
+    if (use_hops) GS_NODE2VEC(16, true);
+    else GS_NODE2VEC(16, false);
+  } else if (group == 8) {
+    if (use_hops) GS_NODE2VEC(8, true);
+    else GS_NODE2VEC(8, false);
+  } else if (group == 4) {
+    if (use_hops) GS_NODE2VEC(4, true);
+    else GS_NODE2VEC(4, false);
+  } else if (group == 2) {
+    GS_NODE2VEC(2, false);
+  } else {
+    GS_NODE2VEC(1, false);
+  }
+#undef GS_NODE2VEC
   return GS_OK;
+}
+
+}  // namespace gs
+
+extern "C" {
+
+int gs_hop_table(const int64_t* indptr, int64_t num_cols, const int64_t* indices, int64_t nnz,
+                 void* hops, gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(num_cols >= 0 && nnz >= 0 && nnz < (int64_t(1) << 32), "hop_table: bad size");
+  if (nnz == 0) return GS_OK;
+  GS_REQUIRE(indptr && indices && hops, "hop_table: null pointer");
+  hipStream_t s = as_stream(stream);
+  GS_LAUNCH("hop_table", s,
+            hop_table_kernel<<<dim3((unsigned)ceil_div(nnz, kBlock)), dim3(kBlock), 0, s>>>(
+                indptr, num_cols, indices, nnz, (Hop*)hops));
+  return GS_OK;
+}
+
+int gs_random_walk(const int64_t* indptr, const int64_t* indices, int64_t num_cols,
+                   const int64_t* seeds, int64_t num_seeds, int64_t walk_length,
+                   uint64_t seed, uint64_t call_id, int64_t* out_traces,
+                   gs_stream_t stream) {
+  return gs::random_walk(indptr, indices, nullptr, num_cols, seeds, num_seeds, walk_length, seed,
+                         call_id, out_traces, stream);
+}
+
+int gs_random_walk_hops(const int64_t* indptr, const int64_t* indices, const void* hops,
+                        int64_t num_cols, const int64_t* seeds, int64_t num_seeds,
+                        int64_t walk_length, uint64_t seed, uint64_t call_id,
+                        int64_t* out_traces, gs_stream_t stream) {
+  return gs::random_walk(indptr, indices, (const gs::Hop*)hops, num_cols, seeds, num_seeds,
+                         walk_length, seed, call_id, out_traces, stream);
+}
+
+int gs_node2vec(const int64_t* indptr, const int64_t* indices, int64_t num_cols,
+                const int64_t* seeds, int64_t num_seeds, int64_t walk_length,
+                double p, double q, uint64_t seed, uint64_t call_id,
+                int64_t* out_traces, gs_stream_t stream) {
+  return gs::node2vec(indptr, indices, nullptr, num_cols, seeds, num_seeds, walk_length, p, q,
+                      seed, call_id, out_traces, stream);
+}
+
+int gs_node2vec_hops(const int64_t* indptr, const int64_t* indices, const int32_t* indices32,
+                     const void* hops, int64_t num_cols, const int64_t* seeds, int64_t num_seeds,
+                     int64_t walk_length, double p, double q, uint64_t seed, uint64_t call_id,
+                     int64_t* out_traces, gs_stream_t stream) {
+  const gs::Hop* h = (const gs::Hop*)hops;
+  if (indices32)
+    return gs::node2vec(indptr, indices32, h, num_cols, seeds, num_seeds, walk_length, p, q, seed,
+                        call_id, out_traces, stream);
+  return gs::node2vec(indptr, indices, h, num_cols, seeds, num_seeds, walk_length, p, q, seed,
+                      call_id, out_traces, stream);
 }
 
 }  // extern "C"

@@ -1,0 +1,61 @@
+"""Walks by groups of lanes and over the hop table against the CPU oracle: call sizes on both
+sides of every choice of group size, walk lengths that are no multiple of a group or of the
+steps held in registers, dead ends, columns of one edge."""
+import numpy as np
+import pytest
+import torch
+
+import gsampler_amd as gs
+from oracle import binding as orc
+from tests.conftest import random_csc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def world():
+    rng = np.random.default_rng(7)
+    nodes = 4000
+    indptr, indices = random_csc(rng, nodes, nodes, 9, empty_frac=0.02, hub_deg=70000)
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    return rng, nodes, indptr, m.csc[1].cpu().numpy(), m
+
+
+def traces(walk, n):
+    return walk.reshape(-1, n).cpu().numpy()
+
+
+# 16, 8, 4, 2 and 1 lanes a walk where candidates are often accepted; twice as many walks where not
+@pytest.mark.parametrize("n,length,p,q", [
+    (1, 1, 2.0, 0.5), (333, 7, 2.0, 0.5), (12501, 17, 2.0, 0.5), (25001, 9, 2.0, 0.5),
+    (50001, 6, 2.0, 0.5), (100001, 5, 2.0, 0.5), (200001, 4, 2.0, 0.5),
+    (1000, 33, 0.25, 4.0), (25000, 5, 0.25, 4.0), (32769, 5, 0.25, 4.0), (150000, 4, 0.5, 4.0),
+])
+def test_node2vec(world, n, length, p, q):
+    rng, nodes, indptr, indices, m = world
+    seeds = rng.integers(-1, nodes + 1, n)
+    want = orc.node2vec(indptr, indices, seeds, length, p, q, 11, 0)
+    d = torch.from_numpy(seeds).to(DEV)
+    for _ in range(3):                       # without the hop table, then with it
+        gs.manual_seed(11)
+        got = traces(m.node2vec(d, length, p, q), n)
+        assert np.array_equal(got, want.reshape(length + 1, n))
+
+
+@pytest.mark.parametrize("n,length", [(1, 80), (65, 8), (1000, 9), (32768, 3), (32769, 3), (70000, 17)])
+def test_random_walk(world, n, length):
+    rng, nodes, indptr, indices, m = world
+    seeds = rng.integers(-1, nodes + 1, n)
+    want = orc.random_walk(indptr, indices, seeds, length, 13, 0)
+    d = torch.from_numpy(seeds).to(DEV)
+    for _ in range(3):
+        gs.manual_seed(13)
+        assert np.array_equal(traces(m.random_walk(d, length), n), want.reshape(length + 1, n))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):            # a stream that did not make the table
+        gs.manual_seed(13)
+        assert np.array_equal(traces(m.random_walk(d, length), n), want.reshape(length + 1, n))
