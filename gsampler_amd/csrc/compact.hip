@@ -53,10 +53,21 @@ static CompactWs carve_compact(void* ws, int64_t range) {
   return w;
 }
 
-// Edges per wavefront and round of the passes over a slice.
-constexpr int kCompactItems = 8;
-constexpr int kCompactRounds = 4;
-constexpr int kCompactRun = kCompactItems * kCompactRounds * kWave;
+// A wavefront of the passes over a slice takes `rounds` rounds of kItems rows of
+// 64 edges.  Four rounds of eight share the look-up of the columns among 2048
+// edges; a short slice is spread thinner, or a handful of work-groups walks
+// through its chains of dependent loads (18 thousand edges in 10 work-groups:
+// mark 60 us, fill 46 us).  Two rows a wavefront up to 2^19 edges (1024
+// work-groups, as many as are resident), one round of eight up to 2^22.
+struct CompactSplit {
+  int items, rounds;
+  int64_t run() const { return (int64_t)items * rounds * kWave; }
+};
+static CompactSplit compact_split(int64_t nnz) {
+  if (nnz <= int64_t(1) << 19) return {2, 1};
+  if (nnz <= int64_t(1) << 22) return {8, 1};
+  return {8, 4};
+}
 
 __global__ __launch_bounds__(kBlock) void compact_clear_kernel(uint4* flags, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -72,18 +83,18 @@ __global__ __launch_bounds__(kBlock) void compact_offsets_of_columns_kernel(
   if (c < n) out[c] = segment_of(batch_ptr, num_batches, c) * stride;
 }
 
-// The keys of kCompactItems rows of 64 edges from e0 on (edges past the end
+// The keys of kItems rows of 64 edges from e0 on (edges past the end
 // repeat the last one: the look-ups below shuffle, so all lanes stay together).
-template <typename IdT>
+template <typename IdT, int kItems>
 __device__ __forceinline__ void slice_keys(const SliceView& view, const SliceView::Run& r,
                                            const IdT* __restrict__ ids, int64_t nnz, int64_t e0,
-                                           int64_t (&key)[kCompactItems],
-                                           int64_t (&place)[kCompactItems],
-                                           int64_t (&column)[kCompactItems]) {
+                                           int64_t (&key)[kItems],
+                                           int64_t (&place)[kItems],
+                                           int64_t (&column)[kItems]) {
   const int lane = lane_id();
   if (r.near()) {
 #pragma unroll
-    for (int j = 0; j < kCompactItems; ++j) {
+    for (int j = 0; j < kItems; ++j) {
       int64_t e = e0 + j * kWave + lane;
       if (e >= nnz) e = nnz - 1;
       place[j] = r.place(e);
@@ -92,34 +103,35 @@ __device__ __forceinline__ void slice_keys(const SliceView& view, const SliceVie
     }
     return;
   }
-  int64_t offset[kCompactItems];
+  int64_t offset[kItems];
 #pragma unroll
-  for (int j = 0; j < kCompactItems; ++j) {
+  for (int j = 0; j < kItems; ++j) {
     int64_t e = e0 + j * kWave + lane;
     if (e >= nnz) e = nnz - 1;
     place[j] = view.position(r, e, &column[j], &offset[j]);
   }
 #pragma unroll
-  for (int j = 0; j < kCompactItems; ++j) key[j] = (int64_t)ids[place[j]] + offset[j];
+  for (int j = 0; j < kItems; ++j) key[j] = (int64_t)ids[place[j]] + offset[j];
 }
 
-template <typename IdT>
+template <typename IdT, int kItems>
 __global__ __launch_bounds__(kBlock) void compact_mark_kernel(const IdT* __restrict__ ids,
                                                               int64_t nnz, SliceView view,
-                                                              uint8_t* flags) {
+                                                              int rounds, uint8_t* flags) {
+  const int64_t run_edges = (int64_t)kItems * rounds * kWave;
   const int64_t run = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  const int64_t first = run * kCompactRun;
+  const int64_t first = run * run_edges;
   if (first >= nnz) return;  // whole wavefronts leave together
-  const int64_t stop = first + kCompactRun < nnz ? first + kCompactRun : nnz;
+  const int64_t stop = first + run_edges < nnz ? first + run_edges : nnz;
   const SliceView::Run r = view.run(first, stop - 1);
-  for (int64_t e0 = first; e0 < stop; e0 += kCompactItems * kWave) {
-    int64_t key[kCompactItems], place[kCompactItems], column[kCompactItems];
+  for (int64_t e0 = first; e0 < stop; e0 += kItems * kWave) {
+    int64_t key[kItems], place[kItems], column[kItems];
     slice_keys(view, r, ids, nnz, e0, key, place, column);
-    uint8_t have[kCompactItems];
+    uint8_t have[kItems];
 #pragma unroll
-    for (int j = 0; j < kCompactItems; ++j) have[j] = flags[key[j]];
+    for (int j = 0; j < kItems; ++j) have[j] = flags[key[j]];
 #pragma unroll
-    for (int j = 0; j < kCompactItems; ++j)
+    for (int j = 0; j < kItems; ++j)
       if (!have[j]) flags[key[j]] = 1;
   }
 }
@@ -237,24 +249,25 @@ __global__ __launch_bounds__(kBlock) void compact_rows_kernel(
   }
 }
 
-template <typename IdT>
+template <typename IdT, int kItems>
 __global__ __launch_bounds__(kBlock) void compact_fill_kernel(
-    const IdT* __restrict__ ids, int64_t nnz, SliceView view, const CompactWord* __restrict__ words,
+    const IdT* __restrict__ ids, int64_t nnz, SliceView view, int rounds, const CompactWord* __restrict__ words,
     const int64_t* __restrict__ group_off, int64_t* __restrict__ out_col,
     int64_t* __restrict__ out_row, int64_t* __restrict__ out_select) {
+  const int64_t run_edges = (int64_t)kItems * rounds * kWave;
   const int64_t run = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  const int64_t first = run * kCompactRun;
+  const int64_t first = run * run_edges;
   if (first >= nnz) return;
-  const int64_t stop = first + kCompactRun < nnz ? first + kCompactRun : nnz;
+  const int64_t stop = first + run_edges < nnz ? first + run_edges : nnz;
   const SliceView::Run r = view.run(first, stop - 1);
   const int lane = lane_id();
-  for (int64_t e0 = first; e0 < stop; e0 += kCompactItems * kWave) {
-    int64_t key[kCompactItems], place[kCompactItems], column[kCompactItems], rank[kCompactItems];
+  for (int64_t e0 = first; e0 < stop; e0 += kItems * kWave) {
+    int64_t key[kItems], place[kItems], column[kItems], rank[kItems];
     slice_keys(view, r, ids, nnz, e0, key, place, column);
 #pragma unroll
-    for (int j = 0; j < kCompactItems; ++j) rank[j] = compact_rank(key[j], words, group_off);
+    for (int j = 0; j < kItems; ++j) rank[j] = compact_rank(key[j], words, group_off);
 #pragma unroll
-    for (int j = 0; j < kCompactItems; ++j) {
+    for (int j = 0; j < kItems; ++j) {
       const int64_t e = e0 + j * kWave + lane;
       if (e >= nnz) continue;
       out_row[e] = rank[j];
@@ -317,15 +330,17 @@ int gs_slice_compact_count(const int64_t* indptr, const int64_t* indices, const 
                                                                                  vecs));
   const SliceView view{sub_indptr, cols, indptr, out_key_offset, num_cols_picked};
   if (nnz > 0) {
-    const dim3 grid((unsigned)ceil_div(ceil_div(nnz, kCompactRun), kBlock / kWave));
-    if (indices32)
-      GS_LAUNCH("compact_mark", s,
-                compact_mark_kernel<int32_t><<<grid, dim3(kBlock), 0, s>>>(indices32, nnz, view,
-                                                                           w.flags));
-    else
-      GS_LAUNCH("compact_mark", s,
-                compact_mark_kernel<int64_t><<<grid, dim3(kBlock), 0, s>>>(indices, nnz, view,
-                                                                           w.flags));
+    const CompactSplit split = compact_split(nnz);
+    const dim3 grid((unsigned)ceil_div(ceil_div(nnz, split.run()), kBlock / kWave));
+#define GS_COMPACT_MARK(IDT, IDS, ITEMS)                                                       \
+  GS_LAUNCH("compact_mark", s,                                                                 \
+            (compact_mark_kernel<IDT, ITEMS>)<<<grid, dim3(kBlock), 0, s>>>(IDS, nnz, view,    \
+                                                                            split.rounds, w.flags))
+    if (indices32 && split.items == 2) GS_COMPACT_MARK(int32_t, indices32, 2);
+    else if (indices32) GS_COMPACT_MARK(int32_t, indices32, 8);
+    else if (split.items == 2) GS_COMPACT_MARK(int64_t, indices, 2);
+    else GS_COMPACT_MARK(int64_t, indices, 8);
+#undef GS_COMPACT_MARK
   }
   GS_LAUNCH("compact_words", s,
             compact_words_kernel<<<dim3((unsigned)w.groups), dim3(kBlock), 0, s>>>(
@@ -363,15 +378,18 @@ int gs_slice_compact_fill(const int64_t* indptr, const int64_t* indices, const i
                 w.words, w.group_off, stride, out_rows));
   if (out_indices == nullptr) return GS_OK;
   const SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
-  const dim3 grid((unsigned)ceil_div(ceil_div(nnz, kCompactRun), kBlock / kWave));
-  if (indices32)
-    GS_LAUNCH("compact_fill", s,
-              compact_fill_kernel<int32_t><<<grid, dim3(kBlock), 0, s>>>(
-                  indices32, nnz, view, w.words, w.group_off, out_coo_col, out_indices, out_select));
-  else
-    GS_LAUNCH("compact_fill", s,
-              compact_fill_kernel<int64_t><<<grid, dim3(kBlock), 0, s>>>(
-                  indices, nnz, view, w.words, w.group_off, out_coo_col, out_indices, out_select));
+  const CompactSplit split = compact_split(nnz);
+  const dim3 grid((unsigned)ceil_div(ceil_div(nnz, split.run()), kBlock / kWave));
+#define GS_COMPACT_FILL(IDT, IDS, ITEMS)                                                       \
+  GS_LAUNCH("compact_fill", s,                                                                 \
+            (compact_fill_kernel<IDT, ITEMS>)<<<grid, dim3(kBlock), 0, s>>>(                   \
+                IDS, nnz, view, split.rounds, w.words, w.group_off, out_coo_col, out_indices,  \
+                out_select))
+  if (indices32 && split.items == 2) GS_COMPACT_FILL(int32_t, indices32, 2);
+  else if (indices32) GS_COMPACT_FILL(int32_t, indices32, 8);
+  else if (split.items == 2) GS_COMPACT_FILL(int64_t, indices, 2);
+  else GS_COMPACT_FILL(int64_t, indices, 8);
+#undef GS_COMPACT_FILL
   return GS_OK;
 }
 

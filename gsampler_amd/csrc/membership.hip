@@ -25,10 +25,19 @@
 namespace gs {
 
 constexpr int kMemberWords = kBlock / kWave;  // flag words per chunk of kBlock edges
-constexpr int kMemberChunksPerWave = 8;
-constexpr int kMemberAhead = 4;  // chunks of a wave whose loads are in flight together
-static_assert(kMemberChunksPerWave % kMemberAhead == 0 && kMemberChunksPerWave * kMemberWords <= kWave,
-              "a wave's flag words fit one word per lane");
+// Chunks one wave takes.  A long run shares the look-up of its columns (and, in
+// the flag pass, the staged table) among more edges; on a short edge list it
+// leaves the machine idle while few waves walk through their chains of dependent
+// loads, so the run shrinks with the list: one chunk while even that makes no
+// more than 1024 work-groups (four of them fit a compute unit), four up to 4 Mi
+// edges, eight beyond.  Fixed runs of eight took, on slices of 5 to 38 thousand
+// edges, 24-49 us to flag and 33-46 us to fill (5 to 19 work-groups).
+constexpr int kMemberMaxRun = 8;
+constexpr int kMemberMaxAhead = 4;  // chunks of a wave whose loads are in flight together
+static_assert(kMemberMaxRun * kMemberWords <= kWave, "a wave's flag words fit one word per lane");
+static int member_run(int64_t chunks) {
+  return chunks <= 4096 ? 1 : chunks <= 16384 ? 4 : kMemberMaxRun;
+}
 constexpr int kMemberThreads = 1024;  // 16 waves share one staged table: 32 Ki edges per 32 KB copied
 constexpr int kMemberLdsSlots = 4096;  // tables up to this size are staged in LDS (32 KB)
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
@@ -339,15 +348,18 @@ struct BucketTable {
 
 // kThreads: work-group size.  A large one shares a staged table among more
 // edges; a small one spreads a short edge list over all compute units.
+// kRun: chunks per wave and run.
 // IdT: int64_t, or int32_t when the ids are read from a matrix's narrow copy.
 // kView: the edges are those of a column slice read in place.
-template <bool kInLds, int kThreads, typename IdT, bool kView>
+template <bool kInLds, int kThreads, int kRun, typename IdT, bool kView>
 __global__ __launch_bounds__(kThreads) void member_flag_kernel(
     const IdT* __restrict__ ids, int64_t nnz,
     const uint64_t* __restrict__ global_table, uint32_t cap,
     const int64_t* __restrict__ picked, const int* __restrict__ wide_flag,
     uint64_t* __restrict__ flags, int64_t* __restrict__ chunk_count,
     uint32_t* __restrict__ staged, const uint32_t* __restrict__ filter, SliceView view) {
+  constexpr int kMemberAhead = kRun < kMemberMaxAhead ? kRun : kMemberMaxAhead;
+  static_assert(kRun % kMemberAhead == 0, "a run is whole parts");
   __shared__ __align__(16) uint32_t lds_keys[kInLds ? kMemberLdsSlots : 1];
   __shared__ uint32_t lds_values[kInLds ? kMemberLdsSlots : 1];
   __shared__ uint32_t lds_fill[kInLds ? kMemberBuckets : 1];
@@ -369,13 +381,13 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
   const uint32_t absent = bucketed ? (uint32_t)kMemberLdsSlots : cap;
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   const int lane = lane_id();
-  // A wave takes runs of kMemberChunksPerWave chunks, the work-groups of the
+  // A wave takes runs of kRun chunks, the work-groups of the
   // launch striding over the runs (a launch with fewer work-groups than runs
   // stages its tables once per work-group, not once per run).
   // The ids of kMemberAhead chunks are requested together, before anything is
   // stored: a store between a load and its use makes the wait for the load
   // (loads and stores count down one in-order counter) a wait for everything.
-  const int64_t num_runs = ceil_div_dev(num_chunks, kMemberChunksPerWave);
+  const int64_t num_runs = ceil_div_dev(num_chunks, kRun);
   for (int64_t run = (int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave;
        run < num_runs; run += (int64_t)gridDim.x * (kThreads / kWave)) {
   // With a view the edges are those of a column slice that was never written:
@@ -385,8 +397,8 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
   vrun.split = INT64_MAX;  // no view: every edge at distance 0, offset 0
   bool scattered = false;  // the same in every lane
   if (kView) {
-    const int64_t e_first = run * kMemberChunksPerWave * kBlock;
-    const int64_t e_stop = e_first + kMemberChunksPerWave * kBlock;
+    const int64_t e_first = run * kRun * kBlock;
+    const int64_t e_stop = e_first + kRun * kBlock;
     vrun = view.run(e_first, (e_stop < nnz ? e_stop : nnz) - 1);
     scattered = !vrun.near();
   }
@@ -400,8 +412,8 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
     const int64_t p = view.position(vrun, e, &c, &offset);
     return (uint64_t)((int64_t)ids[p] + offset);
   };
-  for (int part = 0; part < kMemberChunksPerWave / kMemberAhead; ++part) {
-    const int64_t chunk0 = run * kMemberChunksPerWave + part * kMemberAhead;
+  for (int part = 0; part < kRun / kMemberAhead; ++part) {
+    const int64_t chunk0 = run * kRun + part * kMemberAhead;
     if (chunk0 >= num_chunks) break;
     uint32_t keys[kMemberAhead][kMemberWords];
     if (!kView || !scattered) {
@@ -521,7 +533,7 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
                   : (e >= nnz ? chunk_off[num_chunks] : member_rank_before(e, flags, chunk_off));
 }
 
-// A wave writes the kept edges of kMemberChunksPerWave consecutive chunks.  What
+// A wave writes the kept edges of kRun consecutive chunks.  What
 // it needs to know about them arrives in one round trip (lane l holds flag word
 // l of the wave's chunks, the first lanes also a chunk offset each); the columns
 // of the wave's first and last edge take a search each on the scalar unit (one
@@ -531,30 +543,31 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
 // instead of the compressed pointer.
 // kView: the edges are those of a column slice read in place (without it none of
 // the view's look-ups is compiled in).
-template <bool kEdgeMajor, bool kView>
+template <bool kEdgeMajor, bool kView, int kRun>
 __global__ __launch_bounds__(kBlock) void member_fill_kernel(
     int64_t nnz, const uint64_t* __restrict__ flags, const int64_t* __restrict__ chunk_off,
     const uint32_t* __restrict__ staged, const int64_t* __restrict__ indptr,
     int64_t num_major, const int64_t* __restrict__ edge_major,
     int64_t* __restrict__ out_major, int64_t* __restrict__ out_minor,
     int64_t* __restrict__ out_select, SliceView view) {
+  constexpr int kMemberAhead = kRun < kMemberMaxAhead ? kRun : kMemberMaxAhead;
+  static_assert(kRun % kMemberAhead == 0, "a run is whole parts");
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   const int lane = lane_id();
-  const int64_t first_chunk = wave * kMemberChunksPerWave;
+  const int64_t first_chunk = wave * kRun;
   if (first_chunk >= num_chunks) return;
   const int64_t my_word = first_chunk * kMemberWords + lane;
   const uint64_t lane_word =
-      lane < kMemberChunksPerWave * kMemberWords && my_word < num_chunks * kMemberWords
+      lane < kRun * kMemberWords && my_word < num_chunks * kMemberWords
           ? flags[my_word]
           : 0ull;
   const int64_t lane_off =
-      lane < kMemberChunksPerWave && first_chunk + lane < num_chunks ? chunk_off[first_chunk + lane]
+      lane < kRun && first_chunk + lane < num_chunks ? chunk_off[first_chunk + lane]
                                                                     : 0;
   const int64_t e_first = first_chunk * kBlock;
   const int64_t e_end =
-      (first_chunk + kMemberChunksPerWave) * kBlock < nnz ? (first_chunk + kMemberChunksPerWave) * kBlock
-                                                          : nnz;
+      (first_chunk + kRun) * kBlock < nnz ? (first_chunk + kRun) * kBlock : nnz;
   SegmentSpan span{0, 0};
   SliceView::Run vrun{};
   if (kView) {  // indptr is the view's column pointer: one look-up serves both
@@ -564,7 +577,7 @@ __global__ __launch_bounds__(kBlock) void member_fill_kernel(
     span = segment_span(indptr, num_major, e_first, e_end - 1);
   }
 #pragma unroll
-  for (int part = 0; part < kMemberChunksPerWave / kMemberAhead; ++part) {
+  for (int part = 0; part < kRun / kMemberAhead; ++part) {
     const int c0 = part * kMemberAhead;
     if (first_chunk + c0 >= num_chunks) return;
     uint32_t minor[kMemberAhead][kMemberWords];
@@ -679,29 +692,36 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   if (nnz > 0) {
     const bool small = nnz < kMemberSmallEdges;
     const int threads = small ? kBlock : kMemberThreads;
-    int64_t blocks = ceil_div(w.chunks, (threads / kWave) * kMemberChunksPerWave);
+    const int run = member_run(w.chunks);
+    int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
     // a work-group that stages the 64 KB filter does so once and strides over its runs
     const int64_t resident = (int64_t)(kFilterGroupsPerCu * kMemberThreads / threads) * num_compute_units();
     if (filter && blocks > resident) blocks = resident;
     const dim3 grid((unsigned)blocks);
-#define GS_MEMBER_FLAG_AS(LDS, THREADS, IDT, IDS, VIEW)                                       \
+#define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
-            (member_flag_kernel<LDS, THREADS, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>(     \
+            (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
                 IDS, nnz, w.table, cap, picked, w.wide, w.flags, w.chunk_off, w.staged,       \
                 filter, view))
-#define GS_MEMBER_FLAG(LDS, THREADS)                                                          \
+#define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
-    if (ids32 && in_place) GS_MEMBER_FLAG_AS(LDS, THREADS, int32_t, ids32, true);             \
-    else if (ids32) GS_MEMBER_FLAG_AS(LDS, THREADS, int32_t, ids32, false);                   \
-    else if (in_place) GS_MEMBER_FLAG_AS(LDS, THREADS, int64_t, ids, true);                   \
-    else GS_MEMBER_FLAG_AS(LDS, THREADS, int64_t, ids, false);                                \
+    if (ids32 && in_place) GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, int32_t, ids32, true);        \
+    else if (ids32) GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, int32_t, ids32, false);              \
+    else if (in_place) GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, int64_t, ids, true);              \
+    else GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, int64_t, ids, false);                           \
   } while (0)
-    if (in_lds && small) GS_MEMBER_FLAG(true, kBlock);
-    else if (in_lds) GS_MEMBER_FLAG(true, kMemberThreads);
-    else if (small) GS_MEMBER_FLAG(false, kBlock);
-    else GS_MEMBER_FLAG(false, kMemberThreads);
+#define GS_MEMBER_FLAG(LDS)                                                                   \
+  do {                                                                                        \
+    if (!small) GS_MEMBER_FLAG_IDS(LDS, kMemberThreads, kMemberMaxRun);                       \
+    else if (run == 1) GS_MEMBER_FLAG_IDS(LDS, kBlock, 1);                                    \
+    else if (run == 4) GS_MEMBER_FLAG_IDS(LDS, kBlock, 4);                                    \
+    else GS_MEMBER_FLAG_IDS(LDS, kBlock, kMemberMaxRun);                                      \
+  } while (0)
+    if (in_lds) GS_MEMBER_FLAG(true);
+    else GS_MEMBER_FLAG(false);
 #undef GS_MEMBER_FLAG
+#undef GS_MEMBER_FLAG_IDS
 #undef GS_MEMBER_FLAG_AS
     int rc = exclusive_scan_i64(w.chunk_off, w.chunk_off, w.chunks + 1, w.scan_ws,
                                 w.scan_ws_bytes, s);
@@ -735,12 +755,19 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
     return GS_ERR_WORKSPACE;
   }
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)ceil_div(w.chunks, (kBlock / kWave) * kMemberChunksPerWave));
-#define GS_MEMBER_FILL(MAJOR, VIEW)                                                    \
+  const int run = member_run(w.chunks);
+  const dim3 grid((unsigned)ceil_div(w.chunks, (kBlock / kWave) * run));
+#define GS_MEMBER_FILL_RUN(MAJOR, VIEW, RUN)                                           \
   GS_LAUNCH("member_fill", s,                                                          \
-            (member_fill_kernel<MAJOR, VIEW>)<<<grid, dim3(kBlock), 0, s>>>(           \
+            (member_fill_kernel<MAJOR, VIEW, RUN>)<<<grid, dim3(kBlock), 0, s>>>(      \
                 nnz, w.flags, w.chunk_off, w.staged, indptr, num_major, edge_major,    \
                 out_major, out_minor, out_select, view))
+#define GS_MEMBER_FILL(MAJOR, VIEW)                                                    \
+  do {                                                                                 \
+    if (run == 1) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 1);                                  \
+    else if (run == 4) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 4);                             \
+    else GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberMaxRun);                               \
+  } while (0)
   if (view.sub_indptr != nullptr) {
     GS_REQUIRE(!edge_major, "minor_slice_fill: a slice read in place has no edge list");
     GS_MEMBER_FILL(false, true);
@@ -750,6 +777,7 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
     GS_MEMBER_FILL(false, false);
   }
 #undef GS_MEMBER_FILL
+#undef GS_MEMBER_FILL_RUN
   return GS_OK;
 }
 

@@ -17,6 +17,7 @@ DEV = "cuda:0"
     (4096, 900, 9, 0, 7, False),        # batches of exactly one group, many short columns a run
     (5001, 700, 40, 30000, 4, False),   # columns longer than a run of edges
     (5001, 4000, 800, 0, 5, True),      # above 2^20 edges: the int32 copy of the ids
+    (5001, 12000, 1500, 0, 3, True),    # above 2^22 edges in the slice: four rounds a wavefront
 ])
 def test_rows_numbered_anew(rng, rows, cols, max_deg, hub, batches, narrow):
     indptr, indices = random_csc(rng, cols, rows, max_deg, hub_deg=hub)

@@ -51,6 +51,19 @@ def test_minor_slice_with_a_table_outside_lds(npick):
          orc.minor_slice(indices, picked, indptr=indptr))
 
 
+@pytest.mark.parametrize("npick", [200, 3000])
+@pytest.mark.parametrize("nnz", [1, 256, 257, 4096 * 256, 4096 * 256 + 1, 16384 * 256, 16384 * 256 + 1])
+def test_minor_slice_at_the_borders_of_a_waves_run(nnz, npick):
+    """Runs of one, four and eight chunks of 256 edges a wave, with the table in LDS and outside."""
+    rng = np.random.default_rng(nnz + npick)
+    indptr = np.sort(rng.integers(0, nnz + 1, size=1201))
+    indptr[0], indptr[-1] = 0, nnz
+    indices = rng.integers(0, 20000, size=nnz)
+    picked = rng.integers(0, 21000, size=npick)
+    same(capi.minor_slice(T(indices), T(picked), indptr=T(indptr)),
+         orc.minor_slice(indices, picked, indptr=indptr))
+
+
 @pytest.mark.parametrize("npick", [3, 700, 5000])
 def test_minor_slice_with_ids_beyond_32_bits(npick):
     """Picked ids of 2^32 - 1 and above: ids that agree in their low 32 bits must
