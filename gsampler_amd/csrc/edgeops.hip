@@ -568,32 +568,49 @@ static int coo_sum_launch(const int64_t* row, const int64_t* col, const int64_t*
 // Atomic adds to device memory are executed next to the memory, at a rate far
 // below what the edges stream at, and a tile of a large slice rarely adds
 // twice to the same row.  Large coordinate-form sums therefore go through a
-// counting sort by row range instead: (1) every tile of edges counts its edges
-// per range of kRangeRows rows, (2) a scan over the (range, tile) counts gives
-// every tile a private place in every range, (3) the tile writes
-// (row within range, value) pairs there, (4) a work-group sums a slice of one
-// range in LDS and stores its kRangeRows partial sums, (5) the partial sums of
-// a range are folded into the output.  Every pass streams; none uses an atomic
-// on device memory.  The floor of pass 4 is the rate of fp32 adds in LDS
-// (about a quarter of the integer rate), not memory.
+// partition by row range: (1) a work-group sorts a tile of 8192 edges by range in
+// LDS and writes (row within range, value) to the tile's own place, 6 bytes an
+// edge, with the start and length of every range's run in a table of (range, tile)
+// cells, (2) a work-group per range cuts the tiles into units of about 32 Ki of
+// its entries, (3) a work-group sums a unit in LDS and stores kRangeRows partial
+// sums, (4) the partial sums of a range are folded into the output.  The edges are
+// read once, nothing is counted beforehand, and no pass but the fold uses an
+// atomic on device memory.  The floor is 8 + 6 bytes an edge through pass 1 and
+// 6 + the rate of fp64 adds in LDS through pass 3.  On a slice of 29 M edges and
+// 233 K rows a counting pass, a scan, and a scatter of 8-byte pairs to places
+// chosen by the scan took 353 us, with the sums; this takes 193 (part 106, sums 66).
 constexpr int kRangeShift = 13;
-constexpr int kRangeRows = 1 << kRangeShift;  // 32 KB of LDS accumulators
+constexpr int kRangeRows = 1 << kRangeShift;  // 64 KB of LDS accumulators
 constexpr int kMaxRanges = 1024;
 constexpr int kPartThreads = 512;
-constexpr int kPartItems = 8;
+constexpr int kPartItems = 16;
 constexpr int kPartTile = kPartThreads * kPartItems;
-constexpr int kPartMaxRounds = 8;
-constexpr int kSliceEntries = 32768;  // (row, value) pairs one work-group sums
-constexpr int kSliceItems = 8;
+constexpr int kPartWaveRun = kPartItems * kWave;  // consecutive edges of a wavefront
+// Counters of the sort: a range has up to 32 of them, chosen by lane, because most
+// lanes of a wave meet at the range that holds the hubs' rows and adds to one LDS
+// word are taken one after another.
+constexpr int kPartCounters = kMaxRanges;
+constexpr int kPartMaxCopyBits = 5;
+constexpr int kUnitEntries = 32768;  // entries one work-group sums, to within a tile
 // The accumulators of a range take 64 KB of LDS, so two work-groups share a
 // compute unit: 1024 threads each keep all its wavefront slots busy.
 constexpr int kAccThreads = 1024;
+constexpr int kUnitsThreads = 1024;
+static_assert(kPartTile < (1 << 16) && kRangeRows <= (1 << 16), "16-bit rows, starts and lengths");
+static_assert(kPartTile < kUnitEntries, "every unit begins at a tile of its own");
+
+struct RowUnit {
+  int32_t range, tile0, tile1, unused;
+};
+struct RangeUnits {
+  int32_t base, count;
+};
 
 struct RowRangePlan {
-  int64_t ranges = 0, tiles = 0, max_units = 0;
-  int rounds = 1;  // sub-tiles of kPartTile edges one work-group of the partition passes takes
-  size_t off_offsets = 0, off_scan = 0, scan_bytes = 0, off_entries = 0,
-         off_unit_start = 0, off_partial = 0, total = 0;
+  int64_t ranges = 0, tiles = 0, tile_stride = 0, max_units = 0;
+  int copy_bits = 0;
+  size_t off_cells = 0, off_rows = 0, off_values = 0, off_units = 0, off_range_units = 0,
+         off_total = 0, off_partial = 0, total = 0;
 };
 
 // Worth it when the slice is large and rows repeat; empty plan otherwise.
@@ -604,243 +621,320 @@ static RowRangePlan row_range_plan(int format, int64_t nnz, int64_t num_out) {
       ceil_div(num_out, kRangeRows) > kMaxRanges)
     return p;
   p.ranges = ceil_div(num_out, kRangeRows);
-  // The (range, tile) table costs a strided 8-byte access per cell in both
-  // partition passes: once there are work-groups to spare a tile grows to up
-  // to eight sub-tiles, which shrinks the table by as much.
-  int64_t rounds = nnz / ((int64_t)kPartTile * 8192);
-  p.rounds = (int)(rounds < 1 ? 1 : rounds > kPartMaxRounds ? kPartMaxRounds : rounds);
-  p.tiles = ceil_div(nnz, (int64_t)kPartTile * p.rounds);
-  p.max_units = nnz / kSliceEntries + p.ranges;
+  while (p.copy_bits < kPartMaxCopyBits && (p.ranges << (p.copy_bits + 1)) <= kPartCounters)
+    ++p.copy_bits;
+  p.tiles = ceil_div(nnz, (int64_t)kPartTile);
+  p.tile_stride = (p.tiles + 7) / 8 * 8;
+  p.max_units = nnz / kUnitEntries + p.ranges;
   auto take = [&p](size_t bytes) {
     const size_t at = p.total;
     p.total += (bytes + 255) / 256 * 256;
     return at;
   };
-  const int64_t cells = p.ranges * p.tiles + 1;
-  p.off_offsets = take((size_t)cells * sizeof(int64_t));
-  p.scan_bytes = scan_workspace_bytes(cells);
-  p.off_scan = take(p.scan_bytes);
-  p.off_entries = take((size_t)nnz * sizeof(uint2));
-  p.off_unit_start = take((size_t)(p.ranges + 1) * sizeof(int64_t));
+  p.off_cells = take((size_t)(p.ranges * p.tile_stride) * sizeof(uint32_t));
+  p.off_rows = take((size_t)(p.tiles * kPartTile) * sizeof(uint16_t));
+  p.off_values = take((size_t)(p.tiles * kPartTile) * sizeof(float));
+  p.off_units = take((size_t)p.max_units * sizeof(RowUnit));
+  p.off_range_units = take((size_t)p.ranges * sizeof(RangeUnits));
+  p.off_total = take(sizeof(int));
   p.off_partial = take((size_t)p.max_units * kRangeRows * sizeof(float));
   return p;
 }
 
-// counts[range * tiles + tile] = edges of the tile whose target lies in range
-// Lanes of the wavefront that hold the same value (of `bits` bits) as this one,
-// among the valid ones: one ballot per bit.  Many lanes of a wave meet at the
-// same few counters here (a tile's edges fall into a few dozen row ranges, and
-// the range that holds the hubs' rows draws most of them): the first lane of a
-// set of peers sends one atomic for all of them, where 64 single ones to the
-// same LDS word are taken one after another.  Every lane must call this.
-constexpr int kPeerBits = 6;  // up to 64 ranges: worth the ballots (one per bit of the range)
-__device__ __forceinline__ uint64_t wave_peers(int value, int bits, bool valid) {
-  uint64_t peers = __ballot(valid);
-  for (int b = 0; b < bits; ++b) {
-    const bool bit = (value >> b) & 1;
-    const uint64_t m = __ballot(bit);
-    peers &= bit ? m : ~m;
-  }
-  return peers;
+// cells[range * tile_stride + tile] = first entry of the run inside the tile, and its
+// length in the upper half.
+__device__ __forceinline__ uint32_t run_cell(uint32_t start, uint32_t length) {
+  return start | (length << 16);
 }
 
 // With a view the edges are those of a column slice that was never written:
-// dst_ids and efeat are then the parent's arrays (see SliceView).
-__device__ __forceinline__ SliceView::Run view_run(const SliceView& view, int64_t tile0,
-                                                   int64_t tile, int64_t nnz) {
-  if (!view.on()) {  // every edge at distance 0
-    SliceView::Run r{};
-    r.split = INT64_MAX;
-    return r;
-  }
-  const int64_t stop = tile0 + tile < nnz ? tile0 + tile : nnz;
-  return view.run(tile0, stop - 1);
-}
-
+// dst_ids and efeat are then the parent's arrays (see SliceView).  A wavefront
+// takes consecutive edges, so it looks up the few columns of its own run only.
 template <typename IdT>
-__global__ __launch_bounds__(kPartThreads) void rowsum_hist_kernel(
-    const IdT* __restrict__ dst_ids, int64_t nnz, int64_t num_out, int ranges, int range_bits,
-    int64_t tiles, int rounds, int64_t* __restrict__ counts, SliceView view) {
-  __shared__ int hist[kMaxRanges];
-  for (int j = threadIdx.x; j < ranges; j += kPartThreads) hist[j] = 0;
-  __syncthreads();
-  for (int r = 0; r < rounds; ++r) {
-    const int64_t tile0 = ((int64_t)blockIdx.x * rounds + r) * kPartTile;
-    if (tile0 >= nnz) break;
-    const SliceView::Run vrun = view_run(view, tile0, kPartTile, nnz);
-    int64_t dst[kPartItems];
-    if (vrun.near()) {  // (no view: distance 0)
+__global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
+    const IdT* __restrict__ dst_ids, const int64_t* __restrict__ src_ids,
+    const int64_t* __restrict__ edge_map, int64_t nnz, int64_t num_out, int kind,
+    int op, const float* __restrict__ ufeat, const float* __restrict__ efeat,
+    int ranges, int copy_bits, int64_t tile_stride, uint32_t* __restrict__ cells,
+    uint16_t* __restrict__ rows, float* __restrict__ values, int* __restrict__ unit_total,
+    SliceView view) {
+  __shared__ uint32_t count[kPartCounters + 1];
+  __shared__ uint32_t wave_total[kPartThreads / kWave];
+  __shared__ __align__(16) uint16_t lds_row[kPartTile];
+  __shared__ __align__(16) float lds_val[kPartTile];
+  const int t = threadIdx.x, lane = lane_id();
+  const int counters = ranges << copy_bits;
+  if (blockIdx.x == 0 && t == 0) *unit_total = 0;  // counted up by the next kernel
+  for (int j = t; j < kPartCounters + 1; j += kPartThreads) count[j] = 0;
+
+  // 1. all loads of the run, so that they are in flight together
+  const int64_t first = (int64_t)blockIdx.x * kPartTile + (int64_t)(t / kWave) * kPartWaveRun;
+  int row[kPartItems];
+  float val[kPartItems];
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i) {
+    row[i] = -1;
+    val[i] = 0.f;
+  }
+  if (first < nnz) {  // whole wavefronts
+    SliceView::Run vrun{};
+    vrun.split = INT64_MAX;  // no view: every edge at distance 0
+    if (view.on())
+      vrun = view.run(first, (first + kPartWaveRun < nnz ? first + kPartWaveRun : nnz) - 1);
+    const bool shifted = vrun.near();  // the same in every lane
+    auto take = [&](int i, int64_t p) {
+      const int64_t dst = (int64_t)dst_ids[p];
+      const int64_t eid = edge_map ? edge_map[p] : p;
+      val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
+                                 efeat ? efeat + eid : nullptr);
+      row[i] = dst >= 0 && dst < num_out ? (int)dst : -1;
+    };
+    if (shifted && edge_map == nullptr && ufeat == nullptr && efeat != nullptr) {
+      // no branch between the loads, or each would be waited for inside its own
+      IdT id[kPartItems];
 #pragma unroll
       for (int i = 0; i < kPartItems; ++i) {
-        const int64_t e = tile0 + i * kPartThreads + threadIdx.x;
-        dst[i] = e < nnz ? (int64_t)dst_ids[vrun.place(e)] : -1;
+        const int64_t e = first + i * kWave + lane;
+        const int64_t p = vrun.place(e < nnz ? e : nnz - 1);
+        id[i] = dst_ids[p];
+        val[i] = efeat[p];
+      }
+#pragma unroll
+      for (int i = 0; i < kPartItems; ++i) {
+        const int64_t dst = (int64_t)id[i];
+        row[i] = first + i * kWave + lane < nnz && dst >= 0 && dst < num_out ? (int)dst : -1;
+        val[i] = edge_value<float>(kind, op, nullptr, &val[i]);
+      }
+    } else if (shifted) {
+#pragma unroll
+      for (int i = 0; i < kPartItems; ++i) {
+        const int64_t e = first + i * kWave + lane;
+        if (e < nnz) take(i, vrun.place(e));
       }
     } else {
 #pragma unroll
       for (int i = 0; i < kPartItems; ++i) {
-        const int64_t e = tile0 + i * kPartThreads + threadIdx.x;
+        const int64_t e = first + i * kWave + lane;
         int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
         const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
-        dst[i] = e < nnz ? (int64_t)dst_ids[p] : -1;
+        if (e < nnz) take(i, p);
       }
-    }
-#pragma unroll
-    for (int i = 0; i < kPartItems; ++i) {
-      const bool valid = dst[i] >= 0 && dst[i] < num_out;
-      const int range = valid ? (int)(dst[i] >> kRangeShift) : 0;
-      if (range_bits > kPeerBits) {  // many ranges: lanes rarely meet, one atomic each
-        if (valid) atomicAdd(&hist[range], 1);
-        continue;
-      }
-      const uint64_t peers = wave_peers(range, range_bits, valid);
-      if (valid && (peers & ((1ull << lane_id()) - 1ull)) == 0)  // the first of its peers
-        atomicAdd(&hist[range], __popcll(peers));
     }
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < ranges; j += kPartThreads)
-    counts[(int64_t)j * tiles + blockIdx.x] = hist[j];
-  if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)ranges * tiles] = 0;
-}
 
-// A sub-tile is kept small (4096 edges) so that several work-groups share a
-// compute unit and the loads of one overlap the stores of another; what a tile
-// sends to one range is a contiguous run, filled within a few microseconds, so
-// the 8-byte stores merge into whole lines in L2.  A pair keeps its range above
-// the row bits (the accumulate pass masks it off).
-template <typename IdT>
-__global__ __launch_bounds__(kPartThreads) void rowsum_scatter_kernel(
-    const IdT* __restrict__ dst_ids, const int64_t* __restrict__ src_ids,
-    const int64_t* __restrict__ edge_map, int64_t nnz, int64_t num_out, int kind,
-    int op, const float* __restrict__ ufeat, const float* __restrict__ efeat,
-    int ranges, int range_bits, int64_t tiles, int rounds,
-    const int64_t* __restrict__ offsets, uint2* __restrict__ entries, SliceView view) {
-  __shared__ unsigned cursor[kMaxRanges];  // next free place of the tile per range
-  for (int j = threadIdx.x; j < ranges; j += kPartThreads)
-    cursor[j] = (unsigned)offsets[(int64_t)j * tiles + blockIdx.x];
+  // 2. an edge's place among those of its counter
+  const int copy = lane & ((1 << copy_bits) - 1);
+  uint32_t place[kPartItems];
+#pragma unroll
+  for (int i = 0; i < kPartItems; ++i)
+    place[i] = row[i] >= 0
+                   ? atomicAdd(&count[((row[i] >> kRangeShift) << copy_bits) + copy], 1u)
+                   : 0u;
   __syncthreads();
-  for (int r = 0; r < rounds; ++r) {
-    const int64_t tile0 = ((int64_t)blockIdx.x * rounds + r) * kPartTile;
-    if (tile0 >= nnz) break;
-    const SliceView::Run vrun = view_run(view, tile0, kPartTile, nnz);
-    int64_t dst[kPartItems];
-    float val[kPartItems];
-    const bool shifted = vrun.near();  // the same in every lane (no view: distance 0)
+
+  // 3. counts -> first places (two counters per thread; the last word becomes the total)
+  static_assert(kPartCounters == 2 * kPartThreads, "two counters per thread");
+  const uint32_t c0 = count[2 * t], c1 = count[2 * t + 1];
+  uint32_t incl = c0 + c1;
 #pragma unroll
-    for (int i = 0; i < kPartItems; ++i) {
-      const int64_t e = tile0 + i * kPartThreads + threadIdx.x;
-      dst[i] = -1;
-      val[i] = 0.f;
-      if (e < nnz && shifted) {
-        const int64_t p = vrun.place(e);
-        dst[i] = (int64_t)dst_ids[p];
-        const int64_t eid = edge_map ? edge_map[p] : p;
-        val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
-                                   efeat ? efeat + eid : nullptr);
-      }
-    }
-    if (!shifted) {
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t o = __shfl_up(incl, d, kWave);
+    if (lane >= d) incl += o;
+  }
+  if (lane == kWave - 1) wave_total[t / kWave] = incl;
+  __syncthreads();
+  uint32_t before = incl - (c0 + c1);
+  for (int w = 0; w < t / kWave; ++w) before += wave_total[w];
+  count[2 * t] = before;
+  count[2 * t + 1] = before + c0;
+  if (t == kPartThreads - 1) count[kPartCounters] = before + c0 + c1;
+  __syncthreads();
+
+  // 4. sorted in LDS, the runs' cells, and the tile written in order
 #pragma unroll
-      for (int i = 0; i < kPartItems; ++i) {
-        const int64_t e = tile0 + i * kPartThreads + threadIdx.x;
-        int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
-        const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
-        if (e < nnz) {
-          dst[i] = (int64_t)dst_ids[p];
-          const int64_t eid = edge_map ? edge_map[p] : p;
-          val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
-                                     efeat ? efeat + eid : nullptr);
-        }
-      }
-    }
+  for (int i = 0; i < kPartItems; ++i) {
+    if (row[i] < 0) continue;
+    const uint32_t at = count[((row[i] >> kRangeShift) << copy_bits) + copy] + place[i];
+    lds_row[at] = (uint16_t)(row[i] & (kRangeRows - 1));
+    lds_val[at] = val[i];
+  }
+  for (int r = t; r < ranges; r += kPartThreads) {
+    const uint32_t start = count[r << copy_bits];
+    cells[(int64_t)r * tile_stride + blockIdx.x] =
+        run_cell(start, count[(r + 1) << copy_bits] - start);
+  }
+  const uint32_t total = count[counters];
+  __syncthreads();
+  // places past the total hold what LDS held before; no cell covers them
+  uint4* to_rows = reinterpret_cast<uint4*>(rows + (int64_t)blockIdx.x * kPartTile);
+  float4* to_values = reinterpret_cast<float4*>(values + (int64_t)blockIdx.x * kPartTile);
+  const uint4* from_rows = reinterpret_cast<const uint4*>(lds_row);
+  const float4* from_values = reinterpret_cast<const float4*>(lds_val);
 #pragma unroll
-    for (int i = 0; i < kPartItems; ++i) {
-      const bool valid = dst[i] >= 0 && dst[i] < num_out;
-      const int range = valid ? (int)(dst[i] >> kRangeShift) : 0;
-      if (range_bits > kPeerBits) {
-        if (valid)
-          entries[atomicAdd(&cursor[range], 1u)] =
-              make_uint2((unsigned)dst[i], __float_as_uint(val[i]));
-        continue;
+  for (int i = 0; i < kPartItems / 8; ++i)
+    if ((uint32_t)(i * kPartThreads + t) * 8u < total)
+      to_rows[i * kPartThreads + t] = from_rows[i * kPartThreads + t];
+#pragma unroll
+  for (int i = 0; i < kPartItems / 4; ++i)
+    if ((uint32_t)(i * kPartThreads + t) * 4u < total)
+      to_values[i * kPartThreads + t] = from_values[i * kPartThreads + t];
+}
+
+// A work-group per range: unit k of the range is the tiles whose last entry is
+// between k and k + 1 times kUnitEntries entries into the range.  No unit is left
+// out, since a tile holds fewer entries than a unit; tiles in front of the range's
+// first entry and behind its last belong to none.
+__global__ __launch_bounds__(kUnitsThreads) void rowsum_units_kernel(
+    const uint32_t* __restrict__ cells, int64_t tiles, int64_t tile_stride, int* unit_total,
+    RangeUnits* __restrict__ range_units, RowUnit* __restrict__ units) {
+  constexpr int kPer = 8;
+  __shared__ int64_t smem[kUnitsThreads / kWave + 1];
+  __shared__ int base_of_range;
+  const int r = blockIdx.x, t = threadIdx.x;
+  const uint32_t* mine = cells + (int64_t)r * tile_stride;
+  auto load = [&](int64_t i0, uint32_t (&c)[kPer]) {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) c[j] = i0 + j < tiles ? mine[i0 + j] >> 16 : 0u;
+  };
+  // entries of the range
+  int64_t carry = 0;
+  for (int64_t b = 0; b < tiles; b += kUnitsThreads * kPer) {
+    uint32_t c[kPer];
+    load(b + (int64_t)t * kPer, c);
+    int64_t sum = 0, total;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) sum += c[j];
+    block_exclusive_sum<int64_t, kUnitsThreads>(sum, smem, &total);
+    carry += total;
+    __syncthreads();
+  }
+  if (t == 0) {
+    const int n = carry > 0 ? (int)((carry - 1) / kUnitEntries) + 1 : 0;
+    base_of_range = n > 0 ? atomicAdd(unit_total, n) : 0;
+    range_units[r] = RangeUnits{base_of_range, n};
+  }
+  __syncthreads();
+  if (carry == 0) return;
+  const int base = base_of_range;
+  int64_t run0 = 0;
+  for (int64_t b = 0; b < tiles; b += kUnitsThreads * kPer) {
+    uint32_t c[kPer];
+    const int64_t i0 = b + (int64_t)t * kPer;
+    load(i0, c);
+    int64_t sum = 0, total;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) sum += c[j];
+    int64_t run = run0 + block_exclusive_sum<int64_t, kUnitsThreads>(sum, smem, &total);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (c[j] == 0) continue;
+      const int64_t k = (run + c[j] - 1) / kUnitEntries;
+      if (run == 0 || (run - 1) / kUnitEntries != k) {
+        units[base + k].range = r;
+        units[base + k].tile0 = (int32_t)(i0 + j);
+        if (k > 0) units[base + k - 1].tile1 = (int32_t)(i0 + j);
       }
-      const uint64_t peers = wave_peers(range, range_bits, valid);
-      const uint64_t before = peers & ((1ull << lane_id()) - 1ull);
-      unsigned base = 0;
-      if (valid && before == 0) base = atomicAdd(&cursor[range], (unsigned)__popcll(peers));
-      // the first of the peers took places for all of them
-      base = __shfl(base, valid ? __ffsll((long long)peers) - 1 : lane_id(), kWave);
-      if (valid)
-        entries[base + __popcll(before)] = make_uint2((unsigned)dst[i], __float_as_uint(val[i]));
+      run += c[j];
+      if (run == carry) units[base + k].tile1 = (int32_t)(i0 + j + 1);
     }
+    run0 += total;
+    __syncthreads();
   }
 }
 
-// unit_start[r] = first work unit (slice of kSliceEntries pairs) of range r
-__global__ __launch_bounds__(kMaxRanges) void rowsum_units_kernel(
-    const int64_t* __restrict__ offsets, int ranges, int64_t tiles,
-    int64_t* __restrict__ unit_start) {
-  __shared__ int64_t smem[kMaxRanges / kWave + 1];
-  const int r = threadIdx.x;
-  int64_t units = 0;
-  if (r < ranges) {
-    const int64_t n = offsets[(int64_t)(r + 1) * tiles] - offsets[(int64_t)r * tiles];
-    units = ceil_div_dev(n, (int64_t)kSliceEntries);
-  }
-  int64_t total;
-  const int64_t before = block_exclusive_sum<int64_t, kMaxRanges>(units, smem, &total);
-  if (r < ranges) unit_start[r] = before;
-  if (r == 0) unit_start[ranges] = total;
-}
+// The runs of a unit are cut into chunks of one entry a lane, listed in LDS; a
+// wavefront takes eight chunks at a time.  (A range without hubs has about a
+// hundred entries a tile: chunks of 256 left half of the lanes idle.)
+constexpr int kAccChunk = kWave;
+constexpr int kAccAhead = 8;
+constexpr int kAccTiles = kAccThreads;  // tiles listed at a time
+constexpr int kAccMaxChunks = (kUnitEntries + kPartTile) / kAccChunk + kAccTiles;
 
-__global__ __launch_bounds__(kAccThreads) void rowsum_accumulate_kernel(
-    const uint2* __restrict__ entries, const int64_t* __restrict__ offsets,
-    const int64_t* __restrict__ unit_start, int ranges, int64_t tiles,
-    float* __restrict__ partial) {
+__global__ __launch_bounds__(kAccThreads, 8) void rowsum_accumulate_kernel(
+    const uint16_t* __restrict__ rows, const float* __restrict__ values,
+    const uint32_t* __restrict__ cells, int64_t tile_stride, const RowUnit* __restrict__ units,
+    const int* __restrict__ unit_total, float* __restrict__ partial) {
   // Accumulators in double: this part adds doubles in LDS at twice the rate of
   // floats (602 M entries: 1.55 against 3.05 ms), and a slice's sums then carry
   // no rounding of their own before they are rounded to float once.
   __shared__ double acc[kRangeRows];
+  __shared__ uint2 chunks[kAccMaxChunks];  // tile; start inside it and length
+  __shared__ uint32_t smem[kAccThreads / kWave + 1];
+  const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
   const int64_t u = blockIdx.x;
-  if (u >= unit_start[ranges]) return;
-  const int64_t r = segment_of(unit_start, ranges, u);
-  const int64_t range_end = offsets[(r + 1) * tiles];
-  const int64_t begin = offsets[r * tiles] + (u - unit_start[r]) * kSliceEntries;
-  const int64_t end = begin + kSliceEntries < range_end ? begin + kSliceEntries : range_end;
-  for (int j = threadIdx.x; j < kRangeRows; j += kAccThreads) acc[j] = 0.0;
-  __syncthreads();
-  for (int64_t base = begin; base < end; base += kAccThreads * kSliceItems) {
-    uint2 item[kSliceItems];
-#pragma unroll
-    for (int i = 0; i < kSliceItems; ++i) {
-      const int64_t p = base + i * kAccThreads + threadIdx.x;
-      item[i] = p < end ? entries[p] : make_uint2(~0u, 0u);
+  if (u >= *unit_total) return;
+  const RowUnit unit = units[u];
+  for (int j = t; j < kRangeRows; j += kAccThreads) acc[j] = 0.0;
+  for (int tile0 = unit.tile0; tile0 < unit.tile1; tile0 += kAccTiles) {
+    const int tile = tile0 + t;
+    uint32_t start = 0, length = 0;
+    if (tile < unit.tile1) {
+      const uint32_t cell = cells[(int64_t)unit.range * tile_stride + tile];
+      start = cell & 0xFFFFu;
+      length = cell >> 16;
     }
+    const uint32_t n = (length + kAccChunk - 1) / kAccChunk;
+    uint32_t num_chunks;
+    uint32_t at = block_exclusive_sum<uint32_t, kAccThreads>(n, smem, &num_chunks);
+    for (uint32_t k = 0; k < n; ++k) {
+      const uint32_t left = length - k * kAccChunk;
+      chunks[at + k] = make_uint2((uint32_t)tile, (start + k * kAccChunk) |
+                                                      ((left < kAccChunk ? left : kAccChunk) << 16));
+    }
+    __syncthreads();
+    for (uint32_t c0 = (uint32_t)wave * kAccAhead; c0 < num_chunks;
+         c0 += kAccAhead * (kAccThreads / kWave)) {
+      int row[kAccAhead];
+      float val[kAccAhead];
+      bool live[kAccAhead];
 #pragma unroll
-    for (int i = 0; i < kSliceItems; ++i)
-      if (item[i].x != ~0u)
-        atomicAdd(&acc[item[i].x & (kRangeRows - 1)], (double)__uint_as_float(item[i].y));
+      for (int i = 0; i < kAccAhead; ++i) {
+        const uint32_t c = c0 + i;
+        const uint2 d = chunks[c < num_chunks ? c : num_chunks - 1];
+        const int len = (int)(d.y >> 16);  // at least one
+        const int64_t at = (int64_t)d.x * kPartTile + (d.y & 0xFFFFu) + (lane < len ? lane : len - 1);
+        live[i] = c < num_chunks && lane < len;
+        row[i] = (int)rows[at];
+        val[i] = values[at];
+      }
+#pragma unroll
+      for (int i = 0; i < kAccAhead; ++i) {
+        // one row for the whole wavefront (a sum over sorted targets): adds to one
+        // word would be taken one after another
+        const int row0 = __builtin_amdgcn_readfirstlane(row[i]);
+        if (__all(live[i] && row[i] == row0)) {
+          double sum = (double)val[i];
+#pragma unroll
+          for (int d = kWave / 2; d > 0; d >>= 1) sum += __shfl_down(sum, d, kWave);
+          if (lane == 0) atomicAdd(&acc[row0], sum);
+        } else if (live[i]) {
+          atomicAdd(&acc[row[i]], (double)val[i]);
+        }
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
   float* mine = partial + u * kRangeRows;
-  for (int j = threadIdx.x; j < kRangeRows; j += kAccThreads) mine[j] = (float)acc[j];
+  for (int j = t; j < kRangeRows; j += kAccThreads) mine[j] = (float)acc[j];
 }
 
-// out[row] += the row's partial sums over all slices of its range.  Ranges
-// differ a lot in how many slices they have (the rows of hubs sit in one range
-// and draw half of the edges), so the slices of a range are dealt out over
+// out[row] += the row's partial sums over all units of its range.  Ranges
+// differ a lot in how many units they have (the rows of hubs sit in one range
+// and draw half of the edges), so the units of a range are dealt out over
 // gridDim.y work-groups per block of rows, which add their shares atomically.
 constexpr int kFoldSplit = 8;
 
 __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
-    const float* __restrict__ partial, const int64_t* __restrict__ unit_start,
+    const float* __restrict__ partial, const RangeUnits* __restrict__ range_units,
     int64_t num_out, float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= num_out) return;
-  const int64_t r = i >> kRangeShift;  // uniform over the work-group
-  const int64_t u1 = unit_start[r + 1], step = gridDim.y;
+  const RangeUnits ru = range_units[i >> kRangeShift];  // uniform over the work-group
+  const int64_t u1 = (int64_t)ru.base + ru.count, step = gridDim.y;
   const float* p = partial + (i & (kRangeRows - 1));
   float acc = 0.f;
-  int64_t u = unit_start[r] + blockIdx.y;
+  int64_t u = (int64_t)ru.base + blockIdx.y;
   for (; u + 7 * step < u1; u += 8 * step) {  // eight loads in flight
     float v[8];
 #pragma unroll
@@ -860,46 +954,32 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
                          const float* ufeat, const float* efeat, float* out,
                          void* workspace, hipStream_t s, SliceView view = no_view()) {
   char* ws = (char*)workspace;
-  int64_t* offsets = (int64_t*)(ws + p.off_offsets);
-  uint2* entries = (uint2*)(ws + p.off_entries);
-  int64_t* unit_start = (int64_t*)(ws + p.off_unit_start);
+  uint32_t* cells = (uint32_t*)(ws + p.off_cells);
+  uint16_t* rows = (uint16_t*)(ws + p.off_rows);
+  float* values = (float*)(ws + p.off_values);
+  RowUnit* units = (RowUnit*)(ws + p.off_units);
+  RangeUnits* range_units = (RangeUnits*)(ws + p.off_range_units);
+  int* unit_total = (int*)(ws + p.off_total);
   float* partial = (float*)(ws + p.off_partial);
   const int ranges = (int)p.ranges;
-  int range_bits = 0;
-  while ((1 << range_bits) < ranges) ++range_bits;
   const dim3 tiles_grid((unsigned)p.tiles);
-  if (dst_ids32)
-    GS_LAUNCH("rowsum_hist", s,
-              rowsum_hist_kernel<int32_t><<<tiles_grid, dim3(kPartThreads), 0, s>>>(
-                  dst_ids32, nnz, num_out, ranges, range_bits, p.tiles, p.rounds, offsets, view));
-  else
-    GS_LAUNCH("rowsum_hist", s,
-              rowsum_hist_kernel<int64_t><<<tiles_grid, dim3(kPartThreads), 0, s>>>(
-                  dst_ids, nnz, num_out, ranges, range_bits, p.tiles, p.rounds, offsets, view));
-  int rc = exclusive_scan_i64(offsets, offsets, p.ranges * p.tiles + 1,
-                              ws + p.off_scan, p.scan_bytes, s);
-  if (rc != GS_OK) return rc;
-  if (dst_ids32)
-    GS_LAUNCH("rowsum_scatter", s,
-              rowsum_scatter_kernel<int32_t><<<tiles_grid, dim3(kPartThreads), 0, s>>>(
-                  dst_ids32, src_ids, edge_map, nnz, num_out, kind, op, ufeat, efeat,
-                  ranges, range_bits, p.tiles, p.rounds, offsets, entries, view));
-  else
-    GS_LAUNCH("rowsum_scatter", s,
-              rowsum_scatter_kernel<int64_t><<<tiles_grid, dim3(kPartThreads), 0, s>>>(
-                  dst_ids, src_ids, edge_map, nnz, num_out, kind, op, ufeat, efeat,
-                  ranges, range_bits, p.tiles, p.rounds, offsets, entries, view));
+#define GS_ROWSUM_PART(IDT, IDS)                                                              \
+  GS_LAUNCH("rowsum_part", s,                                                                 \
+            rowsum_part_kernel<IDT><<<tiles_grid, dim3(kPartThreads), 0, s>>>(                \
+                IDS, src_ids, edge_map, nnz, num_out, kind, op, ufeat, efeat, ranges,         \
+                p.copy_bits, p.tile_stride, cells, rows, values, unit_total, view))
+  if (dst_ids32) GS_ROWSUM_PART(int32_t, dst_ids32);
+  else GS_ROWSUM_PART(int64_t, dst_ids);
+#undef GS_ROWSUM_PART
   GS_LAUNCH("rowsum_units", s,
-            rowsum_units_kernel<<<dim3(1), dim3(kMaxRanges), 0, s>>>(
-                offsets, ranges, p.tiles, unit_start));
+            rowsum_units_kernel<<<dim3((unsigned)ranges), dim3(kUnitsThreads), 0, s>>>(
+                cells, p.tiles, p.tile_stride, unit_total, range_units, units));
   GS_LAUNCH("rowsum_accumulate", s,
-            rowsum_accumulate_kernel<<<dim3((unsigned)p.max_units),
-                                       dim3(kAccThreads), 0, s>>>(
-                entries, offsets, unit_start, ranges, p.tiles, partial));
+            rowsum_accumulate_kernel<<<dim3((unsigned)p.max_units), dim3(kAccThreads), 0, s>>>(
+                rows, values, cells, p.tile_stride, units, unit_total, partial));
   GS_LAUNCH("rowsum_fold", s,
             rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kBlock), kFoldSplit),
-                                 dim3(kBlock), 0, s>>>(partial, unit_start,
-                                                       num_out, out));
+                                 dim3(kBlock), 0, s>>>(partial, range_units, num_out, out));
   return GS_OK;
 }
 

@@ -139,6 +139,34 @@ def test_scalar_sums_on_skewed_matrices(shape):
                        onto_cols, rtol=1e-5)
 
 
+@pytest.mark.parametrize("nnz,R,targets", [
+    (1 << 20, 1, "any"),                      # one row, one range, 32 counters for it
+    ((1 << 20) + 1, 8192, "any"),             # one full range; a tile with one edge
+    ((1 << 20) + 8191, 8193, "sorted"),       # a range with one row; one target per wavefront
+    (5_000_000, 32 * 8192, "hub"),            # most counters in use, many units of one range
+    (5_000_000, 32 * 8192 + 1, "any"),        # one range more: half the counters per range
+    (12_000_001, 300_000, "last"),            # every edge in the last range: the others have no unit
+    (33_600_000, 1024 * 8192, "any"),         # as many ranges as there are, a few edges a run
+])
+def test_sums_by_row_range_at_their_borders(nnz, R, targets):
+    """Against float64 sums.  A unit of at most 40 960 edges is summed in double and rounded
+    once; a row's units and the eight shares of its fold are added in float: for the hub,
+    5e6 / 32768 = 153 units in shares of 20, at most 29 roundings of 2^-24 = 1.8e-6."""
+    rng = np.random.default_rng(nnz + R)
+    ids = rng.integers(0, R, size=nnz)
+    if targets == "sorted":
+        ids.sort()
+    elif targets == "hub":
+        ids[rng.random(nnz) < 0.9] = 77_777
+    elif targets == "last":
+        ids = np.maximum(ids, R // 8192 * 8192)
+    e = rng.random(nnz, dtype=np.float32) + np.float32(0.1)
+    want = np.bincount(ids, weights=e.astype(np.float64), minlength=R)  # (on the host: no atomics)
+    d_ids = T(ids)
+    got = capi.spmm(("coo", d_ids, d_ids), "copy_rhs", "sum", None, T(e), 2, R)
+    assert np.allclose(got.cpu().numpy().astype(np.float64), want, rtol=2e-6, atol=0)
+
+
 def test_matrix_sum_div_and_ops_wrappers(g):
     rng, indptr, indices, col = g
     m = gs.Matrix()
