@@ -169,23 +169,78 @@ __device__ __forceinline__ uint64_t quantise(float w, double scale) {
   return w > 0.0f ? (uint64_t)__dmul_rn((double)w, scale) : 0ull;
 }
 
-// First position in cdf[0, n) whose value exceeds t, clamped to n - 1.
-__device__ __forceinline__ int64_t cdf_search(const uint64_t* cdf, int64_t n,
-                                              uint64_t t) {
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (cdf[mid] > t)
-      hi = mid;
-    else
-      lo = mid + 1;
+// Exact max of the weights, integer CDF, one binary search per output slot.  A
+// wavefront takes a column of up to kReplLong edges, the whole work-group one of
+// its longer columns after the other; a lane takes eight neighbouring edges, so
+// that their loads are in flight together and one scan serves 512 edges.  The CDF
+// of a column of up to kReplHeld edges stays in LDS, and its weights in registers
+// between the two passes; longer ones use the scratch slice of the column.  The
+// sums are integers: the split does not change them.
+// What bounds it is the chain of loads of the longest column.  A wavefront per
+// column that read 64 edges at a time took 195 us on 794 columns with 368 Ki edges
+// (a power law: the longest has some twenty thousand); this takes 30 us.
+constexpr int kReplThreads = 512;
+constexpr int kReplWaves = kReplThreads / kWave;
+constexpr int kReplItems = 8;
+constexpr int kReplHeld = kReplItems * kWave;
+constexpr int kReplLong = 2048;
+
+// The weights of edges [j0, j0 + kReplItems) of a column, 0 beyond its end.
+__device__ __forceinline__ void repl_load(const float* __restrict__ w, int64_t j0, int64_t deg,
+                                          float (&out)[kReplItems]) {
+  struct Held {
+    float v[kReplItems];
+  };
+  if (j0 + kReplItems <= deg) {
+    Held h;
+    __builtin_memcpy(&h, w + j0, sizeof(Held));
+#pragma unroll
+    for (int i = 0; i < kReplItems; ++i) out[i] = h.v[i];
+    return;
   }
-  return lo < n ? lo : n - 1;
+#pragma unroll
+  for (int i = 0; i < kReplItems; ++i) out[i] = j0 + i < deg ? w[j0 + i] : 0.0f;
 }
 
-// One wavefront per column: exact max of the weights, integer CDF into the
-// scratch slice of the column, then one binary search per output slot.
-__global__ __launch_bounds__(kBlock) void sample_weighted_replace_kernel(
+__device__ __forceinline__ float repl_max(const float (&w)[kReplItems], float m) {
+#pragma unroll
+  for (int i = 0; i < kReplItems; ++i)
+    if (w[i] > m) m = w[i];
+  return m;
+}
+
+__device__ __forceinline__ float wave_max(float m) {
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    const float o = __shfl_xor(m, d, kWave);
+    if (o > m) m = o;
+  }
+  return m;
+}
+
+// Weights -> quantised inclusive sums over the lane's edges; the last is the lane's total.
+__device__ __forceinline__ void repl_sums(const float (&w)[kReplItems], double scale,
+                                          uint64_t (&q)[kReplItems]) {
+  uint64_t run = 0;
+#pragma unroll
+  for (int i = 0; i < kReplItems; ++i) {
+    run += quantise(w[i], scale);
+    q[i] = run;
+  }
+}
+
+__device__ __forceinline__ double repl_scale(float wmax) {
+  return wmax > 0.0f ? det_div(2147483648.0, (double)wmax) : 0.0;
+}
+
+__device__ __forceinline__ void repl_store(uint64_t* cdf, int64_t j0, int64_t deg, uint64_t before,
+                                           const uint64_t (&q)[kReplItems]) {
+#pragma unroll
+  for (int i = 0; i < kReplItems; ++i)
+    if (j0 + i < deg) cdf[j0 + i] = before + q[i];
+}
+
+__global__ __launch_bounds__(kReplThreads) void sample_weighted_replace_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols,
     const int64_t* __restrict__ indices, const float* __restrict__ probs,
     const int64_t* __restrict__ column_ids, int64_t num_items, int64_t fanout,
@@ -193,46 +248,96 @@ __global__ __launch_bounds__(kBlock) void sample_weighted_replace_kernel(
     const int64_t* __restrict__ cdf_offsets, uint64_t* cdf_scratch,
     int64_t* __restrict__ out_coo_col, int64_t* __restrict__ out_indices,
     int64_t* __restrict__ out_select, ColumnLabels labels) {
-  const int lane = lane_id();
-  const int64_t item = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
-  if (item >= num_items) return;
-  const int64_t c = column_ids ? column_ids[item] : item;
-  int64_t in_start;
-  const int64_t deg = column_degree(indptr, num_cols, c, &in_start);
+  __shared__ uint64_t held[kReplWaves][kReplHeld];
+  __shared__ int64_t col_deg[kReplWaves], col_start[kReplWaves], col_cdf[kReplWaves];
+  __shared__ uint64_t col_total[kReplWaves];
+  __shared__ float wave_wmax[kReplWaves];
+  __shared__ uint64_t smem[kReplWaves + 1];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t item = (int64_t)blockIdx.x * kReplWaves + wave;
+  int64_t deg = 0, in_start = 0, at = 0;
+  if (item < num_items) {
+    deg = column_degree(indptr, num_cols, column_ids ? column_ids[item] : item, &in_start);
+    if (deg > 0) at = cdf_offsets ? cdf_offsets[item] : in_start;
+  }
+  if (lane == 0) {
+    col_deg[wave] = deg;
+    col_start[wave] = in_start;
+    col_cdf[wave] = at;
+  }
+  if (deg > 0 && deg <= kReplHeld) {
+    float w[kReplItems];
+    uint64_t q[kReplItems];
+    repl_load(probs + in_start, lane * kReplItems, deg, w);
+    repl_sums(w, repl_scale(wave_max(repl_max(w, 0.0f))), q);
+    const uint64_t incl = wave_inclusive_sum(q[kReplItems - 1]);
+    repl_store(held[wave], lane * kReplItems, deg, incl - q[kReplItems - 1], q);
+    if (lane == kWave - 1) col_total[wave] = incl;
+  } else if (deg > 0 && deg <= kReplLong) {
+    float wmax = 0.0f;
+    for (int64_t base = 0; base < deg; base += kReplHeld) {
+      float w[kReplItems];
+      repl_load(probs + in_start, base + lane * kReplItems, deg, w);
+      wmax = repl_max(w, wmax);
+    }
+    const double scale = repl_scale(wave_max(wmax));
+    uint64_t carry = 0;
+    for (int64_t base = 0; base < deg; base += kReplHeld) {
+      float w[kReplItems];
+      uint64_t q[kReplItems];
+      repl_load(probs + in_start, base + lane * kReplItems, deg, w);
+      repl_sums(w, scale, q);
+      const uint64_t incl = wave_inclusive_sum(q[kReplItems - 1]);
+      repl_store(cdf_scratch + at, base + lane * kReplItems, deg, carry + incl - q[kReplItems - 1],
+                 q);
+      carry += __shfl((unsigned long long)incl, kWave - 1, kWave);
+    }
+    if (lane == 0) col_total[wave] = carry;
+  }
+  __syncthreads();
+  for (int c = 0; c < kReplWaves; ++c) {
+    const int64_t n = col_deg[c];  // the same for every thread
+    if (n <= kReplLong) continue;
+    const float* from = probs + col_start[c];
+    float wmax = 0.0f;
+    for (int64_t base = 0; base < n; base += kReplThreads * kReplItems) {
+      float w[kReplItems];
+      repl_load(from, base + (int64_t)threadIdx.x * kReplItems, n, w);
+      wmax = repl_max(w, wmax);
+    }
+    wmax = wave_max(wmax);
+    if (lane == 0) wave_wmax[wave] = wmax;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kReplWaves; ++v)
+      if (wave_wmax[v] > wmax) wmax = wave_wmax[v];
+    const double scale = repl_scale(wmax);
+    uint64_t carry = 0;
+    for (int64_t base = 0; base < n; base += kReplThreads * kReplItems) {
+      const int64_t j0 = base + (int64_t)threadIdx.x * kReplItems;
+      float w[kReplItems];
+      uint64_t q[kReplItems];
+      repl_load(from, j0, n, w);
+      repl_sums(w, scale, q);
+      uint64_t sum;
+      const uint64_t before =
+          block_exclusive_sum<uint64_t, kReplThreads>(q[kReplItems - 1], smem, &sum);
+      repl_store(cdf_scratch + col_cdf[c], j0, n, carry + before, q);
+      carry += sum;
+    }
+    if (threadIdx.x == 0) col_total[c] = carry;
+    __syncthreads();
+  }
+  // every CDF was written by this work-group, in front of a barrier
   if (deg == 0) return;
   const int64_t out_start = sub_indptr[item];
-  uint64_t* cdf = cdf_scratch + (cdf_offsets ? cdf_offsets[item] : in_start);
-
-  float wmax = 0.0f;
-  for (int64_t j = lane; j < deg; j += kWave) {
-    const float w = probs[in_start + j];
-    if (w > wmax) wmax = w;
-  }
-#pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) {
-    const float o = __shfl_xor(wmax, d, kWave);
-    if (o > wmax) wmax = o;
-  }
-  const double scale = wmax > 0.0f ? det_div(2147483648.0, (double)wmax) : 0.0;
-  uint64_t carry = 0;
-  for (int64_t base = 0; base < deg; base += kWave) {
-    const int64_t j = base + lane;
-    uint64_t q = (j < deg && wmax > 0.0f) ? quantise(probs[in_start + j], scale) : 0ull;
-    q = wave_inclusive_sum(q);
-    if (j < deg) cdf[j] = carry + q;
-    carry += __shfl(q, kWave - 1, kWave);
-  }
-  const uint64_t total = carry;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  for (int64_t j = lane; j < fanout; j += kWave) {
+  const uint64_t total = col_total[wave];
+  auto pick = [&](const uint64_t* cdf, int64_t j) {
     const uint64_t t = total > 0 ? philox_bounded(key, (uint64_t)item, (uint64_t)j, total) : 0ull;
-    // the scratch was written by other lanes of this wavefront: read past L1
-    int64_t lo = 0, hi = deg;
+    int64_t lo = 0, hi = deg;  // first position whose value exceeds t, or the last one
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
-      const uint64_t v = __hip_atomic_load(cdf + mid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (v > t)
+      if (cdf[mid] > t)
         hi = mid;
       else
         lo = mid + 1;
@@ -241,7 +346,11 @@ __global__ __launch_bounds__(kBlock) void sample_weighted_replace_kernel(
     out_indices[out_start + j] = indices ? indices[p] : p;
     out_select[out_start + j] = p;
     if (out_coo_col) out_coo_col[out_start + j] = labels.of(item);
-  }
+  };
+  if (deg <= kReplHeld)
+    for (int64_t j = lane; j < fanout; j += kWave) pick(held[wave], j);
+  else
+    for (int64_t j = lane; j < fanout; j += kWave) pick(cdf_scratch + at, j);
 }
 
 // ------------------------------------------- persistent packed CDF of a matrix
@@ -1295,8 +1404,8 @@ int gs_csc_col_sample_weighted_fill(
     GS_REQUIRE(column_ids == nullptr || cdf_offsets != nullptr,
                "sample_weighted: cdf_offsets are required with column_ids");
     GS_LAUNCH("sample_weighted_replace", s,
-              sample_weighted_replace_kernel<<<dim3((unsigned)ceil_div(num_items * kWave, kBlock)),
-                                               dim3(kBlock), 0, s>>>(
+              sample_weighted_replace_kernel<<<dim3((unsigned)ceil_div(num_items, kReplWaves)),
+                                               dim3(kReplThreads), 0, s>>>(
                   indptr, num_cols, indices, probs, column_ids, num_items, fanout,
                   key, sub_indptr, cdf_offsets, (uint64_t*)cdf_scratch, out_coo_col,
                   out_indices, out_select, labels));

@@ -113,6 +113,26 @@ def test_weight_cdf_of_one_long_column():
                           orc.weight_cdf(indptr, probs, ids, 2_450_000))
 
 
+@pytest.mark.parametrize("fanout", [1, 64, 65])
+def test_with_replacement_at_the_borders_of_the_column_split(fanout):
+    """Columns held in LDS, taken by one wavefront, taken by the work-group (several of them in
+    one work-group too), and columns without weight; weights that start anywhere."""
+    rng = np.random.default_rng(fanout)
+    deg = np.array([0, 1, 7, 8, 9, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4097, 20001, 0, 3,
+                    600, 2500, 1, 512])
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    indices = rng.integers(0, 10**6, size=indptr[-1])
+    probs = rng.lognormal(0, 2, size=indices.size).astype(np.float32)
+    probs[rng.random(indices.size) < 0.3] = 0.0
+    probs[indptr[17]:indptr[18]] = 0.0        # nothing to pick by: the last position
+    probs[indptr[18]:indptr[19]] = -1.0
+    cols = rng.permutation(np.concatenate([np.arange(deg.size), rng.integers(0, deg.size, 40)]))
+    same(capi.sample_weighted(T(indptr), T(indices), F(probs), T(cols), fanout, True, call_id=3),
+         orc.sample_weighted(indptr, indices, probs, cols, fanout, True, call_id=3))
+    same(capi.sample_weighted(T(indptr), T(indices), F(probs), None, fanout, True),
+         orc.sample_weighted(indptr, indices, probs, None, fanout, True))
+
+
 @pytest.mark.parametrize("fanout", [1, 5, 15, 64])
 @pytest.mark.parametrize("replace", [False, True])
 @pytest.mark.parametrize("packed_rows", [False, True])
