@@ -82,6 +82,8 @@ SIGNATURES = {
     "gs_first_position": (_int, [_p, _i64, _i64, _p, _p]),
     "gs_csc_col_slice_values": (_int, [_p, _p, _i64, _p, _i64, _p, _i64, _p, _p]),
     "gs_list_labels": (_int, [_p, _i64, _p, _p, _i64, _p, _p, _p, _p, _p, _p]),
+    "gs_batch_list_labels": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64,
+                                    *([_p] * 10)]),
     "gs_gather_rows": (_int, [_p, _i64, _i64, _p, _i64, _p, _p, _p]),
     "gs_coo_sort_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_coo_sort_flag_offset": (_i64, [_i64, _i64]),

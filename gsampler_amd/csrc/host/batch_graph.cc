@@ -238,6 +238,63 @@ torch::Tensor Graph::batch_rows_for_relabel(const torch::Tensor& edge_rows,
   return mapped_out_;
 }
 
+// Frontier and labels by way of the list of row ids, for a matrix whose rows are
+// positions in a list with a segment per mini-batch; null where that does not pay
+// (a batch should have a few hundred keys and many times as many edges) or where
+// an edge's row turns out to lie in another batch's segment.  Waits for the size
+// of the frontier, as every caller is about to do.
+Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_seeds,
+                                                     const torch::Tensor& row_ids,
+                                                     const ColumnOrderedEdges& edges) {
+  const int64_t R = row_ids.numel(), S = col_seeds.numel(), E = edges.row.numel();
+  const int64_t B = col_bptr_.numel() - 1;
+  if (R == 0 || S == 0 || R != num_rows_ || S != num_cols_ || !edges.col.defined() ||
+      !row_bptr_.defined() || row_bptr_.numel() != B + 1 || row_encoding_size_ <= 0 ||
+      E < 8 * (R + S) || R + S > B * (GS_LIST_LABELS_MAX_KEYS / 2))
+    return nullptr;
+  if (batch_list_labels_ && batch_list_labels_->base.is_same(edges.row) &&
+      batch_list_labels_->row_ids.is_same(row_ids) &&
+      batch_list_labels_->seeds.is_same(col_seeds) &&
+      batch_list_labels_->row_ids_version == (int64_t)row_ids._version() &&
+      batch_list_labels_->seeds_version == (int64_t)col_seeds._version() &&
+      batch_list_labels_->epoch == cache_epoch())
+    return batch_list_labels_->refused ? nullptr : batch_list_labels_.get();
+  auto out = std::make_unique<BatchListLabels>();
+  out->base = edges.row;
+  out->row_ids = row_ids;
+  out->seeds = col_seeds;
+  out->row_ids_version = row_ids._version();
+  out->seeds_version = col_seeds._version();
+  out->epoch = cache_epoch();
+  torch::Tensor table = ids(row_ids, "row_ids"), list_ptr = ids(row_bptr_, "row_bptr");
+  torch::Tensor first = new_ids(R, edges.row);
+  GS_CALL(gs_first_position(cptr(edges.row), E, R, mptr(first), cur_stream()));
+  Frontier& f = out->frontier;
+  f.num_batches = B;
+  f.unique_ptr = new_ids(B + 1, edges.row);
+  f.unique_buffer = new_ids(R + S, edges.row);
+  out->row = new_ids(E, edges.row);
+  out->col = new_ids(E, edges.row);
+  torch::Tensor labels = new_ids(R + S, edges.row);
+  torch::Tensor scratch = new_ids(R + S + B + 1, edges.row);
+  int64_t* mirror = OffsetMirror::reserve(f.unique_ptr);
+  GS_CALL(gs_batch_list_labels(cptr(col_seeds), cptr(col_bptr_), S, cptr(table), cptr(list_ptr), R,
+                               row_encoding_size_, B, cptr(edges.row), cptr(edges.col),
+                               cptr(edge_bptr_), E, cptr(first), mptr(f.unique_buffer),
+                               mptr(f.unique_ptr), mirror, mptr(labels), mptr(labels) + R,
+                               mptr(out->row), mptr(out->col), mptr(scratch), cur_stream()));
+  OffsetMirror::arm(f.unique_ptr);
+  out->refused = f.total() < 0;
+  batch_list_labels_ = std::move(out);
+  if (batch_list_labels_->refused) {
+    batch_list_labels_->row = batch_list_labels_->col = torch::Tensor();
+    batch_list_labels_->frontier = Frontier{};
+    return nullptr;
+  }
+  BatchOffsets::trust(batch_list_labels_->frontier.unique_ptr);
+  return batch_list_labels_.get();
+}
+
 // Queues unique (count + fill) and relabel for the super-batch; nothing here
 // waits for the device.  The frontier's size is still on its way when this
 // returns: f.frontier() waits for it.
@@ -256,6 +313,12 @@ Graph::Frontier& Graph::batch_relabel_launch(torch::Tensor& col_seeds,
     TORCH_CHECK(edges.col_indptr.numel() == col_seeds.numel() + 1,
                 "BatchGraphRelabel: ", col_seeds.numel(), " seeds for a matrix of ",
                 edges.col_indptr.numel() - 1, " columns");
+  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges)) {
+    *out_row = l->row;
+    *out_col = l->col;
+    if (e_ids) *e_ids = edges.e_ids;
+    return l->frontier;
+  }
   torch::Tensor rows = batch_rows_for_relabel(edges.row, row_ids);
   const int64_t E = rows.numel();
   *out_row = new_ids(E, rows);
@@ -295,6 +358,8 @@ std::tuple<torch::Tensor, torch::Tensor> Graph::BatchGetValidNodes(
   ColumnOrderedEdges edges = column_ordered_edges("BatchGetValidNodes");
   col_seeds = ids(col_seeds, "col_seeds");
   BatchOffsets::check(col_bptr_, col_seeds.numel(), "BatchGetValidNodes");
+  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges))
+    return {l->frontier.frontier(), l->frontier.unique_ptr};
   torch::Tensor rows = batch_rows_for_relabel(edges.row, row_ids);
   Frontier& f = frontier_for(col_seeds, rows, col_bptr_, edge_bptr_);
   return {f.frontier(), f.unique_ptr};

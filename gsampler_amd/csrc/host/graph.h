@@ -420,6 +420,18 @@ class Graph : public torch::CustomClassHolder {
     }
   };
   std::unique_ptr<ListLabels> list_labels_;
+  // The same for a super-batch: the frontier and the labels of every edge.
+  struct BatchListLabels {
+    torch::Tensor base, row_ids, seeds;
+    int64_t row_ids_version = -1, seeds_version = -1, epoch = -1;
+    torch::Tensor row, col;
+    Frontier frontier;
+    bool refused = false;  // the general path serves this matrix
+  };
+  std::unique_ptr<BatchListLabels> batch_list_labels_;
+  BatchListLabels* batch_list_labels_for(const torch::Tensor& col_seeds,
+                                         const torch::Tensor& row_ids,
+                                         const ColumnOrderedEdges& edges);
   bool use_list_labels(const torch::Tensor& col_seeds, const torch::Tensor& row_ids) const;
   ListLabels& list_labels_for(const torch::Tensor& col_seeds, const torch::Tensor& row_ids);
 };

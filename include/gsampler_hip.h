@@ -525,6 +525,30 @@ int gs_list_labels(const int64_t* seeds, int64_t num_seeds, const int64_t* list_
                    gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * The same for a super-batch whose list has a segment per mini-batch
+ * (list_ptr[num_batches + 1]): batch b's frontier is the unique of its seeds ++
+ * the listed ids of its segment in the order of first_pos, labels count from the
+ * beginning of the batch's frontier, and every edge gets its two labels.
+ *   id_stride > 0: the key of a listed id is its remainder by id_stride
+ *   out_frontier[num_seeds + num_ids]  the first unique_ptr[num_batches] are written
+ *   unique_ptr[num_batches + 1]        where each batch's frontier begins
+ *   unique_ptr_mirror                  the same in pinned host memory; its last entry
+ *       is -1, and nothing written is to be used, where an edge's row lies outside
+ *       its batch's segment or a batch has more than GS_LIST_LABELS_MAX_KEYS keys
+ *   scratch[num_seeds + num_ids + num_batches + 1]
+ * Rows are positions in the list, columns positions among the seeds; edge_ptr is
+ * the batch pointer of the edges (its last entry is nnz).
+ * ---------------------------------------------------------------------- */
+int gs_batch_list_labels(const int64_t* seeds, const int64_t* seeds_ptr, int64_t num_seeds,
+                         const int64_t* list_ids, const int64_t* list_ptr, int64_t num_ids,
+                         int64_t id_stride, int64_t num_batches, const int64_t* row,
+                         const int64_t* col, const int64_t* edge_ptr, int64_t nnz,
+                         const int64_t* first_pos, int64_t* out_frontier, int64_t* unique_ptr,
+                         int64_t* unique_ptr_mirror, int64_t* out_list_label,
+                         int64_t* out_seed_label, int64_t* out_row, int64_t* out_col,
+                         int64_t* scratch, gs_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * Edge list -> compressed format, first half: stable sort of the edge
  * positions by their id on the axis to compress (`major`, ids in
  * [0, num_major)).  sorted_major receives the ids in order, perm the positions

@@ -5,8 +5,10 @@ import numpy as np
 import pytest
 import torch
 
+import gsampler_amd as gs
 from gsampler_amd import capi
 from oracle import binding as orc
+from tests.conftest import random_csc
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -64,3 +66,52 @@ def test_list_labels_refuses_what_does_not_fit():
     seeds, ids = T(np.arange(n // 2)), T(np.arange(n // 2 + 1))
     with pytest.raises(capi.GsError, match="exceed"):
         capi.list_labels(seeds, ids, torch.zeros(n // 2 + 1, dtype=torch.int64, device=DEV))
+
+
+@pytest.mark.parametrize("sizes,picks,mode", [
+    ([40, 1, 0, 60], [100, 30, 0, 200], "distinct"),      # a batch of one column, an empty one
+    ([300] * 8, [256] * 8, "repeats"),                    # repeated seeds and repeated picks
+    ([1000, 20], [1048, 20], "distinct"),                 # exactly as many keys as a batch may have
+    ([1000, 20], [1049, 20], "distinct"),                 # one more: the general path
+    ([60, 60], [150, 150], "swapped"),                    # picks in the other batch's segment
+])
+def test_batched_labels_by_way_of_the_list(sizes, picks, mode):
+    """Frontier, offsets and labels of a row-sliced encoded super-batch, and all_nodes() before
+    and after, against the oracle batch by batch."""
+    rng = np.random.default_rng(sum(sizes) + sum(picks))
+    R, C = 1500, 2500
+    indptr, indices = random_csc(rng, C, R, 3000)
+    g = gs.Graph(R, C)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    seeds = np.concatenate([rng.integers(0, C, size=n) if mode == "repeats"
+                            else rng.permutation(C)[:n] for n in sizes])
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    sub, _ = g._CAPI_BatchColSlicing(T(seeds), T(ptr), True)
+    ids, row_ptr = sub._CAPI_BatchGetRows()
+    rp = row_ptr.cpu().numpy()
+    picked = [rp[b] + (rng.integers(0, rp[b + 1] - rp[b], size=n) if mode == "repeats"
+                       else rng.permutation(rp[b + 1] - rp[b])[:n]) for b, n in enumerate(picks)]
+    if mode == "swapped":
+        picked.reverse()
+    picked_ptr = T(np.concatenate([[0], np.cumsum([p.size for p in picked])]))
+    picked = T(np.concatenate(picked))
+    for nodes_first in (False, True):
+        part, _ = sub._CAPI_BatchRowSlicing(picked, picked_ptr)
+        row_ids, d_seeds = ids[picked], T(seeds)
+        if nodes_first:
+            nodes, nodes_ptr = part._CAPI_BatchGetValidNodes(d_seeds, row_ids)
+        frontier, uptr, row, col, _, eptr = part._CAPI_BatchGraphRelabel(d_seeds, row_ids)
+        if not nodes_first:
+            nodes, nodes_ptr = part._CAPI_BatchGetValidNodes(d_seeds, row_ids)
+        assert torch.equal(nodes, frontier) and torch.equal(nodes_ptr, uptr)
+        keys = row_ids[part._CAPI_GetCOORows()].cpu().numpy()
+        at_col = part._CAPI_GetCOOCols().cpu().numpy()
+        frontier, uptr, row, col, eptr = (x.cpu().numpy() for x in (frontier, uptr, row, col, eptr))
+        assert keys.size >= 8 * (picked.numel() + seeds.size) and uptr[-1] == frontier.size
+        for b in range(len(sizes)):
+            s, e, u = (slice(p[b], p[b + 1]) for p in (ptr, eptr, uptr))
+            want = orc.unique_relabel(seeds[s], keys[e],
+                                      edge_col=at_col[e] - ptr[b] if sizes[b] else None)
+            assert np.array_equal(frontier[u], want[0]) and np.array_equal(row[e], want[2])
+            if sizes[b]:
+                assert np.array_equal(col[e], want[3])
