@@ -7,10 +7,11 @@
 //          ballots are the chunk's flag words and counts the kept ones; scan
 //          of the chunk counts; out_indptr[c] = kept edges before indptr[c].
 //          The count pass also leaves, per chunk, the new ids (positions in
-//          the picked set) of the chunk's kept edges in edge order.
-//   fill : kept edge e goes to its rank (chunk offset + popcounts), edge order
-//          preserved; its new id comes from the chunk's staged run, so the fill
-//          pass reads neither the ids nor the table again.
+//          the picked set) of the chunk's kept edges in edge order, and their
+//          places in the chunk.
+//   fill : a lane per kept edge, in output order; the new id and the place come
+//          from the chunk's staged run, so the fill pass reads neither the ids
+//          nor the table nor the flags again.
 //
 // A table slot is  low 32 bits of the id << 32 | position in the picked set.
 // While every picked id is below 2^32 - 1 those bits are the id, and an edge
@@ -25,20 +26,23 @@
 namespace gs {
 
 constexpr int kMemberWords = kBlock / kWave;  // flag words per chunk of kBlock edges
-// Chunks one wave takes.  A long run shares the look-up of its columns (and, in
-// the flag pass, the staged table) among more edges; on a short edge list it
-// leaves the machine idle while few waves walk through their chains of dependent
-// loads, so the run shrinks with the list: one chunk while even that makes no
-// more than 1024 work-groups (four of them fit a compute unit), four up to 4 Mi
-// edges, eight beyond.  Fixed runs of eight took, on slices of 5 to 38 thousand
-// edges, 24-49 us to flag and 33-46 us to fill (5 to 19 work-groups).
-constexpr int kMemberMaxRun = 8;
-constexpr int kMemberMaxAhead = 4;  // chunks of a wave whose loads are in flight together
-static_assert(kMemberMaxRun * kMemberWords <= kWave, "a wave's flag words fit one word per lane");
-static int member_run(int64_t chunks) {
-  return chunks <= 4096 ? 1 : chunks <= 16384 ? 4 : kMemberMaxRun;
-}
+// Chunks one wave takes at a time.  A long run shares the look-up of its columns
+// among more edges; on a short edge list it leaves the machine idle while few waves
+// walk through their chains of dependent loads: one chunk while even that makes no
+// more than 1024 work-groups (four of them fit a compute unit), beyond that two to
+// flag (kMemberWavesPerSimd says why no more) and four to fill.  Fixed
+// runs of eight took, on slices of 5 to 38 thousand edges, 24-49 us to flag and
+// 33-46 us to fill (5 to 19 work-groups).
+constexpr int kMemberFlagRun = 2, kMemberFillRun = 4;
+constexpr int64_t kMemberShortChunks = 4096;
 constexpr int kMemberThreads = 1024;  // 16 waves share one staged table: 32 Ki edges per 32 KB copied
+// Two of the large work-groups share a compute unit, which takes at most 64 registers
+// a lane.  Runs of eight chunks, look-ups of four in flight, and the look-ups of
+// scattered runs unrolled took 90 to 128 registers, one work-group was resident, and
+// a launch of 590 or 890 work-groups left its second round half empty: 136 us on 29 M
+// edges of 512 columns and 110 on 19 M (tables in LDS), 126 on 18.5 M (behind the
+// filter).  Two chunks a run, as many work-groups as are resident: 90, 66 and 78.
+constexpr int kMemberWavesPerSimd = 8;
 constexpr int kMemberLdsSlots = 4096;  // tables up to this size are staged in LDS (32 KB)
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 
@@ -65,6 +69,7 @@ struct MemberWs {
   uint64_t* table;     // [member_table_slots(num_picked)]
   uint64_t* flags;     // [chunks * kMemberWords]
   uint32_t* staged;    // [chunks * kBlock]: per chunk, the new ids of its kept edges, in order
+  uint8_t* staged_pos;  // [chunks * kBlock]: and their places in the chunk
   int64_t* chunk_off;  // [chunks + 1]
   int* wide;           // [1] set when a picked id does not fit the upper half of a slot
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (for tables kept in L2)
@@ -92,6 +97,7 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
   w.table = c.take<uint64_t>((size_t)member_table_slots(num_picked));
   w.flags = c.take<uint64_t>((size_t)w.chunks * kMemberWords);
   w.staged = c.take<uint32_t>((size_t)w.chunks * kBlock);
+  w.staged_pos = c.take<uint8_t>((size_t)w.chunks * kBlock);
   w.chunk_off = c.take<int64_t>((size_t)w.chunks + 1);
   w.wide = c.take<int>(1);
   w.filter = c.take<uint32_t>((size_t)kFilterWords);
@@ -352,14 +358,14 @@ struct BucketTable {
 // IdT: int64_t, or int32_t when the ids are read from a matrix's narrow copy.
 // kView: the edges are those of a column slice read in place.
 template <bool kInLds, int kThreads, int kRun, typename IdT, bool kView>
-__global__ __launch_bounds__(kThreads) void member_flag_kernel(
+__global__ __launch_bounds__(kThreads, kThreads == kMemberThreads ? kMemberWavesPerSimd : 1)
+void member_flag_kernel(
     const IdT* __restrict__ ids, int64_t nnz,
     const uint64_t* __restrict__ global_table, uint32_t cap,
     const int64_t* __restrict__ picked, const int* __restrict__ wide_flag,
     uint64_t* __restrict__ flags, int64_t* __restrict__ chunk_count,
-    uint32_t* __restrict__ staged, const uint32_t* __restrict__ filter, SliceView view) {
-  constexpr int kMemberAhead = kRun < kMemberMaxAhead ? kRun : kMemberMaxAhead;
-  static_assert(kRun % kMemberAhead == 0, "a run is whole parts");
+    uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
+    const uint32_t* __restrict__ filter, SliceView view) {
   __shared__ __align__(16) uint32_t lds_keys[kInLds ? kMemberLdsSlots : 1];
   __shared__ uint32_t lds_values[kInLds ? kMemberLdsSlots : 1];
   __shared__ uint32_t lds_fill[kInLds ? kMemberBuckets : 1];
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
   // A wave takes runs of kRun chunks, the work-groups of the
   // launch striding over the runs (a launch with fewer work-groups than runs
   // stages its tables once per work-group, not once per run).
-  // The ids of kMemberAhead chunks are requested together, before anything is
+  // The ids of the kRun chunks are requested together, before anything is
   // stored: a store between a load and its use makes the wait for the load
   // (loads and stores count down one in-order counter) a wait for everything.
   const int64_t num_runs = ceil_div_dev(num_chunks, kRun);
@@ -412,13 +418,12 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
     const int64_t p = view.position(vrun, e, &c, &offset);
     return (uint64_t)((int64_t)ids[p] + offset);
   };
-  for (int part = 0; part < kRun / kMemberAhead; ++part) {
-    const int64_t chunk0 = run * kRun + part * kMemberAhead;
-    if (chunk0 >= num_chunks) break;
-    uint32_t keys[kMemberAhead][kMemberWords];
+  {
+    const int64_t chunk0 = run * kRun;
+    uint32_t keys[kRun][kMemberWords];
     if (!kView || !scattered) {
 #pragma unroll
-      for (int c = 0; c < kMemberAhead; ++c)
+      for (int c = 0; c < kRun; ++c)
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
           const int64_t e = (chunk0 + c) * kBlock + j * kWave + lane;
@@ -428,18 +433,31 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
                        : member_key((uint64_t)(int64_t)ids[e]);
         }
     } else {
+      // one chunk's look-ups at a time: all of them unrolled would set the kernel's
+      // registers, and with them how many work-groups a compute unit holds
 #pragma unroll
-      for (int c = 0; c < kMemberAhead; ++c)
+      for (int c = 0; c < kRun; ++c)
+#pragma unroll
+        for (int j = 0; j < kMemberWords; ++j) keys[c][j] = kNoKey;
+#pragma unroll 1
+      for (int now = 0; now < kRun; ++now) {
+        uint32_t key[kMemberWords];
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
-          const int64_t e = (chunk0 + c) * kBlock + j * kWave + lane;
+          const int64_t e = (chunk0 + now) * kBlock + j * kWave + lane;
           const uint64_t id = id_of(e);
-          keys[c][j] = e < nnz ? member_key(id) : kNoKey;
+          key[j] = e < nnz ? member_key(id) : kNoKey;
         }
+#pragma unroll
+        for (int c = 0; c < kRun; ++c)
+#pragma unroll
+          for (int j = 0; j < kMemberWords; ++j)
+            if (c == now) keys[c][j] = key[j];
+      }
     }
     if (filtered) {
 #pragma unroll
-      for (int c = 0; c < kMemberAhead; ++c)
+      for (int c = 0; c < kRun; ++c)
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
           const uint32_t bits = filter_bits(keys[c][j]);
@@ -447,18 +465,18 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
         }
     }
     // a table in L2 answers after a round trip: the few look-ups that the filter
-    // lets through go through their probe rounds together for all chunks of the part
-    uint32_t all_slots[kMemberAhead * kMemberWords];
+    // lets through go through their probe rounds together for all chunks of the run
+    uint32_t all_slots[kRun * kMemberWords];
     if (filtered) {
-      uint32_t all_keys[kMemberAhead * kMemberWords];
+      uint32_t all_keys[kRun * kMemberWords];
 #pragma unroll
-      for (int c = 0; c < kMemberAhead; ++c)
+      for (int c = 0; c < kRun; ++c)
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) all_keys[c * kMemberWords + j] = keys[c][j];
       table.find_many(all_keys, all_slots);
     }
 #pragma unroll
-    for (int c = 0; c < kMemberAhead; ++c) {
+    for (int c = 0; c < kRun; ++c) {
       const int64_t chunk = chunk0 + c;
       if (chunk >= num_chunks) break;
       uint32_t slot[kMemberWords];
@@ -472,12 +490,17 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
 #pragma unroll
           for (int j = 0; j < kMemberWords; ++j) slot[j] = all_slots[c * kMemberWords + j];
         }
-      } else {
+      } else {  // (rolled up for the same reason)
 #pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) {
-          const int64_t e = chunk * kBlock + j * kWave + lane;
+        for (int j = 0; j < kMemberWords; ++j) slot[j] = cap;
+#pragma unroll 1
+        for (int now = 0; now < kMemberWords; ++now) {
+          const int64_t e = chunk * kBlock + now * kWave + lane;
           const uint64_t id = id_of(e);
-          slot[j] = e < nnz ? table.find_confirmed(id, picked) : cap;
+          const uint32_t found = e < nnz ? table.find_confirmed(id, picked) : cap;
+#pragma unroll
+          for (int j = 0; j < kMemberWords; ++j)
+            if (j == now) slot[j] = found;
         }
       }
 #pragma unroll
@@ -486,9 +509,11 @@ __global__ __launch_bounds__(kThreads) void member_flag_kernel(
         int before = 0;  // kept edges of the chunk in front of this row of 64
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
-          if (slot[j] < absent)
-            staged[chunk * kBlock + before + __popcll(word[j] & ((1ull << lane) - 1))] =
-                bucketed ? buckets.values[slot[j]] : table.value_at(slot[j]);
+          if (slot[j] < absent) {
+            const int64_t at = chunk * kBlock + before + __popcll(word[j] & ((1ull << lane) - 1));
+            staged[at] = bucketed ? buckets.values[slot[j]] : table.value_at(slot[j]);
+            staged_pos[at] = (uint8_t)(j * kWave + lane);
+          }
           before += __popcll(word[j]);
         }
       }
@@ -533,41 +558,51 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
                   : (e >= nnz ? chunk_off[num_chunks] : member_rank_before(e, flags, chunk_off));
 }
 
-// A wave writes the kept edges of kRun consecutive chunks.  What
-// it needs to know about them arrives in one round trip (lane l holds flag word
-// l of the wave's chunks, the first lanes also a chunk offset each); the columns
-// of the wave's first and last edge take a search each on the scalar unit (one
-// column covers the whole span unless columns are short); then the staged ids of all
-// chunks of a part are requested together, and only then anything is stored.
+// A wave writes the kept edges of kRun consecutive chunks: how many each has comes
+// from the chunk offsets, the columns of the wave's first and last edge take a
+// search each on the scalar unit (one column covers the whole span unless columns
+// are short), and the staged ids and places of all chunks are requested together
+// before anything is stored.  The work goes with the kept edges, not with all of
+// them: a lane per edge that looked its flag up took 88 us on 19 M edges of which
+// one in twenty-five is kept, and 84 on 29 M with one in four; this takes 34 and 69.
 // kEdgeMajor: the id on the other axis comes from edge_major (an edge list)
 // instead of the compressed pointer.
 // kView: the edges are those of a column slice read in place (without it none of
 // the view's look-ups is compiled in).
 template <bool kEdgeMajor, bool kView, int kRun>
 __global__ __launch_bounds__(kBlock) void member_fill_kernel(
-    int64_t nnz, const uint64_t* __restrict__ flags, const int64_t* __restrict__ chunk_off,
-    const uint32_t* __restrict__ staged, const int64_t* __restrict__ indptr,
-    int64_t num_major, const int64_t* __restrict__ edge_major,
-    int64_t* __restrict__ out_major, int64_t* __restrict__ out_minor,
-    int64_t* __restrict__ out_select, SliceView view) {
-  constexpr int kMemberAhead = kRun < kMemberMaxAhead ? kRun : kMemberMaxAhead;
-  static_assert(kRun % kMemberAhead == 0, "a run is whole parts");
+    int64_t nnz, const int64_t* __restrict__ chunk_off, const uint32_t* __restrict__ staged,
+    const uint8_t* __restrict__ staged_pos, const int64_t* __restrict__ indptr, int64_t num_major,
+    const int64_t* __restrict__ edge_major, int64_t* __restrict__ out_major,
+    int64_t* __restrict__ out_minor, int64_t* __restrict__ out_select, SliceView view) {
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
   const int lane = lane_id();
   const int64_t first_chunk = wave * kRun;
   if (first_chunk >= num_chunks) return;
-  const int64_t my_word = first_chunk * kMemberWords + lane;
-  const uint64_t lane_word =
-      lane < kRun * kMemberWords && my_word < num_chunks * kMemberWords
-          ? flags[my_word]
-          : 0ull;
-  const int64_t lane_off =
-      lane < kRun && first_chunk + lane < num_chunks ? chunk_off[first_chunk + lane]
-                                                                    : 0;
+  const int64_t lane_chunk = first_chunk + (lane < kRun ? lane : kRun);
+  const int64_t lane_off = chunk_off[lane_chunk < num_chunks ? lane_chunk : num_chunks];
   const int64_t e_first = first_chunk * kBlock;
-  const int64_t e_end =
-      (first_chunk + kRun) * kBlock < nnz ? (first_chunk + kRun) * kBlock : nnz;
+  const int64_t e_end = e_first + kRun * kBlock < nnz ? e_first + kRun * kBlock : nnz;
+  int kept[kRun];  // the same in every lane
+#pragma unroll
+  for (int c = 0; c < kRun; ++c)
+    kept[c] = (int)wave_uniform_first(__shfl((long long)lane_off, c + 1, kWave) -
+                                      __shfl((long long)lane_off, c, kWave));
+  uint32_t minor[kRun][kMemberWords];
+  int at[kRun][kMemberWords];
+#pragma unroll
+  for (int c = 0; c < kRun; ++c)
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) {
+      minor[c][j] = 0;
+      at[c][j] = 0;
+      if (j * kWave < kept[c]) {
+        const int k = j * kWave + lane < kept[c] ? j * kWave + lane : kept[c] - 1;
+        minor[c][j] = staged[(first_chunk + c) * kBlock + k];
+        at[c][j] = staged_pos[(first_chunk + c) * kBlock + k];
+      }
+    }
   SegmentSpan span{0, 0};
   SliceView::Run vrun{};
   if (kView) {  // indptr is the view's column pointer: one look-up serves both
@@ -577,64 +612,31 @@ __global__ __launch_bounds__(kBlock) void member_fill_kernel(
     span = segment_span(indptr, num_major, e_first, e_end - 1);
   }
 #pragma unroll
-  for (int part = 0; part < kRun / kMemberAhead; ++part) {
-    const int c0 = part * kMemberAhead;
-    if (first_chunk + c0 >= num_chunks) return;
-    uint32_t minor[kMemberAhead][kMemberWords];
-    int64_t major[kMemberAhead][kMemberWords];
+  for (int c = 0; c < kRun; ++c) {
+    const int64_t out0 = __shfl((long long)lane_off, c, kWave);
 #pragma unroll
-    for (int c = 0; c < kMemberAhead; ++c) {
-      int before = 0;
-#pragma unroll
-      for (int j = 0; j < kMemberWords; ++j) {
-        const uint64_t word =
-            __shfl((unsigned long long)lane_word, (c0 + c) * kMemberWords + j, kWave);
-        const int64_t e = (first_chunk + c0 + c) * kBlock + j * kWave + lane;
-        minor[c][j] = 0;
-        major[c][j] = 0;
-        if ((word >> lane) & 1ull) {
-          minor[c][j] = staged[(first_chunk + c0 + c) * kBlock + before +
-                               __popcll(word & ((1ull << lane) - 1))];
-          if (kEdgeMajor) major[c][j] = edge_major[e];
+    for (int j = 0; j < kMemberWords; ++j) {
+      if (j * kWave >= kept[c]) break;  // the whole wave
+      const int64_t e = (first_chunk + c) * kBlock + at[c][j];
+      // with a view: the edge's place in the parent and its column in the slice
+      // (on a scattered run the look-up shuffles: all lanes take it, the ones past
+      // the last kept edge with that edge)
+      int64_t parent_pos = e, major = 0;
+      if (kView) {
+        if (vrun.near()) {
+          parent_pos = vrun.place(e);
+          major = vrun.column(e);
+        } else {
+          int64_t offset;
+          parent_pos = view.position(vrun, e, &major, &offset);
         }
-        before += __popcll(word);
       }
-    }
-#pragma unroll
-    for (int c = 0; c < kMemberAhead; ++c) {
-      const int64_t out0 = __shfl((long long)lane_off, c0 + c, kWave);
-      int before = 0;
-#pragma unroll
-      for (int j = 0; j < kMemberWords; ++j) {
-        const uint64_t word =
-            __shfl((unsigned long long)lane_word, (c0 + c) * kMemberWords + j, kWave);
-        const int64_t e = (first_chunk + c0 + c) * kBlock + j * kWave + lane;
-        // with a view: the edge's place in the parent and its column in the slice
-        // (on a scattered run the look-up shuffles: all lanes take it, kept or not)
-        int64_t parent_pos = 0, slice_col = 0;
-        if (kView) {
-          const int64_t ec = e < nnz ? e : nnz - 1;
-          if (vrun.near()) {
-            parent_pos = vrun.place(ec);
-            slice_col = vrun.column(ec);
-          } else {
-            int64_t offset;
-            parent_pos = view.position(vrun, ec, &slice_col, &offset);
-          }
-        }
-        if ((word >> lane) & 1ull) {
-          const int64_t pos = out0 + before + __popcll(word & ((1ull << lane) - 1));
-          out_minor[pos] = (int64_t)minor[c][j];
-          if (kView) {
-            out_select[pos] = parent_pos;
-            if (out_major) out_major[pos] = slice_col;
-          } else {
-            out_select[pos] = e;
-            if (out_major) out_major[pos] = kEdgeMajor ? major[c][j] : span.segment_at(indptr, e);
-          }
-        }
-        before += __popcll(word);
-      }
+      if (j * kWave + lane >= kept[c]) continue;
+      const int64_t pos = out0 + j * kWave + lane;
+      out_minor[pos] = (int64_t)minor[c][j];
+      out_select[pos] = parent_pos;
+      if (out_major)
+        out_major[pos] = kView ? major : kEdgeMajor ? edge_major[e] : span.segment_at(indptr, e);
     }
   }
 }
@@ -692,17 +694,18 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   if (nnz > 0) {
     const bool small = nnz < kMemberSmallEdges;
     const int threads = small ? kBlock : kMemberThreads;
-    const int run = member_run(w.chunks);
+    const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberFlagRun;
     int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
-    // a work-group that stages the 64 KB filter does so once and strides over its runs
+    // a large list, or work-groups that stage the 64 KB filter: as many of them as are
+    // resident, each staging its tables once and striding over its runs
     const int64_t resident = (int64_t)(kFilterGroupsPerCu * kMemberThreads / threads) * num_compute_units();
-    if (filter && blocks > resident) blocks = resident;
+    if ((filter || !small) && blocks > resident) blocks = resident;
     const dim3 grid((unsigned)blocks);
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
                 IDS, nnz, w.table, cap, picked, w.wide, w.flags, w.chunk_off, w.staged,       \
-                filter, view))
+                w.staged_pos, filter, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
@@ -713,10 +716,9 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   } while (0)
 #define GS_MEMBER_FLAG(LDS)                                                                   \
   do {                                                                                        \
-    if (!small) GS_MEMBER_FLAG_IDS(LDS, kMemberThreads, kMemberMaxRun);                       \
+    if (!small) GS_MEMBER_FLAG_IDS(LDS, kMemberThreads, kMemberFlagRun);                      \
     else if (run == 1) GS_MEMBER_FLAG_IDS(LDS, kBlock, 1);                                    \
-    else if (run == 4) GS_MEMBER_FLAG_IDS(LDS, kBlock, 4);                                    \
-    else GS_MEMBER_FLAG_IDS(LDS, kBlock, kMemberMaxRun);                                      \
+    else GS_MEMBER_FLAG_IDS(LDS, kBlock, kMemberFlagRun);                                     \
   } while (0)
     if (in_lds) GS_MEMBER_FLAG(true);
     else GS_MEMBER_FLAG(false);
@@ -755,18 +757,17 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
     return GS_ERR_WORKSPACE;
   }
   hipStream_t s = as_stream(stream);
-  const int run = member_run(w.chunks);
+  const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberFillRun;
   const dim3 grid((unsigned)ceil_div(w.chunks, (kBlock / kWave) * run));
 #define GS_MEMBER_FILL_RUN(MAJOR, VIEW, RUN)                                           \
   GS_LAUNCH("member_fill", s,                                                          \
             (member_fill_kernel<MAJOR, VIEW, RUN>)<<<grid, dim3(kBlock), 0, s>>>(      \
-                nnz, w.flags, w.chunk_off, w.staged, indptr, num_major, edge_major,    \
+                nnz, w.chunk_off, w.staged, w.staged_pos, indptr, num_major, edge_major, \
                 out_major, out_minor, out_select, view))
 #define GS_MEMBER_FILL(MAJOR, VIEW)                                                    \
   do {                                                                                 \
     if (run == 1) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 1);                                  \
-    else if (run == 4) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 4);                             \
-    else GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberMaxRun);                               \
+    else GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberFillRun);                              \
   } while (0)
   if (view.sub_indptr != nullptr) {
     GS_REQUIRE(!edge_major, "minor_slice_fill: a slice read in place has no edge list");
