@@ -65,6 +65,24 @@ struct EdgeView {
   }
 };
 
+// Element idx of an [nnz, out_len] output -> its edge and its place in the feature.
+// A 64-bit division takes some forty instructions, more than the rest of an element:
+// none for scalars, a 32-bit one while the whole output has fewer than 2^32 elements.
+__device__ __forceinline__ void split_index(int64_t idx, int64_t total, int64_t out_len, int64_t* e,
+                                            int64_t* f) {
+  if (out_len == 1) {
+    *e = idx;
+    *f = 0;
+  } else if (total < (int64_t(1) << 32)) {
+    const uint32_t q = (uint32_t)idx / (uint32_t)out_len;
+    *e = q;
+    *f = (uint32_t)idx - q * (uint32_t)out_len;
+  } else {
+    *e = idx / out_len;
+    *f = idx - *e * out_len;
+  }
+}
+
 // A work-group handles kBlock * ITEMS consecutive elements of an
 // [nnz, out_len] output.  On a compressed form ITEMS = kEdgeItems, so that the
 // look-up of the segments its edges touch is paid once per 2048 elements; an
@@ -95,7 +113,8 @@ __global__ __launch_bounds__(kBlock) void sddmm_kernel(
   for (int j = 0; j < ITEMS; ++j) {
     const int64_t idx = idx0 + j * kBlock + threadIdx.x;
     if (idx >= nnz * out_len) break;
-    const int64_t e = idx / out_len, f = idx - e * out_len;
+    int64_t e, f;
+    split_index(idx, nnz * out_len, out_len, &e, &f);
     int64_t src, dst, eid;
     g.endpoints(sp, e, &src, &dst, &eid);
     const int64_t lf = lhs_off ? lhs_off[f] : f, rf = rhs_off ? rhs_off[f] : f;
@@ -107,6 +126,47 @@ __global__ __launch_bounds__(kBlock) void sddmm_kernel(
                      : rhs + pick(rhs_target, src, eid, dst) * rhs_len + rf * reduce_size;
     out[eid * out_len + f] = apply_op<T>(op, l, r, reduce_size);
   }
+}
+
+// One value an edge on an edge list (the divisions of a layer-wise sampler): lhs_ids
+// and rhs_ids are the id array an operand is read through, null for a value of the
+// edge's own.  Four edges a lane, whose loads are in flight together, and only the
+// ids that an operand needs: 7.3 M edges 41 us one edge a lane with both ids,
+// 28 so (602 M edges: 2.85 and 1.63 ms).
+constexpr int kScalarItems = 4;
+template <typename T>
+__global__ __launch_bounds__(kBlock) void sddmm_scalar_kernel(
+    int64_t nnz, int op, const int64_t* __restrict__ edge_map,
+    const int64_t* __restrict__ lhs_ids, const int64_t* __restrict__ rhs_ids,
+    const T* __restrict__ lhs, const T* __restrict__ rhs, T* __restrict__ out) {
+  const int64_t e0 = (int64_t)blockIdx.x * (kBlock * kScalarItems) + threadIdx.x;
+  int64_t e[kScalarItems], eid[kScalarItems], li[kScalarItems], ri[kScalarItems];
+#pragma unroll
+  for (int j = 0; j < kScalarItems; ++j) {
+    const int64_t at = e0 + j * kBlock;
+    e[j] = eid[j] = at < nnz ? at : nnz - 1;
+  }
+  if (edge_map)
+#pragma unroll
+    for (int j = 0; j < kScalarItems; ++j) eid[j] = edge_map[e[j]];
+#pragma unroll
+  for (int j = 0; j < kScalarItems; ++j) li[j] = ri[j] = eid[j];
+  if (lhs_ids)
+#pragma unroll
+    for (int j = 0; j < kScalarItems; ++j) li[j] = lhs_ids[e[j]];
+  if (rhs_ids)
+#pragma unroll
+    for (int j = 0; j < kScalarItems; ++j) ri[j] = rhs_ids[e[j]];
+  T l[kScalarItems] = {}, r[kScalarItems] = {};
+  if (op != kOpCopyRhs)
+#pragma unroll
+    for (int j = 0; j < kScalarItems; ++j) l[j] = lhs[li[j]];
+  if (op != kOpCopyLhs)
+#pragma unroll
+    for (int j = 0; j < kScalarItems; ++j) r[j] = rhs[ri[j]];
+#pragma unroll
+  for (int j = 0; j < kScalarItems; ++j)
+    if (e0 + j * kBlock < nnz) out[eid[j]] = apply_op<T>(op, &l[j], &r[j], 1);
 }
 
 // Two SDDMMs (u op v) that share one edge sweep.
@@ -405,6 +465,28 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_sum_kernel(
   const int64_t c1 = indptr[c0 + 1] > last
                          ? c0
                          : c0 + segment_of(indptr + c0, num_major - c0, last);
+  if (c0 == c1) {
+    // the whole tile lies inside one column: no accumulators to clear, one add
+    float mine = 0.f;
+    for (int r = 0; r < rounds; ++r) {
+      if (r > 0) load_round(tile0 + (int64_t)r * kSumTile, val);  // (0 past the tile's end)
+      float round_sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < kSumItems; ++i) round_sum += val[i];
+      mine += round_sum;
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
+    if (lane_id() == 0) acc[threadIdx.x / kWave] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float sum = acc[0];
+#pragma unroll
+      for (int w = 1; w < kBlock / kWave; ++w) sum += acc[w];
+      unsafeAtomicAdd(out + c0, sum);
+    }
+    return;
+  }
   const int64_t nseg = c1 - c0 + 1;
   const bool in_lds = nseg <= kSumSegs;
   if (in_lds) {
@@ -1110,7 +1192,19 @@ int gs_sddmm(int format, const int64_t* a, const int64_t* b, int64_t num_major,
                                      dim3(kBlock), 0, s>>>(                               \
                 g, nnz, op, (const T*)lhs, (const T*)rhs, (T*)out, lhs_target, rhs_target, \
                 lhs_len, rhs_len, out_len, reduce_size, lhs_off, rhs_off))
-  if (g.compressed) {
+  // (targets: 0 = row ids, 1 = the edge's own, 2 = column ids)
+#define GS_SDDMM_SCALAR(T)                                                                    \
+  GS_LAUNCH("sddmm", s,                                                                       \
+            sddmm_scalar_kernel<T><<<dim3((unsigned)ceil_div(nnz, kBlock * kScalarItems)),    \
+                                     dim3(kBlock), 0, s>>>(                                   \
+                nnz, op, edge_map, lhs_target == 0 ? a : lhs_target == 2 ? b : nullptr,       \
+                rhs_target == 0 ? a : rhs_target == 2 ? b : nullptr, (const T*)lhs,           \
+                (const T*)rhs, (T*)out))
+  if (!g.compressed && out_len == 1 && reduce_size == 1 && lhs_len == 1 && rhs_len == 1 &&
+      !lhs_off && !rhs_off) {
+    if (dtype == GS_F32) GS_SDDMM_SCALAR(float);
+    else GS_SDDMM_SCALAR(double);
+  } else if (g.compressed) {
     if (dtype == GS_F32) GS_SDDMM_LAUNCH(float, kEdgeItems);
     else GS_SDDMM_LAUNCH(double, kEdgeItems);
   } else {
@@ -1118,6 +1212,7 @@ int gs_sddmm(int format, const int64_t* a, const int64_t* b, int64_t num_major,
     else GS_SDDMM_LAUNCH(double, 1);
   }
 #undef GS_SDDMM_LAUNCH
+#undef GS_SDDMM_SCALAR
   return GS_OK;
 }
 

@@ -29,12 +29,15 @@ constexpr int kMemberWords = kBlock / kWave;  // flag words per chunk of kBlock 
 // Chunks one wave takes at a time.  A long run shares the look-up of its columns
 // among more edges; on a short edge list it leaves the machine idle while few waves
 // walk through their chains of dependent loads: one chunk while even that makes no
-// more than 1024 work-groups (four of them fit a compute unit), beyond that two to
-// flag (kMemberWavesPerSimd says why no more) and four to fill.  Fixed
-// runs of eight took, on slices of 5 to 38 thousand edges, 24-49 us to flag and
-// 33-46 us to fill (5 to 19 work-groups).
-constexpr int kMemberFlagRun = 2, kMemberFillRun = 4;
+// more than 1024 work-groups (four of them fit a compute unit), two beyond that
+// (kMemberWavesPerSimd says why no more).  Fixed runs of eight took, on slices of 5 to 38 thousand
+// edges, 24-49 us to flag and 33-46 us to fill (5 to 19 work-groups).
+constexpr int kMemberLongRun = 2;
 constexpr int64_t kMemberShortChunks = 4096;
+// The fill pass alone goes to four beyond 64 Mi edges (29 M edges: 59 us with two, 69
+// with four; a row slice of 602 M: 3.34 ms with two, 3.10 with four).
+constexpr int kMemberHugeRun = 4;
+constexpr int64_t kMemberHugeChunks = int64_t(1) << 18;
 constexpr int kMemberThreads = 1024;  // 16 waves share one staged table: 32 Ki edges per 32 KB copied
 // Two of the large work-groups share a compute unit, which takes at most 64 registers
 // a lane.  Runs of eight chunks, look-ups of four in flight, and the look-ups of
@@ -564,7 +567,7 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
 // are short), and the staged ids and places of all chunks are requested together
 // before anything is stored.  The work goes with the kept edges, not with all of
 // them: a lane per edge that looked its flag up took 88 us on 19 M edges of which
-// one in twenty-five is kept, and 84 on 29 M with one in four; this takes 34 and 69.
+// one in twenty-five is kept, and 84 on 29 M with one in four; this takes 32 and 59.
 // kEdgeMajor: the id on the other axis comes from edge_major (an edge list)
 // instead of the compressed pointer.
 // kView: the edges are those of a column slice read in place (without it none of
@@ -694,7 +697,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   if (nnz > 0) {
     const bool small = nnz < kMemberSmallEdges;
     const int threads = small ? kBlock : kMemberThreads;
-    const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberFlagRun;
+    const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberLongRun;
     int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
     // a large list, or work-groups that stage the 64 KB filter: as many of them as are
     // resident, each staging its tables once and striding over its runs
@@ -716,9 +719,9 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   } while (0)
 #define GS_MEMBER_FLAG(LDS)                                                                   \
   do {                                                                                        \
-    if (!small) GS_MEMBER_FLAG_IDS(LDS, kMemberThreads, kMemberFlagRun);                      \
+    if (!small) GS_MEMBER_FLAG_IDS(LDS, kMemberThreads, kMemberLongRun);                      \
     else if (run == 1) GS_MEMBER_FLAG_IDS(LDS, kBlock, 1);                                    \
-    else GS_MEMBER_FLAG_IDS(LDS, kBlock, kMemberFlagRun);                                     \
+    else GS_MEMBER_FLAG_IDS(LDS, kBlock, kMemberLongRun);                                     \
   } while (0)
     if (in_lds) GS_MEMBER_FLAG(true);
     else GS_MEMBER_FLAG(false);
@@ -757,7 +760,8 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
     return GS_ERR_WORKSPACE;
   }
   hipStream_t s = as_stream(stream);
-  const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberFillRun;
+  const int run = w.chunks <= kMemberShortChunks ? 1
+                  : w.chunks <= kMemberHugeChunks ? kMemberLongRun : kMemberHugeRun;
   const dim3 grid((unsigned)ceil_div(w.chunks, (kBlock / kWave) * run));
 #define GS_MEMBER_FILL_RUN(MAJOR, VIEW, RUN)                                           \
   GS_LAUNCH("member_fill", s,                                                          \
@@ -767,7 +771,8 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
 #define GS_MEMBER_FILL(MAJOR, VIEW)                                                    \
   do {                                                                                 \
     if (run == 1) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 1);                                  \
-    else GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberFillRun);                              \
+    else if (run == kMemberLongRun) GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberLongRun);   \
+    else GS_MEMBER_FILL_RUN(MAJOR, VIEW, kMemberHugeRun);                              \
   } while (0)
   if (view.sub_indptr != nullptr) {
     GS_REQUIRE(!edge_major, "minor_slice_fill: a slice read in place has no edge list");

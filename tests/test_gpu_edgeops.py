@@ -167,6 +167,40 @@ def test_sums_by_row_range_at_their_borders(nnz, R, targets):
     assert np.allclose(got.cpu().numpy().astype(np.float64), want, rtol=2e-6, atol=0)
 
 
+@pytest.mark.parametrize("E", [1, 255, 1023, 1024, 1025, 4096, 70_001])
+def test_one_value_an_edge_at_the_borders_of_a_tile(E):
+    """Scalar operators on an edge list, through every target and an edge map; the same kernel
+    without it reads the edge's own values."""
+    rng = np.random.default_rng(E)
+    row, col = rng.integers(0, 50, size=E), rng.integers(0, 70, size=E)
+    u, v, e = (rng.random(n, dtype=np.float32) + 0.5 for n in (50, 70, E))
+    of = {0: u, 1: e, 2: v}
+    for perm in (None, rng.permutation(E)):
+        for lt, rt in ((1, 0), (1, 2), (0, 2), (2, 0), (2, 1), (1, 1)):
+            got = capi.sddmm(("coo", T(row), T(col)), "div", T(of[lt]), T(of[rt]), lt, rt,
+                             edge_map=T(perm))
+            want = orc.sddmm(("coo", row, col), "div", of[lt], of[rt], lt, rt, edge_map=perm)
+            assert np.array_equal(got.cpu().numpy(), want)
+        got = capi.sddmm(("coo", T(row), T(col)), "copy_rhs", None, T(v), 1, 2, edge_map=T(perm))
+        assert np.array_equal(got.cpu().numpy(),
+                              orc.sddmm(("coo", row, col), "copy_rhs", None, v, 1, 2, edge_map=perm))
+
+
+@pytest.mark.parametrize("deg", [[2048], [2048, 2048], [1, 2047, 2049, 4095], [5000, 0, 0, 3, 9000],
+                                 [70_000_000, 5_000, 0, 3_000_000]])
+def test_column_sums_of_tiles_inside_one_column(deg):
+    """One, and from 67 M edges four, rounds of 2048 edges a tile, most tiles inside one column."""
+    rng = np.random.default_rng(len(deg))
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    e = rng.random(indptr[-1], dtype=np.float32) + np.float32(0.1)
+    ids = torch.zeros(indptr[-1], dtype=torch.int64, device=DEV)
+    want = np.array([e[a:b].astype(np.float64).sum() for a, b in zip(indptr, indptr[1:])])
+    got = capi.spmm(("csc", T(indptr), ids), "copy_rhs", "sum", None, T(e), 0, len(deg))
+    # a tile: 8 + 4 + 6 + 4 additions; up to 8 545 tiles of a column are added in any order,
+    # whose roundings of 2^-24 are independent: sqrt(8545) of them at most half an ulp each
+    assert np.allclose(got.cpu().numpy(), want, rtol=1e-5, atol=0)
+
+
 def test_matrix_sum_div_and_ops_wrappers(g):
     rng, indptr, indices, col = g
     m = gs.Matrix()

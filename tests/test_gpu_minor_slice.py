@@ -54,7 +54,7 @@ def test_minor_slice_with_a_table_outside_lds(npick):
 @pytest.mark.parametrize("npick", [200, 3000])
 @pytest.mark.parametrize("nnz", [1, 256, 257, 4096 * 256, 4096 * 256 + 1, (1 << 23) - 1, 1 << 23])
 def test_minor_slice_at_the_borders_of_a_waves_run(nnz, npick):
-    """Runs of one and of four chunks of 256 edges a wave, work-groups that stride over the runs,
+    """Runs of one and of two chunks of 256 edges a wave, work-groups that stride over the runs,
     with the table in LDS and outside."""
     rng = np.random.default_rng(nnz + npick)
     indptr = np.sort(rng.integers(0, nnz + 1, size=1201))
