@@ -211,10 +211,10 @@ __device__ __forceinline__ int64_t wave_segment_of(const int64_t* __restrict__ p
   return lo;
 }
 
-// Segments that a tile of consecutive positions [p0, p_last] touches.  The two
-// look-ups run once per wavefront on the scalar unit (p0 and p_last are the
-// same in every lane); a position of the tile is then searched only among the
-// segments in between, and not at all when one segment covers the tile.
+// Segments that a tile of consecutive positions [p0, p_last] touches.  The
+// look-ups run once per wavefront (p0 and p_last are the same in every lane, and
+// every lane must call this); a position of the tile is then searched only among
+// the segments in between, and not at all when one segment covers the tile.
 struct SegmentSpan {
   int64_t lo, hi;
   __device__ __forceinline__ int64_t segment_at(const int64_t* __restrict__ ptr,
@@ -224,6 +224,19 @@ struct SegmentSpan {
 };
 __device__ __forceinline__ SegmentSpan segment_span(const int64_t* __restrict__ ptr, int64_t n,
                                                     int64_t p0, int64_t p_last) {
+  SegmentSpan s;
+  const int64_t last = wave_uniform_first(p_last);
+  s.lo = wave_segment_of(ptr, n, wave_uniform_first(p0));
+  s.hi = ptr[s.lo + 1] > last ? s.lo : s.lo + wave_segment_of(ptr + s.lo, n - s.lo, last);
+  return s;
+}
+
+// The same on the scalar unit.  Where a launch streams at the rate of memory its
+// vector look-ups queue behind the stream and the scalar cache answers sooner: a
+// column slice of 602 M edges takes 3.54 ms so and 3.97 with the other, while the
+// column ids of as many edges took 1.20 ms so and take 0.83.
+__device__ __forceinline__ SegmentSpan segment_span_scalar(const int64_t* __restrict__ ptr,
+                                                           int64_t n, int64_t p0, int64_t p_last) {
   SegmentSpan s;
   s.lo = segment_of(ptr, n, wave_uniform_first(p0));
   s.hi = segment_of(ptr, n, wave_uniform_first(p_last));
@@ -269,8 +282,8 @@ struct SliceView {
   __device__ __forceinline__ bool on() const { return sub_indptr != nullptr; }
 
   // A run of consecutive slice edges [first, last], the same for every lane of
-  // the wavefront: the columns it touches are looked up once, on the scalar
-  // unit.  Columns worth slicing are long, so a run nearly always lies inside
+  // the wavefront: the columns it touches are looked up once, by all lanes
+  // together.  Columns worth slicing are long, so a run nearly always lies inside
   // one column or across the border of two neighbours: an edge's place in the
   // parent is then its number plus one of two distances, chosen by which side
   // of the border it is on, and nothing is searched or loaded per edge.  A run
@@ -308,10 +321,10 @@ struct SliceView {
     // in the same column, which one more look at the pointer tells
     const int64_t first_u = wave_uniform_first(first), last_u = wave_uniform_first(last);
     r.first = first_u;
-    r.span.lo = segment_of(sub_indptr, n, first_u);
+    r.span.lo = wave_segment_of(sub_indptr, n, first_u);
     r.span.hi = r.span.lo;
     if (sub_indptr[r.span.lo + 1] <= last_u)
-      r.span.hi = r.span.lo + segment_of(sub_indptr + r.span.lo, n - r.span.lo, last_u);
+      r.span.hi = r.span.lo + wave_segment_of(sub_indptr + r.span.lo, n - r.span.lo, last_u);
     r.split = INT64_MAX;
     r.shift[0] = r.shift[1] = r.offset[0] = r.offset[1] = 0;
     r.count = 0;

@@ -360,10 +360,7 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_kernel(
 constexpr int kSumItems = 8;
 constexpr int kSumTile = kBlock * kSumItems;
 constexpr int kSumSegs = 2048;   // segments one tile can accumulate in LDS
-// Edges per lane of the coordinate kernel: the short tile while it makes at most
-// as many work-groups as eight per compute unit.
-constexpr int kCooShortItems = 2;
-constexpr int64_t kCooShortEdges = int64_t(1) << 20;
+constexpr int kCooSlots = 4096;  // combining table of the coordinate kernel
 constexpr int kDies = 8;         // accelerator dies of an MI355X, one L2 each
 constexpr int64_t kPrivateMinEdges = 1 << 20;
 
@@ -458,13 +455,10 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_sum_kernel(
   // while the columns are looked up
   float val[kSumItems];
   load_round(tile0, val);
-  // both look-ups on the scalar unit; a long column covers the whole tile, and
-  // then the second one is a single comparison
-  const int64_t c0 = segment_of(indptr, num_major, wave_uniform_first(tile0));
-  const int64_t last = wave_uniform_first(tile_end - 1);
-  const int64_t c1 = indptr[c0 + 1] > last
-                         ? c0
-                         : c0 + segment_of(indptr + c0, num_major - c0, last);
+  // a long column covers the whole tile, and then the second look-up is a single
+  // comparison
+  const SegmentSpan columns = segment_span(indptr, num_major, tile0, tile_end - 1);
+  const int64_t c0 = columns.lo, c1 = columns.hi;
   if (c0 == c1) {
     // the whole tile lies inside one column: no accumulators to clear, one add
     float mine = 0.f;
@@ -548,20 +542,17 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_sum_kernel(
 
 // Coordinate form: outputs arrive in any order, so the tile combines them in
 // a small LDS hash table; an edge that finds no slot within a few probes adds
-// to memory directly.  Short lists take kItems = 2 edges a lane: tiles of 2048
-// left 150 thousand edges to 75 work-groups (42 us, a chain of look-ups, LDS
-// probes and one late burst of atomics in each).
-template <int kItems>
+// to memory directly.  What bounds it is the atomics, one per tile and row present:
+// tiles of 512 edges, for four times the work-groups on a short list, took 74 us on
+// 150 thousand edges of which a hub row draws many, where tiles of 2048 take 42.
 __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
     const int64_t* __restrict__ row, const int64_t* __restrict__ col,
     const int64_t* __restrict__ edge_map, int64_t nnz, int kind, int op,
     const float* __restrict__ ufeat, const float* __restrict__ efeat, float* out,
     int u_target, int64_t copy_stride, SliceView view) {
-  constexpr int kTile = kBlock * kItems;
-  constexpr int kSlots = 2 * kTile;  // at most half full
-  __shared__ long long keys[kSlots];
-  __shared__ float vals[kSlots];
-  for (int j = threadIdx.x; j < kSlots; j += kBlock) {
+  __shared__ long long keys[kCooSlots];
+  __shared__ float vals[kCooSlots];
+  for (int j = threadIdx.x; j < kCooSlots; j += kBlock) {
     keys[j] = -1;
     vals[j] = 0.f;
   }
@@ -569,7 +560,7 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
   // consecutive work-groups run on consecutive dies: with copy_stride > 0 every
   // die adds to a copy of its own
   out += (int64_t)(blockIdx.x % kDies) * copy_stride;
-  const int64_t tile0 = (int64_t)blockIdx.x * kTile;
+  const int64_t tile0 = (int64_t)blockIdx.x * kSumTile;
   const int64_t* dst_ids = u_target == 0 ? col : row;
   const int64_t* src_ids = u_target == 0 ? row : col;
   // all loads of the tile first, so that they are in flight together
@@ -578,11 +569,11 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
   SliceView::Run vrun{};
   vrun.split = INT64_MAX;  // no view: every edge at distance 0
   if (view.on() && tile0 < nnz)
-    vrun = view.run(tile0, (tile0 + kTile < nnz ? tile0 + kTile : nnz) - 1);
-  int64_t dst[kItems];
-  float val[kItems];
+    vrun = view.run(tile0, (tile0 + kSumTile < nnz ? tile0 + kSumTile : nnz) - 1);
+  int64_t dst[kSumItems];
+  float val[kSumItems];
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
+  for (int i = 0; i < kSumItems; ++i) {
     const int64_t e = tile0 + i * kBlock + threadIdx.x;
     dst[i] = -1;
     val[i] = 0.f;
@@ -596,7 +587,7 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
   }
   if (!vrun.near()) {
 #pragma unroll
-    for (int i = 0; i < kItems; ++i) {
+    for (int i = 0; i < kSumItems; ++i) {
       const int64_t e = tile0 + i * kBlock + threadIdx.x;
       int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
       const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
@@ -608,10 +599,10 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
     }
   }
 #pragma unroll
-  for (int i = 0; i < kItems; ++i) {
+  for (int i = 0; i < kSumItems; ++i) {
     if (dst[i] < 0) continue;
     uint32_t slot =
-        (uint32_t)(((uint64_t)dst[i] * 0x9E3779B97F4A7C15ull) >> 40) & (kSlots - 1);
+        (uint32_t)(((uint64_t)dst[i] * 0x9E3779B97F4A7C15ull) >> 40) & (kCooSlots - 1);
     bool placed = false;
     for (int probe = 0; probe < 8 && !placed; ++probe) {
       long long k = keys[slot];
@@ -621,28 +612,22 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
         atomicAdd(&vals[slot], val[i]);
         placed = true;
       }
-      slot = (slot + 1) & (kSlots - 1);
+      slot = (slot + 1) & (kCooSlots - 1);
     }
     if (!placed) unsafeAtomicAdd(out + dst[i], val[i]);
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < kSlots; j += kBlock)
+  for (int j = threadIdx.x; j < kCooSlots; j += kBlock)
     if (keys[j] != -1) unsafeAtomicAdd(out + keys[j], vals[j]);
 }
 
 static int coo_sum_launch(const int64_t* row, const int64_t* col, const int64_t* edge_map,
                           int64_t nnz, int kind, int op, const float* ufeat, const float* efeat,
                           float* out, int u_target, SliceView view, hipStream_t s) {
-  const bool few = nnz < kCooShortEdges;
-  const dim3 grid((unsigned)ceil_div(nnz, (int64_t)kBlock * (few ? kCooShortItems : kSumItems)));
-  if (few)
-    GS_LAUNCH("spmm_coo_sum", s,
-              spmm_coo_sum_kernel<kCooShortItems><<<grid, dim3(kBlock), 0, s>>>(
-                  row, col, edge_map, nnz, kind, op, ufeat, efeat, out, u_target, (int64_t)0, view));
-  else
-    GS_LAUNCH("spmm_coo_sum", s,
-              spmm_coo_sum_kernel<kSumItems><<<grid, dim3(kBlock), 0, s>>>(
-                  row, col, edge_map, nnz, kind, op, ufeat, efeat, out, u_target, (int64_t)0, view));
+  GS_LAUNCH("spmm_coo_sum", s,
+            spmm_coo_sum_kernel<<<dim3((unsigned)ceil_div(nnz, (int64_t)kSumTile)), dim3(kBlock), 0,
+                                  s>>>(row, col, edge_map, nnz, kind, op, ufeat, efeat, out,
+                                       u_target, (int64_t)0, view));
   return GS_OK;
 }
 
@@ -1103,7 +1088,7 @@ static int spmm_launch(int format, const int64_t* a, const int64_t* b,
                   spmm_zero_kernel<<<dim3((unsigned)zb), dim3(kBlock), 0, s>>>(
                       copies, total));
         GS_LAUNCH("spmm_coo_sum", s,
-                  spmm_coo_sum_kernel<kSumItems><<<grid, dim3(kBlock), 0, s>>>(
+                  spmm_coo_sum_kernel<<<grid, dim3(kBlock), 0, s>>>(
                       a, b, edge_map, nnz, kind, op, ufeat, efeat, copies,
                       u_target, num_out, no_view()));
         GS_LAUNCH("spmm_fold", s,

@@ -400,7 +400,7 @@ void member_flag_kernel(
   for (int64_t run = (int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave;
        run < num_runs; run += (int64_t)gridDim.x * (kThreads / kWave)) {
   // With a view the edges are those of a column slice that was never written:
-  // the run's columns are looked up once, on the scalar unit, and an edge's id
+  // the run's columns are looked up once, and an edge's id
   // is read from the parent's array.
   SliceView::Run vrun{};
   vrun.split = INT64_MAX;  // no view: every edge at distance 0, offset 0
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
 
 // A wave writes the kept edges of kRun consecutive chunks: how many each has comes
 // from the chunk offsets, the columns of the wave's first and last edge take a
-// search each on the scalar unit (one column covers the whole span unless columns
+// search each (one column covers the whole span unless columns
 // are short), and the staged ids and places of all chunks are requested together
 // before anything is stored.  The work goes with the kept edges, not with all of
 // them: a lane per edge that looked its flag up took 88 us on 19 M edges of which

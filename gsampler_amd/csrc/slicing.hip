@@ -126,6 +126,8 @@ __global__ __launch_bounds__(kCountThreads) void col_count_small_kernel(
 // writes are coalesced.
 constexpr int kSliceItems = 4;
 constexpr int kSliceTile = kBlock * kSliceItems;
+// Work-groups from which a launch streams at the rate of memory (see segment_span_scalar).
+constexpr unsigned kSliceStreams = 65536;
 
 __global__ __launch_bounds__(kBlock) void col_slice_fill_kernel(
     const int64_t* __restrict__ indptr, const int64_t* __restrict__ indices, const int64_t* __restrict__ column_ids,
@@ -136,9 +138,11 @@ __global__ __launch_bounds__(kBlock) void col_slice_fill_kernel(
   const int64_t e0 = (int64_t)blockIdx.x * kSliceTile;
   if (e0 >= nnz) return;
   const int64_t e_last = e0 + kSliceTile - 1 < nnz ? e0 + kSliceTile - 1 : nnz - 1;
-  // columns that the tile touches: one search per work-group (on the scalar
-  // unit) instead of one per edge; a long column covers whole tiles
-  const SegmentSpan span = segment_span(sub_indptr, num_items, e0, e_last);
+  // columns that the tile touches: one search per wavefront instead of one
+  // per edge; a long column covers whole tiles
+  const SegmentSpan span = gridDim.x < kSliceStreams
+                               ? segment_span(sub_indptr, num_items, e0, e_last)
+                               : segment_span_scalar(sub_indptr, num_items, e0, e_last);
   if (span.lo == span.hi && e0 + kSliceTile <= nnz &&
       (((uintptr_t)out_indices | (uintptr_t)out_select | (uintptr_t)out_coo_col) & 15) == 0) {
     // a whole tile out of one column: two edges (16 bytes) per lane and
@@ -214,7 +218,9 @@ __global__ __launch_bounds__(kBlock) void col_slice_values_kernel(
   const int64_t e0 = (int64_t)blockIdx.x * kValueTile;
   if (e0 >= nnz) return;
   const int64_t e_last = e0 + kValueTile - 1 < nnz ? e0 + kValueTile - 1 : nnz - 1;
-  const SegmentSpan span = segment_span(sub_indptr, num_items, e0, e_last);
+  const SegmentSpan span = gridDim.x < kSliceStreams
+                               ? segment_span(sub_indptr, num_items, e0, e_last)
+                               : segment_span_scalar(sub_indptr, num_items, e0, e_last);
   // one column covers the tile (columns of a slice worth copying are long): its
   // offset is the same for every edge
   int64_t shift = 0;
