@@ -47,7 +47,7 @@ struct EdgeView {
   int64_t num_major;   // segments of indptr
   const int64_t* edge_map;
   // Segments that the edges [e_first, e_last] of one work-group touch
-  // (compressed form only): looked up once, on the scalar unit.
+  // (compressed form only): looked up once per wavefront.
   __device__ __forceinline__ SegmentSpan span(int64_t e_first, int64_t e_last) const {
     if (!compressed) return SegmentSpan{0, 0};
     return segment_span(a, num_major, e_first, e_last);
@@ -641,11 +641,11 @@ static int coo_sum_launch(const int64_t* row, const int64_t* col, const int64_t*
 // cells, (2) a work-group per range cuts the tiles into units of about 32 Ki of
 // its entries, (3) a work-group sums a unit in LDS and stores kRangeRows partial
 // sums, (4) the partial sums of a range are folded into the output.  The edges are
-// read once, nothing is counted beforehand, and no pass but the fold uses an
-// atomic on device memory.  The floor is 8 + 6 bytes an edge through pass 1 and
+// read once, nothing is counted beforehand, and no pass uses an atomic on device
+// memory.  The floor is 8 + 6 bytes an edge through pass 1 and
 // 6 + the rate of fp64 adds in LDS through pass 3.  On a slice of 29 M edges and
 // 233 K rows a counting pass, a scan, and a scatter of 8-byte pairs to places
-// chosen by the scan took 353 us, with the sums; this takes 193 (part 106, sums 66).
+// chosen by the scan took 353 us, with the sums; this takes 190 (part 106, sums 64, fold 10).
 constexpr int kRangeShift = 13;
 constexpr int kRangeRows = 1 << kRangeShift;  // 64 KB of LDS accumulators
 constexpr int kMaxRanges = 1024;
@@ -988,29 +988,53 @@ __global__ __launch_bounds__(kAccThreads, 8) void rowsum_accumulate_kernel(
 
 // out[row] += the row's partial sums over all units of its range.  Ranges
 // differ a lot in how many units they have (the rows of hubs sit in one range
-// and draw half of the edges), so the units of a range are dealt out over
-// gridDim.y work-groups per block of rows, which add their shares atomically.
-constexpr int kFoldSplit = 8;
+// and draw half of the edges), so a work-group takes 128 rows, four a lane, and its
+// eight groups of 32 lanes a share of the units each: a range of 500 units is 63
+// loads deep.  The shares are added in double and the row is rounded once.  (A
+// work-group per share whose shares met in eight float atomics a row took 11.7 us on
+// 233 K rows with 32 units a range and 22 on 1.67 M rows with four; this takes
+// 9.9 and 13.)
+constexpr int kFoldLanes = 32;
+constexpr int kFoldRows = 4 * kFoldLanes;
+constexpr int kFoldShares = kBlock / kFoldLanes;
+static_assert(kRangeRows % kFoldRows == 0, "the rows of a work-group share a range");
 
 __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
     const float* __restrict__ partial, const RangeUnits* __restrict__ range_units,
     int64_t num_out, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= num_out) return;
-  const RangeUnits ru = range_units[i >> kRangeShift];  // uniform over the work-group
-  const int64_t u1 = (int64_t)ru.base + ru.count, step = gridDim.y;
-  const float* p = partial + (i & (kRangeRows - 1));
-  float acc = 0.f;
-  int64_t u = (int64_t)ru.base + blockIdx.y;
-  for (; u + 7 * step < u1; u += 8 * step) {  // eight loads in flight
-    float v[8];
+  __shared__ double share_sum[kFoldShares][kFoldRows];
+  const int share = threadIdx.x / kFoldLanes, lane_row = threadIdx.x % kFoldLanes * 4;
+  const int64_t row0 = (int64_t)blockIdx.x * kFoldRows;
+  const RangeUnits ru = range_units[row0 >> kRangeShift];
+  const int64_t u1 = (int64_t)ru.base + ru.count;
+  // (a unit has the sums of all rows of its range, also of those past num_out)
+  const float* p = partial + (row0 & (kRangeRows - 1)) + lane_row;
+  auto sums_of = [&](int64_t u) { return *reinterpret_cast<const float4*>(p + u * kRangeRows); };
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  auto add = [&](const float4& v) {
+    acc[0] += (double)v.x;
+    acc[1] += (double)v.y;
+    acc[2] += (double)v.z;
+    acc[3] += (double)v.w;
+  };
+  int64_t u = (int64_t)ru.base + share;
+  for (; u + 7 * kFoldShares < u1; u += 8 * kFoldShares) {  // eight loads in flight
+    float4 v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = p[(u + k * step) * kRangeRows];
+    for (int k = 0; k < 8; ++k) v[k] = sums_of(u + k * kFoldShares);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc += v[k];
+    for (int k = 0; k < 8; ++k) add(v[k]);
   }
-  for (; u < u1; u += step) acc += p[u * kRangeRows];
-  if (acc != 0.f) unsafeAtomicAdd(out + i, acc);
+  for (; u < u1; u += kFoldShares) add(sums_of(u));
+#pragma unroll
+  for (int k = 0; k < 4; ++k) share_sum[share][lane_row + k] = acc[k];
+  __syncthreads();
+  const int64_t i = row0 + threadIdx.x;
+  if (threadIdx.x >= kFoldRows || i >= num_out) return;
+  double sum = 0.0;
+#pragma unroll
+  for (int s = 0; s < kFoldShares; ++s) sum += share_sum[s][threadIdx.x];
+  if (sum != 0.0) out[i] += (float)sum;
 }
 
 // dst_ids32: the same ids as dst_ids in 32 bits (a matrix's narrow copy), read
@@ -1045,8 +1069,8 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
             rowsum_accumulate_kernel<<<dim3((unsigned)p.max_units), dim3(kAccThreads), 0, s>>>(
                 rows, values, cells, p.tile_stride, units, unit_total, partial));
   GS_LAUNCH("rowsum_fold", s,
-            rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kBlock), kFoldSplit),
-                                 dim3(kBlock), 0, s>>>(partial, range_units, num_out, out));
+            rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
+                                 s>>>(partial, range_units, num_out, out));
   return GS_OK;
 }
 

@@ -372,7 +372,7 @@ __global__ __launch_bounds__(kReplThreads) void sample_weighted_replace_kernel(
 // 128-byte line per pick for the row id and two for the ends of the column's
 // slice of a global prefix sum.)
 // Both passes take tiles of consecutive edges and look the tile's first and
-// last column up once, on the scalar unit; an edge then searches only among
+// last column up once per wavefront; an edge then searches only among
 // the columns of its tile instead of all of them.
 constexpr int kCdfItems = 8;
 constexpr int kCdfTile = kBlock * kCdfItems;

@@ -150,8 +150,8 @@ def test_scalar_sums_on_skewed_matrices(shape):
 ])
 def test_sums_by_row_range_at_their_borders(nnz, R, targets):
     """Against float64 sums.  A unit of at most 40 960 edges is summed in double and rounded
-    once; a row's units and the eight shares of its fold are added in float: for the hub,
-    5e6 / 32768 = 153 units in shares of 20, at most 29 roundings of 2^-24 = 1.8e-6."""
+    once, a row's units are added in double and rounded once: well inside 2e-6, the bound of
+    units added in float (153 of them for the hub, in eight shares of 20)."""
     rng = np.random.default_rng(nnz + R)
     ids = rng.integers(0, R, size=nnz)
     if targets == "sorted":
