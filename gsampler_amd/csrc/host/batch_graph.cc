@@ -245,7 +245,8 @@ torch::Tensor Graph::batch_rows_for_relabel(const torch::Tensor& edge_rows,
 // of the frontier, as every caller is about to do.
 Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_seeds,
                                                      const torch::Tensor& row_ids,
-                                                     const ColumnOrderedEdges& edges) {
+                                                     const ColumnOrderedEdges& edges,
+                                                     bool want_labels) {
   const int64_t R = row_ids.numel(), S = col_seeds.numel(), E = edges.row.numel();
   const int64_t B = col_bptr_.numel() - 1;
   if (R == 0 || S == 0 || R != num_rows_ || S != num_cols_ || !edges.col.defined() ||
@@ -257,7 +258,8 @@ Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_se
       batch_list_labels_->seeds.is_same(col_seeds) &&
       batch_list_labels_->row_ids_version == (int64_t)row_ids._version() &&
       batch_list_labels_->seeds_version == (int64_t)col_seeds._version() &&
-      batch_list_labels_->epoch == cache_epoch())
+      batch_list_labels_->epoch == cache_epoch() &&
+      (batch_list_labels_->refused || !want_labels || batch_list_labels_->row.defined()))
     return batch_list_labels_->refused ? nullptr : batch_list_labels_.get();
   auto out = std::make_unique<BatchListLabels>();
   out->base = edges.row;
@@ -313,9 +315,11 @@ Graph::Frontier& Graph::batch_relabel_launch(torch::Tensor& col_seeds,
     TORCH_CHECK(edges.col_indptr.numel() == col_seeds.numel() + 1,
                 "BatchGraphRelabel: ", col_seeds.numel(), " seeds for a matrix of ",
                 edges.col_indptr.numel() - 1, " columns");
-  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges)) {
-    *out_row = l->row;
-    *out_col = l->col;
+  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges, true)) {
+    // handed out once: they are the caller's to change
+    *out_row = std::move(l->row);
+    *out_col = std::move(l->col);
+    l->row = l->col = torch::Tensor();
     if (e_ids) *e_ids = edges.e_ids;
     return l->frontier;
   }
@@ -358,7 +362,7 @@ std::tuple<torch::Tensor, torch::Tensor> Graph::BatchGetValidNodes(
   ColumnOrderedEdges edges = column_ordered_edges("BatchGetValidNodes");
   col_seeds = ids(col_seeds, "col_seeds");
   BatchOffsets::check(col_bptr_, col_seeds.numel(), "BatchGetValidNodes");
-  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges))
+  if (BatchListLabels* l = batch_list_labels_for(col_seeds, row_ids, edges, false))
     return {l->frontier.frontier(), l->frontier.unique_ptr};
   torch::Tensor rows = batch_rows_for_relabel(edges.row, row_ids);
   Frontier& f = frontier_for(col_seeds, rows, col_bptr_, edge_bptr_);

@@ -424,14 +424,14 @@ class Graph : public torch::CustomClassHolder {
   struct BatchListLabels {
     torch::Tensor base, row_ids, seeds;
     int64_t row_ids_version = -1, seeds_version = -1, epoch = -1;
-    torch::Tensor row, col;
+    torch::Tensor row, col;  // until a caller takes them
     Frontier frontier;
     bool refused = false;  // the general path serves this matrix
   };
   std::unique_ptr<BatchListLabels> batch_list_labels_;
   BatchListLabels* batch_list_labels_for(const torch::Tensor& col_seeds,
                                          const torch::Tensor& row_ids,
-                                         const ColumnOrderedEdges& edges);
+                                         const ColumnOrderedEdges& edges, bool want_labels);
   bool use_list_labels(const torch::Tensor& col_seeds, const torch::Tensor& row_ids) const;
   ListLabels& list_labels_for(const torch::Tensor& col_seeds, const torch::Tensor& row_ids);
 };

@@ -104,6 +104,10 @@ def test_batched_labels_by_way_of_the_list(sizes, picks, mode):
         if not nodes_first:
             nodes, nodes_ptr = part._CAPI_BatchGetValidNodes(d_seeds, row_ids)
         assert torch.equal(nodes, frontier) and torch.equal(nodes_ptr, uptr)
+        kept = [row.clone(), col.clone()]
+        row.zero_(), col.zero_()          # the caller's own: the next call does not return them
+        frontier, uptr, row, col, _, eptr = part._CAPI_BatchGraphRelabel(d_seeds, row_ids)
+        assert torch.equal(row, kept[0]) and torch.equal(col, kept[1])
         keys = row_ids[part._CAPI_GetCOORows()].cpu().numpy()
         at_col = part._CAPI_GetCOOCols().cpu().numpy()
         frontier, uptr, row, col, eptr = (x.cpu().numpy() for x in (frontier, uptr, row, col, eptr))
