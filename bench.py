@@ -524,9 +524,8 @@ def ladies_kernel_bytes(name, sizes, num_rows):
             "col_slice_fill": 24 * S + 32 * nnz,          # seeds, indptr pair, row id in; 3 outputs
             "gather_rows": 16 * nnz + 16 * kept,          # edge data of both slices: index + value in, value out
             "member_flag": 8 * nnz,                       # row id of every edge
-            "member_fill": 4 * kept + 24 * kept,          # staged ids in; row, column, position out
-            "rowsum_hist": 8 * nnz, "rowsum_scatter": 12 * nnz + 8 * nnz,
-            "rowsum_accumulate": 8 * nnz + 4 * num_rows,
+            "member_fill": 5 * kept + 24 * kept,          # staged ids and places in; row, column, position out
+            "rowsum_part": 8 * nnz + 6 * nnz, "rowsum_accumulate": 6 * nnz + 4 * num_rows,
             "spmm_coo_sum": 12 * nnz + 4 * num_rows,
             "spmm_csc_sum": 4 * kept + 4 * S,
             "sddmm": 2 * 20 * kept,                       # two quotients: value, id and operand in, value out
