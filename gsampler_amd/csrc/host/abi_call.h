@@ -49,6 +49,16 @@ inline gs_stream_t cur_stream() {
   return (gs_stream_t)c10::hip::getCurrentHIPStream().stream();
 }
 
+// Whether the current stream's work is being recorded into a graph instead of run.
+inline bool capturing() {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)cur_stream(), &status) != hipSuccess) {
+    (void)hipGetLastError();  // asked of the default stream while another one is recorded
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 // int64 CUDA tensor, contiguous; the reference aborts on anything else
 // (src/graph_ops.cc:28 "Not implemented warning"), this raises instead.
 inline torch::Tensor ids(const torch::Tensor& t, const char* name) {

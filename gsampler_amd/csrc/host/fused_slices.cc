@@ -76,7 +76,7 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
   torch::Tensor ws = new_workspace(gs_sliced_e_square_sum_workspace_bytes(so.nnz, num_rows_),
                                    m.indptr);
   const torch::Tensor e_ids = m.e_ids.has_value() ? m.e_ids.value() : torch::Tensor();
-  const torch::Tensor& narrow = m.narrow_indices();  // half the bytes behind every id
+  const torch::Tensor narrow = m.narrow_indices();  // half the bytes behind every id
   GS_CALL(gs_sliced_e_square_sum(cptr(m.indptr), cptr(m.indices),
                                  narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
                                  cptr(cols), cols.numel(),
@@ -99,7 +99,7 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
   // is queued into buffers sized by the bound (every edge kept) and runs while
   // the number travels
   AsyncCount kept = AsyncCount::mirrored();
-  const torch::Tensor& narrow = m.narrow_indices();  // half the bytes behind every id
+  const torch::Tensor narrow = m.narrow_indices();  // half the bytes behind every id
   GS_CALL(gs_col_row_slice_count(cptr(m.indptr), cptr(m.indices),
                                  narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
                                  cptr(cols), cptr(key_offset),
@@ -138,7 +138,7 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
                       output_format & kCOO);
   } else {
     const MajorResult& sliced = written_slice(cols);
-    Compressed tmp{sliced.indptr, sliced.minor_ids, c10::nullopt};
+    Compressed tmp(sliced.indptr, sliced.minor_ids);
     r = minor_slice(tmp, rows, output_format & kCOO);
     r.select = sliced.select.index_select(0, r.select);
   }
@@ -180,7 +180,7 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
     // short columns: the batched column slice with rows moved by batch * num_rows
     // is written and row-sliced
     MajorResult sliced = major_slice(m, col, false, col_bptr, stride);
-    Compressed tmp{sliced.indptr, sliced.minor_ids, c10::nullopt};
+    Compressed tmp(sliced.indptr, sliced.minor_ids);
     kept = minor_slice(tmp, picked, false);
     kept.select = sliced.select.index_select(0, kept.select);
   }

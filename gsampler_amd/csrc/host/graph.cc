@@ -222,27 +222,34 @@ MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
   return r;
 }
 
+Compressed::Derived& Compressed::current_derived() const {
+  const int64_t versions[2] = {(int64_t)indptr._version(), (int64_t)indices._version()};
+  Derived& d = derived_;
+  if (d.versions[0] != versions[0] || d.versions[1] != versions[1] || d.epoch != cache_epoch() ||
+      d.source != indices.data_ptr()) {  // edited, or another array
+    d.drop();
+    d.versions[0] = versions[0];
+    d.versions[1] = versions[1];
+    d.epoch = cache_epoch();
+    d.source = indices.data_ptr();
+  }
+  return d;
+}
+
 // The int32 copy pays from a few megabytes of ids on (below that the int64
 // array stays in cache anyway); undefined when the matrix does not qualify.
-const torch::Tensor& Compressed::narrow_indices() const {
+torch::Tensor Compressed::narrow_indices() const {
   constexpr int64_t kMinEdges = int64_t(1) << 20;
-  // one matrix is shared by every handle derived from it and by every sampler
-  // thread: the copy is made (and dropped) under a lock
-  static std::mutex guard;
-  std::lock_guard<std::mutex> lock(guard);
-  const int64_t version = (int64_t)indices._version();
-  if (indices32.defined() &&
-      (indices32_version != version || indices32_source != indices.data_ptr() ||
-       indices32_epoch != cache_epoch() || !narrow_ids_allowed().load()))
-    indices32 = torch::Tensor();  // edited, another array, or switched off
-  if (!indices32.defined() && narrow_ids_allowed().load() && num_minor >= 0 &&
-      num_minor < (int64_t(1) << 31) && indices.is_cuda() && indices.numel() >= kMinEdges) {
-    indices32 = indices.to(torch::kInt32);
-    indices32_version = version;
-    indices32_epoch = cache_epoch();
-    indices32_source = indices.data_ptr();
-  }
-  return indices32;
+  if (indices.numel() < kMinEdges || num_minor < 0 || num_minor >= (int64_t(1) << 31) ||
+      !indices.is_cuda() || capturing())
+    return {};
+  std::lock_guard<std::mutex> lock(derived_.guard);
+  Derived& d = current_derived();
+  if (!narrow_ids_allowed().load())
+    d.narrow.drop();
+  else if (!d.narrow.defined())
+    d.narrow.set(indices.to(torch::kInt32));
+  return d.narrow.on_current_stream();
 }
 
 // picked undefined: sample every column of the matrix itself.
@@ -284,7 +291,7 @@ MajorResult major_sample_uniform(const Compressed& m,
   int64_t* out_col = with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr;
   const int64_t* col_batch_ptr = label_cols ? cptr(hint.col_bptr) : nullptr;
   const int64_t col_batches = label_cols ? hint.col_bptr.numel() - 1 : 0;
-  const torch::Tensor& narrow = m.narrow_indices();
+  const torch::Tensor narrow = m.narrow_indices();
   if (narrow.defined()) {
     GS_CALL(gs_csc_col_sample_uniform_fill_i32(
         cptr(m.indptr), num_major, narrow.data_ptr<int32_t>(),

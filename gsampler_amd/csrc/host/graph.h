@@ -9,6 +9,8 @@
 #include <torch/custom_class.h>
 #include <torch/script.h>
 
+#include <c10/hip/HIPCachingAllocator.h>
+
 #include "abi_call.h"
 
 #include <functional>
@@ -23,6 +25,38 @@ namespace gs {
 // Format bit flags (src/graph_storage.h:31-33).
 constexpr int64_t kCOO = 1, kCSC = 2, kCSR = 4;
 
+// A table that operators derive from a matrix on first use and keep with it.  The
+// kernel that fills it is queued on the stream of whoever asked first, and its memory
+// belongs to that stream: a caller on another one waits for it once, on the host, and
+// announces to the allocator that it reads there.  (An event behind the kernel would
+// spare that wait and cost every first use a gap on the device.)
+class DerivedTable {
+ public:
+  bool defined() const { return table_.defined(); }
+  void drop() { table_ = torch::Tensor(); }
+  void set(torch::Tensor t) {
+    table_ = std::move(t);
+    made_on_ = cur_stream();
+    complete_ = false;
+  }
+  torch::Tensor on_current_stream() {
+    if (!table_.defined() || made_on_ == cur_stream()) return table_;
+    if (!complete_) {
+      const hipError_t e = hipDeviceSynchronize();
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+      complete_ = true;
+    }
+    c10::hip::HIPCachingAllocator::recordStream(table_.storage().data_ptr(),
+                                                c10::hip::getCurrentHIPStream());
+    return table_;
+  }
+
+ private:
+  torch::Tensor table_;
+  gs_stream_t made_on_ = nullptr;
+  bool complete_ = false;
+};
+
 // CSC or CSR: `indptr` over the compressed ("major") axis, `indices` holds the
 // ids on the other ("minor") axis.
 struct Compressed {
@@ -31,27 +65,43 @@ struct Compressed {
   // Exclusive bound of the ids in `indices` when it is known (a loaded or
   // converted matrix), else -1.
   int64_t num_minor = -1;
-  // int32 copy of `indices` for the uniform sampler (half the bytes behind
-  // every random pick); made on the first sampling call of a matrix in device
-  // memory whose ids fit.
-  mutable torch::Tensor indices32;
-  mutable int64_t indices32_version = -1;  // version of `indices` the copy was made from
-  mutable int64_t indices32_epoch = -1;    // and the cache epoch (invalidate_caches)
-  mutable const void* indices32_source = nullptr;  // and its address
-  const torch::Tensor& narrow_indices() const;
+  // Both tables below belong to the ids they were made from: their version, the cache
+  // epoch (invalidate_caches) and their address.  Neither is made or handed out while
+  // the current stream is being captured: the graph would record the kernel that fills
+  // the table, or read one that a later edit of the matrix frees.
+  //
+  // int32 copy of `indices` (half the bytes behind every random pick); made on the
+  // first sampling call of a matrix in device memory whose ids fit.
+  torch::Tensor narrow_indices() const;
   // Where the column behind every edge lies (gs_hop_table), for walks over a
   // square matrix; made at the second walk over the same matrix.
-  mutable torch::Tensor hops;
-  mutable int64_t hops_versions[2] = {-1, -1}, hops_epoch = -1, hops_asked = 0;
-  mutable const void* hops_source = nullptr;
-  mutable gs_stream_t hops_stream = nullptr;
-  const torch::Tensor& hop_table() const;
+  torch::Tensor hop_table() const;
+  struct Derived {
+    std::mutex guard;  // a matrix is shared by every handle and sampler thread
+    DerivedTable narrow, hops;
+    int64_t versions[2] = {-1, -1}, epoch = -1;
+    const void* source = nullptr;
+    int64_t walks = 0;
+    void drop() {
+      narrow.drop();
+      hops.drop();
+      walks = 0;
+    }
+  };
+  Compressed() = default;
+  Compressed(torch::Tensor indptr, torch::Tensor indices)
+      : indptr(std::move(indptr)), indices(std::move(indices)) {}
+  Compressed(const Compressed& o)  // derived tables stay with the matrix they were made for
+      : indptr(o.indptr), indices(o.indices), e_ids(o.e_ids), num_minor(o.num_minor) {}
   // Call after assigning another `indices` or `indptr` to a matrix that was used.
   void forget_derived() {
-    indices32 = torch::Tensor();
-    hops = torch::Tensor();
-    hops_asked = 0;
+    std::lock_guard<std::mutex> lock(derived_.guard);
+    derived_.drop();
   }
+
+ private:
+  mutable Derived derived_;
+  Derived& current_derived() const;  // called under the lock: aged tables dropped
 };
 
 struct Coordinate {

@@ -103,7 +103,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
   auto fits = [&](int64_t columns, int64_t fanout, int64_t most) {
     return small_ok && columns > 0 && fanout >= 1 && fanout < 64 && columns <= most / (fanout + 1);
   };
-  const torch::Tensor& narrow = m.narrow_indices();
+  const torch::Tensor narrow = m.narrow_indices();
   const size_t L = fanouts.size();
   for (;;) {
     std::vector<Layer> out(L);

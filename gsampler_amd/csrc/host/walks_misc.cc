@@ -8,32 +8,20 @@ namespace gs {
 // Kept for matrices of up to 2^24 edges (128 MB): there it stays in the last-level
 // cache, and making it costs a fraction of a walk.  A matrix that is walked once
 // never makes it.
-const torch::Tensor& Compressed::hop_table() const {
+torch::Tensor Compressed::hop_table() const {
   constexpr int64_t kMaxEdges = int64_t(1) << 24;
-  static std::mutex guard;
-  std::lock_guard<std::mutex> lock(guard);
-  const int64_t versions[2] = {(int64_t)indptr._version(), (int64_t)indices._version()};
-  if (hops_versions[0] != versions[0] || hops_versions[1] != versions[1] ||
-      hops_epoch != cache_epoch() || hops_source != indices.data_ptr()) {
-    hops = torch::Tensor();
-    hops_asked = 0;
-    hops_versions[0] = versions[0];
-    hops_versions[1] = versions[1];
-    hops_epoch = cache_epoch();
-    hops_source = indices.data_ptr();
-  }
   const int64_t nnz = indices.numel();
-  if (!hops.defined() && hops_asked++ > 0 && indices.is_cuda() && indptr.is_cuda() && nnz > 0 &&
-      nnz <= kMaxEdges) {
+  if (nnz == 0 || nnz > kMaxEdges || !indices.is_cuda() || !indptr.is_cuda() || capturing())
+    return {};
+  std::lock_guard<std::mutex> lock(derived_.guard);
+  Derived& d = current_derived();
+  if (!d.hops.defined() && d.walks++ > 0) {
     torch::Tensor t = new_ids(nnz, indices);
     GS_CALL(gs_hop_table(cptr(indptr), indptr.numel() - 1, cptr(indices), nnz, t.data_ptr(),
                          cur_stream()));
-    hops = t;
-    hops_stream = cur_stream();
+    d.hops.set(t);
   }
-  // (another stream may run ahead of the kernel that makes it: it walks without)
-  static const torch::Tensor none;
-  return hops.defined() && hops_stream == cur_stream() ? hops : none;
+  return d.hops.on_current_stream();
 }
 
 // Traces are stored step-major ([walk_length + 1][num_seeds] in memory) and
@@ -47,7 +35,7 @@ torch::Tensor Graph::RandomWalk(torch::Tensor seeds, int64_t walk_length) {
   const int64_t n = seeds.numel();
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
-  const torch::Tensor& hops = csc_->hop_table();
+  const torch::Tensor hops = csc_->hop_table();
   GS_CALL(gs_random_walk_hops(cptr(csc_->indptr), cptr(csc_->indices), cptr(hops), num_cols_,
                               cptr(seeds), n, walk_length, rs.seed, next_call_id(), mptr(out),
                               cur_stream()));
@@ -79,8 +67,8 @@ torch::Tensor Graph::Node2Vec(torch::Tensor seeds, int64_t walk_length, double p
   const int64_t n = seeds.numel();
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
-  const torch::Tensor& narrow = csc_->narrow_indices();  // half the bytes behind every candidate
-  const torch::Tensor& hops = csc_->hop_table();
+  const torch::Tensor narrow = csc_->narrow_indices();  // half the bytes behind every candidate
+  const torch::Tensor hops = csc_->hop_table();
   GS_CALL(gs_node2vec_hops(cptr(csc_->indptr), cptr(csc_->indices),
                            narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(hops),
                            num_cols_, cptr(seeds), n, walk_length, p, q, rs.seed, next_call_id(),
