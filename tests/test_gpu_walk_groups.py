@@ -59,3 +59,31 @@ def test_random_walk(world, n, length):
     with torch.cuda.stream(side):            # a stream that did not make the table
         gs.manual_seed(13)
         assert np.array_equal(traces(m.random_walk(d, length), n), want.reshape(length + 1, n))
+
+
+# From 2^20 edges on a walk reads the int32 copy of the ids: the same group sizes, below and
+# above 2^15 walks (with and without the hop table, which a matrix up to 2^24 edges keeps).
+@pytest.fixture(scope="module")
+def wide_world():
+    rng = np.random.default_rng(8)
+    nodes = 130_000
+    indptr, indices = random_csc(rng, nodes, nodes, 17, empty_frac=0.02, hub_deg=70000)
+    assert 1 << 20 <= indices.size <= 1 << 24
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    return rng, nodes, indptr, m.csc[1].cpu().numpy(), m
+
+
+@pytest.mark.parametrize("n,length,p,q", [
+    (333, 18, 2.0, 0.5), (12501, 17, 2.0, 0.5), (25001, 9, 2.0, 0.5), (50001, 6, 2.0, 0.5),
+    (100001, 5, 2.0, 0.5), (200001, 4, 2.0, 0.5), (25000, 5, 0.25, 4.0), (32769, 5, 0.25, 4.0),
+    (200001, 4, 1.0, 1.0),
+])
+def test_node2vec_on_int32_ids(wide_world, n, length, p, q):
+    test_node2vec(wide_world, n, length, p, q)
+
+
+@pytest.mark.parametrize("n,length", [(1000, 17), (32768, 9), (40000, 8)])
+def test_random_walk_on_a_wide_matrix(wide_world, n, length):
+    test_random_walk(wide_world, n, length)
