@@ -415,7 +415,9 @@ class Graph : public torch::CustomClassHolder {
                              const torch::Tensor& efeat, const torch::Tensor& out,
                              int64_t u_target, const char* who) const;
   bool csc_sorted_ = false;  // row ids known to be sorted inside every column
-  torch::Tensor cdf_, cdf_probs_;
+  std::mutex cdf_guard_;
+  DerivedTable cdf_;
+  torch::Tensor cdf_probs_;
   int64_t cdf_version_ = -1, cdf_format_ = 0, cdf_epoch_ = -1;
   torch::Tensor mapped_rows(const torch::Tensor& base, const torch::Tensor& row_ids);
   GraphAndIndex slice_coo(const torch::Tensor& seeds, int64_t axis,

@@ -59,9 +59,11 @@ GraphAndIndex Graph::SamplingProbs(int64_t axis, torch::Tensor edge_probs,
 
 // ----------------------------------------- fused slice + weighted sampling
 torch::Tensor Graph::weight_cdf_for(const torch::Tensor& edge_probs, int64_t format) {
+  // (under one lock: sampler threads share the matrix)
+  std::lock_guard<std::mutex> lock(cdf_guard_);
   if (cdf_.defined() && cdf_format_ == format && cdf_probs_.is_same(edge_probs) &&
       cdf_version_ == (int64_t)edge_probs._version() && cdf_epoch_ == cache_epoch())
-    return cdf_;
+    return cdf_.on_current_stream();
   const Compressed& m = compressed(format);
   torch::Tensor probs = f32(edge_probs, "edge_probs");
   TORCH_CHECK(probs.numel() == m.indices.numel(), "weighted sampling: ", probs.numel(),
@@ -75,12 +77,12 @@ torch::Tensor Graph::weight_cdf_for(const torch::Tensor& edge_probs, int64_t for
   GS_CALL(gs_weight_cdf_build(cptr(m.indptr), n, cptr(m.indices), num_minor,
                               probs.data_ptr<float>(), nnz, mptr(cdf), ws.data_ptr(),
                               ws.numel(), cur_stream()));
-  cdf_ = cdf;
+  cdf_.set(cdf);
   cdf_probs_ = edge_probs;
   cdf_version_ = edge_probs._version();
   cdf_epoch_ = cache_epoch();
   cdf_format_ = format;
-  return cdf_;
+  return cdf;
 }
 
 // Slice + sample through the CDF; the twin of major_sample_uniform.

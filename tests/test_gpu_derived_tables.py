@@ -112,3 +112,29 @@ def test_walks_recorded_into_a_graph(arrays, calls_before):
     torch.cuda.synchronize()
     assert np.array_equal(traces(walk, n), want_walk) and np.array_equal(traces(n2v, n), want_n2v)
     del other
+
+
+def test_second_stream_waits_for_the_weights_cdf(arrays):
+    weights = torch.rand(arrays[1].size, device=DEV) + 0.01
+    seeds = torch.from_numpy(np.random.default_rng(4).permutation(NODES)[:5000]).to(DEV)
+
+    def sample(m):
+        gs.manual_seed(5)
+        sub, index = m._graph._CAPI_SlicingSamplingProbs(1, seeds, weights, 7, False, gs.format._CSC,
+                                                         gs.format._CSC)
+        return sub._CAPI_GetCSCIndptr(), sub._CAPI_GetCSCIndices(), index
+
+    want = sample(matrix(arrays))
+    m = matrix(arrays)
+    noise = torch.rand(1 << 26, device=DEV)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        noise.sort()                                 # the CDF is queued behind this
+        m._graph._CAPI_SlicingSamplingProbs(1, seeds[:0], weights, 7, False, gs.format._CSC,
+                                            gs.format._CSC)
+    with torch.cuda.stream(b):
+        for _ in range(2):
+            for got, expected in zip(sample(m), want):
+                assert torch.equal(got, expected)
+    torch.cuda.synchronize()
