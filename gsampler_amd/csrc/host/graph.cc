@@ -16,7 +16,9 @@ RandomState& random_state() {
   return state;
 }
 
-uint64_t next_call_id() { return random_state().next_call++; }
+uint64_t next_call_id(uint64_t how_many) {
+  return random_state().next_call.fetch_add(how_many, std::memory_order_relaxed);
+}
 
 // ------------------------------------------------------------------ loading
 // A loaded matrix is checked once (a few reductions and one read-back): every
@@ -256,7 +258,7 @@ torch::Tensor Compressed::narrow_indices() const {
 MajorResult major_sample_uniform(const Compressed& m,
                                         const torch::Tensor& picked,
                                         int64_t fanout, bool replace,
-                                        bool with_coo) {
+                                        bool with_coo, c10::optional<uint64_t> call_id) {
   TORCH_CHECK(fanout >= 0, "fanout must be non-negative, got ", fanout);
   const int64_t num_major = m.indptr.numel() - 1;
   const bool fused = picked.defined();
@@ -292,18 +294,19 @@ MajorResult major_sample_uniform(const Compressed& m,
   const int64_t* col_batch_ptr = label_cols ? cptr(hint.col_bptr) : nullptr;
   const int64_t col_batches = label_cols ? hint.col_bptr.numel() - 1 : 0;
   const torch::Tensor narrow = m.narrow_indices();
+  const uint64_t call = call_id.has_value() ? *call_id : next_call_id();
   if (narrow.defined()) {
     GS_CALL(gs_csc_col_sample_uniform_fill_i32(
         cptr(m.indptr), num_major, narrow.data_ptr<int32_t>(),
         fused ? cptr(picked) : nullptr, n, fanout, replace ? 1 : 0, (int)rs.algo,
-        rs.seed, next_call_id(), cptr(r.indptr), cptr(col_span), out_col, mptr(r.minor_ids),
+        rs.seed, call, cptr(r.indptr), cptr(col_span), out_col, mptr(r.minor_ids),
         mptr(r.select),
         col_batch_ptr, col_batches, cur_stream()));
   } else {
     GS_CALL(gs_csc_col_sample_uniform_fill(
         cptr(m.indptr), num_major, cptr(m.indices),
         fused ? cptr(picked) : nullptr, n, fanout, replace ? 1 : 0, (int)rs.algo,
-        rs.seed, next_call_id(), cptr(r.indptr), cptr(col_span), out_col, mptr(r.minor_ids),
+        rs.seed, call, cptr(r.indptr), cptr(col_span), out_col, mptr(r.minor_ids),
         mptr(r.select),
         col_batch_ptr, col_batches, cur_stream()));
   }

@@ -13,6 +13,7 @@
 
 #include "abi_call.h"
 
+#include <atomic>
 #include <functional>
 #include <memory>
 #include <mutex>
@@ -123,11 +124,13 @@ struct MajorResult {
 // seed reproduces a whole run.
 struct RandomState {
   uint64_t seed = 7777;  // the reference's literal, src/cuda/sampling.cu:143
-  uint64_t next_call = 0;
+  std::atomic<uint64_t> next_call{0};
   int64_t algo = 0;      // GS_ALGO_AUTO
 };
 RandomState& random_state();
-uint64_t next_call_id();  // takes one
+// Takes call ids, the first of which it returns.  Threads share the counter: what one
+// has taken is never put back.
+uint64_t next_call_id(uint64_t how_many = 1);
 
 // Views of one mini-batch block: (row, col, indptr by destination -- absent for
 // a mini-batch whose seeds repeat --, source ids, edge ids if the matrix carries
@@ -343,7 +346,8 @@ class Graph : public torch::CustomClassHolder {
                                    const c10::optional<torch::Tensor>& edge_probs, bool blocks,
                                    const LayersIdle& idle);
   Layer large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr, int64_t fanout,
-                    bool replace, const torch::Tensor& cdf, const std::function<void()>& idle);
+                    bool replace, const torch::Tensor& cdf, uint64_t call_id,
+                    const std::function<void()>& idle);
   // Workspace of the small layers, kept between calls (one per matrix, at most
   // 2^20 positions, about 40 MB): its table is empty whenever a call has been
   // queued, so the next call on the same stream starts without clearing it.  A call
@@ -494,11 +498,13 @@ torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, in
 MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo, const torch::Tensor& batch_ptr,
                         int64_t encode_stride);
+// (call_id: one that the caller has taken already)
 MajorResult major_sample_uniform(const Compressed& m, const torch::Tensor& picked,
-                                 int64_t fanout, bool replace, bool with_coo);
+                                 int64_t fanout, bool replace, bool with_coo,
+                                 c10::optional<uint64_t> call_id = c10::nullopt);
 MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
                                   const torch::Tensor& picked, int64_t fanout, bool replace,
-                                  bool with_coo);
+                                  bool with_coo, c10::optional<uint64_t> call_id = c10::nullopt);
 void check_weighted_fanout(int64_t fanout, bool replace, const char* who);
 MajorResult minor_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo);

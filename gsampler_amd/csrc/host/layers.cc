@@ -44,13 +44,13 @@ struct Queued {
 // One layer on the kernels for large layers; waits for its edge and key counts.
 Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr,
                                 int64_t fanout, bool replace, const torch::Tensor& cdf,
-                                const std::function<void()>& idle) {
+                                uint64_t call_id, const std::function<void()>& idle) {
   const Compressed& m = compressed(kCSC);
   const int64_t B = col_bptr.numel() - 1, S = cols.numel();
   Layer l;
   EdgeCount::HintScope batch(col_bptr, /*no_select=*/true);
-  MajorResult r = cdf.defined() ? major_sample_weighted(m, cdf, cols, fanout, replace, false)
-                                : major_sample_uniform(m, cols, fanout, replace, false);
+  MajorResult r = cdf.defined() ? major_sample_weighted(m, cdf, cols, fanout, replace, false, call_id)
+                                : major_sample_uniform(m, cols, fanout, replace, false, call_id);
   l.sampled_indptr = r.indptr;
   l.edge_ptr = EdgeCount::hint().edge_bptr;
   if (!l.edge_ptr.defined()) l.edge_ptr = r.indptr.index_select(0, col_bptr);
@@ -96,7 +96,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
   const int64_t num_cols = m.indptr.numel() - 1;
   const int64_t stride = std::max<int64_t>(std::max(num_cols, num_rows_), 1);
   const RandomState& rs = random_state();
-  const uint64_t first_call = rs.next_call;
+  const uint64_t first_call = next_call_id(fanouts.size());  // a second attempt draws by the same ids
   // (rows of a matrix that was loaded or converted are known to lie below num_rows)
   bool small_ok = m.num_minor >= 0 && m.num_minor <= stride && B <= (int64_t)0xFFFFFFFEll / stride &&
                   (weighted || replace || rs.algo != GS_ALGO_RESERVOIR);
@@ -156,7 +156,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           ptr = torch::arange(0, 2, device_options(m.indptr).dtype(torch::kInt64)) * n;
           BatchOffsets::trust(ptr, n);
         }
-        l = large_layer(cols, ptr, K, replace, cdf, [&] { idle(out, i); });
+        l = large_layer(cols, ptr, K, replace, cdf, first_call + i, [&] { idle(out, i); });
         mirrors = nullptr;  // it has used the thread's pinned words
         l.cols = cols;
         l.col_bptr = ptr;
@@ -207,7 +207,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
       GS_CALL(gs_sample_layer(
           cptr(m.indptr), num_cols, cptr(m.indices),
           narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(cdf), stride, cptr(cols), n,
-          cptr(ptr), B, K, replace ? 1 : 0, rs.seed, next_call_id(), base, base + q.at_ptr,
+          cptr(ptr), B, K, replace ? 1 : 0, rs.seed, first_call + i, base, base + q.at_ptr,
           base + q.at_row, base + q.at_col, base + q.at_edge_ptr,
           blocks ? base + q.at_indptr : nullptr, mirrors + words * i, lw.positions, lw.ws.data_ptr(),
           (size_t)lw.ws.numel(), cur_stream()));
@@ -238,7 +238,6 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
     }
     // a seed that is no id of this matrix: its keys do not fit the small layers' table
     GS_CALL(hipStreamSynchronize((hipStream_t)cur_stream()) == hipSuccess ? GS_OK : GS_ERR_HIP);
-    random_state().next_call = first_call;
     small_ok = false;
   }
 }
@@ -258,8 +257,8 @@ std::vector<c10::optional<torch::Tensor>> Graph::SampleLayers(
   seeds = ids(seeds, "seeds");
   std::vector<c10::optional<torch::Tensor>> out;
   if (seeds.numel() == 0) {  // no columns, no edges: layer after layer
+    next_call_id(fanouts.size());
     for (size_t i = 0; i < fanouts.size(); ++i) {
-      next_call_id();
       const torch::Tensor none = new_ids(0, compressed(kCSC).indptr);
       out.insert(out.end(), {none, none.clone(), none.clone(), c10::nullopt});
     }

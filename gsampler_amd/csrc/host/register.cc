@@ -17,7 +17,7 @@ static void set_random_seed(int64_t seed) {
   random_state().next_call = 0;
 }
 static std::tuple<int64_t, int64_t> get_random_state() {
-  return {(int64_t)random_state().seed, (int64_t)random_state().next_call};
+  return {(int64_t)random_state().seed, (int64_t)random_state().next_call.load()};
 }
 static void set_next_call_id(int64_t id) { random_state().next_call = (uint64_t)id; }
 static void set_sampling_algorithm(int64_t algo) {

@@ -88,7 +88,7 @@ torch::Tensor Graph::weight_cdf_for(const torch::Tensor& edge_probs, int64_t for
 // Slice + sample through the CDF; the twin of major_sample_uniform.
 MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
                                   const torch::Tensor& picked, int64_t fanout, bool replace,
-                                  bool with_coo) {
+                                  bool with_coo, c10::optional<uint64_t> call_id) {
   const int64_t num_major = m.indptr.numel() - 1, n = picked.numel();
   MajorResult r;
   r.indptr = new_ids(n + 1, m.indptr);
@@ -113,7 +113,8 @@ MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
   const RandomState& rs = random_state();
   GS_CALL(gs_csc_col_sample_weighted_fill(
       cptr(m.indptr), num_major, cptr(m.indices), nullptr, cptr(cdf), cptr(picked), n,
-      fanout, replace ? 1 : 0, rs.seed, next_call_id(), cptr(r.indptr), cptr(col_span),
+      fanout, replace ? 1 : 0, rs.seed, call_id.has_value() ? *call_id : next_call_id(),
+      cptr(r.indptr), cptr(col_span),
       nullptr, nullptr,
       with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr,
       mptr(r.minor_ids), mptr(r.select), label_cols ? cptr(hint.col_bptr) : nullptr,

@@ -1,6 +1,8 @@
 """All layers of a node-wise sampler in one call (small layers: three launches each, queued
 without waits) against the layers operator by operator, at sizes where the short path begins,
 ends or has remainders."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -114,3 +116,33 @@ def test_seeds_outside_the_matrix_take_the_other_path(rng):
     assert torch.equal(n0, n1)
     for x, y in zip(b0, b1):
         same(x, y)
+
+
+def test_call_ids_of_other_threads_are_not_taken_back(rng):
+    """A call that has to start over draws by the ids it took; the counter that all threads
+    share never goes back (another thread's draws in between would be repeated)."""
+    m = matrix(rng, 4000, 20, 0, False)
+    seeds = torch.from_numpy(np.concatenate([rng.permutation(4000)[:500], [1 << 40]])).to(DEV)
+    args = (m, seeds, [6, 5, 4], False)
+    sampler = gs.jit.compile(func=single, args=args)
+    sampler(*args)
+    walks, stop, made = [], threading.Event(), []
+    start = torch.zeros(64, dtype=torch.int64, device=DEV)
+
+    def walker():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            while not stop.is_set():
+                walks.append(m.random_walk(start, 30))
+        torch.cuda.synchronize()
+
+    gs.manual_seed(5)
+    other = threading.Thread(target=walker)
+    other.start()
+    try:
+        for _ in range(300):
+            sampler(*args)
+            made.append(1)
+    finally:
+        stop.set()
+        other.join()
+    assert gs.random_state() == (5, 3 * len(made) + len(walks))
