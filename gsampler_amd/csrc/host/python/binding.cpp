@@ -73,9 +73,13 @@ class Batch {
   explicit Batch(c10::intrusive_ptr<gs::BlockBatch> b) : b_(std::move(b)) {}
   gs::BlockBatch& get() { return *b_; }
 
-  // All blocks of the layer; the list is made once.
+  // The blocks may be made before anybody asks for them.
+  void make_ahead() { ahead_ = make_blocks(); }
+
+  // All blocks of the layer, objects of the caller's own: those made ahead go to the
+  // first who asks, another hand-out of the same layer gets others.
   py::list make_blocks() {
-    if (made_) return blocks_;
+    if (ahead_) return py::reinterpret_steal<py::list>(ahead_.release());
     TORCH_CHECK(g_block.type, "the Block class has not been set");
     gs::BlockBatch& b = *b_;
     auto off = b.Offsets();
@@ -112,15 +116,12 @@ class Batch {
         put(o, g_block.edata, PyDict_New());
       PyList_SET_ITEM(out.ptr(), i, block.release().ptr());
     }
-    blocks_ = out;
-    made_ = true;
     return out;
   }
 
  private:
   c10::intrusive_ptr<gs::BlockBatch> b_;
-  py::list blocks_;
-  bool made_ = false;
+  py::object ahead_;  // a list, or nothing
 };
 
 // The C++ object behind a torch custom-class instance.
@@ -171,7 +172,7 @@ std::vector<std::shared_ptr<Batch>> batch_sample_layers(py::handle graph, torch:
   auto done = [&](c10::intrusive_ptr<gs::BlockBatch> b) {
     py::gil_scoped_acquire gil;
     out.push_back(std::make_shared<Batch>(std::move(b)));
-    if (g_block.type) out.back()->make_blocks();
+    if (g_block.type) out.back()->make_ahead();
   };
   std::vector<c10::intrusive_ptr<gs::BlockBatch>> got;
   {

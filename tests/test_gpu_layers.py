@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import gsampler_amd as gs
+from gsampler_amd.utils.block import BlockList
 from tests.conftest import random_csc
 
 pytestmark = pytest.mark.gpu
@@ -146,3 +147,21 @@ def test_call_ids_of_other_threads_are_not_taken_back(rng):
         stop.set()
         other.join()
     assert gs.random_state() == (5, 3 * len(made) + len(walks))
+
+
+@pytest.mark.parametrize("count", [40, 9000])        # short layers, and large ones made ahead
+def test_blocks_handed_out_twice_are_other_objects(rng, count):
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(matrix(rng, 30000, 20, 0, False), False)
+    seeds = torch.cat([torch.from_numpy(rng.permutation(30000)[:count]) for _ in range(5)]).to(DEV)
+    ptr = torch.arange(6, device=DEV) * count
+
+    args = (bm, seeds, ptr, [12, 10, 4], False)
+    sampler = gs.jit.compile(func=batched, args=args)
+    for first in sampler(*args):
+        second = BlockList(first.batch)
+        for a, b in zip(first, second):
+            same(a, b)
+            a.srcdata["feat"], a.edata["w"], a.num_src = 1, 2, -1
+            assert a is not b and "feat" not in b.srcdata and "w" not in b.edata and b.num_src >= 0
+        assert all(x is y for x, y in zip(list(first), first))       # a list keeps its blocks
