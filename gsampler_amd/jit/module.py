@@ -4,8 +4,11 @@
 rebuilt inside the trace from their operator object; lists, ints, floats and
 bools -> compile-time constants; everything else -> run-time input), traces
 `func` with torch.fx, applies the passes of `passes.py` and keeps the resulting
-GraphModule in `.gm`.  Calling the object runs that module.  Same interface as
-the reference's python/gs/jit/module.py:191-259."""
+GraphModule in `.gm`.  Calling the object runs that module's operators; while the
+module is as it was compiled, through a copy of its graph whose sampling layers are
+chained (`_executable`), and once it has been replaced, edited and recompiled or
+hooked, through the module itself.  Same interface as the reference's
+python/gs/jit/module.py:191-259."""
 from typing import Any, List, Sequence, Tuple
 
 import torch
@@ -74,6 +77,7 @@ class compile:  # noqa: N801 -- the reference's public name
             if compact_ms < plain_ms:
                 self.gm, self.compact = other, True
         self._run = self._executable(self.gm)
+        self._compiled = (self.gm, type(self.gm).forward)
 
     def _time(self, gm, args, runs=3):
         """Milliseconds per call of one variant on the example arguments."""
@@ -173,6 +177,15 @@ class compile:  # noqa: N801 -- the reference's public name
         # the positions of the other run-time inputs
         passthrough = tuple(None if k in (MATRIX, BATCH_MATRIX, STATIC) else a
                             for a, k in zip(args, self.kinds))
-        if self._run is not None:
-            return self._run(passthrough, graphs, *(data[i][j][key] for i, j, key in self._data_keys))
+        if self._run is not None and self._as_compiled():
+            # (run on self.gm: constants are looked up there)
+            return self._run.__func__(self.gm, passthrough, graphs,
+                                      *(data[i][j][key] for i, j, key in self._data_keys))
         return self.gm(passthrough, graphs, data)
+
+    def _as_compiled(self):
+        """Whether self.gm still is the module of __init__: its generated code is replaced
+        when an edited graph is recompiled."""
+        gm, forward = self._compiled
+        return (self.gm is gm and type(gm).forward is forward and "forward" not in gm.__dict__
+                and not gm._forward_hooks and not gm._forward_pre_hooks)

@@ -563,3 +563,46 @@ def test_all_nodes_is_read_off_the_block_batch_built_from_the_same_ids():
     t = targets(gm)
     assert "_CAPI_BatchGetValidNodes" not in t
     assert t == ["_CAPI_BatchBlocks", "frontier", "frontier_ptr"]   # the builder came first
+
+
+def scaled(A, x, k):
+    return x * k, x + torch.tensor(3.0)
+
+
+def _scaled_on_the_host():
+    x = torch.arange(4.0)
+    c = gs.jit.compile(func=scaled, args=(gs.Matrix(gs.Graph(4, 4)), x, 2))
+    call = lambda: [t.tolist() for t in c(gs.Matrix(gs.Graph(4, 4)), x, 2)]  # noqa: E731
+    assert call() == [[0, 2, 4, 6], [3, 4, 5, 6]] and c._run is not None
+    return c, call
+
+
+def test_an_edited_module_is_what_a_call_runs():
+    c, call = _scaled_on_the_host()
+    mul = next(n for n in c.gm.graph.nodes if n.op == "call_function" and "mul" in str(n.target))
+    mul.target = torch.add
+    c.gm.recompile()
+    assert call() == [[2, 3, 4, 5], [3, 4, 5, 6]]
+    c.gm = _scaled_on_the_host()[0].gm                  # another module in its place
+    c.gm.forward = lambda *a: [torch.zeros(1)]
+    assert call() == [[0]]
+
+
+def test_a_replaced_constant_is_what_a_call_reads():
+    c, call = _scaled_on_the_host()
+    name = next(n.target for n in c.gm.graph.nodes if n.op == "get_attr" and
+                getattr(c.gm, n.target).numel() == 1)
+    setattr(c.gm, name, torch.tensor(10.0))
+    assert call() == [[0, 2, 4, 6], [10, 11, 12, 13]]
+
+
+@pytest.mark.parametrize("register", ["register_forward_hook", "register_forward_pre_hook"])
+def test_a_hook_of_the_module_sees_a_call(register):
+    c, call = _scaled_on_the_host()
+    seen = []
+    handle = getattr(c.gm, register)(lambda module, *rest: seen.append(module))
+    call()
+    assert seen == [c.gm]
+    handle.remove()
+    call()
+    assert len(seen) == 1
