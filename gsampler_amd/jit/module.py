@@ -145,6 +145,7 @@ class compile:  # noqa: N801 -- the reference's public name
         if self._format_select and not self.use_batchmatrix:
             gm = passes.select_formats(gm)
         gm = passes.sink_block_construction(gm)
+        gm.recompile()
         return gm
 
     # -------------------------------------------------------------------- run
@@ -166,10 +167,10 @@ class compile:  # noqa: N801 -- the reference's public name
         try:
             graph.output(pytree.tree_unflatten(list(flat), info.out_spec)
                          if info.out_spec is not None else flat)
-            run = passes.chain_layers(fx.GraphModule(gm, graph))
         except (TypeError, ValueError):
             return None
-        return run.forward
+        passes.chain_layers(gm, graph)
+        return fx.GraphModule(gm, graph).forward
 
     def __call__(self, *args):
         graphs, data = matrix_parts(args, self.kinds)

@@ -29,6 +29,10 @@ hoisting of tensor constants.  Operator rewrites (observable in
                                                   -> _CAPI_SampleLayers,
                                                      _CAPI_BatchSampleLayers
   select_formats                deterministic on_format / output_format choice
+
+A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
+whoever runs the passes (gm.recompile()): generating it after each of them was
+three quarters of a compilation.
 """
 import operator
 from typing import Dict, Iterable, List, Optional
@@ -50,20 +54,23 @@ def _input_nodes(node: fx.Node) -> Iterable[fx.Node]:
 
 def _finish(gm: fx.GraphModule) -> fx.GraphModule:
     gm.graph.lint()
-    gm.recompile()
     return gm
 
 
-def dce(gm: fx.GraphModule) -> fx.GraphModule:
+def _drop_dead_nodes(graph: fx.Graph) -> None:
     live = set()
-    for node in reversed(gm.graph.nodes):
+    for node in reversed(graph.nodes):
         if node.op in ("output", "placeholder") or node.target in IN_PLACE_OPS:
             live.add(node)
         if node in live:
             live.update(_input_nodes(node))
-    for node in reversed(gm.graph.nodes):
+    for node in reversed(graph.nodes):
         if node not in live:
-            gm.graph.erase_node(node)
+            graph.erase_node(node)
+
+
+def dce(gm: fx.GraphModule) -> fx.GraphModule:
+    _drop_dead_nodes(gm.graph)
     return _finish(gm)
 
 
@@ -577,21 +584,21 @@ def _is_empty_constant(gm: fx.GraphModule, node) -> bool:
             and getattr(getattr(gm, node.target, None), "numel", lambda: -1)() == 0)
 
 
-def chain_layers(gm: fx.GraphModule) -> fx.GraphModule:
-    """Layer after layer of  slice + sample -> relabel,  each layer's frontier the
-    next one's seeds and the sampled matrix and its edge index used for nothing
-    else, becomes one operator call:
+def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
+    """In a copy of gm's graph: layer after layer of  slice + sample -> relabel,  each
+    layer's frontier the next one's seeds and the sampled matrix and its edge index
+    used for nothing else, becomes one operator call:
         _CAPI_SlicingSampling[Probs] -> _CAPI_GraphRelabel          (one mini-batch)
             => _CAPI_SampleLayers(seeds, fanouts, replace, weights)
         _CAPI_BatchFusedSlicingSampling[Probs] -> _CAPI_BatchBlocks  (a super-batch)
             => _CAPI_BatchSampleLayers(seeds, ptr, fanouts, replace, weights)
     (both called through the native binding, which makes the block objects).
-    The operator draws the same samples.  Run on the executed copy of the graph:
-    the operator graph that a compiled sampler shows keeps its layers."""
+    The operator draws the same samples.  The operator graph that a compiled sampler
+    shows keeps its layers."""
     single = {"_CAPI_SlicingSampling": (2, None, 3, 4, 5), "_CAPI_SlicingSamplingProbs": (2, 3, 4, 5, 6)}
     batch = {"_CAPI_BatchFusedSlicingSampling": (1, None, 3, 4), "_CAPI_BatchFusedSlicingSamplingProbs": (1, 3, 4, 5)}
-    order = {n: i for i, n in enumerate(gm.graph.nodes)}
-    draws = [n for n in gm.graph.nodes if _draws_random_numbers(n)]
+    order = {n: i for i, n in enumerate(copy.nodes)}
+    draws = [n for n in copy.nodes if _draws_random_numbers(n)]
 
     def layer_of(node):
         """(matrix, seeds, ptr, weights, fanout, replace, relabel) of one layer, or None."""
@@ -641,26 +648,27 @@ def chain_layers(gm: fx.GraphModule) -> fx.GraphModule:
         if any(a is not None and order[a] > order[first] for a in (graph, seeds, ptr, weights)):
             continue
         fanouts = [layer[4] for _, layer in chain]
-        with gm.graph.inserting_before(first):
+        with copy.inserting_before(first):
             if ptr is None:
-                out = gm.graph.call_function(_library.native.sample_layers,
-                                             args=(graph, seeds, fanouts, replace, weights))
+                out = copy.call_function(_library.native.sample_layers,
+                                         args=(graph, seeds, fanouts, replace, weights))
             else:
-                out = gm.graph.call_function(_library.native.batch_sample_layers,
-                                             args=(graph, seeds, ptr, fanouts, replace, weights))
+                out = copy.call_function(_library.native.batch_sample_layers,
+                                         args=(graph, seeds, ptr, fanouts, replace, weights))
             for i, (_, layer) in enumerate(chain):
                 relabel = layer[6]
                 if ptr is not None:
-                    blocks = gm.graph.call_function(operator.getitem, args=(out, i))
+                    blocks = copy.call_function(operator.getitem, args=(out, i))
                     relabel.replace_all_uses_with(blocks)
                     continue
                 for j in range(4):
                     users = _getitem_users(relabel, j)
                     if users:
-                        item = gm.graph.call_function(operator.getitem, args=(out, 4 * i + j))
+                        item = copy.call_function(operator.getitem, args=(out, 4 * i + j))
                         for u in users:
                             u.replace_all_uses_with(item)
-    return dce(gm)
+    if chains:
+        _drop_dead_nodes(copy)
 
 
 # --------------------------------------------------------------- formats
