@@ -8,9 +8,9 @@ edges are kept, as a sampled multigraph would have them.
 """
 from __future__ import annotations
 
+import math
 from typing import Optional, Tuple
 
-import numpy as np
 import torch
 
 
@@ -69,15 +69,20 @@ def rmat_csc(num_nodes: int, num_edges: int, a: float = 0.57, b: float = 0.19,
 def power_law_cdf(num_nodes: int, exponent: float = 2.1, device="cpu") -> torch.Tensor:
     """Cumulative shares of w_i = (i+1)^(-1/(exponent-1)), float64.
 
-    The prefix sum is made on the host, one term after the other in extended
-    precision.  On the GPU, torch's scan of a float64 vector adds its tiles' sums in
-    the order in which they happen to be ready: of 40 scans of 2.45 M weights no two
-    were alike (up to 8 units in the last place apart), and about one graph of 124 M
-    edges in twenty-five then had an edge in the next column."""
-    w = torch.arange(1, num_nodes + 1, dtype=torch.float64, device=device)
-    w = w.pow(-1.0 / (exponent - 1.0))
-    cdf = np.cumsum(w.cpu().numpy(), dtype=np.longdouble).astype(np.float64)
-    cdf = torch.from_numpy(cdf).to(device)
+    The prefix sum is made in integers of 2^-shift, so it does not depend on the order
+    in which a device adds.  (torch's scan of a float64 vector on the GPU adds its
+    tiles' sums in the order in which they happen to be ready: of 40 scans of 2.45 M
+    weights no two were alike, up to 8 units in the last place apart, and 2 to 7 in 100
+    graphs of 124 M edges then had an edge in the next column.)  The shift leaves the
+    total below 2^62; at 2.45 M weights it is 56 or more, and what the roundings of the
+    terms add up to stays near a unit in the last place of the sum."""
+    a = 1.0 / (exponent - 1.0)
+    # no more than the first term and the integral of x^-a up to num_nodes + 1
+    end = num_nodes + 1.0
+    most = 1.0 + (math.log(end) if a == 1.0 else (end ** (1.0 - a) - 1.0) / (1.0 - a))
+    shift = 61 - math.ceil(math.log2(most))
+    w = torch.arange(1, num_nodes + 1, dtype=torch.float64, device=device).pow(-a)
+    cdf = torch.cumsum(w.mul_(2.0 ** shift).round_().to(torch.int64), 0).to(torch.float64)
     return cdf / cdf[-1]
 
 
