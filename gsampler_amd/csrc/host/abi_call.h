@@ -9,6 +9,7 @@
 #include <hip/hip_runtime_api.h>
 #include <atomic>
 #include <limits>
+#include <thread>
 #include <torch/torch.h>
 
 #include <vector>
@@ -118,15 +119,17 @@ inline torch::Tensor new_workspace(size_t bytes, const torch::Tensor& like) {
 constexpr int64_t kNotYet = std::numeric_limits<int64_t>::min();
 
 // Waits until words[0 .. n) have all been stored to by work queued on `stream`.
-// Every now and then the stream itself is asked, so that a failed kernel ends
-// the wait; once the stream is idle the words hold whatever they will hold.
+// The core is offered to other threads every few microseconds, and every now and
+// then the stream itself is asked, so that a failed kernel ends the wait; once the
+// stream is idle the words hold whatever they will hold.
 inline void await_words(const int64_t* words, size_t n, hipStream_t stream) {
-  constexpr int kPollsPerQuery = 1 << 13;
+  constexpr int kPollsPerYield = 1 << 6, kPollsPerQuery = 1 << 13;
   for (size_t i = 0; i < n; ++i) {
     int polls = 0;
     while (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) == kNotYet) {
       if (++polls < kPollsPerQuery) {
-        __builtin_ia32_pause();
+        if (polls % kPollsPerYield == 0) std::this_thread::yield();
+        else __builtin_ia32_pause();
         continue;
       }
       polls = 0;
