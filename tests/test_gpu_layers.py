@@ -1,6 +1,7 @@
 """All layers of a node-wise sampler in one call (small layers: three launches each, queued
 without waits) against the layers operator by operator, at sizes where the short path begins,
 ends or has remainders."""
+import gc
 import threading
 
 import numpy as np
@@ -8,7 +9,7 @@ import pytest
 import torch
 
 import gsampler_amd as gs
-from gsampler_amd.utils.block import BlockList
+from gsampler_amd.utils.block import Block, BlockList
 from tests.conftest import random_csc
 
 pytestmark = pytest.mark.gpu
@@ -165,3 +166,29 @@ def test_blocks_handed_out_twice_are_other_objects(rng, count):
             a.srcdata["feat"], a.edata["w"], a.num_src = 1, 2, -1
             assert a is not b and "feat" not in b.srcdata and "w" not in b.edata and b.num_src >= 0
         assert all(x is y for x, y in zip(list(first), first))       # a list keeps its blocks
+
+
+def test_no_blocks_are_made_ahead_beside_other_python_threads(rng):
+    """Making them needs the interpreter in the middle of a step, which another thread may
+    hold, and they may never be asked for."""
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(matrix(rng, 30000, 20, 0, False), False)
+    seeds = torch.cat([torch.from_numpy(rng.permutation(30000)[:9000]) for _ in range(5)]).to(DEV)
+    args = (bm, seeds, torch.arange(6, device=DEV) * 9000, [12, 10, 4], False)
+    sampler = gs.jit.compile(func=batched, args=args)
+    blocks = lambda: sum(type(o) is Block for o in gc.get_objects())  # noqa: E731
+    gc.collect()
+    before, stop = blocks(), threading.Event()
+    other = threading.Thread(target=stop.wait)
+    other.start()
+    try:
+        gs.manual_seed(5)
+        got = sampler(*args)
+        assert blocks() == before
+    finally:
+        stop.set()
+        other.join()
+    gs.manual_seed(5)
+    for layer, again in zip(got, sampler(*args)):
+        for x, y in zip(layer, again):
+            same(x, y)
