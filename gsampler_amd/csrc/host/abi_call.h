@@ -441,25 +441,48 @@ inline torch::Tensor piece_of(const torch::Tensor& buffer, int64_t offset, int64
   return torch::Tensor(std::move(impl));
 }
 
-// Pinned host words that live until the process ends, one run per thread: what a
-// kernel reports to an operator that waits for it before it returns.
+// Pinned host words that live until the process ends, one run per thread: what
+// kernels report to an operator that waits for them before it returns.
 class PinnedWords {
  public:
-  // n words, all marked as not yet there; valid until the thread's next take()
+  // n words, all marked as not yet there, for work queued on the current stream; valid
+  // until the thread's next take()
   static int64_t* take(size_t n) {
-    static thread_local int64_t* words = nullptr;
-    static thread_local size_t capacity = 0;
-    if (capacity < n) {
-      if (words) (void)hipHostFree(words);
-      words = nullptr;
-      capacity = 0;
-      const size_t want = n < 4096 ? 4096 : n;
-      const hipError_t e = hipHostMalloc((void**)&words, want * sizeof(int64_t), hipHostMallocDefault);
+    Run& r = run();
+    if (r.out) {
+      // an operator left by an exception: its kernels must not store later
+      const hipError_t e = hipStreamSynchronize(r.stream);
       TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
-      capacity = want;
+      r.out = false;
     }
-    for (size_t i = 0; i < n; ++i) words[i] = kNotYet;
-    return words;
+    if (r.capacity < n) {
+      if (r.words) (void)hipHostFree(r.words);
+      r.words = nullptr;
+      r.capacity = 0;
+      const size_t want = n < 4096 ? 4096 : n;
+      const hipError_t e =
+          hipHostMalloc((void**)&r.words, want * sizeof(int64_t), hipHostMallocDefault);
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+      r.capacity = want;
+    }
+    for (size_t i = 0; i < n; ++i) r.words[i] = kNotYet;
+    r.stream = (hipStream_t)cur_stream();
+    r.out = true;
+    return r.words;
+  }
+  // All words that kernels were given have arrived.
+  static void arrived() { run().out = false; }
+
+ private:
+  struct Run {
+    int64_t* words = nullptr;
+    size_t capacity = 0;
+    hipStream_t stream = nullptr;
+    bool out = false;
+  };
+  static Run& run() {
+    static thread_local Run r;
+    return r;
   }
 };
 

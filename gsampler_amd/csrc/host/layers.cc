@@ -78,6 +78,7 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
   l.e_off = OffsetMirror::values(l.edge_ptr);
   l.f_off = OffsetMirror::values(l.frontier_ptr);
   await_words(distinct, (size_t)B, (hipStream_t)cur_stream());
+  PinnedWords::arrived();
   l.distinct.assign((size_t)B, 1);
   for (int64_t b = 0; b < B; ++b) l.distinct[(size_t)b] = distinct[b] != 0;
   l.frontier = frontier.narrow(0, 0, l.f_off.back());
@@ -156,6 +157,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           ptr = torch::arange(0, 2, device_options(m.indptr).dtype(torch::kInt64)) * n;
           BatchOffsets::trust(ptr, n);
         }
+        PinnedWords::arrived();  // every layer queued so far has been settled
         l = large_layer(cols, ptr, K, replace, cdf, first_call + i, [&] { idle(out, i); });
         mirrors = nullptr;  // it has used the thread's pinned words
         l.cols = cols;
@@ -219,6 +221,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
     }
     if (!retry) settle(L);
     if (!retry) {
+      PinnedWords::arrived();
       for (size_t i = 1; i < L; ++i)
         if (queued[i - 1].buffer.defined()) {  // the pieces, in place of the bounds
           out[i].cols = out[i - 1].frontier;

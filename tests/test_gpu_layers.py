@@ -192,3 +192,40 @@ def test_no_blocks_are_made_ahead_beside_other_python_threads(rng):
     for layer, again in zip(got, sampler(*args)):
         for x, y in zip(layer, again):
             same(x, y)
+
+
+def test_a_call_that_runs_out_of_memory_between_layers_leaves_nothing_behind(rng):
+    """What the first layer's kernels still report must not be taken for the next call's."""
+    m = matrix(rng, 30000, 20, 0, False)
+    seeds = torch.from_numpy(rng.permutation(30000)[:60]).to(DEV)
+    args = (m, seeds, [10, 60, 9], False)            # the second layer's buffer takes a segment
+    sampler = gs.jit.compile(func=single, args=args)
+    gs.manual_seed(5)
+    n0, b0 = sampler(*args)
+    other = (m, seeds[:31].contiguous(), [7, 3], False)
+    sampler2 = gs.jit.compile(func=single, args=other)
+    gs.manual_seed(5)
+    n1, b1 = sampler2(*other)
+    torch.cuda.synchronize()
+    failed = 0
+    for _ in range(3):
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+        try:
+            sampler(*args)
+        except torch.OutOfMemoryError:
+            failed += 1
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        gs.manual_seed(5)
+        n, blocks = sampler2(*other)
+        assert torch.equal(n, n1)
+        for x, y in zip(blocks, b1):
+            same(x, y)
+    assert failed > 0             # (the first time, a segment may still have room)
+    gs.manual_seed(5)
+    n, blocks = sampler(*args)
+    assert torch.equal(n, n0)
+    for x, y in zip(blocks, b0):
+        same(x, y)
