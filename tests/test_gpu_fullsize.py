@@ -414,3 +414,77 @@ def test_ladies_layers_at_full_size_with_unit_interval_weights_through_the_compi
         h_seeds = uniq
     assert np.array_equal(frontier.cpu().numpy(), h_seeds)
     assert blocks[1].num_edges() > 1_000_000
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_chained_super_batch_against_the_oracle(graph, weighted):
+    """The compiled super-batched sampler, all layers in one call: every layer's arrays and
+    blocks against the CPU restatement, layer by layer."""
+    import gsampler_amd as gs
+    indptr, indices, seeds, ptr = graph
+    nodes = indptr.numel() - 1
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(indptr, indices)
+    if weighted:
+        g = torch.Generator(device=indices.device)
+        g.manual_seed(6)
+        m.edata["w"] = torch.rand(indices.numel(), generator=g, device=indices.device) + 0.01
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(m, False)
+
+    def sampler(A, seeds, ptr, fanouts):
+        out = []
+        for k in fanouts:
+            sub = A[:, seeds::ptr]
+            sub = sub.individual_sampling(k, sub.edata["w"] if weighted else None, False)
+            seeds, ptr = sub.all_nodes()
+            out.append(sub.to_dgl_block())
+        return out
+
+    args = (bm, seeds, ptr, FANOUTS)
+    compiled = gs.jit.compile(func=sampler, args=args)
+    assert sum("batch_sample_layers" in str(n.target)
+               for n in compiled._run.__self__.graph.nodes) == 1
+    gs.manual_seed(7777)
+    layers = compiled(*args)
+    h_indptr, h_indices = indptr.cpu().numpy(), indices.cpu().numpy()
+    h_seeds, h_ptr = seeds.cpu().numpy(), ptr.cpu().numpy()
+    if weighted:
+        h_probs = m.edata["w"].cpu().numpy()
+        h_cdf = orc.weight_cdf(h_indptr, h_probs, h_indices, nodes)
+    for call, (layer, fanout) in enumerate(zip(layers, FANOUTS)):
+        if weighted:
+            sub_indptr, coo_col, rows, _ = orc.sample_weighted(
+                h_indptr, h_indices, h_probs, h_seeds, fanout, False, 7777, call, cdf=h_cdf)
+        else:
+            sub_indptr, coo_col, rows, _ = orc.sample_uniform(h_indptr, h_indices, h_seeds, fanout,
+                                                              False, 0, 7777, call)
+        edge_ptr = sub_indptr[h_ptr]
+        uniq, uniq_ptr, row, col = orc.unique_relabel(h_seeds, rows, h_ptr, edge_ptr, coo_col)
+        b = layer.batch
+        same((b.frontier(), b.frontier_ptr(), b.row(), b.col(), b.edge_ptr(), b.col_ptr()),
+             (uniq, uniq_ptr, row, col, edge_ptr, h_ptr))
+        for i in (0, 31, 63):
+            blk = layer[i]
+            lo, hi = edge_ptr[i], edge_ptr[i + 1]
+            same((blk.row, blk.col, blk.srcdata["_ID"], blk.indptr),
+                 (row[lo:hi], col[lo:hi], uniq[uniq_ptr[i]:uniq_ptr[i + 1]],
+                  sub_indptr[h_ptr[i]:h_ptr[i + 1] + 1] - sub_indptr[h_ptr[i]]))
+        h_seeds, h_ptr = uniq, uniq_ptr
+
+
+@pytest.mark.parametrize("walks,length", [(100_000, 20), (1_000_000, 10)])
+def test_node2vec_of_a_matrix_against_the_oracle(graph, walks, length):
+    """Matrix.node2vec reads the int32 copy of the ids from 2^20 edges on."""
+    import gsampler_amd as gs
+    indptr, indices, _, _ = graph
+    nodes = indptr.numel() - 1
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(indptr, indices)
+    m._graph._CAPI_SortCSCIndices()
+    start = torch.arange(walks, device=indices.device) * 7 % nodes
+    gs.manual_seed(7777)
+    got = m.node2vec(start, length, 2.0, 0.5).reshape(-1, walks)
+    want = orc.node2vec(indptr.cpu().numpy(), m.csc[1].cpu().numpy(), start.cpu().numpy(), length,
+                        2.0, 0.5, 7777, 0)
+    assert np.array_equal(got.cpu().numpy(), want.reshape(length + 1, walks))
