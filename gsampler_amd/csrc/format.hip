@@ -50,7 +50,7 @@ namespace gs {
 // work-group first takes the minimum over its tile of edges in LDS and then
 // sends one atomic per id it met -- and only if the value in memory is not
 // already smaller, which it is for every tile but the first few.
-constexpr int kFirstLdsIds = 4096;
+constexpr int kFirstLdsIds = GS_FIRST_POSITION_FEW_IDS;
 constexpr int kFirstTile = kBlock * 32;
 
 __global__ __launch_bounds__(kBlock) void first_position_lds_kernel(

@@ -238,11 +238,34 @@ torch::Tensor Graph::batch_rows_for_relabel(const torch::Tensor& edge_rows,
   return mapped_out_;
 }
 
+// A pass over the edges finds the first edge of every listed id: in LDS for a few
+// thousand ids, with an atomic in device memory for an edge of one of more, where
+// edges soon queue for their id.  all_nodes() and to_dgl_block() together, by the
+// list and by the general path, us:
+//   4 batches of 192 keys, 512 ids                     56 K edges   78   115
+//   16 batches of 192 keys, 2048 ids                  875 K         84   158
+//   16 batches of 450 keys, 4800 ids                   48 K         88   109
+//                                                     177 K        110   109
+//                                                     694 K        262   138
+//   64 batches of 192 keys, 8192 ids                  123 K         86   107
+//                                                     461 K        136   113
+//   64 batches of 1000 keys, 44 800 ids               295 K         91    99
+//                                                     4.1 M        647   171
+// (rows drawn by a power law, for the last two lines evenly).  Below eight edges a key the
+// list is ahead as well (77 against 106 us at 1.6); those calls have always taken the
+// general path.  A batch of more than GS_LIST_LABELS_MAX_KEYS is refused by the device
+// after both passes: half of that on average leaves room for uneven batches.
+static bool list_labels_pay(int64_t ids, int64_t seeds, int64_t edges, int64_t batches) {
+  constexpr int64_t kFewEdges = int64_t(1) << 17;
+  return edges >= 8 * (ids + seeds) &&
+         (ids <= GS_FIRST_POSITION_FEW_IDS || edges <= kFewEdges) &&
+         ids + seeds <= batches * (GS_LIST_LABELS_MAX_KEYS / 2);
+}
+
 // Frontier and labels by way of the list of row ids, for a matrix whose rows are
 // positions in a list with a segment per mini-batch; null where that does not pay
-// (a batch should have a few hundred keys and many times as many edges) or where
-// an edge's row turns out to lie in another batch's segment.  Waits for the size
-// of the frontier, as every caller is about to do.
+// (`list_labels_pay`) or where an edge's row turns out to lie in another batch's
+// segment.  Waits for the size of the frontier, as every caller is about to do.
 Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_seeds,
                                                      const torch::Tensor& row_ids,
                                                      const ColumnOrderedEdges& edges,
@@ -251,7 +274,7 @@ Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_se
   const int64_t B = col_bptr_.numel() - 1;
   if (R == 0 || S == 0 || R != num_rows_ || S != num_cols_ || !edges.col.defined() ||
       !row_bptr_.defined() || row_bptr_.numel() != B + 1 || row_encoding_size_ <= 0 ||
-      E < 8 * (R + S) || R + S > B * (GS_LIST_LABELS_MAX_KEYS / 2))
+      !list_labels_pay(R, S, E, B))
     return nullptr;
   if (batch_list_labels_ && batch_list_labels_->base.is_same(edges.row) &&
       batch_list_labels_->row_ids.is_same(row_ids) &&

@@ -498,6 +498,9 @@ int gs_slice_compact_fill(const int64_t* indptr, const int64_t* indices,
  * picked row instead of per edge (no counterpart in the reference, which
  * hashes every edge, src/cuda/unique_reindex.cu:81-151).
  * ---------------------------------------------------------------------- */
+/* Up to this many ids a work-group takes its minima in LDS; beyond, an edge that
+ * comes before what is known of its id costs an atomic in device memory. */
+#define GS_FIRST_POSITION_FEW_IDS 4096
 int gs_first_position(const int64_t* ids, int64_t n, int64_t num_ids,
                       int64_t* out_first, gs_stream_t stream);
 

@@ -119,3 +119,12 @@ def test_batched_labels_by_way_of_the_list(sizes, picks, mode):
             assert np.array_equal(frontier[u], want[0]) and np.array_equal(row[e], want[2])
             if sizes[b]:
                 assert np.array_equal(col[e], want[3])
+
+
+@pytest.mark.parametrize("sizes,picks", [
+    ([64] * 8, [512] * 8),             # 4096 listed ids, the most that the list pass holds in LDS
+    ([20] * 17, [241] * 17),           # 4097, few edges: by way of the list all the same
+    ([100] * 10, [450] * 10),          # 4500 and several hundred thousand: the general path
+])
+def test_batched_labels_where_the_list_begins_or_ends_to_pay(sizes, picks):
+    test_batched_labels_by_way_of_the_list(sizes, picks, "distinct")
