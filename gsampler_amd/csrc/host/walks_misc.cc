@@ -7,15 +7,16 @@ namespace gs {
 
 // Kept for matrices of up to 2^24 edges (128 MB): there it stays in the last-level
 // cache, and making it costs a fraction of a walk.  A matrix that is walked once
-// never makes it.
+// never makes it, nor one whose calls have too many walks for it.
 torch::Tensor Compressed::hop_table() const {
   constexpr int64_t kMaxEdges = int64_t(1) << 24;
   const int64_t nnz = indices.numel();
-  if (nnz == 0 || nnz > kMaxEdges || !indices.is_cuda() || !indptr.is_cuda() || capturing())
-    return {};
+  if (nnz == 0 || nnz > kMaxEdges || !indices.is_cuda() || !indptr.is_cuda()) return {};
   std::lock_guard<std::mutex> lock(derived_.guard);
   Derived& d = current_derived();
-  if (!d.hops.defined() && d.walks++ > 0) {
+  if (!d.hops.defined() && d.walks++ == 0) return {};
+  if (capturing()) return {};
+  if (!d.hops.defined()) {
     torch::Tensor t = new_ids(nnz, indices);
     GS_CALL(gs_hop_table(cptr(indptr), indptr.numel() - 1, cptr(indices), nnz, t.data_ptr(),
                          cur_stream()));
@@ -35,7 +36,7 @@ torch::Tensor Graph::RandomWalk(torch::Tensor seeds, int64_t walk_length) {
   const int64_t n = seeds.numel();
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
-  const torch::Tensor hops = csc_->hop_table();
+  const torch::Tensor hops = n <= gs_hop_walks(0, 1.0, 1.0) ? csc_->hop_table() : torch::Tensor();
   GS_CALL(gs_random_walk_hops(cptr(csc_->indptr), cptr(csc_->indices), cptr(hops), num_cols_,
                               cptr(seeds), n, walk_length, rs.seed, next_call_id(), mptr(out),
                               cur_stream()));
@@ -68,7 +69,7 @@ torch::Tensor Graph::Node2Vec(torch::Tensor seeds, int64_t walk_length, double p
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
   const torch::Tensor narrow = csc_->narrow_indices();  // half the bytes behind every candidate
-  const torch::Tensor hops = csc_->hop_table();
+  const torch::Tensor hops = n <= gs_hop_walks(1, p, q) ? csc_->hop_table() : torch::Tensor();
   GS_CALL(gs_node2vec_hops(cptr(csc_->indptr), cptr(csc_->indices),
                            narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(hops),
                            num_cols_, cptr(seeds), n, walk_length, p, q, rs.seed, next_call_id(),

@@ -1,7 +1,8 @@
 // walks.hip -- uniform random walk and node2vec over CSC in-neighbours.
-// One thread per walk; traces are stored step-major, out[step * N + walk], so
-// that a wavefront writes 64 consecutive ids per step (the reference uses the
-// same layout, src/cuda/fusion/random_walk.cu:34).  Streams: pos = walk index;
+// A lane per walk, up to sixteen per second-order walk; traces are stored
+// step-major, out[step * N + walk], so that neighbouring lanes write neighbouring
+// ids (the reference uses the same layout, src/cuda/fusion/random_walk.cu:34).
+// Streams: pos = walk index;
 // random walk draw = step; node2vec draw = step << 32 | attempt.
 #include "common.h"
 
@@ -209,10 +210,30 @@ __global__ __launch_bounds__(kBlock) void node2vec_kernel(
   }
 }
 
-// Up to this many walks a call is bound by the latency of its chains of loads: the
-// hop table shortens them.  More walks are bound by lines, of which the table costs
-// as many as it saves, and the column pointer's are the better cached ones.
-constexpr int64_t kHopWalks = int64_t(1) << 15;
+// Whether candidates are mostly rejected, by the ratio of the levels.
+static bool rare_picks(double p, double q) {
+  const double most = p > q ? p : q, least = p < q ? p : q;
+  return (least < 1.0 ? least : 1.0) * 4.0 < most;
+}
+
+// Up to how many walks a call goes by the hop table.  Few walks are bound by the
+// latency of their chains of loads, which the table shortens; more are bound by lines,
+// of which it costs as many as it saves -- a second line a candidate for a group that
+// looks at sixteen at once -- and the column pointer's are the better cached ones.
+// Without / with the table, us, 9 M edges:
+//   first order, 56 steps     1 K walks 47 / 32    16 K 49 / 38     24 K 51 / 51, 33 K 53 / 69
+//     (measured with picks stored eight at a time)
+//   second order, 40 steps
+//     q < 1 (no search)       2 K walks 44 / 35 and 45 / 37         4 K 46 / 49, 8 K 51 / 95
+//     q > 1, picks rare       8 K walks 286 / 243                   16 K 322 / 461
+//     q > 1, others           32 K walks 351 / 296, 493 / 414
+// (with q > 1 the searches take most of the time, and they go three probes at once
+// where there is a table).
+static int64_t hop_walks(bool second_order, double p, double q) {
+  if (!second_order) return int64_t(1) << 14;
+  if (q <= 1.0) return int64_t(1) << 11;
+  return rare_picks(p, q) ? int64_t(1) << 13 : int64_t(1) << 15;
+}
 
 template <typename IdT>
 static int random_walk(const int64_t* indptr, const IdT* indices, const Hop* hops,
@@ -231,7 +252,7 @@ static int random_walk(const int64_t* indptr, const IdT* indices, const Hop* hop
                                               dim3(threads), 0, s>>>(                            \
                 indptr, indices, hops, num_cols, seeds, num_seeds, walk_length,                  \
                 make_key(seed, call_id), out_traces))
-  if (hops && num_seeds <= kHopWalks) GS_RANDOM_WALK(true);
+  if (hops && num_seeds <= hop_walks(false, 1.0, 1.0)) GS_RANDOM_WALK(true);
   else GS_RANDOM_WALK(false);
 #undef GS_RANDOM_WALK
   return GS_OK;
@@ -251,8 +272,7 @@ static int node2vec(const int64_t* indptr, const IdT* indices, const Hop* hops, 
   // As many lanes a walk as keep the call's lanes below what fills the machine:
   // 200 K where most candidates are accepted, 400 K where an accepted one is rare
   // (the best of 1, 2, 4, 8, 16 lanes at 1 K to 1 M walks).
-  const double most = p > q ? p : q, least = p < q ? p : q;
-  const int64_t lanes = (least < 1.0 ? least : 1.0) * 4.0 < most ? 400000 : 200000;
+  const int64_t lanes = rare_picks(p, q) ? 400000 : 200000;
   int group = 16;
   while (group > 1 && num_seeds * group > lanes) group >>= 1;
   const int threads = num_seeds * group < kFewWalks ? kWave : kBlock;
@@ -262,7 +282,7 @@ static int node2vec(const int64_t* indptr, const IdT* indices, const Hop* hops, 
                                               dim3(threads), 0, s>>>(                           \
                 indptr, indices, hops, num_cols, seeds, num_seeds, walk_length, p, q,           \
                 make_key(seed, call_id), out_traces))
-  const bool use_hops = hops && num_seeds <= kHopWalks;
+  const bool use_hops = hops && num_seeds <= hop_walks(true, p, q);
   if (group == 16) {
     if (use_hops) GS_NODE2VEC(16, true);
     else GS_NODE2VEC(16, false);
@@ -296,6 +316,10 @@ int gs_hop_table(const int64_t* indptr, int64_t num_cols, const int64_t* indices
             hop_table_kernel<<<dim3((unsigned)ceil_div(nnz, kBlock)), dim3(kBlock), 0, s>>>(
                 indptr, num_cols, indices, nnz, (Hop*)hops));
   return GS_OK;
+}
+
+int64_t gs_hop_walks(int second_order, double p, double q) {
+  return gs::hop_walks(second_order != 0, p, q);
 }
 
 int gs_random_walk(const int64_t* indptr, const int64_t* indices, int64_t num_cols,

@@ -680,9 +680,9 @@ int gs_sorted_to_indptr(const int64_t* sorted_ids, int64_t nnz, int64_t num_cols
  *    src/cuda/fusion/random_walk.cu:49-70.
  *  gs_hop_table: for every edge, where the column of its row id starts and how
  *    long it is (8 bytes per edge, fewer than 2^32 edges), for walks that go on
- *    from that edge.  The _hops forms take it (nullable; used while a call is bound
- *    by the latency of its chains of loads, up to 2^15 walks), gs_node2vec_hops also
- *    an int32 copy of the row ids (nullable); the traces are the same.
+ *    from that edge.  The _hops forms take it (nullable; used for calls of up to
+ *    gs_hop_walks walks), gs_node2vec_hops also an int32 copy of the row ids
+ *    (nullable); the traces are the same.
  *  gs_node2vec: second-order walk by rejection sampling with integer levels
  *    (return weight p, neighbour-of-previous weight q, otherwise 1); needs row
  *    ids sorted inside every column.  FusedNode2VecCUDA,
@@ -709,6 +709,7 @@ int gs_node2vec_hops(const int64_t* indptr, const int64_t* indices, const int32_
                      const void* hops, int64_t num_cols, const int64_t* seeds, int64_t num_seeds,
                      int64_t walk_length, double p, double q, uint64_t seed, uint64_t call_id,
                      int64_t* out_traces, gs_stream_t stream);
+int64_t gs_hop_walks(int second_order, double p, double q);
 int gs_hop_table(const int64_t* indptr, int64_t num_cols, const int64_t* indices, int64_t nnz,
                  void* hops, gs_stream_t stream);
 int gs_node2vec(const int64_t* indptr, const int64_t* indices, int64_t num_cols,

@@ -87,3 +87,20 @@ def test_node2vec_on_int32_ids(wide_world, n, length, p, q):
 @pytest.mark.parametrize("n,length", [(1000, 17), (32768, 9), (40000, 8)])
 def test_random_walk_on_a_wide_matrix(wide_world, n, length):
     test_random_walk(wide_world, n, length)
+
+
+@pytest.mark.parametrize("n,p,q,makes", [
+    (16384, None, None, True), (16385, None, None, False),            # first order
+    (2048, 2.0, 0.5, True), (2049, 2.0, 0.5, False), (8193, 0.25, 4.0, False),
+])
+def test_hop_table_is_made_for_calls_that_use_it_only(world, n, p, q, makes):
+    _, nodes, indptr, indices, _ = world
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    seeds = torch.arange(n, device=DEV) % nodes
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        m.random_walk(seeds, 3) if p is None else m.node2vec(seeds, 3, p, q)
+    grown = torch.cuda.memory_allocated() - before
+    assert (grown >= 8 * indices.size) == makes and (makes or grown == 0)
