@@ -216,6 +216,9 @@ static bool rare_picks(double p, double q) {
   return (least < 1.0 ? least : 1.0) * 4.0 < most;
 }
 
+// Whether the first candidate stands, all but once in 2^24 (the only level is 0).
+static bool sure_picks(double p, double q) { return p <= 1.0 && q <= 1.0; }
+
 // Up to how many walks a call goes by the hop table.  Few walks are bound by the
 // latency of their chains of loads, which the table shortens; more are bound by lines,
 // of which it costs as many as it saves -- a second line a candidate for a group that
@@ -224,6 +227,7 @@ static bool rare_picks(double p, double q) {
 //   first order, 56 steps     1 K walks 47 / 32    16 K 49 / 38     24 K 51 / 51, 33 K 53 / 69
 //     (measured with picks stored eight at a time)
 //   second order, 40 steps
+//     max(p, q) <= 1          one lane without the table is as fast (first candidates stand)
 //     q < 1 (no search)       2 K walks 44 / 35 and 45 / 37         4 K 46 / 49, 8 K 51 / 95
 //     q > 1, picks rare       8 K walks 286 / 243                   16 K 322 / 461
 //     q > 1, others           32 K walks 351 / 296, 493 / 414
@@ -231,6 +235,7 @@ static bool rare_picks(double p, double q) {
 // where there is a table).
 static int64_t hop_walks(bool second_order, double p, double q) {
   if (!second_order) return int64_t(1) << 14;
+  if (sure_picks(p, q)) return 0;
   if (q <= 1.0) return int64_t(1) << 11;
   return rare_picks(p, q) ? int64_t(1) << 13 : int64_t(1) << 15;
 }
@@ -271,10 +276,12 @@ static int node2vec(const int64_t* indptr, const IdT* indices, const Hop* hops, 
   hipStream_t s = as_stream(stream);
   // As many lanes a walk as keep the call's lanes below what fills the machine:
   // 200 K where most candidates are accepted, 400 K where an accepted one is rare
-  // (the best of 1, 2, 4, 8, 16 lanes at 1 K to 1 M walks).
+  // (the best of 1, 2, 4, 8, 16 lanes at 1 K to 1 M walks); one lane where the first
+  // candidate stands (32 K walks of 20 steps on 9 M edges: 22 us, with four lanes 35).
   const int64_t lanes = rare_picks(p, q) ? 400000 : 200000;
   int group = 16;
   while (group > 1 && num_seeds * group > lanes) group >>= 1;
+  if (sure_picks(p, q)) group = 1;
   const int threads = num_seeds * group < kFewWalks ? kWave : kBlock;
 #define GS_NODE2VEC(G, HOPS)                                                                    \
   GS_LAUNCH("node2vec", s,                                                                      \
@@ -351,7 +358,10 @@ int gs_node2vec_hops(const int64_t* indptr, const int64_t* indices, const int32_
                      int64_t walk_length, double p, double q, uint64_t seed, uint64_t call_id,
                      int64_t* out_traces, gs_stream_t stream) {
   const gs::Hop* h = (const gs::Hop*)hops;
-  if (indices32)
+  // (a lane that takes its first candidate is bound by the latency of its loads while
+  // there are few of them, and a 64-bit id needs no widening: 16 K walks of 20 steps
+  // 20.8 us, 23.6 with the narrow ids; from 64 K walks on those are ahead)
+  if (indices32 && !(gs::sure_picks(p, q) && num_seeds < gs::kFewWalks))
     return gs::node2vec(indptr, indices32, h, num_cols, seeds, num_seeds, walk_length, p, q, seed,
                         call_id, out_traces, stream);
   return gs::node2vec(indptr, indices, h, num_cols, seeds, num_seeds, walk_length, p, q, seed,

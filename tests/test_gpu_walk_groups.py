@@ -104,3 +104,11 @@ def test_hop_table_is_made_for_calls_that_use_it_only(world, n, p, q, makes):
         m.random_walk(seeds, 3) if p is None else m.node2vec(seeds, 3, p, q)
     grown = torch.cuda.memory_allocated() - before
     assert (grown >= 8 * indices.size) == makes and (makes or grown == 0)
+
+
+# max(p, q) <= 1: one lane a walk takes its first candidate, by 64-bit ids below 2^16 walks
+@pytest.mark.parametrize("n,length,p,q", [(1, 9, 0.5, 0.25), (2000, 17, 1.0, 0.5), (30000, 9, 0.25, 0.25),
+                                          (65535, 5, 1.0, 1.0), (65536, 5, 1.0, 1.0), (65536, 5, 0.5, 1.0)])
+def test_node2vec_whose_first_candidates_stand(world, wide_world, n, length, p, q):
+    test_node2vec(world, n, length, p, q)
+    test_node2vec(wide_world, n, length, p, q)
