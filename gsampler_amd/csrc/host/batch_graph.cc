@@ -101,7 +101,7 @@ static MajorResult compact_slice(const Compressed& m, const torch::Tensor& cols,
   torch::Tensor key_offset = new_ids(n, m.indptr);
   *row_bptr = new_ids(B + 1, m.indptr);
   torch::Tensor ws = new_workspace(gs_slice_compact_workspace_bytes(B, stride), m.indptr);
-  const torch::Tensor narrow = m.narrow_indices();
+  const torch::Tensor narrow = m.narrow_indices(nnz);  // two passes read every id of the slice
   const int32_t* ids32 = narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr;
   int64_t* mirror = OffsetMirror::reserve(*row_bptr);
   GS_CALL(gs_slice_compact_count(cptr(m.indptr), cptr(m.indices), ids32, cptr(cols), n,

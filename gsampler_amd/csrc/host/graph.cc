@@ -240,17 +240,20 @@ Compressed::Derived& Compressed::current_derived() const {
 
 // The int32 copy pays from a few megabytes of ids on (below that the int64
 // array stays in cache anyway); undefined when the matrix does not qualify.
-torch::Tensor Compressed::narrow_indices() const {
+torch::Tensor Compressed::narrow_indices(int64_t reads) const {
   constexpr int64_t kMinEdges = int64_t(1) << 20;
   if (indices.numel() < kMinEdges || num_minor < 0 || num_minor >= (int64_t(1) << 31) ||
-      !indices.is_cuda() || capturing())
+      !indices.is_cuda())
     return {};
   std::lock_guard<std::mutex> lock(derived_.guard);
   Derived& d = current_derived();
-  if (!narrow_ids_allowed().load())
+  if (!narrow_ids_allowed().load()) {
     d.narrow.drop();
-  else if (!d.narrow.defined())
-    d.narrow.set(indices.to(torch::kInt32));
+    return {};
+  }
+  if (!d.narrow.defined() && reads >= 0 && (d.reads += reads) < indices.numel()) return {};
+  if (capturing()) return {};
+  if (!d.narrow.defined()) d.narrow.set(indices.to(torch::kInt32));
   return d.narrow.on_current_stream();
 }
 

@@ -71,9 +71,11 @@ struct Compressed {
   // the current stream is being captured: the graph would record the kernel that fills
   // the table, or read one that a later edit of the matrix frees.
   //
-  // int32 copy of `indices` (half the bytes behind every random pick); made on the
-  // first sampling call of a matrix in device memory whose ids fit.
-  torch::Tensor narrow_indices() const;
+  // int32 copy of `indices` (half the bytes behind every random pick), of a matrix in
+  // device memory whose ids fit.  A sampler makes it on its first call; an operator that
+  // gains less tells how many ids it is about to read, and makes the copy once the reads
+  // so told come to as many as the matrix has edges.
+  torch::Tensor narrow_indices(int64_t reads = -1) const;
   // Where the column behind every edge lies (gs_hop_table), for walks over a
   // square matrix; made at the second walk over the same matrix.
   torch::Tensor hop_table() const;
@@ -82,11 +84,11 @@ struct Compressed {
     DerivedTable narrow, hops;
     int64_t versions[2] = {-1, -1}, epoch = -1;
     const void* source = nullptr;
-    int64_t walks = 0;
+    int64_t walks = 0, reads = 0;
     void drop() {
       narrow.drop();
       hops.drop();
-      walks = 0;
+      walks = reads = 0;
     }
   };
   Compressed() = default;

