@@ -141,6 +141,37 @@ __device__ __forceinline__ void store_for_host(int64_t* p, int64_t v) {
 // ------------------------------------------------------------- wave helpers
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
+// Floyd's subset sampling, one lane per output slot: slot i of a column is lane
+// gbase + i of the wavefront (K <= 64 slots, all of them active).  Slot i draws t_i in
+// [0, j_i], j_i = deg - K + i, and keeps t_i unless an earlier slot already holds it, in
+// which case it keeps j_i.  "Already held" <=> some earlier slot drew the same t, or
+// t_i equals the j_m of an earlier slot m that fell back to j_m; m is then unique
+// (m = t_i - (deg - K)), so the fall-back flags form a chain that is settled by
+// visiting slots in increasing order.  Returns the slot's offset inside the column.
+__device__ __forceinline__ int64_t floyd_exchange(int lane, int gbase, int K, int64_t deg,
+                                                  int64_t t) {
+  const int64_t base = deg - K;
+  bool dup = false;
+  for (int m = 0; m < K; ++m) {
+    const int64_t tm = __shfl(t, gbase + m, kWave);
+    dup |= (m < lane) & (tm == t);
+  }
+  const int64_t mi = t - base;  // slot whose j equals my t, if in [0, lane)
+  for (int m = 0; m < K; ++m) {
+    const int dm = __shfl((int)dup, gbase + m, kWave);
+    if (mi == m && m < lane) dup |= (dm != 0);
+  }
+  return dup ? base + lane : t;
+}
+
+// The same with the draws of (key, pos).
+__device__ __forceinline__ int64_t floyd_slot(int lane, int gbase, int K, int64_t deg,
+                                              PhiloxKey key, uint64_t pos) {
+  return floyd_exchange(lane, gbase, K, deg,
+                        (int64_t)philox_bounded(key, pos, (uint64_t)lane,
+                                                (uint64_t)(deg - K + lane) + 1));
+}
+
 // The first active lane's value, in every lane.
 __device__ __forceinline__ int64_t wave_uniform_first(int64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);

@@ -125,26 +125,6 @@ __device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask,
   return 0;
 }
 
-// Floyd's rule among the lanes of one column (sampling.hip): lane `lane` of the
-// `K` from wavefront lane gbase on.
-__device__ __forceinline__ int64_t floyd_pick(int lane, int gbase, int K, int64_t deg,
-                                              PhiloxKey key, uint64_t pos) {
-  const int64_t base = deg - K;
-  const int64_t j = base + lane;
-  const int64_t t = (int64_t)philox_bounded(key, pos, (uint64_t)lane, (uint64_t)j + 1);
-  bool dup = false;
-  for (int m = 0; m < K; ++m) {
-    const int64_t tm = __shfl(t, gbase + m, kWave);
-    dup |= (m < lane) & (tm == t);
-  }
-  const int64_t mi = t - base;
-  for (int m = 0; m < K; ++m) {
-    const int dm = __shfl((int)dup, gbase + m, kWave);
-    if (mi == m && m < lane) dup |= (dm != 0);
-  }
-  return dup ? j : t;
-}
-
 // picked: rows drawn by another kernel, fanout places per column; null: uniform.
 template <typename IdT>
 __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
@@ -197,7 +177,7 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
       } else if (deg <= fanout) {
         if (j < deg) row = (int64_t)indices[start + j];
       } else {
-        row = (int64_t)indices[start + floyd_pick((int)j, group * width + 1, fanout, deg, key,
+        row = (int64_t)indices[start + floyd_slot((int)j, group * width + 1, fanout, deg, key,
                                                   (uint64_t)c)];
       }
     }

@@ -73,32 +73,6 @@ __device__ __forceinline__ void sample_column_generic(
   }
 }
 
-// Floyd's subset sampling, one lane per output slot: slot i of a column is lane
-// gbase + i of the wavefront (K <= 64 slots).  Slot i draws t_i in [0, j_i],
-// j_i = deg - K + i, and keeps t_i unless an earlier slot already holds it, in
-// which case it keeps j_i.  "Already held" <=> some earlier slot drew the same
-// t, or t_i equals the j_m of an earlier slot m that fell back to j_m; m is
-// then unique (m = t_i - (deg - K)), so the fall-back flags form a chain that
-// is settled by visiting slots in increasing order.  Returns the slot's offset
-// inside the column.
-__device__ __forceinline__ int64_t floyd_slot_packed(int lane, int gbase, int K, int64_t deg,
-                                                     PhiloxKey key, uint64_t pos) {
-  const int64_t base = deg - K;
-  const int64_t j = base + lane;
-  const int64_t t = (int64_t)philox_bounded(key, pos, (uint64_t)lane, (uint64_t)j + 1);
-  bool dup = false;
-  for (int m = 0; m < K; ++m) {
-    const int64_t tm = __shfl(t, gbase + m, kWave);
-    dup |= (m < lane) & (tm == t);
-  }
-  const int64_t mi = t - base;  // slot whose j equals my t, if in [0, lane)
-  for (int m = 0; m < K; ++m) {
-    const int dm = __shfl((int)dup, gbase + m, kWave);
-    if (mi == m && m < lane) dup |= (dm != 0);
-  }
-  return dup ? j : t;
-}
-
 // One lane per output slot, a column on exactly `fanout` consecutive lanes: a
 // wavefront holds 64 / fanout columns (twelve at fanout 5, where power-of-two
 // groups would hold eight).  Lanes past the last whole slice idle.  On a
@@ -158,23 +132,11 @@ __global__ __launch_bounds__(kBlock) void sample_uniform_packed_kernel(
       r = philox_bounded(key, (uint64_t)item, (uint64_t)lane, (uint64_t)j + 1);
     }
     p = in_start + (int64_t)r;
-    if (!(kProbe & kProbeNoExchange)) {  // the exchange of floyd_slot_packed on these draws
-      const int gbase = group * fanout;
-      const int64_t t = (int64_t)r, base = deg - fanout;
-      bool dup = false;
-      for (int m = 0; m < fanout; ++m) {
-        const int64_t tm = __shfl(t, gbase + m, kWave);
-        dup |= (m < lane) & (tm == t);
-      }
-      const int64_t mi = t - base;
-      for (int m = 0; m < fanout; ++m) {
-        const int dm = __shfl((int)dup, gbase + m, kWave);
-        if (mi == m && m < lane) dup |= (dm != 0);
-      }
-      p = in_start + (dup ? j : t);
+    if (!(kProbe & kProbeNoExchange)) {  // the exchange of floyd_slot on these draws
+      p = in_start + floyd_exchange(lane, group * fanout, fanout, deg, (int64_t)r);
     }
   } else {
-    p = in_start + floyd_slot_packed(lane, group * fanout, fanout, deg, key, (uint64_t)item);
+    p = in_start + floyd_slot(lane, group * fanout, fanout, deg, key, (uint64_t)item);
   }
   if (p < 0) return;
   const int64_t v = (indices && !(kProbe & kProbeNoIndices)) ? (int64_t)indices[p] : p;
