@@ -188,5 +188,6 @@ class compile:  # noqa: N801 -- the reference's public name
         """Whether self.gm still is the module of __init__: its generated code is replaced
         when an edited graph is recompiled."""
         gm, forward = self._compiled
-        return (self.gm is gm and type(gm).forward is forward and "forward" not in gm.__dict__
-                and not gm._forward_hooks and not gm._forward_pre_hooks)
+        own = gm.__dict__
+        return (self.gm is gm and type(gm).forward is forward and "forward" not in own
+                and not own["_forward_hooks"] and not own["_forward_pre_hooks"])
