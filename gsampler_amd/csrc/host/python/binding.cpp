@@ -3,7 +3,7 @@
 // half a dozen tensors, and a call through torch's custom classes converts every
 // one of them through IValue lists.  Here the objects are filled directly, and the
 // blocks of the layers that are done are made while the host would otherwise wait
-// for the counts of the next one -- in a process with one Python thread.
+// for the counts of the next one, if nobody else wants the interpreter.
 //
 //   sample_layers(graph, seeds, fanouts, replace, weights)
 //       -> (frontier, row, col, None) per layer, one flat tuple
@@ -17,6 +17,8 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <structmember.h>
+
+#include <atomic>
 
 #include "../abi_call.h"
 #include "../graph.h"
@@ -136,11 +138,35 @@ c10::optional<torch::Tensor> optional_tensor(const py::object& o) {
   return py::cast<torch::Tensor>(o);
 }
 
-// The caller holds the interpreter.
-bool only_python_thread() {
-  PyThreadState* first = PyInterpreterState_ThreadHead(PyThreadState_Get()->interp);
-  return PyThreadState_Next(first) == nullptr;
-}
+// Whether the interpreter can be had at once: nobody holds it.  (Asked by a thread that
+// has let go of it; up to Python 3.11 the running thread's state is the process's, later
+// a thread sees its own only, and the answer is whether there is another thread at all.)
+class Interpreter {
+ public:
+  Interpreter() {
+#if PY_VERSION_HEX >= 0x030C0000
+    alone_ = PyThreadState_Next(PyInterpreterState_ThreadHead(PyThreadState_Get()->interp)) == nullptr;
+#endif
+  }
+  bool is_free() const {
+#if PY_VERSION_HEX >= 0x030C0000
+    return alone_;
+#else
+    return _PyThreadState_UncheckedGet() == nullptr;
+#endif
+  }
+
+ private:
+  bool alone_ = true;
+};
+
+// Calls of batch_sample_layers under way, in all threads.
+std::atomic<int> g_calls{0};
+struct CallScope {
+  CallScope() { g_calls.fetch_add(1, std::memory_order_relaxed); }
+  ~CallScope() { g_calls.fetch_sub(1, std::memory_order_relaxed); }
+  static bool only_one() { return g_calls.load(std::memory_order_relaxed) == 1; }
+};
 
 py::tuple sample_layers(py::handle graph, torch::Tensor seeds, std::vector<int64_t> fanouts,
                         bool replace, py::object weights) {
@@ -174,18 +200,23 @@ std::vector<std::shared_ptr<Batch>> batch_sample_layers(py::handle graph, torch:
   auto w = optional_tensor(weights);
   std::vector<std::shared_ptr<Batch>> out;
   // called where the host is about to wait for a layer's counts, with the layers
-  // before it: their blocks are made now instead of after the wait.  Not beside other
-  // Python threads: one that holds the interpreter would keep the next layer's launches
-  // waiting, and every tensor of a block lets go of the interpreter when it is freed.
-  // (32 batches of 1024 on 2 M edges, blocks never asked for, 1 and 8 threads: 3020 and
-  // 635 passes a second with blocks made ahead, 3140 and 5130 without.)
-  gs::Graph::LayerDone done;
-  if (g_block.type && only_python_thread())
-    done = [&](c10::intrusive_ptr<gs::BlockBatch> b) {
+  // before it: their blocks are made now instead of after the wait.  Not while another
+  // thread holds the interpreter, which would keep the next layer's launches waiting,
+  // nor beside another sampler thread: every tensor of a block lets go of the
+  // interpreter when it is freed.  (32 batches of 1024 on 2 M edges, blocks never asked
+  // for, 1 and 8 threads: 3020 and 635 passes a second with blocks always made ahead,
+  // 3140 and 5130 without.)
+  const Interpreter interpreter;
+  const CallScope scope;
+  auto done = [&](c10::intrusive_ptr<gs::BlockBatch> b) {
+    if (g_block.type && CallScope::only_one() && interpreter.is_free()) {
       py::gil_scoped_acquire gil;
       out.push_back(std::make_shared<Batch>(std::move(b)));
       out.back()->make_ahead();
-    };
+    } else {
+      out.push_back(std::make_shared<Batch>(std::move(b)));
+    }
+  };
   std::vector<c10::intrusive_ptr<gs::BlockBatch>> got;
   {
     py::gil_scoped_release nogil;

@@ -168,29 +168,41 @@ def test_blocks_handed_out_twice_are_other_objects(rng, count):
         assert all(x is y for x, y in zip(list(first), first))       # a list keeps its blocks
 
 
-def test_no_blocks_are_made_ahead_beside_other_python_threads(rng):
-    """Making them needs the interpreter in the middle of a step, which another thread may
-    hold, and they may never be asked for."""
+def test_no_blocks_are_made_ahead_while_another_thread_holds_the_interpreter(rng):
+    """Making them would wait for it in the middle of a step, and they may never be asked for;
+    a thread that sleeps changes nothing."""
     bm = gs.BatchMatrix()
     bm.load_from_matrix(matrix(rng, 30000, 20, 0, False), False)
     seeds = torch.cat([torch.from_numpy(rng.permutation(30000)[:9000]) for _ in range(5)]).to(DEV)
     args = (bm, seeds, torch.arange(6, device=DEV) * 9000, [12, 10, 4], False)
     sampler = gs.jit.compile(func=batched, args=args)
     blocks = lambda: sum(type(o) is Block for o in gc.get_objects())  # noqa: E731
-    gc.collect()
-    before, stop = blocks(), threading.Event()
-    other = threading.Thread(target=stop.wait)
-    other.start()
-    try:
-        gs.manual_seed(5)
-        got = sampler(*args)
-        assert blocks() == before
-    finally:
-        stop.set()
-        other.join()
-    gs.manual_seed(5)
-    for layer, again in zip(got, sampler(*args)):
-        for x, y in zip(layer, again):
+    stop = threading.Event()
+
+    def made_ahead(target):
+        other = threading.Thread(target=target)
+        other.start()
+        try:
+            gs.manual_seed(5)
+            gc.collect()
+            before = blocks()
+            got = sampler(*args)
+            return got, blocks() - before
+        finally:
+            stop.set()
+            other.join()
+            stop.clear()
+
+    def spin():
+        while not stop.is_set():
+            pass
+
+    got, ahead = made_ahead(spin)
+    assert ahead == 0
+    again, ahead = made_ahead(stop.wait)
+    assert ahead == 10                               # two layers of five
+    for layer, other in zip(got, again):
+        for x, y in zip(layer, other):
             same(x, y)
 
 
