@@ -13,21 +13,25 @@ namespace gs {
 
 // Offsets and size of A[:, cols]: shared by the operators of this file when
 // they are handed the same tensor of columns (one wait for the size, not two).
-const Graph::SliceOffsets& Graph::slice_offsets_for(const torch::Tensor& cols) {
+std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tensor& cols) {
   const Compressed& m = compressed(kCSC);
-  if (slice_offsets_ && slice_offsets_->cols.is_same(cols) &&
-      slice_offsets_->version == (int64_t)cols._version() &&
-      slice_offsets_->indptr_version == (int64_t)m.indptr._version() &&
-      slice_offsets_->epoch == cache_epoch())
-    return *slice_offsets_;
-  auto so = std::make_unique<SliceOffsets>();
+  {
+    std::lock_guard<std::mutex> lock(slice_offsets_guard_);
+    if (slice_offsets_ && slice_offsets_->cols.is_same(cols) &&
+        slice_offsets_->version == (int64_t)cols._version() &&
+        slice_offsets_->indptr_version == (int64_t)m.indptr._version() &&
+        slice_offsets_->epoch == cache_epoch())
+      return slice_offsets_;
+  }
+  auto so = std::make_shared<SliceOffsets>();
   so->cols = cols;
   so->version = cols._version();
   so->indptr_version = m.indptr._version();
   so->epoch = cache_epoch();
   so->sub_indptr = slice_offsets(m, cols, &so->nnz);
-  slice_offsets_ = std::move(so);
-  return *slice_offsets_;
+  std::lock_guard<std::mutex> lock(slice_offsets_guard_);
+  slice_offsets_ = so;
+  return so;
 }
 
 // Reading a slice in place pays when its columns are long: the kernels look a
@@ -39,10 +43,9 @@ bool Graph::read_in_place(int64_t slice_nnz, int64_t num_cols_picked) {
   return slice_nnz >= (int64_t(1) << 20) && slice_nnz >= 4096 * num_cols_picked;
 }
 
-const MajorResult& Graph::written_slice(const torch::Tensor& cols) {
-  slice_offsets_for(cols);
-  SliceOffsets& so = *slice_offsets_;
-  if (!so.written.indptr.defined()) so.written = major_slice(compressed(kCSC), cols, true, {}, 0);
+const MajorResult& Graph::written_slice(SliceOffsets& so) {
+  std::lock_guard<std::mutex> lock(so.guard);
+  if (!so.written.indptr.defined()) so.written = major_slice(compressed(kCSC), so.cols, true, {}, 0);
   return so.written;
 }
 
@@ -61,10 +64,11 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
               " edge values for ", m.indices.numel(), " edges (scalar edge values only)");
   TORCH_CHECK(out.numel() == num_rows_, "SlicedESquareSum: out has ", out.numel(),
               " entries for ", num_rows_, " rows");
-  const SliceOffsets& so = slice_offsets_for(cols);
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
+  SliceOffsets& so = *shared;
   if (so.nnz == 0) return;
   if (!read_in_place(so.nnz, cols.numel())) {
-    const MajorResult& r = written_slice(cols);
+    const MajorResult& r = written_slice(so);
     torch::Tensor w = efeat.index_select(0, edge_index(m.e_ids, r.select));
     torch::Tensor ws =
         new_workspace(gs_spmm_workspace_bytes(GS_FMT_COO, so.nnz, num_rows_), m.indptr);
@@ -131,13 +135,14 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   cols = ids(cols, "cols");
   rows = ids(rows, "rows");
   const Compressed& m = compressed(kCSC);
-  const SliceOffsets& so = slice_offsets_for(cols);
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
+  SliceOffsets& so = *shared;
   MajorResult r;
   if (read_in_place(so.nnz, cols.numel())) {
     r = col_row_slice(m, cols, so.sub_indptr, so.nnz, torch::Tensor(), rows,
                       output_format & kCOO);
   } else {
-    const MajorResult& sliced = written_slice(cols);
+    const MajorResult& sliced = written_slice(so);
     Compressed tmp(sliced.indptr, sliced.minor_ids);
     r = minor_slice(tmp, rows, output_format & kCOO);
     r.select = sliced.select.index_select(0, r.select);
@@ -172,7 +177,8 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   };
   torch::Tensor key_offset = batch_of(col_bptr, col.numel()) * stride;
   torch::Tensor picked = row + batch_of(row_bptr, row.numel()) * stride;
-  const SliceOffsets& so = slice_offsets_for(col);
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(col);
+  SliceOffsets& so = *shared;
   MajorResult kept;
   if (read_in_place(so.nnz, col.numel())) {
     kept = col_row_slice(m, col, so.sub_indptr, so.nnz, key_offset, picked, false);

@@ -405,16 +405,19 @@ class Graph : public torch::CustomClassHolder {
 
   const Compressed& compressed(int64_t format);
   // Offsets and size of the column slice A[:, cols], kept for the next operator
-  // that is handed the same tensor of columns.
+  // that is handed the same tensor of columns.  (Sampler threads share the matrix: what
+  // one holds stays when another puts its own in its place.)
   struct SliceOffsets {
     torch::Tensor cols, sub_indptr;
     int64_t version = -1, indptr_version = -1, epoch = -1, nnz = 0;
+    std::mutex guard;
     MajorResult written;  // the slice itself, when an operator had to write it
   };
-  std::unique_ptr<SliceOffsets> slice_offsets_;
-  const SliceOffsets& slice_offsets_for(const torch::Tensor& cols);
+  std::mutex slice_offsets_guard_;
+  std::shared_ptr<SliceOffsets> slice_offsets_;
+  std::shared_ptr<SliceOffsets> slice_offsets_for(const torch::Tensor& cols);
   static bool read_in_place(int64_t slice_nnz, int64_t num_cols_picked);
-  const MajorResult& written_slice(const torch::Tensor& cols);
+  const MajorResult& written_slice(SliceOffsets& so);
   // CDF of edge_probs in the edge order of `format` (cached per weights tensor).
   torch::Tensor weight_cdf_for(const torch::Tensor& edge_probs, int64_t format);
   void check_reduce_operands(const std::string& op, const torch::Tensor& ufeat,

@@ -3,10 +3,13 @@ pass over the parent matrix and the row sums of squared edge values of A[:, cols
 Checked against the CPU operators chained by hand (column slice, then row slice or
 sum over the slice): what the reference computes through the intermediate slice
 (src/cuda/fusion/column_row_slicing.cu:148-217, src/graph.cc:457-480)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
 
+import gsampler_amd as gs
 from gsampler_amd import capi
 from oracle import binding as orc
 from tests.conftest import random_csc
@@ -123,3 +126,43 @@ def test_sliced_e_square_sum_parity(ncol, num_rows, use_workspace):
     cpu = orc.e_square_sum(("coo", sub_rows[ok], np.zeros(int(ok.sum()), dtype=np.int64)),
                            w[sel][ok], 2, num_rows)
     assert np.allclose(cpu, want, rtol=1e-5, atol=1e-30)
+
+
+def test_threads_with_other_columns_on_one_matrix():
+    """What an operator holds of a slice stays when another thread's takes its place."""
+    rng = np.random.default_rng(21)
+    deg = rng.integers(100, 9000, size=700)
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    indices = rng.integers(0, 20_000, size=int(deg.sum()))
+    g = gs.Graph(20_000, 700)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor((rng.random(indices.size) + 0.05).astype(np.float32), device=DEV)
+    rows = T(rng.choice(20_000, size=300, replace=False))
+    # short columns' slices are written, long ones' read in place
+    cols = [T(rng.integers(0, 700, size=n)) for n in (3, 40, 300, 500)]
+
+    def once(c):
+        out = torch.zeros(20_000, device=DEV)
+        g._CAPI_SlicedESquareSum(c, w, out)
+        sub, index = g._CAPI_ColRowSlicing(c, rows, gs.format._CSC, gs.format._CSC)
+        return out, sub._CAPI_GetCSCIndptr(), sub._CAPI_GetCSCIndices(), index
+
+    want = [once(c) for c in cols]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(40):
+                got = once(cols[i].clone())
+                same_ids = all(torch.equal(a, b) for a, b in zip(got[1:], want[i][1:]))
+                # two orders of adding some hundred 32-bit terms: 1e-5 apart at most
+                if not (same_ids and torch.allclose(got[0], want[i][0], rtol=1e-5)):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
