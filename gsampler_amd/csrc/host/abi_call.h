@@ -39,8 +39,9 @@ inline std::atomic<int64_t>& cache_epoch_counter() {
 inline int64_t cache_epoch() { return cache_epoch_counter().load(std::memory_order_relaxed); }
 inline void invalidate_caches() { cache_epoch_counter().fetch_add(1); }
 
-// Whether a loaded matrix may keep an int32 copy of its ids for the uniform
-// sampler (4 bytes per edge of device memory for half the bytes behind a pick).
+// Whether a loaded matrix may keep tables made from its ids: an int32 copy (4 bytes
+// per edge for half the bytes behind a pick) and the hop table of its walks (8 bytes
+// per edge, matrices of up to 2^24 edges).
 inline std::atomic<bool>& narrow_ids_allowed() {
   static std::atomic<bool> on{true};
   return on;

@@ -29,7 +29,8 @@ static int64_t abi_version() { return gs_abi_version(); }
 // pointer, another extension, a replayed HIP graph): forget everything derived
 // from tensor contents.
 static void invalidate_all_caches() { invalidate_caches(); }
-// Whether loaded matrices may keep an int32 copy of their ids (on by default).
+// Whether loaded matrices may keep an int32 copy of their ids and the hop table of
+// their walks (on by default).
 static void set_narrow_ids(bool on) { narrow_ids_allowed().store(on); }
 
 }  // namespace gs

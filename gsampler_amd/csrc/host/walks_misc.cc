@@ -14,6 +14,10 @@ torch::Tensor Compressed::hop_table() const {
   if (nnz == 0 || nnz > kMaxEdges || !indices.is_cuda() || !indptr.is_cuda()) return {};
   std::lock_guard<std::mutex> lock(derived_.guard);
   Derived& d = current_derived();
+  if (!narrow_ids_allowed().load()) {
+    d.hops.drop();
+    return {};
+  }
   if (!d.hops.defined() && d.walks++ == 0) return {};
   if (capturing()) return {};
   if (!d.hops.defined()) {

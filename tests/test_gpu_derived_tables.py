@@ -138,3 +138,23 @@ def test_second_stream_waits_for_the_weights_cdf(arrays):
             for got, expected in zip(sample(m), want):
                 assert torch.equal(got, expected)
     torch.cuda.synchronize()
+
+
+def test_tables_can_be_switched_off(arrays):
+    n = 1000
+    seeds = torch.from_numpy(np.random.default_rng(2).integers(0, NODES, n)).to(DEV)
+    want = orc.random_walk(*arrays, seeds.cpu().numpy(), 20, 13, 0).reshape(21, n)
+    m = matrix(arrays)
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        gs.manual_seed(13)
+        assert np.array_equal(traces(m.random_walk(seeds, 20), n), want)
+    assert torch.cuda.memory_allocated() - before >= 8 * arrays[1].size
+    try:
+        torch.ops.gs_ops._CAPI_SetNarrowIds(False)
+        for _ in range(3):
+            gs.manual_seed(13)
+            assert np.array_equal(traces(m.random_walk(seeds, 20), n), want)
+        assert torch.cuda.memory_allocated() == before
+    finally:
+        torch.ops.gs_ops._CAPI_SetNarrowIds(True)
