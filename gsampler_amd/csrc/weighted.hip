@@ -491,77 +491,109 @@ __global__ __launch_bounds__(kBlock) void cdf_pack_kernel(
   }
 }
 
-// Search state of one draw over a column's entries col[1 .. deg] (col[j] is the
-// entry of item j - 1, so its share is the point where item j starts): the
-// item whose interval holds x is the last j in [0, deg) with start(j) <= x, for
-// start(0) = 0 <= x < start(deg) = the column's mass.  Shares of weights are
-// close to a straight line, so guesses interpolate; every other step (mode 1)
-// or every step after kInterpolations guesses (mode 2) is a plain bisection,
-// which bounds the worst case for any weights; mode 0 only bisects.  The entry
-// that last lowered `hi` stays at hand: when the search ends it is the entry
-// of the item found, row id included.
+// Search of one draw over a column's entries col[1 .. deg] (col[j] is the entry of
+// item j - 1, so its share is the point where item j starts): the item whose interval
+// holds x is the last j in [0, deg) with start(j) <= x, for start(0) = 0 <= x <
+// start(deg) = the column's mass.  Shares of weights are close to a straight line, so
+// kInterpolations guesses interpolate; every later step is a plain bisection, which
+// bounds the worst case for any weights.  Where a step looks never changes which item
+// the search ends at.
+//
+// A step looks at a window of four entries by two 16-byte loads: the line is paid for
+// by the first of them, and a draw ends after 2.0 dependent steps where one entry a
+// step took 3.7 (the slowest of 64 lanes 4.3 and 8.2; columns of a power law, lognormal
+// weights).  Windows lie at multiples of 32 bytes, so that they cross no line, but for
+// those at a column's ends, which are moved inside it: every entry of a window is one of
+// col[1 .. deg - 1], in order, so that one comparison an entry narrows both bounds.
+//
+// Positions are 32-bit from a base that the rare longer column is first bisected down
+// to, entries are compared as they lie in memory (share above row id; `beyond` is the
+// least entry that starts after x) and guesses are made from their upper words: a
+// wavefront of fan-out 5 takes 2770 vector instructions where 64-bit positions, shares
+// and guesses of double precision took 3960, 57 % of the issue slots.
 constexpr int kInterpolations = 8;
-// Search mode of the CDF sampler: 0 bisection, 1 alternating, 2 interpolation
-// first (the fastest on prefix sums of real weights, which are nearly linear).
-constexpr int kCdfSearchMode = 2;
+constexpr int kWindow = 4;
+typedef uint64_t EntryPair __attribute__((ext_vector_type(2), aligned(8)));
 struct CdfSearch {
-  int64_t lo, hi;
-  uint64_t a_lo, a_hi, x, e_hi;
-  int guesses;
-  bool flip;
-  __device__ __forceinline__ void begin(int64_t deg, uint64_t mass, uint64_t point) {
-    lo = 0;
-    hi = deg;
-    a_lo = 0;
-    a_hi = mass;
-    e_hi = 0;  // the column's last entry, which nobody has read yet
-    x = point;
-    guesses = 0;
-    flip = true;
-  }
-  __device__ __forceinline__ bool done() const { return hi - lo <= 1; }
-  __device__ __forceinline__ int64_t probe_at() {
-    constexpr int mode = kCdfSearchMode;
-    bool interpolate = false;
-    if (hi - lo > 8) {
-      if (mode == 1) interpolate = flip;
-      if (mode == 2) interpolate = guesses < kInterpolations;
-    }
-    flip = !flip;
-    if (!interpolate) return (lo + hi) >> 1;
-    ++guesses;
-    // (a guess: the hardware's approximate reciprocal will do, and where a probe
-    // lands never changes which item the search ends at)
-    const double frac = (double)(x - a_lo) * __builtin_amdgcn_rcp((double)(a_hi - a_lo));
-    int64_t mid = lo + (int64_t)(frac * (double)(hi - lo));
-    if (mid <= lo) mid = lo + 1;
-    if (mid >= hi) mid = hi - 1;
-    return mid;
-  }
-  __device__ __forceinline__ void narrow(int64_t mid, uint64_t entry, int row_bits) {
-    const uint64_t v = entry >> row_bits;
-    if (v <= x) {
+  int64_t base;       // item `lo` of the search is item base + lo of the column
+  uint32_t lo, hi;    // the item lies in [lo, hi)
+  uint64_t e_lo, e_hi;  // their entries (those of the column's bounds have no row id)
+  __device__ __forceinline__ void narrow(uint32_t mid, uint64_t entry, uint64_t beyond) {
+    if (entry < beyond) {
       lo = mid;
-      a_lo = v;
+      e_lo = entry;
     } else {
       hi = mid;
-      a_hi = v;
       e_hi = entry;
     }
   }
 };
 
-// Leaves the item in s.lo and its interval in [s.a_lo, s.a_hi); its entry is in
-// s.e_hi unless the search ended at the column's last item without having
-// looked at it (s.hi == deg).  `mass` is what the column's shares add up to.
-__device__ __forceinline__ void cdf_locate(CdfSearch& s, const uint64_t* __restrict__ col,
+// Leaves the item at s.base + s.lo, the entry it starts at in s.e_lo and the one it ends
+// at, which carries its row id, in s.e_hi -- unless the search ended at the column's
+// last item, whose entry it has not looked at (returns true).  `mass` is what the
+// column's shares add up to.
+__device__ __forceinline__ bool cdf_locate(CdfSearch& s, const uint64_t* __restrict__ col,
                                            int64_t deg, uint64_t mass, int row_bits,
                                            uint64_t x) {
-  s.begin(deg, mass, x);
-  while (!s.done()) {
-    const int64_t mid = s.probe_at();
-    s.narrow(mid, col[mid], row_bits);
+  const uint64_t beyond = (x + 1) << row_bits;
+  s.base = 0;
+  s.e_lo = 0;
+  s.e_hi = mass << row_bits;
+  int64_t rest = deg;
+  while (rest > 0x7FFFFFFFll) {
+    const int64_t half = rest >> 1;
+    const uint64_t entry = col[s.base + half];
+    if (entry < beyond) {
+      s.base += half;
+      rest -= half;
+      s.e_lo = entry;
+    } else {
+      rest = half;
+      s.e_hi = entry;
+    }
   }
+  const uint64_t* at = col + s.base;
+  s.lo = 0;
+  s.hi = (uint32_t)rest;
+  if (rest <= kWindow) {  // too short for a window
+    while (s.hi - s.lo > 1) {
+      const uint32_t mid = (s.lo + s.hi) >> 1;
+      s.narrow(mid, at[mid], beyond);
+    }
+    return s.base + s.hi == deg;
+  }
+  // windows begin at 1 .. rest - kWindow; `shift` entries above a multiple of 32 bytes
+  const uint32_t shift = (uint32_t)((uintptr_t)at >> 3) & (kWindow - 1);
+  const uint32_t last = (uint32_t)rest - kWindow;
+  int guesses = 0;
+  while (s.hi - s.lo > 1) {
+    uint32_t mid = (s.lo + s.hi) >> 1;
+    if (guesses < kInterpolations) {
+      ++guesses;
+      const float part = (float)(uint32_t)((beyond - s.e_lo) >> 32) *
+                         __builtin_amdgcn_rcpf((float)(uint32_t)((s.e_hi - s.e_lo) >> 32));
+      // (0/0, of shares closer than the upper words tell apart, is a step of 1)
+      const float range = (float)(s.hi - s.lo);
+      const uint32_t step = (uint32_t)fminf(fmaxf(part * range, 1.0f), range);
+      mid = s.lo + step < s.hi ? s.lo + step : s.hi - 1;
+    }
+    const uint32_t aligned = ((mid + shift) & ~(uint32_t)(kWindow - 1)) - shift;
+    const uint32_t first = (uint32_t)min(max((int32_t)aligned, 1), (int32_t)last);
+    const EntryPair p0 = *(const EntryPair*)(at + first);
+    const EntryPair p1 = *(const EntryPair*)(at + first + 2);
+    const bool b0 = p0.x < beyond, b1 = p0.y < beyond, b2 = p1.x < beyond, b3 = p1.y < beyond;
+    const uint32_t count = (uint32_t)b0 + b1 + b2 + b3;
+    if (b0) {
+      s.lo = first + count - 1;
+      s.e_lo = b3 ? p1.y : b2 ? p1.x : b1 ? p0.y : p0.x;
+    }
+    if (!b3) {
+      s.hi = first + count;
+      s.e_hi = !b0 ? p0.x : !b1 ? p0.y : !b2 ? p1.x : p1.y;
+    }
+  }
+  return s.base + s.hi == deg;
 }
 
 constexpr int kMaxCdfFanout = 64;
@@ -580,13 +612,25 @@ constexpr int kMaxCdfFanout = 64;
 // bookkeeping of repeats alone was half of the kernel's time.
 // With replacement: one independent point of the whole mass per output slot.
 // Streams: pos = column position, draw = output slot.
-// The taken intervals live in registers: every access runs over all KMAX slots
-// with a predicate instead of indexing.
-// (Fan-out 10 takes 134 registers left alone: capped at 128 it runs four wavefronts
-// per SIMD instead of three, 342 against 362 us on 592 K columns; the same cap for 15
-// and 16 spills more than it gains.)
+// The taken intervals live in registers, in the order of their starts: every access
+// runs over the slots with a predicate instead of indexing.
+// The picks wait in LDS, packed as the wavefront's columns write them, and leave
+// together at the end: neighbouring lanes then store neighbouring outputs, whole lines
+// at a time (3.5 M columns with fanout 5: 4.5 M write requests of 64 bytes, 6.6 M when
+// they were held in registers and stored by their own lanes, 33 M stored pick by pick).
+// Work-groups are one wavefront where the picks of four would not leave room for others.
+// What bounds it, 3.5 M columns of a 124 M-edge power-law graph, fanout 5: lines, 6.6 a
+// column at 43 G/s of the part's 48; 540 us (698 with a search of one entry a step and
+// the picks in registers).  592 K columns with fanout 10: 232 us (322), 65 K with fanout
+// 15, one wavefront a SIMD and so its own chain of loads: 77 us (89).
+// (Fan-outs up to 10 are capped at 128 registers, four wavefronts a SIMD: 250 us with
+// three for fanout 10.  Three for fanout 5 leave more lines in L2 between the draws of a
+// column, 5.7 a column, and take 607 us.  Non-temporal stores change nothing.)
 template <int KMAX>
-__global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cdf_kernel(
+constexpr int kCdfThreads = KMAX <= 16 ? kBlock : kWave;
+
+template <int KMAX>
+__global__ __launch_bounds__(kCdfThreads<KMAX>, KMAX <= 10 ? 4 : 1) void sample_weighted_cdf_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols,
     const int64_t* __restrict__ indices, const uint64_t* __restrict__ cdf,
     const int64_t* __restrict__ column_ids, int64_t num_items, int fanout,
@@ -594,18 +638,23 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
     int64_t* __restrict__ out_coo_col, int64_t* __restrict__ out_indices,
     int64_t* __restrict__ out_select, ColumnLabels labels,
     const int64_t* __restrict__ col_span, const int64_t* __restrict__ num_dev) {
-  const int64_t item = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (item >= (num_dev ? *num_dev : num_items)) return;
-  // (asked for here, so that its loads travel with the ones below)
-  const int64_t col_label =
-      out_coo_col ? labels.of_near(item, item - lane_id()) : item;
+  constexpr int kThreads = kCdfThreads<KMAX>;
+  __shared__ uint2 s_pick[kThreads * KMAX];  // offset in the column, row id
+  __shared__ uint8_t s_owner[kThreads * KMAX];
+  uint2* const wave_pick = s_pick + threadIdx.x / kWave * (kWave * KMAX);
+  uint8_t* const wave_owner = s_owner + threadIdx.x / kWave * (kWave * KMAX);
+  const int64_t item = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const bool live = item < (num_dev ? *num_dev : num_items);
   const int row_bits = (int)cdf[0];  // the same word for every lane: a scalar load
   const uint64_t row_mask = row_bits ? (~0ull >> (64 - row_bits)) : 0ull;
-  int64_t in_start;
-  const int64_t deg = column_span(col_span, column_ids, indptr, num_cols, item, &in_start);
-  if (deg == 0) return;
-  // (without offsets every column has `fanout` places of its own)
-  const int64_t out_start = sub_indptr ? sub_indptr[item] : item * fanout;
+  int64_t col_label = item, in_start = 0, out_start = 0, deg = 0;
+  if (live) {
+    // (asked for here, so that its loads travel with the ones below)
+    if (out_coo_col) col_label = labels.of_near(item, item - lane_id());
+    deg = column_span(col_span, column_ids, indptr, num_cols, item, &in_start);
+    // (without offsets every column has `fanout` places of its own)
+    out_start = sub_indptr ? sub_indptr[item] : item * fanout;
+  }
   const uint64_t* col = cdf + in_start;  // col[j], 1 <= j <= deg: entry of item j - 1
   // A column's shares add up to 2^cb - 1, or to 0 when it has no positive weight.
   // Which of the two is in the column's last entry, one more random line that a
@@ -613,56 +662,46 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
   // (in a column without mass the first search does: every share is 0).
   const int cb = 64 - row_bits < 62 ? 64 - row_bits : 62;
   const uint64_t full = (1ull << cb) - 1ull;
-  auto row_of = [&](int64_t off, uint64_t entry) -> int64_t {
-    if (row_bits) return (int64_t)(entry & row_mask);
-    return indices ? indices[in_start + off] : in_start + off;
-  };
-  // The picks of a column wait in registers (offset and row id) and leave
-  // together at the end, so that a lane's outputs reach each array back to
-  // back and the wavefront fills whole lines where pick-by-pick stores leave
-  // partial lines to be evicted and reopened (measured on 3.5 M columns with
-  // fanout 5: 33 M write requests and 1.8 ms pick by pick, 1.2 ms held).  What
-  // does not fit the registers is written pick by pick: columns of 2^32 or
-  // more items (no graph seen so far has one, nothing forbids it) and fanouts
-  // above KMAX, which only occur with replacement.
+  // What does not fit is written pick by pick: columns of 2^32 or more items (no graph
+  // seen so far has one, nothing forbids it) and fanouts above KMAX, which only occur
+  // with replacement.
   const bool hold = deg <= 0xFFFFFFFFll && fanout <= KMAX;
-  uint32_t held[KMAX], held_row[KMAX];
-#pragma unroll
-  for (int i = 0; i < KMAX; ++i) held[i] = held_row[i] = 0;
-  int taken = 0;
-  auto pick = [&](int64_t off, uint64_t entry) {
-    if (!hold) {
-      const int64_t p = in_start + off;
-      out_indices[out_start + taken] = row_of(off, entry);
-      if (out_select) out_select[out_start + taken] = p;
-      if (out_coo_col) out_coo_col[out_start + taken] = col_label;
+  const int64_t picks = deg == 0 ? 0 : replace || deg > fanout ? fanout : deg;
+  const int held = hold ? (int)picks : 0;
+  const int held_end = wave_inclusive_sum(held), held_at = held_end - held;
+  auto pick_at = [&](int slot, int64_t off, uint64_t entry) {
+    if (hold) {
+      wave_pick[held_at + slot] = make_uint2((uint32_t)off, (uint32_t)(entry & row_mask));
+      wave_owner[held_at + slot] = (uint8_t)lane_id();
+      return;
     }
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i == taken) {
-        held[i] = (uint32_t)off;
-        held_row[i] = (uint32_t)(entry & row_mask);
-      }
-    ++taken;
+    const int64_t p = in_start + off;
+    out_indices[out_start + slot] =
+        row_bits ? (int64_t)(entry & row_mask) : indices ? indices[p] : p;
+    if (out_select) out_select[out_start + slot] = p;
+    if (out_coo_col) out_coo_col[out_start + slot] = col_label;
   };
   CdfSearch s;
-  if (replace) {
+  if (deg == 0) {
+  } else if (replace) {
     bool mass = true;
     for (int j = 0; j < fanout; ++j) {
-      if (mass) {
-        cdf_locate(s, col, deg, full, row_bits,
-                   philox_bounded(key, (uint64_t)item, (uint64_t)j, full));
-        if (s.hi == deg) {
-          s.e_hi = col[deg];
-          mass = (s.e_hi >> row_bits) != 0;
-        }
+      if (mass && cdf_locate(s, col, deg, full, row_bits,
+                             philox_bounded(key, (uint64_t)item, (uint64_t)j, full))) {
+        s.e_hi = col[deg];
+        mass = (s.e_hi >> row_bits) != 0;
       }
-      if (mass) pick(s.lo, s.e_hi);
-      else pick(deg - 1, s.e_hi);  // no positive weight: the last item
+      pick_at(j, mass ? s.base + s.lo : deg - 1, s.e_hi);  // no positive weight: the last item
     }
   } else if (deg <= fanout) {  // whole column, original order, zero weights included
-    for (int64_t j = 0; j < deg; ++j) pick(j, col[j + 1]);
+    uint64_t entry[KMAX];
+#pragma unroll
+    for (int i = 0; i < KMAX; ++i) entry[i] = col[i < deg ? i + 1 : deg];
+#pragma unroll
+    for (int i = 0; i < KMAX; ++i)
+      if (i < deg) pick_at(i, i, entry[i]);
   } else {
+    // the intervals taken so far, in the order of their starts
     uint64_t start[KMAX], len[KMAX];
 #pragma unroll
     for (int i = 0; i < KMAX; ++i) {
@@ -670,64 +709,61 @@ __global__ __launch_bounds__(kBlock, KMAX <= 10 ? 4 : 1) void sample_weighted_cd
       len[i] = 0;
     }
     uint64_t removed = 0;
-    while (taken < fanout && removed < full) {
-      const uint64_t r =
-          philox_bounded(key, (uint64_t)item, (uint64_t)taken, full - removed);
-      uint64_t x = r;
-      for (int round = 0; round <= taken; ++round) {
-        uint64_t skipped = 0;
+    int taken = 0;
+#pragma unroll 1
+    for (int j = 0; j < fanout; ++j) {
+      if (removed >= full) break;
+      // a point of the mass that is left, moved past the intervals before it
+      uint64_t x = philox_bounded(key, (uint64_t)item, (uint64_t)j, full - removed);
 #pragma unroll
-        for (int i = 0; i < KMAX; ++i) skipped += start[i] <= x ? len[i] : 0ull;
-        if (r + skipped == x) break;
-        x = r + skipped;
-      }
-      cdf_locate(s, col, deg, full, row_bits, x);
-      if (s.hi == deg) {  // ended at the last item without having read its entry
+      for (int i = 0; i < KMAX; ++i)
+        if (i < j) x += start[i] <= x ? len[i] : 0ull;
+      if (cdf_locate(s, col, deg, full, row_bits, x)) {  // the last item's entry is unread
         s.e_hi = col[deg];
         if ((s.e_hi >> row_bits) == 0) break;  // a column without mass
       }
+      uint64_t at = s.e_lo >> row_bits, length = (s.e_hi >> row_bits) - at;
+      removed += length;
+      pick_at(j, s.base + s.lo, s.e_hi);
+      taken = j + 1;
 #pragma unroll
       for (int i = 0; i < KMAX; ++i)
-        if (i == taken) {
-          start[i] = s.a_lo;
-          len[i] = s.a_hi - s.a_lo;
+        if (i <= j) {
+          const bool before = at < start[i];
+          const uint64_t moved_start = start[i], moved_len = len[i];
+          start[i] = before ? at : moved_start;
+          len[i] = before ? length : moved_len;
+          at = before ? moved_start : at;
+          length = before ? moved_len : length;
         }
-      removed += s.a_hi - s.a_lo;
-      pick(s.lo, s.e_hi);
     }
     // fewer than fanout items have positive weight: zero-weight items in order
     if (taken < fanout) {
       uint64_t before = 0;
       for (int64_t off = 0; taken < fanout && off < deg; ++off) {
         const uint64_t entry = col[off + 1], here = entry >> row_bits;
-        if (here == before) pick(off, entry);
+        if (here == before) pick_at(taken++, off, entry);
         before = here;
       }
     }
   }
-  if (!hold) return;
-  if (!row_bits) {
-    int64_t row[KMAX];
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < taken) row[i] = indices ? indices[in_start + held[i]] : in_start + held[i];
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < taken) out_indices[out_start + i] = row[i];
-  } else {
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < taken) out_indices[out_start + i] = (int64_t)held_row[i];
-  }
-  if (out_select) {
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < taken) out_select[out_start + i] = in_start + held[i];
-  }
-  if (out_coo_col) {
-#pragma unroll
-    for (int i = 0; i < KMAX; ++i)
-      if (i < taken) out_coo_col[out_start + i] = col_label;
+  // (the picks are shared among lanes of this wavefront only)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  const int total = __shfl(held_end, kWave - 1, kWave);
+  const int64_t shift = out_start - held_at;
+  for (int q0 = 0; q0 < total; q0 += kWave) {
+    const int q = q0 + lane_id();
+    const bool mine = q < total;
+    const uint2 pick = mine ? wave_pick[q] : make_uint2(0, 0);
+    const int owner = mine ? wave_owner[q] : 0;
+    const int64_t to = __shfl(shift, owner, kWave) + q;
+    const int64_t p = __shfl(in_start, owner, kWave) + pick.x;
+    const int64_t label = __shfl(col_label, owner, kWave);
+    if (!mine) continue;
+    out_indices[to] = row_bits ? (int64_t)pick.y : indices ? indices[p] : p;
+    if (out_select) out_select[to] = p;
+    if (out_coo_col) out_coo_col[to] = label;
   }
 }
 
@@ -741,8 +777,9 @@ static int launch_weighted_cdf(const int64_t* indptr, int64_t num_cols,
                                ColumnLabels labels, const int64_t* col_span,
                                const int64_t* num_dev, hipStream_t s) {
   GS_LAUNCH("sample_weighted_cdf", s,
-            sample_weighted_cdf_kernel<KMAX><<<dim3((unsigned)ceil_div(num_items, kBlock)),
-                                               dim3(kBlock), 0, s>>>(
+            sample_weighted_cdf_kernel<KMAX>
+                <<<dim3((unsigned)ceil_div(num_items, kCdfThreads<KMAX>)),
+                   dim3(kCdfThreads<KMAX>), 0, s>>>(
                 indptr, num_cols, indices, (const uint64_t*)cdf, column_ids, num_items,
                 fanout, replace, key, sub_indptr, out_coo_col, out_indices, out_select, labels,
                 col_span, num_dev));

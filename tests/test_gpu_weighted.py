@@ -162,6 +162,31 @@ def test_cdf_sampling_with_replacement_beyond_the_register_budget():
         capi.sample_weighted(T(indptr), T(indices), None, T(cols), 65, False, cdf=g_cdf)
 
 
+@pytest.mark.parametrize("fanout", [1, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32, 33])
+def test_cdf_columns_of_every_short_length(fanout):
+    """Columns of 0 to 70 entries, each at several distances from a 32-byte boundary:
+    the search's windows at both ends of a column, columns no longer than a window, the
+    picks of a wavefront packed whatever its columns take; weights far from a straight
+    line (so that guesses miss and the search bisects), zero ones, columns of only those."""
+    rng = np.random.default_rng(fanout)
+    deg = np.concatenate([np.arange(71), rng.permutation(71), [4000, 1, 65537]])
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    indices = rng.integers(0, 10**6, size=int(indptr[-1])).astype(np.int64)
+    probs = rng.lognormal(0, 4, size=indices.size).astype(np.float32)
+    probs[rng.random(indices.size) < 0.1] = 0.0
+    for c in (8, 20, 33, 70):
+        probs[indptr[c]:indptr[c + 1]] = 0.0
+    cols = np.concatenate([np.arange(deg.size), rng.integers(0, deg.size, size=333)])
+    for packed in (False, True):
+        cdf = orc.weight_cdf(indptr, probs, indices if packed else None)
+        g_cdf = capi.weight_cdf(T(indptr), F(probs), T(indices) if packed else None)
+        for replace in (False, True):
+            same(capi.sample_weighted(T(indptr), T(indices), None, T(cols), fanout, replace,
+                                      call_id=5, cdf=g_cdf),
+                 orc.sample_weighted(indptr, indices, None, cols, fanout, replace, call_id=5,
+                                     cdf=cdf))
+
+
 @pytest.mark.parametrize("n,k", [(10, 20), (1000, 64), (233000, 512), (5000, 5000)])
 def test_list_sampling_parity(n, k):
     rng = np.random.default_rng(n)
