@@ -128,6 +128,11 @@ SIGNATURES = {
                            _p, _p]),
     "gs_node2vec_hops": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _i64, C.c_double, C.c_double, _u64,
                                 _u64, _p, _p]),
+    "gs_column_marks_bytes": (_sz, [_i64]),
+    "gs_column_marks": (_int, [_p, _i64, _p, _p, _p]),
+    "gs_marks_walks": (_i64, [C.c_double, C.c_double]),
+    "gs_node2vec_marks": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _i64, C.c_double, C.c_double,
+                                 _u64, _u64, _p, _p]),
     "gs_hop_walks": (_i64, [_int, C.c_double, C.c_double]),
     "gs_hop_table": (_int, [_p, _i64, _p, _i64, _p, _p]),
     "gs_segment_sort_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -66,8 +66,8 @@ struct Compressed {
   // Exclusive bound of the ids in `indices` when it is known (a loaded or
   // converted matrix), else -1.
   int64_t num_minor = -1;
-  // Both tables below belong to the ids they were made from: their version, the cache
-  // epoch (invalidate_caches) and their address.  Neither is made or handed out while
+  // The tables below belong to the ids they were made from: their version, the cache
+  // epoch (invalidate_caches) and their address.  None is made or handed out while
   // the current stream is being captured: the graph would record the kernel that fills
   // the table, or read one that a later edit of the matrix frees.
   //
@@ -79,16 +79,20 @@ struct Compressed {
   // Where the column behind every edge lies (gs_hop_table), for walks over a
   // square matrix; made at the second walk over the same matrix.
   torch::Tensor hop_table() const;
+  // Marks of every column (gs_column_marks), for second-order walks over a square matrix
+  // with sorted columns; made once calls that go by them have walked enough steps.
+  torch::Tensor column_marks(int64_t steps) const;
   struct Derived {
     std::mutex guard;  // a matrix is shared by every handle and sampler thread
-    DerivedTable narrow, hops;
+    DerivedTable narrow, hops, marks;
     int64_t versions[2] = {-1, -1}, epoch = -1;
     const void* source = nullptr;
-    int64_t walks = 0, reads = 0;
+    int64_t walks = 0, reads = 0, steps = 0;
     void drop() {
       narrow.drop();
       hops.drop();
-      walks = reads = 0;
+      marks.drop();
+      walks = reads = steps = 0;
     }
   };
   Compressed() = default;

@@ -29,6 +29,31 @@ torch::Tensor Compressed::hop_table() const {
   return d.hops.on_current_stream();
 }
 
+// 32 bytes a column.  Making them reads up to four lines a column, of which they save
+// one or two a step.
+torch::Tensor Compressed::column_marks(int64_t steps) const {
+  constexpr int64_t kMinEdges = int64_t(1) << 20;  // (below, ids stay in cache)
+  constexpr int64_t kStepsPerColumn = 4;
+  const int64_t cols = indptr.numel() - 1;
+  if (indices.numel() < kMinEdges || num_minor < 0 || num_minor >= (int64_t(1) << 31) ||
+      indices.numel() >= (int64_t(1) << 32) || cols >= (int64_t(1) << 31) || !indices.is_cuda() || !indptr.is_cuda())
+    return {};
+  std::lock_guard<std::mutex> lock(derived_.guard);
+  Derived& d = current_derived();
+  if (!narrow_ids_allowed().load()) {
+    d.marks.drop();
+    return {};
+  }
+  if (!d.marks.defined() && (d.steps += steps) < kStepsPerColumn * cols) return {};
+  if (capturing()) return {};
+  if (!d.marks.defined()) {
+    torch::Tensor t = new_ids((int64_t)gs_column_marks_bytes(cols) / 8, indices);
+    GS_CALL(gs_column_marks(cptr(indptr), cols, cptr(indices), t.data_ptr(), cur_stream()));
+    d.marks.set(t);
+  }
+  return d.marks.on_current_stream();
+}
+
 // Traces are stored step-major ([walk_length + 1][num_seeds] in memory) and
 // returned with shape [num_seeds, walk_length + 1] exactly as the reference
 // does (src/cuda/fusion/random_walk.cu:34,67): callers obtain per-step rows
@@ -76,6 +101,14 @@ torch::Tensor Graph::Node2Vec(torch::Tensor seeds, int64_t walk_length, double p
   // some 20 and more where q > 1 has candidates looked up among the neighbours before.
   const int64_t steps = n * walk_length;
   const torch::Tensor narrow = csc_->narrow_indices(q > 1.0 ? 16 * steps : steps);
+  const torch::Tensor marks = n >= gs_marks_walks(p, q) ? csc_->column_marks(steps) : torch::Tensor();
+  if (marks.defined()) {
+    GS_CALL(gs_node2vec_marks(cptr(csc_->indptr), cptr(csc_->indices),
+                              narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+                              marks.data_ptr(), num_cols_, cptr(seeds), n, walk_length, p, q,
+                              rs.seed, next_call_id(), mptr(out), cur_stream()));
+    return out.reshape({n, -1});
+  }
   const torch::Tensor hops = n <= gs_hop_walks(1, p, q) ? csc_->hop_table() : torch::Tensor();
   GS_CALL(gs_node2vec_hops(cptr(csc_->indptr), cptr(csc_->indices),
                            narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(hops),

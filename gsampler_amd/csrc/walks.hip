@@ -210,11 +210,239 @@ __global__ __launch_bounds__(kBlock) void node2vec_kernel(
   }
 }
 
-// Whether candidates are mostly rejected, by the ratio of the levels.
-static bool rare_picks(double p, double q) {
-  const double most = p > q ? p : q, least = p < q ? p : q;
-  return (least < 1.0 ? least : 1.0) * 4.0 < most;
+// What a second-order walk needs to know about a column whose ids are sorted, in 32
+// bytes: where it lies (as pack_span writes it) and the ids at the first 6 of its
+// sevenths.  An id is in the column only between two marks, so
+//   * a candidate that would only be accepted as the return to the previous node is
+//     drawn, compared with the place the marks leave that node and rejected without
+//     being read, six times in seven;
+//   * the search for a candidate among the previous node's neighbours begins with a
+//     seventh of them, usually a line or two.
+constexpr int kMarks = 6;
+struct alignas(32) ColumnMarks {
+  uint64_t span;
+  uint32_t id[kMarks];
+};
+
+// Position of mark m, in [0, kMarks), of a column whose span was packed (deg < 2^24).
+__device__ __forceinline__ uint32_t mark_at(uint32_t deg, int m) {
+  return deg * (uint32_t)(m + 1) / (kMarks + 1);
 }
+
+__global__ __launch_bounds__(kBlock) void column_marks_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_cols, const int64_t* __restrict__ indices,
+    ColumnMarks* __restrict__ marks) {
+  const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (c >= num_cols) return;
+  const int64_t start = indptr[c], deg = indptr[c + 1] - start;
+  ColumnMarks out;
+  out.span = (uint64_t)pack_span(start, deg);
+#pragma unroll
+  for (int m = 0; m < kMarks; ++m)
+    out.id[m] = deg > 0 && out.span != kSpanLookUp ? (uint32_t)indices[start + mark_at((uint32_t)deg, m)] : 0u;
+  marks[c] = out;
+}
+
+// Level of an attempt, an integer in [0, max_scale].
+__device__ __forceinline__ double level_of(const Words4& w, double max_scale) {
+  const double u = (double)((w.z >> 8) + 1u) * 0x1p-24;  // (0, 1]
+  return (double)(int)floor(u * max_scale);
+}
+
+// Positions [*from, *to) of a column in which `target` may lie, by its marks; true if a
+// mark is the target itself.
+__device__ __forceinline__ bool between_marks(const uint32_t (&mark)[kMarks], uint32_t deg,
+                                              uint32_t target, uint32_t* from, uint32_t* to) {
+  int below = 0, upto = 0;
+#pragma unroll
+  for (int m = 0; m < kMarks; ++m) {
+    below += mark[m] < target;
+    upto += mark[m] <= target;
+  }
+  *from = below == 0 ? 0 : mark_at(deg, below - 1) + 1;
+  *to = upto == kMarks ? deg : mark_at(deg, upto);
+  return upto > below;
+}
+
+// The same walk with marks, a lane a walk, for calls that fill the machine.
+// 1 M walks of 80 steps on 124 M edges, p = 2, q = 0.5: the kernel above reads two
+// candidates a step, one of them in vain, 175 M lines in 3.31 ms; this one 130 M in
+// 2.51, both at the part's line rate (52 G/s).  84 M of those are candidates, the rest
+// marks: 2, 4 and 14 of them in place of 6 take 2.62, 2.59 and 2.49 ms (more bytes a
+// column reject more and miss L2 more often).  Non-temporal reads of the candidates
+// leave 4 % more of the marks in L2 and take 2.70 ms.
+// Drawn by each lane for its own walk, attempts of arithmetic only were the bound
+// (2.68 ms; 5.85 at p = 4, q = 0.25, where a candidate in four is accepted: 2.92 now).
+// kSearch: q > 1, where levels in [1, q) need the candidate looked up among the previous
+// node's neighbours and every attempt reads its candidate.
+template <typename IdT, bool kSearch>
+__global__ __launch_bounds__(kBlock) void node2vec_marks_kernel(
+    const int64_t* __restrict__ indptr, const IdT* __restrict__ indices,
+    const ColumnMarks* __restrict__ marks, int64_t num_cols, const int64_t* __restrict__ seeds,
+    int64_t num_seeds, int64_t walk_length, double p, double q, PhiloxKey key,
+    int64_t* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = lane_id();
+  const bool live = i < num_seeds;  // (the other lanes draw for their wavefront's walks)
+  const double max_scale = p > q ? p : q;
+  const double reject_from = max_scale > 1.0 ? max_scale : 1.0;
+  double accept_below = p < q ? p : q;
+  if (accept_below > 1.0) accept_below = 1.0;
+  int64_t curr = live ? seeds[i] : -1, last = -1;
+  int64_t last_start = 0;
+  uint32_t last_deg = 0;
+  uint32_t last_mark[kMarks];
+#pragma unroll
+  for (int m = 0; m < kMarks; ++m) last_mark[m] = 0;
+  bool last_marked = false;
+  if (live) out[i] = curr;
+  for (int64_t step = 1; step <= walk_length; ++step) {
+    int64_t start = 0;
+    uint32_t deg = 0, mark[kMarks];
+#pragma unroll
+    for (int m = 0; m < kMarks; ++m) mark[m] = 0;
+    uint64_t span = 0;
+    if (curr >= 0 && curr < num_cols) {
+      const ColumnMarks c = marks[curr];
+      span = c.span;
+#pragma unroll
+      for (int m = 0; m < kMarks; ++m) mark[m] = c.id[m];
+    }
+    // (the first words of a step depend on no load and are drawn while the marks travel)
+    Words4 w = philox(key, (uint64_t)i, (uint64_t)step << 32);
+    const bool marked = span != kSpanLookUp;
+    if (marked) {
+      start = (int64_t)(span & ((1ull << kSpanStartBits) - 1ull));
+      deg = (uint32_t)(span >> kSpanStartBits);
+    } else {
+      deg = (uint32_t)column_degree(indptr, num_cols, curr, &start);
+    }
+    int64_t pick = -1;
+    // where the previous node may lie in this column (there is none before the first step)
+    uint32_t from = 0, to = last >= 0 ? deg : 0;
+    if (marked && last >= 0 && deg > 0) between_marks(mark, deg, (uint32_t)last, &from, &to);
+    if (kSearch) {
+      if (deg == 1) {
+        pick = (int64_t)indices[start];
+      } else if (deg > 0) {
+        for (uint32_t attempt = 0;; ++attempt) {
+          double y;
+          uint32_t at;
+          bool sure, search;
+          for (;; ++attempt) {
+            if (attempt > 0) w = philox(key, (uint64_t)i, ((uint64_t)step << 32) | attempt);
+            y = level_of(w, max_scale);
+            at = (uint32_t)__umul64hi(((uint64_t)w.y << 32) | w.x, (uint64_t)deg);
+            sure = attempt + 1 >= kMaxAttempts || y < accept_below;
+            search = (y < q) != (y < 1.0) && last_deg > 0;
+            if (sure || (y < reject_from && (search || (y < p && at >= from && at < to)))) break;
+          }
+          const int64_t cand = (int64_t)indices[start + at];
+          pick = cand;
+          if (sure) break;
+          double h = 1.0;
+          if (cand == last) {
+            h = p;
+          } else if (search) {
+            uint32_t lo = 0, hi = last_deg;
+            bool found = false;
+            if (last_marked) found = between_marks(last_mark, last_deg, (uint32_t)cand, &lo, &hi);
+            if (found || sorted_contains<false>(indices + last_start + lo, (int64_t)hi - lo, cand))
+              h = q;
+          }
+          if (y < h) break;
+        }
+      }
+    } else {
+      // An attempt is sure, or accepted if its candidate is the previous node, or
+      // rejected, whatever else its candidate is.  Attempts are drawn for as many walks
+      // as are undecided by all lanes of the wavefront; of each walk the first one that
+      // is not rejected counts.
+      constexpr uint32_t kNone = ~0u;
+      uint32_t chosen = kNone, check0 = kNone, check1 = kNone, next = 1;
+      bool back = false;
+      // what an attempt at position `at` is
+      auto sure_at = [&](uint32_t attempt, double y) {
+        return attempt + 1 >= kMaxAttempts || y < accept_below;
+      };
+      auto note = [&](bool sure, uint32_t at) {  // true: the walk is decided
+        if (sure) chosen = at;
+        else if (check0 == kNone) check0 = at;
+        else if (check1 == kNone) check1 = at;
+        else back = (int64_t)indices[start + at] == last;
+        return sure || back;
+      };
+      bool pending = deg > 1;
+      if (deg == 1) chosen = 0;
+      if (pending) {
+        const double y = level_of(w, max_scale);
+        const uint32_t at = (uint32_t)__umul64hi(((uint64_t)w.y << 32) | w.x, (uint64_t)deg);
+        const bool sure = sure_at(0, y);
+        if (sure || (y < reject_from && y < p && at >= from && at < to)) pending = !note(sure, at);
+      }
+      for (;;) {
+        const uint64_t open = __ballot(pending);
+        if (open == 0) break;
+        const int walks = __popcll(open);
+        const int shift = walks == 1 ? 6 : __clz(walks - 1) - 26;  // lanes a walk: 2^shift
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi(
+            (uint32_t)(open >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)open, 0));
+        // lane k learns which walk is the k-th undecided one, and then its own group's
+        const int order = __builtin_amdgcn_ds_permute((pending ? rank : kWave - 1) << 2,
+                                                      pending ? lane : -1);
+        const int mine = lane >> shift;
+        const int owner = __shfl(order, mine, kWave) & (kWave - 1);
+        const uint32_t attempt = (uint32_t)__shfl((int)next, owner, kWave) +
+                                 (uint32_t)(lane & ((1 << shift) - 1));
+        const uint32_t o_deg = (uint32_t)__shfl((int)deg, owner, kWave);
+        const uint32_t o_from = (uint32_t)__shfl((int)from, owner, kWave);
+        const uint32_t o_to = (uint32_t)__shfl((int)to, owner, kWave);
+        w = philox(key, (uint64_t)(i - lane + owner), ((uint64_t)step << 32) | attempt);
+        const double y = level_of(w, max_scale);
+        const uint32_t at = (uint32_t)__umul64hi(((uint64_t)w.y << 32) | w.x, (uint64_t)o_deg);
+        const bool sure = sure_at(attempt, y);
+        const bool counts =
+            mine < walks &&
+            (sure || (y < reject_from && y < p && at >= o_from && at < o_to));
+        const int group0 = (rank << shift) & (kWave - 1);
+        const uint64_t group = shift == 6 ? ~0ull : (1ull << (1 << shift)) - 1ull;
+        const uint64_t hits = (__ballot(counts) >> group0) & group;
+        const uint64_t sures = __ballot(sure) >> group0;
+        const int first = hits ? __ffsll((unsigned long long)hits) - 1 : 0;
+        const uint32_t found = (uint32_t)__shfl((int)at, group0 + first, kWave);
+        if (pending) {
+          if (hits) {
+            pending = !note((sures >> first) & 1ull, found);
+            next += (uint32_t)first + 1;
+          } else {
+            next += 1u << shift;
+          }
+        }
+      }
+      if (deg > 0) {
+        int64_t c0 = -1, c1 = -1;
+        if (chosen != kNone) pick = (int64_t)indices[start + chosen];
+        if (check0 != kNone) c0 = (int64_t)indices[start + check0];
+        if (check1 != kNone) c1 = (int64_t)indices[start + check1];
+        if (back || (c0 == last && check0 != kNone) || (c1 == last && check1 != kNone)) pick = last;
+      }
+    }
+    last = curr;
+    if (kSearch) {
+      last_start = start;
+      last_deg = deg;
+      last_marked = marked;
+#pragma unroll
+      for (int m = 0; m < kMarks; ++m) last_mark[m] = mark[m];
+    }
+    curr = pick;
+    if (live) out[step * num_seeds + i] = pick;
+  }
+}
+
+// Whether candidates are mostly rejected: only those of level 0, one in max(p, q), are
+// accepted whatever they are.
+static bool rare_picks(double p, double q) { return p > 3.0 || q > 3.0; }
 
 // Whether the first candidate stands, all but once in 2^24 (the only level is 0).
 static bool sure_picks(double p, double q) { return p <= 1.0 && q <= 1.0; }
@@ -238,6 +466,49 @@ static int64_t hop_walks(bool second_order, double p, double q) {
   if (sure_picks(p, q)) return 0;
   if (q <= 1.0) return int64_t(1) << 11;
   return rare_picks(p, q) ? int64_t(1) << 13 : int64_t(1) << 15;
+}
+
+// Up to how many lanes a call spreads its walks over, a group of lanes a walk (the best
+// of 1, 2, 4, 8, 16 lanes at 1.5 K to 300 K walks of 20 steps): about 200 K where every
+// second candidate is accepted, 400 K where fewer are or candidates are searched for
+// (120 K walks on 9 M edges, one lane and two: p = 1, q = 4 872 and 520 us, p = 0.5,
+// q = 2 481 and 309, p = 2, q = 0.5 107 and 98).
+static int64_t walk_lanes(double p, double q) {
+  return q > 1.0 || rare_picks(p, q) ? 400000 : 200000;
+}
+
+// From how many walks on a call goes by marks: those that go by one lane a walk and are
+// bound by lines.  Without / with marks, us:
+//   124 M edges    1 M walks, 80 steps    p = 2, q = 0.5  3308 / 2513    p = 4, q = 0.25  5494 / 2919
+//                                         p = 0.25, q = 4  14 886 / 14 294
+//   9 M edges      300 K walks, 40 steps  388 / 320, 678 / 468, 2078 / 1808
+//                  60 K walks by groups   115 / 154, 168 / 264, 548 / 1296
+static int64_t marks_walks(double p, double q) {
+  return sure_picks(p, q) ? INT64_MAX : walk_lanes(p, q) / 2 + 1;
+}
+
+template <typename IdT>
+static int node2vec_marks(const int64_t* indptr, const IdT* indices, const ColumnMarks* marks,
+                          int64_t num_cols, const int64_t* seeds, int64_t num_seeds,
+                          int64_t walk_length, double p, double q, uint64_t seed,
+                          uint64_t call_id, int64_t* out_traces, gs_stream_t stream) {
+  GS_REQUIRE(num_seeds >= 0 && walk_length >= 0 && num_cols >= 0,
+             "node2vec: negative size");
+  GS_REQUIRE(p > 0.0 && q > 0.0, "node2vec: p and q must be positive");
+  if (num_seeds == 0) return GS_OK;
+  GS_REQUIRE(indptr && seeds && out_traces, "node2vec: null pointer");
+  hipStream_t s = as_stream(stream);
+  const int threads = num_seeds < kFewWalks ? kWave : kBlock;
+#define GS_NODE2VEC_MARKS(SEARCH)                                                                \
+  GS_LAUNCH("node2vec", s,                                                                      \
+            (node2vec_marks_kernel<IdT, SEARCH>)<<<dim3((unsigned)ceil_div(num_seeds, threads)), \
+                                                   dim3(threads), 0, s>>>(                      \
+                indptr, indices, marks, num_cols, seeds, num_seeds, walk_length, p, q,          \
+                make_key(seed, call_id), out_traces))
+  if (q > 1.0) GS_NODE2VEC_MARKS(true);
+  else GS_NODE2VEC_MARKS(false);
+#undef GS_NODE2VEC_MARKS
+  return GS_OK;
 }
 
 template <typename IdT>
@@ -274,11 +545,10 @@ static int node2vec(const int64_t* indptr, const IdT* indices, const Hop* hops, 
   if (num_seeds == 0) return GS_OK;
   GS_REQUIRE(indptr && seeds && out_traces, "node2vec: null pointer");
   hipStream_t s = as_stream(stream);
-  // As many lanes a walk as keep the call's lanes below what fills the machine:
-  // 200 K where most candidates are accepted, 400 K where an accepted one is rare
-  // (the best of 1, 2, 4, 8, 16 lanes at 1 K to 1 M walks); one lane where the first
-  // candidate stands (32 K walks of 20 steps on 9 M edges: 22 us, with four lanes 35).
-  const int64_t lanes = rare_picks(p, q) ? 400000 : 200000;
+  // As many lanes a walk as keep the call's lanes below what fills the machine; one
+  // where the first candidate stands (32 K walks of 20 steps on 9 M edges: 22 us, with
+  // four lanes 35).
+  const int64_t lanes = walk_lanes(p, q);
   int group = 16;
   while (group > 1 && num_seeds * group > lanes) group >>= 1;
   if (sure_picks(p, q)) group = 1;
@@ -323,6 +593,40 @@ int gs_hop_table(const int64_t* indptr, int64_t num_cols, const int64_t* indices
             hop_table_kernel<<<dim3((unsigned)ceil_div(nnz, kBlock)), dim3(kBlock), 0, s>>>(
                 indptr, num_cols, indices, nnz, (Hop*)hops));
   return GS_OK;
+}
+
+size_t gs_column_marks_bytes(int64_t num_cols) {
+  return num_cols > 0 ? sizeof(gs::ColumnMarks) * (size_t)num_cols : 0;
+}
+
+int gs_column_marks(const int64_t* indptr, int64_t num_cols, const int64_t* indices, void* marks,
+                    gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(num_cols >= 0 && num_cols <= (int64_t(1) << 31), "column_marks: bad size");
+  if (num_cols == 0) return GS_OK;
+  GS_REQUIRE(indptr && indices && marks, "column_marks: null pointer");
+  GS_REQUIRE(((uintptr_t)marks & (alignof(ColumnMarks) - 1)) == 0, "column_marks: misaligned");
+  hipStream_t s = as_stream(stream);
+  GS_LAUNCH("column_marks", s,
+            column_marks_kernel<<<dim3((unsigned)ceil_div(num_cols, kBlock)), dim3(kBlock), 0, s>>>(
+                indptr, num_cols, indices, (ColumnMarks*)marks));
+  return GS_OK;
+}
+
+int64_t gs_marks_walks(double p, double q) { return gs::marks_walks(p, q); }
+
+int gs_node2vec_marks(const int64_t* indptr, const int64_t* indices, const int32_t* indices32,
+                      const void* marks, int64_t num_cols, const int64_t* seeds,
+                      int64_t num_seeds, int64_t walk_length, double p, double q, uint64_t seed,
+                      uint64_t call_id, int64_t* out_traces, gs_stream_t stream) {
+  GS_REQUIRE(marks != nullptr && ((uintptr_t)marks & (alignof(gs::ColumnMarks) - 1)) == 0,
+             "node2vec: null or misaligned marks");
+  const gs::ColumnMarks* m = (const gs::ColumnMarks*)marks;
+  if (indices32)
+    return gs::node2vec_marks(indptr, indices32, m, num_cols, seeds, num_seeds, walk_length, p, q,
+                              seed, call_id, out_traces, stream);
+  return gs::node2vec_marks(indptr, indices, m, num_cols, seeds, num_seeds, walk_length, p, q,
+                            seed, call_id, out_traces, stream);
 }
 
 int64_t gs_hop_walks(int second_order, double p, double q) {

@@ -683,6 +683,10 @@ int gs_sorted_to_indptr(const int64_t* sorted_ids, int64_t nnz, int64_t num_cols
  *    from that edge.  The _hops forms take it (nullable; used for calls of up to
  *    gs_hop_walks walks), gs_node2vec_hops also an int32 copy of the row ids
  *    (nullable); the traces are the same.
+ *  gs_column_marks: for every column (at most 2^31 of them, fewer than 2^32 edges,
+ *    ids below 2^32 and sorted inside the column) where it lies and six of its ids, 32 bytes at an address
+ *    divisible by 32 (gs_column_marks_bytes in all), for gs_node2vec_marks: the same
+ *    traces from fewer reads, ahead of the other forms from gs_marks_walks walks on.
  *  gs_node2vec: second-order walk by rejection sampling with integer levels
  *    (return weight p, neighbour-of-previous weight q, otherwise 1); needs row
  *    ids sorted inside every column.  FusedNode2VecCUDA,
@@ -710,6 +714,14 @@ int gs_node2vec_hops(const int64_t* indptr, const int64_t* indices, const int32_
                      int64_t walk_length, double p, double q, uint64_t seed, uint64_t call_id,
                      int64_t* out_traces, gs_stream_t stream);
 int64_t gs_hop_walks(int second_order, double p, double q);
+size_t gs_column_marks_bytes(int64_t num_cols);
+int gs_column_marks(const int64_t* indptr, int64_t num_cols, const int64_t* indices, void* marks,
+                    gs_stream_t stream);
+int64_t gs_marks_walks(double p, double q);
+int gs_node2vec_marks(const int64_t* indptr, const int64_t* indices, const int32_t* indices32,
+                      const void* marks, int64_t num_cols, const int64_t* seeds,
+                      int64_t num_seeds, int64_t walk_length, double p, double q, uint64_t seed,
+                      uint64_t call_id, int64_t* out_traces, gs_stream_t stream);
 int gs_hop_table(const int64_t* indptr, int64_t num_cols, const int64_t* indices, int64_t nnz,
                  void* hops, gs_stream_t stream);
 int gs_node2vec(const int64_t* indptr, const int64_t* indices, int64_t num_cols,

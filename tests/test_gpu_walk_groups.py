@@ -131,3 +131,47 @@ def test_int32_copy_is_made_once_enough_ids_were_read(wide_world):
         grown.append(torch.cuda.memory_allocated() - before)
     made = [i for i, g in enumerate(grown) if g > 0]
     assert made == [-(-indices.size // 200_000) - 1] and grown[made[0]] >= 4 * indices.size
+
+
+# Calls of one lane a walk go by marks of the columns once they have walked enough steps: returns
+# to the previous node (every node's neighbours are near it), ids that repeat in a column, columns
+# of 0 to 8 edges, a hub, and a column too long for its marks; one walk more than the border.
+@pytest.fixture(scope="module")
+def near_world():
+    rng = np.random.default_rng(9)
+    nodes, hub = 200_000, (1 << 24) + 5
+    deg = rng.integers(0, 9, size=nodes)
+    deg[1000], deg[2000] = 60_000, hub
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    col = np.repeat(np.arange(nodes), deg)
+    indices = (col + rng.integers(-3, 4, size=col.size)) % nodes
+    wide = (col == 1000) | (col == 2000)
+    indices[wide] = rng.integers(0, nodes, size=int(wide.sum()))
+    indices[rng.random(indices.size) < 0.002] = 2000
+    indices[rng.random(indices.size) < 0.002] = 1000
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    return rng, nodes, indptr, m.csc[1].cpu().numpy(), m
+
+
+@pytest.mark.parametrize("n,length,p,q", [
+    (100001, 9, 2.0, 0.5), (200001, 5, 4.0, 0.25), (200001, 4, 8.0, 1.0), (200001, 4, 0.5, 2.0),
+    (200001, 4, 0.25, 4.0), (200001, 4, 4.0, 2.0), (100001, 9, 1.5, 0.5), (200002, 3, 1e9, 1e-9),
+])
+def test_node2vec_by_marks(near_world, n, length, p, q):
+    test_node2vec(near_world, n, length, p, q)
+
+
+def test_marks_are_made_once_enough_steps_were_walked(near_world):
+    _, nodes, indptr, indices, _ = near_world
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    m._graph._CAPI_SortCSCIndices()
+    seeds = torch.arange(100_001, device=DEV) % nodes
+    grown = []
+    for n in (100_000, 100_001, 100_001, 100_001, 100_001):
+        before = torch.cuda.memory_allocated()
+        m.node2vec(seeds[:n], 3, 2.0, 0.5)
+        grown.append(torch.cuda.memory_allocated() - before)
+    assert grown[:3] == [0, 0, 0] and grown[3] >= 32 * nodes and grown[4] == 0
