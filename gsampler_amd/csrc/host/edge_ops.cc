@@ -3,6 +3,10 @@
 // names, broadcast shapes and the sparse format, then calls the C ABI.
 #include <algorithm>
 
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+
 #include "abi_call.h"
 #include "graph.h"
 
@@ -173,6 +177,72 @@ void Graph::SDDMM(const std::string& op, torch::Tensor lhs, torch::Tensor rhs,
                    out.data_ptr(), (int)lhs_target, (int)rhs_target, bc.lhs_len,
                    bc.rhs_len, bc.out_len, bc.reduce_size, cptr(bc.lhs_off),
                    cptr(bc.rhs_off), cur_stream()));
+}
+
+// A float32 tensor on the current device that nothing but its values matters of.
+static bool plain_values(const torch::Tensor& t, bool gradients_matter) {
+  return t.defined() && t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
+         t.layout() == torch::kStrided && t.get_device() == c10::hip::current_device() &&
+         !t.is_neg() && !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined() &&
+         !(gradients_matter && t.requires_grad() && at::GradMode::is_enabled());
+}
+
+c10::optional<torch::Tensor> Graph::EdgeScore(const std::vector<int64_t>& kinds,
+                                              std::vector<torch::Tensor> lhs,
+                                              std::vector<torch::Tensor> rhs,
+                                              const std::vector<int64_t>& targets,
+                                              c10::optional<torch::Tensor> weights,
+                                              bool positive_part, double shift,
+                                              int64_t on_format) {
+  const size_t n = kinds.size();
+  TORCH_CHECK(n >= 1 && lhs.size() == n && rhs.size() == n && targets.size() == 2 * n,
+              "EdgeScore: one operand pair and two targets a term");
+  if (n > GS_SCORE_MAX_TERMS || (!weights.has_value() && n > 1) || num_edges_ <= 0) return {};
+  if (on_format != kCOO && on_format != kCSC && on_format != kCSR) return {};
+  if (at::impl::torch_function_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return {};
+  const int64_t per_target[3] = {num_rows_, num_edges_, num_cols_};
+  gs_score_term terms[GS_SCORE_MAX_TERMS];
+  int64_t len = 0;
+  for (size_t k = 0; k < n; ++k) {
+    int64_t lt = targets[2 * k], rt = targets[2 * k + 1];
+    if (kinds[k] == GS_SCORE_VALUE) {
+      if (!plain_values(lhs[k], true) || lhs[k].dim() != 1 || lhs[k].size(0) != num_edges_) return {};
+    } else {
+      // (what SDDMM writes into an array of its own carries no gradients)
+      if (!plain_values(lhs[k], false) || !plain_values(rhs[k], false)) return {};
+      const int64_t dims = kinds[k] == GS_SCORE_PRODUCTS ? 2 : 1;
+      if (lhs[k].dim() != dims || rhs[k].dim() != dims || lt < 0 || lt > 2 || rt < 0 || rt > 2 ||
+          lhs[k].size(0) < per_target[lt] || rhs[k].size(0) < per_target[rt])
+        return {};
+      if (dims == 2) {
+        if (lhs[k].size(1) != rhs[k].size(1) || lhs[k].size(1) < 1 ||
+            lhs[k].size(1) > GS_SCORE_MAX_LEN || (len != 0 && lhs[k].size(1) != len))
+          return {};
+        len = lhs[k].size(1);
+      }
+      rhs[k] = rhs[k].contiguous();
+      if (on_format == kCSR) lt = lt == 1 ? 1 : 2 - lt, rt = rt == 1 ? 1 : 2 - rt;
+    }
+    lhs[k] = lhs[k].contiguous();
+    terms[k] = gs_score_term{(const float*)fptr(lhs[k]),
+                             kinds[k] == GS_SCORE_VALUE ? nullptr : (const float*)fptr(rhs[k]),
+                             (int)kinds[k], (int)lt, (int)rt};
+  }
+  if (weights.has_value()) {
+    if (!plain_values(*weights, true) || weights->dim() != 1 || weights->size(0) != (int64_t)n)
+      return {};
+    weights = weights->contiguous();
+  }
+  CreateSparseFormat(on_format);
+  const StructureArgs s = on_format == kCOO ? structure_of(*coo_)
+                                            : structure_of(compressed(on_format));
+  torch::Tensor out = torch::empty({num_edges_}, lhs[0].options().requires_grad(false));
+  GS_CALL(gs_edge_score(s.format, s.a, s.b, s.num_major, s.nnz, s.edge_map, terms, (int)n, len,
+                        weights.has_value() ? (const float*)fptr(*weights) : nullptr,
+                        positive_part ? 1 : 0, (float)shift, (float*)out.data_ptr(),
+                        cur_stream()));
+  return out;
 }
 
 void Graph::FusedUOPV(const std::string& op, torch::Tensor lhs1,

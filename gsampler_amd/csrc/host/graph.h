@@ -263,6 +263,15 @@ class Graph : public torch::CustomClassHolder {
             torch::Tensor ufeat, torch::Tensor efeat, torch::Tensor out,
             torch::Tensor argu, torch::Tensor arge, int64_t u_target,
             int64_t on_format);
+  // gs_edge_score over the terms (kinds[k], lhs[k], rhs[k], targets[2 k .. 2 k + 1]);
+  // nothing where the call is not one for it: other types, shapes or devices, values
+  // that carry gradients, a transform or a mode that has to see torch's operators.
+  c10::optional<torch::Tensor> EdgeScore(const std::vector<int64_t>& kinds,
+                                         std::vector<torch::Tensor> lhs,
+                                         std::vector<torch::Tensor> rhs,
+                                         const std::vector<int64_t>& targets,
+                                         c10::optional<torch::Tensor> weights,
+                                         bool positive_part, double shift, int64_t on_format);
   void FusedUOPV(const std::string& op, torch::Tensor lhs1, torch::Tensor rhs1,
                  torch::Tensor out1, torch::Tensor lhs2, torch::Tensor rhs2,
                  torch::Tensor out2, int64_t on_format);

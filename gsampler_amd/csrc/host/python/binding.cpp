@@ -9,6 +9,8 @@
 //       -> (frontier, row, col, None) per layer, one flat tuple
 //   batch_sample_layers(graph, seeds, seeds_ptr, fanouts, replace, weights)
 //       -> one BlockBatch per layer
+//   edge_score(graph, kinds, lhs, rhs, targets, weights, positive_part, shift, on_format)
+//       -> a value per edge, or None where the call is not one for the kernel
 //   BlockBatch   the operator library's class of that name with its methods, plus
 //       make_blocks(): the list of Block objects
 //   wrap(batch)  the same around a batch that came through torch
@@ -192,6 +194,39 @@ py::tuple sample_layers(py::handle graph, torch::Tensor seeds, std::vector<int64
   return out;
 }
 
+// -> the scores, or None where torch's own operators have to do it.
+py::object edge_score(py::handle graph, std::vector<int64_t> kinds, py::list lhs, py::list rhs,
+                      std::vector<int64_t> targets, py::object weights, bool positive_part,
+                      double shift, int64_t on_format) {
+  auto g = unwrap<gs::Graph>(graph);
+  std::vector<torch::Tensor> l, r;
+  for (const py::handle& t : lhs) {
+    if (!THPVariable_CheckExact(t.ptr())) return py::none();
+    l.push_back(THPVariable_Unpack(t.ptr()));
+  }
+  for (const py::handle& t : rhs) {
+    if (t.is_none()) {
+      r.emplace_back();
+      continue;
+    }
+    if (!THPVariable_CheckExact(t.ptr())) return py::none();
+    r.push_back(THPVariable_Unpack(t.ptr()));
+  }
+  c10::optional<torch::Tensor> w;
+  if (!weights.is_none()) {
+    if (!THPVariable_CheckExact(weights.ptr())) return py::none();
+    w = THPVariable_Unpack(weights.ptr());
+  }
+  c10::optional<torch::Tensor> out;
+  {
+    py::gil_scoped_release nogil;
+    out = g->EdgeScore(kinds, std::move(l), std::move(r), targets, std::move(w), positive_part,
+                       shift, on_format);
+  }
+  if (!out.has_value()) return py::none();
+  return py::reinterpret_steal<py::object>(wrap_tensor(std::move(*out)));
+}
+
 std::vector<std::shared_ptr<Batch>> batch_sample_layers(py::handle graph, torch::Tensor seeds,
                                                         torch::Tensor ptr,
                                                         std::vector<int64_t> fanouts, bool replace,
@@ -233,6 +268,7 @@ PYBIND11_MODULE(_gs_python, m) {
   m.def("set_block_class", &set_block_class);
   m.def("sample_layers", &sample_layers);
   m.def("batch_sample_layers", &batch_sample_layers);
+  m.def("edge_score", &edge_score);
   m.def("wrap", [](py::handle batch) { return std::make_shared<Batch>(unwrap<gs::BlockBatch>(batch)); });
   py::class_<Batch, std::shared_ptr<Batch>>(m, "BlockBatch")
       .def("make_blocks", &Batch::make_blocks)

@@ -151,7 +151,7 @@ class compile:  # noqa: N801 -- the reference's public name
     # -------------------------------------------------------------------- run
     def _executable(self, gm):
         """What a call runs: a copy of the operator graph whose sampling layers are
-        chained into one operator and whose generated code takes flat inputs and
+        chained into one operator, whose edge scores are one kernel each and whose generated code takes flat inputs and
         builds the result in place (the pytree machinery of a traced module costs
         more than the operators of a small sampler).  None when the graph's inputs
         or result have no such form: the module itself is called then."""
@@ -170,6 +170,8 @@ class compile:  # noqa: N801 -- the reference's public name
         except (TypeError, ValueError):
             return None
         passes.chain_layers(gm, graph)
+        passes.compute_edge_scores(graph)
+        passes.share_leading_rows(graph)
         return fx.GraphModule(gm, graph).forward
 
     def __call__(self, *args):

@@ -30,6 +30,12 @@ hoisting of tensor constants.  Operator rewrites (observable in
                                                      _CAPI_BatchSampleLayers
   select_formats                deterministic on_format / output_format choice
 
+and, in the copy of the graph that calls run (like chain_layers):
+
+  compute_edge_scores           products of features summed over the feature, stacked
+                                and multiplied by a vector  -> one kernel
+  share_leading_rows            features of all rows of a column slice: the parent's, once
+
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
 whoever runs the passes (gm.recompile()): generating it after each of them was
 three quarters of a compilation.
@@ -37,6 +43,7 @@ three quarters of a compilation.
 import operator
 from typing import Dict, Iterable, List, Optional
 
+import torch
 import torch.fx as fx
 
 from .. import _library
@@ -57,10 +64,11 @@ def _finish(gm: fx.GraphModule) -> fx.GraphModule:
     return gm
 
 
-def _drop_dead_nodes(graph: fx.Graph) -> None:
+def _drop_dead_nodes(graph: fx.Graph, replaced=()) -> None:
+    """`replaced`: operators that write in place and have been replaced."""
     live = set()
     for node in reversed(graph.nodes):
-        if node.op in ("output", "placeholder") or node.target in IN_PLACE_OPS:
+        if node.op in ("output", "placeholder") or node.target in IN_PLACE_OPS and node not in replaced:
             live.add(node)
         if node in live:
             live.update(_input_nodes(node))
@@ -669,6 +677,188 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
                             u.replace_all_uses_with(item)
     if chains:
         _drop_dead_nodes(copy)
+
+
+IN_PLACE_FUNCTIONS = {getattr(operator, name) for name in (
+    "iadd", "iand", "iconcat", "ifloordiv", "ilshift", "imatmul", "imod", "imul", "ior", "ipow",
+    "irshift", "isub", "itruediv", "ixor", "setitem", "delitem")}
+
+
+def _writes_in_place(node: fx.Node) -> bool:
+    """Whether a node of the sampler's own may change a tensor that others read."""
+    if node.op not in ("call_method", "call_function"):
+        return node.op == "call_module"
+    name = node.target if node.op == "call_method" else getattr(node.target, "__name__", "")
+    return (name.endswith("_") and not name.endswith("__") or node.target in IN_PLACE_FUNCTIONS
+            or "out" in node.kwargs or node.kwargs.get("inplace") is True)
+
+
+def _call(node, *targets) -> bool:
+    return isinstance(node, fx.Node) and node.op == "call_function" and node.target in targets
+
+
+def _only_user(node: fx.Node, user: fx.Node) -> bool:
+    return set(node.users) == {user}
+
+
+def _dim_one(node: fx.Node, position: int) -> bool:
+    """Whether a call's one option is dim = 1."""
+    given = list(node.args[position:]) + list(node.kwargs.values())
+    return given == [1] and set(node.kwargs) <= {"dim"} and type(given[0]) is int
+
+
+def _sddmm_of(out):
+    """(graph, op, lhs data, rhs data, targets, format, node) of the SDDMM that wrote `out`,
+    an _after_sddmm node, into an array that nothing else sees; else None."""
+    if not _is_wrapped(out, "_after_sddmm") or len(out.args) != 2:
+        return None
+    item = out.args[0]
+    if not (_call(item, operator.getitem) and item.args[1] == 2
+            and _is_wrapped(item.args[0], "_before_sddmm")):
+        return None
+    before = item.args[0]
+    writers = [n for n in item.users if _is_method(n, "_CAPI_SDDMM")]
+    if len(writers) != 1 or set(item.users) != {writers[0], out}:
+        return None
+    w = writers[0]
+    for i, arg in ((0, w.args[2]), (1, w.args[3])):
+        if not (_call(arg, operator.getitem) and arg.args == (before, i)):
+            return None
+    if w.args[1] != before.args[1] or w.args[4] is not item:
+        return None
+    return w.args[0], w.args[1], before.args[2], before.args[3], [w.args[5], w.args[6]], w.args[7], w
+
+
+def compute_edge_scores(copy: fx.Graph) -> None:
+    """In a copy of a graph: (u * v).sum(1) of an SDDMM's products, alone or as a term of
+    stack([...], dim=1) @ weights, whose other terms are quotients e / u and values an edge
+    has; then relu and the addition of a constant times ones_like, where they follow
+    => one _edge_score, which falls back to those operators where it has to (values that
+    carry gradients, other types and shapes)."""
+    from ..ops.fused_op import PRODUCTS, QUOTIENT, VALUE, _edge_score
+    if any(_writes_in_place(n) for n in copy.nodes):
+        return
+
+    def products_of(node):
+        """The SDDMM behind a sum over the feature of its products, or None."""
+        if not ((_call(node, torch.sum) or (isinstance(node, fx.Node) and _is_method(node, "sum")))
+                and len(node.args) >= 1 and _dim_one(node, 1)):
+            return None
+        found = _sddmm_of(node.args[0])
+        if found is None or found[1] != "mul" or not _only_user(node.args[0], node):
+            return None
+        return found
+
+    written = []
+
+    def replace(node, terms, weights, positive_part, shift):
+        """terms: (kind, the SDDMM as _sddmm_of gives it, or the value)"""
+        kinds, lhs, rhs, targets = [], [], [], []
+        for kind, of in terms:
+            kinds.append(kind)
+            lhs.append(of if kind == VALUE else of[2])
+            rhs.append(None if kind == VALUE else of[3])
+            targets += [1, 1] if kind == VALUE else of[4]
+            if kind != VALUE:
+                written.append(of[6])
+                g, on_format = of[0], of[5]
+        with copy.inserting_before(node):
+            new = copy.call_function(_edge_score, args=(g, kinds, lhs, rhs, targets, weights,
+                                                        positive_part, shift, on_format))
+        node.replace_all_uses_with(new)
+
+    for product in list(copy.nodes):
+        if not (_call(product, torch.matmul, operator.matmul) and len(product.args) == 2
+                and not product.kwargs):
+            continue
+        stack, weights = product.args
+        if not (_call(stack, torch.stack) and len(stack.args) >= 1 and _dim_one(stack, 1)
+                and isinstance(stack.args[0], (list, tuple)) and _only_user(stack, product)
+                and all(isinstance(v, fx.Node) for v in (weights, *stack.args[0]))):
+            continue
+        terms = []
+        for value in stack.args[0]:
+            found = products_of(value) if _only_user(value, stack) else None
+            if found is not None:
+                terms.append((PRODUCTS, found))
+                continue
+            found = _sddmm_of(value) if _only_user(value, stack) else None
+            quotient = found is not None and found[1] == "div"
+            terms.append((QUOTIENT, found) if quotient else (VALUE, value))
+        if (not any(kind == PRODUCTS for kind, _ in terms)
+                or len({(of[0], of[5]) for kind, of in terms if kind != VALUE}) != 1):
+            continue
+        last, positive_part, shift = product, False, None
+        after = list(last.users)
+        if (len(after) == 1 and len(after[0].args) == 1 and after[0].args[0] is last
+                and (_call(after[0], torch.relu) and not after[0].kwargs
+                     or _call(after[0], torch.nn.functional.relu)
+                     and after[0].kwargs.get("inplace", False) is False)):
+            last, positive_part = after[0], True
+        ones = [n for n in last.users if _call(n, torch.ones_like) and n.args == (last,) and not n.kwargs]
+        if len(ones) == 1 and len(last.users) == 2:
+            add = next(n for n in last.users if n is not ones[0])
+            scaled = list(ones[0].users)
+            if (_call(add, operator.add, torch.add) and not add.kwargs and len(add.args) == 2
+                    and len(scaled) == 1 and _call(scaled[0], operator.mul, torch.mul)
+                    and len(scaled[0].args) == 2 and not scaled[0].kwargs
+                    and _only_user(scaled[0], add) and set(add.args) == {last, scaled[0]}):
+                constant = [a for a in scaled[0].args if a is not ones[0]]
+                if len(constant) == 1 and type(constant[0]) is float:
+                    last, shift = add, constant[0]
+        replace(last, terms, weights, positive_part, shift)
+    for node in list(copy.nodes):
+        found = products_of(node)
+        if found is not None and node.users and not any(_call(u, torch.stack) for u in node.users):
+            replace(node, [(PRODUCTS, found)], None, False, None)
+    if written:
+        _drop_dead_nodes(copy, written)
+
+
+def share_leading_rows(copy: fx.Graph) -> None:
+    """In a copy of a graph: the rows of a column slice are its parent's, so what is
+    computed from data of all of them in one layer is what the next one computes.  Merges
+    features[arange(number of rows)] and its products with a matrix, which are only read
+    by operators, and reads the rows in place where a product is all that does."""
+    from ..matrix_api.matrix import gen_arange
+    from ..ops.fused_op import _edge_score, _leading_rows
+    if any(_writes_in_place(n) for n in copy.nodes):
+        return
+    for node in list(copy.nodes):
+        if not _is_method(node, "_CAPI_GetNumRows"):
+            continue
+        sliced = node.args[0]
+        if (_call(sliced, operator.getitem) and sliced.args[1] == 0
+                and _is_method(sliced.args[0], "_CAPI_Slicing") and sliced.args[0].args[2] == 1):
+            node.args = (sliced.args[0].args[0],)
+
+    def only_read(node):
+        return all(_call(u, torch.matmul, operator.matmul, _edge_score) or _is_wrapped(u, "_before_sddmm")
+                   or (_call(u, operator.getitem) and u.args[1] is node) for u in node.users)
+
+    seen: Dict[str, fx.Node] = {}
+    for node in list(copy.nodes):
+        if not (_is_method(node, "_CAPI_GetNumRows") or _call(node, gen_arange)
+                or _call(node, operator.getitem, torch.matmul, operator.matmul)
+                and all(isinstance(a, fx.Node) for a in node.args)):
+            continue
+        if not _is_method(node, "_CAPI_GetNumRows") and not only_read(node):
+            continue
+        key = f"{node.op}|{node.target}|{node.args}|{node.kwargs}"
+        if key in seen:
+            node.replace_all_uses_with(seen[key])
+            copy.erase_node(node)
+        else:
+            seen[key] = node
+    for node in list(copy.nodes):
+        if (_call(node, operator.getitem) and _call(node.args[1], gen_arange) and node.users
+                and all(_call(u, torch.matmul, operator.matmul) for u in node.users)
+                and node.args[1].kwargs.get("dtype") is torch.int64
+                and node.args[1].kwargs.get("device") == "cuda" and len(node.args[1].args) == 1):
+            with copy.inserting_before(node):
+                rows = copy.call_function(_leading_rows, args=(node.args[0], node.args[1].args[0]))
+            node.replace_all_uses_with(rows)
+    _drop_dead_nodes(copy)
 
 
 # --------------------------------------------------------------- formats

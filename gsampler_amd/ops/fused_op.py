@@ -7,8 +7,10 @@
 """
 import torch
 
+from .. import _library
 from ..format import _COO, _CSC, _CSR
 from ._common import infer_broadcast_shape
+from .sddmm import _after_sddmm, _before_sddmm
 
 torch.fx.wrap("_before_e_div_u_sum")
 
@@ -32,6 +34,43 @@ def _before_e_div_u_sum(num_rows, num_cols, e, u, u_target):
     n_out = num_cols if u_target == 0 else num_rows
     v = torch.zeros((n_out,) + feat, dtype=e.dtype, device=e.device)
     return u2, e2, v, squeeze
+
+
+# kinds of terms, as gs_edge_score numbers them
+VALUE, QUOTIENT, PRODUCTS = 0, 1, 2
+
+
+def _edge_score(g, kinds, lhs, rhs, targets, weights, positive_part, shift, on_format):
+    """What a compiled sampler's scores are computed by: a weighted sum of terms per edge
+    (no weights: the one term), its positive part, plus a constant -- in one kernel, or by
+    the operators that the sampler was written with where that does not take the call."""
+    out = _library.native.edge_score(g, kinds, lhs, rhs, targets, weights, positive_part,
+                                     shift or 0.0, on_format)
+    if out is not None:
+        return out
+    terms = []
+    for k, kind in enumerate(kinds):
+        if kind == VALUE:
+            terms.append(lhs[k])
+            continue
+        left, right, out, squeeze = _before_sddmm(
+            g._CAPI_GetNumEdges(), "mul" if kind == PRODUCTS else "div", lhs[k], rhs[k])
+        g._CAPI_SDDMM("mul" if kind == PRODUCTS else "div", left, right, out, targets[2 * k],
+                      targets[2 * k + 1], on_format)
+        out = _after_sddmm(out, squeeze)
+        terms.append(torch.sum(out, dim=1) if kind == PRODUCTS else out)
+    out = terms[0] if weights is None else torch.matmul(torch.stack(terms, dim=1), weights)
+    if positive_part:
+        out = torch.relu(out)
+    return out if shift is None else out + shift * torch.ones_like(out)
+
+
+def _leading_rows(x, n):
+    """x[torch.arange(n)], to be read only: a view where that is the same."""
+    if (type(x) is torch.Tensor and x.is_cuda and x.dim() >= 1 and x.is_contiguous()
+            and n <= x.shape[0] and x.device.index == torch.cuda.current_device()):
+        return x.narrow(0, 0, n)
+    return x[torch.arange(n, dtype=torch.int64, device="cuda")]
 
 
 def fused_u_mul_v(m, lhs1, rhs1, lhs2, rhs2, on_format=_COO):

@@ -778,6 +778,12 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
  *   are written through edge_map like gs_sddmm's (the reference's fused kernels
  *   write by edge position, which differs from its own SDDMM on a converted
  *   format).
+ * gs_edge_score: out[eid] = sum over up to four terms of weights[k] * term_k, fp32
+ *   (without weights: one term, as it is), optionally its positive part, plus `shift`.
+ *   A term is a value of the edge's own (lhs), a quotient lhs[t_l] / rhs[t_r], or the
+ *   sum over a feature of 1 to 63 products lhs[t_l, i] * rhs[t_r, i]; all of the last
+ *   kind have one length.  Products and quotients are rounded before they are added;
+ *   the order of additions is fixed (edgeops.hip).
  * gs_spmm: out[dst] = reduce(out[dst], op(u[src], e[eid])), fp32.  Outputs
  *   are accumulators: the caller zero-fills them (python/gs/ops/spmm.py:56).
  *   COO: u_target 0 reduces onto columns, 2 onto rows (atomics).  Compressed:
@@ -798,6 +804,18 @@ int gs_sddmm(int format, const int64_t* a, const int64_t* b, int64_t num_major,
              int rhs_target, int64_t lhs_len, int64_t rhs_len, int64_t out_len,
              int64_t reduce_size, const int64_t* lhs_off, const int64_t* rhs_off,
              gs_stream_t stream);
+enum { GS_SCORE_VALUE = 0, GS_SCORE_QUOTIENT = 1, GS_SCORE_PRODUCTS = 2 };
+#define GS_SCORE_MAX_TERMS 4
+#define GS_SCORE_MAX_LEN 63
+typedef struct gs_score_term {
+  const float* lhs;
+  const float* rhs; /* unused by GS_SCORE_VALUE */
+  int kind, lhs_target, rhs_target;
+} gs_score_term;
+int gs_edge_score(int format, const int64_t* a, const int64_t* b, int64_t num_major,
+                  int64_t nnz, const int64_t* edge_map, const gs_score_term* terms,
+                  int num_terms, int64_t feature_len, const float* weights, int positive_part,
+                  float shift, float* out, gs_stream_t stream);
 int gs_fused_u_op_v(int format, const int64_t* a, const int64_t* b,
                     int64_t num_major, int64_t nnz, const int64_t* edge_map,
                     int op, int dtype,
