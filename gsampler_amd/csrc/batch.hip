@@ -14,6 +14,20 @@ __global__ __launch_bounds__(kBlock) void decode_batch_ids_kernel(
   if (orig) orig[i] = v - b * stride;
 }
 
+// out[i] = ids[i] + batch of item i * stride (without ids: the offset alone).  A few
+// thousand items, whose batch pointer stays in the scalar cache: one launch where the
+// batch of every item, the product and the sum were three (a ShaDow slice: five in all,
+// 26 us with the gaps between them).
+__global__ __launch_bounds__(kBlock) void encode_batch_ids_kernel(
+    const int64_t* __restrict__ ids, const int64_t* __restrict__ batch_ptr, int64_t num_batches,
+    int64_t n, int64_t stride, int64_t* __restrict__ out) {
+  const int64_t first = (int64_t)blockIdx.x * kBlock, i = first + threadIdx.x;
+  const int64_t last = first + kBlock < n ? first + kBlock - 1 : n - 1;
+  const SegmentSpan span = segment_span(batch_ptr, num_batches, first, last);
+  if (i >= n) return;
+  out[i] = (ids ? ids[i] : 0) + span.segment_at(batch_ptr, i) * stride;
+}
+
 // Batch b's piece is indptr[offset[b] .. offset[b+1]] (inclusive) rebased to 0,
 // written at out[offset[b] - offset[0] + b ...]: the pieces tile the output.  A
 // work-group takes kSplitTile consecutive output elements; the pieces start at
@@ -110,6 +124,19 @@ int gs_decode_batch_ids(const int64_t* encoded, int64_t n, int64_t stride,
             decode_batch_ids_kernel<<<dim3((unsigned)ceil_div(n, kBlock)),
                                       dim3(kBlock), 0, s>>>(encoded, n, stride,
                                                             out_orig, out_batch));
+  return GS_OK;
+}
+
+int gs_encode_batch_ids(const int64_t* ids, const int64_t* batch_ptr, int64_t num_batches,
+                        int64_t n, int64_t stride, int64_t* out, gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(n >= 0 && num_batches >= 0, "encode_batch_ids: negative size");
+  if (n == 0) return GS_OK;
+  GS_REQUIRE(num_batches > 0 && batch_ptr && out, "encode_batch_ids: null pointer");
+  hipStream_t s = as_stream(stream);
+  GS_LAUNCH("encode_batch_ids", s,
+            encode_batch_ids_kernel<<<dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, s>>>(
+                ids, batch_ptr, num_batches, n, stride, out));
   return GS_OK;
 }
 

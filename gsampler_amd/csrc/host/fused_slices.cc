@@ -34,13 +34,23 @@ std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tenso
   return so;
 }
 
-// Reading a slice in place pays when its columns are long: the kernels look a
-// run of a few thousand consecutive edges up in the column pointer once, and
-// only runs inside one column (or across one border) are free of per-edge
-// look-ups.  A slice of short columns is small: it is written once (and kept
-// for the next operator on the same columns) and the plain operators run on it.
-bool Graph::read_in_place(int64_t slice_nnz, int64_t num_cols_picked) {
+// A slice of a matrix in device memory is read in place whatever its columns are like:
+// a wavefront looks the columns of its run of edges up once, all lanes together
+// (200 K columns of 2 to 300 edges, 1 K to 150 K of them picked: row sums of squares 43
+// to 387 us in place, 60 to 931 by writing the slice first, row slices 75 to 402 and 103
+// to 866; the row slice of 8.4 M edges in 9.4 K columns 98 and 161).  From pinned host
+// memory the ids would cross the bus again for every pass: there only slices of long
+// columns are, which take fewer bytes in place even so.
+bool Graph::read_in_place(const Compressed& m, int64_t slice_nnz, int64_t num_cols_picked) {
+  if (m.indices.is_cuda()) return true;
   return slice_nnz >= (int64_t(1) << 20) && slice_nnz >= 4096 * num_cols_picked;
+}
+
+// The int32 copy of the ids for passes over a slice: made at once for a large slice of
+// long columns, else when such passes have read as many ids as the matrix has edges.
+static torch::Tensor narrow_for_slice(const Compressed& m, int64_t slice_nnz, int64_t num_cols_picked) {
+  const bool large = slice_nnz >= (int64_t(1) << 20) && slice_nnz >= 4096 * num_cols_picked;
+  return m.narrow_indices(large ? -1 : slice_nnz);
 }
 
 const MajorResult& Graph::written_slice(SliceOffsets& so) {
@@ -67,7 +77,7 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
   SliceOffsets& so = *shared;
   if (so.nnz == 0) return;
-  if (!read_in_place(so.nnz, cols.numel())) {
+  if (!read_in_place(m, so.nnz, cols.numel())) {
     const MajorResult& r = written_slice(so);
     torch::Tensor w = efeat.index_select(0, edge_index(m.e_ids, r.select));
     torch::Tensor ws =
@@ -80,7 +90,7 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
   torch::Tensor ws = new_workspace(gs_sliced_e_square_sum_workspace_bytes(so.nnz, num_rows_),
                                    m.indptr);
   const torch::Tensor e_ids = m.e_ids.has_value() ? m.e_ids.value() : torch::Tensor();
-  const torch::Tensor narrow = m.narrow_indices();  // half the bytes behind every id
+  const torch::Tensor narrow = narrow_for_slice(m, so.nnz, cols.numel());
   GS_CALL(gs_sliced_e_square_sum(cptr(m.indptr), cptr(m.indices),
                                  narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
                                  cptr(cols), cols.numel(),
@@ -103,7 +113,7 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
   // is queued into buffers sized by the bound (every edge kept) and runs while
   // the number travels
   AsyncCount kept = AsyncCount::mirrored();
-  const torch::Tensor narrow = m.narrow_indices();  // half the bytes behind every id
+  const torch::Tensor narrow = narrow_for_slice(m, nnz, n);
   GS_CALL(gs_col_row_slice_count(cptr(m.indptr), cptr(m.indices),
                                  narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
                                  cptr(cols), cptr(key_offset),
@@ -138,7 +148,7 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
   SliceOffsets& so = *shared;
   MajorResult r;
-  if (read_in_place(so.nnz, cols.numel())) {
+  if (read_in_place(m, so.nnz, cols.numel())) {
     r = col_row_slice(m, cols, so.sub_indptr, so.nnz, torch::Tensor(), rows,
                       output_format & kCOO);
   } else {
@@ -170,21 +180,22 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   BatchOffsets::check(row_bptr, row.numel(), "BatchColRowSlicing");
   const Compressed& m = compressed(kCSC);
   const int64_t stride = num_rows_;
-  auto batch_of = [&](const torch::Tensor& bptr, int64_t n) {
-    torch::Tensor b = new_ids(n, m.indptr);
-    GS_CALL(gs_csc2coo(cptr(bptr), bptr.numel() - 1, n, mptr(b), cur_stream()));
-    return b;
+  // (ids in [first item of batch b, ...) moved by b * num_rows)
+  auto encoded = [&](const torch::Tensor& of, const torch::Tensor& bptr, int64_t n) {
+    torch::Tensor e = new_ids(n, m.indptr);
+    GS_CALL(gs_encode_batch_ids(cptr(of), cptr(bptr), bptr.numel() - 1, n, stride, mptr(e),
+                                cur_stream()));
+    return e;
   };
-  torch::Tensor key_offset = batch_of(col_bptr, col.numel()) * stride;
-  torch::Tensor picked = row + batch_of(row_bptr, row.numel()) * stride;
+  torch::Tensor key_offset = encoded(torch::Tensor(), col_bptr, col.numel());
+  torch::Tensor picked = encoded(row, row_bptr, row.numel());
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(col);
   SliceOffsets& so = *shared;
   MajorResult kept;
-  if (read_in_place(so.nnz, col.numel())) {
+  if (read_in_place(m, so.nnz, col.numel())) {
     kept = col_row_slice(m, col, so.sub_indptr, so.nnz, key_offset, picked, false);
   } else {
-    // short columns: the batched column slice with rows moved by batch * num_rows
-    // is written and row-sliced
+    // the batched column slice with rows moved by batch * num_rows is written and row-sliced
     MajorResult sliced = major_slice(m, col, false, col_bptr, stride);
     Compressed tmp(sliced.indptr, sliced.minor_ids);
     kept = minor_slice(tmp, picked, false);

@@ -429,7 +429,7 @@ class Graph : public torch::CustomClassHolder {
   std::mutex slice_offsets_guard_;
   std::shared_ptr<SliceOffsets> slice_offsets_;
   std::shared_ptr<SliceOffsets> slice_offsets_for(const torch::Tensor& cols);
-  static bool read_in_place(int64_t slice_nnz, int64_t num_cols_picked);
+  static bool read_in_place(const Compressed& m, int64_t slice_nnz, int64_t num_cols_picked);
   const MajorResult& written_slice(SliceOffsets& so);
   // CDF of edge_probs in the edge order of `format` (cached per weights tensor).
   torch::Tensor weight_cdf_for(const torch::Tensor& edge_probs, int64_t format);

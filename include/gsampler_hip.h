@@ -741,6 +741,9 @@ int gs_segment_sort_i64(const int64_t* indptr, int64_t num_segments,
  *    id / stride, out_orig = id - batch * stride (either output nullable).
  *    With gs_sorted_to_indptr over out_batch this is GetBatchOffsets,
  *    src/cuda/batch/encoding_decoding.cu:99-122.
+ *  gs_encode_batch_ids: the other way: out[i] = ids[i] + b * stride (ids NULL: the
+ *    offset alone) for the items [batch_ptr[b], batch_ptr[b + 1]) of batch b; the first
+ *    n items, batch_ptr[num_batches] >= n.
  *  gs_split_indptr: batch b gets indptr[offset[b] .. offset[b+1]] rebased to
  *    start at 0, written at out[offset[b] + b ...]; out_len =
  *    offset[num_batches] - offset[0] + num_batches.  SplitIndptrByOffsetCUDA,
@@ -749,6 +752,8 @@ int gs_segment_sort_i64(const int64_t* indptr, int64_t num_segments,
 int gs_decode_batch_ids(const int64_t* encoded, int64_t n, int64_t stride,
                         int64_t* out_orig, int64_t* out_batch,
                         gs_stream_t stream);
+int gs_encode_batch_ids(const int64_t* ids, const int64_t* batch_ptr, int64_t num_batches,
+                        int64_t n, int64_t stride, int64_t* out, gs_stream_t stream);
 int gs_split_indptr(const int64_t* indptr, const int64_t* offset,
                     int64_t num_batches, int64_t out_len, int64_t* out,
                     gs_stream_t stream);

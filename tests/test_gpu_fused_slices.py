@@ -138,7 +138,6 @@ def test_threads_with_other_columns_on_one_matrix():
     g._CAPI_LoadCSC(T(indptr), T(indices))
     w = torch.as_tensor((rng.random(indices.size) + 0.05).astype(np.float32), device=DEV)
     rows = T(rng.choice(20_000, size=300, replace=False))
-    # short columns' slices are written, long ones' read in place
     cols = [T(rng.integers(0, 700, size=n)) for n in (3, 40, 300, 500)]
 
     def once(c):
@@ -166,3 +165,53 @@ def test_threads_with_other_columns_on_one_matrix():
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("most,ncol", [(0, 5), (1, 0), (1, 300), (3, 1), (3, 70_000), (20, 9000), (700, 1500)])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_slices_of_short_columns(most, ncol, pinned):
+    """Columns of 0 to a few hundred edges, which a matrix in device memory is read in place
+    for: runs over more columns than a wavefront has lanes, slices of nothing, repeated
+    columns and ids that the matrix does not have; the written slice of a pinned one."""
+    rng = np.random.default_rng(most + ncol)
+    indptr, indices = random_csc(rng, 4000, 6000, most, hub_deg=3000 if most == 3 else 0)
+    if pinned and indices.size == 0:
+        return                                               # no memory to pin
+    place = (lambda a: T(a).cpu().pin_memory()) if pinned else T
+    g = gs.Graph(6000, 4000)
+    g._CAPI_LoadCSC(place(indptr), place(indices))
+    cols = rng.integers(0, 4000, size=ncol)
+    rows = rng.choice(6000, size=400, replace=False)
+    want = chained_col_row_slice(indptr, indices, cols, rows, None)
+    sub, index = g._CAPI_ColRowSlicing(T(cols), T(rows), gs.format._CSC, gs.format._CSC)
+    same((sub._CAPI_GetCSCIndptr(), sub._CAPI_GetCSCIndices(), index), (want[0], want[2], want[3]))
+    w = (rng.random(indices.size) + 0.05).astype(np.float32)
+    out = torch.zeros(6000, device=DEV)
+    g._CAPI_SlicedESquareSum(T(cols), torch.as_tensor(w, device=DEV), out)
+    _, _, sub_rows, sel = orc.col_slice(indptr, indices, cols)
+    sums = np.zeros(6000)
+    np.add.at(sums, sub_rows, w[sel].astype(np.float64) ** 2)
+    # at most 70 000 terms of 32 bits: rounded some sqrt(n) times 2^-24 apart
+    assert np.allclose(out.cpu().numpy(), sums, rtol=2e-5, atol=1e-30)
+    if ncol == 0:
+        return
+    ptr = np.array([0, ncol // 3, ncol // 3, ncol])
+    rptr = np.array([0, 150, 250, 400])
+    offset = np.repeat([0, 6000, 12000], np.diff(ptr))
+    moved = rows + np.repeat([0, 6000, 12000], np.diff(rptr))
+    want = chained_col_row_slice(indptr, indices, cols, moved, offset)
+    sub, index = g._CAPI_BatchColRowSlcing(T(cols), T(ptr), T(rows), T(rptr))
+    same((sub._CAPI_GetCSCIndptr(), sub._CAPI_GetCSCIndices(), index), (want[0], want[2], want[3]))
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 5000])
+def test_batch_ids_moved_by_their_batch(n):
+    rng = np.random.default_rng(n)
+    ptr = np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=300)), [n]])
+    ids, out = T(rng.integers(0, 10**9, size=n)), torch.empty(n, dtype=torch.int64, device=DEV)
+    batch = T(np.repeat(np.arange(301), np.diff(ptr)))
+    for of in (ids, None):
+        capi.check(capi.lib().gs_encode_batch_ids(of.data_ptr() if of is not None else None, T(ptr).data_ptr(),
+                                                  301, n, 10**10, out.data_ptr(), None))
+        torch.cuda.synchronize()
+        assert torch.equal(out, batch * 10**10 + (ids if of is not None else 0))
