@@ -112,6 +112,11 @@ SIGNATURES = {
     "gs_probe_line_gather": (_int, [_p, _i64, _i64, _u64, _int, _p, _p]),
     "gs_probe_sample_uniform": (_int, [_p, _i64, _p, _p, _i64, _i64, _int, _i64, _u64, _u64, _p,
                                        _p, _p, _p, _p, _p]),
+    "gs_encoded_square_sums_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "gs_encoded_square_sums_pay": (_int, [_i64, _i64, _i64]),
+    "gs_encoded_square_sums": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _p, _p,
+                                      _p, _p, _sz, _p]),
+    "gs_encoded_square_sums_rows": (_int, [_i64, _i64, _i64, _p, _p, _p, _sz, _p]),
     "gs_sliced_e_square_sum_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_sliced_e_square_sum": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _i64, _p, _sz,
                                       _p]),

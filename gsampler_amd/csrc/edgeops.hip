@@ -11,6 +11,7 @@
 // ones and the general-length paths favour simplicity.
 #include "common.h"
 #include "scan.h"
+#include "sums.h"
 
 namespace gs {
 
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
     val[i] = 0.f;
     if (e < nnz && vrun.near()) {
       const int64_t p = vrun.place(e);
-      dst[i] = dst_ids[p];
+      dst[i] = dst_ids[p] + vrun.id_offset(e);
       const int64_t eid = edge_map ? edge_map[p] : p;
       val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
                                  efeat ? efeat + eid : nullptr);
@@ -675,7 +676,7 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
       int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
       const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
       if (e < nnz) {
-        dst[i] = dst_ids[p];
+        dst[i] = dst_ids[p] + offset;
         val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
                                    efeat ? efeat + (edge_map ? edge_map[p] : p) : nullptr);
       }
@@ -800,7 +801,8 @@ __device__ __forceinline__ uint32_t run_cell(uint32_t start, uint32_t length) {
 // With a view the edges are those of a column slice that was never written:
 // dst_ids and efeat are then the parent's arrays (see SliceView).  A wavefront
 // takes consecutive edges, so it looks up the few columns of its own run only.
-template <typename IdT>
+// kKeys: the view moves its columns' ids (keys below 2^31).
+template <typename IdT, bool kKeys>
 __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
     const IdT* __restrict__ dst_ids, const int64_t* __restrict__ src_ids,
     const int64_t* __restrict__ edge_map, int64_t nnz, int64_t num_out, int kind,
@@ -832,8 +834,8 @@ __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
     if (view.on())
       vrun = view.run(first, (first + kPartWaveRun < nnz ? first + kPartWaveRun : nnz) - 1);
     const bool shifted = vrun.near();  // the same in every lane
-    auto take = [&](int i, int64_t p) {
-      const int64_t dst = (int64_t)dst_ids[p];
+    auto take = [&](int i, int64_t p, int64_t offset) {
+      const int64_t dst = (int64_t)dst_ids[p] + (kKeys ? offset : 0);
       const int64_t eid = edge_map ? edge_map[p] : p;
       val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
                                  efeat ? efeat + eid : nullptr);
@@ -851,7 +853,9 @@ __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
       }
 #pragma unroll
       for (int i = 0; i < kPartItems; ++i) {
-        const int64_t dst = (int64_t)id[i];
+        const int64_t e = first + i * kWave + lane;
+        const int64_t dst = (int64_t)id[i] +
+                            (kKeys ? (e < vrun.split ? (int)vrun.offset[0] : (int)vrun.offset[1]) : 0);
         row[i] = first + i * kWave + lane < nnz && dst >= 0 && dst < num_out ? (int)dst : -1;
         val[i] = edge_value<float>(kind, op, nullptr, &val[i]);
       }
@@ -859,7 +863,7 @@ __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
 #pragma unroll
       for (int i = 0; i < kPartItems; ++i) {
         const int64_t e = first + i * kWave + lane;
-        if (e < nnz) take(i, vrun.place(e));
+        if (e < nnz) take(i, vrun.place(e), vrun.id_offset(e));
       }
     } else {
 #pragma unroll
@@ -867,7 +871,7 @@ __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
         const int64_t e = first + i * kWave + lane;
         int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
         const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
-        if (e < nnz) take(i, p);
+        if (e < nnz) take(i, p, offset);
       }
     }
   }
@@ -1005,6 +1009,8 @@ __global__ __launch_bounds__(kAccThreads, 8) void rowsum_accumulate_kernel(
     const uint16_t* __restrict__ rows, const float* __restrict__ values,
     const uint32_t* __restrict__ cells, int64_t tile_stride, const RowUnit* __restrict__ units,
     const int* __restrict__ unit_total, float* __restrict__ partial) {
+  // (they begin at -0, which only additions move: a row of no entry stays -0, a row
+  // whose entries are zeros becomes +0)
   // Accumulators in double: this part adds doubles in LDS at twice the rate of
   // floats (602 M entries: 1.55 against 3.05 ms), and a slice's sums then carry
   // no rounding of their own before they are rounded to float once.
@@ -1015,7 +1021,7 @@ __global__ __launch_bounds__(kAccThreads, 8) void rowsum_accumulate_kernel(
   const int64_t u = blockIdx.x;
   if (u >= *unit_total) return;
   const RowUnit unit = units[u];
-  for (int j = t; j < kRangeRows; j += kAccThreads) acc[j] = 0.0;
+  for (int j = t; j < kRangeRows; j += kAccThreads) acc[j] = -0.0;
   for (int tile0 = unit.tile0; tile0 < unit.tile1; tile0 += kAccTiles) {
     const int tile = tile0 + t;
     uint32_t start = 0, length = 0;
@@ -1093,7 +1099,7 @@ __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
   // (a unit has the sums of all rows of its range, also of those past num_out)
   const float* p = partial + (row0 & (kRangeRows - 1)) + lane_row;
   auto sums_of = [&](int64_t u) { return *reinterpret_cast<const float4*>(p + u * kRangeRows); };
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  double acc[4] = {-0.0, -0.0, -0.0, -0.0};
   auto add = [&](const float4& v) {
     acc[0] += (double)v.x;
     acc[1] += (double)v.y;
@@ -1114,10 +1120,10 @@ __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
   __syncthreads();
   const int64_t i = row0 + threadIdx.x;
   if (threadIdx.x >= kFoldRows || i >= num_out) return;
-  double sum = 0.0;
+  double sum = -0.0;
 #pragma unroll
   for (int s = 0; s < kFoldShares; ++s) sum += share_sum[s][threadIdx.x];
-  if (sum != 0.0) out[i] += (float)sum;
+  if (__double_as_longlong(sum) != INT64_MIN) out[i] += (float)sum;  // INT64_MIN: the bits of -0
 }
 
 // dst_ids32: the same ids as dst_ids in 32 bits (a matrix's narrow copy), read
@@ -1137,13 +1143,18 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
   float* partial = (float*)(ws + p.off_partial);
   const int ranges = (int)p.ranges;
   const dim3 tiles_grid((unsigned)p.tiles);
-#define GS_ROWSUM_PART(IDT, IDS)                                                              \
+#define GS_ROWSUM_PART(IDT, IDS, KEYS)                                                        \
   GS_LAUNCH("rowsum_part", s,                                                                 \
-            rowsum_part_kernel<IDT><<<tiles_grid, dim3(kPartThreads), 0, s>>>(                \
+            (rowsum_part_kernel<IDT, KEYS>)<<<tiles_grid, dim3(kPartThreads), 0, s>>>(        \
                 IDS, src_ids, edge_map, nnz, num_out, kind, op, ufeat, efeat, ranges,         \
                 p.copy_bits, p.tile_stride, cells, rows, values, unit_total, view))
-  if (dst_ids32) GS_ROWSUM_PART(int32_t, dst_ids32);
-  else GS_ROWSUM_PART(int64_t, dst_ids);
+  if (view.sub_indptr != nullptr && view.key_offset != nullptr) {
+    if (dst_ids32) GS_ROWSUM_PART(int32_t, dst_ids32, true);
+    else GS_ROWSUM_PART(int64_t, dst_ids, true);
+  } else {
+    if (dst_ids32) GS_ROWSUM_PART(int32_t, dst_ids32, false);
+    else GS_ROWSUM_PART(int64_t, dst_ids, false);
+  }
 #undef GS_ROWSUM_PART
   GS_LAUNCH("rowsum_units", s,
             rowsum_units_kernel<<<dim3((unsigned)ranges), dim3(kUnitsThreads), 0, s>>>(
@@ -1155,6 +1166,27 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
             rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
                                  s>>>(partial, range_units, num_out, out));
   return GS_OK;
+}
+
+bool sums_by_range(int64_t nnz, int64_t num_out) {
+  return row_range_plan(GS_FMT_COO, nnz, num_out).total > 0;
+}
+
+size_t sliced_square_sum_bytes(int64_t nnz, int64_t num_out) {
+  return row_range_plan(GS_FMT_COO, nnz, num_out).total;
+}
+
+int sliced_square_sum(SliceView view, const int64_t* indices, const int32_t* indices32,
+                      int64_t nnz, const int64_t* edge_map, const float* efeat, float* out,
+                      int64_t num_out, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  const RowRangePlan plan = row_range_plan(GS_FMT_COO, nnz, num_out);
+  if (plan.total > 0 && workspace != nullptr && workspace_bytes >= plan.total)
+    return row_range_sum(plan, indices, indices32, nullptr, edge_map, nnz, num_out, 1,
+                         kOpCopyRhs, nullptr, efeat, out, workspace, s, view);
+  // short slices: combined per tile in LDS, one atomic per (tile, row present);
+  // ids outside [0, num_out) cannot occur for a slice of a checked matrix
+  return coo_sum_launch(indices, indices, edge_map, nnz, 1, kOpCopyRhs, nullptr, efeat, out,
+                        2, view, s);
 }
 
 static int check_view(int format, const int64_t* a, const int64_t* b,
@@ -1473,16 +1505,9 @@ int gs_sliced_e_square_sum(const int64_t* indptr, const int64_t* indices,
   if (slice_nnz == 0) return GS_OK;
   GS_REQUIRE(indptr && indices && cols && sub_indptr && efeat && out,
              "sliced_e_square_sum: null pointer");
-  hipStream_t s = as_stream(stream);
   const SliceView view{sub_indptr, cols, indptr, nullptr, num_cols_picked};
-  const RowRangePlan plan = row_range_plan(GS_FMT_COO, slice_nnz, num_out);
-  if (plan.total > 0 && workspace != nullptr && workspace_bytes >= plan.total)
-    return row_range_sum(plan, indices, indices32, nullptr, edge_map, slice_nnz, num_out, 1,
-                         kOpCopyRhs, nullptr, efeat, out, workspace, s, view);
-  // short slices: combined per tile in LDS, one atomic per (tile, row present);
-  // ids outside [0, num_out) cannot occur for a slice of a checked matrix
-  return coo_sum_launch(indices, indices, edge_map, slice_nnz, 1, kOpCopyRhs, nullptr, efeat, out,
-                        2, view, s);
+  return sliced_square_sum(view, indices, indices32, slice_nnz, edge_map, efeat, out, num_out,
+                           workspace, workspace_bytes, as_stream(stream));
 }
 
 int gs_e_div_u_sum(int format, const int64_t* a, const int64_t* b,

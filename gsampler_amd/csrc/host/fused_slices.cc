@@ -161,6 +161,15 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   return {g, edge_index(m.e_ids, r.select)};
 }
 
+// The ids `of` (undefined: zeros) of every batch moved by batch * stride.
+static torch::Tensor encoded_ids(const torch::Tensor& of, const torch::Tensor& bptr, int64_t n,
+                                 int64_t stride) {
+  torch::Tensor e = new_ids(n, bptr);
+  GS_CALL(gs_encode_batch_ids(cptr(of), cptr(bptr), bptr.numel() - 1, n, stride, mptr(e),
+                              cur_stream()));
+  return e;
+}
+
 // Per batch b: the columns col[col_bptr[b] : col_bptr[b+1]] restricted to the
 // rows row[row_bptr[b] : row_bptr[b+1]]; row ids become positions in `row`.
 // The returned edge index addresses the parent's edges.  One pass over the
@@ -180,15 +189,8 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   BatchOffsets::check(row_bptr, row.numel(), "BatchColRowSlicing");
   const Compressed& m = compressed(kCSC);
   const int64_t stride = num_rows_;
-  // (ids in [first item of batch b, ...) moved by b * num_rows)
-  auto encoded = [&](const torch::Tensor& of, const torch::Tensor& bptr, int64_t n) {
-    torch::Tensor e = new_ids(n, m.indptr);
-    GS_CALL(gs_encode_batch_ids(cptr(of), cptr(bptr), bptr.numel() - 1, n, stride, mptr(e),
-                                cur_stream()));
-    return e;
-  };
-  torch::Tensor key_offset = encoded(torch::Tensor(), col_bptr, col.numel());
-  torch::Tensor picked = encoded(row, row_bptr, row.numel());
+  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, col.numel(), stride);
+  torch::Tensor picked = encoded_ids(row, row_bptr, row.numel(), stride);
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(col);
   SliceOffsets& so = *shared;
   MajorResult kept;
@@ -214,6 +216,80 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   g->edge_bptr_ = kept.indptr.index_select(0, col_bptr);
   BatchOffsets::trust(g->edge_bptr_);
   return {g, edge_index(m.e_ids, kept.select)};
+}
+
+// What a layer-wise sampler asks an encoded slice (BatchColSlicing with encoding) for:
+// its rows with where every batch's begin, and the sums of its squared edge values on
+// them.  The slice is not written; the picked rows' edges come from EncodedRowSlicing.
+// Nothing where the slice has to be written after all: values that are no plain float32
+// edge data, or keys too many or too few for the pass.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> Graph::EncodedSquareSums(
+    torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor efeat) {
+  const Compressed& m = compressed(kCSC);
+  if (!m.indices.is_cuda() || !efeat.defined() || !efeat.is_cuda() ||
+      efeat.scalar_type() != torch::kFloat32 || efeat.dim() != 1 || !efeat.is_contiguous() ||
+      efeat.numel() != m.indices.numel())
+    return {};
+  seeds = ids(seeds, "seeds");
+  col_bptr = ids(col_bptr, "col_bptr");
+  const int64_t B = col_bptr.numel() - 1;
+  TORCH_CHECK(B >= 1, "BatchColSlicing: col_bptr needs at least two entries");
+  BatchOffsets::check(col_bptr, seeds.numel(), "BatchColSlicing");
+  const int64_t stride = num_rows_, n = seeds.numel();
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
+  const int64_t nnz = shared->nnz;
+  if (!gs_encoded_square_sums_pay(nnz, B, stride)) return {};
+  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, n, stride);
+  torch::Tensor row_bptr = new_ids(B + 1, m.indptr);
+  torch::Tensor ws = new_workspace(gs_encoded_square_sums_workspace_bytes(nnz, B, stride), m.indptr);
+  const torch::Tensor narrow = m.narrow_indices(2 * nnz);  // the row slice reads them as well
+  const torch::Tensor e_ids = m.e_ids.has_value() ? m.e_ids.value() : torch::Tensor();
+  int64_t* mirror = OffsetMirror::reserve(row_bptr);
+  GS_CALL(gs_encoded_square_sums(cptr(m.indptr), cptr(m.indices),
+                                 narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+                                 cptr(seeds), n, cptr(shared->sub_indptr), nnz, cptr(key_offset), B,
+                                 stride, cptr(e_ids), efeat.data_ptr<float>(), mptr(row_bptr),
+                                 mirror, ws.data_ptr(), (size_t)ws.numel(), cur_stream()));
+  OffsetMirror::arm(row_bptr);
+  const int64_t bound = std::min(nnz, B * stride);
+  torch::Tensor rows = new_ids(bound, m.indptr);
+  torch::Tensor sums = torch::empty({bound}, efeat.options().requires_grad(false));
+  GS_CALL(gs_encoded_square_sums_rows(nnz, B, stride, mptr(rows), sums.data_ptr<float>(),
+                                      ws.data_ptr(), (size_t)ws.numel(), cur_stream()));
+  const int64_t total = OffsetMirror::values(row_bptr).back();
+  BatchOffsets::trust(row_bptr, total);
+  return std::make_tuple(trim_to(rows, total), row_bptr, trim_to(sums, total));
+}
+
+// BatchRowSlicing of the encoded slice of (seeds, col_bptr) by row_ids, positions in
+// `rows` (EncodedSquareSums) that lie in it; the edge index addresses this matrix's edges.
+GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
+                                       torch::Tensor rows, torch::Tensor row_ids,
+                                       torch::Tensor row_bptr) {
+  seeds = ids(seeds, "seeds");
+  col_bptr = ids(col_bptr, "col_bptr");
+  row_ids = ids(row_ids, "row_ids");
+  row_bptr = ids(row_bptr, "row_bptr");
+  TORCH_CHECK(col_bptr.numel() == row_bptr.numel() && col_bptr.numel() >= 2,
+              "BatchRowSlicing: column and row batch pointers must have the same length");
+  BatchOffsets::check(col_bptr, seeds.numel(), "BatchColSlicing");
+  BatchOffsets::check(row_bptr, row_ids.numel(), "BatchRowSlicing");
+  const Compressed& m = compressed(kCSC);
+  const int64_t stride = num_rows_;
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
+  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, seeds.numel(), stride);
+  torch::Tensor picked = encoded_ids(rows.index_select(0, row_ids), row_bptr, row_ids.numel(), stride);
+  const MajorResult r = col_row_slice(m, seeds, shared->sub_indptr, shared->nnz, key_offset, picked,
+                                      true);
+  GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
+  g->col_bptr_ = col_bptr;
+  g->orig_col_ids_ = seeds;
+  g->row_encoding_size_ = stride;
+  g->edge_bptr_ = g->csc_->indptr.index_select(0, col_bptr);
+  BatchOffsets::trust(g->edge_bptr_);
+  g->row_bptr_ = row_bptr;
+  g->orig_row_ids_ = row_ids;
+  return {g, edge_index(m.e_ids, r.select)};
 }
 
 }  // namespace gs

@@ -314,6 +314,10 @@ class Graph : public torch::CustomClassHolder {
   std::vector<int64_t> BatchGetColCounts();
   GraphAndIndex BatchColSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
                                 bool encoding);
+  c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> EncodedSquareSums(
+      torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor efeat);
+  GraphAndIndex EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
+                                  torch::Tensor row_ids, torch::Tensor row_bptr);
   GraphAndIndex BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr,
                                   torch::Tensor row, torch::Tensor row_bptr);
   GraphAndIndex BatchRowSlicing(torch::Tensor row_ids, torch::Tensor row_bptr);

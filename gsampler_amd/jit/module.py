@@ -171,6 +171,7 @@ class compile:  # noqa: N801 -- the reference's public name
             return None
         passes.chain_layers(gm, graph)
         passes.compute_edge_scores(graph)
+        passes.sum_encoded_slices_in_place(graph)
         passes.share_leading_rows(graph)
         return fx.GraphModule(gm, graph).forward
 

@@ -34,6 +34,9 @@ and, in the copy of the graph that calls run (like chain_layers):
 
   compute_edge_scores           products of features summed over the feature, stacked
                                 and multiplied by a vector  -> one kernel
+  sum_encoded_slices_in_place   an encoded column slice of a super-batch that is summed
+                                (squares onto rows) and sliced by rows picked of it is
+                                never written
   share_leading_rows            features of all rows of a column slice: the parent's, once
 
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
@@ -813,6 +816,101 @@ def compute_edge_scores(copy: fx.Graph) -> None:
             replace(node, [(PRODUCTS, found)], None, False, None)
     if written:
         _drop_dead_nodes(copy, written)
+
+
+def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
+    """In a copy of a graph: s = A._CAPI_BatchColSlicing(seeds, ptr, True) whose matrix s[0]
+    is only asked for its rows and shape, summed once by _CAPI_FusedESquareSum(copy_rhs, sum,
+    e = w[s[1]]) onto rows, and row-sliced by what _CAPI_BatchListSampling[WithProbs] picked of
+    those rows, and whose edge index s[1] only gathers edge data that feeds those operators
+        => _encoded_square_sums(A, seeds, ptr, w) and _encoded_row_slice, whose index
+           addresses A's edges."""
+    from ..ops.fused_op import _encoded_row_slice, _encoded_square_sums
+    order = {n: i for i, n in enumerate(copy.nodes)}
+
+    def free_operator(node, *names):
+        return (node.op == "call_function"
+                and str(getattr(node.target, "__name__", node.target)).split(".")[0] in names)
+
+    for slicing in list(copy.nodes):
+        if not _is_method(slicing, "_CAPI_BatchColSlicing") or slicing.args[3] is not True:
+            continue
+        parent, seeds, ptr = slicing.args[:3]
+        sliced, index = _getitem_users(slicing, 0), _getitem_users(slicing, 1)
+        if len(sliced) != 1 or len(index) != 1 or len(slicing.users) != 2:
+            continue
+        g, idx = sliced[0], index[0]
+        gathered = list(idx.users)
+        if not all(_is_wrapped(n, "data_index") and n.args[1] is idx and n.args[0] is not idx
+                   and isinstance(n.args[0], fx.Node) and n.args[0] in order
+                   and order[n.args[0]] < order[slicing] for n in gathered):
+            continue
+        sums, row_slices, rows, shapes, ok = [], [], [], [], True
+        for user in g.users:
+            if (_is_method(user, "_CAPI_FusedESquareSum") and user.args[0] is g
+                    and user.args[1] == "copy_rhs" and user.args[2] == "sum" and user.args[8] == 2
+                    and user.args[4] in gathered and list(user.all_input_nodes).count(g) == 1):
+                sums.append(user)
+            elif _is_method(user, "_CAPI_BatchRowSlicing") and user.args[0] is g:
+                row_slices.append(user)
+            elif _is_method(user, "_CAPI_BatchGetRows"):
+                rows.append(user)
+            elif _is_method(user, "_CAPI_GetNumRows") or _is_method(user, "_CAPI_GetNumCols"):
+                shapes.append(user)
+            else:
+                ok = False
+        if not ok or len(sums) != 1 or not row_slices:
+            continue
+        total = sums[0]
+        accumulator, before = total.args[5], total.args[5].args[0]
+        if not (_call(accumulator, operator.getitem) and accumulator.args[1] == 0
+                and _is_wrapped(before, "_before_spmm")):
+            continue
+        after = [n for n in accumulator.users if _is_wrapped(n, "_after_spmm")]
+        if (len(after) != 1 or set(accumulator.users) != {total, after[0]}
+                or any(not _only_user(n, before) for n in shapes)
+                or any(not _call(n, operator.getitem) or n.args[1] not in (0, 1)
+                       for r in rows for n in r.users)):
+            continue
+        row_ptrs = [n for r in rows for n in _getitem_users(r, 1)]
+        regather = []
+        row_indices = [i for rs in row_slices for i in _getitem_users(rs, 1)]
+        for w in gathered:
+            for user in w.users:
+                if user is total or user is before:
+                    continue
+                if _is_wrapped(user, "data_index") and user.args[0] is w and user.args[1] in row_indices:
+                    regather.append(user)
+                else:
+                    ok = False
+        for rs in row_slices:
+            picked, picked_ptr = rs.args[1], rs.args[2]
+            if not (_call(picked, operator.getitem) and picked.args[1] == 0
+                    and _call(picked_ptr, operator.getitem) and picked_ptr.args[1] == 1
+                    and picked.args[0] is picked_ptr.args[0]
+                    and free_operator(picked.args[0], "_CAPI_BatchListSampling",
+                                      "_CAPI_BatchListSamplingWithProbs")
+                    and picked.args[0].args and picked.args[0].args[-1] in row_ptrs):
+                ok = False            # rows that may not be the slice's
+        if not ok:
+            continue
+        with copy.inserting_before(slicing):
+            found = copy.call_function(_encoded_square_sums, args=(parent, seeds, ptr, total.args[4].args[0],
+                                                                   total.args[9]))
+            part, ids, ids_ptr, sums_of = (copy.call_function(operator.getitem, args=(found, i))
+                                           for i in range(4))
+        for r in rows:
+            for n in list(r.users):
+                n.replace_all_uses_with(ids if n.args[1] == 0 else ids_ptr)
+        after[0].replace_all_uses_with(sums_of)
+        for rs in row_slices:
+            with copy.inserting_before(rs):
+                picked_edges = copy.call_function(_encoded_row_slice, args=(part, rs.args[1], rs.args[2]))
+            rs.replace_all_uses_with(picked_edges)
+        for node in regather:
+            node.replace_input_with(node.args[0], node.args[0].args[0])
+        _drop_dead_nodes(copy, [total])
+        order = {n: i for i, n in enumerate(copy.nodes)}
 
 
 def share_leading_rows(copy: fx.Graph) -> None:

@@ -11,6 +11,7 @@ from .. import _library
 from ..format import _COO, _CSC, _CSR
 from ._common import infer_broadcast_shape
 from .sddmm import _after_sddmm, _before_sddmm
+from .spmm import _after_spmm, _before_spmm
 
 torch.fx.wrap("_before_e_div_u_sum")
 
@@ -63,6 +64,34 @@ def _edge_score(g, kinds, lhs, rhs, targets, weights, positive_part, shift, on_f
     if positive_part:
         out = torch.relu(out)
     return out if shift is None else out + shift * torch.ones_like(out)
+
+
+def _encoded_square_sums(g, seeds, seeds_ptr, values, on_format):
+    """What a compiled super-batched sampler asks an encoded column slice for: (the slice for
+    _encoded_row_slice, its rows, where every batch's begin, sums of the squared values on
+    them) -- without writing the slice where that can be."""
+    from ..matrix_api.matrix import data_index
+    if type(values) is torch.Tensor and not values.requires_grad:
+        found = g._CAPI_EncodedSquareSums(seeds, seeds_ptr, values)
+        if found is not None:
+            rows, rows_ptr, sums = found
+            return (g, seeds, seeds_ptr, rows), rows, rows_ptr, sums
+    sub, index = g._CAPI_BatchColSlicing(seeds, seeds_ptr, True)
+    rows, rows_ptr = sub._CAPI_BatchGetRows()
+    values = data_index(values, index)
+    out, arg_u, arg_e, squeeze = _before_spmm(sub._CAPI_GetNumRows(), sub._CAPI_GetNumCols(), "copy_rhs",
+                                              "sum", None, values, 2)
+    sub._CAPI_FusedESquareSum("copy_rhs", "sum", None, values, out, arg_u, arg_e, 2, on_format)
+    return (sub, index), rows, rows_ptr, _after_spmm(out, squeeze)
+
+
+def _encoded_row_slice(part, row_ids, rows_ptr):
+    """The picked rows of such a slice: (matrix, index into the sliced matrix's edges)."""
+    from ..matrix_api.matrix import data_index
+    if len(part) == 4:
+        return part[0]._CAPI_EncodedRowSlicing(*part[1:], row_ids, rows_ptr)
+    sub, index = part[0]._CAPI_BatchRowSlicing(row_ids, rows_ptr)
+    return sub, data_index(part[1], index)
 
 
 def _leading_rows(x, n):

@@ -456,6 +456,30 @@ int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indi
                     void* workspace, size_t workspace_bytes, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * What a layer-wise sampler asks such a slice for, without writing it: the sums of
+ * its squared edge values on its rows.
+ *   gs_encoded_square_sums_pay   whether these calls are ahead of writing the slice
+ *   key_offset[num_cols_picked]  batch of the column * stride (gs_encode_batch_ids)
+ *   efeat                        values of the parent's edges (through edge_map, nullable)
+ *   row_ptr[num_batches + 1]     where each batch's rows begin; row_ptr_mirror the
+ *       same in pinned host memory (nullable)
+ * gs_encoded_square_sums_rows then writes the row_ptr[num_batches] row ids, ascending
+ * within a batch, and their sums, from the same workspace (at most
+ * min(nnz, num_batches * stride) of either).
+ * ---------------------------------------------------------------------- */
+size_t gs_encoded_square_sums_workspace_bytes(int64_t nnz, int64_t num_batches, int64_t stride);
+int gs_encoded_square_sums_pay(int64_t nnz, int64_t num_batches, int64_t stride);
+int gs_encoded_square_sums(const int64_t* indptr, const int64_t* indices, const int32_t* indices32,
+                           const int64_t* cols, int64_t num_cols_picked,
+                           const int64_t* sub_indptr, int64_t nnz, const int64_t* key_offset,
+                           int64_t num_batches, int64_t stride, const int64_t* edge_map,
+                           const float* efeat, int64_t* row_ptr, int64_t* row_ptr_mirror,
+                           void* workspace, size_t workspace_bytes, gs_stream_t stream);
+int gs_encoded_square_sums_rows(int64_t nnz, int64_t num_batches, int64_t stride,
+                                int64_t* out_rows, float* out_sums, void* workspace,
+                                size_t workspace_bytes, gs_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * Column slice of a super-batch with its rows numbered anew: batch b's rows are
  * the ids that some edge of its columns has, in increasing order, and batch b's
  * numbers follow batch b - 1's (what the reference gets from ids encoded as

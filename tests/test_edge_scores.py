@@ -192,3 +192,34 @@ def test_compiled_equals_eager(func, kind):
     if kind == "gradients" and want[0].requires_grad:
         (dw,), (dg,) = (torch.autograd.grad(x[0].sum(), weights) for x in (want, got))
         assert torch.equal(dw, dg)
+
+
+# ------------------------------------------------- encoded slices that are not written
+def layer(A, seeds, ptr, power=2, also=None, picks="listed"):
+    sub = A[:, seeds::ptr]
+    sub.edata["p"] = sub.edata["w"] ** power
+    prob = sub.sum("p", axis=1)
+    rows, rows_ptr = sub.all_rows()
+    if picks == "own":
+        part = sub[prob.argsort()[:4]::torch.tensor([0, 2, 4], device=prob.device), :]
+        return part.edata["w"], rows
+    part, index = sub.collective_sampling(3, prob, rows_ptr, False)
+    out = part.div("w", prob[index], axis=1).edata["w"], rows[index]
+    return out + ((sub.edata["w"],) if also == "edges" else (sub.sum("w", axis=1),) if also == "sum" else ())
+
+
+@pytest.mark.parametrize("options,kernel", [
+    ({}, True), (dict(power=3), False), (dict(also="edges"), False), (dict(also="sum"), False),
+    (dict(picks="own"), False)])
+def test_what_is_summed_in_place(options, kernel):
+    bm = gs.BatchMatrix()
+    m = gs.Matrix(gs.Graph(10, 10))
+    m.edata["w"] = torch.rand(7)
+    bm.load_from_matrix(m, True)
+
+    def sampler(A, seeds, ptr):
+        return layer(A, seeds, ptr, **options)
+
+    t = ran(gs.jit.compile(func=sampler, args=(bm, torch.arange(6), torch.tensor([0, 3, 6]))))
+    assert t.count(fused_op._encoded_square_sums) == kernel and ("_CAPI_BatchColSlicing" in t) != kernel
+    assert t.count(fused_op._encoded_row_slice) == kernel and ("_CAPI_BatchRowSlicing" in t) != kernel
