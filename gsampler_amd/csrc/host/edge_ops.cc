@@ -245,6 +245,36 @@ c10::optional<torch::Tensor> Graph::EdgeScore(const std::vector<int64_t>& kinds,
   return out;
 }
 
+c10::optional<torch::Tensor> Graph::NormaliseColumns(torch::Tensor values,
+                                                     c10::optional<torch::Tensor> select,
+                                                     c10::optional<torch::Tensor> row_divisor) {
+  if (!csc_ || csc_->e_ids.has_value() || (coo_ && coo_->e_ids.has_value()) || num_edges_ <= 0 ||
+      csc_->indices.numel() != num_edges_ || !csc_->indices.is_cuda() || !csc_->indptr.is_cuda() ||
+      at::impl::torch_function_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return {};
+  // (the operators this stands for write into arrays of their own, without gradients)
+  if (!plain_values(values, false) || values.dim() != 1 || !values.is_contiguous() ||
+      (!select.has_value() && values.size(0) != num_edges_))
+    return {};
+  if (select.has_value() &&
+      (!select->is_cuda() || select->scalar_type() != torch::kInt64 || select->dim() != 1 ||
+       select->numel() != num_edges_ || !select->is_contiguous()))
+    return {};
+  if (row_divisor.has_value()) {
+    if (!plain_values(*row_divisor, false) || row_divisor->dim() != 1 ||
+        row_divisor->size(0) < num_rows_)
+      return {};
+    row_divisor = row_divisor->contiguous();
+  }
+  torch::Tensor out = torch::empty({num_edges_}, values.options().requires_grad(false));
+  torch::Tensor sums = torch::empty({num_cols_}, out.options().dtype(torch::kFloat64));
+  GS_CALL(gs_normalise_columns(cptr(csc_->indptr), num_cols_, cptr(csc_->indices), num_edges_,
+                               values.data_ptr<float>(), select.has_value() ? cptr(*select) : nullptr,
+                               row_divisor.has_value() ? row_divisor->data_ptr<float>() : nullptr,
+                               sums.data_ptr<double>(), out.data_ptr<float>(), cur_stream()));
+  return out;
+}
+
 void Graph::FusedUOPV(const std::string& op, torch::Tensor lhs1,
                       torch::Tensor rhs1, torch::Tensor out1, torch::Tensor lhs2,
                       torch::Tensor rhs2, torch::Tensor out2, int64_t on_format) {

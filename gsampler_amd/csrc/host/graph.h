@@ -272,6 +272,10 @@ class Graph : public torch::CustomClassHolder {
                                          const std::vector<int64_t>& targets,
                                          c10::optional<torch::Tensor> weights,
                                          bool positive_part, double shift, int64_t on_format);
+  // gs_normalise_columns; nothing where the call is not one for it (see EdgeScore).
+  c10::optional<torch::Tensor> NormaliseColumns(torch::Tensor values,
+                                                c10::optional<torch::Tensor> select,
+                                                c10::optional<torch::Tensor> row_divisor);
   void FusedUOPV(const std::string& op, torch::Tensor lhs1, torch::Tensor rhs1,
                  torch::Tensor out1, torch::Tensor lhs2, torch::Tensor rhs2,
                  torch::Tensor out2, int64_t on_format);

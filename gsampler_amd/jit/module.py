@@ -172,6 +172,7 @@ class compile:  # noqa: N801 -- the reference's public name
         passes.chain_layers(gm, graph)
         passes.compute_edge_scores(graph)
         passes.sum_encoded_slices_in_place(graph)
+        passes.normalise_columns(graph)
         passes.share_leading_rows(graph)
         return fx.GraphModule(gm, graph).forward
 

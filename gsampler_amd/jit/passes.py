@@ -37,6 +37,7 @@ and, in the copy of the graph that calls run (like chain_layers):
   sum_encoded_slices_in_place   an encoded column slice of a super-batch that is summed
                                 (squares onto rows) and sliced by rows picked of it is
                                 never written
+  normalise_columns             edge values divided by row and by their columns' sums
   share_leading_rows            features of all rows of a column slice: the parent's, once
 
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
@@ -814,6 +815,50 @@ def compute_edge_scores(copy: fx.Graph) -> None:
         found = products_of(node)
         if found is not None and node.users and not any(_call(u, torch.stack) for u in node.users):
             replace(node, [(PRODUCTS, found)], None, False, None)
+    if written:
+        _drop_dead_nodes(copy, written)
+
+
+def normalise_columns(copy: fx.Graph) -> None:
+    """In a copy of a graph: q / s[column] with s = sum of q over columns, where q = e /
+    r[row], or an edge value itself, is used for nothing else; and the gather that e comes
+    from, if only this reads it  => one _normalised."""
+    from ..ops.fused_op import _normalised
+    written = []
+    for out in list(copy.nodes):
+        last = _sddmm_of(out) if out.users else None
+        if last is None or last[1] != "div" or last[4] != [1, 2]:
+            continue
+        g, q, s = last[0], last[2], last[3]
+        if not (isinstance(q, fx.Node) and _is_wrapped(s, "_after_spmm") and len(s.users) == 1
+                and _call(s.args[0], operator.getitem) and s.args[0].args[1] == 0
+                and _is_wrapped(s.args[0].args[0], "_before_spmm")):
+            continue
+        total, before_total = s.args[0], s.args[0].args[0]
+        sums = [n for n in total.users if _is_method(n, "_CAPI_SpMM")]
+        before_last = next(iter(s.users))
+        if len(sums) != 1 or set(total.users) != {sums[0], s} or not _is_wrapped(before_last, "_before_sddmm"):
+            continue
+        spmm = sums[0]
+        if not (spmm.args[0] is g and spmm.args[1] == "copy_rhs" and spmm.args[2] == "sum"
+                and spmm.args[4] is q and spmm.args[8] == 0 and before_total.args[5] is q):
+            continue
+        readers = {spmm, before_total, before_last}
+        first = _sddmm_of(q)
+        values, divisor, formats = q, None, (last[5], spmm.args[9], last[5])
+        if (first is not None and first[1] == "div" and first[4] == [1, 0] and first[0] is g
+                and set(q.users) == readers and isinstance(first[2], fx.Node)):
+            values, divisor, formats = first[2], first[3], (first[5], spmm.args[9], last[5])
+            readers = {n.args[0] for n in first[6].all_input_nodes if _call(n, operator.getitem)
+                       and _is_wrapped(n.args[0], "_before_sddmm")}
+            written.append(first[6])
+        select = None
+        if _is_wrapped(values, "data_index") and set(values.users) == readers:
+            values, select = values.args
+        with copy.inserting_before(out):
+            new = copy.call_function(_normalised, args=(g, values, select, divisor, formats))
+        out.replace_all_uses_with(new)
+        written += [spmm, last[6]]
     if written:
         _drop_dead_nodes(copy, written)
 

@@ -66,6 +66,29 @@ def _edge_score(g, kinds, lhs, rhs, targets, weights, positive_part, shift, on_f
     return out if shift is None else out + shift * torch.ones_like(out)
 
 
+def _normalised(g, values, select, divisor, formats):
+    """values[select] / divisor[row] (either may be None), divided by its sums over columns: the
+    end of a LADIES layer, by two passes over the edges where the operators take four or five."""
+    from ..matrix_api.matrix import data_index
+    if all(t is None or type(t) is torch.Tensor for t in (values, select, divisor)):
+        out = g._CAPI_NormaliseColumns(values, select, divisor)
+        if out is not None:
+            return out
+
+    def divided(e, by, target, on_format):
+        left, right, out, squeeze = _before_sddmm(g._CAPI_GetNumEdges(), "div", e, by)
+        g._CAPI_SDDMM("div", left, right, out, 1, target, on_format)
+        return _after_sddmm(out, squeeze)
+
+    e = values if select is None else data_index(values, select)
+    if divisor is not None:
+        e = divided(e, divisor, 0, formats[0])
+    sums, arg_u, arg_e, squeeze = _before_spmm(g._CAPI_GetNumRows(), g._CAPI_GetNumCols(), "copy_rhs",
+                                               "sum", None, e, 0)
+    g._CAPI_SpMM("copy_rhs", "sum", None, e, sums, arg_u, arg_e, 0, formats[1])
+    return divided(e, _after_spmm(sums, squeeze), 2, formats[2])
+
+
 def _encoded_square_sums(g, seeds, seeds_ptr, values, on_format):
     """What a compiled super-batched sampler asks an encoded column slice for: (the slice for
     _encoded_row_slice, its rows, where every batch's begin, sums of the squared values on

@@ -813,6 +813,10 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
  *   sum over a feature of 1 to 63 products lhs[t_l, i] * rhs[t_r, i]; all of the last
  *   kind have one length.  Products and quotients are rounded before they are added;
  *   the order of additions is fixed (edgeops.hip).
+ * gs_normalise_columns: out[e] = q[e] / (sum of q over e's column) with q[e] =
+ *   values[select[e]] / row_divisor[rows[e]], select (identity) and row_divisor (ones)
+ *   nullable, fp32; edges in column order, sums[num_cols] is scratch that ends up with
+ *   the columns' sums.  q is rounded, sums are of 64 bits and rounded before they divide.
  * gs_spmm: out[dst] = reduce(out[dst], op(u[src], e[eid])), fp32.  Outputs
  *   are accumulators: the caller zero-fills them (python/gs/ops/spmm.py:56).
  *   COO: u_target 0 reduces onto columns, 2 onto rows (atomics).  Compressed:
@@ -845,6 +849,10 @@ int gs_edge_score(int format, const int64_t* a, const int64_t* b, int64_t num_ma
                   int64_t nnz, const int64_t* edge_map, const gs_score_term* terms,
                   int num_terms, int64_t feature_len, const float* weights, int positive_part,
                   float shift, float* out, gs_stream_t stream);
+int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t* rows,
+                         int64_t nnz, const float* values, const int64_t* select,
+                         const float* row_divisor, double* sums, float* out,
+                         gs_stream_t stream);
 int gs_fused_u_op_v(int format, const int64_t* a, const int64_t* b,
                     int64_t num_major, int64_t nnz, const int64_t* edge_map,
                     int op, int dtype,

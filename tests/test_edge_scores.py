@@ -223,3 +223,99 @@ def test_what_is_summed_in_place(options, kernel):
     t = ran(gs.jit.compile(func=sampler, args=(bm, torch.arange(6), torch.tensor([0, 3, 6]))))
     assert t.count(fused_op._encoded_square_sums) == kernel and ("_CAPI_BatchColSlicing" in t) != kernel
     assert t.count(fused_op._encoded_row_slice) == kernel and ("_CAPI_BatchRowSlicing" in t) != kernel
+
+
+# ------------------------------------------------------------ columns normalised
+def normalised(A, seeds, divisor):
+    sub = A[:, seeds].div("w", divisor, axis=1)
+    return sub.div("w", sub.sum("w", axis=0), axis=0).edata["w"]
+
+
+def by_columns_only(A, seeds, divisor):
+    sub = A[:, seeds]
+    return sub.div("w", sub.sum("w", axis=0), axis=0).edata["w"], sub.edata["w"]
+
+
+def quotient_kept(A, seeds, divisor):
+    q = A[:, seeds].div("w", divisor, axis=1)
+    return q.div("w", q.sum("w", axis=0), axis=0).edata["w"], q.edata["w"]
+
+
+def sums_kept(A, seeds, divisor):
+    q = A[:, seeds].div("w", divisor, axis=1)
+    s = q.sum("w", axis=0)
+    return q.div("w", s, axis=0).edata["w"], s
+
+
+def by_rows(A, seeds, divisor):
+    q = A[:, seeds].div("w", divisor, axis=1)
+    return q.div("w", q.sum("w", axis=1), axis=1).edata["w"]
+
+
+@pytest.mark.parametrize("func,kernels,divisions", [
+    (normalised, 1, 0), (by_columns_only, 1, 0), (quotient_kept, 1, 1), (sums_kept, 0, 2), (by_rows, 0, 2)])
+def test_what_is_normalised_in_one(func, kernels, divisions):
+    m = gs.Matrix(gs.Graph(10, 10))
+    m.edata["w"] = torch.rand(7)
+    t = ran(gs.jit.compile(func=func, args=(m, torch.arange(3), torch.rand(10))))
+    assert t.count(fused_op._normalised) == kernels and t.count("_CAPI_SDDMM") == divisions
+    assert t.count("_CAPI_SpMM") == (kernels == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("func", [normalised, by_columns_only, quotient_kept, sums_kept, by_rows])
+@pytest.mark.parametrize("kind", ["float32", "float64", "gradients", "edge list"])
+def test_normalised_columns_equal_eager(func, kind):
+    m, seeds = world(), torch.arange(0, 900, 3, device=DEV)
+    if kind == "edge list":
+        row, col = m.coo[:2]
+        order = torch.randperm(row.numel(), device=DEV)
+        w = m.edata["w"]
+        m = gs.Matrix()
+        m.load_graph("COO", [row[order], col[order]])
+        m.edata["w"] = w[order]
+    divisor = torch.rand(m.num_rows(), device=DEV) + 0.5
+    if kind == "gradients":
+        m.edata["w"].requires_grad_()
+        divisor.requires_grad_()
+    if kind == "float64":
+        m.edata["w"], divisor = m.edata["w"].double(), divisor.double()
+        with pytest.raises(RuntimeError):
+            func(m, seeds, divisor)
+        c = gs.jit.compile(func=func, args=(m, seeds, divisor))
+        with pytest.raises(RuntimeError):
+            c(m, seeds, divisor)
+        return
+    want = func(m, seeds, divisor)
+    got = gs.jit.compile(func=func, args=(m, seeds, divisor))(m, seeds, divisor)
+    for a, b in zip(*((x if isinstance(x, tuple) else (x,)) for x in (want, got))):
+        # the eager sums are of 32 bits, up to 4000 terms of one sign in any order
+        assert a.requires_grad == b.requires_grad
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("degrees", [[1], [2048], [2049], [2047, 1, 2048, 0, 5], [0] * 3000 + [10] + [0] * 2500 + [7],
+                                     [3] * 5000, [1] * 2048 + [4100] + [0, 1] * 40, [100_000, 1]])
+@pytest.mark.parametrize("select", [False, True])
+@pytest.mark.parametrize("divide", [False, True])
+def test_normalised_columns_against_64_bits(degrees, select, divide):
+    """Tiles of one column and of thousands, columns of no edge between, over borders of tiles."""
+    g = torch.Generator(device=DEV).manual_seed(len(degrees))
+    deg = torch.tensor(degrees, device=DEV)
+    indptr = torch.zeros(deg.numel() + 1, dtype=torch.int64, device=DEV)
+    torch.cumsum(deg, 0, out=indptr[1:])
+    n = int(indptr[-1])
+    rows = torch.randint(0, 500, (n,), generator=g, device=DEV)
+    graph = gs.Graph(500, deg.numel())
+    graph._CAPI_LoadCSC(indptr, rows)
+    values = torch.randn(n + 100, generator=g, device=DEV).abs()[: n + 100 * select].contiguous() + 0.01
+    index = torch.randint(0, n + 100, (n,), generator=g, device=DEV) if select else None
+    by = torch.rand(500, generator=g, device=DEV) + 0.1 if divide else None
+    got = fused_op._normalised(graph, values, index, by, (gs._COO, gs._CSC, gs._COO))
+    q = values[index] if select else values
+    q = (q / by[rows] if divide else q).double()
+    column = torch.repeat_interleave(torch.arange(deg.numel(), device=DEV), deg)
+    sums = torch.zeros(deg.numel(), dtype=torch.float64, device=DEV).index_add_(0, column, q)
+    # the sum and the quotient are rounded once each
+    torch.testing.assert_close(got.double(), q / sums[column], rtol=2.5 * 2.0 ** -24, atol=0)
