@@ -945,22 +945,30 @@ __global__ __launch_bounds__(kBlock) void table_fill_kernel32(uint32_t* __restri
 // ---------------------------------------------- the K smallest keys by selection
 // Without replacement the pick is "the K smallest keys, in ascending order, ties
 // to the smaller index".  Sorting all n keys for that costs sixteen launches of
-// a radix sort; for K up to kSelMaxPicks the kernels below select instead:
-//   keys     key of every item (kept), histogram of its top 12 bits (the
-//            exponent of a non-negative double) per segment
-//   refine   the bin that holds the K-th smallest key follows from that
-//            histogram (every work-group scans it for itself: 4096 bins); items
-//            of that bin are counted by their next 12 bits
-//   emit     the same again one level down; items below the K-th item's
-//            (bin, sub-bin) cell are certain picks and go to the segment's pick
-//            list, items inside the cell to its candidate list
-//   finish   picks + the smallest candidates of a segment are ordered by
-//            (key, index) in LDS and written out (sixteen work-groups per
-//            segment share the comparisons)
-// The cell of the K-th item holds a handful of items unless keys repeat (items
-// of weight zero all have the key +inf); a cell too large for LDS is narrowed
-// by a byte-wise radix selection over its remaining key bits and indices first.
-constexpr int kSelBins = 4096;
+// a radix sort, and making them all is most of what is left: a key is two divisions
+// and a logarithm of correctly rounded double operations, some hundred instructions.
+// For K up to kSelMaxPicks the kernels below select by a cheap 32-bit key first:
+//   bounds   an approximate key of every item (kept), off by less than kSelMargin of
+//            itself, histogram of its exponent and 1 or 3 bits of its fraction per
+//            segment
+//   emit     the bin that holds the K-th smallest approximate key follows from that
+//            histogram (every work-group scans it for itself); K items lie below the
+//            bin's end, so no key above that end and the margin is among the K
+//            smallest.  The others are the candidates, whose keys are computed and
+//            appended to the segment's list
+//   finish   a segment's candidates are ordered by (key, index) in LDS and the first K
+//            written out (sixteen work-groups per segment share the comparisons)
+// The number of keys below x grows no faster than x, so the candidates are about K times
+// the width of a bin, 1.5 or 1.125, unless keys repeat; a list too long for LDS is
+// narrowed by a byte-wise radix selection over keys and indices first.  Items of weight
+// zero all have the key +inf: where picks come to them, a work-group leaves its own out
+// if enough of them lie before it (100 K items, 300 of them positive, 400 picks: 710 us
+// without that).
+// 2.45 M items, 400 picks, us: keys 25, two levels of histograms 10 and 11 and finish 7
+// when all keys were made; now bounds 18, emit 6, finish 8.  Bounds takes 22 with bins of
+// an eighth and 28 with half as many items a work-group: every work-group adds its bins
+// to the same words in memory.
+constexpr int kSelBins = 2048;
 constexpr int kSelTile = 4096;  // shortest average segment the selection takes on
 constexpr int64_t kSelMaxPicks = 2048;
 constexpr int kFinishThreads = 1024;
@@ -971,9 +979,47 @@ __host__ __device__ inline bool list_can_select(int64_t n, int64_t nseg) {
   return n < (int64_t(1) << 31) && (nseg == 1 || n / nseg >= kSelTile);
 }
 
-__device__ __forceinline__ uint32_t sel_digit1(uint64_t k) { return (uint32_t)(k >> 52); }
-__device__ __forceinline__ uint32_t sel_digit2(uint64_t k) {
-  return (uint32_t)(k >> 40) & (kSelBins - 1);
+// Approximate keys.  Weights outside [2^-100, 2^100] go by their exact key, so that no
+// intermediate overflows or loses bits; a result below 2^-126 may be flushed to 0, which
+// is why no bound lies below kSelLeast.
+constexpr float kSelMargin = 0x1p-10f;  // (2^-20.4 is the most met in 3 10^8 draws)
+constexpr float kSelLeast = 0x1p-120f;
+
+// -log2 of neg_log2_unit's argument, in 32 bits.
+__device__ __forceinline__ float neg_log2_unit_approx(uint64_t r64) {
+  const uint64_t v = (r64 >> 12) + 1;  // u = v / 2^52
+  if (v >> 51) {                       // u >= 1/2: from 1 - u, which keeps its bits
+    const uint64_t c = (1ull << 52) - v;
+    const float t = fmaf((float)(uint32_t)(c >> 32), 0x1p-20f, (float)(uint32_t)c * 0x1p-52f);
+    if (t < 0x1p-4f) {
+      const float series =
+          fmaf(t, fmaf(t, fmaf(t, fmaf(t, 0.2f, 0.25f), 0.33333334f), 0.5f), 1.0f);
+      return 1.4426950f * t * series;
+    }
+    return -__builtin_amdgcn_logf(1.0f - t);
+  }
+  const float u = fmaf((float)(uint32_t)(v >> 32), 0x1p-20f, (float)(uint32_t)v * 0x1p-52f);
+  return -__builtin_amdgcn_logf(u);
+}
+
+__device__ __forceinline__ float weighted_key_approx(PhiloxKey key, uint64_t pos, float w) {
+  if (!(w > 0.0f)) return __uint_as_float(0x7f800000u);  // +inf
+  if (!(w >= 0x1p-100f && w <= 0x1p100f)) {
+    const double k = weighted_key(key, pos, 0, w);
+    // (what is no number from 0 to +inf is ordered behind them by its bits)
+    return k >= 0.0 && !(__double_as_longlong(k) < 0) ? (float)k : __uint_as_float(0x7f800000u);
+  }
+  const Words4 wd = philox(key, pos, 0);
+  return neg_log2_unit_approx(((uint64_t)wd.y << 32) | wd.x) * __builtin_amdgcn_rcpf(w);
+}
+
+__device__ __forceinline__ uint32_t sel_bin(float k, int shift) {
+  return __float_as_uint(k) >> shift;
+}
+// Keys above this are not among as many smallest as lie in the bins up to `bin`.
+__device__ __forceinline__ float sel_bound(uint32_t bin, int shift) {
+  const float end = __uint_as_float(bin + 1 < 0x7f800000u >> shift ? (bin + 1) << shift : 0x7f800000u);
+  return fmaxf(end, kSelLeast) * (1.0f + 4.0f * kSelMargin);
 }
 
 // The bin of a kSelBins-bin histogram that holds the want-th smallest item
@@ -1022,141 +1068,125 @@ __device__ __forceinline__ SegmentSpan sel_span(const int64_t* __restrict__ rang
 }
 
 template <int kSelItems>
-__global__ __launch_bounds__(kBlock) void list_keys_hist_kernel(
+__global__ __launch_bounds__(kBlock) void list_bounds_kernel(
     const float* __restrict__ probs, const int64_t* __restrict__ range, int64_t n,
-    int64_t nseg, PhiloxKey key, uint64_t* __restrict__ keys, uint32_t* hist1) {
+    int64_t nseg, PhiloxKey key, int shift, float* __restrict__ keys, uint32_t* hist,
+    uint32_t* __restrict__ tile_never) {
   __shared__ uint32_t lh[kSelBins];
+  __shared__ uint32_t never;
   const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kSelItems);
   const int64_t i_last = i0 + (kBlock * kSelItems) - 1 < n ? i0 + (kBlock * kSelItems) - 1 : n - 1;
   const SegmentSpan span = sel_span(range, nseg, i0, i_last);
-  for (int b = threadIdx.x; b < kSelBins; b += kBlock) lh[b] = 0;
-  __syncthreads();
-#pragma unroll 4
+  // all loads first, or each would be waited for inside its own branch
+  float w[kSelItems];
+#pragma unroll
   for (int j = 0; j < kSelItems; ++j) {
     const int64_t i = i0 + j * kBlock + threadIdx.x;
-    if (i >= n) break;
-    // non-negative doubles (and +inf) order like their bit patterns
-    const uint64_t k =
-        (uint64_t)__double_as_longlong(weighted_key(key, (uint64_t)i, 0, probs[i]));
+    w[j] = probs[i <= i_last ? i : i_last];
+  }
+  const int bins = (int)(0x80000000u >> shift);
+  for (int b = threadIdx.x; b < bins; b += kBlock) lh[b] = 0;
+  if (threadIdx.x == 0) never = 0;
+  __syncthreads();
+  uint32_t mine = 0;
+#pragma unroll
+  for (int j = 0; j < kSelItems; ++j)
+    mine += (uint32_t)__popcll(__ballot(!(w[j] > 0.0f) && i0 + j * kBlock + threadIdx.x <= i_last));
+  if (mine && lane_id() == 0) atomicAdd(&never, mine);
+#pragma unroll
+  for (int j = 0; j < kSelItems; ++j) {
+    const int64_t i = i0 + j * kBlock + threadIdx.x;
+    if (i > i_last) break;
+    // non-negative floats (and +inf) order like their bit patterns
+    const float k = weighted_key_approx(key, (uint64_t)i, w[j]);
     keys[i] = k;
     const int64_t seg = span.segment_at(range, i);
     if (seg == span.lo)
-      atomicAdd(&lh[sel_digit1(k)], 1u);
+      atomicAdd(&lh[sel_bin(k, shift)], 1u);
     else
-      atomicAdd(&hist1[seg * kSelBins + sel_digit1(k)], 1u);
+      atomicAdd(&hist[seg * kSelBins + sel_bin(k, shift)], 1u);
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < kSelBins; b += kBlock)
-    if (lh[b]) atomicAdd(&hist1[span.lo * kSelBins + b], lh[b]);
-}
-
-template <int kSelItems>
-__global__ __launch_bounds__(kBlock) void list_refine_kernel(
-    const int64_t* __restrict__ range, int64_t n, int64_t nseg, int64_t num_picks,
-    const uint64_t* __restrict__ keys, const uint32_t* __restrict__ hist1, uint32_t* hist2) {
-  __shared__ uint32_t lh[kSelBins];
-  __shared__ uint32_t smem[kBlock / kWave + 1];
-  __shared__ uint32_t found[2];
-  const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kSelItems);
-  const int64_t i_last = i0 + (kBlock * kSelItems) - 1 < n ? i0 + (kBlock * kSelItems) - 1 : n - 1;
-  const SegmentSpan span = sel_span(range, nseg, i0, i_last);
-  for (int64_t seg = span.lo; seg <= span.hi; ++seg) {  // the same in every thread
-    const SelSegment sg = sel_segment(range, n, seg);
-    if (sg.hi - sg.lo <= num_picks) continue;  // taken whole
-    uint32_t b1, below1;
-    find_bin(hist1 + seg * kSelBins, (uint32_t)num_picks, smem, found, &b1, &below1);
-    for (int b = threadIdx.x; b < kSelBins; b += kBlock) lh[b] = 0;
-    __syncthreads();
-#pragma unroll 4
-    for (int j = 0; j < kSelItems; ++j) {
-      const int64_t i = i0 + j * kBlock + threadIdx.x;
-      if (i >= sg.lo && i < sg.hi && i <= i_last) {
-        const uint64_t k = keys[i];
-        if (sel_digit1(k) == b1) atomicAdd(&lh[sel_digit2(k)], 1u);
-      }
-    }
-    __syncthreads();
-    for (int b = threadIdx.x; b < kSelBins; b += kBlock)
-      if (lh[b]) atomicAdd(&hist2[seg * kSelBins + b], lh[b]);
-    __syncthreads();
-  }
+  if (threadIdx.x == 0) tile_never[blockIdx.x] = never;
+  for (int b = threadIdx.x; b < bins; b += kBlock)
+    if (lh[b]) atomicAdd(&hist[span.lo * kSelBins + b], lh[b]);
 }
 
 template <int kSelItems>
 __global__ __launch_bounds__(kBlock) void list_emit_kernel(
-    const int64_t* __restrict__ range, int64_t n, int64_t nseg, int64_t num_picks,
-    const uint64_t* __restrict__ keys, const uint32_t* __restrict__ hist1,
-    const uint32_t* __restrict__ hist2, uint32_t* counts, uint64_t* __restrict__ win_key,
-    int64_t* __restrict__ win_idx, uint64_t* __restrict__ cand_key,
-    int64_t* __restrict__ cand_idx) {
+    const float* __restrict__ probs, const int64_t* __restrict__ range, int64_t n, int64_t nseg,
+    int64_t num_picks, PhiloxKey key, int shift, const float* __restrict__ keys,
+    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ tile_never, uint32_t* counts,
+    uint64_t* __restrict__ cand_key, int64_t* __restrict__ cand_idx) {
   __shared__ uint32_t smem[kBlock / kWave + 1];
   __shared__ uint32_t found[2];
-  __shared__ uint32_t bases[2];
+  __shared__ uint32_t base;
   const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kSelItems);
   const int64_t i_last = i0 + (kBlock * kSelItems) - 1 < n ? i0 + (kBlock * kSelItems) - 1 : n - 1;
+  // (loaded before the histogram is looked at, so that both travel together)
+  float k[kSelItems];
+#pragma unroll
+  for (int j = 0; j < kSelItems; ++j) {
+    const int64_t i = i0 + j * kBlock + threadIdx.x;
+    k[j] = keys[i <= i_last ? i : i_last];
+  }
   const SegmentSpan span = sel_span(range, nseg, i0, i_last);
   for (int64_t seg = span.lo; seg <= span.hi; ++seg) {  // the same in every thread
     const SelSegment sg = sel_segment(range, n, seg);
-    if (sg.hi - sg.lo <= num_picks) continue;
-    uint32_t b1, below1, b2, below2;
-    find_bin(hist1 + seg * kSelBins, (uint32_t)num_picks, smem, found, &b1, &below1);
-    find_bin(hist2 + seg * kSelBins, (uint32_t)num_picks - below1, smem, found, &b2, &below2);
-    uint64_t k[kSelItems];
-    uint32_t is_win = 0, is_cand = 0;  // one bit per item of this thread
+    if (sg.hi - sg.lo <= num_picks) continue;  // taken whole
+    uint32_t bin, below;
+    find_bin(hist + seg * kSelBins, (uint32_t)num_picks, smem, found, &bin, &below);
+    const float bound = sel_bound(bin, shift);
+    uint32_t is_cand = 0;  // one bit per item of this thread
 #pragma unroll
     for (int j = 0; j < kSelItems; ++j) {
       const int64_t i = i0 + j * kBlock + threadIdx.x;
-      k[j] = 0;
-      if (i >= sg.lo && i < sg.hi && i <= i_last) {
-        k[j] = keys[i];
-        const uint32_t d1 = sel_digit1(k[j]), d2 = sel_digit2(k[j]);
-        if (d1 < b1 || (d1 == b1 && d2 < b2))
-          is_win |= 1u << j;
-        else if (d1 == b1 && d2 == b2)
-          is_cand |= 1u << j;
-      }
+      if (i >= sg.lo && i < sg.hi && i <= i_last && k[j] <= bound) is_cand |= 1u << j;
     }
-    uint32_t wins, cands;
-    uint32_t w_at = block_exclusive_sum((uint32_t)__popc(is_win), smem, &wins);
-    uint32_t c_at = block_exclusive_sum((uint32_t)__popc(is_cand), smem, &cands);
-    if (threadIdx.x == 0) {
-      bases[0] = wins ? atomicAdd(&counts[2 * seg], wins) : 0u;
-      bases[1] = cands ? atomicAdd(&counts[2 * seg + 1], cands) : 0u;
+    if (bin == 0x7f800000u >> shift) {
+      // Fewer positive weights than picks: items of weight zero follow in the order of
+      // their indices.  Those of this tile do not if the tiles of the segment before it
+      // have enough of them.
+      constexpr int64_t kTile = kBlock * kSelItems;
+      uint32_t before = 0, all;
+      for (int64_t t = ceil_div_dev(sg.lo, kTile) + threadIdx.x; t < (int64_t)blockIdx.x; t += kBlock)
+        before += tile_never[t];
+      (void)block_exclusive_sum(before, smem, &all);
+      if (all >= (uint32_t)num_picks)
+        for (uint32_t left = is_cand; left; left &= left - 1) {
+          const int j = __ffs((int)left) - 1;
+          if (!(probs[i0 + j * kBlock + threadIdx.x] > 0.0f)) is_cand &= ~(1u << j);
+        }
     }
+    uint32_t cands;
+    uint32_t at = block_exclusive_sum((uint32_t)__popc(is_cand), smem, &cands);
+    if (threadIdx.x == 0) base = cands ? atomicAdd(&counts[seg], cands) : 0u;
     __syncthreads();
-    w_at += bases[0];
-    c_at += bases[1];
-#pragma unroll
-    for (int j = 0; j < kSelItems; ++j) {
+    at += base;
+    while (is_cand) {
+      const int j = __ffs((int)is_cand) - 1;
+      is_cand &= is_cand - 1;
       const int64_t i = i0 + j * kBlock + threadIdx.x;
-      if ((is_win >> j) & 1u) {
-        if (w_at < (uint32_t)kSelMaxPicks) {  // always: fewer than num_picks items lie below the cell
-          win_key[seg * kSelMaxPicks + w_at] = k[j];
-          win_idx[seg * kSelMaxPicks + w_at] = i;
-        }
-        ++w_at;
-      } else if ((is_cand >> j) & 1u) {
-        if ((int64_t)c_at < sg.hi - sg.lo) {
-          cand_key[sg.lo + c_at] = k[j];
-          cand_idx[sg.lo + c_at] = i;
-        }
-        ++c_at;
+      if ((int64_t)at < sg.hi - sg.lo) {  // always
+        // non-negative doubles (and +inf) order like their bit patterns
+        cand_key[sg.lo + at] =
+            (uint64_t)__double_as_longlong(weighted_key(key, (uint64_t)i, 0, probs[i]));
+        cand_idx[sg.lo + at] = i;
       }
+      ++at;
     }
     __syncthreads();
   }
 }
 
-// (key, index) as one number: the low 40 bits of the key (the upper 24 are the
-// same for all candidates of a cell) above the 32-bit index.
+// (key, index) as one number.
 __device__ __forceinline__ unsigned __int128 sel_composite(uint64_t k, int64_t i) {
-  return ((unsigned __int128)(k & ((1ull << 40) - 1)) << 32) | (unsigned __int128)(uint32_t)i;
+  return ((unsigned __int128)k << 32) | (unsigned __int128)(uint32_t)i;
 }
 
 __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
     const int64_t* __restrict__ range, int64_t n, int64_t num_picks,
-    const uint32_t* __restrict__ counts, const uint64_t* __restrict__ win_key,
-    const int64_t* __restrict__ win_idx, const uint64_t* __restrict__ cand_key,
+    const uint32_t* __restrict__ counts, const uint64_t* __restrict__ cand_key,
     const int64_t* __restrict__ cand_idx, const int64_t* __restrict__ out_range,
     int64_t* __restrict__ out_index) {
   __shared__ uint64_t sk[kFinishSlots];
@@ -1172,31 +1202,24 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
       for (int64_t k = threadIdx.x; k < nb; k += kFinishThreads) out_index[out0 + k] = sg.lo + k;
     return;
   }
-  // (fewer than num_picks picks lie below the cell and no list is longer than its
-  // segment; the bounds are restated here because LDS indices follow from them)
-  uint32_t W = counts[2 * seg], M = counts[2 * seg + 1];
-  if (W > (uint32_t)kSelMaxPicks) W = (uint32_t)kSelMaxPicks;
-  if (W > (uint32_t)num_picks) W = (uint32_t)num_picks;
+  // (no list is longer than its segment; restated here because indices follow from it)
+  uint32_t M = counts[seg];
   if ((int64_t)M > nb) M = (uint32_t)nb;
   const uint64_t* ck = cand_key + sg.lo;
   const int64_t* ci = cand_idx + sg.lo;
-  for (uint32_t t = threadIdx.x; t < W; t += kFinishThreads) {
-    sk[t] = win_key[seg * kSelMaxPicks + t];
-    si[t] = win_idx[seg * kSelMaxPicks + t];
-  }
-  uint32_t total = W + M;
+  uint32_t total = M;
   if (total <= (uint32_t)kFinishSlots) {
     for (uint32_t t = threadIdx.x; t < M; t += kFinishThreads) {
-      sk[W + t] = ck[t];
-      si[W + t] = ci[t];
+      sk[t] = ck[t];
+      si[t] = ci[t];
     }
   } else {
     // the `want` smallest of the M candidates: fix the composite of the last
     // of them byte by byte, most significant first
-    uint32_t want = (uint32_t)num_picks - W;
+    uint32_t want = (uint32_t)num_picks;
     unsigned __int128 fixed = 0;
-    for (int d = 0; d < 9; ++d) {
-      const int shift = 8 * (8 - d);
+    for (int d = 0; d < 12; ++d) {
+      const int shift = 8 * (11 - d);
       for (int b = threadIdx.x; b < 256; b += kFinishThreads) hist[b] = 0;
       __syncthreads();
       for (uint32_t t = threadIdx.x; t < M; t += kFinishThreads) {
@@ -1222,7 +1245,7 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
       const uint64_t k = ck[t];
       const int64_t i = ci[t];
       if (sel_composite(k, i) <= fixed) {
-        const uint32_t at = W + atomicAdd(&appended, 1u);
+        const uint32_t at = atomicAdd(&appended, 1u);
         if (at < (uint32_t)kFinishSlots) {
           sk[at] = k;
           si[at] = i;
@@ -1288,12 +1311,11 @@ struct ListWs {
   size_t sort_ws_bytes;
   void* scan_ws;
   size_t scan_ws_bytes;
-  // selection (list_can_select): histograms, then counters, in one block
+  // selection (list_can_select): histograms, then counters, in one block; the
+  // approximate keys lie in keys_in
   uint32_t* sel_block;
   size_t sel_words;
-  uint32_t *hist1, *hist2, *counts;
-  uint64_t* win_key;
-  int64_t* win_idx;
+  uint32_t *hist, *counts, *tile_never;
   size_t total;
 };
 
@@ -1321,13 +1343,11 @@ static ListWs carve_list(void* ws, int64_t n, int64_t nseg) {
   w.scan_ws_bytes = scan_workspace_bytes(nseg + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
   const size_t segs = list_can_select(n, nseg) ? (size_t)nseg : 0;
-  w.sel_words = segs * (2 * kSelBins + 2);
+  w.sel_words = segs * (kSelBins + 1);
   w.sel_block = c.take<uint32_t>(w.sel_words);
-  w.hist1 = w.sel_block;
-  w.hist2 = w.hist1 ? w.hist1 + segs * kSelBins : nullptr;
-  w.counts = w.hist2 ? w.hist2 + segs * kSelBins : nullptr;
-  w.win_key = c.take<uint64_t>(segs * (size_t)kSelMaxPicks);
-  w.win_idx = c.take<int64_t>(segs * (size_t)kSelMaxPicks);
+  w.hist = w.sel_block;
+  w.counts = w.hist ? w.hist + segs * kSelBins : nullptr;
+  w.tile_never = c.take<uint32_t>(segs ? m / (kBlock * 4) + 1 : 0);
   w.total = c.total();
   return w;
 }
@@ -1536,7 +1556,11 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
   if (num_picks >= 1 && num_picks <= kSelMaxPicks && list_can_select(n, num_segments)) {
     // few items per thread while that still fills the device, else sixteen (fewer
     // work-groups meet at the same histogram bins)
-    const bool deep = n >= (int64_t(1) << 21);
+    const bool deep = n >= (int64_t(1) << 20);
+    // bins half a power of two wide, an eighth where many picks make candidates dear
+    // (they are compared with one another): 233 K items 24 and 27 us with 400 picks, 69
+    // and 58 with 2048
+    const int shift = num_picks <= 512 ? 22 : 20;
     const dim3 tiles((unsigned)ceil_div(n, kBlock * (deep ? 16 : 4)));
     GS_LAUNCH("list_zero", s,
               table_fill_kernel32<<<dim3((unsigned)ceil_div((int64_t)w.sel_words, kBlock * 8)),
@@ -1545,16 +1569,14 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
   GS_LAUNCH(name, s,                                                                  \
             if (deep) kernel<16><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__);         \
             else kernel<4><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__))
-    GS_SEL_LAUNCH("list_keys", list_keys_hist_kernel, probs, range, n, num_segments, key,
-                  w.keys_in, w.hist1);
-    GS_SEL_LAUNCH("list_refine", list_refine_kernel, range, n, num_segments, num_picks,
-                  w.keys_in, w.hist1, w.hist2);
-    GS_SEL_LAUNCH("list_emit", list_emit_kernel, range, n, num_segments, num_picks, w.keys_in,
-                  w.hist1, w.hist2, w.counts, w.win_key, w.win_idx, w.keys_out, w.vals_out);
+    GS_SEL_LAUNCH("list_bounds", list_bounds_kernel, probs, range, n, num_segments, key, shift,
+                  (float*)w.keys_in, w.hist, w.tile_never);
+    GS_SEL_LAUNCH("list_emit", list_emit_kernel, probs, range, n, num_segments, num_picks, key, shift,
+                  (const float*)w.keys_in, w.hist, w.tile_never, w.counts, w.keys_out, w.vals_out);
 #undef GS_SEL_LAUNCH
     GS_LAUNCH("list_finish", s,
               list_finish_kernel<<<dim3((unsigned)num_segments, kFinishSplit), dim3(kFinishThreads), 0, s>>>(
-                  range, n, num_picks, w.counts, w.win_key, w.win_idx, w.keys_out, w.vals_out,
+                  range, n, num_picks, w.counts, w.keys_out, w.vals_out,
                   out_range, out_index));
     return GS_OK;
   }

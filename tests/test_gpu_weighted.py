@@ -241,6 +241,40 @@ def test_list_selection_cases(case):
              orc.list_sample_weighted(probs, k, call_id=2))
 
 
+@pytest.mark.parametrize("case", ["wide", "tiny", "huge", "denormal", "not_a_number", "one_size", "hardly_more"])
+@pytest.mark.parametrize("k", [1, 512, 513, 2048])
+def test_list_selection_by_approximate_keys(case, k):
+    """Weights over the whole range of a float: keys that overflow or vanish in 32 bits, weights
+    whose reciprocal does, bins that end at infinity; lists hardly longer than the picks."""
+    rng = np.random.default_rng(k + len(case))
+    n = k + 3 if case == "hardly_more" else 150_000
+    with np.errstate(over="ignore"):
+        probs = {"wide": np.exp2(rng.uniform(-149, 128, n)), "tiny": np.exp2(rng.uniform(-126, -96, n)),
+                 "huge": np.exp2(rng.uniform(96, 128, n)), "denormal": np.exp2(rng.uniform(-149, -120, n)),
+                 "not_a_number": np.exp2(rng.uniform(-40, 40, n)), "one_size": np.ones(n),
+                 "hardly_more": rng.lognormal(0, 20, n)}[case].astype(np.float32)
+    if case == "not_a_number":               # never picked, as weights of zero
+        probs[rng.random(n) < 0.01] = np.nan
+    if case == "hardly_more":
+        probs[::2] = 0.0
+    same(capi.list_sample_weighted(F(probs), k, call_id=6), orc.list_sample_weighted(probs, k, call_id=6))
+
+
+@pytest.mark.parametrize("k", [1, 300, 2048])
+@pytest.mark.parametrize("positive", [0, 1, 290, 5000])
+def test_batched_list_selection_that_comes_to_weights_of_zero(k, positive):
+    """Items of weight zero follow in the order of their indices: found by the counts of the
+    tiles before, whose borders are not the segments'."""
+    rng = np.random.default_rng(k + positive)
+    ranges = np.concatenate([[0], np.cumsum([5000, 61_003, 1023, 40_001, 2500])])
+    probs = np.zeros(ranges[-1], dtype=np.float32)
+    for lo, hi in zip(ranges, ranges[1:]):
+        probs[lo + rng.permutation(hi - lo)[:positive]] = 0.5
+    same(capi.list_sample_weighted(F(probs), k, range_=T(ranges), call_id=7),
+         orc.list_sample_weighted(probs, k, range_=ranges, call_id=7))
+    same(capi.list_sample_weighted(F(probs), k, call_id=7), orc.list_sample_weighted(probs, k, call_id=7))
+
+
 def test_batched_list_selection_parity():
     """Segments long enough for the selection path, ragged, one of them empty, one taken
     whole, one with fewer positive weights than picks."""
