@@ -328,6 +328,7 @@ struct SliceView {
     int64_t shift[2], offset[2];
     int count;                // columns held by the lanes (0: none are)
     int32_t lane_start;       // this lane's column: first edge, relative to `first`, not below 0
+    bool lane_owns;           // whether it holds a column, and that has edges
     int64_t lane_shift, lane_offset;
     // At most two neighbouring columns.  Callers branch on this once per run,
     // around their whole loop over the run's edges, not per edge: a branch
@@ -360,6 +361,7 @@ struct SliceView {
     r.shift[0] = r.shift[1] = r.offset[0] = r.offset[1] = 0;
     r.count = 0;
     r.lane_start = 0;
+    r.lane_owns = false;
     r.lane_shift = r.lane_offset = 0;
     if (r.near()) {
       r.shift[0] = indptr[cols[r.span.lo]] - sub_indptr[r.span.lo];
@@ -375,10 +377,33 @@ struct SliceView {
       const int64_t start = sub_indptr[c];
       r.lane_start = start > first_u ? (int32_t)(start - first_u) : 0;
       // (an id outside the matrix is an empty column: its pointer is not read)
-      r.lane_shift = sub_indptr[c + 1] > start ? indptr[cols[c]] - start : 0;
+      const bool edges = sub_indptr[c + 1] > start;
+      r.lane_owns = edges && lane_id() < r.count;
+      r.lane_shift = edges ? indptr[cols[c]] - start : 0;
       if (key_offset) r.lane_offset = key_offset[c];
     }
     return r;
+  }
+  // The same as `position` below for a row of 64 edges: v = row + lane, or an edge
+  // before that but not before `row` (lanes past the end).  A column that starts in the
+  // row marks its first edge, and an edge takes the last mark at or before its own: three
+  // shuffles one after the other where the search takes seven.
+  __device__ __forceinline__ int64_t row_position(const Run& r, int64_t row, int64_t v,
+                                                  int64_t* col, int64_t* offset) const {
+    if (r.count == 0) return position(r, v, col, offset);  // the same in every lane
+    const int32_t from = r.lane_start - (int32_t)(row - r.first);
+    // the column of the row's first edge: the last that starts at or before it
+    const int head = 63 - __clzll((long long)(__ballot(r.lane_owns && from <= 0) | 1ull));
+    const bool marks = r.lane_owns && from > 0 && from < kWave;
+    // (lane 0 is no column's mark: there a zero from every other lane; lanes that nothing
+    // was sent to read zero)
+    const int mark = __builtin_amdgcn_ds_permute(marks ? from * 4 : 0, marks ? lane_id() + 1 : 0);
+    const uint64_t below = __ballot(mark != 0) & ((2ull << (int)(v - row)) - 1ull);
+    const int marked = __shfl(mark, 63 - __clzll((long long)(below | 1ull)), kWave);
+    const int i = below ? marked - 1 : head;
+    *col = r.span.lo + i;
+    *offset = key_offset ? (int64_t)__shfl((long long)r.lane_offset, i, kWave) : 0;
+    return v + (int64_t)__shfl((long long)r.lane_shift, i, kWave);
   }
   // Position in the parent of edge v of a run that is not near(): *col = its
   // column position, *offset = what to add to its id.  Every lane of the

@@ -107,9 +107,9 @@ __device__ __forceinline__ void slice_keys(const SliceView& view, const SliceVie
   int64_t offset[kItems];
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
-    int64_t e = e0 + j * kWave + lane;
-    if (e >= nnz) e = nnz - 1;
-    place[j] = view.position(r, e, &column[j], &offset[j]);
+    const int64_t row = e0 + j * kWave < nnz ? e0 + j * kWave : nnz - 1;
+    const int64_t e = row + lane < nnz ? row + lane : nnz - 1;
+    place[j] = view.row_position(r, row, e, &column[j], &offset[j]);
   }
 #pragma unroll
   for (int j = 0; j < kItems; ++j) key[j] = (int64_t)ids[place[j]] + offset[j];

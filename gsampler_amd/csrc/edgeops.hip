@@ -824,7 +824,8 @@ __global__ __launch_bounds__(kBlock) void spmm_coo_sum_kernel(
     for (int i = 0; i < kSumItems; ++i) {
       const int64_t e = tile0 + i * kBlock + threadIdx.x;
       int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
-      const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
+      const int64_t row = wave_uniform_first(e) < nnz ? wave_uniform_first(e) : nnz - 1;
+      const int64_t p = view.row_position(vrun, row, e < nnz ? e : nnz - 1, &col, &offset);
       if (e < nnz) {
         dst[i] = dst_ids[p] + offset;
         val[i] = edge_value<float>(kind, op, ufeat ? ufeat + src_ids[p] : nullptr,
@@ -1020,7 +1021,8 @@ __global__ __launch_bounds__(kPartThreads, 6) void rowsum_part_kernel(
       for (int i = 0; i < kPartItems; ++i) {
         const int64_t e = first + i * kWave + lane;
         int64_t col, offset;  // (looked up by all lanes together, a lane past the end included)
-        const int64_t p = view.position(vrun, e < nnz ? e : nnz - 1, &col, &offset);
+        const int64_t row = first + i * kWave < nnz ? first + i * kWave : nnz - 1;
+        const int64_t p = view.row_position(vrun, row, e < nnz ? e : nnz - 1, &col, &offset);
         if (e < nnz) take(i, p, offset);
       }
     }

@@ -3,15 +3,14 @@
 // and relabel that id to its position in the set.
 //
 //   count: hash the picked ids (smallest position wins for repeated ids); a
-//          wave tests 256 consecutive edges as four coalesced rows whose
-//          ballots are the chunk's flag words and counts the kept ones; scan
-//          of the chunk counts; out_indptr[c] = kept edges before indptr[c].
-//          The count pass also leaves, per chunk, the new ids (positions in
-//          the picked set) of the chunk's kept edges in edge order, and their
-//          places in the chunk.
+//          wave tests a chunk of 256 consecutive edges as four coalesced rows, sends
+//          away by a filter in LDS what is not picked, looks the rest up, and leaves
+//          the new ids (positions in the picked set) of the chunk's kept edges in
+//          edge order, their places in the chunk, and their number; scan of the
+//          chunk counts; out_indptr[c] = kept edges before indptr[c].
 //   fill : a lane per kept edge, in output order; the new id and the place come
 //          from the chunk's staged run, so the fill pass reads neither the ids
-//          nor the table nor the flags again.
+//          nor the table again.
 //
 // A table slot is  low 32 bits of the id << 32 | position in the picked set.
 // While every picked id is below 2^32 - 1 those bits are the id, and an edge
@@ -25,7 +24,7 @@
 
 namespace gs {
 
-constexpr int kMemberWords = kBlock / kWave;  // flag words per chunk of kBlock edges
+constexpr int kMemberWords = kBlock / kWave;  // rows of 64 edges per chunk of kBlock edges
 // Chunks one wave takes at a time.  A long run shares the look-up of its columns
 // among more edges; on a short edge list it leaves the machine idle while few waves
 // walk through their chains of dependent loads: one chunk while even that makes no
@@ -38,15 +37,15 @@ constexpr int64_t kMemberShortChunks = 4096;
 // with four; a row slice of 602 M: 3.34 ms with two, 3.10 with four).
 constexpr int kMemberHugeRun = 4;
 constexpr int64_t kMemberHugeChunks = int64_t(1) << 18;
-constexpr int kMemberThreads = 1024;  // 16 waves share one staged table: 32 Ki edges per 32 KB copied
+constexpr int kMemberThreads = 1024;  // 16 waves share one staged table
 // Two of the large work-groups share a compute unit, which takes at most 64 registers
-// a lane.  Runs of eight chunks, look-ups of four in flight, and the look-ups of
-// scattered runs unrolled took 90 to 128 registers, one work-group was resident, and
-// a launch of 590 or 890 work-groups left its second round half empty: 136 us on 29 M
-// edges of 512 columns and 110 on 19 M (tables in LDS), 126 on 18.5 M (behind the
-// filter).  Two chunks a run, as many work-groups as are resident: 90, 66 and 78.
+// a lane.  Runs of eight chunks with a look-up for every row took 90 to 128 registers,
+// one work-group was resident, and a launch of 590 or 890 work-groups left its second
+// round half empty: 136 us on 29 M edges of 512 columns and 110 on 19 M.  Two chunks a
+// run, as many work-groups as are resident: 90 and 66 (and four chunks a run 64 and 45
+// where two now take 64 and 43).
 constexpr int kMemberWavesPerSimd = 8;
-constexpr int kMemberLdsSlots = 4096;  // tables up to this size are staged in LDS (32 KB)
+constexpr int kMemberLdsSlots = 4096;  // tables up to this size are staged in LDS (24 KB)
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 
 // A table too large for LDS is looked up in L2, one request per probe, and the
@@ -55,22 +54,39 @@ constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups o
 // them away first: a word of 32 bits per id group, three bits per picked id
 // (a blocked Bloom filter; with up to eight ids per word about one absent id in
 // twenty passes).  Only ids that pass go on to the table.
-constexpr int kFilterWords = 16384;            // 64 KB of LDS
-constexpr int kFilterGroupsPerCu = 2;          // work-groups of 1024 threads that fit a compute unit
-constexpr int64_t kFilterMaxIds = 8 * kFilterWords;  // beyond: too many bits set to be worth a look
+constexpr int kFilterWords = 14336;            // 56 KB of LDS, two work-groups a compute unit
+constexpr int kFilterBits = 3;
+constexpr int kResidentPerCu = 2;              // work-groups of 1024 threads that fit a compute unit
+constexpr int64_t kFilterMaxIds = 131072;      // beyond: too many bits set to be worth a look
 
-__device__ __forceinline__ uint32_t filter_word(uint32_t key) {
-  return (key * 0x9E3779B1u) >> 18;  // top 14 bits: [0, kFilterWords)
-}
-__device__ __forceinline__ uint32_t filter_bits(uint32_t key) {
-  const uint32_t h = key * 0x85EBCA6Bu;
-  return (1u << (h >> 27)) | (1u << ((h >> 22) & 31u)) | (1u << ((h >> 17) & 31u));
-}
-static_assert(kFilterWords == 1 << 14, "filter_word keeps 14 bits");
+// Ids that may be picked, by a word of 32 bits per id group in LDS: an id whose bits
+// are not all set is not picked.  One multiplication serves the word and the bits.
+template <int kWords, int kBits>
+struct IdFilter {
+  __device__ __forceinline__ static uint32_t hash(uint32_t key) { return key * 0x9E3779B1u; }
+  __device__ __forceinline__ static uint32_t word(uint32_t h) {
+    return (kWords & (kWords - 1)) == 0 ? h >> (32 - __builtin_ctz(kWords))
+                                        : __umulhi(h, (uint32_t)kWords);
+  }
+  // (shifts go by the low five bits of their count)
+  __device__ __forceinline__ static uint32_t bits(uint32_t h) {
+    uint32_t b = 0;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) b |= 1u << ((h >> (13 - 5 * i)) & 31u);
+    return b;
+  }
+  __device__ __forceinline__ static bool passes(const uint32_t* words, uint32_t key) {
+    const uint32_t h = hash(key), w = words[word(h)];
+    uint32_t all = 1u;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) all &= w >> ((h >> (13 - 5 * i)) & 31u);
+    return all != 0u;
+  }
+};
+using L2Filter = IdFilter<kFilterWords, kFilterBits>;
 
 struct MemberWs {
   uint64_t* table;     // [member_table_slots(num_picked)]
-  uint64_t* flags;     // [chunks * kMemberWords]
   uint32_t* staged;    // [chunks * kBlock]: per chunk, the new ids of its kept edges, in order
   uint8_t* staged_pos;  // [chunks * kBlock]: and their places in the chunk
   int64_t* chunk_off;  // [chunks + 1]
@@ -98,7 +114,6 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
   MemberWs w;
   w.chunks = ceil_div(nnz > 0 ? nnz : 1, kBlock);
   w.table = c.take<uint64_t>((size_t)member_table_slots(num_picked));
-  w.flags = c.take<uint64_t>((size_t)w.chunks * kMemberWords);
   w.staged = c.take<uint32_t>((size_t)w.chunks * kBlock);
   w.staged_pos = c.take<uint8_t>((size_t)w.chunks * kBlock);
   w.chunk_off = c.take<int64_t>((size_t)w.chunks + 1);
@@ -139,7 +154,10 @@ __device__ __forceinline__ void member_insert_one(const int64_t* __restrict__ pi
   const uint64_t id = (uint64_t)picked[i];
   if (id > kMaxPackedKey) *wide = 1;  // every writer stores the same value
   const uint32_t key = member_tag(id);
-  if (filter) atomicOr(filter + filter_word(key), filter_bits(key));
+  if (filter) {
+    const uint32_t h = L2Filter::hash(key);
+    atomicOr(filter + L2Filter::word(h), L2Filter::bits(h));
+  }
   const uint64_t mine = ((uint64_t)key << 32) | (uint64_t)i;
   uint32_t slot = member_home(key, cap);
   for (uint32_t probes = 0; probes < cap; ++probes) {  // the table has free slots: ends early
@@ -193,62 +211,44 @@ __global__ __launch_bounds__(kBlock) void member_clear_kernel(uint64_t* table, i
   for (; i < n; i += stride) table[i] = kEmptySlot;
 }
 
-// A small table (the picked set of a layer-wise sampler is a few hundred ids)
-// is copied into LDS once per work-group, keys and positions apart: 64 lanes
-// probing 64 different slots cost the vector cache a tag look-up each, the LDS
-// a few cycles in all.
-template <bool kInLds, bool kWithValues>
 struct MemberTable {
   const uint64_t* slots;
-  const uint32_t* keys;
-  const uint32_t* values;
   uint32_t cap;
 
-  __device__ __forceinline__ void stage(const uint64_t* __restrict__ table, uint32_t capacity,
-                                        uint32_t* lds_keys, uint32_t* lds_values) {
-    slots = table;
-    keys = lds_keys;
-    values = lds_values;
-    cap = capacity;
-    if (!kInLds) return;
-    for (uint32_t i = threadIdx.x; i < capacity; i += blockDim.x) {
-      const uint64_t t = table[i];
-      lds_keys[i] = (uint32_t)(t >> 32);
-      if (kWithValues) lds_values[i] = (uint32_t)t;
-    }
-    __syncthreads();
-  }
   __device__ __forceinline__ uint32_t key_at(uint32_t slot) const {
-    return kInLds ? keys[slot] : (uint32_t)(slots[slot] >> 32);
+    return (uint32_t)(slots[slot] >> 32);
   }
   __device__ __forceinline__ uint32_t value_at(uint32_t slot) const {
-    return kInLds ? values[slot] : (uint32_t)slots[slot];
+    return (uint32_t)slots[slot];
   }
 
   // N look-ups in step: the probes of a round are issued together, so a lane
   // waits for the longest of its N probe runs instead of their sum.  slot[j]
-  // is where key[j] sits, cap when it is absent (or kNoKey).
+  // is where key[j] sits, cap when it is absent (or kNoKey); value[j] is its position.
   template <int N>
-  __device__ __forceinline__ void find_many(const uint32_t (&key)[N], uint32_t (&slot)[N]) const {
+  __device__ __forceinline__ void find_many(const uint32_t (&key)[N], uint32_t (&slot)[N],
+                                            uint32_t (&value)[N]) const {
     uint32_t open = 0;  // bit j: key j is still probing
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       slot[j] = cap;
+      value[j] = 0;
       if (key[j] != kNoKey) {
         slot[j] = member_home(key[j], cap);
         open |= 1u << j;
       }
     }
     for (uint32_t probes = 0; open != 0 && probes < cap; ++probes) {
-      uint32_t cur[N];
+      uint64_t cur[N];
 #pragma unroll
-      for (int j = 0; j < N; ++j) cur[j] = (open >> j) & 1u ? key_at(slot[j]) : 0u;
+      for (int j = 0; j < N; ++j) cur[j] = (open >> j) & 1u ? slots[slot[j]] : 0ull;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         if (!((open >> j) & 1u)) continue;
-        if (cur[j] == key[j]) {
+        if ((uint32_t)(cur[j] >> 32) == key[j]) {
           open &= ~(1u << j);
-        } else if (cur[j] == kNoKey) {
+          value[j] = (uint32_t)cur[j];
+        } else if ((uint32_t)(cur[j] >> 32) == kNoKey) {
           open &= ~(1u << j);
           slot[j] = cap;
         } else if (++slot[j] == cap) {
@@ -277,28 +277,31 @@ struct MemberTable {
   }
 };
 
-// The same small table, rebuilt in LDS as buckets of four keys: a look-up reads
+// A small table (the picked set of a layer-wise sampler is a few hundred ids) is
+// rebuilt in LDS once per work-group, as buckets of four keys: 64 lanes
+// probing 64 different slots cost the vector cache a tag look-up each, the LDS
+// a few cycles in all.  A look-up reads
 // one bucket (16 bytes, one instruction) and compares four keys, and goes on to
 // the next bucket only from a full one.  With at most two keys per bucket on
-// average nearly every look-up ends at its first bucket, where the linear table
-// makes a wave repeat its probe loop until the longest of its 256 probe runs
-// has ended -- the pass is bound by the instructions it issues.  For picked
+// average nearly every look-up ends at its first bucket, where a linear table
+// makes a wave repeat its probe loop until the longest of its probe runs
+// has ended.  For picked
 // sets whose ids all fit 32 bits (a match of the key is then a match of the id).
 constexpr int kMemberBuckets = kMemberLdsSlots / 4;
 struct BucketTable {
   const uint4* keys;       // [kMemberBuckets] filled from .x on; kNoKey = free
-  const uint32_t* values;  // [kMemberLdsSlots] position in the picked set, by slot
 
   __device__ __forceinline__ static uint32_t home(uint32_t key) {
     return __umulhi(key * 0x9E3779B1u, (uint32_t)kMemberBuckets);
   }
 
-  // fill: a counter per bucket, only used here
+  // fill: a counter per bucket, only used here; also(key) is called for every key,
+  // after a barrier
+  template <typename Also>
   __device__ __forceinline__ void stage(const uint64_t* __restrict__ table, uint32_t capacity,
-                                        uint32_t* lds_keys, uint32_t* lds_values,
-                                        uint32_t* fill) {
+                                        uint32_t* lds_keys, uint16_t* lds_values,
+                                        uint32_t* fill, Also also) {
     keys = reinterpret_cast<const uint4*>(lds_keys);
-    values = lds_values;
     for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberLdsSlots; i += blockDim.x)
       lds_keys[i] = kNoKey;
     for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberBuckets; i += blockDim.x) fill[i] = 0;
@@ -307,12 +310,13 @@ struct BucketTable {
       const uint64_t t = table[i];
       if (t == kEmptySlot) continue;
       const uint32_t key = (uint32_t)(t >> 32);
+      also(key);
       uint32_t b = home(key);
       for (int tries = 0; tries < kMemberBuckets; ++tries) {  // fewer keys than slots: ends early
         const uint32_t at = atomicAdd(&fill[b], 1u);
         if (at < 4u) {
           lds_keys[b * 4 + at] = key;
-          lds_values[b * 4 + at] = (uint32_t)t;
+          lds_values[b * 4 + at] = (uint16_t)t;
           break;
         }
         b = (b + 1) & (kMemberBuckets - 1);
@@ -321,43 +325,66 @@ struct BucketTable {
     __syncthreads();
   }
 
-  // N look-ups in step; slot[j] is where key[j] sits, kMemberLdsSlots when it
-  // is absent (or kNoKey).
-  template <int N>
-  __device__ __forceinline__ void find_many(const uint32_t (&key)[N], uint32_t (&slot)[N]) const {
-    uint32_t b[N];
-    uint32_t open = 0;  // bit j: key j goes on to the next bucket
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      slot[j] = kMemberLdsSlots;
-      b[j] = home(key[j]);
-      if (key[j] != kNoKey) open |= 1u << j;
+  // Where a key sits, kMemberLdsSlots when it is absent (or kNoKey).
+  __device__ __forceinline__ uint32_t find(uint32_t key) const {
+    uint32_t b = home(key);
+    if (key == kNoKey) return kMemberLdsSlots;
+    for (int rounds = 0; rounds < kMemberBuckets; ++rounds) {
+      const uint4 k = keys[b];
+      const uint32_t hit = k.x == key ? 0u : k.y == key ? 1u : k.z == key ? 2u : k.w == key ? 3u : 4u;
+      if (hit < 4u) return b * 4 + hit;
+      if (k.w == kNoKey) break;  // a bucket with room would hold the key
+      b = (b + 1) & (kMemberBuckets - 1);
     }
-    for (int rounds = 0; open != 0 && rounds < kMemberBuckets; ++rounds) {
-      uint4 k[N];
-#pragma unroll
-      for (int j = 0; j < N; ++j) k[j] = keys[b[j]];
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        if (!((open >> j) & 1u)) continue;
-        const int hit = k[j].x == key[j] ? 0 : k[j].y == key[j] ? 1 : k[j].z == key[j] ? 2
-                        : k[j].w == key[j] ? 3 : -1;
-        if (hit >= 0) {
-          slot[j] = b[j] * 4 + hit;
-          open &= ~(1u << j);
-        } else if (k[j].w == kNoKey) {
-          open &= ~(1u << j);  // a bucket with room would hold the key
-        } else {
-          b[j] = (b[j] + 1) & (kMemberBuckets - 1);
-        }
-      }
-    }
+    return kMemberLdsSlots;
   }
 };
 
+// The key of an id in a column whose ids are `offset` more than they say; for 32-bit ids
+// 0 <= offset < 2^31, so that a sum below zero, kNoKey here, is found by clamping the id.
+__device__ __forceinline__ uint32_t offset_key(int32_t id, int64_t offset) {
+  const int32_t least = -1 - (int32_t)offset;
+  return (uint32_t)(id > least ? id : least) + (uint32_t)offset;
+}
+__device__ __forceinline__ uint32_t offset_key(int64_t id, int64_t offset) {
+  return member_key((uint64_t)(id + offset));
+}
+
+// How many lanes below this one are in the set, and `base`.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t set, uint32_t base) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)set, base));
+}
+// Between a wave's writes to its own part of LDS and its reads of other lanes' words.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// What the ids of a run are tested with: the table in LDS and a filter of all its ids
+// in front of it, or the table in L2 and the filter that the insert pass left.
+template <bool kInLds, int kThreads>
+struct MemberShared {
+  static constexpr int kWords = !kInLds ? kFilterWords : kThreads == kMemberThreads ? 4096 : 2048;
+  using Filter = IdFilter<kWords, kInLds ? 2 : kFilterBits>;
+  __align__(16) uint32_t keys[kInLds ? kMemberLdsSlots : 4];
+  uint16_t values[kInLds ? kMemberLdsSlots : 2];  // fewer than kMemberLdsSlots / 2 ids
+  uint32_t filter[kWords];
+  uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
+  uint8_t queue_place[kThreads * kMemberWords];
+};
+
+// Whether a row of 64 edges holds picked ids is told by the filter, a word of LDS and
+// eight instructions an edge; the edges that pass are packed into the wave's queue, and
+// only they, 64 at a time, go through a look-up and are written out.  Most edges of a
+// slice are not kept, and the pass is bound by the instructions it issues: with a look-up
+// for every row 78 vector and 38 scalar instructions a row and 91 us on 31 M edges of which
+// a quarter is kept (two thirds of it the vector units), 66 on 19 M with one kept in
+// twenty-five; now 42 and 30, 64 us and 43 (reading the ids and writing what is kept take 33
+// and 17 at the rate of a copy).  Behind the filter, table in L2: 83 -> 52 on 18.5 M edges.
 // kThreads: work-group size.  A large one shares a staged table among more
 // edges; a small one spreads a short edge list over all compute units.
-// kRun: chunks per wave and run.
+// kRun: chunks per wave and run, whose ids are in flight together.
 // IdT: int64_t, or int32_t when the ids are read from a matrix's narrow copy.
 // kView: the edges are those of a column slice read in place.
 template <bool kInLds, int kThreads, int kRun, typename IdT, bool kView>
@@ -366,191 +393,225 @@ void member_flag_kernel(
     const IdT* __restrict__ ids, int64_t nnz,
     const uint64_t* __restrict__ global_table, uint32_t cap,
     const int64_t* __restrict__ picked, const int* __restrict__ wide_flag,
-    uint64_t* __restrict__ flags, int64_t* __restrict__ chunk_count,
+    int64_t* __restrict__ chunk_count,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
     const uint32_t* __restrict__ filter, SliceView view) {
-  __shared__ __align__(16) uint32_t lds_keys[kInLds ? kMemberLdsSlots : 1];
-  __shared__ uint32_t lds_values[kInLds ? kMemberLdsSlots : 1];
-  __shared__ uint32_t lds_fill[kInLds ? kMemberBuckets : 1];
-  __shared__ uint32_t lds_filter[kInLds ? 1 : kFilterWords];
+  using Shared = MemberShared<kInLds, kThreads>;
+  using Filter = typename Shared::Filter;
+  __shared__ Shared sh;
   const bool wide = *wide_flag != 0;  // the same for every thread of the launch
-  const bool bucketed = kInLds && !wide;
-  const bool filtered = !kInLds && !wide && filter != nullptr;
-  if (filtered) {
-    for (int i = threadIdx.x; i < kFilterWords; i += kThreads) lds_filter[i] = filter[i];
+  const bool filtered = kInLds || filter != nullptr;
+  const MemberTable table{global_table, cap};
+  BucketTable buckets;
+  if (kInLds) {
+    static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
+    for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
+    buckets.stage(global_table, cap, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
+      const uint32_t h = Filter::hash(key);
+      atomicOr(&sh.filter[Filter::word(h)], Filter::bits(h));
+    });
+  } else if (filtered) {
+    for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = filter[i];
     __syncthreads();
   }
-  MemberTable<kInLds, true> table;
-  BucketTable buckets;
-  if (bucketed) {
-    buckets.stage(global_table, cap, lds_keys, lds_values, lds_fill);
-  } else {
-    table.stage(global_table, cap, lds_keys, lds_values);
-  }
-  const uint32_t absent = bucketed ? (uint32_t)kMemberLdsSlots : cap;
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   const int lane = lane_id();
-  // A wave takes runs of kRun chunks, the work-groups of the
-  // launch striding over the runs (a launch with fewer work-groups than runs
-  // stages its tables once per work-group, not once per run).
-  // The ids of the kRun chunks are requested together, before anything is
-  // stored: a store between a load and its use makes the wait for the load
-  // (loads and stores count down one in-order counter) a wait for everything.
+  const int wave = threadIdx.x / kWave;
+  const uint32_t queue0 = wave_uniform_first(wave * kBlock);  // where this wave's queue starts
+  // A wave takes runs of kRun chunks, the waves of the launch striding over them (a launch
+  // with fewer waves than runs stages its tables once per work-group, not once per run).
+  // The short columns of a slice are often neighbours, and a wave that took neighbouring
+  // runs would be at them when all others have ended (126 us where this takes 69).
+  constexpr int kRunEdges = kRun * kBlock;
   const int64_t num_runs = ceil_div_dev(num_chunks, kRun);
-  for (int64_t run = (int64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave;
-       run < num_runs; run += (int64_t)gridDim.x * (kThreads / kWave)) {
-  // With a view the edges are those of a column slice that was never written:
-  // the run's columns are looked up once, and an edge's id
-  // is read from the parent's array.
-  SliceView::Run vrun{};
-  vrun.split = INT64_MAX;  // no view: every edge at distance 0, offset 0
-  bool scattered = false;  // the same in every lane
-  if (kView) {
-    const int64_t e_first = run * kRun * kBlock;
-    const int64_t e_stop = e_first + kRun * kBlock;
-    vrun = view.run(e_first, (e_stop < nnz ? e_stop : nnz) - 1);
-    scattered = !vrun.near();
-  }
-  // id of edge e, or of the last edge for a lane past the end: on a scattered
-  // run the look-up shuffles, so all lanes go through it together
-  auto id_of = [&](int64_t e) -> uint64_t {
-    if (e >= nnz) e = nnz - 1;
-    if (!kView) return (uint64_t)(int64_t)ids[e];
-    if (!scattered) return (uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e));
-    int64_t c, offset;
-    const int64_t p = view.position(vrun, e, &c, &offset);
-    return (uint64_t)((int64_t)ids[p] + offset);
+  const int64_t waves = (int64_t)gridDim.x * (kThreads / kWave);
+  const int64_t self = wave_uniform_first((int64_t)blockIdx.x * (kThreads / kWave) + wave);
+
+  int kept = 0;  // of the chunk at hand; the same in every lane
+  // writes the lanes' edges that were found behind the chunk's others
+  auto keep = [&](int64_t chunk, bool found, uint32_t value, uint32_t place) {
+    const uint64_t peers = __ballot(found);
+    if (found) {
+      const uint32_t at = lanes_below(peers, kept);
+      (staged + chunk * kBlock)[at] = value;
+      (staged_pos + chunk * kBlock)[at] = (uint8_t)place;
+    }
+    kept += __popcll(peers);
   };
-  {
-    const int64_t chunk0 = run * kRun;
+  auto finish_chunk = [&](int64_t chunk) {
+    if (lane == 0) {
+      chunk_count[chunk] = kept;
+      if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
+    }
+    kept = 0;
+  };
+  auto flag_chunk = [&](int64_t chunk, const uint32_t (&key)[kMemberWords]) {
+    uint32_t end = queue0;
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) {
+      const bool may = !filtered || Filter::passes(sh.filter, key[j]);
+      const uint64_t peers = __ballot(may);
+      if (may) {
+        const uint32_t at = lanes_below(peers, end);
+        sh.queue_key[at] = key[j];
+        sh.queue_place[at] = (uint8_t)(j * kWave + lane);
+      }
+      end += __popcll(peers);
+    }
+    wave_lds_fence();
+    if (kInLds) {
+      for (uint32_t q0 = queue0; q0 < end; q0 += kWave) {
+        const uint32_t q = q0 + lane < end ? q0 + lane : end - 1;
+        const uint32_t slot = buckets.find(q0 + lane < end ? sh.queue_key[q] : kNoKey);
+        keep(chunk, slot < kMemberLdsSlots, sh.values[slot & (kMemberLdsSlots - 1)], sh.queue_place[q]);
+      }
+    } else {
+      // a table in L2 answers after a round trip: two edges a lane go through their
+      // probe rounds together
+      constexpr int kN = 2;
+#pragma unroll 1
+      for (uint32_t q0 = queue0; q0 < end; q0 += kN * kWave) {
+        uint32_t k[kN], slot[kN], place[kN], value[kN];
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+          const uint32_t at = q0 + i * kWave + lane, q = at < end ? at : end - 1;
+          k[i] = at < end ? sh.queue_key[q] : kNoKey;
+          place[i] = sh.queue_place[q];
+        }
+        table.find_many(k, slot, value);
+#pragma unroll
+        for (int i = 0; i < kN; ++i) keep(chunk, slot[i] < cap, value[i], place[i]);
+      }
+    }
+    wave_lds_fence();  // the next chunk's queue overwrites this one's
+    finish_chunk(chunk);
+  };
+
+  // A run over several columns, or of a call with wide ids.
+  auto slow_run = [&](int64_t run, const SliceView::Run& vrun) {
+    // id of the lane's edge of a row, or of the last edge for a lane past the end: on a
+    // run of several columns the look-up shuffles, so all lanes go through it together
+    auto id_of = [&](int64_t row, bool* in) -> uint64_t {
+      *in = row + lane < nnz;
+      if (row >= nnz) row = nnz - 1;
+      const int64_t e = *in ? row + lane : nnz - 1;
+      if (!kView) return (uint64_t)(int64_t)ids[e];
+      if (vrun.near()) return (uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e));
+      int64_t c, offset;
+      const int64_t p = view.row_position(vrun, row, e, &c, &offset);
+      return (uint64_t)((int64_t)ids[p] + offset);
+    };
+    // (one chunk's look-ups at a time: all of them unrolled would set the kernel's
+    // registers, and with them how many work-groups a compute unit holds)
+#pragma unroll 1
+    for (int64_t chunk = run * kRun; chunk < num_chunks && chunk < (run + 1) * kRun; ++chunk) {
+      if (!wide) {
+        uint32_t key[kMemberWords];
+#pragma unroll
+        for (int j = 0; j < kMemberWords; ++j) {
+          bool in;
+          const uint64_t id = id_of(chunk * kBlock + j * kWave, &in);
+          key[j] = in ? member_key(id) : kNoKey;
+        }
+        flag_chunk(chunk, key);
+      } else {
+#pragma unroll 1
+        for (int j = 0; j < kMemberWords; ++j) {
+          bool in;
+          const uint64_t id = id_of(chunk * kBlock + j * kWave, &in);
+          const bool may = in && (!filtered || Filter::passes(sh.filter, member_tag(id)));
+          const uint32_t slot = may ? table.find_confirmed(id, picked) : cap;
+          keep(chunk, slot < cap, slot < cap ? table.value_at(slot) : 0u, j * kWave + lane);
+        }
+        finish_chunk(chunk);
+      }
+    }
+  };
+
+  for (int64_t run = self; run < num_runs; run += waves) {
+    const int64_t chunk0 = run * kRun, e_first = run * kRunEdges;
+    const bool whole = e_first + kRunEdges <= nnz;
+    // With a view the edges are those of a column slice that was never written:
+    // the run's columns are looked up once, and an edge's id
+    // is read from the parent's array.
+    SliceView::Run vrun{};
+    vrun.split = INT64_MAX;  // no view: every edge at distance 0, offset 0
+    if (kView) vrun = view.run(e_first, (whole ? e_first + kRunEdges : nnz) - 1);
+    if (wide || (kView && !vrun.near())) {
+      slow_run(run, vrun);
+      continue;
+    }
+    // The ids of the run are requested together, before anything is
+    // stored: a store between a load and its use makes the wait for the load
+    // (loads and stores count down one in-order counter) a wait for everything.
     uint32_t keys[kRun][kMemberWords];
-    if (!kView || !scattered) {
+    const int64_t shift = wave_uniform_first(vrun.shift[0]);
+    const int64_t offset = wave_uniform_first(vrun.offset[0]);
+    if (whole && vrun.span.lo == vrun.span.hi &&
+        (sizeof(IdT) == 8 || (offset >= 0 && offset <= INT32_MAX))) {
+      // all in one column: the lanes' places follow from the wave's
+      const IdT* from = ids + (e_first + shift);
+      IdT id[kRun][kMemberWords];
+#pragma unroll
+      for (int c = 0; c < kRun; ++c)
+#pragma unroll
+        for (int j = 0; j < kMemberWords; ++j) id[c][j] = from[c * kBlock + j * kWave + lane];
+#pragma unroll
+      for (int c = 0; c < kRun; ++c)
+#pragma unroll
+        for (int j = 0; j < kMemberWords; ++j) keys[c][j] = offset_key(id[c][j], offset);
+    } else {
 #pragma unroll
       for (int c = 0; c < kRun; ++c)
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
           const int64_t e = (chunk0 + c) * kBlock + j * kWave + lane;
-          keys[c][j] =
-              e >= nnz ? kNoKey
-              : kView  ? member_key((uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e)))
-                       : member_key((uint64_t)(int64_t)ids[e]);
-        }
-    } else {
-      // one chunk's look-ups at a time: all of them unrolled would set the kernel's
-      // registers, and with them how many work-groups a compute unit holds
-#pragma unroll
-      for (int c = 0; c < kRun; ++c)
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) keys[c][j] = kNoKey;
-#pragma unroll 1
-      for (int now = 0; now < kRun; ++now) {
-        uint32_t key[kMemberWords];
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) {
-          const int64_t e = (chunk0 + now) * kBlock + j * kWave + lane;
-          const uint64_t id = id_of(e);
-          key[j] = e < nnz ? member_key(id) : kNoKey;
-        }
-#pragma unroll
-        for (int c = 0; c < kRun; ++c)
-#pragma unroll
-          for (int j = 0; j < kMemberWords; ++j)
-            if (c == now) keys[c][j] = key[j];
-      }
-    }
-    if (filtered) {
-#pragma unroll
-      for (int c = 0; c < kRun; ++c)
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) {
-          const uint32_t bits = filter_bits(keys[c][j]);
-          if ((lds_filter[filter_word(keys[c][j])] & bits) != bits) keys[c][j] = kNoKey;
-        }
-    }
-    // a table in L2 answers after a round trip: the few look-ups that the filter
-    // lets through go through their probe rounds together for all chunks of the run
-    uint32_t all_slots[kRun * kMemberWords];
-    if (filtered) {
-      uint32_t all_keys[kRun * kMemberWords];
-#pragma unroll
-      for (int c = 0; c < kRun; ++c)
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) all_keys[c * kMemberWords + j] = keys[c][j];
-      table.find_many(all_keys, all_slots);
-    }
-#pragma unroll
-    for (int c = 0; c < kRun; ++c) {
-      const int64_t chunk = chunk0 + c;
-      if (chunk >= num_chunks) break;
-      uint32_t slot[kMemberWords];
-      uint64_t word[kMemberWords];
-      if (bucketed) {
-        buckets.find_many(keys[c], slot);
-      } else if (!wide) {
-        if (!filtered) {
-          table.find_many(keys[c], slot);
-        } else {
-#pragma unroll
-          for (int j = 0; j < kMemberWords; ++j) slot[j] = all_slots[c * kMemberWords + j];
-        }
-      } else {  // (rolled up for the same reason)
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) slot[j] = cap;
-#pragma unroll 1
-        for (int now = 0; now < kMemberWords; ++now) {
-          const int64_t e = chunk * kBlock + now * kWave + lane;
-          const uint64_t id = id_of(e);
-          const uint32_t found = e < nnz ? table.find_confirmed(id, picked) : cap;
-#pragma unroll
-          for (int j = 0; j < kMemberWords; ++j)
-            if (j == now) slot[j] = found;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kMemberWords; ++j) word[j] = __ballot(slot[j] < absent);
-      {
-        int before = 0;  // kept edges of the chunk in front of this row of 64
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) {
-          if (slot[j] < absent) {
-            const int64_t at = chunk * kBlock + before + __popcll(word[j] & ((1ull << lane) - 1));
-            staged[at] = bucketed ? buckets.values[slot[j]] : table.value_at(slot[j]);
-            staged_pos[at] = (uint8_t)(j * kWave + lane);
+          if (kView) {
+            keys[c][j] = e >= nnz ? kNoKey
+                                  : member_key((uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e)));
+          } else {  // (a lane past the end reads the last edge: a branch would wait for the load in it)
+            const uint32_t key = member_key((uint64_t)(int64_t)ids[e < nnz ? e : nnz - 1]);
+            keys[c][j] = e < nnz ? key : kNoKey;
           }
-          before += __popcll(word[j]);
         }
-      }
-      if (lane == 0) {
-        int total = 0;
-#pragma unroll
-        for (int j = 0; j < kMemberWords; ++j) {
-          flags[chunk * kMemberWords + j] = word[j];
-          total += __popcll(word[j]);
-        }
-        chunk_count[chunk] = total;
-        if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
-      }
     }
-  }
+#pragma unroll
+    for (int c = 0; c < kRun; ++c)
+      if (chunk0 + c < num_chunks) flag_chunk(chunk0 + c, keys[c]);
   }
 }
 
-// Kept edges at positions < e.
+// Kept edges at positions < e: those of the chunks before, and how many of the chunk's
+// kept places, which are in order, lie below.  Two rounds of sixteen places each.
 __device__ __forceinline__ int64_t member_rank_before(
-    int64_t e, const uint64_t* __restrict__ flags,
+    int64_t e, const uint8_t* __restrict__ staged_pos,
     const int64_t* __restrict__ chunk_off) {
   const int64_t chunk = e / kBlock;
-  int64_t r = chunk_off[chunk];
+  const int64_t r = chunk_off[chunk];
+  const int kept = (int)(chunk_off[chunk + 1] - r);
   const int in_chunk = (int)(e - chunk * kBlock);
-  const int full = in_chunk / kWave, rem = in_chunk % kWave;
-  for (int w = 0; w < full; ++w) r += __popcll(flags[chunk * kMemberWords + w]);
-  if (rem) r += __popcll(flags[chunk * kMemberWords + full] & ((1ull << rem) - 1));
-  return r;
+  if (in_chunk == 0 || kept == 0) return r;
+  const uint8_t* places = staged_pos + chunk * kBlock;
+  constexpr int kFan = 16;
+  static_assert(kFan * kFan >= kBlock, "two rounds reach every place");
+  int below = 0;
+#pragma unroll
+  for (int i = 1; i < kFan; ++i) {  // whole blocks of kFan places
+    const int at = i * kFan - 1;
+    below += at < kept && places[at < kept ? at : 0] < in_chunk ? kFan : 0;
+  }
+  int more = 0;
+#pragma unroll
+  for (int i = 0; i < kFan; ++i) {
+    const int at = below + i;
+    more += at < kept && places[at < kept ? at : 0] < in_chunk ? 1 : 0;
+  }
+  return r + below + more;
 }
 
 __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
-    const uint64_t* __restrict__ flags, const int64_t* __restrict__ chunk_off,
+    const uint8_t* __restrict__ staged_pos, const int64_t* __restrict__ chunk_off,
     int64_t nnz, int64_t* __restrict__ out_indptr, int64_t* __restrict__ out_total) {
   const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
@@ -558,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
   if (indptr == nullptr || c > num_major) return;
   const int64_t e = indptr[c];
   out_indptr[c] = nnz == 0 ? 0
-                  : (e >= nnz ? chunk_off[num_chunks] : member_rank_before(e, flags, chunk_off));
+                  : (e >= nnz ? chunk_off[num_chunks] : member_rank_before(e, staged_pos, chunk_off));
 }
 
 // A wave writes the kept edges of kRun consecutive chunks: how many each has comes
@@ -701,13 +762,13 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
     int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
     // a large list, or work-groups that stage the 64 KB filter: as many of them as are
     // resident, each staging its tables once and striding over its runs
-    const int64_t resident = (int64_t)(kFilterGroupsPerCu * kMemberThreads / threads) * num_compute_units();
+    const int64_t resident = (int64_t)(kResidentPerCu * kMemberThreads / threads) * num_compute_units();
     if ((filter || !small) && blocks > resident) blocks = resident;
     const dim3 grid((unsigned)blocks);
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
-                IDS, nnz, w.table, cap, picked, w.wide, w.flags, w.chunk_off, w.staged,       \
+                IDS, nnz, w.table, cap, picked, w.wide, w.chunk_off, w.staged,       \
                 w.staged_pos, filter, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
@@ -735,7 +796,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   const int64_t n = indptr ? num_major + 1 : 1;
   GS_LAUNCH("member_indptr", s,
             member_indptr_kernel<<<dim3((unsigned)ceil_div(n, kBlock)),
-                                   dim3(kBlock), 0, s>>>(indptr, num_major, w.flags,
+                                   dim3(kBlock), 0, s>>>(indptr, num_major, w.staged_pos,
                                                          w.chunk_off, nnz,
                                                          out_indptr, out_total));
   return GS_OK;

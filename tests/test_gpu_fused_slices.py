@@ -92,6 +92,31 @@ def test_col_row_slice_with_per_column_key_offsets():
                                 indices32=T(indices).to(torch.int32)), want)
 
 
+@pytest.mark.parametrize("npick", [600, 5000])
+@pytest.mark.parametrize("offset", [0, 70_000, 2**31 - 1, 2**31, 2**32 - 1000, -500])
+def test_col_row_slice_of_columns_of_every_length(offset, npick):
+    """9 M edges, for which every wave strides over runs: columns without edges, of a few, that
+    end at the borders of rows, and long ones, next to each other, more than 64 of them in a
+    run; the offsets of half of them at the ends of what 32-bit arithmetic can hold."""
+    rng = np.random.default_rng(npick + offset % 1000)
+    deg = np.concatenate([rng.integers(0, 4, size=3000), rng.integers(0, 3, size=500) * 64,
+                          rng.integers(0, 900, size=500), rng.integers(50_000, 60_000, size=160),
+                          rng.integers(0, 2, size=700) * rng.integers(0, 130, size=700)])
+    deg[rng.choice(4000, 300)] = 1
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    assert 1 << 23 <= indptr[-1] < 1 << 24
+    indices = rng.integers(0, 60_000, size=int(indptr[-1]))
+    cols = np.arange(len(deg))
+    key_offset = np.where(rng.random(len(deg)) < 0.5, offset, 0)
+    picked = rng.choice(60_000, size=npick, replace=False)
+    picked[npick // 2:] += offset
+    want = chained_col_row_slice(indptr, indices, cols, picked, key_offset)
+    narrow = T(indices).to(torch.int32)
+    same(capi.col_row_slice(T(indptr), T(indices), T(cols), T(picked), T(key_offset)), want)
+    same(capi.col_row_slice(T(indptr), T(indices), T(cols), T(picked), T(key_offset),
+                            indices32=narrow), want)
+
+
 @pytest.mark.parametrize("ncol,num_rows", [(0, 100), (3, 5000), (600, 5200), (512, 100_000)])
 @pytest.mark.parametrize("use_workspace", [True, False])
 def test_sliced_e_square_sum_parity(ncol, num_rows, use_workspace):

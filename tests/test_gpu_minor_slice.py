@@ -65,6 +65,20 @@ def test_minor_slice_at_the_borders_of_a_waves_run(nnz, npick):
          orc.minor_slice(indices, picked, indptr=indptr))
 
 
+@pytest.mark.parametrize("npick", [1, 2046, 2047, 2048, 131_072, 131_073])
+@pytest.mark.parametrize("num_ids", [1, 2300, 200_000])
+def test_minor_slice_at_the_borders_of_table_and_filter(num_ids, npick):
+    """The most ids of a table in LDS and of the filter and one more, with all, most and few
+    of the edges kept: a full queue of candidates, and candidates that are none."""
+    rng = np.random.default_rng(npick + num_ids)
+    ids = rng.integers(0, num_ids, size=70_001)
+    picked = rng.permutation(max(num_ids, npick))[:npick]
+    indptr = np.sort(rng.integers(0, len(ids) + 1, size=901))
+    indptr[0], indptr[-1] = 0, len(ids)
+    same(capi.minor_slice(T(ids), T(picked), indptr=T(indptr)),
+         orc.minor_slice(ids, picked, indptr=indptr))
+
+
 @pytest.mark.parametrize("npick", [3, 700, 5000])
 def test_minor_slice_with_ids_beyond_32_bits(npick):
     """Picked ids of 2^32 - 1 and above: ids that agree in their low 32 bits must
