@@ -25,7 +25,12 @@
 // layer's frontier offsets), launches are sized by its bound, and nothing is waited
 // for between layers.
 // GraphSAGE [25,10], 1024 seeds, 100 K nodes: 16 launches and four waits, 128 us,
-// before; seven launches and one wait now.
+// before; seven launches and one wait, 50 us, now.  The launches are chains of dependent
+// loads, a round trip to memory each, so every load is sent off as soon as its address is
+// known: ahead of the number of columns (a place below the bound is read whatever it
+// holds), of the sum over the tiles, of the work-group's own dedup, and of the stores that
+// empty the table (the six launches: 48.7 us without that, 41.8 with it; the nine of
+// [15,10,5] in 8 batches 110.7 and 99.8).
 #include "common.h"
 #include "hashtable.h"
 
@@ -92,6 +97,11 @@ struct LayerColumns {
   const int64_t* ptr;  // [B + 1] offsets of the batches, null: one batch of `count`
   int64_t B, count;    // count: bound of the number of columns when ptr is given
   __device__ __forceinline__ int64_t num() const { return ptr ? ptr[B] : count; }
+  // A place among those of the bound, for a load that does not wait for the number of
+  // columns (what lies past that number is not looked at).
+  __device__ __forceinline__ int64_t place(int64_t p, int64_t width) const {
+    return p < count * width ? p : 0;
+  }
   __device__ __forceinline__ int64_t lo(int64_t b) const { return ptr ? ptr[b] : 0; }
   __device__ __forceinline__ int64_t hi(int64_t b) const { return ptr ? ptr[b + 1] : count; }
   // batch of a column, at or after batch b0
@@ -103,13 +113,13 @@ struct LayerColumns {
   }
 };
 
-// The slot of a key in the global table after (key, position) went in.
+// The slot of a key in the global table after (key, position) went in; `cur` is what its
+// first slot was seen to hold.
 __device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask, uint32_t key,
-                                                 uint32_t position) {
+                                                 uint32_t position, uint64_t cur) {
   const uint64_t mine = ((uint64_t)key << 32) | position;
   uint32_t slot = hash32(key) & mask;
   for (uint32_t probes = 0; probes <= mask; ++probes) {  // at most half full: ends early
-    uint64_t cur = table[slot];
     if (cur == kEmptySlot) {
       cur = atomicCAS((unsigned long long*)(table + slot), (unsigned long long)kEmptySlot,
                       (unsigned long long)mine);
@@ -121,6 +131,7 @@ __device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask,
       return slot;
     }
     slot = (slot + 1) & mask;
+    cur = table[slot];
   }
   return 0;
 }
@@ -133,29 +144,30 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
     const int64_t* __restrict__ picked, uint64_t* table, uint32_t mask,
     uint32_t* __restrict__ slot_of, int32_t* wide) {
   __shared__ uint32_t tags[kPickSlots], mins[kPickSlots], global_slot[kPickSlots];
-  const int64_t n = cols.num();
   constexpr int kWaves = kPickThreads / kWave;
   const int64_t first_col = (int64_t)blockIdx.x * (kWaves * cols_per_wave);
-  if (first_col >= n) return;  // uniform per work-group
-  for (int i = threadIdx.x; i < kPickSlots; i += kPickThreads) {
-    tags[i] = kNoSlot;
-    mins[i] = 0xFFFFFFFFu;
-  }
   const int wave_lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int width = fanout + 1;
   const int group = wave_lane / width;
   const int lane = wave_lane - group * width;  // 0: the seed, j + 1: pick j
   const int64_t c = first_col + wave * cols_per_wave + group;
+  // one round trip for the number of columns and the id, of a place that may be no column's
+  const int64_t id = cols.ids[cols.place(c, 1)];
+  const int64_t n = cols.num();
+  if (first_col >= n) return;  // uniform per work-group
+  for (int i = threadIdx.x; i < kPickSlots; i += kPickThreads) {
+    tags[i] = kNoSlot;
+    mins[i] = 0xFFFFFFFFu;
+  }
   const bool live = group < cols_per_wave && c < n;
   uint32_t my_key = kNoSlot, position = 0;
   if (live) {
-    const int64_t id = cols.ids[c];
+    int64_t start;
+    const int64_t deg = column_degree(indptr, num_cols, id, &start);
     const int64_t b0 = cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(first_col)) : 0;
     const int64_t b = cols.batch_of(c, b0);
     const int64_t s_lo = cols.lo(b), ns = cols.hi(b) - s_lo;
     const int64_t fb = s_lo * width;
-    int64_t start;
-    const int64_t deg = column_degree(indptr, num_cols, id, &start);
     int64_t row = -1;
     if (lane == 0) {
       row = id;
@@ -183,6 +195,8 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
     }
     if (row >= 0) my_key = (uint32_t)b * stride + (uint32_t)row;
   }
+  // (looked at now, so that the answer is there when the work-group knows whose key it is)
+  const uint64_t seen = my_key != kNoSlot ? table[hash32(my_key) & mask] : 0ull;
   __syncthreads();
   uint32_t at = 0;
   if (my_key != kNoSlot) {
@@ -197,7 +211,7 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
   }
   __syncthreads();
   if (my_key != kNoSlot && mins[at] == position)
-    global_slot[at] = layer_insert(table, mask, my_key, position);
+    global_slot[at] = layer_insert(table, mask, my_key, position, seen);
   __syncthreads();
   if (live) slot_of[position] = my_key != kNoSlot ? global_slot[at] : kNoSlot;
 }
@@ -224,20 +238,21 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
     uint32_t* __restrict__ keys, LayerWord* __restrict__ words, uint2* __restrict__ tile_cnt) {
   __shared__ uint32_t wave_first[kBlock / kWave], wave_edge[kBlock / kWave];
   const int width = fanout + 1;
-  const int64_t N = cols.num() * width;
   const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
-  if (p0 >= N) return;
   const int wave = threadIdx.x / kWave, lane = lane_id();
   const int64_t wave_p0 = p0 + (int64_t)wave * kLayerWordsPerWave * kWave;
   uint32_t s[kLayerWordsPerWave];
   uint64_t e[kLayerWordsPerWave];
 #pragma unroll
-  for (int j = 0; j < kLayerWordsPerWave; ++j) {
-    const int64_t p = wave_p0 + j * kWave + lane;
-    s[j] = p < N ? slot_of[p] : kNoSlot;
-  }
+  for (int j = 0; j < kLayerWordsPerWave; ++j)
+    s[j] = slot_of[cols.place(wave_p0 + j * kWave + lane, width)];
+  const int64_t N = cols.num() * width;
+  if (p0 >= N) return;
 #pragma unroll
-  for (int j = 0; j < kLayerWordsPerWave; ++j) e[j] = s[j] != kNoSlot ? table[s[j]] : 0ull;
+  for (int j = 0; j < kLayerWordsPerWave; ++j) {
+    if (wave_p0 + j * kWave + lane >= N) s[j] = kNoSlot;
+    e[j] = s[j] != kNoSlot ? table[s[j]] : 0ull;
+  }
   const TileBatches batches =
       tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
   LayerWord mine{0ull, 0ull, 0u, 0u, 0ull};
@@ -296,21 +311,55 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
     const int32_t* __restrict__ wide, LayerOut out) {
   __shared__ uint2 before[kLayerMaxTiles];  // first occurrences and edges before a tile
   __shared__ uint64_t smem[kBlock / kWave + 1];
-  // the table is done with: its share emptied by every work-group of the launch
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < table_slots;
-       i += (int64_t)gridDim.x * kBlock)
-    table[i] = kEmptySlot;
+  // The table is done with: its share emptied by every work-group of the launch, last of
+  // all (loads behind stores are waited for with them).
+  auto empty_table = [&] {
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < table_slots;
+         i += (int64_t)gridDim.x * kBlock)
+      table[i] = kEmptySlot;
+  };
   const int width = fanout + 1;
-  const int64_t n = cols.num(), N = n * width;
-  const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
-  if (blockIdx.x != 0 && (int64_t)blockIdx.x >= tiles) return;
+  // What a position needs does not wait for the counts: its word, its key, and the word of
+  // its key's first position travel while the tiles are added up, and so do the words of
+  // the tile's first batch.
+  constexpr int kItems = kLayerTile / kBlock;
+  const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
+  LayerWord word[kItems];
+  uint32_t key[kItems], first_of[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    const int64_t q = cols.place(p0 + i * kBlock + threadIdx.x, width);
+    word[i] = words[q / kWave];
+    key[i] = keys[q];
+    first_of[i] = first[q];
+  }
   constexpr int kPer = kLayerMaxTiles / kBlock;
   uint2 cnt[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    cnt[j] = tile_cnt[(int64_t)threadIdx.x * kPer + j < gridDim.x ? threadIdx.x * kPer + j : 0];
+  const int64_t n = cols.num(), N = n * width;
+  const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
+  if (blockIdx.x != 0 && (int64_t)blockIdx.x >= tiles) return empty_table();
+  const TileBatches batches =
+      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
+  LayerWord first_word[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    const int64_t p = p0 + i * kBlock + threadIdx.x;
+    // (no key was sent to this position: nothing was written there)
+    const bool edge = p < N && ((word[i].edge >> (int)(p % kWave)) & 1ull);
+    if (!edge) first_of[i] = 0;
+    first_word[i] = words[first_of[i] / kWave];
+  }
+  int64_t b = batches.b_lo;
+  int64_t s_lo = cols.lo(b), ns = cols.hi(b) - s_lo, fb = s_lo * width;
+  LayerWord word_b = words[cols.place(fb, width) / kWave];
+  LayerWord word_q = words[cols.place(fb + (ns > 0 ? ns - 1 : 0), width) / kWave];
   uint64_t sum = 0;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const int64_t t = (int64_t)threadIdx.x * kPer + j;
-    cnt[j] = t < tiles ? tile_cnt[t] : make_uint2(0u, 0u);
+    if ((int64_t)threadIdx.x * kPer + j >= tiles) cnt[j] = make_uint2(0u, 0u);
     sum += ((uint64_t)cnt[j].y << 32) | cnt[j].x;
   }
   uint64_t total;
@@ -322,28 +371,31 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
   }
   __syncthreads();
   const uint32_t all_first = (uint32_t)total, all_edges = (uint32_t)(total >> 32);
-  auto ranks = [&](int64_t p, uint32_t* f, uint32_t* e) {  // counts before position p <= N
-    if (p >= N) {
+  auto ranks_in = [&](const LayerWord& w, int64_t p, uint32_t* f, uint32_t* e) {
+    if (p >= N) {  // counts before position p <= N
       *f = all_first;
       *e = all_edges;
       return;
     }
-    const LayerWord w = words[p / kWave];
     const uint2 t = before[p / kLayerTile];
     const uint64_t below = (1ull << (int)(p % kWave)) - 1ull;
     *f = t.x + w.first_before + (uint32_t)__popcll(w.first & below);
     *e = t.y + w.edge_before + (uint32_t)__popcll(w.edge & below);
   };
-  auto rank_first = [&](uint32_t p) {
-    const LayerWord w = words[p / kWave];
+  auto ranks = [&](int64_t p, uint32_t* f, uint32_t* e) {
+    ranks_in(words[p < N ? p / kWave : 0], p, f, e);
+  };
+  auto rank_in = [&](const LayerWord& w, uint32_t p) {
     return before[p / kLayerTile].x + w.first_before +
            (uint32_t)__popcll(w.first & ((1ull << (int)(p % kWave)) - 1ull));
   };
-  auto seeds_distinct = [&](int64_t fb, int64_t ns, uint32_t f0) {
+  auto rank_first = [&](uint32_t p) { return rank_in(words[p / kWave], p); };
+  // w: the word of the batch's last seed
+  auto seeds_distinct = [&](const LayerWord& w, int64_t fb, int64_t ns, uint32_t f0) {
     if (ns == 0) return true;
     const int64_t q = fb + ns - 1;
-    return ((words[q / kWave].first >> (int)(q % kWave)) & 1ull) &&
-           rank_first((uint32_t)q) - f0 == (uint32_t)(ns - 1);
+    return ((w.first >> (int)(q % kWave)) & 1ull) &&
+           rank_in(w, (uint32_t)q) - f0 == (uint32_t)(ns - 1);
   };
   if (blockIdx.x == 0) {
     for (int64_t b = threadIdx.x; b <= cols.B; b += kBlock) {
@@ -355,28 +407,28 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
       store_for_host(out.mirror + b, f);
       store_for_host(out.mirror + (cols.B + 1) + b, e);
       if (b < cols.B) {
-        const int64_t s_hi = cols.hi(b);
+        const int64_t s_hi = cols.hi(b), last = s_lo * width + (s_hi > s_lo ? s_hi - s_lo - 1 : 0);
         if (out.block_indptr) {
           uint32_t f1, e1;
           ranks(s_hi * width, &f1, &e1);
           out.block_indptr[s_hi + b] = e1 - e;  // the last offset of the block
         }
         store_for_host(out.mirror + 2 * (cols.B + 1) + b,
-                       seeds_distinct(s_lo * width, s_hi - s_lo, f) ? 1 : 0);
+                       seeds_distinct(words[cols.place(last, width) / kWave], s_lo * width,
+                                      s_hi - s_lo, f)
+                           ? 1
+                           : 0);
       } else {
         store_for_host(out.mirror + 3 * cols.B + 2, *wide);
       }
     }
   }
-  const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
-  if (p0 >= N) return;
-  const TileBatches batches =
-      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
-  int64_t b = -1, s_lo = 0, ns = 0, fb = 0;
-  uint32_t f0 = 0, e0 = 0;
-  bool distinct = true;
+  if (p0 >= N) return empty_table();
+  uint32_t f0, e0;
+  ranks_in(word_b, fb, &f0, &e0);
+  bool distinct = seeds_distinct(word_q, fb, ns, f0);
 #pragma unroll
-  for (int i = 0; i < kLayerTile / kBlock; ++i) {
+  for (int i = 0; i < kItems; ++i) {
     const int64_t p = p0 + i * kBlock + threadIdx.x;
     if (p >= N) break;
     const int64_t b_now = batches.of(cols, width, p);
@@ -386,15 +438,15 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
       ns = cols.hi(b) - s_lo;
       fb = s_lo * width;
       ranks(fb, &f0, &e0);
-      distinct = seeds_distinct(fb, ns, f0);
+      distinct = seeds_distinct(words[cols.place(fb + (ns > 0 ? ns - 1 : 0), width) / kWave], fb, ns, f0);
     }
-    const LayerWord w = words[p / kWave];
+    const LayerWord& w = word[i];
     const int bit = (int)(p % kWave);
     const uint64_t below = (1ull << bit) - 1ull;
     const uint2 t = before[blockIdx.x];
     if ((w.first >> bit) & 1ull)
       out.frontier[t.x + w.first_before + (uint32_t)__popcll(w.first & below)] =
-          (int64_t)(keys[p] - (uint32_t)b * stride);
+          (int64_t)(key[i] - (uint32_t)b * stride);
     const uint32_t local = (uint32_t)(p - fb);
     if (local < (uint32_t)ns) continue;
     const uint32_t slot = local - (uint32_t)ns;
@@ -403,10 +455,11 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
     if (out.block_indptr && slot - c * (uint32_t)fanout == 0)
       out.block_indptr[s_lo + c + b] = e - e0;
     if ((w.edge >> bit) & 1ull) {
-      out.row[e] = rank_first(first[p]) - f0;
+      out.row[e] = rank_in(first_word[i], first_of[i]) - f0;
       out.col[e] = distinct ? c : rank_first(first[fb + c]) - f0;
     }
   }
+  empty_table();
 }
 
 __global__ __launch_bounds__(kBlock) void layer_clear_kernel(uint64_t* table, int64_t slots,
