@@ -33,6 +33,48 @@ static int static_scratch(int64_t** out) {
   return GS_OK;
 }
 
+// What N requested columns, `first` and every `step`-th after it, come to in the output; an
+// id outside the matrix, and a place past the end, count nothing.  Their ids and then their
+// pointers are asked for together, with no branch between a load and its use (each would
+// be waited for inside its own: one work-group took 8 to 14 us for some hundred columns,
+// now 5).
+template <int N>
+__device__ __forceinline__ void count_columns(const int64_t* __restrict__ indptr, int64_t num_cols,
+                                              const int64_t* __restrict__ column_ids,
+                                              int64_t num_items, int64_t first, int64_t step,
+                                              int64_t fanout, int replace,
+                                              int64_t* __restrict__ col_span, int64_t (&cnt)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) cnt[k] = 0;
+  if (num_items == 0) return;  // (there may be no ids)
+  int64_t id[N], begin[N], end[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int64_t i = first + k * step < num_items ? first + k * step : num_items - 1;
+    id[k] = column_ids ? column_ids[i] : i;
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const bool inside = id[k] >= 0 && id[k] < num_cols;
+    begin[k] = indptr[inside ? id[k] : 0];
+    end[k] = indptr[inside ? id[k] + 1 : 0];
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int64_t i = first + k * step;
+    const bool inside = id[k] >= 0 && id[k] < num_cols;
+    const int64_t deg = inside ? end[k] - begin[k] : 0;
+    if (i >= num_items) continue;
+    if (col_span) col_span[i] = pack_span(inside ? begin[k] : 0, deg);
+    if (fanout < 0)
+      cnt[k] = deg;
+    else if (replace)
+      cnt[k] = deg == 0 ? 0 : fanout;
+    else
+      cnt[k] = deg < fanout ? deg : fanout;
+  }
+}
+
 // One work-group of kCountThreads threads per tile of the scan that follows
 // (kScanTile consecutive columns): writes the output counts and the tile's sum,
 // so that the scan only has its down sweep left to turn the counts into
@@ -47,24 +89,10 @@ __global__ __launch_bounds__(kCountThreads) void col_count_kernel(
   __shared__ int64_t smem[kCountThreads / kWave + 1];
   const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
   int64_t cnt[kCountItems], sum = 0;
+  count_columns(indptr, num_cols, column_ids, num_items, base, (int64_t)kCountThreads, fanout,
+                replace, col_span, cnt);
 #pragma unroll
-  for (int k = 0; k < kCountItems; ++k) {
-    const int64_t i = base + k * kCountThreads;
-    cnt[k] = 0;
-    if (i < num_items) {
-      int64_t in_start;
-      const int64_t deg =
-          column_degree(indptr, num_cols, column_ids ? column_ids[i] : i, &in_start);
-      if (col_span) col_span[i] = pack_span(in_start, deg);
-      if (fanout < 0)
-        cnt[k] = deg;
-      else if (replace)
-        cnt[k] = deg == 0 ? 0 : fanout;
-      else
-        cnt[k] = deg < fanout ? deg : fanout;
-    }
-    sum += cnt[k];
-  }
+  for (int k = 0; k < kCountItems; ++k) sum += cnt[k];
 #pragma unroll
   for (int k = 0; k < kCountItems; ++k) {
     const int64_t i = base + k * kCountThreads;
@@ -76,7 +104,7 @@ __global__ __launch_bounds__(kCountThreads) void col_count_kernel(
 }
 
 // Up to kSmallCountItems columns: one work-group counts and scans in a single
-// launch (every thread asks for its eight columns' pointers at once), where the
+// launch, where the
 // tiled pair of launches above costs a small sampling step one launch more per
 // layer than it has work for.
 constexpr int kSmallCountPer = 8;
@@ -87,36 +115,31 @@ __global__ __launch_bounds__(kCountThreads) void col_count_small_kernel(
     int replace, int64_t* __restrict__ sub_indptr, int64_t* total_mirror,
     int64_t* __restrict__ col_span) {
   __shared__ int64_t smem[kCountThreads / kWave + 1];
-  // thread t owns columns t * 8 .. t * 8 + 7: its prefix sums leave in one run
-  const int64_t base = (int64_t)threadIdx.x * kSmallCountPer;
-  int64_t cnt[kSmallCountPer], sum = 0;
+  // thread t owns kPer columns from t * kPer on: its prefix sums leave in one run
+  auto count = [&](auto per) {
+    constexpr int kPer = decltype(per)::value;
+    const int64_t base = (int64_t)threadIdx.x * kPer;
+    int64_t cnt[kPer], sum = 0;
+    count_columns(indptr, num_cols, column_ids, num_items, base, (int64_t)1, fanout, replace,
+                  col_span, cnt);
 #pragma unroll
-  for (int k = 0; k < kSmallCountPer; ++k) {
-    const int64_t i = base + k;
-    cnt[k] = 0;
-    if (i < num_items) {
-      int64_t in_start;
-      const int64_t deg =
-          column_degree(indptr, num_cols, column_ids ? column_ids[i] : i, &in_start);
-      if (col_span) col_span[i] = pack_span(in_start, deg);
-      if (fanout < 0)
-        cnt[k] = deg;
-      else if (replace)
-        cnt[k] = deg == 0 ? 0 : fanout;
-      else
-        cnt[k] = deg < fanout ? deg : fanout;
+    for (int k = 0; k < kPer; ++k) sum += cnt[k];
+    int64_t total;
+    int64_t run = block_exclusive_sum<int64_t, kCountThreads>(sum, smem, &total);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int64_t i = base + k;
+      if (i <= num_items) sub_indptr[i] = run;
+      run += cnt[k];
     }
-    sum += cnt[k];
-  }
-  int64_t total;
-  int64_t run = block_exclusive_sum<int64_t, kCountThreads>(sum, smem, &total);
-#pragma unroll
-  for (int k = 0; k < kSmallCountPer; ++k) {
-    const int64_t i = base + k;
-    if (i <= num_items) sub_indptr[i] = run;
-    run += cnt[k];
-  }
-  if (threadIdx.x == 0 && total_mirror) store_for_host(total_mirror, total);
+    if (threadIdx.x == 0 && total_mirror) store_for_host(total_mirror, total);
+  };
+  if (num_items < kCountThreads)
+    count(std::integral_constant<int, 1>{});
+  else if (num_items < 2 * kCountThreads)
+    count(std::integral_constant<int, 2>{});
+  else
+    count(std::integral_constant<int, kSmallCountPer>{});
 }
 
 // Edge-parallel slice: thread e owns output edge e, finds its column by binary

@@ -940,6 +940,30 @@ __device__ __forceinline__ int64_t batch_in_span(const int64_t* __restrict__ ptr
   return s.lo == s.hi ? s.lo : s.lo + segment_of(ptr + s.lo, s.hi - s.lo + 1, x);
 }
 
+// The batches of a group, one a lane, for a group of several but no more than a
+// wavefront has lanes (small batches): which of them a position belongs to is then told
+// by comparing it with borders that are there already, where a search per position waits
+// for a load per step (a few thousand keys of 16 batches: flag 12 us, fill 17; now 5 and 7).
+struct LaneBatches {
+  static constexpr int kRows = 4;  // rows of 64 positions in flight (all 16 of a wave: 246 registers)
+  int64_t start;  // first position of this lane's batch, INT64_MAX past the last
+  __device__ __forceinline__ static bool serves(const BatchSpan& s) {
+    return s.hi > s.lo && s.hi - s.lo < kWave;
+  }
+  __device__ __forceinline__ LaneBatches(const int64_t* __restrict__ ptr, const BatchSpan& s)
+      : start(s.lo + lane_id() <= s.hi ? ptr[s.lo + lane_id()] : INT64_MAX) {}
+  // Which lane's batch holds p, one of the 64 positions from `row` (the same in every
+  // lane) on.  All lanes call this together.
+  __device__ __forceinline__ int of(int64_t row, int64_t p) const {
+    const int head = __popcll(__ballot(start <= row)) - 1;
+    const int tail = __popcll(__ballot(start <= row + kWave - 1)) - 1;
+    int i = head;
+    for (int k = head + 1; k <= tail; ++k)
+      if (p >= (int64_t)__shfl((long long)start, k, kWave)) i = k;
+    return i;
+  }
+};
+
 // One work-group per group of kGroup positions; a wave takes kWordsPerWave
 // consecutive words, lane l the positions l, l + 64, ...: coalesced rows whose
 // ballots are the words.
@@ -954,29 +978,51 @@ __global__ __launch_bounds__(kBlock) void unique_flag_kernel(
   const int64_t p0 = word0 * kWave;
   const BatchSpan span = batch_span(group_batch, group);
   const int64_t fb_lo = flat_ptr[span.lo];
-  uint32_t f[kWordsPerWave];
-#pragma unroll
-  for (int j = 0; j < kWordsPerWave; ++j) {
-    const int64_t p = p0 + j * kWave + lane;
-    f[j] = p < N ? first[p] : 0u;
-  }
   uint64_t my_bits = 0;
   uint32_t my_before = 0, total = 0;
-#pragma unroll
-  for (int j = 0; j < kWordsPerWave; ++j) {
-    const int64_t p = p0 + j * kWave + lane;
-    bool is_first = false;
-    if (p < N) {
-      const int64_t fb =
-          span.lo == span.hi ? fb_lo : flat_ptr[batch_in_span(flat_ptr, span, p)];
-      is_first = (int64_t)f[j] == p - fb;
-    }
+  auto word = [&](int j, bool is_first) {
     const uint64_t bits = __ballot(is_first);
     if (lane == j) {
       my_bits = bits;
       my_before = total;
     }
     total += (uint32_t)__popcll(bits);
+  };
+  if (LaneBatches::serves(span)) {
+    const LaneBatches few(flat_ptr, span);
+#pragma unroll 1
+    for (int j0 = 0; j0 < kWordsPerWave; j0 += LaneBatches::kRows) {
+      uint32_t f[LaneBatches::kRows];
+#pragma unroll
+      for (int j = 0; j < LaneBatches::kRows; ++j) {
+        const int64_t p = p0 + (j0 + j) * kWave + lane;
+        f[j] = first[p < N ? p : N - 1];
+      }
+#pragma unroll
+      for (int j = 0; j < LaneBatches::kRows; ++j) {
+        const int64_t row = p0 + (j0 + j) * kWave, p = row + lane;
+        const int64_t fb = (int64_t)__shfl((long long)few.start, few.of(row, p), kWave);
+        word(j0 + j, p < N && (int64_t)f[j] == p - fb);
+      }
+    }
+  } else {
+    uint32_t f[kWordsPerWave];
+#pragma unroll
+    for (int j = 0; j < kWordsPerWave; ++j) {
+      const int64_t p = p0 + j * kWave + lane;
+      f[j] = p < N ? first[p] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kWordsPerWave; ++j) {
+      const int64_t p = p0 + j * kWave + lane;
+      bool is_first = false;
+      if (p < N) {
+        const int64_t fb =
+            span.lo == span.hi ? fb_lo : flat_ptr[batch_in_span(flat_ptr, span, p)];
+        is_first = (int64_t)f[j] == p - fb;
+      }
+      word(j, is_first);
+    }
   }
   if (lane == 0) wave_total[wave] = total;
   __syncthreads();
@@ -1088,6 +1134,34 @@ __device__ __forceinline__ void fill_group(
   RankWord mine{0ull, 0u, 0u};  // lane j holds word j of this wave
   if (lane < kWordsPerWave && (word0 + lane) * kWave < N) mine = words[word0 + lane];
   int64_t* out = out_unique + group_off[group];
+  auto store = [&](int j, uint64_t key) {
+    const uint64_t bits = __shfl((unsigned long long)mine.bits, j, kWave);
+    const uint32_t before = __shfl(mine.before, j, kWave);
+    if ((bits >> lane) & 1ull)
+      out[before + __popcll(bits & ((1ull << lane) - 1ull))] = (int64_t)key;
+  };
+  if (LaneBatches::serves(span)) {
+    const LaneBatches few(flat_ptr, span);
+    const BatchInfo* b = batch + (span.lo + lane < span.hi ? span.lo + lane : span.hi);
+    const int64_t rows_before = b->r_lo, seeds_to = b->s_lo + b->ns;
+#pragma unroll 1
+    for (int j0 = 0; j0 < kWordsPerWave; j0 += LaneBatches::kRows) {
+      uint64_t key[LaneBatches::kRows];
+#pragma unroll
+      for (int j = 0; j < LaneBatches::kRows; ++j) {
+        const int64_t row = (word0 + j0 + j) * kWave < N ? (word0 + j0 + j) * kWave : N - 1;
+        const int64_t p = row + lane < N ? row + lane : N - 1;
+        const int i = few.of(row, p);
+        const int64_t r = (int64_t)__shfl((long long)rows_before, i, kWave);
+        const int64_t s = (int64_t)__shfl((long long)seeds_to, i, kWave);
+        // a flat position: place among the seeds + rows before, or among the rows + seeds so far
+        key[j] = (uint64_t)*(p < r + s ? k.seeds + (p - r) : k.rows + (p - s));
+      }
+#pragma unroll
+      for (int j = 0; j < LaneBatches::kRows; ++j) store(j0 + j, key[j]);
+    }
+    return;
+  }
   uint64_t key[kWordsPerWave];
 #pragma unroll
   for (int j = 0; j < kWordsPerWave; ++j) {
@@ -1099,12 +1173,7 @@ __device__ __forceinline__ void fill_group(
     }
   }
 #pragma unroll
-  for (int j = 0; j < kWordsPerWave; ++j) {
-    const uint64_t bits = __shfl((unsigned long long)mine.bits, j, kWave);
-    const uint32_t before = __shfl(mine.before, j, kWave);
-    if ((bits >> lane) & 1ull)
-      out[before + __popcll(bits & ((1ull << lane) - 1ull))] = (int64_t)key[j];
-  }
+  for (int j = 0; j < kWordsPerWave; ++j) store(j, key[j]);
 }
 
 __global__ __launch_bounds__(kBlock) void unique_fill_kernel(

@@ -179,6 +179,31 @@ def test_unique_relabel_hubs_and_ragged_batches():
                 orc.unique_relabel(seeds, rows, sp, rp, edge_col))
 
 
+@pytest.mark.parametrize("most", [1, 7, 130, 260])
+@pytest.mark.parametrize("B", [2, 63, 64, 65, 66, 300])
+def test_unique_relabel_with_many_batches_in_a_group_of_positions(B, most):
+    """Groups of 4096 positions that hold batches of a few keys, of none, of rows of 64 keys and
+    one off: as many batches as a wavefront has lanes, fewer, and more."""
+    rng = np.random.default_rng(B * 1000 + most)
+    s_sizes, r_sizes = rng.integers(0, most + 1, size=(2, B))
+    s_sizes[rng.random(B) < 0.2] = 0
+    r_sizes[rng.random(B) < 0.2] = 0
+    r_sizes[:2] = 64 - s_sizes[0] % 64, 4 * most + 1
+    r_sizes[s_sizes == 0] = 0  # an edge has a column
+    sp = np.concatenate([[0], np.cumsum(s_sizes)])
+    rp = np.concatenate([[0], np.cumsum(r_sizes)])
+    seeds = rng.integers(0, 40 + most, size=sp[-1])
+    rows = rng.integers(0, 40 + most, size=rp[-1])
+    edge_col = np.concatenate([np.empty(0, np.int64)] + [rng.integers(sp[b], sp[b + 1], size=r_sizes[b])
+                                                         for b in range(B) if r_sizes[b]])
+    assert_same(capi.unique_relabel(T(seeds), T(rows), T(sp), T(rp), T(edge_col)),
+                orc.unique_relabel(seeds, rows, sp, rp, edge_col))
+    for part in (dict(want_row=False, want_col=False), dict(fused=False)):
+        got = capi.unique_relabel(T(seeds), T(rows), T(sp), T(rp), T(edge_col), **part)
+        want = orc.unique_relabel(seeds, rows, sp, rp, edge_col)
+        assert_same(got[:2], want[:2])
+
+
 @pytest.mark.parametrize("B", [1, 3])
 def test_unique_relabel_buckets_beyond_their_regions(B):
     """The partition pass gives every bucket a region of at most 8192 entries.  Ids
