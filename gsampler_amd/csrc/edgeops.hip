@@ -1240,13 +1240,15 @@ constexpr int kFoldRows = 4 * kFoldLanes;
 constexpr int kFoldShares = kBlock / kFoldLanes;
 static_assert(kRangeRows % kFoldRows == 0, "the rows of a work-group share a range");
 
+// range_units: null when every range has `parts` units, one range after the other.
 __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
-    const float* __restrict__ partial, const RangeUnits* __restrict__ range_units,
+    const float* __restrict__ partial, const RangeUnits* __restrict__ range_units, int parts,
     int64_t num_out, float* __restrict__ out) {
   __shared__ double share_sum[kFoldShares][kFoldRows];
   const int share = threadIdx.x / kFoldLanes, lane_row = threadIdx.x % kFoldLanes * 4;
   const int64_t row0 = (int64_t)blockIdx.x * kFoldRows;
-  const RangeUnits ru = range_units[row0 >> kRangeShift];
+  const int range = (int)(row0 >> kRangeShift);
+  const RangeUnits ru = range_units ? range_units[range] : RangeUnits{range * parts, parts};
   const int64_t u1 = (int64_t)ru.base + ru.count;
   // (a unit has the sums of all rows of its range, also of those past num_out)
   const float* p = partial + (row0 & (kRangeRows - 1)) + lane_row;
@@ -1316,8 +1318,112 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
                 rows, values, cells, p.tile_stride, units, unit_total, partial));
   GS_LAUNCH("rowsum_fold", s,
             rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
-                                 s>>>(partial, range_units, num_out, out));
+                                 s>>>(partial, range_units, 0, num_out, out));
   return GS_OK;
+}
+
+// ---------------------------------------- short slices: every range reads every edge
+// Below the edges that are worth a partition, atomics on device memory are dear for
+// another reason: the rows of hubs are in every tile, and adds to one word are
+// executed one after another.  There the ids are few enough for a work-group per range of
+// rows and part of the edges to read the ids of its whole part (from L2) and add the
+// values of its own rows in LDS; the parts are folded as above.
+// 170 K edges of 233 K rows of a power-law graph: 46 us with an atomic a tile and row, now
+// 19 and 4 for the fold; 900 K edges 159 and 75; 8 K edges 18 and 12.  With 10 K rows 43
+// and 15, 177 and 18.  A range more is a pass more over the ids: at 500 K rows (62 ranges)
+// both take the same, at 1 M 57 against 101 on 300 K edges, hence the bound on the ranges.
+constexpr int kScanThreads = 1024;
+constexpr int kScanWaves = kScanThreads / kWave;
+constexpr int kScanRows = 4;    // rows of 64 edges in flight
+constexpr int kScanRun = 1024;  // edges whose columns are looked up together
+// Two work-groups a compute unit (one: 42 and 105 us on 300 K and 900 K edges where two
+// take 35 and 75).
+constexpr int kScanGroups = 512;
+constexpr int kScanMaxRanges = 32;
+constexpr int64_t kScanMinEdges = 2048;
+
+struct RowScanPlan {
+  int64_t ranges = 0, parts = 0, wave_edges = 0;
+  size_t total = 0;
+};
+static RowScanPlan row_scan_plan(int64_t nnz, int64_t num_out) {
+  RowScanPlan p;
+  const int64_t ranges = ceil_div(num_out > 0 ? num_out : 1, kRangeRows);
+  if (nnz < kScanMinEdges || nnz >= kPrivateMinEdges || num_out <= 0 || ranges > kScanMaxRanges)
+    return p;
+  int64_t parts = kScanGroups / ranges;
+  // whole rows of a wavefront, as many for each
+  const int64_t wave_edges = ceil_div(ceil_div(nnz, parts * kScanWaves), kWave) * kWave;
+  parts = ceil_div(nnz, wave_edges * kScanWaves);
+  p.ranges = ranges;
+  p.parts = parts;
+  p.wave_edges = wave_edges;
+  p.total = (size_t)(ranges * parts) * kRangeRows * sizeof(float);
+  return p;
+}
+
+template <typename IdT>
+__global__ __launch_bounds__(kScanThreads, 8) void rowsum_scan_kernel(
+    const IdT* __restrict__ dst_ids, const int64_t* __restrict__ edge_map, int64_t nnz,
+    int64_t num_out, const float* __restrict__ efeat, int ranges, int parts, int64_t wave_edges,
+    float* __restrict__ partial, SliceView view) {
+  __shared__ double acc[kRangeRows];
+  const int t = threadIdx.x, lane = lane_id();
+  const int range = blockIdx.x % ranges, part = blockIdx.x / ranges;
+  const int64_t row0 = (int64_t)range << kRangeShift;
+  const uint32_t rows = (uint32_t)(num_out - row0 < kRangeRows ? num_out - row0 : kRangeRows);
+  for (int j = t; j < kRangeRows; j += kScanThreads) acc[j] = -0.0;
+  __syncthreads();
+  const int64_t first =
+      wave_uniform_first(((int64_t)part * kScanWaves + t / kWave) * wave_edges);
+  const int64_t stop = first + wave_edges < nnz ? first + wave_edges : nnz;
+  for (int64_t run = first; run < stop; run += kScanRun) {
+    const int64_t run_stop = run + kScanRun < stop ? run + kScanRun : stop;
+    const SliceView::Run r = view.run(run, run_stop - 1);
+#pragma unroll 1
+    for (int64_t e0 = run; e0 < run_stop; e0 += kScanRows * kWave) {
+      int64_t place[kScanRows], key[kScanRows];
+#pragma unroll
+      for (int i = 0; i < kScanRows; ++i) {
+        // (a lane, or a row, past the end reads the last edge)
+        const int64_t at = e0 + i * kWave < run_stop ? e0 + i * kWave : run_stop - 1;
+        const int64_t e = at + lane < run_stop ? at + lane : run_stop - 1;
+        if (r.near()) {
+          place[i] = r.place(e);
+          key[i] = r.id_offset(e);
+        } else {
+          int64_t col;
+          place[i] = view.row_position(r, at, e, &col, &key[i]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kScanRows; ++i) key[i] += (int64_t)dst_ids[place[i]] - row0;
+      float val[kScanRows];
+#pragma unroll
+      for (int i = 0; i < kScanRows; ++i) {
+        const bool mine = e0 + i * kWave + lane < run_stop && (uint64_t)key[i] < (uint64_t)rows;
+        if (!mine) key[i] = -1;
+        val[i] = mine ? efeat[edge_map ? edge_map[place[i]] : place[i]] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < kScanRows; ++i) {
+        const double sq = (double)(val[i] * val[i]);
+        // one row for the whole wavefront: adds to one word would be taken one after another
+        const int key0 = __builtin_amdgcn_readfirstlane((int)key[i]);
+        if (key0 >= 0 && __all((int)key[i] == key0)) {
+          double sum = sq;
+#pragma unroll
+          for (int d = kWave / 2; d > 0; d >>= 1) sum += __shfl_down(sum, d, kWave);
+          if (lane == 0) atomicAdd(&acc[key0], sum);
+        } else if (key[i] >= 0) {
+          atomicAdd(&acc[key[i]], sq);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  float* mine = partial + ((int64_t)range * parts + part) * kRangeRows;
+  for (int j = t; j < kRangeRows; j += kScanThreads) mine[j] = (float)acc[j];
 }
 
 bool sums_by_range(int64_t nnz, int64_t num_out) {
@@ -1325,7 +1431,8 @@ bool sums_by_range(int64_t nnz, int64_t num_out) {
 }
 
 size_t sliced_square_sum_bytes(int64_t nnz, int64_t num_out) {
-  return row_range_plan(GS_FMT_COO, nnz, num_out).total;
+  const size_t scan = row_scan_plan(nnz, num_out).total;
+  return scan > 0 ? scan : row_range_plan(GS_FMT_COO, nnz, num_out).total;
 }
 
 int sliced_square_sum(SliceView view, const int64_t* indices, const int32_t* indices32,
@@ -1335,6 +1442,23 @@ int sliced_square_sum(SliceView view, const int64_t* indices, const int32_t* ind
   if (plan.total > 0 && workspace != nullptr && workspace_bytes >= plan.total)
     return row_range_sum(plan, indices, indices32, nullptr, edge_map, nnz, num_out, 1,
                          kOpCopyRhs, nullptr, efeat, out, workspace, s, view);
+  const RowScanPlan scan = row_scan_plan(nnz, num_out);
+  if (scan.total > 0 && workspace != nullptr && workspace_bytes >= scan.total) {
+    float* partial = (float*)workspace;
+    const dim3 grid((unsigned)(scan.ranges * scan.parts));
+#define GS_ROWSUM_SCAN(IDT, IDS)                                                              \
+  GS_LAUNCH("rowsum_scan", s,                                                                 \
+            rowsum_scan_kernel<IDT><<<grid, dim3(kScanThreads), 0, s>>>(                      \
+                IDS, edge_map, nnz, num_out, efeat, (int)scan.ranges, (int)scan.parts,        \
+                scan.wave_edges, partial, view))
+    if (indices32) GS_ROWSUM_SCAN(int32_t, indices32);
+    else GS_ROWSUM_SCAN(int64_t, indices);
+#undef GS_ROWSUM_SCAN
+    GS_LAUNCH("rowsum_fold", s,
+              rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
+                                   s>>>(partial, nullptr, (int)scan.parts, num_out, out));
+    return GS_OK;
+  }
   // short slices: combined per tile in LDS, one atomic per (tile, row present);
   // ids outside [0, num_out) cannot occur for a slice of a checked matrix
   return coo_sum_launch(indices, indices, edge_map, nnz, 1, kOpCopyRhs, nullptr, efeat, out,
@@ -1670,7 +1794,7 @@ int gs_e_square_sum(int format, const int64_t* a, const int64_t* b,
 
 size_t gs_sliced_e_square_sum_workspace_bytes(int64_t slice_nnz, int64_t num_out) {
   if (slice_nnz < 0 || num_out < 0) return 0;
-  return gs::row_range_plan(GS_FMT_COO, slice_nnz, num_out).total;
+  return gs::sliced_square_sum_bytes(slice_nnz, num_out);
 }
 
 int gs_sliced_e_square_sum(const int64_t* indptr, const int64_t* indices,

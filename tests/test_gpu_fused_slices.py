@@ -153,6 +153,47 @@ def test_sliced_e_square_sum_parity(ncol, num_rows, use_workspace):
     assert np.allclose(cpu, want, rtol=1e-5, atol=1e-30)
 
 
+@pytest.mark.parametrize("num_rows", [1, 8192, 8193, 262_144, 262_145])
+@pytest.mark.parametrize("nnz", [2047, 2048, 2049, 17 * 1024, 300_001, (1 << 20) - 1])
+def test_short_sliced_sums_by_ranges_of_rows(nnz, num_rows):
+    """Every range of rows reads every edge: at the borders of ranges and parts, columns of no,
+    one and many edges, a row of half the edges; entries keep what they hold, and -0 where no
+    edge adds.  Squares are not negative, so a sum is off by its roundings alone: the square,
+    a part, the parts' sum and the add, 2^-24 each."""
+    rng = np.random.default_rng(nnz + num_rows)
+    deg = np.concatenate([rng.integers(0, 4, size=200), [nnz // 3, 0, 0, 1, 63, 64, 65]])
+    deg = np.concatenate([deg, [nnz - deg.sum()]])
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    indices = rng.integers(0, num_rows, size=nnz)
+    indices[rng.random(nnz) < 0.5] = num_rows - 1
+    cols = rng.permutation(len(deg))
+    w = rng.random(nnz).astype(np.float32)
+    w[rng.random(nnz) < 0.1] = 0
+    e_map = rng.permutation(nnz)
+    held = np.where(rng.random(num_rows) < 0.5, np.float32(-0.0), np.float32(0.25))
+    want = np.zeros(num_rows)
+    np.add.at(want, indices, (w[e_map] * w[e_map]).astype(np.float64))
+    none = np.bincount(indices, minlength=num_rows) == 0
+    lib, outs = capi.lib(), []
+    need = lib.gs_sliced_e_square_sum_workspace_bytes(nnz, num_rows)
+    assert (need > 0) == (nnz >= 2048 and num_rows <= 262_144)
+    args = [T(indptr), T(indices), T(cols), T(e_map), torch.as_tensor(w, device=DEV)]
+    sub = capi.col_count(args[0], args[2], -1, False)
+    ws = torch.empty(need + 1, dtype=torch.uint8, device=DEV)
+    for narrow in (None, args[1].to(torch.int32)):
+        out = torch.as_tensor(held, device=DEV)
+        capi.check(lib.gs_sliced_e_square_sum(
+            args[0].data_ptr(), args[1].data_ptr(), None if narrow is None else narrow.data_ptr(),
+            args[2].data_ptr(), len(cols), sub.data_ptr(), nnz, args[3].data_ptr(),
+            args[4].data_ptr(), out.data_ptr(), num_rows, ws.data_ptr(), need,
+            torch.cuda.current_stream().cuda_stream))
+        got = out.cpu().numpy()
+        if need:
+            assert np.allclose(got, held + want, rtol=4 * 2.0**-24, atol=0)
+        assert np.array_equal(got[none].view(np.int32), held[none].view(np.int32))
+        assert not np.signbit(got[~none]).any()
+
+
 def test_threads_with_other_columns_on_one_matrix():
     """What an operator holds of a slice stays when another thread's takes its place."""
     rng = np.random.default_rng(21)
