@@ -297,17 +297,27 @@ struct BucketTable {
 
   // fill: a counter per bucket, only used here; also(key) is called for every key,
   // after a barrier
-  template <typename Also>
+  template <int kThreads, typename Also>
   __device__ __forceinline__ void stage(const uint64_t* __restrict__ table, uint32_t capacity,
                                         uint32_t* lds_keys, uint16_t* lds_values,
                                         uint32_t* fill, Also also) {
     keys = reinterpret_cast<const uint4*>(lds_keys);
-    for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberLdsSlots; i += blockDim.x)
+    // (the whole table is asked for first: a slot at a time, each waited for inside its own
+    // round of the loop, took a small work-group a trip to memory per slot of its share)
+    constexpr int kShare = kMemberLdsSlots / kThreads;
+    uint64_t slots[kShare];
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const uint32_t i = j * kThreads + threadIdx.x;
+      slots[j] = i < capacity ? table[i] : kEmptySlot;
+    }
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberLdsSlots; i += kThreads)
       lds_keys[i] = kNoKey;
-    for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberBuckets; i += blockDim.x) fill[i] = 0;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberBuckets; i += kThreads) fill[i] = 0;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < capacity; i += blockDim.x) {
-      const uint64_t t = table[i];
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const uint64_t t = slots[j];
       if (t == kEmptySlot) continue;
       const uint32_t key = (uint32_t)(t >> 32);
       also(key);
@@ -369,7 +379,7 @@ struct MemberShared {
   using Filter = IdFilter<kWords, kInLds ? 2 : kFilterBits>;
   __align__(16) uint32_t keys[kInLds ? kMemberLdsSlots : 4];
   uint16_t values[kInLds ? kMemberLdsSlots : 2];  // fewer than kMemberLdsSlots / 2 ids
-  uint32_t filter[kWords];
+  __align__(16) uint32_t filter[kWords];
   uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
   uint8_t queue_place[kThreads * kMemberWords];
 };
@@ -406,12 +416,23 @@ void member_flag_kernel(
   if (kInLds) {
     static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
     for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
-    buckets.stage(global_table, cap, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
+    buckets.template stage<kThreads>(global_table, cap, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
       const uint32_t h = Filter::hash(key);
       atomicOr(&sh.filter[Filter::word(h)], Filter::bits(h));
     });
   } else if (filtered) {
-    for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = filter[i];
+    constexpr int kVecs = Shared::kWords / 4, kShare = (kVecs + kThreads - 1) / kThreads;
+    uint4 words[kShare];  // (all in flight, as above)
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const int i = j * kThreads + threadIdx.x;
+      words[j] = reinterpret_cast<const uint4*>(filter)[i < kVecs ? i : kVecs - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const int i = j * kThreads + threadIdx.x;
+      if (i < kVecs) reinterpret_cast<uint4*>(sh.filter)[i] = words[j];
+    }
     __syncthreads();
   }
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
