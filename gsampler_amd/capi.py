@@ -83,6 +83,7 @@ SIGNATURES = {
     "gs_first_position": (_int, [_p, _i64, _i64, _p, _p]),
     "gs_csc_col_slice_values": (_int, [_p, _p, _i64, _p, _i64, _p, _i64, _p, _p]),
     "gs_list_labels": (_int, [_p, _i64, _p, _p, _i64, _p, _p, _p, _p, _p, _p]),
+    "gs_list_edge_labels": (_int, [_p, _p, _p, _i64, _i64, _p, _i64, _p, _p, _p, _p]),
     "gs_batch_list_labels": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64,
                                     *([_p] * 10)]),
     "gs_gather_rows": (_int, [_p, _i64, _i64, _p, _i64, _p, _p, _p]),
@@ -532,6 +533,18 @@ def list_labels(seeds, list_ids, first_pos):
                                _ptr(seed_label), _stream()))
     count.arm()
     return frontier[:count.get()], list_label, seed_label
+
+
+def list_edge_labels(row, col, list_label, seed_label, indptr=None):
+    """(list_label[row], seed_label[col]); `indptr` in place of `col` for edges grouped by column."""
+    row, list_label, seed_label = _i64t(row, "row"), _i64t(list_label, "list_label"), _i64t(seed_label, "seed_label")
+    out_row, out_col = torch.empty_like(row), torch.empty_like(row)
+    check(lib().gs_list_edge_labels(_ptr(row), None if col is None else _ptr(_i64t(col, "col")),
+                                    None if indptr is None else _ptr(_i64t(indptr, "indptr")),
+                                    seed_label.numel(), row.numel(), _ptr(list_label),
+                                    list_label.numel(), _ptr(seed_label), _ptr(out_row),
+                                    _ptr(out_col), _stream()))
+    return out_row, out_col
 
 
 def coo_sort(major: torch.Tensor, num_major: int, verify: bool = True):

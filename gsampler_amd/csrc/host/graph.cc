@@ -656,8 +656,15 @@ Graph::GraphRelabel(torch::Tensor col_seeds, torch::Tensor row_ids) {
   if (use_list_labels(col_seeds, row_ids)) {
     ListLabels& l = list_labels_for(col_seeds, row_ids);
     // the gathers are queued before the host waits for the size of the frontier
-    torch::Tensor out_row = l.label_by_local.index_select(0, coo_->row);
-    torch::Tensor out_col = l.seed_label.index_select(0, coo_->col);
+    const int64_t E = coo_->row.numel();
+    torch::Tensor out_row = new_ids(E, coo_->row), out_col = new_ids(E, coo_->row);
+    // (a column slice's edge list is its compressed form, column by column)
+    const bool grouped = csc_ && csc_->indices.is_same(coo_->row) &&
+                         csc_->indptr.numel() == col_seeds.numel() + 1;
+    GS_CALL(gs_list_edge_labels(cptr(coo_->row), cptr(coo_->col),
+                                grouped ? cptr(csc_->indptr) : nullptr, col_seeds.numel(), E,
+                                cptr(l.label_by_local), row_ids.numel(), cptr(l.seed_label),
+                                mptr(out_row), mptr(out_col), cur_stream()));
     return {l.frontier(), out_row, out_col, coo_->e_ids};
   }
   torch::Tensor rows = mapped_rows(coo_->row, row_ids);

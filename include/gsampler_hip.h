@@ -551,6 +551,18 @@ int gs_list_labels(const int64_t* seeds, int64_t num_seeds, const int64_t* list_
                    int64_t* out_list_label, int64_t* out_seed_label,
                    gs_stream_t stream);
 
+/* ----------------------------------------------------------------------
+ * The labels of the edges from those of their rows and columns:
+ *   out_row[e] = list_label[row[e]], out_col[e] = seed_label[column of e]
+ * The column comes from col or, for edges grouped by column, from
+ * indptr[num_cols + 1] (either may be null; indptr is taken where both are given).
+ * Rows are positions in the list [0, num_ids), columns [0, num_cols).
+ * ---------------------------------------------------------------------- */
+int gs_list_edge_labels(const int64_t* row, const int64_t* col, const int64_t* indptr,
+                        int64_t num_cols, int64_t nnz, const int64_t* list_label,
+                        int64_t num_ids, const int64_t* seed_label, int64_t* out_row,
+                        int64_t* out_col, gs_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * The same for a super-batch whose list has a segment per mini-batch
  * (list_ptr[num_batches + 1]): batch b's frontier is the unique of its seeds ++

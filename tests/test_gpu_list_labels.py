@@ -51,6 +51,37 @@ def test_list_labels_match_unique_over_the_edges(S, R, E, mode):
     _check(seeds, list_ids, row, col)
 
 
+@pytest.mark.parametrize("most", [0, 1, 63, 400, 3000])
+@pytest.mark.parametrize("cols", [1, 2, 500])
+def test_edge_labels_by_column_number_and_by_pointer(cols, most):
+    """Runs of 512 edges inside one column, across the border of two and over many, with
+    columns of no edge between; the number of edges no multiple of anything."""
+    rng = np.random.default_rng(cols * 10_000 + most)
+    deg = rng.integers(0, most + 1, size=cols)
+    deg[rng.random(cols) < 0.2] = 0
+    deg[-1] += 7
+    indptr = np.concatenate([[0], np.cumsum(deg)])
+    col = np.repeat(np.arange(cols), deg)
+    row = rng.integers(0, 300, size=col.size)
+    list_label, seed_label = rng.integers(0, 10**6, size=300), rng.integers(0, 10**6, size=cols)
+    for how in (dict(col=T(col)), dict(col=None, indptr=T(indptr))):
+        got = capi.list_edge_labels(T(row), list_label=T(list_label), seed_label=T(seed_label), **how)
+        assert np.array_equal(got[0].cpu().numpy(), list_label[row])
+        assert np.array_equal(got[1].cpu().numpy(), seed_label[col])
+
+
+@pytest.mark.parametrize("R", [1, 4095, 4096, 4097])
+@pytest.mark.parametrize("E", [1, 1024, 16_383, 16_384, 16_385, 100_003])
+def test_first_positions_at_the_borders_of_a_tile(E, R):
+    rng = np.random.default_rng(E + R)
+    row = rng.integers(-2, R + 2, size=E)                    # ids outside are passed over
+    row[-1] = R - 1
+    want = np.full(R, np.iinfo(np.int64).max)
+    ok = (row >= 0) & (row < R)
+    np.minimum.at(want, row[ok], np.flatnonzero(ok))
+    assert np.array_equal(capi.first_position(T(row), R).cpu().numpy(), want)
+
+
 def test_list_labels_large_ids_and_all_used():
     rng = np.random.default_rng(5)
     seeds = rng.integers(2**40, 2**41, size=300)
