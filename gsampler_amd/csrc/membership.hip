@@ -37,7 +37,7 @@ constexpr int64_t kMemberShortChunks = 4096;
 // with four; a row slice of 602 M: 3.34 ms with two, 3.10 with four).
 constexpr int kMemberHugeRun = 4;
 constexpr int64_t kMemberHugeChunks = int64_t(1) << 18;
-constexpr int kMemberThreads = 1024;  // 16 waves share one staged table
+constexpr int kMemberThreads = 1024;  // 16 waves share one table
 // Two of the large work-groups share a compute unit, which takes at most 64 registers
 // a lane.  Runs of eight chunks with a look-up for every row took 90 to 128 registers,
 // one work-group was resident, and a launch of 590 or 890 work-groups left its second
@@ -45,7 +45,7 @@ constexpr int kMemberThreads = 1024;  // 16 waves share one staged table
 // run, as many work-groups as are resident: 90 and 66 (and four chunks a run 64 and 45
 // where two now take 64 and 43).
 constexpr int kMemberWavesPerSimd = 8;
-constexpr int kMemberLdsSlots = 4096;  // tables up to this size are staged in LDS (24 KB)
+constexpr int kMemberLdsSlots = 4096;  // tables up to this size are built in LDS (32 KB)
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 
 // A table too large for LDS is looked up in L2, one request per probe, and the
@@ -184,21 +184,6 @@ __global__ __launch_bounds__(kBlock) void member_insert_kernel(
   member_insert_one(picked, i, table, cap, wide, filter);
 }
 
-// Both in one work-group, for a table small enough (the picked set of a
-// layer-wise sampler): clear, barrier, insert.
-constexpr int kMemberSetupThreads = 1024;
-__global__ __launch_bounds__(kMemberSetupThreads) void member_setup_kernel(
-    const int64_t* __restrict__ picked, int64_t n, uint64_t* table, uint32_t cap,
-    int* __restrict__ wide) {
-  for (uint32_t i = threadIdx.x; i < cap; i += kMemberSetupThreads) table[i] = kEmptySlot;
-  if (threadIdx.x == 0) *wide = 0;
-  // the table is read and written below by other threads of this work-group
-  __threadfence_block();
-  __syncthreads();
-  for (int64_t i = threadIdx.x; i < n; i += kMemberSetupThreads)
-    member_insert_one(picked, i, table, cap, wide, nullptr);
-}
-
 // Empties the table and lowers the wide-id flag.
 __global__ __launch_bounds__(kBlock) void member_clear_kernel(uint64_t* table, int64_t n,
                                                               int* __restrict__ wide,
@@ -278,61 +263,79 @@ struct MemberTable {
 };
 
 // A small table (the picked set of a layer-wise sampler is a few hundred ids) is
-// rebuilt in LDS once per work-group, as buckets of four keys: 64 lanes
+// built in LDS by every work-group for itself, from the ids (a launch that built it in
+// memory for all took 5 to 6 us in front of the flag pass), as buckets of four keys: 64 lanes
 // probing 64 different slots cost the vector cache a tag look-up each, the LDS
 // a few cycles in all.  A look-up reads
 // one bucket (16 bytes, one instruction) and compares four keys, and goes on to
 // the next bucket only from a full one.  With at most two keys per bucket on
 // average nearly every look-up ends at its first bucket, where a linear table
 // makes a wave repeat its probe loop until the longest of its probe runs
-// has ended.  For picked
-// sets whose ids all fit 32 bits (a match of the key is then a match of the id).
+// has ended.
 constexpr int kMemberBuckets = kMemberLdsSlots / 4;
+constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of fewer ids are kept in LDS
 struct BucketTable {
   const uint4* keys;       // [kMemberBuckets] filled from .x on; kNoKey = free
+  const uint32_t* values;  // [kMemberLdsSlots] position in the picked set, by slot
 
   __device__ __forceinline__ static uint32_t home(uint32_t key) {
     return __umulhi(key * 0x9E3779B1u, (uint32_t)kMemberBuckets);
   }
 
   // fill: a counter per bucket, only used here; also(key) is called for every key,
-  // after a barrier
+  // after a barrier.  Returns whether an id does not fit 32 bits (and a key is then no
+  // more than a part of its id), the same for every thread.
   template <int kThreads, typename Also>
-  __device__ __forceinline__ void stage(const uint64_t* __restrict__ table, uint32_t capacity,
-                                        uint32_t* lds_keys, uint16_t* lds_values,
-                                        uint32_t* fill, Also also) {
+  __device__ __forceinline__ bool stage(const int64_t* __restrict__ picked, uint32_t num_picked,
+                                        uint32_t* lds_keys, uint32_t* lds_values, uint32_t* fill,
+                                        Also also) {
     keys = reinterpret_cast<const uint4*>(lds_keys);
-    // (the whole table is asked for first: a slot at a time, each waited for inside its own
-    // round of the loop, took a small work-group a trip to memory per slot of its share)
-    constexpr int kShare = kMemberLdsSlots / kThreads;
-    uint64_t slots[kShare];
+    values = lds_values;
+    constexpr int kShare = kMemberLdsIds / kThreads;
+    uint64_t id[kShare];
+    bool wide = false;
 #pragma unroll
     for (int j = 0; j < kShare; ++j) {
       const uint32_t i = j * kThreads + threadIdx.x;
-      slots[j] = i < capacity ? table[i] : kEmptySlot;
+      id[j] = i < num_picked ? (uint64_t)picked[i] : 0;
     }
     for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberLdsSlots; i += kThreads)
       lds_keys[i] = kNoKey;
     for (uint32_t i = threadIdx.x; i < (uint32_t)kMemberBuckets; i += kThreads) fill[i] = 0;
-    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) wide |= id[j] > kMaxPackedKey;
+    wide = __syncthreads_or(wide) != 0;
+    uint32_t slot[kShare];
 #pragma unroll
     for (int j = 0; j < kShare; ++j) {
-      const uint64_t t = slots[j];
-      if (t == kEmptySlot) continue;
-      const uint32_t key = (uint32_t)(t >> 32);
+      const uint32_t i = j * kThreads + threadIdx.x;
+      if (i >= num_picked) continue;
+      const uint32_t key = member_tag(id[j]);
       also(key);
       uint32_t b = home(key);
       for (int tries = 0; tries < kMemberBuckets; ++tries) {  // fewer keys than slots: ends early
         const uint32_t at = atomicAdd(&fill[b], 1u);
         if (at < 4u) {
-          lds_keys[b * 4 + at] = key;
-          lds_values[b * 4 + at] = (uint16_t)t;
+          slot[j] = b * 4 + at;
+          lds_keys[slot[j]] = key;
+          lds_values[slot[j]] = i;
           break;
         }
         b = (b + 1) & (kMemberBuckets - 1);
       }
     }
     __syncthreads();
+    if (wide) return true;
+    // a repeated id: a look-up ends at the first of its slots, whose position is the smallest
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const uint32_t i = j * kThreads + threadIdx.x;
+      if (i >= num_picked) continue;
+      const uint32_t first = find(member_tag(id[j]));
+      if (first != slot[j]) atomicMin(&lds_values[first], i);
+    }
+    __syncthreads();
+    return false;
   }
 
   // Where a key sits, kMemberLdsSlots when it is absent (or kNoKey).
@@ -347,6 +350,26 @@ struct BucketTable {
       b = (b + 1) & (kMemberBuckets - 1);
     }
     return kMemberLdsSlots;
+  }
+
+  // The smallest position of an id among ids that may not fit 32 bits, kNoKey when it is
+  // absent: every match of the keys is confirmed against the picked id.
+  __device__ __forceinline__ uint32_t find_confirmed(uint64_t id,
+                                                     const int64_t* __restrict__ picked) const {
+    const uint32_t tag = member_tag(id);
+    uint32_t b = home(tag), best = kNoKey;
+    for (int rounds = 0; rounds < kMemberBuckets; ++rounds) {
+      const uint32_t* k = reinterpret_cast<const uint32_t*>(keys + b);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (k[e] != tag) continue;
+        const uint32_t at = values[b * 4 + e];
+        if (at < best && (uint64_t)picked[at] == id) best = at;
+      }
+      if (k[3] == kNoKey) break;
+      b = (b + 1) & (kMemberBuckets - 1);
+    }
+    return best;
   }
 };
 
@@ -378,7 +401,7 @@ struct MemberShared {
   static constexpr int kWords = !kInLds ? kFilterWords : kThreads == kMemberThreads ? 4096 : 2048;
   using Filter = IdFilter<kWords, kInLds ? 2 : kFilterBits>;
   __align__(16) uint32_t keys[kInLds ? kMemberLdsSlots : 4];
-  uint16_t values[kInLds ? kMemberLdsSlots : 2];  // fewer than kMemberLdsSlots / 2 ids
+  uint32_t values[kInLds ? kMemberLdsSlots : 4];
   __align__(16) uint32_t filter[kWords];
   uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
   uint8_t queue_place[kThreads * kMemberWords];
@@ -402,25 +425,29 @@ __global__ __launch_bounds__(kThreads, kThreads == kMemberThreads ? kMemberWaves
 void member_flag_kernel(
     const IdT* __restrict__ ids, int64_t nnz,
     const uint64_t* __restrict__ global_table, uint32_t cap,
-    const int64_t* __restrict__ picked, const int* __restrict__ wide_flag,
+    const int64_t* __restrict__ picked, uint32_t num_picked, const int* __restrict__ wide_flag,
     int64_t* __restrict__ chunk_count,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
     const uint32_t* __restrict__ filter, SliceView view) {
   using Shared = MemberShared<kInLds, kThreads>;
   using Filter = typename Shared::Filter;
   __shared__ Shared sh;
-  const bool wide = *wide_flag != 0;  // the same for every thread of the launch
   const bool filtered = kInLds || filter != nullptr;
   const MemberTable table{global_table, cap};
   BucketTable buckets;
+  bool wide;  // the same for every thread of the launch
   if (kInLds) {
     static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
     for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
-    buckets.template stage<kThreads>(global_table, cap, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
-      const uint32_t h = Filter::hash(key);
-      atomicOr(&sh.filter[Filter::word(h)], Filter::bits(h));
-    });
-  } else if (filtered) {
+    wide = buckets.template stage<kThreads>(
+        picked, num_picked, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
+          const uint32_t h = Filter::hash(key);
+          atomicOr(&sh.filter[Filter::word(h)], Filter::bits(h));
+        });
+  } else {
+    wide = *wide_flag != 0;
+  }
+  if (!kInLds && filtered) {
     constexpr int kVecs = Shared::kWords / 4, kShare = (kVecs + kThreads - 1) / kThreads;
     uint4 words[kShare];  // (all in flight, as above)
 #pragma unroll
@@ -541,8 +568,14 @@ void member_flag_kernel(
           bool in;
           const uint64_t id = id_of(chunk * kBlock + j * kWave, &in);
           const bool may = in && (!filtered || Filter::passes(sh.filter, member_tag(id)));
-          const uint32_t slot = may ? table.find_confirmed(id, picked) : cap;
-          keep(chunk, slot < cap, slot < cap ? table.value_at(slot) : 0u, j * kWave + lane);
+          uint32_t value = kNoKey;
+          if (may && kInLds) {
+            value = buckets.find_confirmed(id, picked);
+          } else if (may) {
+            const uint32_t slot = table.find_confirmed(id, picked);
+            if (slot < cap) value = table.value_at(slot);
+          }
+          keep(chunk, value != kNoKey, value, j * kWave + lane);
         }
         finish_chunk(chunk);
       }
@@ -761,13 +794,9 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   }
   hipStream_t s = as_stream(stream);
   const uint32_t cap = (uint32_t)member_table_slots(num_picked);
-  const bool in_lds = cap <= (uint64_t)kMemberLdsSlots;
+  const bool in_lds = num_picked < kMemberLdsIds;
   uint32_t* filter = !in_lds && num_picked <= kFilterMaxIds ? w.filter : nullptr;
-  if (in_lds) {
-    GS_LAUNCH("member_insert", s,
-              member_setup_kernel<<<dim3(1), dim3(kMemberSetupThreads), 0, s>>>(
-                  picked, num_picked, w.table, cap, w.wide));
-  } else {
+  if (!in_lds) {
     GS_LAUNCH("member_clear", s,
               member_clear_kernel<<<dim3((unsigned)ceil_div((int64_t)cap, kBlock * 4)),
                                     dim3(kBlock), 0, s>>>(w.table, (int64_t)cap, w.wide, filter));
@@ -789,7 +818,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
-                IDS, nnz, w.table, cap, picked, w.wide, w.chunk_off, w.staged,       \
+                IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, w.staged,       \
                 w.staged_pos, filter, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
