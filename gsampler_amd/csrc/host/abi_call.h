@@ -40,8 +40,8 @@ inline int64_t cache_epoch() { return cache_epoch_counter().load(std::memory_ord
 inline void invalidate_caches() { cache_epoch_counter().fetch_add(1); }
 
 // Whether a loaded matrix may keep tables made from its ids: an int32 copy (4 bytes
-// per edge for half the bytes behind a pick) and the hop table of its walks (8 bytes
-// per edge, matrices of up to 2^24 edges).
+// per edge for half the bytes behind a pick), the hop table of its walks (8 bytes
+// per edge, matrices of up to 2^24 edges) and the marks of its columns (32 bytes each).
 inline std::atomic<bool>& narrow_ids_allowed() {
   static std::atomic<bool> on{true};
   return on;
