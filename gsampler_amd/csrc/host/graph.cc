@@ -657,6 +657,12 @@ Graph::GraphRelabel(torch::Tensor col_seeds, torch::Tensor row_ids) {
     ListLabels& l = list_labels_for(col_seeds, row_ids);
     // the gathers are queued before the host waits for the size of the frontier
     const int64_t E = coo_->row.numel();
+    // (lists shorter than the matrix: an edge may point past one, which the gathers refuse)
+    if (row_ids.numel() < num_rows_ || col_seeds.numel() < num_cols_) {
+      torch::Tensor out_row = l.label_by_local.index_select(0, coo_->row);
+      torch::Tensor out_col = l.seed_label.index_select(0, coo_->col);
+      return {l.frontier(), out_row, out_col, coo_->e_ids};
+    }
     torch::Tensor out_row = new_ids(E, coo_->row), out_col = new_ids(E, coo_->row);
     // (a column slice's edge list is its compressed form, column by column)
     const bool grouped = csc_ && csc_->indices.is_same(coo_->row) &&

@@ -70,6 +70,28 @@ def test_edge_labels_by_column_number_and_by_pointer(cols, most):
         assert np.array_equal(got[1].cpu().numpy(), seed_label[col])
 
 
+@pytest.mark.parametrize("short_rows,short_cols", [(0, 0), (3, 0), (0, 2), (3, 2)])
+def test_lists_shorter_than_the_matrix(short_rows, short_cols):
+    """Seeds and row ids may be fewer than the columns and the rows of the matrix as long as
+    no edge needs the missing ones; the labels are the same by either way to them."""
+    rng = np.random.default_rng(short_rows * 10 + short_cols)
+    R, C = 60, 40
+    indptr, indices = random_csc(rng, C, R - short_rows, 4000)
+    indptr[C - short_cols:] = indptr[C - short_cols]
+    indices = indices[:indptr[-1]]
+    g = gs.Graph(R, C)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    seeds = rng.permutation(1000)[:C - short_cols]
+    row_ids = rng.permutation(1000)[:R - short_rows]
+    assert indices.size >= 8 * (seeds.size + row_ids.size)
+    col = np.repeat(np.arange(C), np.diff(indptr))
+    want = orc.unique_relabel(seeds, row_ids[indices], edge_col=col)
+    frontier, row, col, _ = g._CAPI_GraphRelabel(T(seeds), T(row_ids))
+    assert np.array_equal(frontier.cpu().numpy(), want[0])
+    assert np.array_equal(row.cpu().numpy(), want[2])
+    assert np.array_equal(col.cpu().numpy(), want[3])
+
+
 @pytest.mark.parametrize("R", [1, 4095, 4096, 4097])
 @pytest.mark.parametrize("E", [1, 1024, 16_383, 16_384, 16_385, 100_003])
 def test_first_positions_at_the_borders_of_a_tile(E, R):
