@@ -697,6 +697,13 @@ def _writes_in_place(node: fx.Node) -> bool:
             or "out" in node.kwargs or node.kwargs.get("inplace") is True)
 
 
+def _written_between(order: Dict[fx.Node, int], nodes) -> bool:
+    """Whether a node of the sampler's own may write from the first of `nodes` to the last:
+    what they read must then be read where they stand."""
+    first, last = min(order[n] for n in nodes), max(order[n] for n in nodes)
+    return any(first < at < last and _writes_in_place(n) for n, at in order.items())
+
+
 def _call(node, *targets) -> bool:
     return isinstance(node, fx.Node) and node.op == "call_function" and node.target in targets
 
@@ -822,8 +829,9 @@ def compute_edge_scores(copy: fx.Graph) -> None:
 def normalise_columns(copy: fx.Graph) -> None:
     """In a copy of a graph: q / s[column] with s = sum of q over columns, where q = e /
     r[row], or an edge value itself, is used for nothing else; and the gather that e comes
-    from, if only this reads it  => one _normalised."""
+    from, if only this reads it  => one _normalised, in the last one's place."""
     from ..ops.fused_op import _normalised
+    order = {n: i for i, n in enumerate(copy.nodes)}
     written = []
     for out in list(copy.nodes):
         last = _sddmm_of(out) if out.users else None
@@ -846,15 +854,21 @@ def normalise_columns(copy: fx.Graph) -> None:
         readers = {spmm, before_total, before_last}
         first = _sddmm_of(q)
         values, divisor, formats = q, None, (last[5], spmm.args[9], last[5])
+        replaced = [before_total, spmm, before_last, last[6], out]
         if (first is not None and first[1] == "div" and first[4] == [1, 0] and first[0] is g
                 and set(q.users) == readers and isinstance(first[2], fx.Node)):
             values, divisor, formats = first[2], first[3], (first[5], spmm.args[9], last[5])
             readers = {n.args[0] for n in first[6].all_input_nodes if _call(n, operator.getitem)
                        and _is_wrapped(n.args[0], "_before_sddmm")}
-            written.append(first[6])
+            replaced += [first[6], *readers]
         select = None
         if _is_wrapped(values, "data_index") and set(values.users) == readers:
+            replaced.append(values)
             values, select = values.args
+        if _written_between(order, replaced):
+            continue
+        if divisor is not None:
+            written.append(first[6])
         with copy.inserting_before(out):
             new = copy.call_function(_normalised, args=(g, values, select, divisor, formats))
         out.replace_all_uses_with(new)
@@ -867,7 +881,8 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
     """In a copy of a graph: s = A._CAPI_BatchColSlicing(seeds, ptr, True) whose matrix s[0]
     is only asked for its rows and shape, summed once by _CAPI_FusedESquareSum(copy_rhs, sum,
     e = w[s[1]]) onto rows, and row-sliced by what _CAPI_BatchListSampling[WithProbs] picked of
-    those rows, and whose edge index s[1] only gathers edge data that feeds those operators
+    those rows, whose edge index s[1] only gathers edge data that feeds those operators, and
+    nothing written to from there to the row slice
         => _encoded_square_sums(A, seeds, ptr, w) and _encoded_row_slice, whose index
            addresses A's edges."""
     from ..ops.fused_op import _encoded_row_slice, _encoded_square_sums
@@ -937,7 +952,7 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
                                       "_CAPI_BatchListSamplingWithProbs")
                     and picked.args[0].args and picked.args[0].args[-1] in row_ptrs):
                 ok = False            # rows that may not be the slice's
-        if not ok:
+        if not ok or _written_between(order, [slicing, *gathered, total, *row_slices, *regather]):
             continue
         with copy.inserting_before(slicing):
             found = copy.call_function(_encoded_square_sums, args=(parent, seeds, ptr, total.args[4].args[0],

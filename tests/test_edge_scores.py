@@ -225,6 +225,37 @@ def test_what_is_summed_in_place(options, kernel):
     assert t.count(fused_op._encoded_row_slice) == kernel and ("_CAPI_BatchRowSlicing" in t) != kernel
 
 
+def written_between(A, seeds, ptr, w, scale):
+    """w changes after the slice has been made and before its rows are picked."""
+    A.edata["w"] = w
+    sub = A[:, seeds::ptr]
+    sub.edata["p"] = sub.edata["w"] ** 2
+    prob = sub.sum("p", axis=1)
+    _, rows_ptr = sub.all_rows()
+    changed = w.mul_(scale)
+    part, _ = sub.collective_sampling(3, prob, rows_ptr, False)
+    return part.edata["w"], changed
+
+
+def written_after(A, seeds, ptr, w, scale):
+    A.edata["w"] = w
+    return layer(A, seeds, ptr) + (w.mul_(scale),)
+
+
+def order_of(compiled, *targets):
+    return [n.target for n in compiled._run.__self__.graph.nodes if n.target in targets]
+
+
+@pytest.mark.parametrize("func,kernel", [(written_between, False), (written_after, True)])
+def test_slice_that_is_written_to_before_its_rows_are_read(func, kernel):
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(gs.Matrix(gs.Graph(10, 10)), True)
+    c = gs.jit.compile(func=func, args=(bm, torch.arange(6), torch.tensor([0, 3, 6]), torch.rand(7),
+                                        torch.rand(7)))
+    assert order_of(c, fused_op._encoded_row_slice, "_CAPI_BatchRowSlicing", "mul_") == (
+        [fused_op._encoded_row_slice, "mul_"] if kernel else ["mul_", "_CAPI_BatchRowSlicing"])
+
+
 # ------------------------------------------------------------ columns normalised
 def normalised(A, seeds, divisor):
     sub = A[:, seeds].div("w", divisor, axis=1)
@@ -252,8 +283,19 @@ def by_rows(A, seeds, divisor):
     return q.div("w", q.sum("w", axis=1), axis=1).edata["w"]
 
 
+def divisor_written(A, seeds, divisor):
+    q = A[:, seeds].div("w", divisor, axis=1)
+    changed = divisor.mul_(torch.arange(1.0, 1.0 + divisor.numel(), device=divisor.device))
+    return q.div("w", q.sum("w", axis=0), axis=0).edata["w"], changed
+
+
+def divisor_written_after(A, seeds, divisor):
+    q = A[:, seeds].div("w", divisor, axis=1)
+    return q.div("w", q.sum("w", axis=0), axis=0).edata["w"], divisor.mul_(2.0)
+
+
 @pytest.mark.parametrize("func,kernels,divisions", [
-    (normalised, 1, 0), (by_columns_only, 1, 0), (quotient_kept, 1, 1), (sums_kept, 0, 2), (by_rows, 0, 2)])
+    (divisor_written, 0, 2), (divisor_written_after, 1, 0), (normalised, 1, 0), (by_columns_only, 1, 0), (quotient_kept, 1, 1), (sums_kept, 0, 2), (by_rows, 0, 2)])
 def test_what_is_normalised_in_one(func, kernels, divisions):
     m = gs.Matrix(gs.Graph(10, 10))
     m.edata["w"] = torch.rand(7)
