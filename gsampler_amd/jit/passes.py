@@ -689,12 +689,27 @@ IN_PLACE_FUNCTIONS = {getattr(operator, name) for name in (
 
 
 def _writes_in_place(node: fx.Node) -> bool:
-    """Whether a node of the sampler's own may change a tensor that others read."""
+    """Whether a node of the sampler's own may change a tensor that others read.  Of the
+    functions only those of torch, Python's operators and this package are known; any other
+    (one given to torch.fx.wrap) may write."""
     if node.op not in ("call_method", "call_function"):
         return node.op == "call_module"
-    name = node.target if node.op == "call_method" else getattr(node.target, "__name__", "")
-    return (name.endswith("_") and not name.endswith("__") or node.target in IN_PLACE_FUNCTIONS
-            or "out" in node.kwargs or node.kwargs.get("inplace") is True)
+    if "out" in node.kwargs or node.kwargs.get("inplace") is True:
+        return True
+    if node.op == "call_method":
+        return node.target.endswith("_") and not node.target.endswith("__")
+    if node.target in IN_PLACE_FUNCTIONS:
+        return True
+    if isinstance(node.target, torch._ops.OpOverload):
+        return node.target._schema.is_mutable
+    if isinstance(node.target, torch._ops.OpOverloadPacket):
+        schemas = [getattr(node.target, name)._schema for name in node.target.overloads()]
+        return node.target.__name__.endswith("_") or all(s.is_mutable for s in schemas)
+    name, module = getattr(node.target, "__name__", ""), getattr(node.target, "__module__", None) or ""
+    known = (module.partition(".")[0] in ("torch", "_operator", "builtins", "math", __name__.partition(".")[0])
+             or node.target in (_library.native.sample_layers, _library.native.batch_sample_layers)
+             or getattr(torch, name, None) is node.target)
+    return not known or name.endswith("_") and not name.endswith("__")
 
 
 def _written_between(order: Dict[fx.Node, int], nodes) -> bool:

@@ -1,6 +1,7 @@
 """Edge scores of attention samplers: what the compiled graph runs in one kernel, what it leaves
 to the operators it was written with, and that the two give the same bits -- the samples drawn by
 the scores depend on every one of them."""
+import math
 import operator
 
 import numpy as np
@@ -292,6 +293,49 @@ def divisor_written(A, seeds, divisor):
 def divisor_written_after(A, seeds, divisor):
     q = A[:, seeds].div("w", divisor, axis=1)
     return q.div("w", q.sum("w", axis=0), axis=0).edata["w"], divisor.mul_(2.0)
+
+
+@torch.fx.wrap
+def scaled_by_ten(x):
+    return x.mul_(10.0)
+
+
+def by_a_function(x):
+    return scaled_by_ten(x)
+
+
+def by_an_overload(x):
+    return torch.ops.aten.mul_.Scalar(x, 10.0)
+
+
+def by_a_packet(x):
+    return torch.ops.aten.mul_(x, 10.0)
+
+
+def by_an_option(x):
+    return F.relu(x, True)
+
+
+def by_an_output(x):
+    return torch.add(x, 1.0, out=x)
+
+
+def not_at_all(x):
+    return torch.ops.aten.mul(x, 10.0) + F.relu(x) - torch.sum(x, dim=0) * math.sqrt(2.0)
+
+
+@pytest.mark.parametrize("write", [by_a_function, by_an_overload, by_a_packet, by_an_option, by_an_output,
+                                   not_at_all])
+def test_writes_however_they_are_spelt(write):
+    def sampler(A, seeds, divisor):
+        q = A[:, seeds].div("w", divisor, axis=1)
+        changed = write(divisor)
+        return q.div("w", q.sum("w", axis=0), axis=0).edata["w"], changed
+
+    m = gs.Matrix(gs.Graph(10, 10))
+    m.edata["w"] = torch.rand(7)
+    t = ran(gs.jit.compile(func=sampler, args=(m, torch.arange(3), torch.rand(10))))
+    assert (fused_op._normalised in t) == (write is not_at_all)
 
 
 @pytest.mark.parametrize("func,kernels,divisions", [
