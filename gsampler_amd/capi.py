@@ -92,7 +92,7 @@ SIGNATURES = {
     "gs_coo_sort": (_int, [_p, _i64, _i64, _p, _p, _p, _sz, _p]),
     "gs_sddmm": (_int, [_int, _p, _p, _i64, _i64, _p, _int, _int, _p, _p, _p, _int, _int,
                         _i64, _i64, _i64, _i64, _p, _p, _p]),
-    "gs_normalise_columns": (_int, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p]),
+    "gs_normalise_columns": (_int, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _p]),
     "gs_edge_score": (_int, [_int, _p, _p, _i64, _i64, _p, _p, _int, _i64, _p, _int, C.c_float,
                              _p, _p]),
     "gs_fused_u_op_v": (_int, [_int, _p, _p, _i64, _i64, _p, _int, _int, _p, _p, _p, _p, _p,

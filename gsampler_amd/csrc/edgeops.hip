@@ -677,8 +677,9 @@ __global__ __launch_bounds__(kBlock) void normalise_clear_kernel(double* sums, i
 template <bool kSelect, bool kDivide>
 __global__ __launch_bounds__(kBlock) void normalise_sum_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols, const int64_t* __restrict__ rows,
-    int64_t nnz, const float* __restrict__ values, const int64_t* __restrict__ select,
-    const float* __restrict__ row_divisor, double* __restrict__ sums, float* __restrict__ out) {
+    int64_t nnz, const float* __restrict__ values, int64_t num_values,
+    const int64_t* __restrict__ select, const float* __restrict__ row_divisor,
+    double* __restrict__ sums, float* __restrict__ out) {
   __shared__ double acc[kSumSegs];
   __shared__ int32_t begins[kSumSegs];
   const int64_t tile0 = (int64_t)blockIdx.x * kSumTile;
@@ -691,7 +692,13 @@ __global__ __launch_bounds__(kBlock) void normalise_sum_kernel(
     row[i] = kDivide ? rows[e] : 0;
   }
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i) v[i] = values[at[i]];
+  for (int i = 0; i < kSumItems; ++i)
+    v[i] = values[!kSelect || (uint64_t)at[i] < (uint64_t)num_values ? at[i] : 0];
+  if (kSelect) {  // (edge data may be shorter than the edges that `select` names)
+#pragma unroll
+    for (int i = 0; i < kSumItems; ++i)
+      if ((uint64_t)at[i] >= (uint64_t)num_values) v[i] = 0.f;
+  }
   if (kDivide) {
 #pragma unroll
     for (int i = 0; i < kSumItems; ++i) v[i] /= row_divisor[row[i]];
@@ -1681,14 +1688,16 @@ int gs_edge_score(int format, const int64_t* a, const int64_t* b, int64_t num_ma
 }
 
 int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t* rows,
-                         int64_t nnz, const float* values, const int64_t* select,
-                         const float* row_divisor, double* sums, float* out,
+                         int64_t nnz, const float* values, int64_t num_values,
+                         const int64_t* select, const float* row_divisor, double* sums, float* out,
                          gs_stream_t stream) {
   using namespace gs;
   GS_REQUIRE(num_cols >= 0 && nnz >= 0, "normalise_columns: negative size");
   if (nnz == 0) return GS_OK;
   GS_REQUIRE(num_cols > 0 && indptr && values && sums && out && (rows || !row_divisor),
              "normalise_columns: null pointer");
+  GS_REQUIRE(num_values >= 1 && (select || num_values >= nnz), "normalise_columns: %lld values",
+             (long long)num_values);
   hipStream_t s = as_stream(stream);
   const dim3 grid((unsigned)ceil_div(nnz, (int64_t)kSumTile));
   GS_LAUNCH("normalise_clear", s,
@@ -1697,7 +1706,7 @@ int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t*
 #define GS_NORMALISE_SUM(SELECT, DIVIDE)                                                     \
   GS_LAUNCH("normalise_sum", s,                                                              \
             (normalise_sum_kernel<SELECT, DIVIDE>)<<<grid, dim3(kBlock), 0, s>>>(            \
-                indptr, num_cols, rows, nnz, values, select, row_divisor, sums, out))
+                indptr, num_cols, rows, nnz, values, num_values, select, row_divisor, sums, out))
   if (select && row_divisor) GS_NORMALISE_SUM(true, true);
   else if (select) GS_NORMALISE_SUM(true, false);
   else if (row_divisor) GS_NORMALISE_SUM(false, true);

@@ -254,7 +254,7 @@ c10::optional<torch::Tensor> Graph::NormaliseColumns(torch::Tensor values,
     return {};
   // (the operators this stands for write into arrays of their own, without gradients)
   if (!plain_values(values, false) || values.dim() != 1 || !values.is_contiguous() ||
-      (!select.has_value() && values.size(0) != num_edges_))
+      values.size(0) == 0 || (!select.has_value() && values.size(0) != num_edges_))
     return {};
   if (select.has_value() &&
       (!select->is_cuda() || select->scalar_type() != torch::kInt64 || select->dim() != 1 ||
@@ -269,7 +269,8 @@ c10::optional<torch::Tensor> Graph::NormaliseColumns(torch::Tensor values,
   torch::Tensor out = torch::empty({num_edges_}, values.options().requires_grad(false));
   torch::Tensor sums = torch::empty({num_cols_}, out.options().dtype(torch::kFloat64));
   GS_CALL(gs_normalise_columns(cptr(csc_->indptr), num_cols_, cptr(csc_->indices), num_edges_,
-                               values.data_ptr<float>(), select.has_value() ? cptr(*select) : nullptr,
+                               values.data_ptr<float>(), values.size(0),
+                               select.has_value() ? cptr(*select) : nullptr,
                                row_divisor.has_value() ? row_divisor->data_ptr<float>() : nullptr,
                                sums.data_ptr<double>(), out.data_ptr<float>(), cur_stream()));
   return out;

@@ -827,8 +827,9 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
  *   the order of additions is fixed (edgeops.hip).
  * gs_normalise_columns: out[e] = q[e] / (sum of q over e's column) with q[e] =
  *   values[select[e]] / row_divisor[rows[e]], select (identity) and row_divisor (ones)
- *   nullable, fp32; edges in column order, sums[num_cols] is scratch that ends up with
- *   the columns' sums.  q is rounded, sums are of 64 bits and rounded before they divide.
+ *   nullable, fp32; a place outside the num_values values reads 0, as gs_gather_rows has
+ *   it.  Edges in column order, sums[num_cols] is scratch that ends up with the columns'
+ *   sums.  q is rounded, sums are of 64 bits and rounded before they divide.
  * gs_spmm: out[dst] = reduce(out[dst], op(u[src], e[eid])), fp32.  Outputs
  *   are accumulators: the caller zero-fills them (python/gs/ops/spmm.py:56).
  *   COO: u_target 0 reduces onto columns, 2 onto rows (atomics).  Compressed:
@@ -862,8 +863,8 @@ int gs_edge_score(int format, const int64_t* a, const int64_t* b, int64_t num_ma
                   int num_terms, int64_t feature_len, const float* weights, int positive_part,
                   float shift, float* out, gs_stream_t stream);
 int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t* rows,
-                         int64_t nnz, const float* values, const int64_t* select,
-                         const float* row_divisor, double* sums, float* out,
+                         int64_t nnz, const float* values, int64_t num_values,
+                         const int64_t* select, const float* row_divisor, double* sums, float* out,
                          gs_stream_t stream);
 int gs_fused_u_op_v(int format, const int64_t* a, const int64_t* b,
                     int64_t num_major, int64_t nnz, const int64_t* edge_map,

@@ -381,6 +381,25 @@ def test_normalised_columns_equal_eager(func, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("func", [normalised, by_columns_only])
+@pytest.mark.parametrize("length", [0, 1, 2000])
+def test_edge_data_shorter_than_the_edges(func, length):
+    """Edges past its end have the value 0, as the gather gives it."""
+    m, seeds = world(), torch.arange(0, 900, 3, device=DEV)
+    divisor = torch.rand(m.num_rows(), device=DEV) + 0.5
+    m.edata["w"] = m.edata["w"][:length].clone()
+    compiled = gs.jit.compile(func=func, args=(m, seeds, divisor))
+    if length == 0:
+        for f in (func, compiled):
+            with pytest.raises(RuntimeError, match="gather_rows"):
+                f(m, seeds, divisor)
+        return
+    want, got = func(m, seeds, divisor), compiled(m, seeds, divisor)
+    for a, b in zip(*((x if isinstance(x, tuple) else (x,)) for x in (want, got))):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=0, equal_nan=True)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("degrees", [[1], [2048], [2049], [2047, 1, 2048, 0, 5], [0] * 3000 + [10] + [0] * 2500 + [7],
                                      [3] * 5000, [1] * 2048 + [4100] + [0, 1] * 40, [100_000, 1]])
 @pytest.mark.parametrize("select", [False, True])
