@@ -18,6 +18,8 @@
 // large graph, an id encoded as id + batch * num_rows) the insert pass raises a
 // flag, and every match of the 32-bit halves is then confirmed against the
 // picked id itself.
+#include <algorithm>
+
 #include "common.h"
 #include "hashtable.h"
 #include "scan.h"
@@ -56,7 +58,6 @@ constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups o
 // twenty passes).  Only ids that pass go on to the table.
 constexpr int kFilterWords = 14336;            // 56 KB of LDS, two work-groups a compute unit
 constexpr int kFilterBits = 3;
-constexpr int kResidentPerCu = 2;              // work-groups of 1024 threads that fit a compute unit
 constexpr int64_t kFilterMaxIds = 131072;      // beyond: too many bits set to be worth a look
 
 // Ids that may be picked, by a word of 32 bits per id group in LDS: an id whose bits
@@ -406,6 +407,11 @@ struct MemberShared {
   uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
   uint8_t queue_place[kThreads * kMemberWords];
 };
+// Work-groups that a compute unit holds, with 160 KB of LDS and 2048 threads: two of 1024
+// threads, of kBlock threads three with the table in LDS and two with the filter.
+template <bool kInLds, int kThreads>
+constexpr int kMemberResident = std::min(160 * 1024 / (int)sizeof(MemberShared<kInLds, kThreads>),
+                                         2048 / kThreads);
 
 // Whether a row of 64 edges holds picked ids is told by the filter, a word of LDS and
 // eight instructions an edge; the edges that pass are packed into the wave's queue, and
@@ -809,11 +815,16 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
     const bool small = nnz < kMemberSmallEdges;
     const int threads = small ? kBlock : kMemberThreads;
     const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberLongRun;
+    // a large list, or work-groups that stage a table or a filter: as many of them as are
+    // resident, each staging once and striding over its runs (row slices of 1 M and 8 M edges,
+    // us, with a small work-group for every 2048 edges and with these: 300 picks 21 and 18, 42
+    // and 28; 2047 picks 34 and 26, 79 and 39; 5000 picks 34 and 33, 65 and 60)
+    const int per_cu =
+        in_lds ? (small ? kMemberResident<true, kBlock> : kMemberResident<true, kMemberThreads>)
+               : (small ? kMemberResident<false, kBlock> : kMemberResident<false, kMemberThreads>);
+    const int64_t resident = (int64_t)per_cu * num_compute_units();
     int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
-    // a large list, or work-groups that stage the 64 KB filter: as many of them as are
-    // resident, each staging its tables once and striding over its runs
-    const int64_t resident = (int64_t)(kResidentPerCu * kMemberThreads / threads) * num_compute_units();
-    if ((filter || !small) && blocks > resident) blocks = resident;
+    if ((in_lds || filter || !small) && blocks > resident) blocks = resident;
     const dim3 grid((unsigned)blocks);
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
