@@ -114,6 +114,45 @@ def test_minor_slice_with_ids_beyond_32_bits(npick):
          orc.minor_slice(ids, narrow, indptr=indptr))
 
 
+@pytest.mark.parametrize("distinct", [1, 16, 700])
+@pytest.mark.parametrize("wide", [False, True])
+def test_minor_slice_by_many_copies_of_few_ids(distinct, wide):
+    """The longest list whose table is built in LDS, most of it repeats: the smallest position
+    wins.  wide: four ids share each low half."""
+    rng = np.random.default_rng(distinct)
+    ids = rng.integers(0, 2000, size=70_001)
+    pool = rng.permutation(2000)[:distinct]
+    if wide:
+        ids = ids + rng.integers(0, 4, size=ids.size) * 2**32
+        pool = pool + rng.integers(0, 4, size=distinct) * 2**32
+        pool[0] += 2**33
+    picked = rng.choice(pool, size=2047)
+    indptr = np.sort(rng.integers(0, ids.size + 1, size=901))
+    indptr[0], indptr[-1] = 0, ids.size
+    same(capi.minor_slice(T(ids), T(picked), indptr=T(indptr)),
+         orc.minor_slice(ids, picked, indptr=indptr))
+
+
+def test_copies_of_one_id_cost_no_more_than_as_many_ids():
+    """A table with a slot for every copy walks n / 4 full buckets for the n-th of them."""
+    rng = np.random.default_rng(5)
+    ids = T(rng.integers(0, 200_000, size=2_000_000))
+    indptr = T(np.linspace(0, 2_000_000, 1001))
+
+    def least(picked):
+        events = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+                  for _ in range(12)]
+        for before, after in events:
+            before.record()
+            capi.minor_slice(ids, picked, indptr=indptr)
+            after.record()
+        torch.cuda.synchronize()
+        return min(before.elapsed_time(after) for before, after in events)
+
+    apart, alike = T(rng.permutation(200_000)[:2047]), T(np.full(2047, 77))
+    assert least(alike) < 4.0 * least(apart)   # (1.7 times; with a slot for every copy 35)
+
+
 def test_reference_rowwise_slicing_through_the_api():
     # tests/test_rowwise_slicing.cc:7-24
     indptr = torch.cat([torch.zeros(10, dtype=torch.int64), torch.arange(3) * 2]).to(DEV)
