@@ -47,18 +47,20 @@ constexpr int kMemberThreads = 1024;  // 16 waves share one table
 // run, as many work-groups as are resident: 90 and 66 (and four chunks a run 64 and 45
 // where two now take 64 and 43).
 constexpr int kMemberWavesPerSimd = 8;
-constexpr int kMemberLdsSlots = 4096;  // tables up to this size are built in LDS (32 KB)
+constexpr int kMemberLdsSlots = 4096;  // of a table in LDS (32 KB)
+constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of fewer ids have theirs in LDS
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 
 // A table too large for LDS is looked up in L2, one request per probe, and the
 // flag pass then runs at the rate of those requests.  Most edges are not kept
 // (a slice picks a small part of the rows), so a filter that does fit LDS sends
 // them away first: a word of 32 bits per id group, three bits per picked id
-// (a blocked Bloom filter; with up to eight ids per word about one absent id in
-// twenty passes).  Only ids that pass go on to the table.
+// (a blocked Bloom filter; of absent ids one in twenty-four passes with 65 536 ids, 4.6 a
+// word, and one in five at the bound).  Only ids that pass go on to the table.
 constexpr int kFilterWords = 14336;            // 56 KB of LDS, two work-groups a compute unit
 constexpr int kFilterBits = 3;
-constexpr int64_t kFilterMaxIds = 131072;      // beyond: too many bits set to be worth a look
+// (16 M edges of 2.33 M rows, us: 131 072 picked ids 144 with the filter, one more 240 without)
+constexpr int64_t kFilterMaxIds = 131072;
 
 // Ids that may be picked, by a word of 32 bits per id group in LDS: an id whose bits
 // are not all set is not picked.  One multiplication serves the word and the bits.
@@ -87,27 +89,32 @@ struct IdFilter {
 using L2Filter = IdFilter<kFilterWords, kFilterBits>;
 
 struct MemberWs {
-  uint64_t* table;     // [member_table_slots(num_picked)]
+  uint64_t* table;     // [member_table_slots(num_picked)], a table in L2
   uint32_t* staged;    // [chunks * kBlock]: per chunk, the new ids of its kept edges, in order
   uint8_t* staged_pos;  // [chunks * kBlock]: and their places in the chunk
   int64_t* chunk_off;  // [chunks + 1]
   int* wide;           // [1] set when a picked id does not fit the upper half of a slot
-  uint32_t* filter;    // [kFilterWords] which ids may be in the table (for tables kept in L2)
+  uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
   void* scan_ws;
   size_t scan_ws_bytes;
   int64_t chunks;
   size_t total;
 };
 
-// Slots of the table: four per picked id (fewer probes for the ids that are
-// not there, which are most: 1.4 instead of 2.5 on average) while the table
-// fits in LDS or stays a small part of a die's L2, else two.
+// Whether every work-group builds the table in LDS for itself, and whether a filter lies in
+// front of a table in L2.
+static bool member_in_lds(int64_t num_picked) { return num_picked < kMemberLdsIds; }
+static bool member_filtered(int64_t num_picked) {
+  return !member_in_lds(num_picked) && num_picked <= kFilterMaxIds;
+}
+
+// Slots of the table in L2: four per picked id (fewer probes for the ids that are
+// not there, which are most: 1.4 instead of 2.5 on average) while that stays a small
+// part of a die's L2, else two.
 constexpr int64_t kMemberRoomyIds = 65536;   // 4 slots * 8 B * 65536 = 2 MB
 static uint64_t member_table_slots(int64_t num_picked) {
-  const uint64_t roomy = (uint64_t)(4 * num_picked + 2), tight = (uint64_t)(2 * num_picked + 2);
-  if (roomy <= (uint64_t)kMemberLdsSlots) return roomy;   // in LDS, roomy
-  if (tight <= (uint64_t)kMemberLdsSlots) return tight;   // still in LDS
-  return num_picked <= kMemberRoomyIds ? roomy : tight;   // in L2
+  if (member_in_lds(num_picked)) return 0;
+  return (uint64_t)((num_picked <= kMemberRoomyIds ? 4 : 2) * num_picked + 2);
 }
 
 static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
@@ -119,7 +126,7 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
   w.staged_pos = c.take<uint8_t>((size_t)w.chunks * kBlock);
   w.chunk_off = c.take<int64_t>((size_t)w.chunks + 1);
   w.wide = c.take<int>(1);
-  w.filter = c.take<uint32_t>((size_t)kFilterWords);
+  w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
   w.total = c.total();
@@ -274,7 +281,6 @@ struct MemberTable {
 // makes a wave repeat its probe loop until the longest of its probe runs
 // has ended.
 constexpr int kMemberBuckets = kMemberLdsSlots / 4;
-constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of fewer ids are kept in LDS
 struct BucketTable {
   const uint4* keys;       // [kMemberBuckets] filled from .x on; kNoKey = free
   const uint32_t* values;  // [kMemberLdsSlots] position in the picked set, by slot
@@ -831,8 +837,8 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   }
   hipStream_t s = as_stream(stream);
   const uint32_t cap = (uint32_t)member_table_slots(num_picked);
-  const bool in_lds = num_picked < kMemberLdsIds;
-  uint32_t* filter = !in_lds && num_picked <= kFilterMaxIds ? w.filter : nullptr;
+  const bool in_lds = member_in_lds(num_picked);
+  uint32_t* filter = member_filtered(num_picked) ? w.filter : nullptr;
   if (!in_lds) {
     GS_LAUNCH("member_clear", s,
               member_clear_kernel<<<dim3((unsigned)ceil_div((int64_t)cap, kBlock * 4)),
