@@ -12,7 +12,9 @@
 namespace gs {
 
 // Offsets and size of A[:, cols]: shared by the operators of this file when
-// they are handed the same tensor of columns (one wait for the size, not two).
+// they are handed the same tensor of columns (one wait for the size, not two)
+// on the same stream: another one would have to wait for what is queued on the
+// first, and memory that is freed there may be written again while it reads.
 std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tensor& cols) {
   const Compressed& m = compressed(kCSC);
   {
@@ -20,7 +22,7 @@ std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tenso
     if (slice_offsets_ && slice_offsets_->cols.is_same(cols) &&
         slice_offsets_->version == (int64_t)cols._version() &&
         slice_offsets_->indptr_version == (int64_t)m.indptr._version() &&
-        slice_offsets_->epoch == cache_epoch())
+        slice_offsets_->epoch == cache_epoch() && slice_offsets_->stream == cur_stream())
       return slice_offsets_;
   }
   auto so = std::make_shared<SliceOffsets>();
@@ -28,6 +30,7 @@ std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tenso
   so->version = cols._version();
   so->indptr_version = m.indptr._version();
   so->epoch = cache_epoch();
+  so->stream = cur_stream();
   so->sub_indptr = slice_offsets(m, cols, &so->nnz);
   std::lock_guard<std::mutex> lock(slice_offsets_guard_);
   slice_offsets_ = so;

@@ -431,6 +431,7 @@ class Graph : public torch::CustomClassHolder {
   struct SliceOffsets {
     torch::Tensor cols, sub_indptr;
     int64_t version = -1, indptr_version = -1, epoch = -1, nnz = 0;
+    void* stream = nullptr;  // whose kernels write the tensors
     std::mutex guard;
     MajorResult written;  // the slice itself, when an operator had to write it
   };

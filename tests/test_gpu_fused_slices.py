@@ -233,6 +233,37 @@ def test_threads_with_other_columns_on_one_matrix():
     assert not bad
 
 
+@pytest.mark.parametrize("pinned", [False, True])
+def test_a_second_stream_with_the_same_columns(pinned):
+    """What one stream has queued of a slice is not read on another that does not wait for it."""
+    place = (lambda a: T(a).cpu().pin_memory()) if pinned else T
+    rng = np.random.default_rng(22)
+    indptr, indices = random_csc(rng, 3000, 6000, 60)
+    g = gs.Graph(6000, 3000)
+    g._CAPI_LoadCSC(place(indptr), place(indices))
+    w = torch.as_tensor((rng.random(indices.size) + 0.05).astype(np.float32), device=DEV)
+    cols, rows = rng.integers(0, 3000, size=900), rng.choice(6000, size=400, replace=False)
+    want = chained_col_row_slice(indptr, indices, cols, rows, None)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    c, r = T(cols), T(rows)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        out = torch.zeros(6000, device=DEV)
+        g._CAPI_SlicedESquareSum(c, w, out)
+        torch.cuda._sleep(20_000_000)
+        sums = torch.zeros(6000, device=DEV)
+        g._CAPI_SlicedESquareSum(c, w, sums)
+    with torch.cuda.stream(second):
+        sub, index = g._CAPI_ColRowSlicing(c, r, gs.format._CSC, gs.format._CSC)
+        got = (sub._CAPI_GetCSCIndptr(), sub._CAPI_GetCSCIndices(), index)
+    second.synchronize()
+    assert not first.query()                                # the first one was not waited for
+    same(got, (want[0], want[2], want[3]))
+    first.synchronize()
+    # two orders of adding at most 900 x 60 terms of 32 bits
+    assert torch.allclose(out, sums, rtol=1e-5)
+
+
 @pytest.mark.parametrize("most,ncol", [(0, 5), (1, 0), (1, 300), (3, 1), (3, 70_000), (20, 9000), (700, 1500)])
 @pytest.mark.parametrize("pinned", [False, True])
 def test_slices_of_short_columns(most, ncol, pinned):
