@@ -194,14 +194,17 @@ def test_short_sliced_sums_by_ranges_of_rows(nnz, num_rows):
         assert not np.signbit(got[~none]).any()
 
 
-def test_threads_with_other_columns_on_one_matrix():
-    """What an operator holds of a slice stays when another thread's takes its place."""
+@pytest.mark.parametrize("pinned", [False, True])
+def test_threads_with_other_columns_on_one_matrix(pinned):
+    """What an operator holds of a slice stays when another thread's takes its place: read in
+    place, and, of a matrix in pinned host memory, the written slices of three of the threads."""
+    place = (lambda a: T(a).cpu().pin_memory()) if pinned else T
     rng = np.random.default_rng(21)
     deg = rng.integers(100, 9000, size=700)
     indptr = np.concatenate([[0], np.cumsum(deg)])
     indices = rng.integers(0, 20_000, size=int(deg.sum()))
     g = gs.Graph(20_000, 700)
-    g._CAPI_LoadCSC(T(indptr), T(indices))
+    g._CAPI_LoadCSC(place(indptr), place(indices))
     w = torch.as_tensor((rng.random(indices.size) + 0.05).astype(np.float32), device=DEV)
     rows = T(rng.choice(20_000, size=300, replace=False))
     cols = [T(rng.integers(0, 700, size=n)) for n in (3, 40, 300, 500)]
