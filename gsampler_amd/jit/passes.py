@@ -992,7 +992,8 @@ def share_leading_rows(copy: fx.Graph) -> None:
     """In a copy of a graph: the rows of a column slice are its parent's, so what is
     computed from data of all of them in one layer is what the next one computes.  Merges
     features[arange(number of rows)] and its products with a matrix, which are only read
-    by operators, and reads the rows in place where a product is all that does."""
+    by operators, and reads the rows in place where products for edge operators are all that
+    does (any other product may be kept for its gradient, with the rows as they were)."""
     from ..matrix_api.matrix import gen_arange
     from ..ops.fused_op import _edge_score, _leading_rows
     if any(_writes_in_place(n) for n in copy.nodes):
@@ -1004,6 +1005,9 @@ def share_leading_rows(copy: fx.Graph) -> None:
         if (_call(sliced, operator.getitem) and sliced.args[1] == 0
                 and _is_method(sliced.args[0], "_CAPI_Slicing") and sliced.args[0].args[2] == 1):
             node.args = (sliced.args[0].args[0],)
+
+    def for_edges(node):
+        return all(_call(u, _edge_score) or _is_wrapped(u, "_before_sddmm") for u in node.users)
 
     def only_read(node):
         return all(_call(u, torch.matmul, operator.matmul, _edge_score) or _is_wrapped(u, "_before_sddmm")
@@ -1025,7 +1029,7 @@ def share_leading_rows(copy: fx.Graph) -> None:
             seen[key] = node
     for node in list(copy.nodes):
         if (_call(node, operator.getitem) and _call(node.args[1], gen_arange) and node.users
-                and all(_call(u, torch.matmul, operator.matmul) for u in node.users)
+                and all(_call(u, torch.matmul, operator.matmul) and for_edges(u) for u in node.users)
                 and node.args[1].kwargs.get("dtype") is torch.int64
                 and node.args[1].kwargs.get("device") == "cuda" and len(node.args[1].args) == 1):
             with copy.inserting_before(node):

@@ -61,6 +61,10 @@ def rows_escape(A, seeds, feats, W, weights):
     return u, feats[A[:, seeds[:5]].rows()], u @ W
 
 
+def products_of_rows(A, seeds, feats, W, weights):
+    return feats[A[:, seeds].rows()] @ W, feats[A[:, seeds[:5]].rows()] @ W
+
+
 def ran(compiled):
     return [n.target for n in compiled._run.__self__.graph.nodes]
 
@@ -73,12 +77,12 @@ def cpu_args(nodes=10):
 
 @pytest.mark.parametrize("func,kernels,sddmm", [
     (scores, 1, 0), (two_layers, 2, 0), (plain_sum, 1, 0), (in_place, 0, 1), (products_wanted, 0, 1),
-    (other_sums, 0, 3), (rows_escape, 0, 0)])
+    (other_sums, 0, 3), (rows_escape, 0, 0), (products_of_rows, 0, 0)])
 def test_what_becomes_an_edge_score(func, kernels, sddmm):
     c = gs.jit.compile(func=func, args=cpu_args())
     t = ran(c)
     assert t.count(fused_op._edge_score) == kernels and t.count("_CAPI_SDDMM") == sddmm
-    in_place_free = func is not in_place and func is not rows_escape
+    in_place_free = func not in (in_place, rows_escape, products_of_rows)
     assert t.count(fused_op._leading_rows) == (1 if in_place_free else 0)
     if func is two_layers:                   # the rows' features once for both layers
         assert t.count(torch.matmul) + t.count(operator.matmul) == 3
@@ -193,6 +197,20 @@ def test_compiled_equals_eager(func, kind):
     if kind == "gradients" and want[0].requires_grad:
         (dw,), (dg,) = (torch.autograd.grad(x[0].sum(), weights) for x in (want, got))
         assert torch.equal(dw, dg)
+
+
+@pytest.mark.gpu
+def test_features_may_change_before_the_gradient_of_their_products():
+    """Rows are gathered into an array of their own, which the product keeps."""
+    m, seeds = world(), torch.arange(0, 600, 3, device=DEV)
+    feats, W = torch.randn((3000, 20), device=DEV), torch.randn((20, 12), device=DEV, requires_grad=True)
+    args = (m, seeds, feats, W, torch.rand(4, device=DEV))
+    c = gs.jit.compile(func=products_of_rows, args=args)
+    out, want = c(*args), 2.0 * feats.double().sum(0)
+    feats.mul_(3.0)
+    (out[0].sum() + out[1].sum()).backward()
+    # sums of 3000 terms in another order
+    assert torch.allclose(W.grad, want.float()[:, None].expand(20, 12), rtol=1e-4, atol=1e-3)
 
 
 # ------------------------------------------------- encoded slices that are not written
