@@ -267,9 +267,9 @@ __device__ __forceinline__ bool between_marks(const uint32_t (&mark)[kMarks], ui
 // The same walk with marks, a lane a walk, for calls that fill the machine.
 // 1 M walks of 80 steps on 124 M edges, p = 2, q = 0.5: the kernel above reads two
 // candidates a step, one of them in vain, 175 M lines in 3.31 ms; this one 130 M in
-// 2.51, both at the part's line rate (52 G/s).  84 M of those are candidates, the rest
-// marks: 2, 4 and 14 of them in place of 6 take 2.62, 2.59 and 2.49 ms (more bytes a
-// column reject more and miss L2 more often).  Non-temporal reads of the candidates
+// 2.52, both at the part's line rate (52 G/s).  80 M of those are the chosen candidates,
+// the rest marks and candidates read to be rejected: 2, 4 and 14 marks in place of 6 take
+// 2.62, 2.59 and 2.49 ms (more bytes a column reject more and miss L2 more often).  Non-temporal reads of the candidates
 // leave 4 % more of the marks in L2 and take 2.70 ms.
 // Drawn by each lane for its own walk, attempts of arithmetic only were the bound
 // (2.68 ms; 5.85 at p = 4, q = 0.25, where a candidate in four is accepted: 2.92 now).

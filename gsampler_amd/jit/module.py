@@ -151,9 +151,11 @@ class compile:  # noqa: N801 -- the reference's public name
     # -------------------------------------------------------------------- run
     def _executable(self, gm):
         """What a call runs: a copy of the operator graph whose sampling layers are
-        chained into one operator, whose edge scores are one kernel each and whose generated code takes flat inputs and
-        builds the result in place (the pytree machinery of a traced module costs
-        more than the operators of a small sampler).  None when the graph's inputs
+        chained into one operator, whose edge scores and normalisations are one
+        operator each, which sums slices without writing them where that can be, and
+        whose generated code takes flat inputs and builds the result in place (the
+        pytree machinery of a traced module costs more than the operators of a small
+        sampler).  None when the graph's inputs
         or result have no such form: the module itself is called then."""
         codegen = gm.graph._codegen
         info = getattr(codegen, "pytree_info", None)
