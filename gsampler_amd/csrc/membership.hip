@@ -88,11 +88,18 @@ struct IdFilter {
 };
 using L2Filter = IdFilter<kFilterWords, kFilterBits>;
 
+// Up to this many chunks the offsets of chunks and columns take one launch
+// (member_offsets_kernel), in which a work-group adds up the counts of all chunks before
+// its own: two bytes each, 256 KB at this bound (4.2 us on 4 M edges, 6.4 on 17 M and 8.7
+// at the bound, where three launches that read every count once take 15.2).
+constexpr int64_t kOffsetsMaxChunks = int64_t(1) << 17;
+
 struct MemberWs {
   uint64_t* table;     // [member_table_slots(num_picked)], a table in L2
   uint32_t* staged;    // [chunks * kBlock]: per chunk, the new ids of its kept edges, in order
   uint8_t* staged_pos;  // [chunks * kBlock]: and their places in the chunk
   int64_t* chunk_off;  // [chunks + 1]
+  uint16_t* chunk_kept;  // [chunks] kept edges of a chunk, for lists of up to kOffsetsMaxChunks
   int* wide;           // [1] set when a picked id does not fit the upper half of a slot
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
   void* scan_ws;
@@ -125,6 +132,8 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
   w.staged = c.take<uint32_t>((size_t)w.chunks * kBlock);
   w.staged_pos = c.take<uint8_t>((size_t)w.chunks * kBlock);
   w.chunk_off = c.take<int64_t>((size_t)w.chunks + 1);
+  w.chunk_kept =
+      c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
   w.wide = c.take<int>(1);
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
@@ -469,7 +478,7 @@ void member_flag_kernel(
     const IdT* __restrict__ ids, int64_t nnz,
     const uint64_t* __restrict__ global_table, uint32_t cap,
     const int64_t* __restrict__ picked, uint32_t num_picked, const int* __restrict__ wide_flag,
-    int64_t* __restrict__ chunk_count,
+    int64_t* __restrict__ chunk_count, uint16_t* __restrict__ chunk_kept,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
     const uint32_t* __restrict__ filter, SliceView view) {
   using Shared = MemberShared<kInLds, kThreads>;
@@ -531,8 +540,12 @@ void member_flag_kernel(
   };
   auto finish_chunk = [&](int64_t chunk) {
     if (lane == 0) {
-      chunk_count[chunk] = kept;
-      if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
+      if (chunk_kept) {
+        chunk_kept[chunk] = (uint16_t)kept;
+      } else {
+        chunk_count[chunk] = kept;
+        if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
+      }
     }
     kept = 0;
   };
@@ -678,16 +691,13 @@ void member_flag_kernel(
   }
 }
 
-// Kept edges at positions < e: those of the chunks before, and how many of the chunk's
-// kept places, which are in order, lie below.  Two rounds of sixteen places each.
-__device__ __forceinline__ int64_t member_rank_before(
-    int64_t e, const uint8_t* __restrict__ staged_pos,
-    const int64_t* __restrict__ chunk_off) {
+// How many of the kept edges of e's chunk, whose places are in order, lie before e.  Two
+// rounds of sixteen places each.
+__device__ __forceinline__ int member_below(int64_t e, int kept,
+                                            const uint8_t* __restrict__ staged_pos) {
   const int64_t chunk = e / kBlock;
-  const int64_t r = chunk_off[chunk];
-  const int kept = (int)(chunk_off[chunk + 1] - r);
   const int in_chunk = (int)(e - chunk * kBlock);
-  if (in_chunk == 0 || kept == 0) return r;
+  if (in_chunk == 0 || kept == 0) return 0;
   const uint8_t* places = staged_pos + chunk * kBlock;
   constexpr int kFan = 16;
   static_assert(kFan * kFan >= kBlock, "two rounds reach every place");
@@ -703,8 +713,86 @@ __device__ __forceinline__ int64_t member_rank_before(
     const int at = below + i;
     more += at < kept && places[at < kept ? at : 0] < in_chunk ? 1 : 0;
   }
-  return r + below + more;
+  return below + more;
 }
+
+// Offsets of the chunks and of the columns of a list of up to kOffsetsMaxChunks chunks in
+// one launch.  A work-group takes kOffsetsTile chunks and the columns that begin in them;
+// what the chunks before it keep it adds up for itself, while two of its wavefronts look
+// for its columns.  Bound by that chain of loads.  Tile sums, their scan and the columns
+// in three launches took 15 us behind the flag pass on 8 to 29 M edges, this takes 9 to 10
+// (tiles of 2048 chunks 11, and 16 where 19 K columns are short and meet in few tiles).
+constexpr int kOffsetsThreads = 1024;
+constexpr int kOffsetsTile = 512;
+__global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_major,
+    const uint8_t* __restrict__ staged_pos, const uint16_t* __restrict__ chunk_kept,
+    int64_t nnz, int64_t* __restrict__ chunk_off, int64_t* __restrict__ out_indptr,
+    int64_t* __restrict__ out_total) {
+  __shared__ uint32_t smem[kOffsetsThreads / kWave + 1];
+  __shared__ uint32_t before[kOffsetsTile + 1];  // kept edges of the tile before each chunk
+  __shared__ int64_t col_range[2];
+  const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
+  const int64_t chunk0 = (int64_t)blockIdx.x * kOffsetsTile;
+  const bool last_tile = blockIdx.x + 1 == gridDim.x;
+  const int t = threadIdx.x, wave = t / kWave;
+  const bool owns = t < kOffsetsTile && chunk0 + t < num_chunks;
+  const uint32_t own = owns ? chunk_kept[chunk0 + t] : 0u;
+  constexpr int kSearchers = 2;  // wavefronts that look for the tile's columns meanwhile
+  uint32_t mine = 0;
+  if (wave < kSearchers) {
+    if (indptr) {
+      const int64_t e = wave_uniform_first((chunk0 + (wave ? kOffsetsTile : 0)) * kBlock);
+      int64_t c;
+      if (wave ? last_tile : blockIdx.x == 0) c = wave ? num_major + 1 : 0;
+      else c = indptr[0] >= e ? 0 : wave_segment_of(indptr, num_major + 1, e - 1) + 1;
+      if (lane_id() == 0) col_range[wave] = c;
+    }
+  } else {
+    // the chunks before the tile, eight a load
+    const uint4* vecs = reinterpret_cast<const uint4*>(chunk_kept);
+    const int64_t num_vecs = chunk0 / 8;
+    constexpr int kAhead = 8, kAdders = kOffsetsThreads - kSearchers * kWave;
+    for (int64_t v0 = t - kSearchers * kWave; v0 < num_vecs; v0 += kAhead * kAdders) {
+      uint4 v[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        const int64_t at = v0 + j * kAdders;
+        v[j] = vecs[at < num_vecs ? at : 0];
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        // (a chunk keeps at most 256: sums of four fit the halves)
+        const uint32_t s = v[j].x + v[j].y + v[j].z + v[j].w;
+        if (v0 + j * kAdders < num_vecs) mine += (s & 0xFFFFu) + (s >> 16);
+      }
+    }
+  }
+  uint32_t base, in_tile;
+  (void)block_exclusive_sum<uint32_t, kOffsetsThreads>(mine, smem, &base);
+  const uint32_t run = block_exclusive_sum<uint32_t, kOffsetsThreads>(own, smem, &in_tile);
+  if (t < kOffsetsTile) before[t] = run;
+  if (t == 0) before[kOffsetsTile] = in_tile;
+  if (owns) chunk_off[chunk0 + t] = (int64_t)base + run;
+  const int64_t total = (int64_t)base + in_tile;  // of the last tile: of all
+  if (last_tile && t == 0) {
+    chunk_off[num_chunks] = total;
+    if (out_total) store_for_host(out_total, total);
+  }
+  if (indptr == nullptr) return;
+  __syncthreads();
+  for (int64_t c = col_range[0] + t; c < col_range[1]; c += kOffsetsThreads) {
+    const int64_t e = indptr[c];
+    int64_t r = total;
+    if (e < nnz) {
+      const int64_t i = e / kBlock - chunk0;
+      r = base + before[i] + member_below(e, (int)(before[i + 1] - before[i]), staged_pos);
+    }
+    out_indptr[c] = r;
+  }
+}
+
+// The columns alone, behind a scan of the chunks' counts.
 
 __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
@@ -715,8 +803,13 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
   if (c == 0 && out_total) store_for_host(out_total, nnz > 0 ? chunk_off[num_chunks] : 0);
   if (indptr == nullptr || c > num_major) return;
   const int64_t e = indptr[c];
-  out_indptr[c] = nnz == 0 ? 0
-                  : (e >= nnz ? chunk_off[num_chunks] : member_rank_before(e, staged_pos, chunk_off));
+  int64_t r = 0;
+  if (nnz > 0) {
+    const int64_t chunk = e < nnz ? e / kBlock : num_chunks;
+    r = chunk_off[chunk];
+    if (e < nnz) r += member_below(e, (int)(chunk_off[chunk + 1] - r), staged_pos);
+  }
+  out_indptr[c] = r;
 }
 
 // A wave writes the kept edges of kRun consecutive chunks: how many each has comes
@@ -848,6 +941,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
                                      dim3(kBlock), 0, s>>>(picked, num_picked,
                                                            w.table, cap, w.wide, filter));
   }
+  uint16_t* kept = w.chunks <= kOffsetsMaxChunks ? w.chunk_kept : nullptr;
   if (nnz > 0) {
     const bool small = nnz < kMemberSmallEdges;
     const int threads = small ? kBlock : kMemberThreads;
@@ -866,8 +960,8 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
-                IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, w.staged,       \
-                w.staged_pos, filter, view))
+                IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, kept,   \
+                w.staged, w.staged_pos, filter, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
@@ -887,6 +981,14 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
 #undef GS_MEMBER_FLAG
 #undef GS_MEMBER_FLAG_IDS
 #undef GS_MEMBER_FLAG_AS
+    if (kept) {
+      GS_LAUNCH("member_offsets", s,
+                member_offsets_kernel<<<dim3((unsigned)ceil_div(w.chunks, kOffsetsTile)),
+                                        dim3(kOffsetsThreads), 0, s>>>(
+                    indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,
+                    out_total));
+      return GS_OK;
+    }
     int rc = exclusive_scan_i64(w.chunk_off, w.chunk_off, w.chunks + 1, w.scan_ws,
                                 w.scan_ws_bytes, s);
     if (rc != GS_OK) return rc;

@@ -65,6 +65,23 @@ def test_minor_slice_at_the_borders_of_a_waves_run(nnz, npick):
          orc.minor_slice(indices, picked, indptr=indptr))
 
 
+@pytest.mark.parametrize("nnz", [512 * 256 - 1, 512 * 256, 512 * 256 + 1, 3 * 512 * 256 + 700,
+                                 1 << 25, (1 << 25) + 1])
+def test_minor_slice_at_the_borders_of_an_offsets_tile(nnz):
+    """The offsets of chunks and columns: one tile of 512 chunks, several, the most that
+    one launch takes and one edge more.  Columns begin at every border, on either side of
+    it, several at one place, none in some tiles, and behind the last edge."""
+    rng = np.random.default_rng(nnz)
+    borders = np.arange(0, nnz, 512 * 256)
+    starts = np.concatenate([[0, 0, nnz, nnz, nnz], borders, borders + 1, borders[1:] - 1,
+                             np.repeat(borders[::3], 3), rng.integers(0, min(nnz, 300_000), size=1500)])
+    indptr = np.sort(np.minimum(starts, nnz))
+    ids = rng.integers(0, 1000, size=nnz)
+    picked = rng.integers(0, 1100, size=60)
+    same(capi.minor_slice(T(ids), T(picked), indptr=T(indptr)),
+         orc.minor_slice(ids, picked, indptr=indptr))
+
+
 @pytest.mark.parametrize("npick", [1, 2046, 2047, 2048, 131_072, 131_073])
 @pytest.mark.parametrize("num_ids", [1, 2300, 200_000])
 def test_minor_slice_at_the_borders_of_table_and_filter(num_ids, npick):
