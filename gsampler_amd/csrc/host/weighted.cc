@@ -200,10 +200,6 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
   if (range.defined()) BatchOffsets::check(range, n, "list sampling");
   torch::Tensor ws = new_workspace(gs_list_sample_workspace_bytes(n, nseg), probs);
   torch::Tensor out_range = new_ids(nseg + 1, probs);
-  GS_CALL(gs_list_sample_weighted_count(cptr(range), n, nseg, num_picks,
-                                        replace ? 1 : 0, mptr(out_range),
-                                        ws.data_ptr(), ws.numel(), cur_stream()));
-  BatchOffsets::trust(out_range);
   // The number of picks follows from the sizes alone, so it is worked out here
   // instead of being read back from the device (which would wait for all the
   // work queued so far): the segment sizes of a range are already on the host,
@@ -220,10 +216,11 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
   }
   torch::Tensor out = new_ids(total, probs);
   const RandomState& rs = random_state();
-  GS_CALL(gs_list_sample_weighted_fill(
+  GS_CALL(gs_list_sample_weighted(
       probs.data_ptr<float>(), cptr(range), n, nseg, num_picks, replace ? 1 : 0,
-      rs.seed, next_call_id(), cptr(out_range), total, mptr(out), ws.data_ptr(),
+      rs.seed, next_call_id(), mptr(out_range), total, mptr(out), ws.data_ptr(),
       ws.numel(), cur_stream()));
+  BatchOffsets::trust(out_range, total);
   return {out, out_range};
 }
 

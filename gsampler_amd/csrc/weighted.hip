@@ -848,10 +848,15 @@ __global__ void list_counts_kernel(const int64_t* __restrict__ range, int64_t n,
 }
 
 // The same for at most kBlock - 1 segments, with the running sum: one launch
-// instead of counts + scan.
+// instead of counts + scan.  words: zeroed as well (the selection's histograms and
+// counters; a launch of its own for them takes 4.7 us in a row of launches).
 __global__ __launch_bounds__(kBlock) void list_offsets_kernel(
     const int64_t* __restrict__ range, int64_t n, int64_t nseg, int64_t num_picks, int replace,
-    int64_t* __restrict__ out_range) {
+    int64_t* __restrict__ out_range, uint32_t* __restrict__ words, int64_t num_words) {
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < num_words;
+       i += (int64_t)gridDim.x * kBlock)
+    words[i] = 0u;
+  if (blockIdx.x != 0) return;
   __shared__ int64_t smem[kBlock / kWave + 1];
   const int64_t b = threadIdx.x;
   int64_t cnt = 0;
@@ -1512,8 +1517,8 @@ int gs_list_sample_weighted_count(const int64_t* range, int64_t n,
   hipStream_t s = as_stream(stream);
   if (num_segments < kBlock) {
     GS_LAUNCH("list_counts", s,
-              list_offsets_kernel<<<dim3(1), dim3(kBlock), 0, s>>>(range, n, num_segments,
-                                                                   num_picks, replace, out_range));
+              list_offsets_kernel<<<dim3(1), dim3(kBlock), 0, s>>>(
+                  range, n, num_segments, num_picks, replace, out_range, nullptr, 0));
     return GS_OK;
   }
   GS_LAUNCH("list_counts", s,
@@ -1524,13 +1529,20 @@ int gs_list_sample_weighted_count(const int64_t* range, int64_t n,
                             w.scan_ws_bytes, s);
 }
 
-int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
-                                 int64_t n, int64_t num_segments,
-                                 int64_t num_picks, int replace, uint64_t seed,
-                                 uint64_t call_id, const int64_t* out_range,
-                                 int64_t total_picks, int64_t* out_index,
-                                 void* workspace, size_t workspace_bytes,
-                                 gs_stream_t stream) {
+// Whether the picks go by selection.
+static bool list_selects(int64_t n, int64_t num_segments, int64_t num_picks, int replace) {
+  return !replace && num_picks >= 1 && num_picks <= gs::kSelMaxPicks &&
+         gs::list_can_select(n, num_segments);
+}
+static dim3 list_zero_grid(const gs::ListWs& w) {
+  return dim3((unsigned)gs::ceil_div((int64_t)w.sel_words, gs::kBlock * 8));
+}
+
+// zeroed: the selection's histograms and counters are zero already.
+static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_t num_segments,
+                     int64_t num_picks, int replace, uint64_t seed, uint64_t call_id,
+                     const int64_t* out_range, int64_t total_picks, int64_t* out_index,
+                     void* workspace, size_t workspace_bytes, gs_stream_t stream, bool zeroed) {
   using namespace gs;
   GS_REQUIRE(n >= 0 && num_segments >= 1 && num_picks >= 0 && total_picks >= 0,
              "list_sample_fill: bad sizes");
@@ -1553,7 +1565,7 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
                   w.keys_in, out_index));
     return GS_OK;
   }
-  if (num_picks >= 1 && num_picks <= kSelMaxPicks && list_can_select(n, num_segments)) {
+  if (list_selects(n, num_segments, num_picks, replace)) {
     // few items per thread while that still fills the device, else sixteen (fewer
     // work-groups meet at the same histogram bins)
     const bool deep = n >= (int64_t(1) << 20);
@@ -1562,9 +1574,10 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
     // and 58 with 2048
     const int shift = num_picks <= 512 ? 22 : 20;
     const dim3 tiles((unsigned)ceil_div(n, kBlock * (deep ? 16 : 4)));
-    GS_LAUNCH("list_zero", s,
-              table_fill_kernel32<<<dim3((unsigned)ceil_div((int64_t)w.sel_words, kBlock * 8)),
-                                    dim3(kBlock), 0, s>>>(w.sel_block, (int64_t)w.sel_words));
+    if (!zeroed)
+      GS_LAUNCH("list_zero", s,
+                table_fill_kernel32<<<list_zero_grid(w), dim3(kBlock), 0, s>>>(
+                    w.sel_block, (int64_t)w.sel_words));
 #define GS_SEL_LAUNCH(name, kernel, ...)                                              \
   GS_LAUNCH(name, s,                                                                  \
             if (deep) kernel<16><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__);         \
@@ -1602,6 +1615,46 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
                                                      out_range, total_picks,
                                                      out_index));
   return GS_OK;
+}
+
+int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
+                                 int64_t n, int64_t num_segments,
+                                 int64_t num_picks, int replace, uint64_t seed,
+                                 uint64_t call_id, const int64_t* out_range,
+                                 int64_t total_picks, int64_t* out_index,
+                                 void* workspace, size_t workspace_bytes,
+                                 gs_stream_t stream) {
+  return list_fill(probs, range, n, num_segments, num_picks, replace, seed, call_id, out_range,
+                   total_picks, out_index, workspace, workspace_bytes, stream, false);
+}
+
+int gs_list_sample_weighted(const float* probs, const int64_t* range, int64_t n,
+                            int64_t num_segments, int64_t num_picks, int replace, uint64_t seed,
+                            uint64_t call_id, int64_t* out_range, int64_t total_picks,
+                            int64_t* out_index, void* workspace, size_t workspace_bytes,
+                            gs_stream_t stream) {
+  using namespace gs;
+  const bool begin = total_picks > 0 && n > 0 && num_segments >= 1 && num_segments < kBlock &&
+                     (range != nullptr || num_segments == 1) && out_range &&
+                     list_selects(n, num_segments, num_picks, replace);
+  if (begin) {
+    const ListWs w = carve_list(workspace, n, num_segments);
+    if (workspace == nullptr || workspace_bytes < w.total) {
+      set_error("list_sample workspace too small: %zu < %zu", workspace_bytes, w.total);
+      return GS_ERR_WORKSPACE;
+    }
+    hipStream_t s = as_stream(stream);
+    GS_LAUNCH("list_counts", s,
+              list_offsets_kernel<<<list_zero_grid(w), dim3(kBlock), 0, s>>>(
+                  range, n, num_segments, num_picks, replace, out_range, w.sel_block,
+                  (int64_t)w.sel_words));
+  } else {
+    const int rc = gs_list_sample_weighted_count(range, n, num_segments, num_picks, replace,
+                                                 out_range, workspace, workspace_bytes, stream);
+    if (rc != GS_OK) return rc;
+  }
+  return list_fill(probs, range, n, num_segments, num_picks, replace, seed, call_id, out_range,
+                   total_picks, out_index, workspace, workspace_bytes, stream, begin);
 }
 
 }  // extern "C"

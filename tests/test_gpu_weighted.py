@@ -290,6 +290,32 @@ def test_batched_list_selection_parity():
              orc.list_sample_weighted(probs, k, range_=ranges, call_id=3))
 
 
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("k", [0, 1, 300, 2048, 2049])
+@pytest.mark.parametrize("nseg", [1, 2, 255, 256])
+def test_list_sampling_in_one_call(nseg, k, replace):
+    """Counts and picks by one call, in a workspace that holds anything: lists that are
+    selected from (the counts' launch clears what that needs), sorted and drawn with
+    replacement; up to 255 segments the counts take one launch, beyond it a scan."""
+    rng = np.random.default_rng(nseg + k)
+    sizes = rng.integers(3000, 6000, size=nseg)
+    ranges = np.concatenate([[0], np.cumsum(sizes)])
+    n = int(ranges[-1])
+    probs = rng.random(n).astype(np.float32)
+    want, want_range = orc.list_sample_weighted(probs, k, replace, ranges if nseg > 1 else None, 7777, 3)
+    l = capi.lib()
+    g_probs, g_range = F(probs), T(ranges) if nseg > 1 else None
+    ws = torch.full((l.gs_list_sample_workspace_bytes(n, nseg),), 0xA5, dtype=torch.uint8, device=DEV)
+    out_range = torch.empty(nseg + 1, dtype=torch.int64, device=DEV)
+    out = torch.empty(len(want), dtype=torch.int64, device=DEV)
+    for _ in range(2):
+        capi.check(l.gs_list_sample_weighted(
+            g_probs.data_ptr(), g_range.data_ptr() if nseg > 1 else None, n, nseg, k, int(replace),
+            7777, 3, out_range.data_ptr(), len(want), out.data_ptr() if len(want) else None,
+            ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+        same((out, out_range), (want, want_range))
+
+
 def test_operators_through_the_api():
     rng = np.random.default_rng(6)
     indptr, indices = random_csc(rng, 500, 400, 60)
