@@ -1108,6 +1108,241 @@ __global__ __launch_bounds__(kOffsetsThreads) void unique_offsets_kernel(
   }
 }
 
+// ---------------------------------------------------------------- few keys
+// A call of up to kFewKeys keys is bound by its launches: plan, scatter, dedup, flag and
+// offsets take 4 to 8 us each whatever there is to do.  Two launches take their place.
+// The keys are not partitioned first: a work-group owns a bin of a batch's hash values, about
+// kFewBinKeys keys, reads all keys of the batch and keeps those of its bin, so that nothing
+// has to be agreed on between work-groups.  That reads a batch once per bin, from L2.
+// Count, frontier and labels together, us of a row of calls, five launches before and two
+// now, and the host's part of a call, 22 and 12:
+//   one batch of 600 keys   23 13     2.8 K  26 16     15 K  27 18     30 K  29 22     65 K  29 31
+//   16 batches, 15 K keys   31 21     50 K   35 26     64 batches, 65 K  32 28     500  35 36
+constexpr int64_t kFewKeys = int64_t(1) << 16;
+constexpr int64_t kFewOfOneBatch = kFewKeys * 3 / 4;
+constexpr int kFewBatches = 512;
+constexpr int kFewThreads = 1024;
+constexpr int kFewBinKeys = 512;
+constexpr uint32_t kFewSlots = 2048;  // of a bin's table: four times the keys it gets on average
+constexpr uint32_t kFewClaims = kFewSlots * 3 / 4;
+constexpr uint32_t kFewListed = 2048;  // keys of a bin that are found again without a second look
+// first[position] of a call that went this way carries a mark where the position is itself
+// a first occurrence.  (Positions are below 2^31 - 1.)
+constexpr uint32_t kFirstMark = 0x80000000u;
+// Bin of a key: a hash of 32 bits, for every work-group hashes every key of its batch.
+__device__ __forceinline__ uint32_t few_bin(uint64_t key, uint32_t bins) {
+  const uint32_t x = (uint32_t)key + (uint32_t)(key >> 32) * 33u;
+  return __umulhi(x * 0x9E3779B1u, bins);
+}
+
+__global__ __launch_bounds__(kFewThreads) void unique_few_kernel(
+    Keys k, int64_t N, BatchInfo* __restrict__ batch, int64_t* __restrict__ flat_ptr,
+    int32_t* __restrict__ group_batch, int64_t groups, int32_t* __restrict__ etile_batch,
+    int64_t etiles, uint32_t* __restrict__ first) {
+  __shared__ uint64_t keys[kFewSlots];
+  __shared__ uint32_t mins[kFewSlots + 1];  // (the last one: of the key that marks empty slots)
+  __shared__ uint64_t list_key[kFewListed];
+  __shared__ uint32_t list_pos[kFewListed];
+  __shared__ int64_t l_flat[kFewBatches + 1], l_rows[kFewBatches + 1], l_bin[kFewBatches + 1];
+  __shared__ int64_t smem[kFewThreads / kWave + 1];
+  __shared__ uint32_t listed, claimed, overflow;
+  const int t = threadIdx.x;
+  for (uint32_t i = t; i <= kFewSlots; i += kFewThreads) {
+    if (i < kFewSlots) keys[i] = kEmptySlot;
+    mins[i] = 0xFFFFFFFFu;
+  }
+  if (t == 0) listed = claimed = overflow = 0;
+  // where every batch's keys and bins begin
+  int64_t s_lo = 0, r_lo = 0, n = 0, ns = 0;
+  if (t <= k.B) {
+    s_lo = seeds_lo(k, t);
+    r_lo = rows_lo(k, t);
+  }
+  if (t < k.B) {
+    ns = seeds_lo(k, t + 1) - s_lo;
+    n = ns + rows_lo(k, t + 1) - r_lo;
+  }
+  int64_t bins;
+  const int64_t bin0 = block_exclusive_sum<int64_t, kFewThreads>(ceil_div_dev(n, kFewBinKeys), smem, &bins);
+  if (t <= k.B) {
+    l_flat[t] = s_lo + r_lo;
+    l_rows[t] = r_lo;
+    l_bin[t] = bin0;
+  }
+  __syncthreads();
+  if (blockIdx.x + 1 == gridDim.x) {  // what the passes behind look up
+    if (t <= k.B) flat_ptr[t] = s_lo + r_lo;
+    if (t < k.B) batch[t] = BatchInfo{s_lo + r_lo, n, s_lo, ns, r_lo, 0, 0, 0, 0, 0};
+    for (int64_t i = t; i <= groups; i += kFewThreads) {
+      const int64_t p = i * kGroup < N ? i * kGroup : N - 1;
+      group_batch[i] = (int32_t)segment_of(l_flat, k.B, p);
+    }
+    for (int64_t i = t; i <= etiles; i += kFewThreads) {
+      const int64_t e = i * kRelabelTile < k.E ? i * kRelabelTile : k.E - 1;
+      etile_batch[i] = k.E > 0 ? (int32_t)segment_of(l_rows, k.B, e) : 0;
+    }
+  }
+  if ((int64_t)blockIdx.x >= bins) return;
+  const int64_t b = segment_of(l_bin, k.B, (int64_t)blockIdx.x);
+  const uint32_t bin = (uint32_t)(blockIdx.x - l_bin[b]);
+  const uint32_t of = (uint32_t)((b + 1 < k.B ? l_bin[b + 1] : bins) - l_bin[b]);
+  const int64_t fb = l_flat[b];
+  n = l_flat[b + 1] - fb;
+  r_lo = l_rows[b];
+  s_lo = fb - r_lo;
+  ns = l_flat[b + 1] - l_rows[b + 1] - s_lo;
+  uint32_t* first_b = first + fb;
+  const uint32_t n32 = (uint32_t)n, ns32 = (uint32_t)ns;
+  const int64_t *seeds_b = k.seeds + s_lo, *rows_b = k.rows + (r_lo - ns);
+  auto key_of = [&](uint32_t p) {  // (one load from either array: no branch between the loads of a round)
+    return (uint64_t)(p < ns32 ? seeds_b : rows_b)[p];
+  };
+  auto store = [&](uint32_t p, uint32_t f) { first_b[p] = f == p ? f | kFirstMark : f; };
+  // the slot of a key: kFewSlots for the key that marks empty ones, more if there is none
+  auto slot_of = [&](uint64_t key, bool insert) {
+    if (key == kEmptySlot) return kFewSlots;
+    uint32_t s = slot_hash(key) % kFewSlots;
+    for (uint32_t probes = 0; probes < kFewSlots; ++probes) {
+      uint64_t cur = keys[s];
+      if (cur == kEmptySlot && insert && *(volatile uint32_t*)&claimed < kFewClaims) {
+        cur = atomicCAS((unsigned long long*)&keys[s], (unsigned long long)kEmptySlot,
+                        (unsigned long long)key);
+        if (cur == kEmptySlot) {
+          atomicAdd(&claimed, 1u);
+          return s;
+        }
+      }
+      if (cur == key) return s;
+      if (cur == kEmptySlot) break;
+      s = (s + 1) % kFewSlots;
+    }
+    return kFewSlots + 1;
+  };
+  constexpr int kAhead = 8;
+  auto each_key = [&](auto&& f) {  // of the bin
+    for (uint32_t p0 = t; p0 < n32; p0 += kAhead * kFewThreads) {
+      uint64_t key[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        const uint32_t p = p0 + j * kFewThreads;
+        key[j] = key_of(p < n32 ? p : n32 - 1);
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        const uint32_t p = p0 + j * kFewThreads;
+        if (p < n32 && few_bin(key[j], of) == bin) f(key[j], p);
+      }
+    }
+  };
+  // The bin's keys are listed first and inserted from there: a wavefront meets a key of the
+  // bin in most of its loads, and the few lanes that hold one would each go through the probes.
+  each_key([&](uint64_t key, uint32_t p) {
+    const uint32_t at = atomicAdd(&listed, 1u);
+    if (at >= kFewListed) return;
+    list_key[at] = key;
+    list_pos[at] = p;
+  });
+  __syncthreads();
+  constexpr int kMine = (int)kFewListed / kFewThreads;
+  uint32_t slot[kMine];
+  auto insert = [&](uint64_t key, uint32_t p) {
+    const uint32_t s = slot_of(key, true);
+    if (s > kFewSlots) overflow = 1;
+    else if (mins[s] > p) atomicMin(&mins[s], p);
+    return s;
+  };
+  const bool all_listed = listed <= kFewListed;
+  if (all_listed) {
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      const uint32_t i = j * kFewThreads + t;
+      slot[j] = i < listed ? insert(list_key[i], list_pos[i]) : 0u;
+    }
+  } else {
+    each_key([&](uint64_t key, uint32_t p) { insert(key, p); });
+  }
+  __syncthreads();
+  if (overflow) {
+    // keys made to meet in one bin: every one looks for itself among those before it
+    each_key([&](uint64_t key, uint32_t p) {
+      uint32_t q = 0;
+      while (key_of(q) != key) ++q;
+      store(p, q);
+    });
+  } else if (all_listed) {
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      const uint32_t i = j * kFewThreads + t;
+      if (i < listed) store(list_pos[i], mins[slot[j]]);
+    }
+  } else {
+    each_key([&](uint64_t key, uint32_t p) { store(p, mins[slot_of(key, false)]); });
+  }
+}
+
+// Rank words, offsets of the groups and unique_ptr of such a call: one work-group, as
+// unique_flag_kernel and unique_offsets_kernel leave them.
+__global__ __launch_bounds__(kFewThreads) void unique_few_offsets_kernel(
+    const int64_t* __restrict__ flat_ptr, int64_t B, int64_t N, int64_t groups,
+    const uint32_t* __restrict__ first, RankWord* __restrict__ words,
+    int64_t* __restrict__ group_off, int64_t* __restrict__ unique_ptr,
+    int64_t* __restrict__ unique_ptr_ws, int64_t* unique_ptr_mirror,
+    const BatchInfo* __restrict__ batch, int64_t* distinct_mirror) {
+  constexpr int kWaves = kFewThreads / kWave, kWords = (int)(kFewKeys / kWave), kAhead = 16;
+  static_assert(kWords == kFewThreads, "a thread a word");
+  __shared__ uint64_t bits[kWords];
+  __shared__ uint32_t before[kWords + 1];
+  __shared__ uint32_t smem[kWaves + 1];
+  const int t = threadIdx.x, wave = t / kWave, lane = lane_id();
+  const int64_t b_pos = t <= B ? flat_ptr[t] : N;
+  const int64_t b_ns = distinct_mirror && t < B ? batch[t].ns : 0;
+  bits[t] = 0;
+  __syncthreads();
+  // neighbouring words go to neighbouring wavefronts
+  for (int w0 = wave; (int64_t)w0 * kWave < N; w0 += kAhead * kWaves) {
+    uint32_t f[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int64_t p = (int64_t)(w0 + j * kWaves) * kWave + lane;
+      f[j] = first[p < N ? p : N - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int w = w0 + j * kWaves;
+      const uint64_t hit = __ballot((int64_t)w * kWave + lane < N && (f[j] & kFirstMark));
+      if (lane == 0 && (int64_t)w * kWave < N) bits[w] = hit;
+    }
+  }
+  __syncthreads();
+  uint32_t total;
+  const uint32_t run =
+      block_exclusive_sum<uint32_t, kFewThreads>((uint32_t)__popcll(bits[t]), smem, &total);
+  before[t] = run;
+  if (t == 0) before[kWords] = total;
+  __syncthreads();
+  if ((int64_t)t * kWave < N)
+    words[t] = RankWord{bits[t], run - before[t / kGroupWords * kGroupWords], 0u};
+  if (t <= groups) group_off[t] = t < groups ? before[t * kGroupWords] : total;
+  auto rank = [&](int64_t p) {  // first occurrences before p
+    if (p >= N) return (int64_t)total;
+    return (int64_t)before[p / kWave] +
+           __popcll(bits[p / kWave] & ((1ull << (int)(p % kWave)) - 1ull));
+  };
+  if (t > B) return;
+  const int64_t r = rank(b_pos);
+  if (distinct_mirror && t < B) {
+    int64_t ok = 1;  // (see unique_offsets_kernel)
+    if (b_ns > 0) {
+      const int64_t q = b_pos + b_ns - 1;
+      ok = rank(q) - r == b_ns - 1 && ((bits[q / kWave] >> (int)(q % kWave)) & 1ull);
+    }
+    store_for_host(distinct_mirror + t, ok);
+  }
+  unique_ptr[t] = r;
+  unique_ptr_ws[t] = r;
+  if (unique_ptr_mirror) store_for_host(unique_ptr_mirror + t, r);
+}
+
 // ---------------------------------------------------------------- fill
 // Streaming: first occurrences write their key to the frontier.  A wave reads
 // the keys of its kWordsPerWave rows of 64 positions in one go (whole rows:
@@ -1322,7 +1557,7 @@ __device__ __forceinline__ void relabel_tile(
     if (!one_batch) info = batch[batch_in_span(k.rows_ptr, span, e)];
     // row key e of batch b sits at flat position
     //   fb + (seeds of b) + (e - rows_ptr[b])  =  e + seeds_ptr[b + 1]
-    if (out_row) row_first[i] = first[e + info.s_lo + info.ns];
+    if (out_row) row_first[i] = first[e + info.s_lo + info.ns] & ~kFirstMark;
     if (out_col && !kByIndptr) col[i] = edge_col[e];
   }
   if (kByIndptr && out_col) {
@@ -1362,7 +1597,8 @@ __device__ __forceinline__ void relabel_tile(
         col_label.v[j] =
             seeds_distinct
                 ? col[i + j] - info.s_lo
-                : rank_of(info.fb + first[col[i + j] + info.r_lo], words, group_off) - rank0;
+                : rank_of(info.fb + (first[col[i + j] + info.r_lo] & ~kFirstMark), words, group_off) -
+                      rank0;
     }
     const int64_t e = edge_of(i);
     if (e + 1 < k.E && wide_stores) {
@@ -1489,6 +1725,17 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
     return GS_OK;
   }
   const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
+  if (N <= (B == 1 ? kFewOfOneBatch : kFewKeys) && B <= kFewBatches) {
+    GS_LAUNCH("unique_few", s,
+              unique_few_kernel<<<dim3((unsigned)(N / kFewBinKeys + B)), dim3(kFewThreads), 0, s>>>(
+                  k, N, w.batch, w.flat_ptr, w.group_batch, w.groups, w.etile_batch, w.etiles,
+                  w.first));
+    GS_LAUNCH("unique_few_offsets", s,
+              unique_few_offsets_kernel<<<dim3(1), dim3(kFewThreads), 0, s>>>(
+                  w.flat_ptr, B, N, w.groups, w.first, w.words, w.group_off, unique_ptr,
+                  w.unique_ptr, unique_ptr_mirror, w.batch, distinct_mirror));
+    return GS_OK;
+  }
   const UnitTables units{w.max_tiles,  w.max_buckets,  w.groups,      w.etiles,
                          w.tile_batch, w.bucket_batch, w.group_batch, w.etile_batch,
                          w.bucket_base, w.bucket_cap};

@@ -204,6 +204,54 @@ def test_unique_relabel_with_many_batches_in_a_group_of_positions(B, most):
         assert_same(got[:2], want[:2])
 
 
+def _bin_of(ids, bins):
+    """Bin of an id below 2^32 among those that a call of few keys is cut into."""
+    return ((ids * 0x9E3779B1 & 0xFFFFFFFF) * bins) >> 32
+
+
+@pytest.mark.parametrize("kind", ["mixed", "distinct", "one bin", "hub", "any int64"])
+@pytest.mark.parametrize("n", [1, 63, 513, 4097, 49_152, 49_153, 65_535, 65_536, 65_537])
+def test_unique_relabel_of_few_keys(n, kind):
+    """Calls around the largest that goes without a partition, as one batch and cut into
+    batches (some of them empty): ids that repeat, that never do, that are made to meet in one
+    bin (more than its table takes), one that fills its bin's list, and ids of any value,
+    the one that marks an empty slot among them."""
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, max(2, n // 3), size=n)
+    if kind == "distinct":
+        keys = rng.permutation(4 * n)[:n]
+    elif kind == "one bin":
+        few = min(n, 4097)  # (each then looks through those before it)
+        of = -(-n // 512)
+        pool = np.arange(few * of * 2, dtype=np.int64)
+        pool = pool[_bin_of(pool, of) == 0][:few]
+        keys[:pool.size] = pool
+        keys = rng.permutation(keys)
+    elif kind == "hub":
+        keys[rng.random(n) < 0.7] = 5
+    elif kind == "any int64":
+        keys = rng.choice(np.array([-1, -2, 0, 2**32 - 1, 2**32, 2**62, -2**63, 7 + 2**40, 7]), size=n)
+        keys[::3] = rng.integers(-2**63, 2**63 - 1, size=keys[::3].size)
+    S = max(1, n // 7)
+    seeds, rows = keys[:S], keys[S:]
+    edge_col = rng.integers(0, S, size=n - S)
+    assert_same(capi.unique_relabel(T(seeds), T(rows), edge_col=T(edge_col)),
+                orc.unique_relabel(seeds, rows, edge_col=edge_col))
+    for B in (2, 70, 512, 513):
+        sp = np.concatenate([[0], np.sort(rng.integers(0, S + 1, size=B - 1)), [S]])
+        rp = np.concatenate([[0], np.sort(rng.integers(0, n - S + 1, size=B - 1)), [n - S]])
+        rp = np.where(sp == 0, 0, rp)  # an edge has a column
+        rp = np.maximum.accumulate(rp)
+        if any(sp[b] == sp[b + 1] and rp[b] < rp[b + 1] for b in range(B)):
+            got = capi.unique_relabel(T(seeds), T(rows), T(sp), T(rp), want_col=False)
+            assert_same(got[:3], orc.unique_relabel(seeds, rows, sp, rp)[:3])
+            continue
+        col = np.concatenate([np.empty(0, np.int64)] + [rng.integers(sp[b], sp[b + 1], size=rp[b + 1] - rp[b])
+                                                        for b in range(B) if rp[b] < rp[b + 1]])
+        assert_same(capi.unique_relabel(T(seeds), T(rows), T(sp), T(rp), T(col)),
+                    orc.unique_relabel(seeds, rows, sp, rp, col))
+
+
 @pytest.mark.parametrize("B", [1, 3])
 def test_unique_relabel_buckets_beyond_their_regions(B):
     """The partition pass gives every bucket a region of at most 8192 entries.  Ids
