@@ -48,7 +48,7 @@ constexpr int kMemberThreads = 1024;  // 16 waves share one table
 // where two now take 64 and 43).
 constexpr int kMemberWavesPerSimd = 8;
 constexpr int kMemberLdsSlots = 4096;  // of a table in LDS (32 KB)
-constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of fewer ids have theirs in LDS
+constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of up to so many ids have theirs in LDS
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 
 // A table too large for LDS is looked up in L2, one request per probe, and the
@@ -110,7 +110,7 @@ struct MemberWs {
 
 // Whether every work-group builds the table in LDS for itself, and whether a filter lies in
 // front of a table in L2.
-static bool member_in_lds(int64_t num_picked) { return num_picked < kMemberLdsIds; }
+static bool member_in_lds(int64_t num_picked) { return num_picked <= kMemberLdsIds; }
 static bool member_filtered(int64_t num_picked) {
   return !member_in_lds(num_picked) && num_picked <= kFilterMaxIds;
 }

@@ -82,7 +82,7 @@ def test_minor_slice_at_the_borders_of_an_offsets_tile(nnz):
          orc.minor_slice(ids, picked, indptr=indptr))
 
 
-@pytest.mark.parametrize("npick", [1, 2046, 2047, 2048, 131_072, 131_073])
+@pytest.mark.parametrize("npick", [1, 2046, 2047, 2048, 2049, 131_072, 131_073])
 @pytest.mark.parametrize("num_ids", [1, 2300, 200_000])
 def test_minor_slice_at_the_borders_of_table_and_filter(num_ids, npick):
     """The most ids of a table in LDS and of the filter and one more, with all, most and few
