@@ -109,6 +109,9 @@ SIGNATURES = {
     "gs_minor_slice_fill": (_int, [_p, _i64, _i64, _p, _i64, _p, _p, _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_count": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p, _p,
                                       _sz, _p]),
+    "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
+                                            _p, _p, _sz, _p]),
+    "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),
     "gs_col_row_slice_fill": (_int, [_p, _p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "gs_probe_stream_copy": (_int, [_p, _p, _i64, _p]),
     "gs_probe_line_gather": (_int, [_p, _i64, _i64, _u64, _int, _p, _p]),
@@ -756,12 +759,13 @@ def minor_slice(ids, picked, indptr=None, edge_major=None, with_major=True):
 
 
 def col_row_slice(indptr, indices, cols, rows, key_offset=None, with_major=True,
-                  indices32=None):
+                  indices32=None, out_first=None):
     """A[rows, cols] read from the parent matrix, the column slice never written.
     -> (out_indptr[len(cols) + 1], out_major | None = position of the edge's column in
     `cols`, out_minor = position of its row in `rows`, out_select = its position in the
     parent's `indices`).  `key_offset[len(cols)]` is added to the row ids of a column's
-    edges before they are looked up among `rows`."""
+    edges before they are looked up among `rows`.  `out_first[len(rows)]`: receives the first
+    edge of the column slice that is kept as each of `rows` (2^63 - 1 where none is)."""
     indptr, indices = _i64t(indptr, "indptr"), _i64t(indices, "indices")
     cols, rows = _i64t(cols, "cols"), _i64t(rows, "rows")
     if key_offset is not None:
@@ -774,12 +778,11 @@ def col_row_slice(indptr, indices, cols, rows, key_offset=None, with_major=True,
     ws = _workspace(l.gs_minor_slice_workspace_bytes(nnz, nrow), dev)
     out_indptr = torch.empty(ncol + 1, dtype=torch.int64, device=dev)
     total = torch.empty(1, dtype=torch.int64, device=dev)
-    check(l.gs_col_row_slice_count(_ptr(indptr), _ptr(indices),
-                                   indices32.data_ptr() if indices32 is not None else None,
-                                   _ptr(cols), _ptr(key_offset),
-                                   ncol, sub_indptr.data_ptr(), nnz, _ptr(rows), nrow,
-                                   out_indptr.data_ptr(), total.data_ptr(), ws.data_ptr(),
-                                   ws.numel(), _stream()))
+    check(l.gs_col_row_slice_count_first(
+        _ptr(indptr), _ptr(indices), indices32.data_ptr() if indices32 is not None else None,
+        _ptr(cols), _ptr(key_offset), ncol, sub_indptr.data_ptr(), nnz, _ptr(rows), nrow,
+        out_indptr.data_ptr(), total.data_ptr(), _ptr(out_first), ws.data_ptr(), ws.numel(),
+        _stream()))
     kept = int(total.item())
     out_minor = torch.empty(kept, dtype=torch.int64, device=dev)
     out_select = torch.empty(kept, dtype=torch.int64, device=dev)

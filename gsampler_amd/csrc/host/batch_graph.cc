@@ -292,8 +292,7 @@ Graph::BatchListLabels* Graph::batch_list_labels_for(const torch::Tensor& col_se
   out->seeds_version = col_seeds._version();
   out->epoch = cache_epoch();
   torch::Tensor table = ids(row_ids, "row_ids"), list_ptr = ids(row_bptr_, "row_bptr");
-  torch::Tensor first = new_ids(R, edges.row);
-  GS_CALL(gs_first_position(cptr(edges.row), E, R, mptr(first), cur_stream()));
+  torch::Tensor first = first_edges(edges.row, R);
   Frontier& f = out->frontier;
   f.num_batches = B;
   f.unique_ptr = new_ids(B + 1, edges.row);

@@ -107,7 +107,7 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
 static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
                                  const torch::Tensor& sub_indptr, int64_t nnz,
                                  const torch::Tensor& key_offset, const torch::Tensor& picked,
-                                 bool with_coo) {
+                                 bool with_coo, torch::Tensor* firsts = nullptr) {
   const int64_t n = cols.numel(), np = picked.numel();
   MajorResult r;
   torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, np), m.indptr);
@@ -117,11 +117,13 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
   // the number travels
   AsyncCount kept = AsyncCount::mirrored();
   const torch::Tensor narrow = narrow_for_slice(m, nnz, n);
-  GS_CALL(gs_col_row_slice_count(cptr(m.indptr), cptr(m.indices),
-                                 narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
-                                 cptr(cols), cptr(key_offset),
-                                 n, cptr(sub_indptr), nnz, cptr(picked), np, mptr(r.indptr),
-                                 kept.mirror(), ws.data_ptr(), ws.numel(), cur_stream()));
+  // (the relabel of a slice with far fewer rows than edges goes by its rows' first edges)
+  if (firsts && nnz >= 8 * np && gs_col_row_slice_tells_first(nnz, np)) *firsts = new_ids(np, m.indptr);
+  GS_CALL(gs_col_row_slice_count_first(
+      cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+      cptr(cols), cptr(key_offset), n, cptr(sub_indptr), nnz, cptr(picked), np, mptr(r.indptr),
+      kept.mirror(), firsts && firsts->defined() ? mptr(*firsts) : nullptr, ws.data_ptr(),
+      ws.numel(), cur_stream()));
   kept.arm();
   const int64_t size = nnz <= kBoundLimit ? nnz : kept.get();
   r.minor_ids = new_ids(size, m.indptr);
@@ -151,9 +153,10 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
   SliceOffsets& so = *shared;
   MajorResult r;
+  torch::Tensor firsts;
   if (read_in_place(m, so.nnz, cols.numel())) {
     r = col_row_slice(m, cols, so.sub_indptr, so.nnz, torch::Tensor(), rows,
-                      output_format & kCOO);
+                      output_format & kCOO, &firsts);
   } else {
     const MajorResult& sliced = written_slice(so);
     Compressed tmp(sliced.indptr, sliced.minor_ids);
@@ -161,7 +164,16 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
     r.select = sliced.select.index_select(0, r.select);
   }
   GraphPtr g = derive(kCSC, output_format, r, rows.numel(), cols.numel());
+  g->keep_row_firsts(firsts, r.minor_ids);
   return {g, edge_index(m.e_ids, r.select)};
+}
+
+void Graph::keep_row_firsts(const torch::Tensor& firsts, const torch::Tensor& edge_rows) {
+  if (!firsts.defined()) return;
+  row_firsts_ = firsts;
+  row_firsts_of_ = edge_rows;
+  row_firsts_version_ = (int64_t)edge_rows._version();
+  row_firsts_epoch_ = cache_epoch();
 }
 
 // The ids `of` (undefined: zeros) of every batch moved by batch * stride.
@@ -282,9 +294,11 @@ GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bp
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
   torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, seeds.numel(), stride);
   torch::Tensor picked = encoded_ids(rows.index_select(0, row_ids), row_bptr, row_ids.numel(), stride);
+  torch::Tensor firsts;
   const MajorResult r = col_row_slice(m, seeds, shared->sub_indptr, shared->nnz, key_offset, picked,
-                                      true);
+                                      true, &firsts);
   GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
+  g->keep_row_firsts(firsts, r.minor_ids);
   g->col_bptr_ = col_bptr;
   g->orig_col_ids_ = seeds;
   g->row_encoding_size_ = stride;

@@ -585,6 +585,18 @@ bool Graph::use_list_labels(const torch::Tensor& col_seeds,
   return R > 0 && coo_ && coo_->row.numel() >= 8 * (R + S);
 }
 
+// For every id below num_ids something that grows with the first edge that carries it, the
+// largest value where none does.
+torch::Tensor Graph::first_edges(const torch::Tensor& edge_rows, int64_t num_ids) {
+  if (row_firsts_.defined() && row_firsts_of_.is_same(edge_rows) &&
+      row_firsts_version_ == (int64_t)edge_rows._version() &&
+      row_firsts_epoch_ == cache_epoch() && row_firsts_.numel() == num_ids)
+    return row_firsts_;
+  torch::Tensor first = new_ids(num_ids, edge_rows);
+  GS_CALL(gs_first_position(cptr(edge_rows), edge_rows.numel(), num_ids, mptr(first), cur_stream()));
+  return first;
+}
+
 // The frontier is the unique of seeds ++ row_ids[coo.row] in first-occurrence
 // order.  Every edge of local row l carries the same key row_ids[l], so the
 // listed ids, ordered by the first edge that uses them, give the same frontier
@@ -608,9 +620,8 @@ Graph::ListLabels& Graph::list_labels_for(const torch::Tensor& col_seeds,
   out->seeds_version = col_seeds._version();
   out->epoch = cache_epoch();
   torch::Tensor table = ids(row_ids, "row_ids");
-  const int64_t R = table.numel(), S = col_seeds.numel(), E = base.numel();
-  torch::Tensor first = new_ids(R, base);
-  GS_CALL(gs_first_position(cptr(base), E, R, mptr(first), cur_stream()));
+  const int64_t R = table.numel(), S = col_seeds.numel();
+  torch::Tensor first = first_edges(base, R);
   if (R + S <= GS_LIST_LABELS_MAX_KEYS) {
     // few enough keys for one work-group: frontier and labels in one launch
     torch::Tensor frontier = new_ids(R + S, base);

@@ -503,6 +503,12 @@ class Graph : public torch::CustomClassHolder {
     }
   };
   std::unique_ptr<ListLabels> list_labels_;
+  // Which edge of a row slice is the first of each of its rows, as the pass that made the
+  // slice has met them; nothing once the rows of the edges have been written to.
+  torch::Tensor row_firsts_, row_firsts_of_;
+  int64_t row_firsts_version_ = -1, row_firsts_epoch_ = -1;
+  void keep_row_firsts(const torch::Tensor& firsts, const torch::Tensor& edge_rows);
+  torch::Tensor first_edges(const torch::Tensor& edge_rows, int64_t num_ids);
   // The same for a super-batch: the frontier and the labels of every edge.
   struct BatchListLabels {
     torch::Tensor base, row_ids, seeds;

@@ -50,6 +50,9 @@ constexpr int kMemberWavesPerSimd = 8;
 constexpr int kMemberLdsSlots = 4096;  // of a table in LDS (32 KB)
 constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of up to so many ids have theirs in LDS
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
+// Work-groups of a launch that stages its table in LDS, at most: what is resident on 256
+// compute units is 512 large ones or 768 small ones.
+constexpr int64_t kMemberMostGroups = 1024;
 
 // A table too large for LDS is looked up in L2, one request per probe, and the
 // flag pass then runs at the rate of those requests.  Most edges are not kept
@@ -102,6 +105,8 @@ struct MemberWs {
   uint16_t* chunk_kept;  // [chunks] kept edges of a chunk, for lists of up to kOffsetsMaxChunks
   int* wide;           // [1] set when a picked id does not fit the upper half of a slot
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
+  uint32_t* firsts;    // [first_groups * num_picked] per work-group of the flag pass, the first edge it kept by each id
+  int64_t first_groups;
   void* scan_ws;
   size_t scan_ws_bytes;
   int64_t chunks;
@@ -136,6 +141,8 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
       c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
   w.wide = c.take<int>(1);
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
+  w.first_groups = member_in_lds(num_picked) ? std::min(w.chunks, kMemberMostGroups) : 0;
+  w.firsts = c.take<uint32_t>((size_t)(w.first_groups * num_picked));
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
   w.total = c.total();
@@ -449,6 +456,7 @@ struct MemberShared {
   using Filter = IdFilter<kWords, kInLds ? 2 : kFilterBits>;
   __align__(16) uint32_t keys[kInLds ? kMemberLdsSlots : 4];
   uint32_t values[kInLds ? kMemberLdsSlots : 4];
+  uint32_t first[kInLds ? kMemberLdsIds : 4];  // first edge kept by each picked id
   __align__(16) uint32_t filter[kWords];
   uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
   uint8_t queue_place[kThreads * kMemberWords];
@@ -480,7 +488,7 @@ void member_flag_kernel(
     const int64_t* __restrict__ picked, uint32_t num_picked, const int* __restrict__ wide_flag,
     int64_t* __restrict__ chunk_count, uint16_t* __restrict__ chunk_kept,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
-    const uint32_t* __restrict__ filter, SliceView view) {
+    const uint32_t* __restrict__ filter, uint32_t* __restrict__ firsts, SliceView view) {
   using Shared = MemberShared<kInLds, kThreads>;
   using Filter = typename Shared::Filter;
   __shared__ Shared sh;
@@ -491,6 +499,7 @@ void member_flag_kernel(
   if (kInLds) {
     static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
     for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
+    for (int i = threadIdx.x; i < kMemberLdsIds; i += kThreads) sh.first[i] = UINT32_MAX;
     wide = buckets.template stage<kThreads>(
         picked, num_picked, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
           const uint32_t h = Filter::hash(key);
@@ -535,6 +544,10 @@ void member_flag_kernel(
       const uint32_t at = lanes_below(peers, kept);
       (staged + chunk * kBlock)[at] = value;
       (staged_pos + chunk * kBlock)[at] = (uint8_t)place;
+      if (kInLds && firsts) {
+        const uint32_t e = (uint32_t)(chunk * kBlock) + place;
+        if (sh.first[value] > e) atomicMin(&sh.first[value], e);
+      }
     }
     kept += __popcll(peers);
   };
@@ -689,6 +702,48 @@ void member_flag_kernel(
     for (int c = 0; c < kRun; ++c)
       if (chunk0 + c < num_chunks) flag_chunk(chunk0 + c, keys[c]);
   }
+  if (kInLds && firsts) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < num_picked; i += kThreads)
+      firsts[(int64_t)blockIdx.x * num_picked + i] = sh.first[i];
+  }
+}
+
+// Which edge is the first of each picked id is what a relabel of the slice goes by.  A pass over
+// the kept edges' rows told it (58 MB and 19 us on 7.2 M of 28.8 M edges, behind a launch of 5
+// that cleared its output); here the flag pass keeps the least in LDS, a compare an edge it
+// keeps, and the work-groups' lists of them are read beside the offsets: LADIES 691 -> 662 us.
+// The first edge kept by each of kWave picked ids, of those that the flag pass's work-groups
+// have found: the place of an edge among all, which orders the ids as the kept edges do.
+__device__ __forceinline__ void member_first(int64_t part, const uint32_t* __restrict__ firsts,
+                                             int64_t groups, int64_t num_picked,
+                                             int64_t* __restrict__ out_first) {
+  constexpr int kWaves = 1024 / kWave, kAhead = 8;
+  __shared__ uint32_t least[kWaves][kWave];
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  const int64_t i = part * kWave + lane, at = i < num_picked ? i : num_picked - 1;
+  uint32_t m = UINT32_MAX;
+  for (int64_t g0 = wave; g0 < groups; g0 += kAhead * kWaves) {
+    uint32_t v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int64_t g = g0 + j * kWaves;
+      v[j] = firsts[(g < groups ? g : g0) * num_picked + at];
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) m = v[j] < m ? v[j] : m;
+  }
+  least[wave][lane] = m;
+  __syncthreads();
+  if (wave > 0 || i >= num_picked) return;
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) m = least[w][lane] < m ? least[w][lane] : m;
+  out_first[i] = m == UINT32_MAX ? INT64_MAX : (int64_t)m;
+}
+__global__ __launch_bounds__(1024) void member_first_kernel(
+    const uint32_t* __restrict__ firsts, int64_t groups, int64_t num_picked,
+    int64_t* __restrict__ out_first) {
+  member_first(blockIdx.x, firsts, groups, num_picked, out_first);
 }
 
 // How many of the kept edges of e's chunk, whose places are in order, lie before e.  Two
@@ -723,18 +778,24 @@ __device__ __forceinline__ int member_below(int64_t e, int kept,
 // in three launches took 15 us behind the flag pass on 8 to 29 M edges, this takes 9 to 10
 // (tiles of 2048 chunks 11, and 16 where 19 K columns are short and meet in few tiles).
 constexpr int kOffsetsThreads = 1024;
+static_assert(kOffsetsThreads == 1024, "member_first() runs in these work-groups too");
 constexpr int kOffsetsTile = 512;
 __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
     const uint8_t* __restrict__ staged_pos, const uint16_t* __restrict__ chunk_kept,
     int64_t nnz, int64_t* __restrict__ chunk_off, int64_t* __restrict__ out_indptr,
-    int64_t* __restrict__ out_total) {
+    int64_t* __restrict__ out_total, unsigned tiles, const uint32_t* __restrict__ firsts,
+    int64_t first_groups, int64_t num_picked, int64_t* __restrict__ out_first) {
+  if (blockIdx.x >= tiles) {  // (there are such only where out_first is asked for)
+    member_first(blockIdx.x - tiles, firsts, first_groups, num_picked, out_first);
+    return;
+  }
   __shared__ uint32_t smem[kOffsetsThreads / kWave + 1];
   __shared__ uint32_t before[kOffsetsTile + 1];  // kept edges of the tile before each chunk
   __shared__ int64_t col_range[2];
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   const int64_t chunk0 = (int64_t)blockIdx.x * kOffsetsTile;
-  const bool last_tile = blockIdx.x + 1 == gridDim.x;
+  const bool last_tile = blockIdx.x + 1 == tiles;
   const int t = threadIdx.x, wave = t / kWave;
   const bool owns = t < kOffsetsTile && chunk0 + t < num_chunks;
   const uint32_t own = owns ? chunk_kept[chunk0 + t] : 0u;
@@ -793,7 +854,6 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
 }
 
 // The columns alone, behind a scan of the chunks' counts.
-
 __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
     const uint8_t* __restrict__ staged_pos, const int64_t* __restrict__ chunk_off,
@@ -910,10 +970,14 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
                                   int64_t num_major, int64_t* out_indptr,
                                   int64_t* out_total, void* workspace,
                                   size_t workspace_bytes, gs_stream_t stream,
-                                  gs::SliceView view) {
+                                  gs::SliceView view, int64_t* out_first = nullptr) {
   using namespace gs;
   GS_REQUIRE(nnz >= 0 && num_picked >= 0 && num_major >= 0,
              "minor_slice_count: negative size");
+  GS_REQUIRE(!out_first || (num_picked >= 1 && member_in_lds(num_picked) && nnz >= 1 &&
+                            nnz < (int64_t)UINT32_MAX),
+             "minor_slice_count: no first edges of %lld ids among %lld edges",
+             (long long)num_picked, (long long)nnz);
   GS_REQUIRE((nnz == 0 || ids || ids32) && (num_picked == 0 || picked),
              "minor_slice_count: null pointer");
   GS_REQUIRE((indptr == nullptr) == (out_indptr == nullptr),
@@ -956,12 +1020,14 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
     const int64_t resident = (int64_t)per_cu * num_compute_units();
     int64_t blocks = ceil_div(w.chunks, (threads / kWave) * run);
     if ((in_lds || filter || !small) && blocks > resident) blocks = resident;
+    if (in_lds && blocks > kMemberMostGroups) blocks = kMemberMostGroups;
+    uint32_t* firsts = out_first ? w.firsts : nullptr;
     const dim3 grid((unsigned)blocks);
 #define GS_MEMBER_FLAG_AS(LDS, THREADS, RUN, IDT, IDS, VIEW)                                  \
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
                 IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, kept,   \
-                w.staged, w.staged_pos, filter, view))
+                w.staged, w.staged_pos, filter, firsts, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
@@ -981,14 +1047,19 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
 #undef GS_MEMBER_FLAG
 #undef GS_MEMBER_FLAG_IDS
 #undef GS_MEMBER_FLAG_AS
+    const unsigned first_parts = out_first ? (unsigned)ceil_div(num_picked, kWave) : 0u;
     if (kept) {
+      const unsigned tiles = (unsigned)ceil_div(w.chunks, kOffsetsTile);
       GS_LAUNCH("member_offsets", s,
-                member_offsets_kernel<<<dim3((unsigned)ceil_div(w.chunks, kOffsetsTile)),
-                                        dim3(kOffsetsThreads), 0, s>>>(
+                member_offsets_kernel<<<dim3(tiles + first_parts), dim3(kOffsetsThreads), 0, s>>>(
                     indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,
-                    out_total));
+                    out_total, tiles, firsts, blocks, num_picked, out_first));
       return GS_OK;
     }
+    if (out_first)
+      GS_LAUNCH("member_first", s,
+                member_first_kernel<<<dim3(first_parts), dim3(1024), 0, s>>>(firsts, blocks,
+                                                                             num_picked, out_first));
     int rc = exclusive_scan_i64(w.chunk_off, w.chunk_off, w.chunks + 1, w.scan_ws,
                                 w.scan_ws_bytes, s);
     if (rc != GS_OK) return rc;
@@ -1087,13 +1158,31 @@ int gs_col_row_slice_count(const int64_t* indptr, const int64_t* indices,
                            const int64_t* rows, int64_t num_rows_picked,
                            int64_t* out_indptr, int64_t* out_total, void* workspace,
                            size_t workspace_bytes, gs_stream_t stream) {
+  return gs_col_row_slice_count_first(indptr, indices, indices32, cols, key_offset,
+                                      num_cols_picked, sub_indptr, slice_nnz, rows,
+                                      num_rows_picked, out_indptr, out_total, nullptr, workspace,
+                                      workspace_bytes, stream);
+}
+
+int gs_col_row_slice_tells_first(int64_t slice_nnz, int64_t num_rows_picked) {
+  return num_rows_picked >= 1 && gs::member_in_lds(num_rows_picked) && slice_nnz >= 1 &&
+         slice_nnz < (int64_t)UINT32_MAX;
+}
+
+int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
+                                 const int32_t* indices32, const int64_t* cols,
+                                 const int64_t* key_offset, int64_t num_cols_picked,
+                                 const int64_t* sub_indptr, int64_t slice_nnz,
+                                 const int64_t* rows, int64_t num_rows_picked,
+                                 int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
+                                 void* workspace, size_t workspace_bytes, gs_stream_t stream) {
   int rc = check_slice_view(indptr, indices, cols, num_cols_picked, sub_indptr, slice_nnz,
                             "col_row_slice_count");
   if (rc != GS_OK) return rc;
   const gs::SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
   return minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
                                 num_cols_picked, out_indptr, out_total, workspace,
-                                workspace_bytes, stream, view);
+                                workspace_bytes, stream, view, out_first);
 }
 
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,

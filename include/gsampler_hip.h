@@ -679,6 +679,10 @@ int gs_minor_slice_fill(const int64_t* ids, int64_t nnz, int64_t num_picked,
  *    are told apart as id + batch * stride on both sides.
  *    indices32 (nullable): the same row ids as `indices` in 32 bits; read instead
  *    of `indices` when given (half the bytes of the pass).
+ *    count_first (where gs_col_row_slice_tells_first says 1): also, for every position in
+ *    `rows`, out_first[num_rows_picked] = the first edge v of the slice that is kept as it,
+ *    INT64_MAX where there is none -- ordered as the kept edges' places are, which
+ *    gs_first_position tells of the output.
  *  fill: out_minor[kept] = position in `rows`, out_select[kept] = position of the
  *    edge in the PARENT's indices, out_major[kept] (nullable) = position of its
  *    column in `cols`.
@@ -695,6 +699,14 @@ int gs_col_row_slice_count(const int64_t* indptr, const int64_t* indices,
                            const int64_t* rows, int64_t num_rows_picked,
                            int64_t* out_indptr, int64_t* out_total, void* workspace,
                            size_t workspace_bytes, gs_stream_t stream);
+int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
+                                 const int32_t* indices32, const int64_t* cols,
+                                 const int64_t* key_offset, int64_t num_cols_picked,
+                                 const int64_t* sub_indptr, int64_t slice_nnz,
+                                 const int64_t* rows, int64_t num_rows_picked,
+                                 int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
+                                 void* workspace, size_t workspace_bytes, gs_stream_t stream);
+int gs_col_row_slice_tells_first(int64_t slice_nnz, int64_t num_rows_picked);
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,
                           int64_t num_cols_picked, const int64_t* sub_indptr,
                           int64_t slice_nnz, int64_t num_rows_picked, int64_t* out_major,

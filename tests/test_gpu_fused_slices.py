@@ -58,6 +58,40 @@ def test_col_row_slice_parity(ncol, nrow):
     same((got[0], got[2], got[3]), (want[0], want[2], want[3]))
 
 
+@pytest.mark.parametrize("nrow", [1, 64, 65, 2048])
+@pytest.mark.parametrize("nnz", [1, 300, 70_001, (1 << 23) + 5, (1 << 25) + 1])
+def test_col_row_slice_tells_the_first_edge_of_every_row(nnz, nrow):
+    """First edges from work-groups of every size, one to several hundred of them, beside the
+    offsets and (the longest list) in a launch of their own: rows that repeat, that no edge
+    has, that have one edge; row ids moved by a column's offset, and beyond 32 bits."""
+    rng = np.random.default_rng(nnz + nrow)
+    ids = rng.integers(0, 5000, size=nnz)
+    ids[-1] = 777_777
+    indptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, size=3)), [nnz]])
+    cols = rng.permutation(4)
+    rows = rng.permutation(6000)[:nrow]
+    rows[-1] = 777_777
+    if nrow > 2:
+        rows[1] = rows[0]
+    want = np.concatenate([ids[indptr[c]:indptr[c + 1]] for c in cols])
+    sizes = np.diff(indptr)[cols]
+    for offset in (None, np.arange(4) * 10_000, np.arange(4) * 2**33):
+        keys, picked = want, rows
+        if offset is not None:
+            keys = want + np.repeat(offset, sizes)
+            picked = rows + offset[rng.integers(0, 4, size=nrow)]
+        first = torch.empty(nrow, dtype=torch.int64, device=DEV)
+        got = capi.col_row_slice(T(indptr), T(ids), T(cols), T(picked), out_first=first,
+                                 key_offset=T(offset) if offset is not None else None)
+        expect = np.full(nrow, 2**63 - 1)
+        order = np.argsort(picked, kind="stable")
+        found = np.searchsorted(picked[order], keys)
+        hit = (found < nrow) & (picked[order][np.minimum(found, nrow - 1)] == keys)
+        np.minimum.at(expect, order[found[hit]], np.nonzero(hit)[0])
+        assert np.array_equal(first.cpu().numpy(), expect)
+        assert np.array_equal(got[2].cpu().numpy(), order[found[hit]])
+
+
 def test_col_row_slice_of_long_columns():
     """Columns far longer than a work-group's run of edges (the layer-wise
     sampler's case), columns without edges in between, a column id outside the
