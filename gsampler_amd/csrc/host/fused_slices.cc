@@ -230,6 +230,11 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   g->orig_row_ids_ = row;
   g->edge_bptr_ = kept.indptr.index_select(0, col_bptr);
   BatchOffsets::trust(g->edge_bptr_);
+  if (row.is_same(col) && row_bptr.is_same(col_bptr)) {
+    g->square_rows_ = kept.minor_ids;
+    g->square_rows_version_ = (int64_t)kept.minor_ids._version();
+    g->square_rows_epoch_ = cache_epoch();
+  }
   return {g, edge_index(m.e_ids, kept.select)};
 }
 

@@ -507,6 +507,12 @@ class Graph : public torch::CustomClassHolder {
   // slice has met them; nothing once the rows of the edges have been written to.
   torch::Tensor row_firsts_, row_firsts_of_;
   int64_t row_firsts_version_ = -1, row_firsts_epoch_ = -1;
+  // The rows of the edges of A[list, list], while each is still a position of the list in the
+  // segment of its edge's mini-batch: what the slice wrote.
+  torch::Tensor square_rows_;
+  int64_t square_rows_version_ = -1, square_rows_epoch_ = -1;
+  bool rows_are_the_seeds(const torch::Tensor& col_seeds, const torch::Tensor& row_ids,
+                          const torch::Tensor& edge_rows) const;
   void keep_row_firsts(const torch::Tensor& firsts, const torch::Tensor& edge_rows);
   torch::Tensor first_edges(const torch::Tensor& edge_rows, int64_t num_ids);
   // The same for a super-batch: the frontier and the labels of every edge.

@@ -393,3 +393,33 @@ def test_batch_ids_moved_by_their_batch(n):
                                                   301, n, 10**10, out.data_ptr(), None))
         torch.cuda.synchronize()
         assert torch.equal(out, batch * 10**10 + (ids if of is not None else 0))
+
+
+@pytest.mark.parametrize("order", ["blocks", "nodes first", "edge list first", "rows written"])
+@pytest.mark.parametrize("sizes", [[40], [64, 0, 300, 1], [3] * 70, [9000, 30_000]])
+def test_relabel_of_the_subgraph_that_a_list_induces(sizes, order):
+    """A[list, list]: the frontier from the list alone and labels by position are those that
+    the general path has (a copy of the list as row ids takes it), with nodes that are in a
+    batch several times, batches without nodes, few and many edges."""
+    rng = np.random.default_rng(sum(sizes))
+    n, degree = 12_000, 6 if sum(sizes) > 10_000 else 300
+    indptr = np.arange(n + 1) * degree
+    indices = rng.integers(0, 500 if sum(sizes) < 1000 else n, size=n * degree)
+    g = gs.Graph(n, n)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    seeds = np.concatenate([rng.integers(0, 400 if k < 1000 else n, size=k) for k in sizes])
+    seeds, ptr = T(seeds), T(np.concatenate([[0], np.cumsum(sizes)]))
+    results = []
+    for rows in (seeds, seeds.clone()):
+        sub, _ = g._CAPI_BatchColRowSlcing(seeds, ptr, seeds, ptr)
+        if order == "edge list first":
+            assert sub._CAPI_GetCOORows().numel() == sub._CAPI_GetNumEdges()
+        elif order == "rows written":
+            edge_rows = sub._CAPI_BatchGetCSCIndices()[0]
+            edge_rows.copy_(torch.where(edge_rows % 2 == 0, edge_rows, torch.zeros_like(edge_rows)))
+        nodes = sub._CAPI_BatchGetValidNodes(seeds, rows) if order == "nodes first" else ()
+        results.append((*nodes, *sub._CAPI_BatchGraphRelabel(seeds, rows)[:4]))
+        results[-1] += tuple(sub._CAPI_BatchGetValidNodes(seeds, rows))
+    assert len(results[0]) == len(results[1])
+    for mine, general in zip(*results):
+        assert torch.equal(mine, general)
