@@ -353,7 +353,11 @@ class Graph : public torch::CustomClassHolder {
   std::vector<c10::intrusive_ptr<BlockBatch>> BatchSampleLayers(
       torch::Tensor seeds, torch::Tensor col_bptr, std::vector<int64_t> fanouts, bool replace,
       c10::optional<torch::Tensor> edge_probs);
-  // The same; `done` takes the finished layers one by one where the host would
+  // ... or their nodes alone: frontier and where every mini-batch's begins, per layer.
+  std::vector<torch::Tensor> BatchSampleNodes(torch::Tensor seeds, torch::Tensor col_bptr,
+                                              std::vector<int64_t> fanouts, bool replace,
+                                              c10::optional<torch::Tensor> edge_probs);
+  // The blocks again; `done` takes the finished layers one by one where the host would
   // otherwise only wait for the next one.  Returns the layers it was not called for.
   using LayerDone = std::function<void(c10::intrusive_ptr<BlockBatch>)>;
   std::vector<c10::intrusive_ptr<BlockBatch>> BatchSampleLayersWhile(
@@ -367,9 +371,9 @@ class Graph : public torch::CustomClassHolder {
   std::vector<Layer> sample_layers(const torch::Tensor& seeds, const torch::Tensor& col_bptr,
                                    const std::vector<int64_t>& fanouts, bool replace,
                                    const c10::optional<torch::Tensor>& edge_probs, bool blocks,
-                                   const LayersIdle& idle);
+                                   const LayersIdle& idle, bool labels = true);
   Layer large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr, int64_t fanout,
-                    bool replace, const torch::Tensor& cdf, uint64_t call_id,
+                    bool replace, const torch::Tensor& cdf, uint64_t call_id, bool labels,
                     const std::function<void()>& idle);
   // Workspace of the small layers, kept between calls (one per matrix, at most
   // 2^19 positions, 14 to 18 MB): its table is empty whenever a call has been

@@ -44,7 +44,8 @@ struct Queued {
 // One layer on the kernels for large layers; waits for its edge and key counts.
 Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& col_bptr,
                                 int64_t fanout, bool replace, const torch::Tensor& cdf,
-                                uint64_t call_id, const std::function<void()>& idle) {
+                                uint64_t call_id, bool labels_wanted,
+                                const std::function<void()>& idle) {
   const Compressed& m = compressed(kCSC);
   const int64_t B = col_bptr.numel() - 1, S = cols.numel();
   Layer l;
@@ -56,10 +57,12 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
   if (!l.edge_ptr.defined()) l.edge_ptr = r.indptr.index_select(0, col_bptr);
   const torch::Tensor& rows = r.minor_ids;
   const int64_t E = rows.numel();
-  l.row = new_ids(E, rows);
   const torch::Tensor labels = EdgeCount::hint().col_labels;
-  const bool prefilled = labels.defined() && labels.numel() == E && E > 0;
-  l.col = prefilled ? labels : new_ids(E, rows);
+  const bool prefilled = labels_wanted && labels.defined() && labels.numel() == E && E > 0;
+  if (labels_wanted) {
+    l.row = new_ids(E, rows);
+    l.col = prefilled ? labels : new_ids(E, rows);
+  }
   torch::Tensor ws = new_workspace(gs_unique_workspace_bytes(S, E, B), rows);
   l.frontier_ptr = new_ids(B + 1, rows);
   int64_t* distinct = PinnedWords::take((size_t)B);
@@ -70,10 +73,15 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
   OffsetMirror::arm(l.frontier_ptr);
   const int64_t bound = S + E <= kBoundLimit ? S + E : OffsetMirror::values(l.frontier_ptr).back();
   torch::Tensor frontier = new_ids(bound, rows);
-  GS_CALL(gs_unique_fill_relabel(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E, B,
-                                 cptr(l.frontier_ptr), mptr(frontier), nullptr, cptr(r.indptr),
-                                 mptr(l.row), mptr(l.col), prefilled ? 1 : 0, ws.data_ptr(),
-                                 ws.numel(), cur_stream()));
+  if (labels_wanted)
+    GS_CALL(gs_unique_fill_relabel(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E,
+                                   B, cptr(l.frontier_ptr), mptr(frontier), nullptr,
+                                   cptr(r.indptr), mptr(l.row), mptr(l.col), prefilled ? 1 : 0,
+                                   ws.data_ptr(), ws.numel(), cur_stream()));
+  else
+    GS_CALL(gs_unique_fill(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E, B,
+                           cptr(l.frontier_ptr), mptr(frontier), ws.data_ptr(), ws.numel(),
+                           cur_stream()));
   idle();
   l.e_off = OffsetMirror::values(l.edge_ptr);
   l.f_off = OffsetMirror::values(l.frontier_ptr);
@@ -89,7 +97,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
                                                const torch::Tensor& col_bptr,
                                                const std::vector<int64_t>& fanouts, bool replace,
                                                const c10::optional<torch::Tensor>& edge_probs,
-                                               bool blocks, const LayersIdle& idle) {
+                                               bool blocks, const LayersIdle& idle, bool labels) {
   const Compressed& m = compressed(kCSC);
   const bool weighted = edge_probs.has_value();
   const torch::Tensor cdf = weighted ? weight_cdf_for(edge_probs.value(), kCSC) : torch::Tensor();
@@ -158,7 +166,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           BatchOffsets::trust(ptr, n);
         }
         PinnedWords::arrived();  // every layer queued so far has been settled
-        l = large_layer(cols, ptr, K, replace, cdf, first_call + i, [&] { idle(out, i); });
+        l = large_layer(cols, ptr, K, replace, cdf, first_call + i, labels, [&] { idle(out, i); });
         mirrors = nullptr;  // it has used the thread's pinned words
         l.cols = cols;
         l.col_bptr = ptr;
@@ -270,6 +278,20 @@ std::vector<c10::optional<torch::Tensor>> Graph::SampleLayers(
   for (Layer& l : sample_layers(seeds, {}, fanouts, replace, edge_probs, false,
                                 [](std::vector<Layer>&, size_t) {}))
     out.insert(out.end(), {l.frontier, l.row, l.col, c10::nullopt});
+  return out;
+}
+
+std::vector<torch::Tensor> Graph::BatchSampleNodes(torch::Tensor seeds, torch::Tensor col_bptr,
+                                                   std::vector<int64_t> fanouts, bool replace,
+                                                   c10::optional<torch::Tensor> edge_probs) {
+  check_layers(fanouts, replace, edge_probs.has_value());
+  seeds = ids(seeds, "seeds");
+  col_bptr = ids(col_bptr, "col_bptr");
+  BatchOffsets::check(col_bptr, seeds.numel(), "BatchSampleNodes");
+  std::vector<torch::Tensor> out;
+  for (Layer& l : sample_layers(seeds, col_bptr, fanouts, replace, edge_probs, false,
+                                [](std::vector<Layer>&, size_t) {}, /*labels=*/false))
+    out.insert(out.end(), {l.frontier, l.frontier_ptr});
   return out;
 }
 

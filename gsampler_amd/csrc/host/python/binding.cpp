@@ -9,6 +9,8 @@
 //       -> (frontier, row, col, None) per layer, one flat tuple
 //   batch_sample_layers(graph, seeds, seeds_ptr, fanouts, replace, weights)
 //       -> one BlockBatch per layer
+//   batch_sample_nodes(graph, seeds, seeds_ptr, fanouts, replace, weights)
+//       -> (frontier, frontier_ptr) per layer, one flat tuple
 //   edge_score(graph, kinds, lhs, rhs, targets, weights, positive_part, shift, on_format)
 //       -> a value per edge, or None where the call is not one for the kernel
 //   BlockBatch   the operator library's class of that name with its methods, plus
@@ -194,6 +196,25 @@ py::tuple sample_layers(py::handle graph, torch::Tensor seeds, std::vector<int64
   return out;
 }
 
+py::tuple batch_sample_nodes(py::handle graph, torch::Tensor seeds, torch::Tensor ptr,
+                             std::vector<int64_t> fanouts, bool replace, py::object weights) {
+  auto g = unwrap<gs::Graph>(graph);
+  auto w = optional_tensor(weights);
+  std::vector<torch::Tensor> got;
+  {
+    py::gil_scoped_release nogil;
+    got = g->BatchSampleNodes(std::move(seeds), std::move(ptr), std::move(fanouts), replace,
+                              std::move(w));
+  }
+  py::tuple out(got.size());
+  for (size_t i = 0; i < got.size(); ++i) {
+    PyObject* v = wrap_tensor(std::move(got[i]));
+    if (!v) throw py::error_already_set();
+    PyTuple_SET_ITEM(out.ptr(), (Py_ssize_t)i, v);
+  }
+  return out;
+}
+
 // -> the scores, or None where torch's own operators have to do it.
 py::object edge_score(py::handle graph, std::vector<int64_t> kinds, py::list lhs, py::list rhs,
                       std::vector<int64_t> targets, py::object weights, bool positive_part,
@@ -268,6 +289,7 @@ PYBIND11_MODULE(_gs_python, m) {
   m.def("set_block_class", &set_block_class);
   m.def("sample_layers", &sample_layers);
   m.def("batch_sample_layers", &batch_sample_layers);
+  m.def("batch_sample_nodes", &batch_sample_nodes);
   m.def("edge_score", &edge_score);
   m.def("wrap", [](py::handle batch) { return std::make_shared<Batch>(unwrap<gs::BlockBatch>(batch)); });
   py::class_<Batch, std::shared_ptr<Batch>>(m, "BlockBatch")

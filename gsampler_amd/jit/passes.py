@@ -604,7 +604,9 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
             => _CAPI_SampleLayers(seeds, fanouts, replace, weights)
         _CAPI_BatchFusedSlicingSampling[Probs] -> _CAPI_BatchBlocks  (a super-batch)
             => _CAPI_BatchSampleLayers(seeds, ptr, fanouts, replace, weights)
-    (both called through the native binding, which makes the block objects).
+        _CAPI_BatchFusedSlicingSampling[Probs] -> _CAPI_BatchGetValidNodes
+            => the nodes of such layers, without their blocks
+    (called through the native binding, which makes the block objects).
     The operator draws the same samples.  The operator graph that a compiled sampler
     shows keeps its layers."""
     single = {"_CAPI_SlicingSampling": (2, None, 3, 4, 5), "_CAPI_SlicingSamplingProbs": (2, 3, 4, 5, 6)}
@@ -625,7 +627,11 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
         if len(sampled) != 1 or len(node.users) != 1 or len(sampled[0].users) != 1:
             return None
         relabel = next(iter(sampled[0].users))
-        if not _is_method(relabel, "_CAPI_BatchBlocks" if is_batch else "_CAPI_GraphRelabel"):
+        nodes_only = is_batch and _is_method(relabel, "_CAPI_BatchGetValidNodes")
+        if nodes_only:
+            if any(not _call(u, operator.getitem) or u.args[1] not in (0, 1) for u in relabel.users):
+                return None
+        elif not _is_method(relabel, "_CAPI_BatchBlocks" if is_batch else "_CAPI_GraphRelabel"):
             return None
         seeds, fanout, replace = args[at[0]], args[at[2]], args[at[3]]
         if (relabel.args[0] is not sampled[0] or relabel.args[1] is not seeds
@@ -647,6 +653,10 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
                        and (layer[2] is None) == (current[-1][1][2] is None))
             if follows and layer[2] is None:
                 follows = layer[1] in _getitem_users(prev, 0)
+            elif follows and layer[6].target != prev.target:
+                follows = False
+            elif follows and _is_method(prev, "_CAPI_BatchGetValidNodes"):
+                follows = layer[1] in _getitem_users(prev, 0) and layer[2] in _getitem_users(prev, 1)
             elif follows:
                 follows = (_is_method(layer[1], "frontier") and layer[1].args[0] is prev
                            and _is_method(layer[2], "frontier_ptr") and layer[2].args[0] is prev)
@@ -656,7 +666,8 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
         current = [(node, layer)]
         chains.append(current)
     for chain in chains:
-        first, (graph, seeds, ptr, weights, _, replace, _) = chain[0]
+        first, (graph, seeds, ptr, weights, _, replace, end) = chain[0]
+        nodes_only = _is_method(end, "_CAPI_BatchGetValidNodes")
         if any(a is not None and order[a] > order[first] for a in (graph, seeds, ptr, weights)):
             continue
         fanouts = [layer[4] for _, layer in chain]
@@ -665,18 +676,20 @@ def chain_layers(gm: fx.GraphModule, copy: fx.Graph) -> None:
                 out = copy.call_function(_library.native.sample_layers,
                                          args=(graph, seeds, fanouts, replace, weights))
             else:
-                out = copy.call_function(_library.native.batch_sample_layers,
+                out = copy.call_function(_library.native.batch_sample_nodes if nodes_only
+                                         else _library.native.batch_sample_layers,
                                          args=(graph, seeds, ptr, fanouts, replace, weights))
             for i, (_, layer) in enumerate(chain):
                 relabel = layer[6]
-                if ptr is not None:
+                if ptr is not None and not nodes_only:
                     blocks = copy.call_function(operator.getitem, args=(out, i))
                     relabel.replace_all_uses_with(blocks)
                     continue
-                for j in range(4):
+                outputs = 2 if nodes_only else 4
+                for j in range(outputs):
                     users = _getitem_users(relabel, j)
                     if users:
-                        item = copy.call_function(operator.getitem, args=(out, 4 * i + j))
+                        item = copy.call_function(operator.getitem, args=(out, outputs * i + j))
                         for u in users:
                             u.replace_all_uses_with(item)
     if chains:
@@ -707,7 +720,8 @@ def _writes_in_place(node: fx.Node) -> bool:
         return node.target.__name__.endswith("_") or all(s.is_mutable for s in schemas)
     name, module = getattr(node.target, "__name__", ""), getattr(node.target, "__module__", None) or ""
     known = (module.partition(".")[0] in ("torch", "_operator", "builtins", "math", __name__.partition(".")[0])
-             or node.target in (_library.native.sample_layers, _library.native.batch_sample_layers)
+             or node.target in (_library.native.sample_layers, _library.native.batch_sample_layers,
+                                _library.native.batch_sample_nodes)
              or getattr(torch, name, None) is node.target)
     return not known or name.endswith("_") and not name.endswith("__")
 

@@ -111,6 +111,41 @@ def test_super_batch(rng, cuts, fanouts, replace, weighted):
             same(x, y)
 
 
+@pytest.mark.parametrize("cuts,fanouts,replace,weighted", [
+    ([0, 8], [3, 2], False, False),
+    ([0, 0, 30, 30, 64], [10, 5], False, False),         # batches without seeds
+    ([0, 500, 1100], [8, 4], True, True),
+    ([0, 9000, 33000], [40, 2], False, False),           # a large layer, then a short bound
+    ([0, 300, 700], [64, 3], False, True),
+])
+def test_nodes_of_a_super_batch(rng, cuts, fanouts, replace, weighted):
+    """Layers of which the sampler asks the nodes alone, and the induced subgraph behind
+    them."""
+    m = matrix(rng, 40000 if cuts[-1] > 5000 else 3000, 40, 700, weighted)
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(m, False)
+    seeds = torch.from_numpy(rng.integers(0, m.num_cols(), size=cuts[-1])).to(DEV)
+
+    def nodes(A, seeds, ptr, fanouts, replace):
+        for k in fanouts:
+            sub = A[:, seeds::ptr]
+            sub = sub.individual_sampling(k, sub.edata["w"] if "w" in A.edata else None, replace)
+            seeds, ptr = sub.all_nodes()
+        return seeds, ptr, A[seeds::ptr, seeds::ptr].all_nodes()
+
+    args = (seeds, torch.tensor(cuts, device=DEV), fanouts, replace)
+    compiled = gs.jit.compile(func=nodes, args=(bm, *args))
+    assert sum("batch_sample_nodes" in str(n.target) for n in compiled._run.__self__.graph.nodes) == 1
+    gs.manual_seed(5)
+    got = compiled(bm, *args)
+    assert gs.random_state() == (5, len(fanouts))
+    gs.manual_seed(5)
+    run_time = tuple(a if isinstance(a, torch.Tensor) else None for a in (None, *args))
+    want = compiled.gm(run_time, [bm._graph], [[bm.row_ndata, bm.col_ndata, bm.edata]])
+    for a, b in zip((*got[:2], *got[2]), (*want[:2], *want[2])):
+        assert torch.equal(a, b)
+
+
 def test_seeds_outside_the_matrix_take_the_other_path(rng):
     m = matrix(rng, 500, 20, 0, False)
     seeds = torch.tensor([3, -1, 499, 500, 1 << 40, 7], device=DEV)
