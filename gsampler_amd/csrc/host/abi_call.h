@@ -306,6 +306,16 @@ class OffsetMirror {
   }
 };
 
+// prefix[index] for offsets of the library's own and checked places among them, on its way
+// to the host at once: who splits a result by batch asks for it there.
+inline torch::Tensor taken_offsets(const torch::Tensor& prefix, const torch::Tensor& index) {
+  torch::Tensor out = new_ids(index.numel(), prefix);
+  int64_t* mirror = OffsetMirror::reserve(out);
+  GS_CALL(gs_take_i64(cptr(prefix), cptr(index), index.numel(), mptr(out), mirror, cur_stream()));
+  OffsetMirror::arm(out);
+  return out;
+}
+
 // The number of edges a sampling operator produced.  A plain operator copies the
 // last entry of its prefix array to the host (AsyncCount).  A super-batched
 // operator needs the per-batch edge pointer prefix[col_bptr] on the host anyway
@@ -347,11 +357,7 @@ class EdgeCount {
   void arm(const torch::Tensor& prefix) {
     Hint& h = hint();
     if (h.col_bptr.defined()) {
-      edge_bptr_ = new_ids(h.col_bptr.numel(), prefix);
-      int64_t* mirror = OffsetMirror::reserve(edge_bptr_);
-      GS_CALL(gs_take_i64(cptr(prefix), cptr(h.col_bptr), h.col_bptr.numel(), mptr(edge_bptr_),
-                          mirror, cur_stream()));
-      OffsetMirror::arm(edge_bptr_);
+      edge_bptr_ = taken_offsets(prefix, h.col_bptr);
       h.edge_bptr = edge_bptr_;
     } else {
       count_.arm();

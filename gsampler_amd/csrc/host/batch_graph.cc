@@ -155,8 +155,8 @@ GraphAndIndex Graph::BatchColSlicing(torch::Tensor seeds, torch::Tensor col_bptr
   GraphPtr g = derive(kCSC, kCSC | kCOO, r, new_rows, seeds.numel());
   g->col_bptr_ = col_bptr;
   g->orig_col_ids_ = seeds;
-  g->edge_bptr_ = r.indptr.index_select(0, col_bptr);
-  BatchOffsets::trust(g->edge_bptr_);
+  g->edge_bptr_ = taken_offsets(r.indptr, col_bptr);
+  BatchOffsets::trust(g->edge_bptr_, g->num_edges_);
   if (encoding) {
     g->row_bptr_ = row_bptr;
     g->orig_row_ids_ = orig_rows;

@@ -34,16 +34,21 @@ void BlockBatch::fetch() {
   // Offsets by destination of every block: the columns of the sampled matrix
   // are the destinations, so its indptr, cut at the batch boundaries and
   // rebased, is the blocks' indptr (the relabelled edges keep their order).
-  // Two small launches, made when the first block is asked for rather than in
+  // A small launch, made when the first block is asked for rather than in
   // the sampler's launch sequence.
   const int64_t total = sampled_indptr.numel() - 1 + num_batches;
   indptr = new_ids(total, sampled_indptr);
-  GS_CALL(gs_split_indptr(cptr(sampled_indptr), cptr(col_bptr), num_batches, total, mptr(indptr),
-                          cur_stream()));
-  if (have_host_) return;
-  distinct = new_ids(num_batches, sampled_indptr);
-  GS_CALL(gs_batch_seeds_distinct(cptr(frontier), cptr(frontier_ptr), cptr(col_seeds),
-                                  cptr(col_bptr), num_batches, mptr(distinct), cur_stream()));
+  if (have_host_) {
+    GS_CALL(gs_split_indptr(cptr(sampled_indptr), cptr(col_bptr), num_batches, total, mptr(indptr),
+                            cur_stream()));
+    return;
+  }
+  distinct = new_ids(num_batches, sampled_indptr);  // (in host memory only: the key of its mirror)
+  int64_t* mirror = OffsetMirror::reserve(distinct);
+  GS_CALL(gs_batch_block_offsets(cptr(sampled_indptr), cptr(col_bptr), num_batches, total,
+                                 mptr(indptr), cptr(frontier), cptr(frontier_ptr), cptr(col_seeds),
+                                 mirror, cur_stream()));
+  OffsetMirror::arm(distinct);
   f_off_ = OffsetMirror::values(frontier_ptr);
   e_off_ = OffsetMirror::values(coo_ptr);
   c_off_ = OffsetMirror::values(col_bptr);

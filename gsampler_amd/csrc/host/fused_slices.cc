@@ -228,8 +228,8 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   g->row_bptr_ = row_bptr;
   g->orig_col_ids_ = col;
   g->orig_row_ids_ = row;
-  g->edge_bptr_ = kept.indptr.index_select(0, col_bptr);
-  BatchOffsets::trust(g->edge_bptr_);
+  g->edge_bptr_ = taken_offsets(kept.indptr, col_bptr);
+  BatchOffsets::trust(g->edge_bptr_, g->num_edges_);
   if (row.is_same(col) && row_bptr.is_same(col_bptr)) {
     g->square_rows_ = kept.minor_ids;
     g->square_rows_version_ = (int64_t)kept.minor_ids._version();
@@ -307,8 +307,8 @@ GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bp
   g->col_bptr_ = col_bptr;
   g->orig_col_ids_ = seeds;
   g->row_encoding_size_ = stride;
-  g->edge_bptr_ = g->csc_->indptr.index_select(0, col_bptr);
-  BatchOffsets::trust(g->edge_bptr_);
+  g->edge_bptr_ = taken_offsets(g->csc_->indptr, col_bptr);
+  BatchOffsets::trust(g->edge_bptr_, g->num_edges_);
   g->row_bptr_ = row_bptr;
   g->orig_row_ids_ = row_ids;
   return {g, edge_index(m.e_ids, r.select)};

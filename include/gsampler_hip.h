@@ -824,6 +824,12 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
                             const int64_t* seeds, const int64_t* seeds_ptr,
                             int64_t num_batches, int64_t* out_distinct,
                             gs_stream_t stream);
+/* gs_split_indptr by seeds_ptr and gs_batch_seeds_distinct in one launch; the flags go to
+ * distinct_mirror[num_batches], which may be pinned host memory. */
+int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int64_t num_batches,
+                           int64_t out_len, int64_t* out, const int64_t* frontier,
+                           const int64_t* frontier_ptr, const int64_t* seeds,
+                           int64_t* distinct_mirror, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Edge-wise compute operators.  Common arguments: (format, a, b, num_major,

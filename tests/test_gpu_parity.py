@@ -434,6 +434,31 @@ def test_unique_relabel_one_huge_batch():
                 orc.unique_relabel(seeds, rows, edge_col=edge_col))
 
 
+@pytest.mark.parametrize("sizes", [[1], [0, 0], [5, 0, 1024, 3], [1023] * 3, [2] * 300])
+def test_block_offsets_and_flags_in_one_launch(sizes):
+    """The blocks' column pointers and whether a batch's seeds are distinct, against the two
+    calls: batches without columns, tiles of the pointers that end inside a batch, more
+    batches than a work-group has threads."""
+    rng = np.random.default_rng(len(sizes))
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    S, B = int(ptr[-1]), len(sizes)
+    indptr = T(np.concatenate([[0], np.cumsum(rng.integers(0, 9, size=S))]))
+    seeds = rng.integers(0, 3000, size=S)
+    rows = rng.integers(0, 3000, size=B)
+    frontier, frontier_ptr = capi.unique_relabel(T(seeds), T(rows), T(ptr), T(np.arange(B + 1)))[:2]
+    l, seeds, ptr = capi.lib(), T(seeds), T(ptr)
+    out = [torch.full((S + B,), -7, dtype=torch.int64, device=DEV) for _ in range(2)]
+    flags = torch.full((B,), -7, dtype=torch.int64, device=DEV)
+    mirror = torch.full((B,), -7, dtype=torch.int64).pin_memory()
+    P = lambda t: t.data_ptr()
+    capi.check(l.gs_split_indptr(P(indptr), P(ptr), B, S + B, P(out[0]), None))
+    capi.check(l.gs_batch_seeds_distinct(P(frontier), P(frontier_ptr), P(seeds), P(ptr), B, P(flags), None))
+    capi.check(l.gs_batch_block_offsets(P(indptr), P(ptr), B, S + B, P(out[1]), P(frontier),
+                                        P(frontier_ptr), P(seeds), P(mirror), None))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1]) and torch.equal(flags.cpu(), mirror)
+
+
 def test_graphsage_layers_end_to_end():
     """Three fused slice+sample + unique/relabel layers on an R-MAT graph, super-batch
     of 8, compared with the oracle layer by layer."""
