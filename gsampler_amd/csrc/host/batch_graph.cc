@@ -226,12 +226,17 @@ torch::Tensor Graph::batch_rows_for_relabel(const torch::Tensor& edge_rows,
   if (row_ids.numel() == 0) return edge_rows;
   if (!(mapped_out_.defined() && mapped_from_.is_same(edge_rows) &&
         mapped_by_.is_same(row_ids))) {
-    torch::Tensor enc = ids(row_ids, "row_ids").index_select(0, edge_rows);
-    const int64_t B = edge_bptr_.numel() - 1;
-    torch::Tensor orig = enc;
-    if (row_encoding_size_ > 0)
-      orig = std::get<1>(batch_offsets(enc, B, row_encoding_size_));
-    mapped_out_ = orig;
+    torch::Tensor table = ids(row_ids, "row_ids");
+    if (table.numel() >= num_rows_) {  // (the edges' rows lie below num_rows)
+      mapped_out_ = new_ids(edge_rows.numel(), edge_rows);
+      GS_CALL(gs_local_ids(cptr(table), table.numel(), cptr(edge_rows), edge_rows.numel(),
+                           row_encoding_size_, mptr(mapped_out_), cur_stream()));
+    } else {
+      mapped_out_ = table.index_select(0, edge_rows);
+      if (row_encoding_size_ > 0)
+        mapped_out_ = std::get<1>(
+            batch_offsets(mapped_out_, edge_bptr_.numel() - 1, row_encoding_size_));
+    }
     mapped_from_ = edge_rows;
     mapped_by_ = row_ids;
   }

@@ -185,6 +185,28 @@ static torch::Tensor encoded_ids(const torch::Tensor& of, const torch::Tensor& b
   return e;
 }
 
+torch::Tensor Graph::SliceOffsets::kept_key_offset(const torch::Tensor& bptr) {
+  std::lock_guard<std::mutex> lock(guard);
+  return key_offset.defined() && key_bptr.is_same(bptr) &&
+                 key_bptr_version == (int64_t)bptr._version()
+             ? key_offset
+             : torch::Tensor();
+}
+void Graph::SliceOffsets::keep_key_offset(const torch::Tensor& bptr, const torch::Tensor& offset) {
+  std::lock_guard<std::mutex> lock(guard);
+  key_offset = offset;
+  key_bptr = bptr;
+  key_bptr_version = (int64_t)bptr._version();
+}
+torch::Tensor Graph::key_offsets_for(SliceOffsets& so, const torch::Tensor& col_bptr) {
+  torch::Tensor offset = so.kept_key_offset(col_bptr);
+  if (!offset.defined()) {
+    offset = encoded_ids(torch::Tensor(), col_bptr, so.cols.numel(), num_rows_);
+    so.keep_key_offset(col_bptr, offset);
+  }
+  return offset;
+}
+
 // Per batch b: the columns col[col_bptr[b] : col_bptr[b+1]] restricted to the
 // rows row[row_bptr[b] : row_bptr[b+1]]; row ids become positions in `row`.
 // The returned edge index addresses the parent's edges.  One pass over the
@@ -204,8 +226,17 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
   BatchOffsets::check(row_bptr, row.numel(), "BatchColRowSlicing");
   const Compressed& m = compressed(kCSC);
   const int64_t stride = num_rows_;
-  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, col.numel(), stride);
-  torch::Tensor picked = encoded_ids(row, row_bptr, row.numel(), stride);
+  torch::Tensor key_offset, picked;
+  if (row.is_same(col) && row_bptr.is_same(col_bptr)) {
+    key_offset = new_ids(col.numel(), col_bptr);
+    picked = new_ids(row.numel(), row_bptr);
+    GS_CALL(gs_pick_batch_ids(cptr(row), row.numel(), nullptr, cptr(row_bptr), row_bptr.numel() - 1,
+                              row.numel(), stride, nullptr, mptr(picked), mptr(key_offset),
+                              cur_stream()));
+  } else {
+    key_offset = encoded_ids(torch::Tensor(), col_bptr, col.numel(), stride);
+    picked = encoded_ids(row, row_bptr, row.numel(), stride);
+  }
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(col);
   SliceOffsets& so = *shared;
   MajorResult kept;
@@ -259,7 +290,7 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> Graph::En
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
   const int64_t nnz = shared->nnz;
   if (!gs_encoded_square_sums_pay(nnz, B, stride)) return {};
-  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, n, stride);
+  torch::Tensor key_offset = key_offsets_for(*shared, col_bptr);
   torch::Tensor row_bptr = new_ids(B + 1, m.indptr);
   torch::Tensor ws = new_workspace(gs_encoded_square_sums_workspace_bytes(nnz, B, stride), m.indptr);
   const torch::Tensor narrow = m.narrow_indices(2 * nnz);  // the row slice reads them as well
@@ -283,9 +314,30 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> Graph::En
 
 // BatchRowSlicing of the encoded slice of (seeds, col_bptr) by row_ids, positions in
 // `rows` (EncodedSquareSums) that lie in it; the edge index addresses this matrix's edges.
-GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
-                                       torch::Tensor rows, torch::Tensor row_ids,
-                                       torch::Tensor row_bptr) {
+// `picked`: rows[row_ids], moved by batch * num_rows.
+GraphAndIndex Graph::encoded_row_slice(const torch::Tensor& seeds, const torch::Tensor& col_bptr,
+                                       const torch::Tensor& picked, const torch::Tensor& row_ids,
+                                       const torch::Tensor& row_bptr) {
+  const Compressed& m = compressed(kCSC);
+  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
+  torch::Tensor key_offset = key_offsets_for(*shared, col_bptr);
+  torch::Tensor firsts;
+  const MajorResult r = col_row_slice(m, seeds, shared->sub_indptr, shared->nnz, key_offset, picked,
+                                      true, &firsts);
+  GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
+  g->keep_row_firsts(firsts, r.minor_ids);
+  g->col_bptr_ = col_bptr;
+  g->orig_col_ids_ = seeds;
+  g->row_encoding_size_ = num_rows_;
+  g->edge_bptr_ = taken_offsets(g->csc_->indptr, col_bptr);
+  BatchOffsets::trust(g->edge_bptr_, g->num_edges_);
+  g->row_bptr_ = row_bptr;
+  g->orig_row_ids_ = row_ids;
+  return {g, edge_index(m.e_ids, r.select)};
+}
+
+static void check_encoded(torch::Tensor& seeds, torch::Tensor& col_bptr, torch::Tensor& row_ids,
+                          torch::Tensor& row_bptr) {
   seeds = ids(seeds, "seeds");
   col_bptr = ids(col_bptr, "col_bptr");
   row_ids = ids(row_ids, "row_ids");
@@ -294,24 +346,29 @@ GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bp
               "BatchRowSlicing: column and row batch pointers must have the same length");
   BatchOffsets::check(col_bptr, seeds.numel(), "BatchColSlicing");
   BatchOffsets::check(row_bptr, row_ids.numel(), "BatchRowSlicing");
-  const Compressed& m = compressed(kCSC);
-  const int64_t stride = num_rows_;
-  const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
-  torch::Tensor key_offset = encoded_ids(torch::Tensor(), col_bptr, seeds.numel(), stride);
-  torch::Tensor picked = encoded_ids(rows.index_select(0, row_ids), row_bptr, row_ids.numel(), stride);
-  torch::Tensor firsts;
-  const MajorResult r = col_row_slice(m, seeds, shared->sub_indptr, shared->nnz, key_offset, picked,
-                                      true, &firsts);
-  GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
-  g->keep_row_firsts(firsts, r.minor_ids);
-  g->col_bptr_ = col_bptr;
-  g->orig_col_ids_ = seeds;
-  g->row_encoding_size_ = stride;
-  g->edge_bptr_ = taken_offsets(g->csc_->indptr, col_bptr);
-  BatchOffsets::trust(g->edge_bptr_, g->num_edges_);
-  g->row_bptr_ = row_bptr;
-  g->orig_row_ids_ = row_ids;
-  return {g, edge_index(m.e_ids, r.select)};
+}
+
+GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
+                                       torch::Tensor rows, torch::Tensor row_ids,
+                                       torch::Tensor row_bptr) {
+  check_encoded(seeds, col_bptr, row_ids, row_bptr);
+  torch::Tensor picked =
+      encoded_ids(rows.index_select(0, row_ids), row_bptr, row_ids.numel(), num_rows_);
+  return encoded_row_slice(seeds, col_bptr, picked, row_ids, row_bptr);
+}
+
+std::tuple<GraphPtr, torch::Tensor, torch::Tensor> Graph::EncodedPickedRows(
+    torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows, torch::Tensor row_ids,
+    torch::Tensor row_bptr) {
+  check_encoded(seeds, col_bptr, row_ids, row_bptr);
+  rows = ids(rows, "rows");
+  const int64_t n = row_ids.numel();
+  torch::Tensor picked = new_ids(n, row_ids), names = new_ids(n, row_ids);
+  GS_CALL(gs_pick_batch_ids(cptr(rows), rows.numel(), cptr(row_ids), cptr(row_bptr),
+                            row_bptr.numel() - 1, n, num_rows_, mptr(names), mptr(picked), nullptr,
+                            cur_stream()));
+  auto got = encoded_row_slice(seeds, col_bptr, picked, row_ids, row_bptr);
+  return {std::get<0>(got), std::get<1>(got), names};
 }
 
 }  // namespace gs

@@ -322,6 +322,10 @@ class Graph : public torch::CustomClassHolder {
       torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor efeat);
   GraphAndIndex EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
                                   torch::Tensor row_ids, torch::Tensor row_bptr);
+  // The same for row_ids known to lie in `rows` (a sampler's picks of them); and rows[row_ids].
+  std::tuple<GraphPtr, torch::Tensor, torch::Tensor> EncodedPickedRows(
+      torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows, torch::Tensor row_ids,
+      torch::Tensor row_bptr);
   GraphAndIndex BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr,
                                   torch::Tensor row, torch::Tensor row_bptr);
   GraphAndIndex BatchRowSlicing(torch::Tensor row_ids, torch::Tensor row_bptr);
@@ -438,12 +442,21 @@ class Graph : public torch::CustomClassHolder {
     void* stream = nullptr;  // whose kernels write the tensors
     std::mutex guard;
     MajorResult written;  // the slice itself, when an operator had to write it
+    // of a super-batch cut by key_bptr: what every column's row ids are moved by
+    torch::Tensor key_offset, key_bptr;
+    int64_t key_bptr_version = -1;
+    torch::Tensor kept_key_offset(const torch::Tensor& bptr);
+    void keep_key_offset(const torch::Tensor& bptr, const torch::Tensor& offset);
   };
   std::mutex slice_offsets_guard_;
   std::shared_ptr<SliceOffsets> slice_offsets_;
   std::shared_ptr<SliceOffsets> slice_offsets_for(const torch::Tensor& cols);
   static bool read_in_place(const Compressed& m, int64_t slice_nnz, int64_t num_cols_picked);
   const MajorResult& written_slice(SliceOffsets& so);
+  torch::Tensor key_offsets_for(SliceOffsets& so, const torch::Tensor& col_bptr);
+  GraphAndIndex encoded_row_slice(const torch::Tensor& seeds, const torch::Tensor& col_bptr,
+                                  const torch::Tensor& picked, const torch::Tensor& row_ids,
+                                  const torch::Tensor& row_bptr);
   // CDF of edge_probs in the edge order of `format` (cached per weights tensor).
   torch::Tensor weight_cdf_for(const torch::Tensor& edge_probs, int64_t format);
   void check_reduce_operands(const std::string& op, const torch::Tensor& ufeat,

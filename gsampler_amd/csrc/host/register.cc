@@ -120,6 +120,7 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_BatchSampleLayers", &Graph::BatchSampleLayers)
       .def("_CAPI_NormaliseColumns", &Graph::NormaliseColumns)
       .def("_CAPI_EncodedSquareSums", &Graph::EncodedSquareSums)
+      .def("_CAPI_EncodedPickedRows", &Graph::EncodedPickedRows)
       .def("_CAPI_EncodedRowSlicing", &Graph::EncodedRowSlicing);
 }
 

@@ -913,7 +913,7 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
     those rows, whose edge index s[1] only gathers edge data that feeds those operators, and
     nothing written to from there to the row slice
         => _encoded_square_sums(A, seeds, ptr, w) and _encoded_row_slice, whose index
-           addresses A's edges."""
+           addresses A's edges and which has the ids of the picked rows at hand."""
     from ..ops.fused_op import _encoded_row_slice, _encoded_square_sums
     order = {n: i for i, n in enumerate(copy.nodes)}
 
@@ -981,7 +981,10 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
                                       "_CAPI_BatchListSamplingWithProbs")
                     and picked.args[0].args and picked.args[0].args[-1] in row_ptrs):
                 ok = False            # rows that may not be the slice's
-        if not ok or _written_between(order, [slicing, *gathered, total, *row_slices, *regather]):
+        names = [n for r in rows for ids in _getitem_users(r, 0) for n in ids.users
+                 if _call(n, operator.getitem) and n.args[0] is ids
+                 and any(n.args[1] is rs.args[1] and order[rs] < order[n] for rs in row_slices)]
+        if not ok or _written_between(order, [slicing, *gathered, total, *row_slices, *regather, *names]):
             continue
         with copy.inserting_before(slicing):
             found = copy.call_function(_encoded_square_sums, args=(parent, seeds, ptr, total.args[4].args[0],
@@ -994,7 +997,11 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
         after[0].replace_all_uses_with(sums_of)
         for rs in row_slices:
             with copy.inserting_before(rs):
-                picked_edges = copy.call_function(_encoded_row_slice, args=(part, rs.args[1], rs.args[2]))
+                of = [n for n in names if n.args[1] is rs.args[1] and order[rs] < order[n]]
+                picked_edges = copy.call_function(_encoded_row_slice,
+                                                  args=(part, *rs.args[1:3], *([ids] if of else [])))
+                for n in of:
+                    n.replace_all_uses_with(copy.call_function(operator.getitem, args=(picked_edges, 2)))
             rs.replace_all_uses_with(picked_edges)
         for node in regather:
             node.replace_input_with(node.args[0], node.args[0].args[0])

@@ -108,13 +108,16 @@ def _encoded_square_sums(g, seeds, seeds_ptr, values, on_format):
     return (sub, index), rows, rows_ptr, _after_spmm(out, squeeze)
 
 
-def _encoded_row_slice(part, row_ids, rows_ptr):
-    """The picked rows of such a slice: (matrix, index into the sliced matrix's edges)."""
+def _encoded_row_slice(part, row_ids, rows_ptr, rows=None):
+    """The rows picked of such a slice: (matrix, index into the sliced matrix's edges), and
+    rows[row_ids] where its rows are given."""
     from ..matrix_api.matrix import data_index
     if len(part) == 4:
-        return part[0]._CAPI_EncodedRowSlicing(*part[1:], row_ids, rows_ptr)
+        sub, index, names = part[0]._CAPI_EncodedPickedRows(*part[1:], row_ids, rows_ptr)
+        return (sub, index) if rows is None else (sub, index, names)
     sub, index = part[0]._CAPI_BatchRowSlicing(row_ids, rows_ptr)
-    return sub, data_index(part[1], index)
+    index = data_index(part[1], index)
+    return (sub, index) if rows is None else (sub, index, rows[row_ids])
 
 
 def _leading_rows(x, n):

@@ -824,6 +824,17 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
                             const int64_t* seeds, const int64_t* seeds_ptr,
                             int64_t num_batches, int64_t* out_distinct,
                             gs_stream_t stream);
+/* gs_pick_batch_ids: with id = ids[index[i]] (index nullable: ids[i]) for item i of batch b,
+ * out_id[i] = id, out_moved[i] = id + b * stride and out_offset[i] = b * stride, each
+ * nullable.  A place outside [0, num_ids) counts as id 0.
+ * gs_local_ids: out[e] = table[rows[e]], its remainder by stride where stride > 0; a row
+ * outside [0, num_ids) reads table[0]. */
+int gs_pick_batch_ids(const int64_t* ids, int64_t num_ids, const int64_t* index,
+                      const int64_t* batch_ptr, int64_t num_batches, int64_t n, int64_t stride,
+                      int64_t* out_id, int64_t* out_moved, int64_t* out_offset,
+                      gs_stream_t stream);
+int gs_local_ids(const int64_t* table, int64_t num_ids, const int64_t* rows, int64_t n,
+                 int64_t stride, int64_t* out, gs_stream_t stream);
 /* gs_split_indptr by seeds_ptr and gs_batch_seeds_distinct in one launch; the flags go to
  * distinct_mirror[num_batches], which may be pinned host memory. */
 int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int64_t num_batches,

@@ -395,6 +395,35 @@ def test_batch_ids_moved_by_their_batch(n):
         assert torch.equal(out, batch * 10**10 + (ids if of is not None else 0))
 
 
+@pytest.mark.parametrize("n", [1, 256, 257, 5000])
+def test_batch_ids_picked_from_a_list(n):
+    rng = np.random.default_rng(n)
+    ptr = np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=300)), [n]])
+    ids, index = T(rng.integers(0, 10**9, size=700)), T(rng.integers(0, 700, size=n))
+    batch = T(np.repeat(np.arange(301), np.diff(ptr)))
+    direct, l = T(rng.integers(0, 10**9, size=n)), capi.lib()
+    for source, at, name in ((ids, index, ids[index]), (direct, None, direct)):
+        outs = [torch.full((n,), -7, dtype=torch.int64, device=DEV) for _ in range(3)]
+        for wanted in ((0, 1, 2), (1,), (0, 2)):
+            for o in outs:
+                o.fill_(-7)
+            capi.check(l.gs_pick_batch_ids(
+                source.data_ptr(), source.numel(), at.data_ptr() if at is not None else None,
+                T(ptr).data_ptr(), 301, n, 10**10,
+                *(outs[i].data_ptr() if i in wanted else None for i in range(3)), None))
+            torch.cuda.synchronize()
+            for i, want in enumerate((name, name + batch * 10**10, batch * 10**10)):
+                assert torch.equal(outs[i], want if i in wanted else torch.full_like(want, -7))
+    # ids behind local rows, as they are and without their batch
+    moved = name + batch * 10**10
+    rows, out = T(rng.integers(0, n, size=3 * n + 1)), torch.empty(3 * n + 1, dtype=torch.int64, device=DEV)
+    for stride, want in ((0, moved[rows]), (10**10, name[rows])):
+        capi.check(l.gs_local_ids(moved.data_ptr(), n, rows.data_ptr(), rows.numel(), stride,
+                                  out.data_ptr(), None))
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("order", ["blocks", "nodes first", "edge list first", "rows written"])
 @pytest.mark.parametrize("sizes", [[40], [64, 0, 300, 1], [3] * 70, [9000, 30_000]])
 def test_relabel_of_the_subgraph_that_a_list_induces(sizes, order):
