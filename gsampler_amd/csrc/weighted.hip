@@ -970,10 +970,17 @@ __global__ __launch_bounds__(kBlock) void table_fill_kernel32(uint32_t* __restri
 // if enough of them lie before it (100 K items, 300 of them positive, 400 picks: 710 us
 // without that).
 // 2.45 M items, 400 picks, us: keys 25, two levels of histograms 10 and 11 and finish 7
-// when all keys were made; now bounds 18, emit 6, finish 8.  Bounds takes 22 with bins of
-// an eighth and 28 with half as many items a work-group: every work-group adds its bins
-// to the same words in memory.
+// when all keys were made; now bounds 16, emit 6, finish 8.
 constexpr int kSelBins = 2048;
+// Long segments: neighbouring work-groups add to one of eight histograms, and half as many
+// items a work-group, twice as many of them, fill the device better than the adds to the same
+// words cost.  One segment of 1 M, 2.45 M and 10 M items, 400, 400 and 1000 picks, all of the
+// selection: 35, 38 and 93 us with one histogram and sixteen items a thread, 28, 35 and 73;
+// shorter segments only pay for clearing and reading eight (20 K items 20 and 22, eight
+// segments of 233 K 41 and 41).  Bounds alone is then at the instructions of its draws, 12 of
+// 16 us at 2.45 M.
+constexpr int kSelCopies = 8;
+constexpr int64_t kSelLongSegment = int64_t(1) << 19;
 constexpr int kSelTile = 4096;  // shortest average segment the selection takes on
 constexpr int64_t kSelMaxPicks = 2048;
 constexpr int kFinishThreads = 1024;
@@ -1031,15 +1038,19 @@ __device__ __forceinline__ float sel_bound(uint32_t bin, int shift) {
 // (1-based, want <= number of items), and the number of items in the bins
 // below it.  Called by the whole work-group; the result is the same in every
 // thread.
-__device__ __forceinline__ void find_bin(const uint32_t* __restrict__ hist, uint32_t want,
+__device__ __forceinline__ void find_bin(const uint32_t* __restrict__ hist, int copies,
+                                         int64_t copy_words, int bins, uint32_t want,
                                          uint32_t* smem, uint32_t* found, uint32_t* bin,
                                          uint32_t* below) {
   constexpr int kPer = kSelBins / kBlock;
-  uint32_t c[kPer], sum = 0;
+  const int first = threadIdx.x * kPer;
+  uint32_t c[kPer] = {}, sum = 0;
+  if (first < bins) {
+    for (int copy = 0; copy < copies; ++copy)
 #pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    c[j] = hist[threadIdx.x * kPer + j];
-    sum += c[j];
+      for (int j = 0; j < kPer; ++j) c[j] += hist[copy * copy_words + first + j];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) sum += c[j];
   }
   uint32_t total;
   uint32_t run = block_exclusive_sum(sum, smem, &total);
@@ -1075,10 +1086,11 @@ __device__ __forceinline__ SegmentSpan sel_span(const int64_t* __restrict__ rang
 template <int kSelItems>
 __global__ __launch_bounds__(kBlock) void list_bounds_kernel(
     const float* __restrict__ probs, const int64_t* __restrict__ range, int64_t n,
-    int64_t nseg, PhiloxKey key, int shift, float* __restrict__ keys, uint32_t* hist,
+    int64_t nseg, PhiloxKey key, int shift, float* __restrict__ keys, uint32_t* hists, int copies,
     uint32_t* __restrict__ tile_never) {
   __shared__ uint32_t lh[kSelBins];
   __shared__ uint32_t never;
+  uint32_t* hist = hists + (int64_t)(blockIdx.x % copies) * nseg * kSelBins;
   const int64_t i0 = (int64_t)blockIdx.x * (kBlock * kSelItems);
   const int64_t i_last = i0 + (kBlock * kSelItems) - 1 < n ? i0 + (kBlock * kSelItems) - 1 : n - 1;
   const SegmentSpan span = sel_span(range, nseg, i0, i_last);
@@ -1121,8 +1133,8 @@ template <int kSelItems>
 __global__ __launch_bounds__(kBlock) void list_emit_kernel(
     const float* __restrict__ probs, const int64_t* __restrict__ range, int64_t n, int64_t nseg,
     int64_t num_picks, PhiloxKey key, int shift, const float* __restrict__ keys,
-    const uint32_t* __restrict__ hist, const uint32_t* __restrict__ tile_never, uint32_t* counts,
-    uint64_t* __restrict__ cand_key, int64_t* __restrict__ cand_idx) {
+    const uint32_t* __restrict__ hist, int copies, const uint32_t* __restrict__ tile_never,
+    uint32_t* counts, uint64_t* __restrict__ cand_key, int64_t* __restrict__ cand_idx) {
   __shared__ uint32_t smem[kBlock / kWave + 1];
   __shared__ uint32_t found[2];
   __shared__ uint32_t base;
@@ -1140,7 +1152,8 @@ __global__ __launch_bounds__(kBlock) void list_emit_kernel(
     const SelSegment sg = sel_segment(range, n, seg);
     if (sg.hi - sg.lo <= num_picks) continue;  // taken whole
     uint32_t bin, below;
-    find_bin(hist + seg * kSelBins, (uint32_t)num_picks, smem, found, &bin, &below);
+    find_bin(hist + seg * kSelBins, copies, nseg * kSelBins, (int)(0x80000000u >> shift),
+             (uint32_t)num_picks, smem, found, &bin, &below);
     const float bound = sel_bound(bin, shift);
     uint32_t is_cand = 0;  // one bit per item of this thread
 #pragma unroll
@@ -1321,6 +1334,7 @@ struct ListWs {
   uint32_t* sel_block;
   size_t sel_words;
   uint32_t *hist, *counts, *tile_never;
+  int copies;  // of the histograms, [copies][segments][kSelBins]
   size_t total;
 };
 
@@ -1348,10 +1362,11 @@ static ListWs carve_list(void* ws, int64_t n, int64_t nseg) {
   w.scan_ws_bytes = scan_workspace_bytes(nseg + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
   const size_t segs = list_can_select(n, nseg) ? (size_t)nseg : 0;
-  w.sel_words = segs * (kSelBins + 1);
+  w.copies = nseg > 0 && n / nseg >= kSelLongSegment ? kSelCopies : 1;
+  w.sel_words = segs * ((size_t)w.copies * kSelBins + 1);
   w.sel_block = c.take<uint32_t>(w.sel_words);
   w.hist = w.sel_block;
-  w.counts = w.hist ? w.hist + segs * kSelBins : nullptr;
+  w.counts = w.hist ? w.hist + segs * w.copies * kSelBins : nullptr;
   w.tile_never = c.take<uint32_t>(segs ? m / (kBlock * 4) + 1 : 0);
   w.total = c.total();
   return w;
@@ -1567,25 +1582,26 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
   }
   if (list_selects(n, num_segments, num_picks, replace)) {
     // few items per thread while that still fills the device, else sixteen (fewer
-    // work-groups meet at the same histogram bins)
-    const bool deep = n >= (int64_t(1) << 20);
+    // work-groups meet at the same histogram bins), eight where there are copies of those
+    const int items = n < (int64_t(1) << 20) ? 4 : w.copies > 1 ? 8 : 16;
     // bins half a power of two wide, an eighth where many picks make candidates dear
     // (they are compared with one another): 233 K items 24 and 27 us with 400 picks, 69
     // and 58 with 2048
     const int shift = num_picks <= 512 ? 22 : 20;
-    const dim3 tiles((unsigned)ceil_div(n, kBlock * (deep ? 16 : 4)));
+    const dim3 tiles((unsigned)ceil_div(n, kBlock * items));
     if (!zeroed)
       GS_LAUNCH("list_zero", s,
                 table_fill_kernel32<<<list_zero_grid(w), dim3(kBlock), 0, s>>>(
                     w.sel_block, (int64_t)w.sel_words));
 #define GS_SEL_LAUNCH(name, kernel, ...)                                              \
   GS_LAUNCH(name, s,                                                                  \
-            if (deep) kernel<16><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__);         \
+            if (items == 16) kernel<16><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__);     \
+            else if (items == 8) kernel<8><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__);  \
             else kernel<4><<<tiles, dim3(kBlock), 0, s>>>(__VA_ARGS__))
     GS_SEL_LAUNCH("list_bounds", list_bounds_kernel, probs, range, n, num_segments, key, shift,
-                  (float*)w.keys_in, w.hist, w.tile_never);
+                  (float*)w.keys_in, w.hist, w.copies, w.tile_never);
     GS_SEL_LAUNCH("list_emit", list_emit_kernel, probs, range, n, num_segments, num_picks, key, shift,
-                  (const float*)w.keys_in, w.hist, w.tile_never, w.counts, w.keys_out, w.vals_out);
+                  (const float*)w.keys_in, w.hist, w.copies, w.tile_never, w.counts, w.keys_out, w.vals_out);
 #undef GS_SEL_LAUNCH
     GS_LAUNCH("list_finish", s,
               list_finish_kernel<<<dim3((unsigned)num_segments, kFinishSplit), dim3(kFinishThreads), 0, s>>>(

@@ -275,6 +275,23 @@ def test_batched_list_selection_that_comes_to_weights_of_zero(k, positive):
     same(capi.list_sample_weighted(F(probs), k, call_id=7), orc.list_sample_weighted(probs, k, call_id=7))
 
 
+@pytest.mark.parametrize("sizes", [[(1 << 19) - 1], [1 << 19], [1 << 20], [(1 << 20) + 4099],
+                                   [3, 0, (1 << 21) + 77, 9000]])
+@pytest.mark.parametrize("zeros", [0.0, 0.9999])
+def test_list_selection_with_copies_of_the_histograms(sizes, zeros):
+    """Lists around the shortest whose work-groups share eight histograms, in each of the
+    items a thread takes; short and empty segments beside a long one; picks that come to
+    weights of zero."""
+    rng = np.random.default_rng(sum(sizes))
+    ranges = np.concatenate([[0], np.cumsum(sizes)])
+    probs = rng.random(ranges[-1]).astype(np.float32)
+    probs[rng.random(probs.size) < zeros] = 0.0
+    range_ = ranges if len(sizes) > 1 else None
+    for k in (1, 400, 2048):
+        same(capi.list_sample_weighted(F(probs), k, range_=T(range_) if range_ is not None else None, call_id=9),
+             orc.list_sample_weighted(probs, k, range_=range_, call_id=9))
+
+
 def test_batched_list_selection_parity():
     """Segments long enough for the selection path, ragged, one of them empty, one taken
     whole, one with fewer positive weights than picks."""
