@@ -138,6 +138,8 @@ SIGNATURES = {
     "gs_list_sample_weighted_count": (_int, [_p, _i64, _i64, _i64, _int, _p, _p, _sz, _p]),
     "gs_list_sample_weighted": (_int, [_p, _p, _i64, _i64, _i64, _int, _u64, _u64, _p,
                                        _i64, _p, _p, _sz, _p]),
+    "gs_list_sample_weighted_values": (_int, [_p, _p, _i64, _i64, _i64, _int, _u64, _u64, _p,
+                                              _i64, _p, _p, _p, _sz, _p]),
     "gs_list_sample_weighted_fill": (_int, [_p, _p, _i64, _i64, _i64, _int, _u64, _u64, _p,
                                             _i64, _p, _p, _sz, _p]),
     "gs_random_walk": (_int, [_p, _p, _i64, _p, _i64, _i64, _u64, _u64, _p, _p]),

@@ -179,8 +179,7 @@ void Graph::SDDMM(const std::string& op, torch::Tensor lhs, torch::Tensor rhs,
                    cptr(bc.rhs_off), cur_stream()));
 }
 
-// A float32 tensor on the current device that nothing but its values matters of.
-static bool plain_values(const torch::Tensor& t, bool gradients_matter) {
+bool plain_values(const torch::Tensor& t, bool gradients_matter) {
   return t.defined() && t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
          t.layout() == torch::kStrided && t.get_device() == c10::hip::current_device() &&
          !t.is_neg() && !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined() &&

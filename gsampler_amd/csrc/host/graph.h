@@ -564,6 +564,8 @@ MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
 void check_weighted_fanout(int64_t fanout, bool replace, const char* who);
 MajorResult minor_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo);
+// A float32 tensor on the current device that nothing but its values matters of.
+bool plain_values(const torch::Tensor& t, bool gradients_matter);
 // First n entries of a buffer sized by an upper bound: a view, or a copy when
 // the view would pin a large buffer for a small result.
 torch::Tensor trim_to(const torch::Tensor& buffer, int64_t n);
@@ -573,6 +575,10 @@ torch::Tensor GatherRows(torch::Tensor table, torch::Tensor ids);
 torch::Tensor ListSampling(int64_t num_items, int64_t num_picks, bool replace);
 torch::Tensor ListSamplingProbs(torch::Tensor probs, int64_t num_picks,
                                 bool replace);
+// Either of these for a compiled sampler, with the picks' weights: (index, offsets, weights);
+// nothing where the call is not one for it (see Graph::EdgeScore).
+c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> ListSamplingPicked(
+    torch::Tensor probs, int64_t num_picks, bool replace, c10::optional<torch::Tensor> range);
 std::tuple<torch::Tensor, torch::Tensor> BatchListSamplingProbs(
     torch::Tensor probs, int64_t num_picks, bool replace, torch::Tensor range);
 std::tuple<torch::Tensor, torch::Tensor> BatchListSampling(

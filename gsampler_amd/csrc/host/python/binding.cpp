@@ -13,6 +13,8 @@
 //       -> (frontier, frontier_ptr) per layer, one flat tuple
 //   edge_score(graph, kinds, lhs, rhs, targets, weights, positive_part, shift, on_format)
 //       -> a value per edge, or None where the call is not one for the kernel
+//   list_sampling(probs, num_picks, replace, ranges or None)
+//       -> (picks, their offsets, their weights), or None likewise
 //   BlockBatch   the operator library's class of that name with its methods, plus
 //       make_blocks(): the list of Block objects
 //   wrap(batch)  the same around a batch that came through torch
@@ -248,6 +250,26 @@ py::object edge_score(py::handle graph, std::vector<int64_t> kinds, py::list lhs
   return py::reinterpret_steal<py::object>(wrap_tensor(std::move(*out)));
 }
 
+py::object list_sampling(py::handle probs, int64_t num_picks, bool replace, py::object ranges) {
+  if (!THPVariable_CheckExact(probs.ptr())) return py::none();
+  torch::Tensor p = THPVariable_Unpack(probs.ptr());
+  auto r = optional_tensor(ranges);
+  c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> got;
+  {
+    py::gil_scoped_release nogil;
+    got = gs::ListSamplingPicked(std::move(p), num_picks, replace, std::move(r));
+  }
+  if (!got.has_value()) return py::none();
+  py::tuple out(3);
+  torch::Tensor* parts[] = {&std::get<0>(*got), &std::get<1>(*got), &std::get<2>(*got)};
+  for (Py_ssize_t i = 0; i < 3; ++i) {
+    PyObject* v = wrap_tensor(std::move(*parts[i]));
+    if (!v) throw py::error_already_set();
+    PyTuple_SET_ITEM(out.ptr(), i, v);
+  }
+  return out;
+}
+
 std::vector<std::shared_ptr<Batch>> batch_sample_layers(py::handle graph, torch::Tensor seeds,
                                                         torch::Tensor ptr,
                                                         std::vector<int64_t> fanouts, bool replace,
@@ -291,6 +313,7 @@ PYBIND11_MODULE(_gs_python, m) {
   m.def("batch_sample_layers", &batch_sample_layers);
   m.def("batch_sample_nodes", &batch_sample_nodes);
   m.def("edge_score", &edge_score);
+  m.def("list_sampling", &list_sampling);
   m.def("wrap", [](py::handle batch) { return std::make_shared<Batch>(unwrap<gs::BlockBatch>(batch)); });
   py::class_<Batch, std::shared_ptr<Batch>>(m, "BlockBatch")
       .def("make_blocks", &Batch::make_blocks)

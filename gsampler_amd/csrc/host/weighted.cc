@@ -1,5 +1,8 @@
 // weighted.cc -- weighted per-column sampling and the collective (list)
 // sampling operators.
+#include <ATen/autocast_mode.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+
 #include "abi_call.h"
 #include "graph.h"
 
@@ -191,7 +194,7 @@ torch::Tensor ListSampling(int64_t num_items, int64_t num_picks, bool replace) {
 
 static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
     const torch::Tensor& probs_in, int64_t num_picks, bool replace,
-    const torch::Tensor& range) {
+    const torch::Tensor& range, torch::Tensor* values = nullptr) {
   TORCH_CHECK(num_picks >= 0, "list sampling: negative number of picks");
   torch::Tensor probs = f32(probs_in, "probs");
   const int64_t n = probs.numel();
@@ -215,11 +218,12 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
     total = picks_of(n);
   }
   torch::Tensor out = new_ids(total, probs);
+  if (values) *values = torch::empty({total}, probs.options().requires_grad(false));
   const RandomState& rs = random_state();
-  GS_CALL(gs_list_sample_weighted(
+  GS_CALL(gs_list_sample_weighted_values(
       probs.data_ptr<float>(), cptr(range), n, nseg, num_picks, replace ? 1 : 0,
-      rs.seed, next_call_id(), mptr(out_range), total, mptr(out), ws.data_ptr(),
-      ws.numel(), cur_stream()));
+      rs.seed, next_call_id(), mptr(out_range), total, mptr(out),
+      values ? values->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), cur_stream()));
   BatchOffsets::trust(out_range, total);
   return {out, out_range};
 }
@@ -232,6 +236,17 @@ torch::Tensor ListSamplingProbs(torch::Tensor probs, int64_t num_picks,
 std::tuple<torch::Tensor, torch::Tensor> BatchListSamplingProbs(
     torch::Tensor probs, int64_t num_picks, bool replace, torch::Tensor range) {
   return list_weighted(probs, num_picks, replace, ids(range, "range"));
+}
+
+c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> ListSamplingPicked(
+    torch::Tensor probs, int64_t num_picks, bool replace, c10::optional<torch::Tensor> range) {
+  if (!plain_values(probs, true) || probs.dim() != 1 || !probs.is_contiguous() ||
+      at::impl::torch_function_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return {};
+  torch::Tensor values;
+  auto got = list_weighted(probs, num_picks, replace,
+                           range.has_value() ? ids(*range, "range") : torch::Tensor(), &values);
+  return std::make_tuple(std::get<0>(got), std::get<1>(got), values);
 }
 
 // Uniform batched selection = weighted selection with unit weights over the

@@ -875,14 +875,17 @@ __global__ __launch_bounds__(kBlock) void list_take_kernel(
     const int64_t* __restrict__ sorted_vals, const int64_t* __restrict__ range,
     int64_t n, int64_t nseg, int64_t num_picks,
     const int64_t* __restrict__ out_range, int64_t total,
-    int64_t* __restrict__ out_index) {
+    int64_t* __restrict__ out_index, const float* __restrict__ probs,
+    float* __restrict__ out_value) {
   const int64_t o = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (o >= total) return;
   const int64_t b = nseg == 1 ? 0 : segment_of(out_range, nseg, o);
   const int64_t lo = range ? range[b] : 0;
   const int64_t nb = (range ? range[b + 1] : n) - lo;
   const int64_t k = o - out_range[b];
-  out_index[o] = nb <= num_picks ? lo + k : sorted_vals[lo + k];
+  const int64_t i = nb <= num_picks ? lo + k : sorted_vals[lo + k];
+  out_index[o] = i;
+  if (out_value) out_value[o] = probs[i];
 }
 
 // Integer CDF of a list segment by segment is a device-wide problem; segments
@@ -892,7 +895,7 @@ __global__ __launch_bounds__(kBlock) void list_replace_kernel(
     const float* __restrict__ probs, const int64_t* __restrict__ range,
     int64_t n, int64_t nseg, int64_t num_picks, PhiloxKey key,
     const int64_t* __restrict__ out_range, uint64_t* cdf_scratch,
-    int64_t* __restrict__ out_index) {
+    int64_t* __restrict__ out_index, float* __restrict__ out_value) {
   const int lane = lane_id();
   const int64_t b = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
   if (b >= nseg) return;
@@ -934,7 +937,9 @@ __global__ __launch_bounds__(kBlock) void list_replace_kernel(
       else
         l = mid + 1;
     }
-    out_index[out_start + k] = lo + (l < nb ? l : nb - 1);
+    const int64_t i = lo + (l < nb ? l : nb - 1);
+    out_index[out_start + k] = i;
+    if (out_value) out_value[out_start + k] = probs[i];
   }
 }
 
@@ -1206,7 +1211,12 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
     const int64_t* __restrict__ range, int64_t n, int64_t num_picks,
     const uint32_t* __restrict__ counts, const uint64_t* __restrict__ cand_key,
     const int64_t* __restrict__ cand_idx, const int64_t* __restrict__ out_range,
-    int64_t* __restrict__ out_index) {
+    int64_t* __restrict__ out_index, const float* __restrict__ probs,
+    float* __restrict__ out_value) {
+  auto pick = [&](int64_t at, int64_t i) {
+    out_index[at] = i;
+    if (out_value) out_value[at] = probs[i];
+  };
   __shared__ uint64_t sk[kFinishSlots];
   __shared__ int64_t si[kFinishSlots];
   __shared__ uint32_t hist[256];
@@ -1217,7 +1227,7 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
   const int64_t nb = sg.hi - sg.lo, out0 = out_range[seg];
   if (nb <= num_picks) {  // taken whole, in the original order
     if (blockIdx.y == 0)
-      for (int64_t k = threadIdx.x; k < nb; k += kFinishThreads) out_index[out0 + k] = sg.lo + k;
+      for (int64_t k = threadIdx.x; k < nb; k += kFinishThreads) pick(out0 + k, sg.lo + k);
     return;
   }
   // (no list is longer than its segment; restated here because indices follow from it)
@@ -1318,7 +1328,7 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
   __syncthreads();
   for (uint32_t m = threadIdx.x; m < mine; m += kFinishThreads) {
     const uint32_t t = my_items[m], r = rank_of_item[t];
-    if (r < (uint32_t)num_picks) out_index[out0 + r] = si[t];
+    if (r < (uint32_t)num_picks) pick(out0 + r, si[t]);
   }
 }
 
@@ -1557,7 +1567,8 @@ static dim3 list_zero_grid(const gs::ListWs& w) {
 static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_t num_segments,
                      int64_t num_picks, int replace, uint64_t seed, uint64_t call_id,
                      const int64_t* out_range, int64_t total_picks, int64_t* out_index,
-                     void* workspace, size_t workspace_bytes, gs_stream_t stream, bool zeroed) {
+                     float* out_value, void* workspace, size_t workspace_bytes,
+                     gs_stream_t stream, bool zeroed) {
   using namespace gs;
   GS_REQUIRE(n >= 0 && num_segments >= 1 && num_picks >= 0 && total_picks >= 0,
              "list_sample_fill: bad sizes");
@@ -1577,7 +1588,7 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
               list_replace_kernel<<<dim3((unsigned)ceil_div(num_segments * kWave, kBlock)),
                                     dim3(kBlock), 0, s>>>(
                   probs, range, n, num_segments, num_picks, key, out_range,
-                  w.keys_in, out_index));
+                  w.keys_in, out_index, out_value));
     return GS_OK;
   }
   if (list_selects(n, num_segments, num_picks, replace)) {
@@ -1606,7 +1617,7 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
     GS_LAUNCH("list_finish", s,
               list_finish_kernel<<<dim3((unsigned)num_segments, kFinishSplit), dim3(kFinishThreads), 0, s>>>(
                   range, n, num_picks, w.counts, w.keys_out, w.vals_out,
-                  out_range, out_index));
+                  out_range, out_index, probs, out_value));
     return GS_OK;
   }
   GS_LAUNCH("list_keys", s,
@@ -1629,7 +1640,7 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
                                dim3(kBlock), 0, s>>>(w.vals_out, range, n,
                                                      num_segments, num_picks,
                                                      out_range, total_picks,
-                                                     out_index));
+                                                     out_index, probs, out_value));
   return GS_OK;
 }
 
@@ -1641,7 +1652,7 @@ int gs_list_sample_weighted_fill(const float* probs, const int64_t* range,
                                  void* workspace, size_t workspace_bytes,
                                  gs_stream_t stream) {
   return list_fill(probs, range, n, num_segments, num_picks, replace, seed, call_id, out_range,
-                   total_picks, out_index, workspace, workspace_bytes, stream, false);
+                   total_picks, out_index, nullptr, workspace, workspace_bytes, stream, false);
 }
 
 int gs_list_sample_weighted(const float* probs, const int64_t* range, int64_t n,
@@ -1649,6 +1660,16 @@ int gs_list_sample_weighted(const float* probs, const int64_t* range, int64_t n,
                             uint64_t call_id, int64_t* out_range, int64_t total_picks,
                             int64_t* out_index, void* workspace, size_t workspace_bytes,
                             gs_stream_t stream) {
+  return gs_list_sample_weighted_values(probs, range, n, num_segments, num_picks, replace, seed,
+                                        call_id, out_range, total_picks, out_index, nullptr,
+                                        workspace, workspace_bytes, stream);
+}
+
+int gs_list_sample_weighted_values(const float* probs, const int64_t* range, int64_t n,
+                                   int64_t num_segments, int64_t num_picks, int replace,
+                                   uint64_t seed, uint64_t call_id, int64_t* out_range,
+                                   int64_t total_picks, int64_t* out_index, float* out_value,
+                                   void* workspace, size_t workspace_bytes, gs_stream_t stream) {
   using namespace gs;
   const bool begin = total_picks > 0 && n > 0 && num_segments >= 1 && num_segments < kBlock &&
                      (range != nullptr || num_segments == 1) && out_range &&
@@ -1670,7 +1691,7 @@ int gs_list_sample_weighted(const float* probs, const int64_t* range, int64_t n,
     if (rc != GS_OK) return rc;
   }
   return list_fill(probs, range, n, num_segments, num_picks, replace, seed, call_id, out_range,
-                   total_picks, out_index, workspace, workspace_bytes, stream, begin);
+                   total_picks, out_index, out_value, workspace, workspace_bytes, stream, begin);
 }
 
 }  // extern "C"

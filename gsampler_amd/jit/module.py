@@ -176,6 +176,7 @@ class compile:  # noqa: N801 -- the reference's public name
         passes.sum_encoded_slices_in_place(graph)
         passes.normalise_columns(graph)
         passes.share_leading_rows(graph)
+        passes.weights_of_picks(graph)
         return fx.GraphModule(gm, graph).forward
 
     def __call__(self, *args):

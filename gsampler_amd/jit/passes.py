@@ -39,6 +39,7 @@ and, in the copy of the graph that calls run (like chain_layers):
                                 never written
   normalise_columns             edge values divided by row and by their columns' sums
   share_leading_rows            features of all rows of a column slice: the parent's, once
+  weights_of_picks              picks of a list by weight and their weights  -> one operator
 
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
 whoever runs the passes (gm.recompile()): generating it after each of them was
@@ -1007,6 +1008,43 @@ def sum_encoded_slices_in_place(copy: fx.Graph) -> None:
             node.replace_input_with(node.args[0], node.args[0].args[0])
         _drop_dead_nodes(copy, [total])
         order = {n: i for i, n in enumerate(copy.nodes)}
+
+
+def weights_of_picks(copy: fx.Graph) -> None:
+    """In a copy of a graph: picks of a list by its weights, and weights[picks]  => one
+    _picks_and_weights."""
+    from ..ops.fused_op import _picks_and_weights
+    order = {n: i for i, n in enumerate(copy.nodes)}
+    names = {"_CAPI_ListSamplingWithProbs": 3, "_CAPI_BatchListSamplingWithProbs": 4}
+    replaced = []
+    for node in list(copy.nodes):
+        if node.op != "call_function" or node.kwargs:
+            continue
+        name = str(getattr(node.target, "__name__", node.target)).split(".")[0]
+        if len(node.args) != names.get(name) or not isinstance(node.args[0], fx.Node):
+            continue
+        batched = len(node.args) == 4
+        if batched and any(not _call(u, operator.getitem) or u.args[1] not in (0, 1) for u in node.users):
+            continue
+        picks = _getitem_users(node, 0) if batched else [node]
+        weights = [u for u in node.args[0].users if _call(u, operator.getitem)
+                   and u.args[0] is node.args[0] and any(u.args[1] is p for p in picks)]
+        if not weights or _written_between(order, [node, *weights]):
+            continue
+        with copy.inserting_before(node):
+            both = copy.call_function(_picks_and_weights, args=node.args)
+            parts = [copy.call_function(operator.getitem, args=(both, i)) for i in range(3)]
+        for w in weights:
+            w.replace_all_uses_with(parts[2])
+        if batched:
+            for i in (0, 1):
+                for u in _getitem_users(node, i):
+                    u.replace_all_uses_with(parts[i])
+        else:
+            node.replace_all_uses_with(parts[0])
+        replaced += [node, *weights]
+    if replaced:
+        _drop_dead_nodes(copy, replaced)
 
 
 def share_leading_rows(copy: fx.Graph) -> None:

@@ -120,6 +120,18 @@ def _encoded_row_slice(part, row_ids, rows_ptr, rows=None):
     return (sub, index) if rows is None else (sub, index, rows[row_ids])
 
 
+def _picks_and_weights(probs, num_picks, replace, ranges=None):
+    """(picks of a list by weight, their offsets in a list cut by `ranges`, probs[picks])."""
+    out = _library.native.list_sampling(probs, num_picks, replace, ranges)
+    if out is not None:
+        return out
+    if ranges is None:
+        picks, offsets = torch.ops.gs_ops._CAPI_ListSamplingWithProbs(probs, num_picks, replace), None
+    else:
+        picks, offsets = torch.ops.gs_ops._CAPI_BatchListSamplingWithProbs(probs, num_picks, replace, ranges)
+    return picks, offsets, probs[picks]
+
+
 def _leading_rows(x, n):
     """x[torch.arange(n)], to be read only: a view where that is the same."""
     if (type(x) is torch.Tensor and x.is_cuda and x.dim() >= 1 and x.is_contiguous()

@@ -313,7 +313,8 @@ int gs_weighted_key_probe(uint64_t seed, uint64_t call_id, uint64_t pos,
  *    the min(K, n_b) smallest keys in ascending key order (a segment with
  *    n_b <= K keeps its order); with replacement K picks through an integer
  *    CDF (stream pos = segment, draw = pick).  The form without a suffix is both in
- *    one call, for a caller that knows the number of picks.  ListSamplingProbsCUDA
+ *    one call, for a caller that knows the number of picks; the one of that name with
+ *    `values` also writes the picks' weights to out_value.  ListSamplingProbsCUDA
  *    (src/cuda/list_sampling_probs.cu:85-89), BatchListSamplingProbsCUDA
  *    (src/cuda/batch/list_sampling_probs.cu:102-107; the reference rejects
  *    replace there).
@@ -341,6 +342,13 @@ int gs_list_sample_weighted(const float* probs, const int64_t* range,
                             int64_t total_picks, int64_t* out_index,
                             void* workspace, size_t workspace_bytes,
                             gs_stream_t stream);
+int gs_list_sample_weighted_values(const float* probs, const int64_t* range,
+                                   int64_t n, int64_t num_segments,
+                                   int64_t num_picks, int replace, uint64_t seed,
+                                   uint64_t call_id, int64_t* out_range,
+                                   int64_t total_picks, int64_t* out_index, float* out_value,
+                                   void* workspace, size_t workspace_bytes,
+                                   gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Unique in first-occurrence order + relabel, for one batch or a super-batch.

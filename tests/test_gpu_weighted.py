@@ -333,6 +333,68 @@ def test_list_sampling_in_one_call(nseg, k, replace):
         same((out, out_range), (want, want_range))
 
 
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("n,k", [(100, 7), (100, 200), (9000, 400), (9000, 2049), (700_000, 512)])
+def test_picks_come_with_their_weights(n, k, replace):
+    """Selected, sorted, taken whole and drawn with replacement, from one list and from one
+    cut into segments; a compiled sampler asks for both at once."""
+    from gsampler_amd.ops import fused_op
+    rng = np.random.default_rng(n + k)
+    probs = F(rng.random(n).astype(np.float32))
+    ranges = T(np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=4)), [n]]))
+    ops = torch.ops.gs_ops
+    for r in (None, ranges):
+        def run(fused):
+            gs.manual_seed(11)
+            if fused:
+                return fused_op._picks_and_weights(probs, k, replace, r)
+            if r is None:
+                return (ops._CAPI_ListSamplingWithProbs(probs, k, replace),)
+            return ops._CAPI_BatchListSamplingWithProbs(probs, k, replace, r)
+        got, want = run(True), run(False)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[2], probs[want[0]])
+        assert r is None or torch.equal(got[1], want[1])
+    with_grad = probs.clone().requires_grad_()
+    gs.manual_seed(11)
+    picks, _, weights = fused_op._picks_and_weights(with_grad, k, replace)
+    weights.sum().backward()
+    assert torch.equal(with_grad.grad, torch.bincount(picks, minlength=n).float())
+
+
+def picks(A, seeds, K, probs):
+    sub = A[:, seeds]
+    picked, index = sub.collective_sampling(K, probs, False)
+    return picked.div("w", probs[index], axis=1).edata["w"], index
+
+
+def picks_of_changed_weights(A, seeds, K, probs):
+    probs = probs * 1.0
+    sub = A[:, seeds]
+    picked, index = sub.collective_sampling(K, probs, False)
+    doubled = probs.mul_(2.0)
+    return picked.div("w", probs[index], axis=1).edata["w"], index, doubled
+
+
+@pytest.mark.parametrize("func,fused", [(picks, True), (picks_of_changed_weights, False)])
+def test_compiled_samplers_read_the_weights_of_their_picks_once(func, fused):
+    from gsampler_amd.ops import fused_op
+    rng = np.random.default_rng(3)
+    indptr, indices = random_csc(rng, 500, 400, 60)
+    m = gs.Matrix()
+    m.load_graph("CSC", [T(indptr), T(indices)])
+    m.edata["w"] = F(rng.random(indices.size).astype(np.float32))
+    args = (m, T(rng.permutation(500)[:60]), 50, F(rng.random(m.num_rows()).astype(np.float32)))
+    compiled = gs.jit.compile(func=func, args=args)
+    targets = [n.target for n in compiled._run.__self__.graph.nodes]
+    assert (fused_op._picks_and_weights in targets) == fused
+    gs.manual_seed(2)
+    got = compiled(*args)
+    gs.manual_seed(2)
+    want = func(*args)
+    # (the formats that a compiled sampler takes put the edges in another order)
+    assert torch.equal(got[1], want[1]) and torch.equal(got[0].sort().values, want[0].sort().values)
+
+
 def test_operators_through_the_api():
     rng = np.random.default_rng(6)
     indptr, indices = random_csc(rng, 500, 400, 60)
