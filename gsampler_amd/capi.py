@@ -96,6 +96,7 @@ SIGNATURES = {
     "gs_sddmm": (_int, [_int, _p, _p, _i64, _i64, _p, _int, _int, _p, _p, _p, _int, _int,
                         _i64, _i64, _i64, _i64, _p, _p, _p]),
     "gs_normalise_columns": (_int, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _p]),
+    "gs_normalise_columns_cleared": (_int, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _p]),
     "gs_edge_score": (_int, [_int, _p, _p, _i64, _i64, _p, _p, _int, _i64, _p, _int, C.c_float,
                              _p, _p]),
     "gs_fused_u_op_v": (_int, [_int, _p, _p, _i64, _i64, _p, _int, _int, _p, _p, _p, _p, _p,
@@ -113,7 +114,7 @@ SIGNATURES = {
     "gs_col_row_slice_count": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p, _p,
                                       _sz, _p]),
     "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
-                                            _p, _p, _sz, _p]),
+                                            _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),
     "gs_col_row_slice_fill": (_int, [_p, _p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "gs_probe_stream_copy": (_int, [_p, _p, _i64, _p]),
@@ -128,6 +129,8 @@ SIGNATURES = {
     "gs_sliced_e_square_sum_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_sliced_e_square_sum": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _i64, _p, _sz,
                                       _p]),
+    "gs_sliced_e_square_sums": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _p, _p, _i64, _p, _sz,
+                                       _p]),
     "gs_weight_cdf_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_weight_cdf_build": (_int, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _sz, _p]),
     "gs_csc_col_sample_weighted_fill": (_int, [_p, _i64, _p, _p, _p, _p, _i64, _i64, _int, _u64,
@@ -764,13 +767,14 @@ def minor_slice(ids, picked, indptr=None, edge_major=None, with_major=True):
 
 
 def col_row_slice(indptr, indices, cols, rows, key_offset=None, with_major=True,
-                  indices32=None, out_first=None):
+                  indices32=None, out_first=None, col_zeros=None):
     """A[rows, cols] read from the parent matrix, the column slice never written.
     -> (out_indptr[len(cols) + 1], out_major | None = position of the edge's column in
     `cols`, out_minor = position of its row in `rows`, out_select = its position in the
     parent's `indices`).  `key_offset[len(cols)]` is added to the row ids of a column's
     edges before they are looked up among `rows`.  `out_first[len(rows)]`: receives the first
-    edge of the column slice that is kept as each of `rows` (2^63 - 1 where none is)."""
+    edge of the column slice that is kept as each of `rows` (2^63 - 1 where none is).
+    `col_zeros[len(cols)]` (float64) is cleared."""
     indptr, indices = _i64t(indptr, "indptr"), _i64t(indices, "indices")
     cols, rows = _i64t(cols, "cols"), _i64t(rows, "rows")
     if key_offset is not None:
@@ -786,7 +790,8 @@ def col_row_slice(indptr, indices, cols, rows, key_offset=None, with_major=True,
     check(l.gs_col_row_slice_count_first(
         _ptr(indptr), _ptr(indices), indices32.data_ptr() if indices32 is not None else None,
         _ptr(cols), _ptr(key_offset), ncol, sub_indptr.data_ptr(), nnz, _ptr(rows), nrow,
-        out_indptr.data_ptr(), total.data_ptr(), _ptr(out_first), ws.data_ptr(), ws.numel(),
+        out_indptr.data_ptr(), total.data_ptr(), _ptr(out_first),
+        col_zeros.data_ptr() if col_zeros is not None else None, ws.data_ptr(), ws.numel(),
         _stream()))
     kept = int(total.item())
     out_minor = torch.empty(kept, dtype=torch.int64, device=dev)

@@ -164,19 +164,13 @@ static EncodedSumsWs carve_encoded_sums(void* ws, int64_t nnz, int64_t range) {
   w.rows.group_cnt = c.take<int64_t>((size_t)w.rows.groups);
   w.rows.group_off = c.take<int64_t>((size_t)w.rows.groups + 1);
   w.sums = c.take<float>((size_t)w.rows.groups * kCompactGroup);
-  w.sum_ws_bytes = sliced_square_sum_bytes(nnz, range);
+  w.sum_ws_bytes = sliced_square_sum_bytes(nnz, w.rows.groups * kCompactGroup);
   w.sum_ws = c.take<uint8_t>(w.sum_ws_bytes);
   w.total = c.total();
   return w;
 }
 
 constexpr uint32_t kMinusZero = 0x80000000u;
-
-__global__ __launch_bounds__(kBlock) void encoded_sums_clear_kernel(uint4* sums, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * kBlock;
-  for (; i < n; i += stride) sums[i] = make_uint4(kMinusZero, kMinusZero, kMinusZero, kMinusZero);
-}
 
 __device__ __forceinline__ bool compact_flag(uint8_t flag) { return flag != 0; }
 __device__ __forceinline__ bool compact_flag(float sum) { return __float_as_uint(sum) != kMinusZero; }
@@ -455,7 +449,8 @@ int gs_encoded_square_sums_pay(int64_t nnz, int64_t num_batches, int64_t stride)
       num_batches > ((int64_t(1) << 31) - 1) / stride)
     return 0;
   const int64_t keys = num_batches * stride;
-  if (nnz >= (int64_t(1) << 20)) return gs::sums_by_range(nnz, keys) ? 1 : 0;
+  if (nnz >= (int64_t(1) << 20))
+    return gs::sums_by_range(nnz, gs::ceil_div(keys, gs::kCompactGroup) * gs::kCompactGroup) ? 1 : 0;
   return keys <= (int64_t(1) << 22) || keys / 16 <= nnz ? 1 : 0;
 }
 
@@ -481,18 +476,12 @@ int gs_encoded_square_sums(const int64_t* indptr, const int64_t* indices, const 
     return GS_ERR_WORKSPACE;
   }
   hipStream_t s = as_stream(stream);
-  const int64_t vecs = w.rows.groups * (kCompactGroup / 4);
-  int64_t blocks = ceil_div(vecs, kBlock * 4);
-  if (blocks > 8192) blocks = 8192;
-  GS_LAUNCH("encoded_sums_clear", s,
-            encoded_sums_clear_kernel<<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(
-                (uint4*)w.sums, vecs));
-  if (nnz > 0) {
-    const SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
-    rc = sliced_square_sum(view, indices, indices32, nnz, edge_map, efeat, w.sums, range, w.sum_ws,
-                           w.sum_ws_bytes, s);
-    if (rc != GS_OK) return rc;
-  }
+  // (all groups whole, so that those of the last one past the keys count as none too)
+  const SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
+  rc = sliced_square_sum(view, indices, indices32, nnz, edge_map, efeat, w.sums,
+                         w.rows.groups * kCompactGroup, w.sum_ws, w.sum_ws_bytes, s,
+                         SumsOnto{true, -0.f});
+  if (rc != GS_OK) return rc;
   GS_LAUNCH("compact_words", s,
             compact_words_kernel<float><<<dim3((unsigned)w.rows.groups), dim3(kBlock), 0, s>>>(
                 w.sums, w.rows.words, w.rows.group_cnt));

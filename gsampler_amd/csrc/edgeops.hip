@@ -459,10 +459,10 @@ __global__ __launch_bounds__(kBlock) void spmm_fold_kernel(
   if (acc != 0.f) out[i] += acc;
 }
 
-__global__ __launch_bounds__(kBlock) void spmm_zero_kernel(float* p, int64_t n) {
+__global__ __launch_bounds__(kBlock) void spmm_zero_kernel(float* p, int64_t n, float value) {
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kBlock)
-    p[i] = 0.f;
+    p[i] = value;
 }
 
 // Per-die copies pay off when there are many edges per output row.
@@ -1248,9 +1248,10 @@ constexpr int kFoldShares = kBlock / kFoldLanes;
 static_assert(kRangeRows % kFoldRows == 0, "the rows of a work-group share a range");
 
 // range_units: null when every range has `parts` units, one range after the other.
+// onto.fresh: `out` need not have been cleared (a launch of 2 to 4 us and the way to it).
 __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
     const float* __restrict__ partial, const RangeUnits* __restrict__ range_units, int parts,
-    int64_t num_out, float* __restrict__ out) {
+    int64_t num_out, float* __restrict__ out, SumsOnto onto) {
   __shared__ double share_sum[kFoldShares][kFoldRows];
   const int share = threadIdx.x / kFoldLanes, lane_row = threadIdx.x % kFoldLanes * 4;
   const int64_t row0 = (int64_t)blockIdx.x * kFoldRows;
@@ -1284,7 +1285,9 @@ __global__ __launch_bounds__(kBlock) void rowsum_fold_kernel(
   double sum = -0.0;
 #pragma unroll
   for (int s = 0; s < kFoldShares; ++s) sum += share_sum[s][threadIdx.x];
-  if (__double_as_longlong(sum) != INT64_MIN) out[i] += (float)sum;  // INT64_MIN: the bits of -0
+  const bool any = __double_as_longlong(sum) != INT64_MIN;  // (the bits of -0)
+  if (onto.fresh) out[i] = any ? onto.base + (float)sum : onto.base;
+  else if (any) out[i] += (float)sum;
 }
 
 // dst_ids32: the same ids as dst_ids in 32 bits (a matrix's narrow copy), read
@@ -1293,7 +1296,8 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
                          const int64_t* src_ids, const int64_t* edge_map,
                          int64_t nnz, int64_t num_out, int kind, int op,
                          const float* ufeat, const float* efeat, float* out,
-                         void* workspace, hipStream_t s, SliceView view = no_view()) {
+                         void* workspace, hipStream_t s, SliceView view = no_view(),
+                         SumsOnto onto = {}) {
   char* ws = (char*)workspace;
   uint32_t* cells = (uint32_t*)(ws + p.off_cells);
   uint16_t* rows = (uint16_t*)(ws + p.off_rows);
@@ -1325,7 +1329,7 @@ static int row_range_sum(const RowRangePlan& p, const int64_t* dst_ids, const in
                 rows, values, cells, p.tile_stride, units, unit_total, partial));
   GS_LAUNCH("rowsum_fold", s,
             rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
-                                 s>>>(partial, range_units, 0, num_out, out));
+                                 s>>>(partial, range_units, 0, num_out, out, onto));
   return GS_OK;
 }
 
@@ -1444,11 +1448,12 @@ size_t sliced_square_sum_bytes(int64_t nnz, int64_t num_out) {
 
 int sliced_square_sum(SliceView view, const int64_t* indices, const int32_t* indices32,
                       int64_t nnz, const int64_t* edge_map, const float* efeat, float* out,
-                      int64_t num_out, void* workspace, size_t workspace_bytes, hipStream_t s) {
+                      int64_t num_out, void* workspace, size_t workspace_bytes, hipStream_t s,
+                      SumsOnto onto) {
   const RowRangePlan plan = row_range_plan(GS_FMT_COO, nnz, num_out);
   if (plan.total > 0 && workspace != nullptr && workspace_bytes >= plan.total)
     return row_range_sum(plan, indices, indices32, nullptr, edge_map, nnz, num_out, 1,
-                         kOpCopyRhs, nullptr, efeat, out, workspace, s, view);
+                         kOpCopyRhs, nullptr, efeat, out, workspace, s, view, onto);
   const RowScanPlan scan = row_scan_plan(nnz, num_out);
   if (scan.total > 0 && workspace != nullptr && workspace_bytes >= scan.total) {
     float* partial = (float*)workspace;
@@ -1463,9 +1468,16 @@ int sliced_square_sum(SliceView view, const int64_t* indices, const int32_t* ind
 #undef GS_ROWSUM_SCAN
     GS_LAUNCH("rowsum_fold", s,
               rowsum_fold_kernel<<<dim3((unsigned)ceil_div(num_out, kFoldRows)), dim3(kBlock), 0,
-                                   s>>>(partial, nullptr, (int)scan.parts, num_out, out));
+                                   s>>>(partial, nullptr, (int)scan.parts, num_out, out, onto));
     return GS_OK;
   }
+  if (onto.fresh) {
+    const int64_t blocks = ceil_div(num_out, (int64_t)kBlock * 4);
+    GS_LAUNCH("spmm_zero", s,
+              spmm_zero_kernel<<<dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(kBlock), 0,
+                                 s>>>(out, num_out, onto.base));
+  }
+  if (nnz == 0) return GS_OK;
   // short slices: combined per tile in LDS, one atomic per (tile, row present);
   // ids outside [0, num_out) cannot occur for a slice of a checked matrix
   return coo_sum_launch(indices, indices, edge_map, nnz, 1, kOpCopyRhs, nullptr, efeat, out,
@@ -1508,7 +1520,7 @@ static int spmm_launch(int format, const int64_t* a, const int64_t* b,
         if (zb > 4096) zb = 4096;
         GS_LAUNCH("spmm_zero", s,
                   spmm_zero_kernel<<<dim3((unsigned)zb), dim3(kBlock), 0, s>>>(
-                      copies, total));
+                      copies, total, 0.f));
         GS_LAUNCH("spmm_coo_sum", s,
                   spmm_coo_sum_kernel<<<grid, dim3(kBlock), 0, s>>>(
                       a, b, edge_map, nnz, kind, op, ufeat, efeat, copies,
@@ -1691,6 +1703,19 @@ int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t*
                          int64_t nnz, const float* values, int64_t num_values,
                          const int64_t* select, const float* row_divisor, double* sums, float* out,
                          gs_stream_t stream) {
+  if (nnz > 0 && num_cols > 0 && sums)
+    GS_LAUNCH("normalise_clear", gs::as_stream(stream),
+              gs::normalise_clear_kernel<<<dim3((unsigned)gs::ceil_div(num_cols, gs::kBlock)),
+                                           dim3(gs::kBlock), 0, gs::as_stream(stream)>>>(sums,
+                                                                                        num_cols));
+  return gs_normalise_columns_cleared(indptr, num_cols, rows, nnz, values, num_values, select,
+                                      row_divisor, sums, out, stream);
+}
+
+int gs_normalise_columns_cleared(const int64_t* indptr, int64_t num_cols, const int64_t* rows,
+                                 int64_t nnz, const float* values, int64_t num_values,
+                                 const int64_t* select, const float* row_divisor, double* sums,
+                                 float* out, gs_stream_t stream) {
   using namespace gs;
   GS_REQUIRE(num_cols >= 0 && nnz >= 0, "normalise_columns: negative size");
   if (nnz == 0) return GS_OK;
@@ -1700,9 +1725,6 @@ int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t*
              (long long)num_values);
   hipStream_t s = as_stream(stream);
   const dim3 grid((unsigned)ceil_div(nnz, (int64_t)kSumTile));
-  GS_LAUNCH("normalise_clear", s,
-            normalise_clear_kernel<<<dim3((unsigned)ceil_div(num_cols, kBlock)), dim3(kBlock), 0,
-                                     s>>>(sums, num_cols));
 #define GS_NORMALISE_SUM(SELECT, DIVIDE)                                                     \
   GS_LAUNCH("normalise_sum", s,                                                              \
             (normalise_sum_kernel<SELECT, DIVIDE>)<<<grid, dim3(kBlock), 0, s>>>(            \
@@ -1822,6 +1844,23 @@ int gs_sliced_e_square_sum(const int64_t* indptr, const int64_t* indices,
   const SliceView view{sub_indptr, cols, indptr, nullptr, num_cols_picked};
   return sliced_square_sum(view, indices, indices32, slice_nnz, edge_map, efeat, out, num_out,
                            workspace, workspace_bytes, as_stream(stream));
+}
+
+int gs_sliced_e_square_sums(const int64_t* indptr, const int64_t* indices,
+                            const int32_t* indices32, const int64_t* cols,
+                            int64_t num_cols_picked, const int64_t* sub_indptr,
+                            int64_t slice_nnz, const int64_t* edge_map, const float* efeat,
+                            float* out, int64_t num_out, void* workspace, size_t workspace_bytes,
+                            gs_stream_t stream) {
+  using namespace gs;
+  GS_REQUIRE(num_cols_picked >= 0 && slice_nnz >= 0 && num_out >= 0,
+             "sliced_e_square_sums: negative size");
+  if (num_out == 0) return GS_OK;
+  GS_REQUIRE(out && (slice_nnz == 0 || (indptr && indices && cols && sub_indptr && efeat)),
+             "sliced_e_square_sums: null pointer");
+  const SliceView view{sub_indptr, cols, indptr, nullptr, num_cols_picked};
+  return sliced_square_sum(view, indices, indices32, slice_nnz, edge_map, efeat, out, num_out,
+                           workspace, workspace_bytes, as_stream(stream), SumsOnto{true, 0.f});
 }
 
 int gs_e_div_u_sum(int format, const int64_t* a, const int64_t* b,

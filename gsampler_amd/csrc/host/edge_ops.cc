@@ -266,12 +266,19 @@ c10::optional<torch::Tensor> Graph::NormaliseColumns(torch::Tensor values,
     row_divisor = row_divisor->contiguous();
   }
   torch::Tensor out = torch::empty({num_edges_}, values.options().requires_grad(false));
-  torch::Tensor sums = torch::empty({num_cols_}, out.options().dtype(torch::kFloat64));
-  GS_CALL(gs_normalise_columns(cptr(csc_->indptr), num_cols_, cptr(csc_->indices), num_edges_,
-                               values.data_ptr<float>(), values.size(0),
-                               select.has_value() ? cptr(*select) : nullptr,
-                               row_divisor.has_value() ? row_divisor->data_ptr<float>() : nullptr,
-                               sums.data_ptr<double>(), out.data_ptr<float>(), cur_stream()));
+  torch::Tensor sums;  // (of 64 bits: the slice that made this matrix may have left them cleared)
+  {
+    std::lock_guard<std::mutex> lock(column_zeros_guard_);
+    std::swap(sums, column_zeros_);
+  }
+  const bool cleared = sums.defined() && sums.numel() == num_cols_;
+  if (!cleared) sums = new_ids(num_cols_, csc_->indptr);
+  auto* normalise = cleared ? &gs_normalise_columns_cleared : &gs_normalise_columns;
+  GS_CALL(normalise(cptr(csc_->indptr), num_cols_, cptr(csc_->indices), num_edges_,
+                    values.data_ptr<float>(), values.size(0),
+                    select.has_value() ? cptr(*select) : nullptr,
+                    row_divisor.has_value() ? row_divisor->data_ptr<float>() : nullptr,
+                    (double*)mptr(sums), out.data_ptr<float>(), cur_stream()));
   return out;
 }
 

@@ -6,6 +6,9 @@
 // shape of a layer-wise sampler (examples/ladies/ladies.py:7-21 of the
 // reference); the reference fuses the second pair only, and only for
 // super-batches (src/cuda/fusion/column_row_slicing.cu).
+#include <ATen/autocast_mode.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+
 #include "abi_call.h"
 #include "graph.h"
 
@@ -102,12 +105,34 @@ void Graph::SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Ten
                                  ws.data_ptr(), (size_t)ws.numel(), cur_stream()));
 }
 
+c10::optional<torch::Tensor> Graph::SlicedSquareSums(torch::Tensor cols, torch::Tensor efeat) {
+  const Compressed& m = compressed(kCSC);
+  if (!plain_values(efeat, true) || efeat.dim() != 1 || !efeat.is_contiguous() ||
+      efeat.numel() != m.indices.numel() || !m.indices.is_cuda() ||
+      at::impl::torch_function_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA))
+    return {};
+  cols = ids(cols, "cols");
+  const std::shared_ptr<SliceOffsets> so = slice_offsets_for(cols);
+  torch::Tensor out = torch::empty({num_rows_}, efeat.options().requires_grad(false));
+  torch::Tensor ws = new_workspace(gs_sliced_e_square_sum_workspace_bytes(so->nnz, num_rows_),
+                                   m.indptr);
+  const torch::Tensor e_ids = m.e_ids.has_value() ? m.e_ids.value() : torch::Tensor();
+  const torch::Tensor narrow = narrow_for_slice(m, so->nnz, cols.numel());
+  GS_CALL(gs_sliced_e_square_sums(cptr(m.indptr), cptr(m.indices),
+                                  narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+                                  cptr(cols), cols.numel(), cptr(so->sub_indptr), so->nnz,
+                                  cptr(e_ids), efeat.data_ptr<float>(), out.data_ptr<float>(),
+                                  num_rows_, ws.data_ptr(), (size_t)ws.numel(), cur_stream()));
+  return out;
+}
+
 // Shared by the plain and the super-batched form.  key_offset (per picked
 // column) and `picked` carry the batch in their values when there are batches.
 static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
                                  const torch::Tensor& sub_indptr, int64_t nnz,
                                  const torch::Tensor& key_offset, const torch::Tensor& picked,
-                                 bool with_coo, torch::Tensor* firsts = nullptr) {
+                                 bool with_coo, torch::Tensor* firsts = nullptr,
+                                 torch::Tensor* zeros = nullptr) {
   const int64_t n = cols.numel(), np = picked.numel();
   MajorResult r;
   torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, np), m.indptr);
@@ -118,12 +143,18 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
   AsyncCount kept = AsyncCount::mirrored();
   const torch::Tensor narrow = narrow_for_slice(m, nnz, n);
   // (the relabel of a slice with far fewer rows than edges goes by its rows' first edges)
-  if (firsts && nnz >= 8 * np && gs_col_row_slice_tells_first(nnz, np)) *firsts = new_ids(np, m.indptr);
+  // (and its edges' values are often divided by sums over their columns: cleared in passing)
+  const bool tells = firsts && nnz >= 8 * np && gs_col_row_slice_tells_first(nnz, np);
+  if (zeros) {
+    const torch::Tensor buffer = new_ids((tells ? np : 0) + n, m.indptr);
+    *zeros = piece_of(buffer, 0, n, false);
+    if (tells) *firsts = piece_of(buffer, n, np, false);
+  }
   GS_CALL(gs_col_row_slice_count_first(
       cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
       cptr(cols), cptr(key_offset), n, cptr(sub_indptr), nnz, cptr(picked), np, mptr(r.indptr),
-      kept.mirror(), firsts && firsts->defined() ? mptr(*firsts) : nullptr, ws.data_ptr(),
-      ws.numel(), cur_stream()));
+      kept.mirror(), tells ? mptr(*firsts) : nullptr, zeros ? (double*)mptr(*zeros) : nullptr,
+      ws.data_ptr(), ws.numel(), cur_stream()));
   kept.arm();
   const int64_t size = nnz <= kBoundLimit ? nnz : kept.get();
   r.minor_ids = new_ids(size, m.indptr);
@@ -153,10 +184,10 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(cols);
   SliceOffsets& so = *shared;
   MajorResult r;
-  torch::Tensor firsts;
+  torch::Tensor firsts, zeros;
   if (read_in_place(m, so.nnz, cols.numel())) {
     r = col_row_slice(m, cols, so.sub_indptr, so.nnz, torch::Tensor(), rows,
-                      output_format & kCOO, &firsts);
+                      output_format & kCOO, &firsts, &zeros);
   } else {
     const MajorResult& sliced = written_slice(so);
     Compressed tmp(sliced.indptr, sliced.minor_ids);
@@ -165,6 +196,7 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   }
   GraphPtr g = derive(kCSC, output_format, r, rows.numel(), cols.numel());
   g->keep_row_firsts(firsts, r.minor_ids);
+  g->column_zeros_ = zeros;
   return {g, edge_index(m.e_ids, r.select)};
 }
 
@@ -321,11 +353,12 @@ GraphAndIndex Graph::encoded_row_slice(const torch::Tensor& seeds, const torch::
   const Compressed& m = compressed(kCSC);
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(seeds);
   torch::Tensor key_offset = key_offsets_for(*shared, col_bptr);
-  torch::Tensor firsts;
+  torch::Tensor firsts, zeros;
   const MajorResult r = col_row_slice(m, seeds, shared->sub_indptr, shared->nnz, key_offset, picked,
-                                      true, &firsts);
+                                      true, &firsts, &zeros);
   GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
   g->keep_row_firsts(firsts, r.minor_ids);
+  g->column_zeros_ = zeros;
   g->col_bptr_ = col_bptr;
   g->orig_col_ids_ = seeds;
   g->row_encoding_size_ = num_rows_;

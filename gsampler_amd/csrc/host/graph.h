@@ -246,6 +246,8 @@ class Graph : public torch::CustomClassHolder {
   // straight from this matrix instead of from a written slice (fused_slices.cc).
   // out[row] += sum of efeat^2 over the edges of A[:, cols];
   void SlicedESquareSum(torch::Tensor cols, torch::Tensor efeat, torch::Tensor out);
+  // The sums alone; nothing where the call is not one for it (see EdgeScore).
+  c10::optional<torch::Tensor> SlicedSquareSums(torch::Tensor cols, torch::Tensor efeat);
   // A[rows, cols], the edge index addressing this matrix's edges.
   GraphAndIndex ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64_t on_format,
                               int64_t output_format);
@@ -523,6 +525,9 @@ class Graph : public torch::CustomClassHolder {
   // Which edge of a row slice is the first of each of its rows, as the pass that made the
   // slice has met them; nothing once the rows of the edges have been written to.
   torch::Tensor row_firsts_, row_firsts_of_;
+  // A value a column that is zero, for the first sum over columns that asks for one.
+  torch::Tensor column_zeros_;
+  std::mutex column_zeros_guard_;
   int64_t row_firsts_version_ = -1, row_firsts_epoch_ = -1;
   // The rows of the edges of A[list, list], while each is still a position of the list in the
   // segment of its edge's mini-batch: what the slice wrote.

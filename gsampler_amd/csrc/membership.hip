@@ -785,7 +785,8 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
     const uint8_t* __restrict__ staged_pos, const uint16_t* __restrict__ chunk_kept,
     int64_t nnz, int64_t* __restrict__ chunk_off, int64_t* __restrict__ out_indptr,
     int64_t* __restrict__ out_total, unsigned tiles, const uint32_t* __restrict__ firsts,
-    int64_t first_groups, int64_t num_picked, int64_t* __restrict__ out_first) {
+    int64_t first_groups, int64_t num_picked, int64_t* __restrict__ out_first,
+    double* __restrict__ col_zeros) {
   if (blockIdx.x >= tiles) {  // (there are such only where out_first is asked for)
     member_first(blockIdx.x - tiles, firsts, first_groups, num_picked, out_first);
     return;
@@ -850,6 +851,7 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
       r = base + before[i] + member_below(e, (int)(before[i + 1] - before[i]), staged_pos);
     }
     out_indptr[c] = r;
+    if (col_zeros && c < num_major) col_zeros[c] = 0.0;
   }
 }
 
@@ -857,11 +859,12 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
 __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
     const uint8_t* __restrict__ staged_pos, const int64_t* __restrict__ chunk_off,
-    int64_t nnz, int64_t* __restrict__ out_indptr, int64_t* __restrict__ out_total) {
+    double* __restrict__ col_zeros, int64_t nnz, int64_t* __restrict__ out_indptr, int64_t* __restrict__ out_total) {
   const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
   if (c == 0 && out_total) store_for_host(out_total, nnz > 0 ? chunk_off[num_chunks] : 0);
   if (indptr == nullptr || c > num_major) return;
+  if (col_zeros && c < num_major) col_zeros[c] = 0.0;
   const int64_t e = indptr[c];
   int64_t r = 0;
   if (nnz > 0) {
@@ -970,7 +973,8 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
                                   int64_t num_major, int64_t* out_indptr,
                                   int64_t* out_total, void* workspace,
                                   size_t workspace_bytes, gs_stream_t stream,
-                                  gs::SliceView view, int64_t* out_first = nullptr) {
+                                  gs::SliceView view, int64_t* out_first = nullptr,
+                                  double* col_zeros = nullptr) {
   using namespace gs;
   GS_REQUIRE(nnz >= 0 && num_picked >= 0 && num_major >= 0,
              "minor_slice_count: negative size");
@@ -1053,7 +1057,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
       GS_LAUNCH("member_offsets", s,
                 member_offsets_kernel<<<dim3(tiles + first_parts), dim3(kOffsetsThreads), 0, s>>>(
                     indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,
-                    out_total, tiles, firsts, blocks, num_picked, out_first));
+                    out_total, tiles, firsts, blocks, num_picked, out_first, col_zeros));
       return GS_OK;
     }
     if (out_first)
@@ -1068,7 +1072,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   GS_LAUNCH("member_indptr", s,
             member_indptr_kernel<<<dim3((unsigned)ceil_div(n, kBlock)),
                                    dim3(kBlock), 0, s>>>(indptr, num_major, w.staged_pos,
-                                                         w.chunk_off, nnz,
+                                                         w.chunk_off, col_zeros, nnz,
                                                          out_indptr, out_total));
   return GS_OK;
 }
@@ -1160,8 +1164,8 @@ int gs_col_row_slice_count(const int64_t* indptr, const int64_t* indices,
                            size_t workspace_bytes, gs_stream_t stream) {
   return gs_col_row_slice_count_first(indptr, indices, indices32, cols, key_offset,
                                       num_cols_picked, sub_indptr, slice_nnz, rows,
-                                      num_rows_picked, out_indptr, out_total, nullptr, workspace,
-                                      workspace_bytes, stream);
+                                      num_rows_picked, out_indptr, out_total, nullptr, nullptr,
+                                      workspace, workspace_bytes, stream);
 }
 
 int gs_col_row_slice_tells_first(int64_t slice_nnz, int64_t num_rows_picked) {
@@ -1175,14 +1179,15 @@ int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
                                  const int64_t* sub_indptr, int64_t slice_nnz,
                                  const int64_t* rows, int64_t num_rows_picked,
                                  int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
-                                 void* workspace, size_t workspace_bytes, gs_stream_t stream) {
+                                 double* col_zeros, void* workspace, size_t workspace_bytes,
+                                 gs_stream_t stream) {
   int rc = check_slice_view(indptr, indices, cols, num_cols_picked, sub_indptr, slice_nnz,
                             "col_row_slice_count");
   if (rc != GS_OK) return rc;
   const gs::SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
   return minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
                                 num_cols_picked, out_indptr, out_total, workspace,
-                                workspace_bytes, stream, view, out_first);
+                                workspace_bytes, stream, view, out_first, col_zeros);
 }
 
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,

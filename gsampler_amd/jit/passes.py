@@ -39,6 +39,7 @@ and, in the copy of the graph that calls run (like chain_layers):
                                 never written
   normalise_columns             edge values divided by row and by their columns' sums
   share_leading_rows            features of all rows of a column slice: the parent's, once
+  sum_slices_into_new_arrays    sums over a column slice that is not written
   weights_of_picks              picks of a list by weight and their weights  -> one operator
 
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
@@ -1043,6 +1044,37 @@ def weights_of_picks(copy: fx.Graph) -> None:
         else:
             node.replace_all_uses_with(parts[0])
         replaced += [node, *weights]
+    if replaced:
+        _drop_dead_nodes(copy, replaced)
+
+
+def sum_slices_into_new_arrays(copy: fx.Graph) -> None:
+    """In a copy of a graph: a cleared array, the squares of a column slice's values added to
+    it, and the array as it is then  => one _sliced_square_sums, which need not clear it."""
+    from ..ops.fused_op import _sliced_square_sums
+    order = {n: i for i, n in enumerate(copy.nodes)}
+    replaced = []
+    for total in list(copy.nodes):
+        if not _is_method(total, "_CAPI_SlicedESquareSum") or len(total.args) != 4 or total.users:
+            continue
+        g, cols, values, accumulator = total.args
+        if not (_call(accumulator, operator.getitem) and accumulator.args[1] == 0
+                and _is_wrapped(accumulator.args[0], "_before_spmm")):
+            continue
+        before = accumulator.args[0]
+        after = [n for n in accumulator.users if _is_wrapped(n, "_after_spmm")]
+        shape = before.args[1]
+        if (len(before.args) != 7 or list(before.args[2:5]) != ["copy_rhs", "sum", None]
+                or before.args[5] is not values or before.args[6] != 2
+                or not (_is_method(before.args[0], "_CAPI_GetNumRows") and before.args[0].args[0] is g)
+                or not (isinstance(shape, fx.Node) and _is_method(shape, "numel") and shape.args[0] is cols)
+                or len(after) != 1 or set(accumulator.users) != {total, after[0]}
+                or _written_between(order, [before, total, after[0]])):
+            continue
+        with copy.inserting_before(total):
+            new = copy.call_function(_sliced_square_sums, args=(g, cols, values))
+        after[0].replace_all_uses_with(new)
+        replaced.append(total)
     if replaced:
         _drop_dead_nodes(copy, replaced)
 

@@ -89,6 +89,17 @@ def _normalised(g, values, select, divisor, formats):
     return divided(e, _after_spmm(sums, squeeze), 2, formats[2])
 
 
+def _sliced_square_sums(g, cols, values):
+    """Sums of the squared values over the edges of the column slice g[:, cols] onto its rows."""
+    if type(values) is torch.Tensor and not values.requires_grad:
+        out = g._CAPI_SlicedSquareSums(cols, values)
+        if out is not None:
+            return out
+    out, _, _, squeeze = _before_spmm(g._CAPI_GetNumRows(), cols.numel(), "copy_rhs", "sum", None, values, 2)
+    g._CAPI_SlicedESquareSum(cols, values, out)
+    return _after_spmm(out, squeeze)
+
+
 def _encoded_square_sums(g, seeds, seeds_ptr, values, on_format):
     """What a compiled super-batched sampler asks an encoded column slice for: (the slice for
     _encoded_row_slice, its rows, where every batch's begin, sums of the squared values on

@@ -687,8 +687,9 @@ int gs_minor_slice_fill(const int64_t* ids, int64_t nnz, int64_t num_picked,
  *    are told apart as id + batch * stride on both sides.
  *    indices32 (nullable): the same row ids as `indices` in 32 bits; read instead
  *    of `indices` when given (half the bytes of the pass).
- *    count_first (where gs_col_row_slice_tells_first says 1): also, for every position in
- *    `rows`, out_first[num_rows_picked] = the first edge v of the slice that is kept as it,
+ *    count_first: also clears col_zeros[num_cols_picked] (nullable: the sums over columns that
+ *    are to be made of the kept edges), and, where gs_col_row_slice_tells_first says 1, for
+ *    every position in `rows` (nullable), out_first[num_rows_picked] = the first edge v of the slice that is kept as it,
  *    INT64_MAX where there is none -- ordered as the kept edges' places are, which
  *    gs_first_position tells of the output.
  *  fill: out_minor[kept] = position in `rows`, out_select[kept] = position of the
@@ -713,7 +714,8 @@ int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
                                  const int64_t* sub_indptr, int64_t slice_nnz,
                                  const int64_t* rows, int64_t num_rows_picked,
                                  int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
-                                 void* workspace, size_t workspace_bytes, gs_stream_t stream);
+                                 double* col_zeros, void* workspace, size_t workspace_bytes,
+                                 gs_stream_t stream);
 int gs_col_row_slice_tells_first(int64_t slice_nnz, int64_t num_rows_picked);
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,
                           int64_t num_cols_picked, const int64_t* sub_indptr,
@@ -874,7 +876,8 @@ int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int6
  *   values[select[e]] / row_divisor[rows[e]], select (identity) and row_divisor (ones)
  *   nullable, fp32; a place outside the num_values values reads 0, as gs_gather_rows has
  *   it.  Edges in column order, sums[num_cols] is scratch that ends up with the columns'
- *   sums.  q is rounded, sums are of 64 bits and rounded before they divide.
+ *   sums.  q is rounded, sums are of 64 bits and rounded before they divide.  The form with
+ *   `cleared` takes sums that are zero already, a launch less.
  * gs_spmm: out[dst] = reduce(out[dst], op(u[src], e[eid])), fp32.  Outputs
  *   are accumulators: the caller zero-fills them (python/gs/ops/spmm.py:56).
  *   COO: u_target 0 reduces onto columns, 2 onto rows (atomics).  Compressed:
@@ -911,6 +914,10 @@ int gs_normalise_columns(const int64_t* indptr, int64_t num_cols, const int64_t*
                          int64_t nnz, const float* values, int64_t num_values,
                          const int64_t* select, const float* row_divisor, double* sums, float* out,
                          gs_stream_t stream);
+int gs_normalise_columns_cleared(const int64_t* indptr, int64_t num_cols, const int64_t* rows,
+                                 int64_t nnz, const float* values, int64_t num_values,
+                                 const int64_t* select, const float* row_divisor, double* sums,
+                                 float* out, gs_stream_t stream);
 int gs_fused_u_op_v(int format, const int64_t* a, const int64_t* b,
                     int64_t num_major, int64_t nnz, const int64_t* edge_map,
                     int op, int dtype,
@@ -939,7 +946,8 @@ int gs_e_square_sum(int format, const int64_t* a, const int64_t* b,
  * caller zero-fills.  The workspace is optional
  * (NULL / 0 is valid, then every edge is an atomic add).  No counterpart in the
  * reference, which writes the slice and then runs ESquareSumCOO over it
- * (src/cuda/fusion/fused_coo_e_square_sum.cu:13-60). */
+ * (src/cuda/fusion/fused_coo_e_square_sum.cu:13-60).
+ * gs_sliced_e_square_sums: the same into an array that holds nothing yet. */
 size_t gs_sliced_e_square_sum_workspace_bytes(int64_t slice_nnz, int64_t num_out);
 int gs_sliced_e_square_sum(const int64_t* indptr, const int64_t* indices,
                            const int32_t* indices32, const int64_t* cols,
@@ -947,6 +955,12 @@ int gs_sliced_e_square_sum(const int64_t* indptr, const int64_t* indices,
                            int64_t slice_nnz, const int64_t* edge_map, const float* efeat,
                            float* out, int64_t num_out, void* workspace,
                            size_t workspace_bytes, gs_stream_t stream);
+int gs_sliced_e_square_sums(const int64_t* indptr, const int64_t* indices,
+                            const int32_t* indices32, const int64_t* cols,
+                            int64_t num_cols_picked, const int64_t* sub_indptr,
+                            int64_t slice_nnz, const int64_t* edge_map, const float* efeat,
+                            float* out, int64_t num_out, void* workspace,
+                            size_t workspace_bytes, gs_stream_t stream);
 int gs_e_div_u_sum(int format, const int64_t* a, const int64_t* b,
                    int64_t num_major, int64_t nnz, const int64_t* edge_map,
                    const float* ufeat, const float* efeat, float* out,

@@ -452,3 +452,51 @@ def test_relabel_of_the_subgraph_that_a_list_induces(sizes, order):
     assert len(results[0]) == len(results[1])
     for mine, general in zip(*results):
         assert torch.equal(mine, general)
+
+
+@pytest.mark.parametrize("rows", [1, 9000, 400_000])
+@pytest.mark.parametrize("nnz", [0, 1, 2047, 2048, 70_001, (1 << 21) + 3])
+def test_square_sums_into_an_array_that_holds_nothing(nnz, rows):
+    """By ranges that are partitioned, ranges that every work-group reads and atomics: the
+    same values as onto a cleared array, whatever the new one held."""
+    rng = np.random.default_rng(nnz + rows)
+    indices = T(np.minimum(rng.integers(0, rows, size=nnz + 5), rng.integers(0, rows, size=nnz + 5)))
+    indptr, cols = T([0, nnz // 3, nnz, nnz + 5]), T([1, 0])
+    w = torch.as_tensor(rng.integers(1, 3, size=nnz + 5).astype(np.float32), device=DEV)  # sums below 2^24
+    want = capi.sliced_e_square_sum(indptr, indices, cols, w, rows)
+    l = capi.lib()
+    sub = capi.col_count(indptr, cols, -1, False)
+    for size in (l.gs_sliced_e_square_sum_workspace_bytes(nnz, rows), 0):
+        ws = torch.empty(max(size, 1), dtype=torch.uint8, device=DEV)
+        out = torch.full((rows + 1,), 77.0, device=DEV)
+        capi.check(l.gs_sliced_e_square_sums(
+            indptr.data_ptr(), indices.data_ptr(), None, cols.data_ptr(), 2, sub.data_ptr(), nnz, None,
+            w.data_ptr(), out.data_ptr(), rows, ws.data_ptr() if size else None, size, None))
+        torch.cuda.synchronize()
+        assert torch.equal(out[:-1], want) and out[-1].item() == 77.0
+
+
+@pytest.mark.parametrize("nnz", [0, 5000, (1 << 25) + 1])
+def test_row_slices_clear_the_sums_of_their_columns(nnz):
+    indptr = T(np.sort(np.concatenate([[0, 0, nnz, nnz], np.random.default_rng(1).integers(0, nnz + 1, 700)])))
+    ncol = indptr.numel() - 1
+    zeros = torch.full((ncol + 1,), 5.0, dtype=torch.float64, device=DEV)
+    capi.col_row_slice(indptr, torch.zeros(max(nnz, 1), dtype=torch.int64, device=DEV),
+                       torch.arange(ncol, device=DEV), T([3, 0]), col_zeros=zeros)
+    assert not zeros[:-1].any() and zeros[-1].item() == 5.0
+
+
+def test_normalised_columns_of_one_slice_several_times():
+    """The first takes the sums that the slice left cleared, the next ones clear their own."""
+    rng = np.random.default_rng(4)
+    indptr, indices = random_csc(rng, 300, 2000, 90)
+    g = gs.Graph(2000, 300)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.random(indices.size).astype(np.float32) + 0.1, device=DEV)
+    sub, index = g._CAPI_ColRowSlicing(T(rng.permutation(300)[:200]), T(rng.permutation(2000)[:900]),
+                                       gs.format._CSC, gs.format._CSC | gs.format._COO)
+    got = [sub._CAPI_NormaliseColumns(w, index, None) for _ in range(3)]
+    assert all(torch.allclose(g, got[0], rtol=1e-6) for g in got)
+    col = torch.repeat_interleave(torch.arange(200, device=DEV), torch.diff(sub._CAPI_GetCSCIndptr()))
+    sums = torch.zeros(200, dtype=torch.float64, device=DEV).index_add_(0, col, w[index].double())
+    assert torch.allclose(got[0].double(), w[index].double() / sums[col], rtol=1e-6)
