@@ -76,6 +76,7 @@ SIGNATURES = {
     "gs_layer_max_positions": (_i64, []),
     "gs_layer_workspace_bytes": (_sz, [_i64, _int]),
     "gs_layer_begin": (_int, [_i64, _int, _p, _sz, _p]),
+    "gs_sample_layer_next": (_int, [_p, _p, _p]),
     "gs_sample_layer": (_int, [_p, _i64, _p, _p, _p, _i64, _p, _i64, _p, _i64, _i64, _int, _u64,
                                _u64, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _sz, _p]),
     "gs_slice_compact_workspace_bytes": (_sz, [_i64, _i64]),

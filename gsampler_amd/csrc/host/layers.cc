@@ -126,7 +126,15 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
     int64_t n = seeds.numel();
     bool known = true;
     size_t settled = 0;  // layers whose sizes are on the host
+    // A layer's labels wait for the next one's picks, beside which they run.
+    gs_layer unlabelled{};
+    auto label = [&] {
+      if (unlabelled.columns)
+        GS_CALL(gs_sample_layer_next(&unlabelled, nullptr, cur_stream()));
+      unlabelled = gs_layer{};
+    };
     auto settle = [&](size_t upto) {
+      label();
       for (; settled < upto; ++settled) {
         Queued& q = queued[settled];
         if (!q.buffer.defined()) continue;
@@ -165,6 +173,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           ptr = torch::arange(0, 2, device_options(m.indptr).dtype(torch::kInt64)) * n;
           BatchOffsets::trust(ptr, n);
         }
+        label();
         PinnedWords::arrived();  // every layer queued so far has been settled
         l = large_layer(cols, ptr, K, replace, cdf, first_call + i, labels, [&] { idle(out, i); });
         mirrors = nullptr;  // it has used the thread's pinned words
@@ -184,6 +193,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           std::swap(lw, layer_ws_);
       }
       if (lw.positions < positions) {
+        label();
         // room for the layers that can be queued behind this one as well
         int64_t most = positions, bound = positions;
         for (size_t j = i + 1; j < L && fits(bound, fanouts[j], kQueuedPositions); ++j) {
@@ -214,13 +224,15 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
       q.buffer = new_ids(at, m.indptr);
       q.mirror = mirrors + words * i;
       int64_t* base = mptr(q.buffer);
-      GS_CALL(gs_sample_layer(
+      const gs_layer next{
           cptr(m.indptr), num_cols, cptr(m.indices),
           narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, cptr(cdf), stride, cptr(cols), n,
           cptr(ptr), B, K, replace ? 1 : 0, rs.seed, first_call + i, base, base + q.at_ptr,
           base + q.at_row, base + q.at_col, base + q.at_edge_ptr,
           blocks ? base + q.at_indptr : nullptr, mirrors + words * i, lw.positions, lw.ws.data_ptr(),
-          (size_t)lw.ws.numel(), cur_stream()));
+          (size_t)lw.ws.numel(), (int)(i & 1)};
+      GS_CALL(gs_sample_layer_next(unlabelled.columns ? &unlabelled : nullptr, &next, cur_stream()));
+      unlabelled = next;
       // the next layer's columns, as far as they are known
       cols = piece_of(q.buffer, 0, positions, false);
       ptr = piece_of(q.buffer, q.at_ptr, B + 1, false);

@@ -19,8 +19,14 @@
 //           are edges; counts per tile of 1024 positions
 //   label   every work-group adds up the tiles' counts for itself (at most 1024),
 //           then writes frontier, labels and offsets of its tile, and empties its
-//           share of the table for the next layer.  Work-group 0 reports the
+//           share of the table for the layer after the next.  Work-group 0 reports the
 //           offsets of all batches to the host.
+// A layer whose columns are the frontier of one that is queued ahead of it does not wait
+// for that one's labels: its pick finds column c by the tiles' counts, in the list of new keys
+// that flag left of each tile, and runs beside the label pass in one launch, with a table of its
+// own.  L layers are 2 L + 1 dependent launches.
+// GraphSAGE [25,10], 1024 seeds: six launches 44.5 us, label 6.0 and pick 9.2 of them; five
+// 39.5, the two together 10.8 (51.5 and 47.1 us a pass).
 // The number of columns is read from the device (the last entry of the previous
 // layer's frontier offsets), launches are sized by its bound, and nothing is waited
 // for between layers.
@@ -37,6 +43,8 @@
 namespace gs {
 
 constexpr int kPickThreads = 512;
+constexpr int kLayerMaxBatches = 511;  // whose offsets a pick beside the labels finds for itself
+static_assert(kLayerMaxBatches < kPickThreads, "a thread a batch");
 constexpr int kPickSlots = 1024;  // LDS table of a work-group's keys, at most half full
 constexpr int kPickShift = 22;    // 32 - log2(kPickSlots)
 constexpr int kLayerTile = 1024;  // positions per work-group of flag and label
@@ -55,10 +63,10 @@ struct alignas(16) LayerWord {
 };
 
 struct LayerWs {
-  uint64_t* table;     // [slots] key << 32 | first position, empty between layers
+  uint64_t* table[2];  // [slots] key << 32 | first position, empty when a layer begins with it
   uint32_t* slot;      // [positions] slot of the position's key, kNoSlot: no key here
   uint32_t* first;     // [positions] first position of the key
-  uint32_t* key;       // [positions] the key, written where it occurs first
+  uint32_t* key;       // [positions] a tile's new keys in order, from its first position on
   LayerWord* words;    // [tiles * kLayerWords]
   uint2* tile_cnt;     // [tiles] first occurrences, edges
   int64_t* picked;     // [columns * fanout] rows of a weighted layer
@@ -79,7 +87,9 @@ static LayerWs carve_layer(void* ws, int64_t positions, int weighted) {
   const int64_t n = positions > 0 ? positions : 1;
   w.slots = layer_table_slots(n);
   w.tiles = ceil_div(n, kLayerTile);
-  w.table = c.take<uint64_t>((size_t)w.slots);  // first, so that its place does not depend on the rest
+  // (first, so that their places do not depend on the rest)
+  w.table[0] = c.take<uint64_t>((size_t)w.slots);
+  w.table[1] = c.take<uint64_t>((size_t)w.slots);
   w.wide = c.take<int32_t>(1);
   w.slot = c.take<uint32_t>((size_t)n);
   w.first = c.take<uint32_t>((size_t)n);
@@ -136,49 +146,63 @@ __device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask,
   return 0;
 }
 
-// picked: rows drawn by another kernel, fanout places per column; null: uniform.
-template <typename IdT>
-__global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
-    const int64_t* __restrict__ indptr, int64_t num_cols, const IdT* __restrict__ indices,
-    LayerColumns cols, int fanout, int cols_per_wave, int replace, PhiloxKey key, uint32_t stride,
-    const int64_t* __restrict__ picked, uint64_t* table, uint32_t mask,
-    uint32_t* __restrict__ slot_of, int32_t* wide) {
-  __shared__ uint32_t tags[kPickSlots], mins[kPickSlots], global_slot[kPickSlots];
-  constexpr int kWaves = kPickThreads / kWave;
-  const int64_t first_col = (int64_t)blockIdx.x * (kWaves * cols_per_wave);
-  const int wave_lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int width = fanout + 1;
-  const int group = wave_lane / width;
-  const int lane = wave_lane - group * width;  // 0: the seed, j + 1: pick j
-  const int64_t c = first_col + wave * cols_per_wave + group;
-  // one round trip for the number of columns and the id, of a place that may be no column's
-  const int64_t id = cols.ids[cols.place(c, 1)];
-  const int64_t n = cols.num();
-  if (first_col >= n) return;  // uniform per work-group
-  for (int i = threadIdx.x; i < kPickSlots; i += kPickThreads) {
-    tags[i] = kNoSlot;
-    mins[i] = 0xFFFFFFFFu;
+// A column that a lane works for: its id, its batch's first column and how many that has.
+struct PickColumn {
+  int64_t id, b, s_lo, ns;
+};
+
+// What a lane of a pick knows before its column is.
+struct PickLane {
+  int64_t first_col, c;  // of the work-group; this lane's
+  int group, lane, width;
+  bool in_group;
+  __device__ __forceinline__ PickLane(unsigned block, int fanout, int cols_per_wave) {
+    const int wave_lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    first_col = (int64_t)block * (kPickThreads / kWave * cols_per_wave);
+    width = fanout + 1;
+    group = wave_lane / width;
+    lane = wave_lane - group * width;  // 0: the seed, j + 1: pick j
+    c = first_col + wave * cols_per_wave + group;
+    in_group = group < cols_per_wave;
   }
-  const bool live = group < cols_per_wave && c < n;
+};
+
+struct PickShared {
+  uint32_t tags[kPickSlots], mins[kPickSlots], global_slot[kPickSlots];
+  __device__ __forceinline__ void clear() {
+    for (int i = threadIdx.x; i < kPickSlots; i += kPickThreads) {
+      tags[i] = kNoSlot;
+      mins[i] = 0xFFFFFFFFu;
+    }
+  }
+};
+
+// The rest of a pick, behind sh.clear(): `column(&start, &deg)` gives the lane's column and where
+// it lies, and is called by live lanes only.
+// picked: rows drawn by another kernel, fanout places per column; null: uniform.
+template <typename IdT, typename Column>
+__device__ __forceinline__ void pick_columns(const PickLane& l, bool live, Column column,
+                                             const IdT* __restrict__ indices, int fanout,
+                                             int replace, PhiloxKey key, uint32_t stride,
+                                             const int64_t* __restrict__ picked, uint64_t* table,
+                                             uint32_t mask, uint32_t* __restrict__ slot_of,
+                                             int32_t* wide, PickShared& sh) {
   uint32_t my_key = kNoSlot, position = 0;
   if (live) {
-    int64_t start;
-    const int64_t deg = column_degree(indptr, num_cols, id, &start);
-    const int64_t b0 = cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(first_col)) : 0;
-    const int64_t b = cols.batch_of(c, b0);
-    const int64_t s_lo = cols.lo(b), ns = cols.hi(b) - s_lo;
-    const int64_t fb = s_lo * width;
+    int64_t start, deg;
+    const PickColumn col = column(&start, &deg);
+    const int64_t fb = col.s_lo * l.width, c = l.c;
     int64_t row = -1;
-    if (lane == 0) {
-      row = id;
-      if ((uint64_t)id >= (uint64_t)stride) {  // no id of this matrix: the caller takes another path
+    if (l.lane == 0) {
+      row = col.id;
+      if ((uint64_t)col.id >= (uint64_t)stride) {  // no id of this matrix: the caller takes another path
         *wide = 1;
         row = 0;
       }
-      position = (uint32_t)(fb + (c - s_lo));
+      position = (uint32_t)(fb + (c - col.s_lo));
     } else {
-      position = (uint32_t)(fb + ns + (c - s_lo) * fanout + (lane - 1));
-      const int64_t j = lane - 1;
+      position = (uint32_t)(fb + col.ns + (c - col.s_lo) * fanout + (l.lane - 1));
+      const int64_t j = l.lane - 1;
       if (picked) {
         const int64_t have = replace ? (deg > 0 ? fanout : 0) : (deg < fanout ? deg : fanout);
         if (j < have) row = picked[c * fanout + j];
@@ -189,11 +213,11 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
       } else if (deg <= fanout) {
         if (j < deg) row = (int64_t)indices[start + j];
       } else {
-        row = (int64_t)indices[start + floyd_slot((int)j, group * width + 1, fanout, deg, key,
+        row = (int64_t)indices[start + floyd_slot((int)j, l.group * l.width + 1, fanout, deg, key,
                                                   (uint64_t)c)];
       }
     }
-    if (row >= 0) my_key = (uint32_t)b * stride + (uint32_t)row;
+    if (row >= 0) my_key = (uint32_t)col.b * stride + (uint32_t)row;
   }
   // (looked at now, so that the answer is there when the work-group knows whose key it is)
   const uint64_t seen = my_key != kNoSlot ? table[hash32(my_key) & mask] : 0ull;
@@ -202,18 +226,43 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
   if (my_key != kNoSlot) {
     at = (my_key * 0x85EBCA6Bu) >> kPickShift;
     for (;;) {
-      uint32_t cur = tags[at];
-      if (cur == kNoSlot) cur = atomicCAS(&tags[at], kNoSlot, my_key);
+      uint32_t cur = sh.tags[at];
+      if (cur == kNoSlot) cur = atomicCAS(&sh.tags[at], kNoSlot, my_key);
       if (cur == kNoSlot || cur == my_key) break;
       at = (at + 1) & (kPickSlots - 1);
     }
-    if (mins[at] > position) atomicMin(&mins[at], position);
+    if (sh.mins[at] > position) atomicMin(&sh.mins[at], position);
   }
   __syncthreads();
-  if (my_key != kNoSlot && mins[at] == position)
-    global_slot[at] = layer_insert(table, mask, my_key, position, seen);
+  if (my_key != kNoSlot && sh.mins[at] == position)
+    sh.global_slot[at] = layer_insert(table, mask, my_key, position, seen);
   __syncthreads();
-  if (live) slot_of[position] = my_key != kNoSlot ? global_slot[at] : kNoSlot;
+  if (live) slot_of[position] = my_key != kNoSlot ? sh.global_slot[at] : kNoSlot;
+}
+
+template <typename IdT>
+__global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_cols, const IdT* __restrict__ indices,
+    LayerColumns cols, int fanout, int cols_per_wave, int replace, PhiloxKey key, uint32_t stride,
+    const int64_t* __restrict__ picked, uint64_t* table, uint32_t mask,
+    uint32_t* __restrict__ slot_of, int32_t* wide) {
+  __shared__ PickShared sh;
+  const PickLane l(blockIdx.x, fanout, cols_per_wave);
+  // one round trip for the number of columns and the id, of a place that may be no column's
+  const int64_t id = cols.ids[cols.place(l.c, 1)];
+  const int64_t n = cols.num();
+  if (l.first_col >= n) return;  // uniform per work-group
+  sh.clear();
+  pick_columns(
+      l, l.in_group && l.c < n,
+      [&](int64_t* start, int64_t* deg) {
+        *deg = column_degree(indptr, num_cols, id, start);
+        const int64_t b0 =
+            cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(l.first_col)) : 0;
+        const int64_t b = cols.batch_of(l.c, b0);
+        return PickColumn{id, b, cols.lo(b), cols.hi(b) - cols.lo(b)};
+      },
+      indices, fanout, replace, key, stride, picked, table, mask, slot_of, wide, sh);
 }
 
 // What the work-groups of a tile know about the batches in it.
@@ -241,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
   const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
   const int wave = threadIdx.x / kWave, lane = lane_id();
   const int64_t wave_p0 = p0 + (int64_t)wave * kLayerWordsPerWave * kWave;
-  uint32_t s[kLayerWordsPerWave];
+  uint32_t s[kLayerWordsPerWave], rank[kLayerWordsPerWave];
   uint64_t e[kLayerWordsPerWave];
 #pragma unroll
   for (int j = 0; j < kLayerWordsPerWave; ++j)
@@ -265,13 +314,13 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
       const uint32_t f = (uint32_t)e[j];
       first[p] = f;
       is_first = f == (uint32_t)p;
-      if (is_first) keys[p] = (uint32_t)(e[j] >> 32);
       const int64_t b = batches.of(cols, width, p);
       const int64_t s_lo = cols.lo(b);
       is_edge = p - s_lo * width >= cols.hi(b) - s_lo;
     }
     const uint64_t fw = __ballot(is_first), ew = __ballot(is_edge);
     if (lane == j) mine = LayerWord{fw, ew, firsts, edges, 0ull};
+    rank[j] = is_first ? firsts + (uint32_t)__popcll(fw & ((1ull << lane) - 1ull)) : kNoSlot;
     firsts += (uint32_t)__popcll(fw);
     edges += (uint32_t)__popcll(ew);
   }
@@ -290,6 +339,9 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
     fa += wave_first[w];
     ea += wave_edge[w];
   }
+#pragma unroll
+  for (int j = 0; j < kLayerWordsPerWave; ++j)
+    if (rank[j] != kNoSlot) keys[p0 + fb + rank[j]] = (uint32_t)(e[j] >> 32);
   if (lane < kLayerWordsPerWave) {
     mine.first_before += fb;
     mine.edge_before += eb;
@@ -304,49 +356,74 @@ struct LayerOut {
   int64_t* mirror;
 };
 
-__global__ __launch_bounds__(kBlock) void layer_label_kernel(
-    LayerColumns cols, int fanout, uint32_t stride, const uint32_t* __restrict__ first,
-    const uint32_t* __restrict__ keys, const LayerWord* __restrict__ words,
-    const uint2* __restrict__ tile_cnt, uint64_t* __restrict__ table, int64_t table_slots,
-    const int32_t* __restrict__ wide, LayerOut out) {
-  __shared__ uint2 before[kLayerMaxTiles];  // first occurrences and edges before a tile
-  __shared__ uint64_t smem[kBlock / kWave + 1];
+// What a layer's flag pass left, and what its label pass empties.
+struct LayerLabels {
+  LayerColumns cols;
+  int fanout;
+  uint32_t stride;
+  const uint32_t *first, *keys;
+  const LayerWord* words;
+  const uint2* tile_cnt;
+  uint64_t* table;
+  int64_t table_slots;
+  const int32_t* wide;
+  LayerOut out;
+};
+struct LabelShared {
+  uint2 before[kLayerMaxTiles];  // first occurrences and edges before a tile
+  uint64_t smem[kPickThreads / kWave + 1];
+};
+
+// Work-group `block` of `blocks`.  kThreads: of the launch (alone 11.6 us with 256 and 12.8
+// with 512 on 150 K positions).
+template <int kThreads>
+__device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned block,
+                                           unsigned blocks, LabelShared& sh) {
+  const LayerColumns& cols = layer.cols;
+  const int fanout = layer.fanout;
+  const uint32_t stride = layer.stride;
+  const uint32_t *__restrict__ first = layer.first, *__restrict__ keys = layer.keys;
+  const LayerWord* __restrict__ words = layer.words;
+  const uint2* __restrict__ tile_cnt = layer.tile_cnt;
+  uint64_t* __restrict__ table = layer.table;
+  const LayerOut& out = layer.out;
+  uint2* before = sh.before;
   // The table is done with: its share emptied by every work-group of the launch, last of
   // all (loads behind stores are waited for with them).
   auto empty_table = [&] {
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < table_slots;
-         i += (int64_t)gridDim.x * kBlock)
+    for (int64_t i = (int64_t)block * kThreads + threadIdx.x; i < layer.table_slots;
+         i += (int64_t)blocks * kThreads)
       table[i] = kEmptySlot;
   };
   const int width = fanout + 1;
-  // What a position needs does not wait for the counts: its word, its key, and the word of
+  // What a position needs does not wait for the counts: its word, a key, and the word of
   // its key's first position travel while the tiles are added up, and so do the words of
   // the tile's first batch.
-  constexpr int kItems = kLayerTile / kBlock;
-  const int64_t p0 = (int64_t)blockIdx.x * kLayerTile;
+  constexpr int kItems = kLayerTile / kThreads;
+  const int64_t p0 = (int64_t)block * kLayerTile;
   LayerWord word[kItems];
   uint32_t key[kItems], first_of[kItems];
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
-    const int64_t q = cols.place(p0 + i * kBlock + threadIdx.x, width);
+    const int64_t q = cols.place(p0 + i * kThreads + threadIdx.x, width);
     word[i] = words[q / kWave];
     key[i] = keys[q];
     first_of[i] = first[q];
   }
-  constexpr int kPer = kLayerMaxTiles / kBlock;
+  constexpr int kPer = kLayerMaxTiles / kThreads;
   uint2 cnt[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j)
-    cnt[j] = tile_cnt[(int64_t)threadIdx.x * kPer + j < gridDim.x ? threadIdx.x * kPer + j : 0];
+    cnt[j] = tile_cnt[(int64_t)threadIdx.x * kPer + j < blocks ? threadIdx.x * kPer + j : 0];
   const int64_t n = cols.num(), N = n * width;
   const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
-  if (blockIdx.x != 0 && (int64_t)blockIdx.x >= tiles) return empty_table();
+  if (block != 0 && (int64_t)block >= tiles) return empty_table();
   const TileBatches batches =
       tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
   LayerWord first_word[kItems];
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
-    const int64_t p = p0 + i * kBlock + threadIdx.x;
+    const int64_t p = p0 + i * kThreads + threadIdx.x;
     // (no key was sent to this position: nothing was written there)
     const bool edge = p < N && ((word[i].edge >> (int)(p % kWave)) & 1ull);
     if (!edge) first_of[i] = 0;
@@ -363,7 +440,7 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
     sum += ((uint64_t)cnt[j].y << 32) | cnt[j].x;
   }
   uint64_t total;
-  uint64_t run = block_exclusive_sum<uint64_t>(sum, smem, &total);
+  uint64_t run = block_exclusive_sum<uint64_t, kThreads>(sum, sh.smem, &total);
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     before[threadIdx.x * kPer + j] = make_uint2((uint32_t)run, (uint32_t)(run >> 32));
@@ -397,8 +474,8 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
     return ((w.first >> (int)(q % kWave)) & 1ull) &&
            rank_in(w, (uint32_t)q) - f0 == (uint32_t)(ns - 1);
   };
-  if (blockIdx.x == 0) {
-    for (int64_t b = threadIdx.x; b <= cols.B; b += kBlock) {
+  if (block == 0) {
+    for (int64_t b = threadIdx.x; b <= cols.B; b += kThreads) {
       const int64_t s_lo = b < cols.B ? cols.lo(b) : n;
       uint32_t f, e;
       ranks(s_lo * width, &f, &e);
@@ -419,7 +496,7 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
                            ? 1
                            : 0);
       } else {
-        store_for_host(out.mirror + 3 * cols.B + 2, *wide);
+        store_for_host(out.mirror + 3 * cols.B + 2, *layer.wide);
       }
     }
   }
@@ -427,9 +504,17 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
   uint32_t f0, e0;
   ranks_in(word_b, fb, &f0, &e0);
   bool distinct = seeds_distinct(word_q, fb, ns, f0);
+  const uint2 t = before[block];
+  // the frontier's share of the tile: its new keys, in order
+  const uint32_t tile_firsts = ((int64_t)block + 1 < tiles ? before[block + 1].x : all_first) - t.x;
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
-    const int64_t p = p0 + i * kBlock + threadIdx.x;
+    const uint32_t r = i * kThreads + threadIdx.x;
+    if (r < tile_firsts) out.frontier[t.x + r] = (int64_t)(key[i] % stride);
+  }
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    const int64_t p = p0 + i * kThreads + threadIdx.x;
     if (p >= N) break;
     const int64_t b_now = batches.of(cols, width, p);
     if (b_now != b) {
@@ -443,10 +528,6 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
     const LayerWord& w = word[i];
     const int bit = (int)(p % kWave);
     const uint64_t below = (1ull << bit) - 1ull;
-    const uint2 t = before[blockIdx.x];
-    if ((w.first >> bit) & 1ull)
-      out.frontier[t.x + w.first_before + (uint32_t)__popcll(w.first & below)] =
-          (int64_t)(key[i] - (uint32_t)b * stride);
     const uint32_t local = (uint32_t)(p - fb);
     if (local < (uint32_t)ns) continue;
     const uint32_t slot = local - (uint32_t)ns;
@@ -462,11 +543,89 @@ __global__ __launch_bounds__(kBlock) void layer_label_kernel(
   empty_table();
 }
 
-__global__ __launch_bounds__(kBlock) void layer_clear_kernel(uint64_t* table, int64_t slots,
-                                                             int32_t* wide) {
+__global__ __launch_bounds__(kBlock) void layer_label_kernel(LayerLabels layer) {
+  __shared__ LabelShared sh;
+  label_tile<kBlock>(layer, blockIdx.x, gridDim.x, sh);
+}
+
+// Labels of a layer and picks of the one whose columns are its frontier: the first
+// `pick_blocks` work-groups pick.
+template <typename IdT>
+__global__ __launch_bounds__(kPickThreads) void layer_label_pick_kernel(
+    LayerLabels before, unsigned pick_blocks, const int64_t* __restrict__ indptr, int64_t num_cols,
+    const IdT* __restrict__ indices, int fanout, int cols_per_wave, int replace, PhiloxKey key,
+    uint64_t* table, uint32_t mask, uint32_t* __restrict__ slot_of, int32_t* wide) {
+  if (blockIdx.x >= pick_blocks) {
+    __shared__ LabelShared label;
+    label_tile<kPickThreads>(before, blockIdx.x - pick_blocks, gridDim.x - pick_blocks, label);
+    return;
+  }
+  __shared__ PickShared sh;
+  __shared__ uint32_t tile_first[kLayerMaxTiles + 1];  // columns before a tile's
+  __shared__ uint32_t batch_first[kLayerMaxBatches + 1];
+  __shared__ uint32_t smem[kPickThreads / kWave + 1];
+  const int t = threadIdx.x;
+  const PickLane l(blockIdx.x, fanout, cols_per_wave);
+  const LayerColumns& prev = before.cols;
+  const int prev_width = before.fanout + 1;
+  constexpr int kPer = kLayerMaxTiles / kPickThreads;
+  const int64_t most_tiles = (prev.count * prev_width + kLayerTile - 1) / kLayerTile;
+  uint32_t cnt[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    cnt[j] = before.tile_cnt[t * kPer + j < most_tiles ? t * kPer + j : 0].x;
+  const int64_t prev_n = prev.num(), N = prev_n * prev_width;
+  const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
+  // where a batch's keys begin, and the word of that position
+  const int64_t p = t < prev.B ? prev.lo(t) * prev_width : N;
+  const LayerWord word = before.words[p < N ? p / kWave : 0];
+  sh.clear();
+  uint32_t sum = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    if (t * kPer + j >= tiles) cnt[j] = 0;
+    sum += cnt[j];
+  }
+  uint32_t n;
+  uint32_t run = block_exclusive_sum<uint32_t, kPickThreads>(sum, smem, &n);
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    tile_first[t * kPer + j] = run;
+    run += cnt[j];
+  }
+  if (t == 0) tile_first[kLayerMaxTiles] = n;
+  if (l.first_col >= (int64_t)n) return;  // uniform per work-group
+  __syncthreads();
+  if (t <= prev.B)
+    batch_first[t] = p >= N ? n
+                            : tile_first[p / kLayerTile] + word.first_before +
+                                  (uint32_t)__popcll(word.first & ((1ull << (int)(p % kWave)) - 1ull));
+  __syncthreads();
+  pick_columns(
+      l, l.in_group && l.c < (int64_t)n,
+      [&](int64_t* start, int64_t* deg) {
+        const uint32_t c = (uint32_t)l.c;
+        int lo = 0, hi = (int)tiles;  // tile_first[lo] <= c < tile_first[hi], whose tiles are done
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (tile_first[mid] <= c) lo = mid;
+          else hi = mid;
+        }
+        const uint32_t found = before.keys[(int64_t)lo * kLayerTile + (c - tile_first[lo])];
+        const uint32_t b = found / before.stride;
+        const int64_t id = (int64_t)(found - b * before.stride);
+        *deg = column_degree(indptr, num_cols, id, start);
+        return PickColumn{id, b, batch_first[b], batch_first[b + 1] - batch_first[b]};
+      },
+      indices, fanout, replace, key, before.stride, (const int64_t*)nullptr, table, mask, slot_of,
+      wide, sh);
+}
+
+__global__ __launch_bounds__(kBlock) void layer_clear_kernel(uint64_t* table0, uint64_t* table1,
+                                                             int64_t slots, int32_t* wide) {
   int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i == 0) *wide = 0;
-  for (; i < slots; i += (int64_t)gridDim.x * kBlock) table[i] = kEmptySlot;
+  for (; i < slots; i += (int64_t)gridDim.x * kBlock) table0[i] = table1[i] = kEmptySlot;
 }
 
 // weighted.hip: draws of a weighted layer into fanout places per column, the number
@@ -501,8 +660,8 @@ int gs_layer_begin(int64_t max_positions, int weighted, void* workspace, size_t 
   if (blocks > 2048) blocks = 2048;
   hipStream_t s = as_stream(stream);
   GS_LAUNCH("layer_clear", s,
-            layer_clear_kernel<<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(w.table, w.slots,
-                                                                               w.wide));
+            layer_clear_kernel<<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(
+                w.table[0], w.table[1], w.slots, w.wide));
   return GS_OK;
 }
 
@@ -515,58 +674,108 @@ int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indi
                     int64_t* out_block_indptr, int64_t* mirror,
                     int64_t max_positions, void* workspace, size_t workspace_bytes,
                     gs_stream_t stream) {
+  const gs_layer layer{indptr, num_cols, indices, indices32, cdf, id_stride, columns, num_columns,
+                       col_ptr, num_batches, fanout, replace, seed, call_id, out_frontier,
+                       out_frontier_ptr, out_row, out_col, out_edge_ptr, out_block_indptr, mirror,
+                       max_positions, workspace, workspace_bytes, 0};
+  const int rc = gs_sample_layer_next(nullptr, &layer, stream);
+  return rc != GS_OK ? rc : gs_sample_layer_next(&layer, nullptr, stream);
+}
+
+static int check_layer(const gs_layer& l) {
   using namespace gs;
-  GS_REQUIRE(num_cols >= 0 && num_columns >= 1, "sample_layer: no columns");
-  GS_REQUIRE(num_batches >= 1 && (col_ptr || num_batches == 1),
-             "sample_layer: %lld batches need col_ptr", (long long)num_batches);
-  GS_REQUIRE(fanout >= 1 && fanout < kWave, "sample_layer: fanout %lld", (long long)fanout);
-  GS_REQUIRE(id_stride >= 1 && id_stride >= num_cols &&
-                 num_batches <= (int64_t)0xFFFFFFFEll / id_stride,
-             "sample_layer: %lld batches of ids below %lld", (long long)num_batches,
-             (long long)id_stride);
-  const int64_t positions = num_columns * (fanout + 1);
-  GS_REQUIRE(positions <= max_positions && max_positions <= gs_layer_max_positions(),
-             "sample_layer: %lld positions", (long long)positions);
-  GS_REQUIRE(indptr && columns && out_frontier && out_frontier_ptr && out_row && out_col &&
-                 out_edge_ptr && mirror,
+  GS_REQUIRE(l.num_cols >= 0 && l.num_columns >= 1, "sample_layer: no columns");
+  GS_REQUIRE(l.num_batches >= 1 && (l.col_ptr || l.num_batches == 1),
+             "sample_layer: %lld batches need col_ptr", (long long)l.num_batches);
+  GS_REQUIRE(l.fanout >= 1 && l.fanout < kWave, "sample_layer: fanout %lld", (long long)l.fanout);
+  GS_REQUIRE(l.id_stride >= 1 && l.id_stride >= l.num_cols &&
+                 l.num_batches <= (int64_t)0xFFFFFFFEll / l.id_stride,
+             "sample_layer: %lld batches of ids below %lld", (long long)l.num_batches,
+             (long long)l.id_stride);
+  GS_REQUIRE(l.num_columns * (l.fanout + 1) <= l.max_positions &&
+                 l.max_positions <= gs_layer_max_positions(),
+             "sample_layer: %lld positions", (long long)(l.num_columns * (l.fanout + 1)));
+  GS_REQUIRE(l.indptr && l.columns && l.out_frontier && l.out_frontier_ptr && l.out_row &&
+                 l.out_col && l.out_edge_ptr && l.mirror && (l.table == 0 || l.table == 1),
              "sample_layer: null pointer");
-  const LayerWs w = carve_layer(workspace, max_positions, cdf != nullptr);
-  if (workspace == nullptr || workspace_bytes < w.total) {
-    set_error("layer workspace too small: %zu < %zu", workspace_bytes, w.total);
+  const LayerWs w = carve_layer(l.workspace, l.max_positions, l.cdf != nullptr);
+  if (l.workspace == nullptr || l.workspace_bytes < w.total) {
+    set_error("layer workspace too small: %zu < %zu", l.workspace_bytes, w.total);
     return GS_ERR_WORKSPACE;
   }
-  const int64_t slots = layer_table_slots(positions);  // of the table, what this layer uses
+  return GS_OK;
+}
+
+int gs_sample_layer_next(const gs_layer* before, const gs_layer* layer, gs_stream_t stream) {
+  using namespace gs;
+  int rc = before ? check_layer(*before) : GS_OK;
+  if (rc == GS_OK && layer) rc = check_layer(*layer);
+  if (rc != GS_OK) return rc;
   hipStream_t s = as_stream(stream);
-  const PhiloxKey key = make_key(seed, call_id);
-  const LayerColumns cols{columns, col_ptr, num_batches, num_columns};
-  const int cols_per_wave = kWave / ((int)fanout + 1);
+  LayerLabels labels{};
+  unsigned label_grid = 0;
+  if (before) {
+    const gs_layer& l = *before;
+    const LayerWs w = carve_layer(l.workspace, l.max_positions, l.cdf != nullptr);
+    const int64_t positions = l.num_columns * (l.fanout + 1);
+    labels = LayerLabels{LayerColumns{l.columns, l.col_ptr, l.num_batches, l.num_columns},
+                         (int)l.fanout, (uint32_t)l.id_stride, w.first, w.key, w.words, w.tile_cnt,
+                         w.table[l.table], layer_table_slots(positions), w.wide,
+                         LayerOut{l.out_frontier, l.out_frontier_ptr, l.out_row, l.out_col,
+                                  l.out_edge_ptr, l.out_block_indptr, l.mirror}};
+    label_grid = (unsigned)ceil_div(positions, kLayerTile);
+  }
+  // (beside the labels of the layer before, whose frontier its columns are)
+  const bool beside = before && layer && !layer->cdf && layer->table != before->table &&
+                      layer->workspace == before->workspace &&
+                      layer->max_positions == before->max_positions && !before->cdf &&
+                      layer->columns == before->out_frontier &&
+                      layer->col_ptr == before->out_frontier_ptr &&
+                      layer->num_batches == before->num_batches &&
+                      layer->id_stride == before->id_stride &&
+                      layer->num_batches <= kLayerMaxBatches;
+  if (before && !beside)
+    GS_LAUNCH("layer_label", s,
+              layer_label_kernel<<<dim3(label_grid), dim3(kBlock), 0, s>>>(labels));
+  if (!layer) return GS_OK;
+  const gs_layer& l = *layer;
+  const LayerWs w = carve_layer(l.workspace, l.max_positions, l.cdf != nullptr);
+  const int64_t positions = l.num_columns * (l.fanout + 1);
+  const int64_t slots = layer_table_slots(positions);  // of the table, what this layer uses
+  const PhiloxKey key = make_key(l.seed, l.call_id);
+  const LayerColumns cols{l.columns, l.col_ptr, l.num_batches, l.num_columns};
+  const int cols_per_wave = kWave / ((int)l.fanout + 1);
   const unsigned pick_grid =
-      (unsigned)ceil_div(num_columns, (kPickThreads / kWave) * cols_per_wave);
-  const unsigned tile_grid = (unsigned)ceil_div(positions, kLayerTile);
-  if (cdf) {
-    int rc = launch_weighted_places(indptr, num_cols, indices, cdf, columns,
-                                    col_ptr ? col_ptr + num_batches : nullptr, num_columns, fanout,
-                                    replace, key, w.picked, s);
+      (unsigned)ceil_div(l.num_columns, (kPickThreads / kWave) * cols_per_wave);
+  uint64_t* table = w.table[l.table];
+  if (l.cdf) {
+    rc = launch_weighted_places(l.indptr, l.num_cols, l.indices, l.cdf, l.columns,
+                                l.col_ptr ? l.col_ptr + l.num_batches : nullptr, l.num_columns,
+                                l.fanout, l.replace, key, w.picked, s);
     if (rc != GS_OK) return rc;
   }
 #define GS_PICK(T, IDS)                                                                       \
-  GS_LAUNCH("layer_pick", s,                                                                  \
-            layer_pick_kernel<T><<<dim3(pick_grid), dim3(kPickThreads), 0, s>>>(              \
-                indptr, num_cols, IDS, cols, (int)fanout, cols_per_wave, replace, key,        \
-                (uint32_t)id_stride, cdf ? w.picked : nullptr, w.table, (uint32_t)(slots - 1), \
-                w.slot, w.wide))
-  if (indices32) GS_PICK(int32_t, indices32);
-  else GS_PICK(int64_t, indices);
+  do {                                                                                        \
+    if (beside)                                                                               \
+      GS_LAUNCH("layer_label_pick", s,                                                        \
+                layer_label_pick_kernel<T><<<dim3(pick_grid + label_grid), dim3(kPickThreads), 0, \
+                                             s>>>(                                            \
+                    labels, pick_grid, l.indptr, l.num_cols, IDS, (int)l.fanout, cols_per_wave, \
+                    l.replace, key, table, (uint32_t)(slots - 1), w.slot, w.wide));           \
+    else                                                                                      \
+      GS_LAUNCH("layer_pick", s,                                                              \
+                layer_pick_kernel<T><<<dim3(pick_grid), dim3(kPickThreads), 0, s>>>(          \
+                    l.indptr, l.num_cols, IDS, cols, (int)l.fanout, cols_per_wave, l.replace, \
+                    key, (uint32_t)l.id_stride, l.cdf ? w.picked : nullptr, table,            \
+                    (uint32_t)(slots - 1), w.slot, w.wide));                                  \
+  } while (0)
+  if (l.indices32) GS_PICK(int32_t, l.indices32);
+  else GS_PICK(int64_t, l.indices);
 #undef GS_PICK
   GS_LAUNCH("layer_flag", s,
-            layer_flag_kernel<<<dim3(tile_grid), dim3(kBlock), 0, s>>>(
-                cols, (int)fanout, w.table, w.slot, w.first, w.key, w.words, w.tile_cnt));
-  const LayerOut out{out_frontier, out_frontier_ptr, out_row, out_col,
-                     out_edge_ptr, out_block_indptr, mirror};
-  GS_LAUNCH("layer_label", s,
-            layer_label_kernel<<<dim3(tile_grid), dim3(kBlock), 0, s>>>(
-                cols, (int)fanout, (uint32_t)id_stride, w.first, w.key, w.words, w.tile_cnt,
-                w.table, slots, w.wide, out));
+            layer_flag_kernel<<<dim3((unsigned)ceil_div(positions, kLayerTile)), dim3(kBlock), 0,
+                                s>>>(cols, (int)l.fanout, table, w.slot, w.first, w.key, w.words,
+                                     w.tile_cnt));
   return GS_OK;
 }
 

@@ -470,6 +470,33 @@ int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indi
                     int64_t* out_row, int64_t* out_col, int64_t* out_edge_ptr,
                     int64_t* out_block_indptr, int64_t* mirror, int64_t max_positions,
                     void* workspace, size_t workspace_bytes, gs_stream_t stream);
+/* The same for a chain of layers: labels of `before`, picks of `layer` (either may be NULL).
+ * Every layer is given twice, first as `layer`, then as `before`, on one stream; where the
+ * columns of `layer` are the frontier of `before` (its outputs as columns and col_ptr, the
+ * same workspace and table != before->table) and neither is weighted the two run beside
+ * each other.  `table`: 0 or 1, which of the workspace's two tables the layer hashes into;
+ * one that an unfinished layer has is not to be used. */
+typedef struct gs_layer {
+  const int64_t* indptr;
+  int64_t num_cols;
+  const int64_t* indices;
+  const int32_t* indices32;
+  const int64_t* cdf;
+  int64_t id_stride;
+  const int64_t* columns;
+  int64_t num_columns;
+  const int64_t* col_ptr;
+  int64_t num_batches, fanout;
+  int replace;
+  uint64_t seed, call_id;
+  int64_t *out_frontier, *out_frontier_ptr, *out_row, *out_col, *out_edge_ptr, *out_block_indptr;
+  int64_t* mirror;
+  int64_t max_positions;
+  void* workspace;
+  size_t workspace_bytes;
+  int table;
+} gs_layer;
+int gs_sample_layer_next(const gs_layer* before, const gs_layer* layer, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * What a layer-wise sampler asks such a slice for, without writing it: the sums of

@@ -111,6 +111,33 @@ def test_super_batch(rng, cuts, fanouts, replace, weighted):
             same(x, y)
 
 
+@pytest.mark.parametrize("batches", [1, 511, 512])
+@pytest.mark.parametrize("replace", [False, True])
+def test_chains_of_short_layers_around_the_most_batches(rng, batches, replace):
+    """Picks beside the labels of the layer before, for as many batches as they find the
+    offsets of, and one more (a launch each): three layers, batches that are empty, that
+    repeat one seed, whose seeds have no neighbours, and tiles without a new key."""
+    nodes = 4000
+    indptr, indices = random_csc(rng, nodes, nodes, 9, hub_deg=0)
+    degree = np.diff(indptr)
+    m = gs.Matrix(gs.Graph(nodes, nodes))
+    m._graph._CAPI_LoadCSC(torch.from_numpy(indptr).to(DEV), torch.from_numpy(indices).to(DEV))
+    bm = gs.BatchMatrix()
+    bm.load_from_matrix(m, False)
+    sizes = rng.integers(0, 6, size=batches)
+    sizes[-1] = 2100                                   # two tiles of one repeated seed
+    cuts = np.concatenate([[0], np.cumsum(sizes)])
+    seeds = rng.integers(0, nodes, size=cuts[-1])
+    seeds[cuts[-2]:] = seeds[-1]
+    if (degree == 0).any():
+        seeds[:3] = np.nonzero(degree == 0)[0][0]
+    args = (torch.from_numpy(seeds).to(DEV), torch.from_numpy(cuts).to(DEV), [5, 3, 4], replace)
+    got, want = both(batched, bm, args, 3)
+    for layer, other in zip(got, want):
+        for name in ("frontier", "frontier_ptr", "row", "col", "edge_ptr", "indptr", "col_ptr"):
+            assert torch.equal(getattr(layer.batch, name)(), getattr(other.batch, name)()), name
+
+
 @pytest.mark.parametrize("cuts,fanouts,replace,weighted", [
     ([0, 8], [3, 2], False, False),
     ([0, 0, 30, 30, 64], [10, 5], False, False),         # batches without seeds
