@@ -117,6 +117,8 @@ SIGNATURES = {
     "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
                                             _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),
+    "gs_col_row_slice_labels": (_int, [_p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p, _p,
+                                       _p, _sz, _p]),
     "gs_col_row_slice_fill": (_int, [_p, _p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "gs_probe_stream_copy": (_int, [_p, _p, _i64, _p]),
     "gs_probe_line_gather": (_int, [_p, _i64, _i64, _u64, _int, _p, _p]),

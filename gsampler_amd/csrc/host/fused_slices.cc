@@ -200,6 +200,72 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   return {g, edge_index(m.e_ids, r.select)};
 }
 
+// Plain float32 values on the GPU, one a place, which nothing else has to see.
+static bool plain_row_of_values(const torch::Tensor& t) {
+  return plain_values(t, false) && t.dim() == 1 && t.is_contiguous() && t.size(0) > 0;
+}
+
+// Worth it when the slice's edges outnumber its rows and columns by far, as
+// `use_list_labels` says of those that are kept; here the number of these is not waited for.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, c10::optional<torch::Tensor>>>
+Graph::RelabelledRows(torch::Tensor cols, torch::Tensor rows, c10::optional<torch::Tensor> values,
+                      c10::optional<torch::Tensor> row_divisor) {
+  const Compressed& m = compressed(kCSC);
+  const int64_t R = rows.numel(), S = cols.numel();
+  if (m.e_ids.has_value() || !m.indices.is_cuda() || !m.indptr.is_cuda() || R == 0 || S == 0 ||
+      R + S > GS_LIST_LABELS_MAX_KEYS)
+    return {};
+  if (values.has_value() &&
+      (!plain_row_of_values(*values) || at::impl::torch_function_mode_enabled() ||
+       at::autocast::is_autocast_enabled(at::kCUDA)))
+    return {};
+  if (row_divisor.has_value() &&
+      (!values.has_value() || !plain_row_of_values(*row_divisor) || row_divisor->size(0) < R))
+    return {};
+  cols = ids(cols, "cols");
+  rows = ids(rows, "rows");
+  const std::shared_ptr<SliceOffsets> so = slice_offsets_for(cols);
+  const int64_t nnz = so->nnz;
+  if (nnz < 8 * (R + S) || nnz > kBoundLimit || !gs_col_row_slice_tells_first(nnz, R)) return {};
+  const torch::Tensor narrow = narrow_for_slice(m, nnz, S);
+  torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, R), m.indptr);
+  torch::Tensor indptr = new_ids(S + 1, m.indptr);
+  // first edges, labels of the rows, labels of the columns, sums of the columns
+  torch::Tensor small = new_ids(2 * R + 2 * S, m.indptr);
+  int64_t* const first = mptr(small);
+  int64_t* const row_label = first + R;
+  int64_t* const col_label = row_label + R;
+  double* const sums = (double*)(col_label + S);
+  AsyncCount kept = AsyncCount::mirrored();
+  GS_CALL(gs_col_row_slice_count_first(
+      cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+      cptr(cols), nullptr, S, cptr(so->sub_indptr), nnz, cptr(rows), R, mptr(indptr),
+      kept.mirror(), first, sums, ws.data_ptr(), ws.numel(), cur_stream()));
+  kept.arm();
+  torch::Tensor frontier = new_ids(R + S, m.indptr);
+  AsyncCount nodes = AsyncCount::mirrored();
+  GS_CALL(gs_list_labels(cptr(cols), S, cptr(rows), first, R, mptr(frontier), nullptr,
+                         nodes.mirror(), row_label, col_label, cur_stream()));
+  nodes.arm();
+  torch::Tensor row = new_ids(nnz, m.indptr), col = new_ids(nnz, m.indptr), out;
+  if (values.has_value()) out = torch::empty({nnz}, values->options().requires_grad(false));
+  GS_CALL(gs_col_row_slice_labels(
+      cptr(m.indptr), cptr(cols), S, cptr(so->sub_indptr), nnz, R, row_label, col_label,
+      mptr(row), mptr(col), out.defined() ? values->data_ptr<float>() : nullptr,
+      out.defined() ? values->size(0) : 0,
+      row_divisor.has_value() ? row_divisor->data_ptr<float>() : nullptr,
+      out.defined() ? out.data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), cur_stream()));
+  const int64_t k = kept.get();
+  if (out.defined() && k > 0)
+    GS_CALL(gs_normalise_columns_cleared(cptr(indptr), S, nullptr, k, out.data_ptr<float>(), k,
+                                         nullptr, nullptr, sums, out.data_ptr<float>(), cur_stream()));
+  const int64_t n = nodes.get();
+  if (k == 0 && out.defined()) return {};  // (the operators say what the values of no edges are)
+  c10::optional<torch::Tensor> normalised;
+  if (out.defined()) normalised = trim_to(out, k);
+  return std::make_tuple(trim_to(frontier, n), trim_to(row, k), trim_to(col, k), normalised);
+}
+
 void Graph::keep_row_firsts(const torch::Tensor& firsts, const torch::Tensor& edge_rows) {
   if (!firsts.defined()) return;
   row_firsts_ = firsts;

@@ -278,6 +278,13 @@ class Graph : public torch::CustomClassHolder {
   c10::optional<torch::Tensor> NormaliseColumns(torch::Tensor values,
                                                 c10::optional<torch::Tensor> select,
                                                 c10::optional<torch::Tensor> row_divisor);
+  // For a compiled sampler: the row slice A[rows, cols] as GraphRelabel(cols, rows) of it
+  // and, with `values` of this matrix's edges, NormaliseColumns leave it, (frontier, row,
+  // column, values), the slice itself not written; nothing where the call is not one for it.
+  c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor,
+                           c10::optional<torch::Tensor>>>
+  RelabelledRows(torch::Tensor cols, torch::Tensor rows, c10::optional<torch::Tensor> values,
+                 c10::optional<torch::Tensor> row_divisor);
   void FusedUOPV(const std::string& op, torch::Tensor lhs1, torch::Tensor rhs1,
                  torch::Tensor out1, torch::Tensor lhs2, torch::Tensor rhs2,
                  torch::Tensor out2, int64_t on_format);

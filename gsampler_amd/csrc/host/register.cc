@@ -119,6 +119,7 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_BatchBlocks", &Graph::BatchBlocks)
       .def("_CAPI_SampleLayers", &Graph::SampleLayers)
       .def("_CAPI_BatchSampleLayers", &Graph::BatchSampleLayers)
+      .def("_CAPI_RelabelledRows", &Graph::RelabelledRows)
       .def("_CAPI_NormaliseColumns", &Graph::NormaliseColumns)
       .def("_CAPI_EncodedSquareSums", &Graph::EncodedSquareSums)
       .def("_CAPI_EncodedPickedRows", &Graph::EncodedPickedRows)

@@ -178,6 +178,7 @@ class compile:  # noqa: N801 -- the reference's public name
         passes.share_leading_rows(graph)
         passes.weights_of_picks(graph)
         passes.sum_slices_into_new_arrays(graph)
+        passes.relabel_row_slices(graph)
         return fx.GraphModule(gm, graph).forward
 
     def __call__(self, *args):

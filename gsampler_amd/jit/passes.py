@@ -1079,6 +1079,53 @@ def sum_slices_into_new_arrays(copy: fx.Graph) -> None:
         _drop_dead_nodes(copy, replaced)
 
 
+def relabel_row_slices(copy: fx.Graph) -> None:
+    """In a copy of a graph: a row slice A[rows, cols] that is relabelled by cols and rows,
+    whose edges' normalised values may be wanted, and nothing else  => one _relabelled_rows."""
+    from ..ops.fused_op import _normalised, _relabelled_rows
+    order = {n: i for i, n in enumerate(copy.nodes)}
+    replaced = []
+    for cut in list(copy.nodes):
+        if not _is_method(cut, "_CAPI_ColRowSlicing") or len(cut.args) != 5 or cut.kwargs:
+            continue
+        g, cols, rows, *formats = cut.args
+        if any(not _call(u, operator.getitem) or u.args[1] not in (0, 1) for u in cut.users):
+            continue
+        readers = {u for m in _getitem_users(cut, 0) for u in m.users}
+        labels = [u for u in readers if _is_method(u, "_CAPI_GraphRelabel")]
+        values = [u for u in readers if _call(u, _normalised)]
+        if len(labels) != 1 or len(values) > 1 or len(readers) != len(labels) + len(values):
+            continue
+        label = labels[0]
+        if label.args[1] is not cols or label.args[2] is not rows or label.kwargs:
+            continue
+        inputs, wanted = [], {u for i in _getitem_users(cut, 1) for u in i.users}
+        if values:
+            m, e, select, divisor, value_formats = values[0].args
+            if not (_call(select, operator.getitem) and select.args[0] is cut and select.args[1] == 1):
+                continue
+            inputs = [e, divisor, value_formats]
+        if wanted != set(values):
+            continue
+        first = min([label, *values], key=order.get)
+        # (an operand that is there before the slice is read; the divisor may be made from it later)
+        if any(isinstance(a, fx.Node) and order.get(a, -1) >= order[first] for a in inputs):
+            continue
+        if _written_between(order, [cut, label, *values]):
+            continue
+        with copy.inserting_before(first):
+            new = copy.call_function(_relabelled_rows, args=(g, cols, rows, tuple(formats), *inputs))
+            parts = [copy.call_function(operator.getitem, args=(new, i)) for i in range(2)]
+        label.replace_all_uses_with(parts[0])
+        replaced.append(label)
+        for v in values:
+            v.replace_all_uses_with(parts[1])
+            replaced.append(v)
+        replaced.append(cut)
+    if replaced:
+        _drop_dead_nodes(copy, replaced)
+
+
 def share_leading_rows(copy: fx.Graph) -> None:
     """In a copy of a graph: the rows of a column slice are its parent's, so what is
     computed from data of all of them in one layer is what the next one computes.  Merges

@@ -89,6 +89,19 @@ def _normalised(g, values, select, divisor, formats):
     return divided(e, _after_spmm(sums, squeeze), 2, formats[2])
 
 
+def _relabelled_rows(g, cols, rows, formats, values=None, divisor=None, value_formats=None):
+    """What a compiled sampler hands on of the row slice g[rows, cols]: its relabelled edges
+    (_CAPI_GraphRelabel) and, if `values` of g's edges are given, these as _normalised leaves
+    them on the slice, which is not written where that can be."""
+    if all(t is None or type(t) is torch.Tensor for t in (values, divisor)):
+        out = g._CAPI_RelabelledRows(cols, rows, values, divisor)
+        if out is not None:
+            return out[:3] + (None,), out[3]
+    sub, index = g._CAPI_ColRowSlicing(cols, rows, *formats)
+    e = None if values is None else _normalised(sub, values, index, divisor, value_formats)
+    return sub._CAPI_GraphRelabel(cols, rows), e
+
+
 def _sliced_square_sums(g, cols, values):
     """Sums of the squared values over the edges of the column slice g[:, cols] onto its rows."""
     if type(values) is torch.Tensor and not values.requires_grad:

@@ -749,6 +749,17 @@ int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const i
                           int64_t slice_nnz, int64_t num_rows_picked, int64_t* out_major,
                           int64_t* out_minor, int64_t* out_select, void* workspace,
                           size_t workspace_bytes, gs_stream_t stream);
+/* In place of the fill, for a slice whose edges are only handed on: out_row[kept] =
+ * row_label[position in `rows`], out_col[kept] = col_label[position in `cols`] (labels are
+ * below 2^32), and with
+ * values of the parent's edges (num_values of them, 0 for edges past them) out_values[kept]
+ * = values[position in the parent] (/ row_divisor[position in `rows`]). */
+int gs_col_row_slice_labels(const int64_t* indptr, const int64_t* cols, int64_t num_cols_picked,
+                            const int64_t* sub_indptr, int64_t slice_nnz, int64_t num_rows_picked,
+                            const int64_t* row_label, const int64_t* col_label, int64_t* out_row,
+                            int64_t* out_col, const float* values, int64_t num_values,
+                            const float* row_divisor, float* out_values, void* workspace,
+                            size_t workspace_bytes, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Format conversion.

@@ -500,3 +500,112 @@ def test_normalised_columns_of_one_slice_several_times():
     col = torch.repeat_interleave(torch.arange(200, device=DEV), torch.diff(sub._CAPI_GetCSCIndptr()))
     sums = torch.zeros(200, dtype=torch.float64, device=DEV).index_add_(0, col, w[index].double())
     assert torch.allclose(got[0].double(), w[index].double() / sums[col], rtol=1e-6)
+
+
+def columns_of(lengths, rng, num_rows):
+    indptr = np.concatenate([[0], np.cumsum(lengths)])
+    return indptr, rng.integers(0, num_rows, size=int(indptr[-1])).astype(np.int64)
+
+
+@pytest.mark.parametrize("values", ["divided", "plain", None])
+@pytest.mark.parametrize("shape", ["one long", "two", "some", "many", "past a run", "huge"])
+def test_row_slice_that_is_only_handed_on(shape, values):
+    """Labels, frontier and normalised values of a row slice that is not written are those of
+    one that is: runs of edges in one column, in two, in up to 64 and in more, columns and
+    rows that repeat.  Values, divisors and so the sums are exact: equal bit for bit."""
+    rng = np.random.default_rng(len(shape))
+    lengths = {"one long": [5000], "two": [0, 300, 0, 4100, 7], "some": rng.integers(0, 60, 400),
+               "many": rng.integers(0, 9, 1700), "past a run": [3] * 5 + [0] * 90 + [2] * 400 + [20_000, 255, 257],
+               "huge": rng.integers(0, 9000, 500)}[shape]
+    indptr, indices = columns_of(lengths, rng, 3000)
+    n, R = len(lengths), 200 if shape == "many" else 300
+    if shape == "some":
+        R = 100
+    cols, rows = rng.permutation(n), rng.integers(0, 3100, size=R)
+    if n > 20:
+        cols[3], rows[7] = cols[9], rows[8]
+    g = gs.Graph(3100, n)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+    by = torch.as_tensor((2.0 ** rng.integers(-2, 3, size=R + 5)).astype(np.float32), device=DEV)
+    cols, rows = T(cols), T(rows)
+    e = w if values else None
+    divisor = by if values == "divided" else None
+    got = g._CAPI_RelabelledRows(cols, rows, e, divisor)
+    sub, index = g._CAPI_ColRowSlicing(cols, rows, gs.format._CSC, gs.format._CSC | gs.format._COO)
+    want = sub._CAPI_GraphRelabel(cols, rows)
+    assert (got is None) == (shape == "many")  # more keys than one work-group takes
+    if got is None:
+        return
+    for a, b in zip(got[:3], want):
+        assert torch.equal(a, b)
+    if values:
+        assert torch.equal(got[3], sub._CAPI_NormaliseColumns(w, index, divisor))
+    else:
+        assert got[3] is None
+
+
+def test_row_slices_that_have_to_be_written():
+    """No edge is kept, edge data of other types, too few edges for the pass, a parent with
+    edge ids of its own; and edge data shorter than the edges."""
+    rng = np.random.default_rng(8)
+    indptr, indices = columns_of([2000, 3000], rng, 500)
+    g = gs.Graph(900, 2)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    cols, rows, w = T([1, 0]), T(rng.permutation(500)[:90]), torch.rand(5000, device=DEV)
+    absent = T([600, 700])
+    assert g._CAPI_RelabelledRows(cols, absent, w, None) is None
+    frontier, row, col, _ = g._CAPI_RelabelledRows(cols, absent, None, None)
+    assert torch.equal(frontier, cols) and row.numel() == col.numel() == 0
+    assert g._CAPI_RelabelledRows(cols, rows, w.double(), None) is None
+    assert g._CAPI_RelabelledRows(cols, rows, w[::2], None) is None
+    assert g._CAPI_RelabelledRows(cols, rows, w, torch.ones(89, device=DEV)) is None
+    assert g._CAPI_RelabelledRows(cols, T(rng.permutation(900)[:700]), w, None) is None
+    assert g._CAPI_RelabelledRows(cols, rows, w, torch.ones(90, device=DEV)) is not None
+    short = g._CAPI_RelabelledRows(cols, rows, w[:2500], None)[3]
+    sub, index = g._CAPI_ColRowSlicing(cols, rows, gs.format._CSC, gs.format._CSC)
+    assert torch.allclose(short, sub._CAPI_NormaliseColumns(w[:2500], index, None), rtol=1e-6)
+
+
+def handed_on(A, seeds, k, also):
+    sub = A[:, seeds]
+    sub.edata["p"] = sub.edata["w"] ** 2
+    prob = sub.sum("p", axis=1)
+    picked, index = sub.collective_sampling(k, prob, False)
+    picked = picked.div("w", prob[index], axis=1)
+    picked = picked.div("w", picked.sum("w", axis=0), axis=0)
+    block = picked.to_dgl_block(prefetch_edata={"w"})
+    more = picked.sum("w", axis=1) if also == "sums" else index
+    return picked.all_nodes(), block, more
+
+
+@pytest.mark.parametrize("also", [None, "sums"])
+def test_which_row_slices_are_only_handed_on(also):
+    from gsampler_amd.ops.fused_op import _relabelled_rows
+    rng = np.random.default_rng(21)
+    indptr, indices = random_csc(rng, 500, 500, 300)
+    m = gs.Matrix(gs.Graph(500, 500))
+    m._graph._CAPI_LoadCSC(T(indptr), T(indices))
+    m.edata["w"] = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+
+    def sampler(A, seeds):
+        return handed_on(A, seeds, 30, also)
+
+    seeds = T(rng.permutation(500)[:64])
+    compiled = gs.jit.compile(func=sampler, args=(m, seeds))
+    targets = [n.target for n in compiled._run.__self__.graph.nodes]
+    assert targets.count(_relabelled_rows) == (also != "sums")
+    results = []
+    for run in (compiled, handed_on_by_operators(compiled)):
+        gs.manual_seed(3)
+        nodes, block, more = run(m, seeds)
+        results.append([nodes, block.row, block.col, block.edata["w"], more])
+    for a, b in zip(*results):
+        assert torch.allclose(a.double(), b.double(), rtol=1e-6)
+
+
+def handed_on_by_operators(compiled):
+    import copy
+    other = copy.copy(compiled)
+    other._run = None  # the operator graph itself
+    return other
