@@ -285,6 +285,15 @@ class Graph : public torch::CustomClassHolder {
                            c10::optional<torch::Tensor>>>
   RelabelledRows(torch::Tensor cols, torch::Tensor rows, c10::optional<torch::Tensor> values,
                  c10::optional<torch::Tensor> row_divisor);
+  // The same of a super-batch, as EncodedPickedRows (with `seeds` and the names of the picked
+  // rows) and BatchBlocks leave it, and of the subgraphs that lists of nodes induce, as
+  // BatchColRowSlcing of a list by itself does.
+  c10::optional<std::tuple<c10::intrusive_ptr<BlockBatch>, c10::optional<torch::Tensor>>>
+  EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
+                torch::Tensor row_ids, torch::Tensor row_bptr,
+                c10::optional<torch::Tensor> values, c10::optional<torch::Tensor> row_divisor);
+  c10::optional<c10::intrusive_ptr<BlockBatch>> SubgraphBlocks(torch::Tensor nodes,
+                                                               torch::Tensor nodes_ptr);
   void FusedUOPV(const std::string& op, torch::Tensor lhs1, torch::Tensor rhs1,
                  torch::Tensor out1, torch::Tensor lhs2, torch::Tensor rhs2,
                  torch::Tensor out2, int64_t on_format);

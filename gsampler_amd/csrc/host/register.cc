@@ -120,6 +120,8 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_SampleLayers", &Graph::SampleLayers)
       .def("_CAPI_BatchSampleLayers", &Graph::BatchSampleLayers)
       .def("_CAPI_RelabelledRows", &Graph::RelabelledRows)
+      .def("_CAPI_EncodedBlocks", &Graph::EncodedBlocks)
+      .def("_CAPI_SubgraphBlocks", &Graph::SubgraphBlocks)
       .def("_CAPI_NormaliseColumns", &Graph::NormaliseColumns)
       .def("_CAPI_EncodedSquareSums", &Graph::EncodedSquareSums)
       .def("_CAPI_EncodedPickedRows", &Graph::EncodedPickedRows)

@@ -1080,48 +1080,65 @@ def sum_slices_into_new_arrays(copy: fx.Graph) -> None:
 
 
 def relabel_row_slices(copy: fx.Graph) -> None:
-    """In a copy of a graph: a row slice A[rows, cols] that is relabelled by cols and rows,
-    whose edges' normalised values may be wanted, and nothing else  => one _relabelled_rows."""
-    from ..ops.fused_op import _normalised, _relabelled_rows
+    """In a copy of a graph: a row slice that is relabelled by its columns and rows, whose
+    edges' normalised values may be wanted, and nothing else: A[rows, cols]  => one
+    _relabelled_rows, the picked rows of an encoded slice  => one _encoded_blocks, lists of
+    nodes by themselves  => one _subgraph_blocks."""
+    from ..ops.fused_op import (_encoded_blocks, _encoded_row_slice, _normalised, _relabelled_rows,
+                                _subgraph_blocks)
     order = {n: i for i, n in enumerate(copy.nodes)}
     replaced = []
     for cut in list(copy.nodes):
-        if not _is_method(cut, "_CAPI_ColRowSlicing") or len(cut.args) != 5 or cut.kwargs:
+        single = _is_method(cut, "_CAPI_ColRowSlicing") and len(cut.args) == 5
+        picked = _call(cut, _encoded_row_slice) and len(cut.args) == 4
+        square = (_is_method(cut, "_CAPI_BatchColRowSlcing") and len(cut.args) == 5
+                  and cut.args[3] is cut.args[1] and cut.args[4] is cut.args[2])
+        if not (single or picked or square) or cut.kwargs:
             continue
-        g, cols, rows, *formats = cut.args
-        if any(not _call(u, operator.getitem) or u.args[1] not in (0, 1) for u in cut.users):
+        if any(not _call(u, operator.getitem) or u.args[1] not in (0, 1, 2) for u in cut.users):
             continue
-        readers = {u for m in _getitem_users(cut, 0) for u in m.users}
-        labels = [u for u in readers if _is_method(u, "_CAPI_GraphRelabel")]
+        sub, index, names = (_getitem_users(cut, i) for i in range(3))
+        readers = {u for m in sub for u in m.users}
+        labels = [u for u in readers
+                  if _is_method(u, "_CAPI_GraphRelabel" if single else "_CAPI_BatchBlocks")]
         values = [u for u in readers if _call(u, _normalised)]
         if len(labels) != 1 or len(values) > 1 or len(readers) != len(labels) + len(values):
             continue
         label = labels[0]
-        if label.args[1] is not cols or label.args[2] is not rows or label.kwargs:
+        if label.kwargs or len(label.args) != 3 or label.args[0] not in sub:
             continue
-        inputs, wanted = [], {u for i in _getitem_users(cut, 1) for u in i.users}
-        if values:
-            m, e, select, divisor, value_formats = values[0].args
-            if not (_call(select, operator.getitem) and select.args[0] is cut and select.args[1] == 1):
+        seeds, ids = label.args[1:]
+        if picked:
+            if ids not in names or {u for n in names for u in n.users} != {label}:
                 continue
-            inputs = [e, divisor, value_formats]
-        if wanted != set(values):
+        elif seeds is not cut.args[1] or ids is not (cut.args[2] if single else cut.args[1]):
+            continue
+        inputs = []
+        if values:
+            if square or values[0].args[0] not in sub or values[0].args[2] not in index:
+                continue
+            inputs = [values[0].args[1], *values[0].args[3:]]
+            if any(a in index or a in sub for a in inputs):
+                continue
+        if {u for i in index for u in i.users} != set(values):
             continue
         first = min([label, *values], key=order.get)
-        # (an operand that is there before the slice is read; the divisor may be made from it later)
-        if any(isinstance(a, fx.Node) and order.get(a, -1) >= order[first] for a in inputs):
-            continue
-        if _written_between(order, [cut, label, *values]):
+        # (made where the first of its readers stands: what the other one reads has to be there)
+        if any(isinstance(a, fx.Node) and order.get(a, len(order)) >= order[first]
+               for a in (seeds, *inputs)) or _written_between(order, [cut, label, *values]):
             continue
         with copy.inserting_before(first):
-            new = copy.call_function(_relabelled_rows, args=(g, cols, rows, tuple(formats), *inputs))
-            parts = [copy.call_function(operator.getitem, args=(new, i)) for i in range(2)]
+            if square:
+                new = copy.call_function(_subgraph_blocks, args=cut.args[:3])
+                parts = [new]
+            else:
+                new = (copy.call_function(_relabelled_rows, args=(*cut.args[:3], tuple(cut.args[3:]), *inputs))
+                       if single else copy.call_function(_encoded_blocks, args=(*cut.args, seeds, *inputs)))
+                parts = [copy.call_function(operator.getitem, args=(new, i)) for i in range(2)]
         label.replace_all_uses_with(parts[0])
-        replaced.append(label)
         for v in values:
             v.replace_all_uses_with(parts[1])
-            replaced.append(v)
-        replaced.append(cut)
+        replaced += [cut, label, *values]
     if replaced:
         _drop_dead_nodes(copy, replaced)
 

@@ -102,6 +102,28 @@ def _relabelled_rows(g, cols, rows, formats, values=None, divisor=None, value_fo
     return sub._CAPI_GraphRelabel(cols, rows), e
 
 
+def _encoded_blocks(part, row_ids, rows_ptr, rows, seeds, values=None, divisor=None,
+                    value_formats=None):
+    """The same of a super-batched sampler: the blocks of _encoded_row_slice(part, ...)."""
+    if (len(part) == 4 and part[1] is seeds and part[3] is rows
+            and all(t is None or type(t) is torch.Tensor for t in (values, divisor))):
+        out = part[0]._CAPI_EncodedBlocks(*part[1:], row_ids, rows_ptr, values, divisor)
+        if out is not None:
+            return out
+    sub, index, names = _encoded_row_slice(part, row_ids, rows_ptr, rows)
+    e = None if values is None else _normalised(sub, values, index, divisor, value_formats)
+    return sub._CAPI_BatchBlocks(seeds, names), e
+
+
+def _subgraph_blocks(g, nodes, nodes_ptr):
+    """The blocks of the subgraphs that lists of nodes induce."""
+    out = g._CAPI_SubgraphBlocks(nodes, nodes_ptr)
+    if out is not None:
+        return out
+    sub, _ = g._CAPI_BatchColRowSlcing(nodes, nodes_ptr, nodes, nodes_ptr)
+    return sub._CAPI_BatchBlocks(nodes, nodes)
+
+
 def _sliced_square_sums(g, cols, values):
     """Sums of the squared values over the edges of the column slice g[:, cols] onto its rows."""
     if type(values) is torch.Tensor and not values.requires_grad:

@@ -545,6 +545,55 @@ def test_row_slice_that_is_only_handed_on(shape, values):
         assert got[3] is None
 
 
+def same_blocks(got, want):
+    for part in ("frontier", "frontier_ptr", "row", "col", "indptr", "edge_ptr", "col_ptr"):
+        assert torch.equal(getattr(got, part)(), getattr(want, part)()), part
+    assert got.edge_ids() is None and want.edge_ids() is None and got.totals() == want.totals()
+
+
+def batches_of(rng, num_ids, sizes):
+    lists = [rng.choice(num_ids, size=k, replace=False) for k in sizes]
+    return T(np.concatenate(lists)), T(np.concatenate([[0], np.cumsum(sizes)]))
+
+
+@pytest.mark.parametrize("values", [True, False])
+@pytest.mark.parametrize("seeds,picks", [([40], [90]), ([64, 0, 300, 1], [0, 90, 120, 60]), ([3] * 70, [5] * 70),
+                                         ([1900, 20, 20, 20], [200, 9, 9, 9])])
+def test_encoded_row_slice_that_is_only_handed_on(seeds, picks, values):
+    rng = np.random.default_rng(len(seeds))
+    indptr, indices = columns_of(rng.integers(0, 500, 2500), rng, 2500)
+    g = gs.Graph(2500, 2500)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+    refused = max(seeds) + max(picks) > 2048  # more keys in a batch than one work-group takes
+    seeds, ptr = batches_of(rng, 2500, seeds)
+    rows, rows_ptr, _ = g._CAPI_EncodedSquareSums(seeds, ptr, w)
+    counts, starts = torch.diff(rows_ptr).tolist(), rows_ptr.tolist()
+    chosen = [a + rng.choice(n, size=min(k, n), replace=False) for a, n, k in zip(starts, counts, picks)]
+    row_ids, row_ptr = T(np.concatenate(chosen)), T(np.concatenate([[0], np.cumsum([len(c) for c in chosen])]))
+    by = torch.as_tensor((2.0 ** rng.integers(-2, 3, size=row_ids.numel())).astype(np.float32), device=DEV)
+    extra = (w, by) if values else (None, None)
+    got = g._CAPI_EncodedBlocks(seeds, ptr, rows, row_ids, row_ptr, *extra)
+    assert (got is None) == refused
+    if refused:
+        return
+    sub, index, names = g._CAPI_EncodedPickedRows(seeds, ptr, rows, row_ids, row_ptr)
+    same_blocks(got[0], sub._CAPI_BatchBlocks(seeds, names))
+    assert torch.equal(got[1], sub._CAPI_NormaliseColumns(w, index, by)) if values else got[1] is None
+
+
+@pytest.mark.parametrize("sizes", [[40], [64, 0, 300, 1], [3] * 70, [3000, 20_000]])
+def test_subgraphs_that_are_only_handed_on(sizes):
+    rng = np.random.default_rng(len(sizes))
+    indptr, indices = columns_of(rng.integers(0, 60, 30_000), rng, 30_000)
+    g = gs.Graph(30_000, 30_000)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    nodes, ptr = batches_of(rng, 30_000, sizes)
+    nodes[1] = nodes[0]
+    sub, _ = g._CAPI_BatchColRowSlcing(nodes, ptr, nodes, ptr)
+    same_blocks(g._CAPI_SubgraphBlocks(nodes, ptr), sub._CAPI_BatchBlocks(nodes, nodes))
+
+
 def test_row_slices_that_have_to_be_written():
     """No edge is kept, edge data of other types, too few edges for the pass, a parent with
     edge ids of its own; and edge data shorter than the edges."""
@@ -602,6 +651,50 @@ def test_which_row_slices_are_only_handed_on(also):
         results.append([nodes, block.row, block.col, block.edata["w"], more])
     for a, b in zip(*results):
         assert torch.allclose(a.double(), b.double(), rtol=1e-6)
+
+
+@pytest.mark.parametrize("also", [None, "sums"])
+def test_which_slices_of_batches_are_only_handed_on(also):
+    from gsampler_amd.ops.fused_op import _encoded_blocks, _subgraph_blocks
+    rng = np.random.default_rng(22)
+    indptr, indices = random_csc(rng, 500, 500, 300)
+    bm, m = gs.BatchMatrix(), gs.Matrix(gs.Graph(500, 500))
+    m._graph._CAPI_LoadCSC(T(indptr), T(indices))
+    m.edata["w"] = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+
+    def layers(A, seeds, ptr):
+        sub = A[:, seeds::ptr]
+        sub.edata["p"] = sub.edata["w"] ** 2
+        prob = sub.sum("p", axis=1)
+        _, rows_ptr = sub.all_rows()
+        picked, index = sub.collective_sampling(30, prob, rows_ptr, False)
+        picked = picked.div("w", prob[index], axis=1)
+        picked = picked.div("w", picked.sum("w", axis=0), axis=0)
+        nodes, ptr = picked.all_nodes()
+        return nodes, picked.to_dgl_block(prefetch_edata={"w"}), picked.sum("w", axis=1) if also else index
+
+    def subgraphs(A, nodes, ptr):
+        sub = A[nodes::ptr, nodes::ptr]
+        return sub.to_dgl_block(), sub.all_nodes()[0], sub.sum("w", axis=1) if also else ptr
+
+    def flat(out):
+        tensors = [t for t in out if isinstance(t, torch.Tensor)]
+        for blocks in (b for b in out if not isinstance(b, torch.Tensor)):
+            tensors += [t for b in blocks for t in (b.row, b.col, b.srcdata["_ID"], *b.edata.values())]
+        return tensors
+
+    for func, encoded, target in ((layers, True, _encoded_blocks), (subgraphs, False, _subgraph_blocks)):
+        bm.load_from_matrix(m, encoded)
+        args = (bm, *batches_of(rng, 500, [40, 0, 64]))
+        compiled = gs.jit.compile(func=func, args=args)
+        targets = [n.target for n in compiled._run.__self__.graph.nodes]
+        assert targets.count(target) == (also is None), func.__name__
+        results = []
+        for run in (compiled, handed_on_by_operators(compiled)):
+            gs.manual_seed(3)
+            results.append(flat(run(*args)))
+        for a, b in zip(*results):
+            assert torch.allclose(a.double(), b.double(), rtol=1e-6)
 
 
 def handed_on_by_operators(compiled):
