@@ -18,26 +18,46 @@ namespace gs {
 // they are handed the same tensor of columns (one wait for the size, not two)
 // on the same stream: another one would have to wait for what is queued on the
 // first, and memory that is freed there may be written again while it reads.
-std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tensor& cols) {
+// `wait`: for the size as well (the host copy of one that is not waited for keeps the offsets).
+std::shared_ptr<Graph::SliceOffsets> Graph::slice_offsets_for(const torch::Tensor& cols, bool wait) {
   const Compressed& m = compressed(kCSC);
+  wait |= cols.numel() > (1 << 16);
+  std::shared_ptr<SliceOffsets> so;
   {
     std::lock_guard<std::mutex> lock(slice_offsets_guard_);
     if (slice_offsets_ && slice_offsets_->cols.is_same(cols) &&
         slice_offsets_->version == (int64_t)cols._version() &&
         slice_offsets_->indptr_version == (int64_t)m.indptr._version() &&
         slice_offsets_->epoch == cache_epoch() && slice_offsets_->stream == cur_stream())
-      return slice_offsets_;
+      so = slice_offsets_;
   }
-  auto so = std::make_shared<SliceOffsets>();
-  so->cols = cols;
-  so->version = cols._version();
-  so->indptr_version = m.indptr._version();
-  so->epoch = cache_epoch();
-  so->stream = cur_stream();
-  so->sub_indptr = slice_offsets(m, cols, &so->nnz);
-  std::lock_guard<std::mutex> lock(slice_offsets_guard_);
-  slice_offsets_ = so;
+  if (!so) {
+    so = std::make_shared<SliceOffsets>();
+    so->cols = cols;
+    so->version = cols._version();
+    so->indptr_version = m.indptr._version();
+    so->epoch = cache_epoch();
+    so->stream = cur_stream();
+    so->sub_indptr = wait ? slice_offsets(m, cols, &so->nnz) : slice_offsets_ahead(m, cols, &so->total);
+    std::lock_guard<std::mutex> lock(slice_offsets_guard_);
+    slice_offsets_ = so;
+  }
+  if (wait) {
+    std::lock_guard<std::mutex> lock(so->guard);
+    if (so->nnz < 0) so->nnz = OffsetMirror::values(so->total)[0];
+  }
   return so;
+}
+
+// A sampler whose picks do not depend on the slice (FastGCN) asks for its offsets before it
+// picks: their number is at hand when the slice is made, where the device stood still while
+// it travelled to the host (FastGCN of 1024 seeds 228 -> 215 us a pass).
+void Graph::PrepareSlice(torch::Tensor cols) {
+  if (!csc_ || !csc_->indices.is_cuda() || !csc_->indptr.is_cuda() || !cols.is_cuda() ||
+      cols.scalar_type() != torch::kInt64 || cols.dim() != 1 || !cols.is_contiguous() ||
+      cols.numel() == 0)
+    return;
+  slice_offsets_for(cols, false);
 }
 
 // A slice of a matrix in device memory is read in place whatever its columns are like:
@@ -577,12 +597,13 @@ c10::optional<c10::intrusive_ptr<BlockBatch>> Graph::SubgraphBlocks(torch::Tenso
   const int64_t n = nodes.numel(), B = nodes_ptr.numel() - 1;
   if (!m.indices.is_cuda() || n == 0 || B < 1) return {};
   BatchOffsets::check(nodes_ptr, n, "BatchColRowSlicing");
-  const std::shared_ptr<SliceOffsets> so = slice_offsets_for(nodes);
-  const int64_t nnz = so->nnz;
-  if (nnz < n || nnz > kBoundLimit) return {};
+  slice_offsets_for(nodes, false);
   torch::Tensor picked = new_ids(n, nodes), key_offset = new_ids(n, nodes);
   GS_CALL(gs_pick_batch_ids(cptr(nodes), n, nullptr, cptr(nodes_ptr), B, n, num_rows_, nullptr,
                             mptr(picked), mptr(key_offset), cur_stream()));
+  const std::shared_ptr<SliceOffsets> so = slice_offsets_for(nodes);
+  const int64_t nnz = so->nnz;
+  if (nnz < n || nnz > kBoundLimit) return {};
   const torch::Tensor narrow = narrow_for_slice(m, nnz, n);
   torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, n), m.indptr);
   torch::Tensor indptr = new_ids(n + 1, m.indptr), label = new_ids(n, m.indptr);

@@ -191,16 +191,31 @@ const Compressed& Graph::compressed(int64_t format) {
 }
 
 // ---------------------------------------------------- operators, major axis
-torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, int64_t* nnz) {
+static torch::Tensor queue_slice_offsets(const Compressed& m, const torch::Tensor& picked,
+                                         torch::Tensor offsets, int64_t* mirror) {
   const int64_t n = picked.numel();
-  torch::Tensor offsets = new_ids(n + 1, m.indptr);
   torch::Tensor ws = new_workspace(gs_scan_workspace_bytes(n + 1), m.indptr);
-  AsyncCount count = AsyncCount::mirrored();
   GS_CALL(gs_csc_col_count(cptr(m.indptr), m.indptr.numel() - 1, cptr(picked), n, -1, 0,
-                           mptr(offsets), count.mirror(), nullptr, ws.data_ptr(), ws.numel(),
+                           mptr(offsets), mirror, nullptr, ws.data_ptr(), ws.numel(),
                            cur_stream()));
+  return offsets;
+}
+
+torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, int64_t* nnz) {
+  AsyncCount count = AsyncCount::mirrored();
+  torch::Tensor offsets = queue_slice_offsets(m, picked, new_ids(picked.numel() + 1, m.indptr),
+                                              count.mirror());
   count.arm();
   *nnz = count.get();
+  return offsets;
+}
+
+torch::Tensor slice_offsets_ahead(const Compressed& m, const torch::Tensor& picked,
+                                  torch::Tensor* total) {
+  torch::Tensor offsets = new_ids(picked.numel() + 1, m.indptr);
+  *total = offsets.narrow(0, picked.numel(), 1);
+  queue_slice_offsets(m, picked, offsets, OffsetMirror::reserve(*total));
+  OffsetMirror::arm(*total);
   return offsets;
 }
 

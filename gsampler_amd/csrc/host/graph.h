@@ -292,6 +292,8 @@ class Graph : public torch::CustomClassHolder {
   EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
                 torch::Tensor row_ids, torch::Tensor row_bptr,
                 c10::optional<torch::Tensor> values, c10::optional<torch::Tensor> row_divisor);
+  // Queues what an operator that slices these columns would wait for first.
+  void PrepareSlice(torch::Tensor cols);
   c10::optional<c10::intrusive_ptr<BlockBatch>> SubgraphBlocks(torch::Tensor nodes,
                                                                torch::Tensor nodes_ptr);
   void FusedUOPV(const std::string& op, torch::Tensor lhs1, torch::Tensor rhs1,
@@ -456,7 +458,9 @@ class Graph : public torch::CustomClassHolder {
   // one holds stays when another puts its own in its place.)
   struct SliceOffsets {
     torch::Tensor cols, sub_indptr;
-    int64_t version = -1, indptr_version = -1, epoch = -1, nnz = 0;
+    int64_t version = -1, indptr_version = -1, epoch = -1;
+    int64_t nnz = -1;        // (waited for under the guard)
+    torch::Tensor total;     // where it is on its way to the host from
     void* stream = nullptr;  // whose kernels write the tensors
     std::mutex guard;
     MajorResult written;  // the slice itself, when an operator had to write it
@@ -468,7 +472,7 @@ class Graph : public torch::CustomClassHolder {
   };
   std::mutex slice_offsets_guard_;
   std::shared_ptr<SliceOffsets> slice_offsets_;
-  std::shared_ptr<SliceOffsets> slice_offsets_for(const torch::Tensor& cols);
+  std::shared_ptr<SliceOffsets> slice_offsets_for(const torch::Tensor& cols, bool wait = true);
   static bool read_in_place(const Compressed& m, int64_t slice_nnz, int64_t num_cols_picked);
   const MajorResult& written_slice(SliceOffsets& so);
   torch::Tensor key_offsets_for(SliceOffsets& so, const torch::Tensor& col_bptr);
@@ -571,6 +575,9 @@ class Graph : public torch::CustomClassHolder {
 
 // Offsets of the slice along the compressed axis by `picked`, and its size.
 torch::Tensor slice_offsets(const Compressed& m, const torch::Tensor& picked, int64_t* nnz);
+// The same without waiting for the number of edges: it stays with the last of the offsets.
+torch::Tensor slice_offsets_ahead(const Compressed& m, const torch::Tensor& picked,
+                                  torch::Tensor* total);
 // Operators along the compressed axis (graph.cc) and across it (slicing.cc).
 MajorResult major_slice(const Compressed& m, const torch::Tensor& picked,
                         bool with_coo, const torch::Tensor& batch_ptr,

@@ -119,6 +119,7 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_BatchBlocks", &Graph::BatchBlocks)
       .def("_CAPI_SampleLayers", &Graph::SampleLayers)
       .def("_CAPI_BatchSampleLayers", &Graph::BatchSampleLayers)
+      .def("_CAPI_PrepareSlice", &Graph::PrepareSlice)
       .def("_CAPI_RelabelledRows", &Graph::RelabelledRows)
       .def("_CAPI_EncodedBlocks", &Graph::EncodedBlocks)
       .def("_CAPI_SubgraphBlocks", &Graph::SubgraphBlocks)

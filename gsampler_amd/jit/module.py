@@ -179,6 +179,7 @@ class compile:  # noqa: N801 -- the reference's public name
         passes.weights_of_picks(graph)
         passes.sum_slices_into_new_arrays(graph)
         passes.relabel_row_slices(graph)
+        passes.count_slices_ahead(graph)
         return fx.GraphModule(gm, graph).forward
 
     def __call__(self, *args):

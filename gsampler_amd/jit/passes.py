@@ -1143,6 +1143,27 @@ def relabel_row_slices(copy: fx.Graph) -> None:
         _drop_dead_nodes(copy, replaced)
 
 
+def count_slices_ahead(copy: fx.Graph) -> None:
+    """In a copy of a graph: the offsets of a row slice's columns, which it waits for first, are
+    asked for before its rows are picked where nothing has asked for them yet."""
+    from ..ops.fused_op import _picks_and_weights, _relabelled_rows
+    order = {n: i for i, n in enumerate(copy.nodes)}
+    for cut in list(copy.nodes):
+        if not (_call(cut, _relabelled_rows) or _is_method(cut, "_CAPI_ColRowSlicing")):
+            continue
+        g, cols, rows = cut.args[:3]
+        pick = rows.args[0] if _call(rows, operator.getitem) else rows
+        name = str(getattr(pick.target, "__name__", pick.target)).split(".")[0]
+        if not (_call(pick, _picks_and_weights) or pick.op == "call_function" and name in (
+                "_CAPI_ListSampling", "_CAPI_ListSamplingWithProbs")):
+            continue
+        asked = {u for u in cols.users if g in u.all_input_nodes and order.get(u, -1) < order[cut]}
+        if asked or max(order[g], order[cols]) >= order[pick]:
+            continue
+        with copy.inserting_before(pick):
+            copy.call_method("_CAPI_PrepareSlice", args=(g, cols))
+
+
 def share_leading_rows(copy: fx.Graph) -> None:
     """In a copy of a graph: the rows of a column slice are its parent's, so what is
     computed from data of all of them in one layer is what the next one computes.  Merges
