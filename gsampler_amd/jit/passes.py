@@ -41,6 +41,10 @@ and, in the copy of the graph that calls run (like chain_layers):
   share_leading_rows            features of all rows of a column slice: the parent's, once
   sum_slices_into_new_arrays    sums over a column slice that is not written
   weights_of_picks              picks of a list by weight and their weights  -> one operator
+  relabel_row_slices            row slices that are only relabelled (and whose normalised
+                                values are wanted) are not written
+  count_slices_ahead            the size of a row slice is on its way before its rows are
+                                picked
 
 A pass rewrites `gm.graph` and checks it; the module's code is generated once, by
 whoever runs the passes (gm.recompile()): generating it after each of them was
