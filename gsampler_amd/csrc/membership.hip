@@ -1054,8 +1054,15 @@ __global__ __launch_bounds__(kBlock) void member_label_kernel(
     for (int j = 0; j < kMemberWords; ++j) {
       if (j * kWave + lane >= kept[c]) continue;
       const int64_t pos = out0 + j * kWave + lane;
-      edges.row[pos] = (int64_t)row[c][j];
-      edges.col[pos] = (int64_t)col[c][j];
+      // (past L2 where the list is long: the passes over the values behind this one find more
+      // there, LADIES 577 -> 569 us; what a short list leaves may be read from it)
+      if (kRun > 1) {
+        __builtin_nontemporal_store((int64_t)row[c][j], edges.row + pos);
+        __builtin_nontemporal_store((int64_t)col[c][j], edges.col + pos);
+      } else {
+        edges.row[pos] = (int64_t)row[c][j];
+        edges.col[pos] = (int64_t)col[c][j];
+      }
       if (kValues) edges.out[pos] = edges.row_divisor ? v[c][j] / by[c][j] : v[c][j];
     }
   }
