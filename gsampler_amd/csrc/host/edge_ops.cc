@@ -266,12 +266,9 @@ c10::optional<torch::Tensor> Graph::NormaliseColumns(torch::Tensor values,
     row_divisor = row_divisor->contiguous();
   }
   torch::Tensor out = torch::empty({num_edges_}, values.options().requires_grad(false));
-  torch::Tensor sums;  // (of 64 bits: the slice that made this matrix may have left them cleared)
-  {
-    std::lock_guard<std::mutex> lock(column_zeros_guard_);
-    std::swap(sums, column_zeros_);
-  }
-  const bool cleared = sums.defined() && sums.numel() == num_cols_;
+  // (of 64 bits: the slice that made this matrix may have left them cleared)
+  torch::Tensor sums = take_column_zeros();
+  const bool cleared = sums.defined();
   if (!cleared) sums = new_ids(num_cols_, csc_->indptr);
   auto* normalise = cleared ? &gs_normalise_columns_cleared : &gs_normalise_columns;
   GS_CALL(normalise(cptr(csc_->indptr), num_cols_, cptr(csc_->indices), num_edges_,

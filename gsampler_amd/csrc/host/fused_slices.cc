@@ -216,7 +216,7 @@ GraphAndIndex Graph::ColRowSlicing(torch::Tensor cols, torch::Tensor rows, int64
   }
   GraphPtr g = derive(kCSC, output_format, r, rows.numel(), cols.numel());
   g->keep_row_firsts(firsts, r.minor_ids);
-  g->column_zeros_ = zeros;
+  g->keep_column_zeros(zeros);
   return {g, edge_index(m.e_ids, r.select)};
 }
 
@@ -319,6 +319,22 @@ void Graph::keep_row_firsts(const torch::Tensor& firsts, const torch::Tensor& ed
   row_firsts_of_ = edge_rows;
   row_firsts_version_ = (int64_t)edge_rows._version();
   row_firsts_epoch_ = cache_epoch();
+}
+
+void Graph::keep_column_zeros(const torch::Tensor& zeros) {
+  if (!zeros.defined()) return;
+  column_zeros_ = zeros;
+  column_zeros_stream_ = cur_stream();
+}
+
+// (nothing where they are not this call's to use)
+torch::Tensor Graph::take_column_zeros() {
+  torch::Tensor zeros;
+  std::lock_guard<std::mutex> lock(column_zeros_guard_);
+  if (column_zeros_.defined() && column_zeros_.numel() == num_cols_ &&
+      column_zeros_stream_ == cur_stream() && !capturing())
+    std::swap(zeros, column_zeros_);
+  return zeros;
 }
 
 // The ids `of` (undefined: zeros) of every batch moved by batch * stride.
@@ -471,7 +487,7 @@ GraphAndIndex Graph::encoded_row_slice(const torch::Tensor& seeds, const torch::
                                       true, &firsts, &zeros);
   GraphPtr g = derive(kCSC, kCSC | kCOO, r, row_ids.numel(), seeds.numel());
   g->keep_row_firsts(firsts, r.minor_ids);
-  g->column_zeros_ = zeros;
+  g->keep_column_zeros(zeros);
   g->col_bptr_ = col_bptr;
   g->orig_col_ids_ = seeds;
   g->row_encoding_size_ = num_rows_;

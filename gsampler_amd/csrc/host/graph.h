@@ -545,9 +545,14 @@ class Graph : public torch::CustomClassHolder {
   // Which edge of a row slice is the first of each of its rows, as the pass that made the
   // slice has met them; nothing once the rows of the edges have been written to.
   torch::Tensor row_firsts_, row_firsts_of_;
-  // A value a column that is zero, for the first sum over columns that asks for one.
+  // A value a column that is zero, for the first sum over columns that asks for one on the
+  // stream whose slice cleared them: another stream's kernels would still add to memory
+  // that goes back to this one, and a graph that is being recorded would not clear them.
   torch::Tensor column_zeros_;
+  gs_stream_t column_zeros_stream_ = nullptr;
   std::mutex column_zeros_guard_;
+  void keep_column_zeros(const torch::Tensor& zeros);
+  torch::Tensor take_column_zeros();
   int64_t row_firsts_version_ = -1, row_firsts_epoch_ = -1;
   // The rows of the edges of A[list, list], while each is still a position of the list in the
   // segment of its edge's mini-batch: what the slice wrote.

@@ -502,6 +502,63 @@ def test_normalised_columns_of_one_slice_several_times():
     assert torch.allclose(got[0].double(), w[index].double() / sums[col], rtol=1e-6)
 
 
+def sliced_for_sums(rng, num_rows=3000):
+    """A row slice whose sums over columns have storage of their own (more rows than first
+    edges are told of), and the normalised values it is to have."""
+    indptr, indices = random_csc(rng, 300, num_rows, 90)
+    g = gs.Graph(num_rows, 300)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.random(indices.size).astype(np.float32) + 0.1, device=DEV)
+
+    def slice_():
+        return g._CAPI_ColRowSlicing(cols, rows, gs.format._CSC, gs.format._CSC | gs.format._COO)
+
+    cols, rows = T(rng.permutation(300)[:200]), T(rng.permutation(num_rows)[:2500])
+    sub, index = slice_()
+    sub._CAPI_NormaliseColumns(w, index, None)            # (takes what the slice cleared)
+    return slice_, w, sub._CAPI_NormaliseColumns(w, index, None)
+
+
+def test_normalised_columns_on_another_stream_than_the_slice():
+    """Sums that the slice's stream cleared are not used by another stream: their memory goes
+    back to the first one, which may hand it out while the second still adds to it."""
+    slice_, w, want = sliced_for_sums(np.random.default_rng(12))
+    other = torch.cuda.Stream()
+    busy = torch.rand(4096, 4096, device=DEV)
+    for _ in range(3):
+        sub, index = slice_()
+        other.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(other):
+            for _ in range(20):
+                busy @ busy                               # the kernels below start after this
+            got = sub._CAPI_NormaliseColumns(w, index, None)
+        # what this stream gets of the size of the sums, written before they are made
+        taken = [torch.full((200,), 1e30, dtype=torch.float64, device=DEV) for _ in range(64)]
+        other.synchronize()
+        assert torch.allclose(got, want, rtol=1e-6)
+        assert all((t == 1e30).all() for t in taken)
+
+
+def test_normalised_columns_recorded_behind_a_slice():
+    """A graph that is recorded clears the sums itself: every replay has the eager result."""
+    slice_, w, want = sliced_for_sums(np.random.default_rng(13))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        sub, index = slice_()
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            got = sub._CAPI_NormaliseColumns(w, index, None)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.allclose(got, want, rtol=1e-6)
+        assert torch.allclose(sub._CAPI_NormaliseColumns(w, index, None), want, rtol=1e-6)
+
+
 def columns_of(lengths, rng, num_rows):
     indptr = np.concatenate([[0], np.cumsum(lengths)])
     return indptr, rng.integers(0, num_rows, size=int(indptr[-1])).astype(np.int64)
