@@ -138,21 +138,23 @@ __global__ __launch_bounds__(kBlock) void seeds_distinct_kernel(
   if (b < num_batches) distinct[b] = seeds_distinct(b, frontier, frontier_ptr, seeds, seeds_ptr);
 }
 
-// Both for the hand-over of a layer's blocks, the flags straight to the host: one launch of
-// 6 us where the pointers, the flags and the flags' copy were three, 11 us and the gaps.
+// Both for the hand-over of a layer's blocks, the flags straight to the host as well: one
+// launch of 6 us where the pointers, the flags and the flags' copy were three, 11 us and the
+// gaps.
 __global__ __launch_bounds__(kBlock) void block_offsets_kernel(
     const int64_t* __restrict__ indptr, const int64_t* __restrict__ seeds_ptr,
     int64_t num_batches, int64_t out_len, int64_t* __restrict__ out, unsigned tiles,
     const int64_t* __restrict__ frontier, const int64_t* __restrict__ frontier_ptr,
-    const int64_t* __restrict__ seeds, int64_t* distinct_mirror) {
+    const int64_t* __restrict__ seeds, int64_t* __restrict__ distinct, int64_t* distinct_mirror) {
   if (blockIdx.x < tiles) {
     split_tile(blockIdx.x, indptr, seeds_ptr, num_batches, out_len, out);
     return;
   }
   const int64_t b = (int64_t)(blockIdx.x - tiles) * kBlock + threadIdx.x;
-  if (b < num_batches)
-    store_for_host(distinct_mirror + b,
-                   seeds_distinct(b, frontier, frontier_ptr, seeds, seeds_ptr));
+  if (b >= num_batches) return;
+  const int64_t flag = seeds_distinct(b, frontier, frontier_ptr, seeds, seeds_ptr);
+  distinct[b] = flag;
+  if (distinct_mirror) store_for_host(distinct_mirror + b, flag);
 }
 
 }  // namespace gs
@@ -177,12 +179,12 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
 
 int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int64_t num_batches,
                            int64_t out_len, int64_t* out, const int64_t* frontier,
-                           const int64_t* frontier_ptr, const int64_t* seeds,
+                           const int64_t* frontier_ptr, const int64_t* seeds, int64_t* distinct,
                            int64_t* distinct_mirror, gs_stream_t stream) {
   using namespace gs;
   GS_REQUIRE(num_batches >= 0 && out_len >= 0, "batch_block_offsets: negative size");
   if (num_batches == 0) return GS_OK;
-  GS_REQUIRE(indptr && seeds_ptr && (out || out_len == 0) && frontier_ptr && distinct_mirror,
+  GS_REQUIRE(indptr && seeds_ptr && (out || out_len == 0) && frontier_ptr && distinct,
              "batch_block_offsets: null pointer");
   hipStream_t s = as_stream(stream);
   const unsigned tiles = (unsigned)ceil_div(out_len, kSplitTile);
@@ -190,7 +192,7 @@ int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int6
             block_offsets_kernel<<<dim3(tiles + (unsigned)ceil_div(num_batches, kBlock)),
                                    dim3(kBlock), 0, s>>>(indptr, seeds_ptr, num_batches, out_len,
                                                          out, tiles, frontier, frontier_ptr, seeds,
-                                                         distinct_mirror));
+                                                         distinct, distinct_mirror));
   return GS_OK;
 }
 

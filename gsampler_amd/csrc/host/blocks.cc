@@ -43,11 +43,11 @@ void BlockBatch::fetch() {
                             cur_stream()));
     return;
   }
-  distinct = new_ids(num_batches, sampled_indptr);  // (in host memory only: the key of its mirror)
+  distinct = new_ids(num_batches, sampled_indptr);
   int64_t* mirror = OffsetMirror::reserve(distinct);
   GS_CALL(gs_batch_block_offsets(cptr(sampled_indptr), cptr(col_bptr), num_batches, total,
                                  mptr(indptr), cptr(frontier), cptr(frontier_ptr), cptr(col_seeds),
-                                 mirror, cur_stream()));
+                                 mptr(distinct), mirror, cur_stream()));
   OffsetMirror::arm(distinct);
   f_off_ = OffsetMirror::values(frontier_ptr);
   e_off_ = OffsetMirror::values(coo_ptr);

@@ -349,12 +349,16 @@ __global__ __launch_bounds__(kBlock) void list_edges_kernel(
   }
 }
 
-// The batch pointer of the frontier for the host: its last entry -1 if refused.
+// The batch pointer of the frontier for the host: its last entry -1 if refused, on the device
+// too (the host copy may be made again from there).
 __global__ __launch_bounds__(kBlock) void batch_list_publish_kernel(
-    const int64_t* __restrict__ unique_ptr, int64_t num_batches, const int* __restrict__ refused,
+    int64_t* __restrict__ unique_ptr, int64_t num_batches, const int* __restrict__ refused,
     int64_t* mirror) {
-  for (int64_t b = threadIdx.x; b <= num_batches; b += kBlock)
-    store_for_host(mirror + b, b == num_batches && *refused ? -1 : unique_ptr[b]);
+  for (int64_t b = threadIdx.x; b <= num_batches; b += kBlock) {
+    const bool none = b == num_batches && *refused;
+    if (none) unique_ptr[b] = -1;
+    store_for_host(mirror + b, none ? -1 : unique_ptr[b]);
+  }
 }
 
 }  // namespace gs

@@ -614,8 +614,8 @@ int gs_list_edge_labels(const int64_t* row, const int64_t* col, const int64_t* i
  *   id_stride > 0: the key of a listed id is its remainder by id_stride
  *   out_frontier[num_seeds + num_ids]  the first unique_ptr[num_batches] are written
  *   unique_ptr[num_batches + 1]        where each batch's frontier begins
- *   unique_ptr_mirror                  the same in pinned host memory; its last entry
- *       is -1, and nothing written is to be used, where an edge's row lies outside
+ *   unique_ptr_mirror                  the same in pinned host memory; the last entry
+ *       of both is -1, and nothing written is to be used, where an edge's row lies outside
  *       its batch's segment or a batch has more than GS_LIST_LABELS_MAX_KEYS keys
  *   scratch[num_seeds + num_ids + num_batches + 1]
  * Rows are positions in the list, columns positions among the seeds; edge_ptr is
@@ -884,10 +884,11 @@ int gs_pick_batch_ids(const int64_t* ids, int64_t num_ids, const int64_t* index,
 int gs_local_ids(const int64_t* table, int64_t num_ids, const int64_t* rows, int64_t n,
                  int64_t stride, int64_t* out, gs_stream_t stream);
 /* gs_split_indptr by seeds_ptr and gs_batch_seeds_distinct in one launch; the flags go to
- * distinct_mirror[num_batches], which may be pinned host memory. */
+ * distinct[num_batches] and, where it is given, to distinct_mirror, which may be pinned host
+ * memory. */
 int gs_batch_block_offsets(const int64_t* indptr, const int64_t* seeds_ptr, int64_t num_batches,
                            int64_t out_len, int64_t* out, const int64_t* frontier,
-                           const int64_t* frontier_ptr, const int64_t* seeds,
+                           const int64_t* frontier_ptr, const int64_t* seeds, int64_t* distinct,
                            int64_t* distinct_mirror, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------

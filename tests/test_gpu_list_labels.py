@@ -121,6 +121,26 @@ def test_list_labels_refuses_what_does_not_fit():
         capi.list_labels(seeds, ids, torch.zeros(n // 2 + 1, dtype=torch.int64, device=DEV))
 
 
+@pytest.mark.parametrize("seeds,picks", [([30, 20], [9, 40]), ([30, 2000], [9, 48]), ([30, 2000], [9, 49])])
+def test_a_refused_batch_is_told_on_the_device_too(seeds, picks):
+    """The last offset of the frontier is -1 in both copies where a batch has too many keys."""
+    rng = np.random.default_rng(sum(picks))
+    S, R = sum(seeds), sum(picks)
+    sp, lp = (T(np.concatenate([[0], np.cumsum(n)])) for n in (seeds, picks))
+    cols, ids, first = T(rng.permutation(5000)[:S]), T(rng.permutation(5000)[:R]), T(np.arange(R))
+    frontier, labels, scratch = (torch.empty(n, dtype=torch.int64, device=DEV)
+                                 for n in (S + R, S + R, S + R + 3))
+    unique_ptr = torch.full((3,), -7, dtype=torch.int64, device=DEV)
+    mirror = torch.full((3,), -7, dtype=torch.int64).pin_memory()
+    P = lambda t: t.data_ptr()
+    capi.check(capi.lib().gs_batch_list_labels(
+        P(cols), P(sp), S, P(ids), P(lp), R, 10**6, 2, None, None, None, 0, P(first), P(frontier),
+        P(unique_ptr), P(mirror), P(labels), P(labels) + 8 * R, None, None, P(scratch), None))
+    torch.cuda.synchronize()
+    assert torch.equal(unique_ptr.cpu(), mirror)
+    assert (mirror[-1] == -1) == (seeds[1] + picks[1] > capi.LIST_LABELS_MAX_KEYS)
+
+
 @pytest.mark.parametrize("sizes,picks,mode", [
     ([40, 1, 0, 60], [100, 30, 0, 200], "distinct"),      # a batch of one column, an empty one
     ([300] * 8, [256] * 8, "repeats"),                    # repeated seeds and repeated picks

@@ -448,15 +448,16 @@ def test_block_offsets_and_flags_in_one_launch(sizes):
     frontier, frontier_ptr = capi.unique_relabel(T(seeds), T(rows), T(ptr), T(np.arange(B + 1)))[:2]
     l, seeds, ptr = capi.lib(), T(seeds), T(ptr)
     out = [torch.full((S + B,), -7, dtype=torch.int64, device=DEV) for _ in range(2)]
-    flags = torch.full((B,), -7, dtype=torch.int64, device=DEV)
+    flags, kept = (torch.full((B,), -7, dtype=torch.int64, device=DEV) for _ in range(2))
     mirror = torch.full((B,), -7, dtype=torch.int64).pin_memory()
     P = lambda t: t.data_ptr()
     capi.check(l.gs_split_indptr(P(indptr), P(ptr), B, S + B, P(out[0]), None))
     capi.check(l.gs_batch_seeds_distinct(P(frontier), P(frontier_ptr), P(seeds), P(ptr), B, P(flags), None))
     capi.check(l.gs_batch_block_offsets(P(indptr), P(ptr), B, S + B, P(out[1]), P(frontier),
-                                        P(frontier_ptr), P(seeds), P(mirror), None))
+                                        P(frontier_ptr), P(seeds), P(kept), P(mirror), None))
     torch.cuda.synchronize()
     assert torch.equal(out[0], out[1]) and torch.equal(flags.cpu(), mirror)
+    assert torch.equal(flags, kept)  # the host copy is not the only one
 
 
 def test_graphsage_layers_end_to_end():
