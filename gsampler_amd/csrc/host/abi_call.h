@@ -232,14 +232,18 @@ class OffsetMirror {
   static void prefetch(const torch::Tensor& offsets) { (void)entry_for(offsets); }
   // For a kernel that stores the array to the host itself: the pinned block it
   // should write to (as many entries as `offsets` has), and arm() once that
-  // kernel is queued.
+  // kernel is queued.  (The block that was reserved, and no other, is waited for:
+  // another thread may have aged the caches in between.)
   static int64_t* reserve(const torch::Tensor& offsets) {
-    return entry_for(offsets, /*copy=*/false).pinned;
+    Entry& e = entry_for(offsets, /*copy=*/false);
+    reserved() = &e;
+    return e.pinned;
   }
   static void arm(const torch::Tensor& offsets) {
-    Entry& e = entry_for(offsets, false);
-    e.stream = (hipStream_t)cur_stream();
-    e.pending = true;
+    Entry* e = reserved();
+    TORCH_CHECK(e && e->tensor.is_same(offsets), "OffsetMirror: nothing was reserved");
+    e->stream = (hipStream_t)cur_stream();
+    e->pending = true;
   }
   static const std::vector<int64_t>& values(const torch::Tensor& offsets) {
     Entry& e = entry_for(offsets);
@@ -267,6 +271,10 @@ class OffsetMirror {
   static constexpr size_t kEntries = 64;
   static void check(hipError_t e) {
     TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+  }
+  static Entry*& reserved() {
+    static thread_local Entry* e = nullptr;
+    return e;
   }
   static Entry& entry_for(const torch::Tensor& offsets, bool copy = true) {
     static thread_local std::vector<Entry> ring(kEntries);

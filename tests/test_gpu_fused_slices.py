@@ -559,6 +559,44 @@ def test_normalised_columns_recorded_behind_a_slice():
         assert torch.allclose(sub._CAPI_NormaliseColumns(w, index, None), want, rtol=1e-6)
 
 
+def test_offsets_for_the_host_while_another_thread_ages_the_caches():
+    """Every load of a matrix ages what is kept of tensors' contents, from any thread, also
+    between the launch of a kernel that reports to the host and the wait for its report:
+    sizes, offsets and the flags of batches with repeated seeds stay what they are."""
+    rng = np.random.default_rng(31)
+    indptr, indices = random_csc(rng, 3000, 3000, 40)
+    g = gs.Graph(3000, 3000)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    seeds, ptr = T(rng.permutation(3000)[:96]), T(np.arange(0, 97, 8))
+    seeds[0::16] = seeds[1::16]
+    repeated = [True, False] * 6
+
+    def step():
+        gs.manual_seed(4)
+        sub, _ = g._CAPI_BatchFusedSlicingSampling(seeds, ptr, 5, False)
+        batch = sub._CAPI_BatchBlocks(seeds, torch.empty(0, dtype=torch.int64, device=DEV))
+        parts = batch.blocks()
+        assert [o is None for o in parts[2]] == repeated
+        cut, index = g._CAPI_BatchColSlicing(seeds, ptr, True)
+        return [*batch.offsets(), batch.row().tolist(), batch.frontier().tolist(),
+                cut._CAPI_BatchGetRows()[1].tolist(), index.numel()]
+
+    want, stop = step(), threading.Event()
+
+    def age():
+        while not stop.is_set():
+            torch.ops.gs_ops._CAPI_InvalidateCaches()
+
+    other = threading.Thread(target=age)
+    other.start()
+    try:
+        for _ in range(100):
+            assert step() == want
+    finally:
+        stop.set()
+        other.join()
+
+
 def columns_of(lengths, rng, num_rows):
     indptr = np.concatenate([[0], np.cumsum(lengths)])
     return indptr, rng.integers(0, num_rows, size=int(indptr[-1])).astype(np.int64)
