@@ -67,8 +67,8 @@ SIGNATURES = {
     "gs_decode_batch_ids": (_int, [_p, _i64, _i64, _p, _p, _p]),
     "gs_encode_batch_ids": (_int, [_p, _p, _i64, _i64, _i64, _p, _p]),
     "gs_split_indptr": (_int, [_p, _p, _i64, _i64, _p, _p]),
-    "gs_pick_batch_ids": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _p]),
-    "gs_local_ids": (_int, [_p, _i64, _p, _i64, _i64, _p, _p]),
+    "gs_pick_batch_ids": (_int, [_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _p, _p]),
+    "gs_local_ids": (_int, [_p, _i64, _p, _i64, _i64, _p, _p, _p]),
     "gs_batch_block_offsets": (_int, [_p, _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "gs_batch_seeds_distinct": (_int, [_p, _p, _p, _p, _i64, _p, _p]),
     "gs_unique_count_distinct": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _sz,

@@ -30,18 +30,21 @@ __global__ __launch_bounds__(kBlock) void encode_batch_ids_kernel(
 
 // The same for ids picked from a list: id = ids[index[i]] (without index: ids[i]), which goes
 // out as it is, moved by its batch, and the move alone, whatever of the three is wanted: one
-// launch where a gather and up to two of the above were.  A place outside the list reads no id.
+// launch where a gather and up to two of the above were.  A place outside the list reads no id
+// and raises `refused`.
 __global__ __launch_bounds__(kBlock) void pick_batch_ids_kernel(
     const int64_t* __restrict__ ids, int64_t num_ids, const int64_t* __restrict__ index,
     const int64_t* __restrict__ batch_ptr, int64_t num_batches, int64_t n, int64_t stride,
     int64_t* __restrict__ out_id, int64_t* __restrict__ out_moved,
-    int64_t* __restrict__ out_offset) {
+    int64_t* __restrict__ out_offset, int64_t* refused) {
   const int64_t first = (int64_t)blockIdx.x * kBlock, i = first + threadIdx.x;
   const int64_t last = first + kBlock < n ? first + kBlock - 1 : n - 1;
   const int64_t at = i < n ? (index ? index[i] : i) : 0;
-  const int64_t id = (uint64_t)at < (uint64_t)num_ids ? ids[at] : 0;
+  const bool listed = (uint64_t)at < (uint64_t)num_ids;
+  const int64_t id = listed ? ids[at] : 0;
   const SegmentSpan span = segment_span(batch_ptr, num_batches, first, last);
   if (i >= n) return;
+  if (!listed && refused) store_for_host(refused, 1);
   const int64_t offset = span.segment_at(batch_ptr, i) * stride;
   if (out_id) out_id[i] = id;
   if (out_moved) out_moved[i] = id + offset;
@@ -50,17 +53,24 @@ __global__ __launch_bounds__(kBlock) void pick_batch_ids_kernel(
 
 // out[e] = the id behind local row rows[e], its remainder by stride where that is not 0 (ids
 // encoded as id + batch * stride): a gather, the quotients, and the batch pointer that came
-// with those and that nobody read were three launches.
+// with those and that nobody read were three launches.  A row outside the list reads its
+// first id and raises `refused`.
 __global__ __launch_bounds__(kBlock) void local_ids_kernel(
     const int64_t* __restrict__ table, int64_t num_ids, const int64_t* __restrict__ rows,
-    int64_t n, int64_t stride, int64_t* __restrict__ out) {
+    int64_t n, int64_t stride, int64_t* __restrict__ out, int64_t* refused) {
   constexpr int kItems = 4;
   const int64_t e0 = (int64_t)blockIdx.x * (kBlock * kItems) + threadIdx.x;
   int64_t v[kItems];
+  bool outside = false;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) v[j] = rows[e0 + j * kBlock < n ? e0 + j * kBlock : n - 1];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) v[j] = table[(uint64_t)v[j] < (uint64_t)num_ids ? v[j] : 0];
+  for (int j = 0; j < kItems; ++j) {
+    const bool listed = (uint64_t)v[j] < (uint64_t)num_ids;
+    outside |= !listed;
+    v[j] = table[listed ? v[j] : 0];
+  }
+  if (outside && refused) store_for_host(refused, 1);
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     if (stride > 0 && (uint64_t)v[j] >= (uint64_t)stride) v[j] %= stride;
@@ -229,7 +239,7 @@ int gs_encode_batch_ids(const int64_t* ids, const int64_t* batch_ptr, int64_t nu
 int gs_pick_batch_ids(const int64_t* ids, int64_t num_ids, const int64_t* index,
                       const int64_t* batch_ptr, int64_t num_batches, int64_t n, int64_t stride,
                       int64_t* out_id, int64_t* out_moved, int64_t* out_offset,
-                      gs_stream_t stream) {
+                      int64_t* refused, gs_stream_t stream) {
   using namespace gs;
   GS_REQUIRE(n >= 0 && num_ids >= 0 && num_batches >= 0, "pick_batch_ids: negative size");
   if (n == 0) return GS_OK;
@@ -238,12 +248,12 @@ int gs_pick_batch_ids(const int64_t* ids, int64_t num_ids, const int64_t* index,
   GS_LAUNCH("pick_batch_ids", s,
             pick_batch_ids_kernel<<<dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, s>>>(
                 ids, num_ids, index, batch_ptr, num_batches, n, stride, out_id, out_moved,
-                out_offset));
+                out_offset, refused));
   return GS_OK;
 }
 
 int gs_local_ids(const int64_t* table, int64_t num_ids, const int64_t* rows, int64_t n,
-                 int64_t stride, int64_t* out, gs_stream_t stream) {
+                 int64_t stride, int64_t* out, int64_t* refused, gs_stream_t stream) {
   using namespace gs;
   GS_REQUIRE(n >= 0 && num_ids >= 0 && stride >= 0, "local_ids: negative size");
   if (n == 0) return GS_OK;
@@ -251,7 +261,7 @@ int gs_local_ids(const int64_t* table, int64_t num_ids, const int64_t* rows, int
   hipStream_t s = as_stream(stream);
   GS_LAUNCH("local_ids", s,
             local_ids_kernel<<<dim3((unsigned)ceil_div(n, kBlock * 4)), dim3(kBlock), 0, s>>>(
-                table, num_ids, rows, n, stride, out));
+                table, num_ids, rows, n, stride, out, refused));
   return GS_OK;
 }
 

@@ -213,6 +213,51 @@ class AsyncCount {
   int64_t value_ = 0;
 };
 
+// A word of pinned host memory that kernels on their way may raise: whether one of them did is
+// there once anything queued behind them has been waited for.  For what an operator that
+// waits for a count anyway has to refuse.
+class HostFlag {
+ public:
+  HostFlag() {
+    Ring& r = ring();
+    slot_ = (int)(r.next++ % kSlots);
+    if (r.lowered[slot_]) {
+      // an operator left by an exception: its kernels must not store later
+      const hipError_t e = hipStreamSynchronize(r.stream[slot_]);
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+    }
+    r.words[slot_] = 0;
+    r.stream[slot_] = (hipStream_t)cur_stream();
+    r.lowered[slot_] = true;
+  }
+  int64_t* word() const { return ring().words + slot_; }
+  bool raised() const {
+    Ring& r = ring();
+    r.lowered[slot_] = false;
+    return __atomic_load_n(r.words + slot_, __ATOMIC_ACQUIRE) != 0;
+  }
+
+ private:
+  static constexpr int kSlots = 16;
+  struct Ring {
+    int64_t* words = nullptr;
+    hipStream_t stream[kSlots] = {};
+    bool lowered[kSlots] = {};
+    unsigned next = 0;
+  };
+  static Ring& ring() {
+    static thread_local Ring* r = [] {
+      Ring* x = new Ring();
+      const hipError_t e =
+          hipHostMalloc((void**)&x->words, kSlots * sizeof(int64_t), hipHostMallocDefault);
+      TORCH_CHECK(e == hipSuccess, "HIP error: ", hipGetErrorString(e));
+      return x;
+    }();
+    return *r;
+  }
+  int slot_;
+};
+
 // Last element of a device prefix array.
 inline int64_t read_last(const torch::Tensor& prefix) {
   if (!prefix.is_cuda()) return prefix[prefix.numel() - 1].item<int64_t>();

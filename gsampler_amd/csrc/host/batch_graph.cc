@@ -220,27 +220,38 @@ Graph::ColumnOrderedEdges Graph::column_ordered_edges(const char* who) {
 }
 
 // Global row ids of every edge as the relabel pass needs them: rows of an
-// encoded (compacted) batch graph are decoded back through row_ids.
+// encoded (compacted) batch graph are decoded back through row_ids.  Rows that the list does
+// not have (written by the caller, or a list that is too short) are refused by frontier_of().
 torch::Tensor Graph::batch_rows_for_relabel(const torch::Tensor& edge_rows,
                                             const torch::Tensor& row_ids) {
   if (row_ids.numel() == 0) return edge_rows;
   if (!(mapped_out_.defined() && mapped_from_.is_same(edge_rows) &&
         mapped_by_.is_same(row_ids))) {
     torch::Tensor table = ids(row_ids, "row_ids");
-    if (table.numel() >= num_rows_) {  // (the edges' rows lie below num_rows)
-      mapped_out_ = new_ids(edge_rows.numel(), edge_rows);
-      GS_CALL(gs_local_ids(cptr(table), table.numel(), cptr(edge_rows), edge_rows.numel(),
-                           row_encoding_size_, mptr(mapped_out_), cur_stream()));
-    } else {
-      mapped_out_ = table.index_select(0, edge_rows);
-      if (row_encoding_size_ > 0)
-        mapped_out_ = std::get<1>(
-            batch_offsets(mapped_out_, edge_bptr_.numel() - 1, row_encoding_size_));
-    }
+    mapped_refused_.emplace();
+    mapped_out_ = new_ids(edge_rows.numel(), edge_rows);
+    GS_CALL(gs_local_ids(cptr(table), table.numel(), cptr(edge_rows), edge_rows.numel(),
+                         row_encoding_size_, mptr(mapped_out_), mapped_refused_->word(),
+                         cur_stream()));
     mapped_from_ = edge_rows;
     mapped_by_ = row_ids;
   }
   return mapped_out_;
+}
+
+// The frontier, once it has arrived; behind it the kernel that mapped the rows has, too.
+const torch::Tensor& Graph::frontier_of(Frontier& f, const char* who) {
+  const torch::Tensor& frontier = f.frontier();
+  if (!mapped_refused_.has_value()) return frontier;
+  const bool refused = mapped_refused_->raised();
+  mapped_refused_.reset();
+  if (refused) {
+    const int64_t listed = mapped_by_.numel();
+    mapped_out_ = mapped_from_ = mapped_by_ = torch::Tensor();
+    frontier_.reset();
+    TORCH_CHECK(false, who, ": the row of an edge lies outside the ", listed, " row ids given");
+  }
+  return frontier;
 }
 
 // A pass over the edges finds the first edge of every listed id: in LDS for a few
@@ -414,7 +425,7 @@ Graph::BatchGraphRelabel(torch::Tensor col_seeds, torch::Tensor row_ids) {
   torch::Tensor out_row, out_col;
   c10::optional<torch::Tensor> e_ids;
   Frontier& f = batch_relabel_launch(col_seeds, row_ids, &out_row, &out_col, &e_ids);
-  return {f.frontier(), f.unique_ptr, out_row, out_col, e_ids, edge_bptr_};
+  return {frontier_of(f, "BatchGraphRelabel"), f.unique_ptr, out_row, out_col, e_ids, edge_bptr_};
 }
 
 std::tuple<torch::Tensor, torch::Tensor> Graph::BatchGetValidNodes(
@@ -432,7 +443,7 @@ std::tuple<torch::Tensor, torch::Tensor> Graph::BatchGetValidNodes(
   }
   torch::Tensor rows = batch_rows_for_relabel(edges.row, row_ids);
   Frontier& f = frontier_for(col_seeds, rows, col_bptr_, edge_bptr_);
-  return {f.frontier(), f.unique_ptr};
+  return {frontier_of(f, "BatchGetValidNodes"), f.unique_ptr};
 }
 
 // ------------------------------------------------------------ free operators

@@ -141,7 +141,7 @@ c10::intrusive_ptr<BlockBatch> Graph::BatchBlocks(torch::Tensor col_seeds,
   // (the pointer arrays are on their way to the host or there already: the
   // sampler sent the edge pointer, the unique pass the frontier pointer, and the
   // column pointer is the caller's or the previous layer's frontier pointer)
-  out->frontier = f.frontier();  // waits for the number of unique ids
+  out->frontier = frontier_of(f, "BatchBlocks");  // waits for the number of unique ids
   return out;
 }
 

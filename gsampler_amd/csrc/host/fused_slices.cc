@@ -393,7 +393,7 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
     picked = new_ids(row.numel(), row_bptr);
     GS_CALL(gs_pick_batch_ids(cptr(row), row.numel(), nullptr, cptr(row_bptr), row_bptr.numel() - 1,
                               row.numel(), stride, nullptr, mptr(picked), mptr(key_offset),
-                              cur_stream()));
+                              nullptr, cur_stream()));
   } else {
     key_offset = encoded_ids(torch::Tensor(), col_bptr, col.numel(), stride);
     picked = encoded_ids(row, row_bptr, row.numel(), stride);
@@ -510,6 +510,12 @@ static void check_encoded(torch::Tensor& seeds, torch::Tensor& col_bptr, torch::
   BatchOffsets::check(row_bptr, row_ids.numel(), "BatchRowSlicing");
 }
 
+// Behind a wait for something queued after the picks' ids.
+static void check_picks(const HostFlag& refused, const torch::Tensor& rows) {
+  TORCH_CHECK(!refused.raised(), "BatchRowSlicing: a picked row lies outside the ", rows.numel(),
+              " rows of the slice");
+}
+
 GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
                                        torch::Tensor rows, torch::Tensor row_ids,
                                        torch::Tensor row_bptr) {
@@ -526,10 +532,12 @@ std::tuple<GraphPtr, torch::Tensor, torch::Tensor> Graph::EncodedPickedRows(
   rows = ids(rows, "rows");
   const int64_t n = row_ids.numel();
   torch::Tensor picked = new_ids(n, row_ids), names = new_ids(n, row_ids);
+  HostFlag refused;
   GS_CALL(gs_pick_batch_ids(cptr(rows), rows.numel(), cptr(row_ids), cptr(row_bptr),
                             row_bptr.numel() - 1, n, num_rows_, mptr(names), mptr(picked), nullptr,
-                            cur_stream()));
-  auto got = encoded_row_slice(seeds, col_bptr, picked, row_ids, row_bptr);
+                            refused.word(), cur_stream()));
+  auto got = encoded_row_slice(seeds, col_bptr, picked, row_ids, row_bptr);  // (waits for a count)
+  check_picks(refused, rows);
   return {std::get<0>(got), std::get<1>(got), names};
 }
 
@@ -567,8 +575,9 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   if (nnz < 8 * (R + S) || nnz > kBoundLimit || !gs_col_row_slice_tells_first(nnz, R)) return {};
   torch::Tensor key_offset = key_offsets_for(*so, col_bptr);
   torch::Tensor picked = new_ids(R, row_ids), names = new_ids(R, row_ids);
+  HostFlag refused;
   GS_CALL(gs_pick_batch_ids(cptr(rows), rows.numel(), cptr(row_ids), cptr(row_bptr), B, R, num_rows_,
-                            mptr(names), mptr(picked), nullptr, cur_stream()));
+                            mptr(names), mptr(picked), nullptr, refused.word(), cur_stream()));
   const torch::Tensor narrow = narrow_for_slice(m, nnz, S);
   torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, R), m.indptr);
   torch::Tensor indptr = new_ids(S + 1, m.indptr), unique_ptr = new_ids(B + 1, m.indptr);
@@ -595,6 +604,7 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   HandedOn edges;
   edges.queue(m, seeds, so->sub_indptr, nnz, R, row_label, col_label, values, row_divisor, ws);
   const int64_t k = kept.get();
+  check_picks(refused, rows);
   edges.finish(k, indptr, sums);
   c10::intrusive_ptr<BlockBatch> out = blocks_of(edges, indptr, col_bptr, seeds);
   const int64_t total = OffsetMirror::values(unique_ptr).back();
@@ -616,7 +626,7 @@ c10::optional<c10::intrusive_ptr<BlockBatch>> Graph::SubgraphBlocks(torch::Tenso
   slice_offsets_for(nodes, false);
   torch::Tensor picked = new_ids(n, nodes), key_offset = new_ids(n, nodes);
   GS_CALL(gs_pick_batch_ids(cptr(nodes), n, nullptr, cptr(nodes_ptr), B, n, num_rows_, nullptr,
-                            mptr(picked), mptr(key_offset), cur_stream()));
+                            mptr(picked), mptr(key_offset), nullptr, cur_stream()));
   const std::shared_ptr<SliceOffsets> so = slice_offsets_for(nodes);
   const int64_t nnz = so->nnz;
   if (nnz < n || nnz > kBoundLimit) return {};

@@ -448,6 +448,7 @@ class Graph : public torch::CustomClassHolder {
   Frontier& frontier_for(const torch::Tensor& seeds, const torch::Tensor& rows,
                          const torch::Tensor& seeds_ptr,
                          const torch::Tensor& rows_ptr, LabelRequest* labels = nullptr);
+  const torch::Tensor& frontier_of(Frontier& f, const char* who);
   Frontier& batch_relabel_launch(torch::Tensor& col_seeds, const torch::Tensor& row_ids,
                                  torch::Tensor* out_row, torch::Tensor* out_col,
                                  c10::optional<torch::Tensor>* e_ids);
@@ -520,6 +521,7 @@ class Graph : public torch::CustomClassHolder {
   int64_t row_encoding_size_ = 0;
   std::unique_ptr<Frontier> frontier_;
   torch::Tensor mapped_out_, mapped_from_, mapped_by_;
+  c10::optional<HostFlag> mapped_refused_;  // while nobody has waited for what mapped them
   // Relabel of a matrix whose rows are positions in a short list of ids
   // (row slicing leaves it that way): label of every list entry and of every
   // seed, computed from the list instead of from every edge.

@@ -876,13 +876,15 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
  * out_id[i] = id, out_moved[i] = id + b * stride and out_offset[i] = b * stride, each
  * nullable.  A place outside [0, num_ids) counts as id 0.
  * gs_local_ids: out[e] = table[rows[e]], its remainder by stride where stride > 0; a row
- * outside [0, num_ids) reads table[0]. */
+ * outside [0, num_ids) reads table[0].
+ * refused (nullable, may be pinned host memory): set to 1 where there is such a place or row,
+ * else left alone. */
 int gs_pick_batch_ids(const int64_t* ids, int64_t num_ids, const int64_t* index,
                       const int64_t* batch_ptr, int64_t num_batches, int64_t n, int64_t stride,
                       int64_t* out_id, int64_t* out_moved, int64_t* out_offset,
-                      gs_stream_t stream);
+                      int64_t* refused, gs_stream_t stream);
 int gs_local_ids(const int64_t* table, int64_t num_ids, const int64_t* rows, int64_t n,
-                 int64_t stride, int64_t* out, gs_stream_t stream);
+                 int64_t stride, int64_t* out, int64_t* refused, gs_stream_t stream);
 /* gs_split_indptr by seeds_ptr and gs_batch_seeds_distinct in one launch; the flags go to
  * distinct[num_batches] and, where it is given, to distinct_mirror, which may be pinned host
  * memory. */

@@ -410,7 +410,7 @@ def test_batch_ids_picked_from_a_list(n):
             capi.check(l.gs_pick_batch_ids(
                 source.data_ptr(), source.numel(), at.data_ptr() if at is not None else None,
                 T(ptr).data_ptr(), 301, n, 10**10,
-                *(outs[i].data_ptr() if i in wanted else None for i in range(3)), None))
+                *(outs[i].data_ptr() if i in wanted else None for i in range(3)), None, None))
             torch.cuda.synchronize()
             for i, want in enumerate((name, name + batch * 10**10, batch * 10**10)):
                 assert torch.equal(outs[i], want if i in wanted else torch.full_like(want, -7))
@@ -419,9 +419,70 @@ def test_batch_ids_picked_from_a_list(n):
     rows, out = T(rng.integers(0, n, size=3 * n + 1)), torch.empty(3 * n + 1, dtype=torch.int64, device=DEV)
     for stride, want in ((0, moved[rows]), (10**10, name[rows])):
         capi.check(l.gs_local_ids(moved.data_ptr(), n, rows.data_ptr(), rows.numel(), stride,
-                                  out.data_ptr(), None))
+                                  out.data_ptr(), None, None))
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("outside", [-1, 700, 2**40, -2**63])
+@pytest.mark.parametrize("n", [1, 1024, 1025, 5000])
+def test_places_outside_a_list_are_told(n, outside):
+    rng = np.random.default_rng(n)
+    ids, ptr = T(rng.integers(0, 10**9, size=700)), T([0, n])
+    out = torch.empty(n, dtype=torch.int64, device=DEV)
+    l, flag = capi.lib(), torch.empty(1, dtype=torch.int64, device=DEV)
+    for at in (None, 0, n - 1):
+        index = T(rng.integers(0, 700, size=n))
+        if at is not None:
+            index[at] = outside
+        for call in (lambda: l.gs_pick_batch_ids(ids.data_ptr(), 700, index.data_ptr(), ptr.data_ptr(), 1, n,
+                                                 10, out.data_ptr(), None, None, flag.data_ptr(), None),
+                     lambda: l.gs_local_ids(ids.data_ptr(), 700, index.data_ptr(), n, 0, out.data_ptr(),
+                                            flag.data_ptr(), None)):
+            flag.zero_()
+            capi.check(call())
+            torch.cuda.synchronize()
+            assert flag.item() == (at is not None)
+            keep = torch.arange(n, device=DEV) != (-1 if at is None else at)
+            assert torch.equal(out[keep], ids[index[keep]])
+
+
+def test_rows_and_picks_that_a_list_does_not_have_are_refused():
+    """Picks outside the rows of an encoded slice, edges whose rows the caller wrote outside
+    the list, lists that are too short; the calls that follow are served."""
+    rng = np.random.default_rng(17)
+    indptr, indices = columns_of(rng.integers(1, 90, 400), rng, 400)
+    g = gs.Graph(400, 400)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.ones(indices.size, device=DEV)
+    seeds, ptr = batches_of(rng, 400, [20, 30])
+    rows, rows_ptr, _ = g._CAPI_EncodedSquareSums(seeds, ptr, w)
+    good, good_ptr = T([1, 5, int(rows_ptr[1]) + 2]), T([0, 2, 3])
+    for wrong in (-1, rows.numel(), 2**40):
+        bad = good.clone()
+        bad[1] = wrong
+        for call in (g._CAPI_EncodedPickedRows, lambda *a: g._CAPI_EncodedBlocks(*a, None, None)):
+            with pytest.raises(RuntimeError, match="picked row lies outside"):
+                call(seeds, ptr, rows, bad, good_ptr)
+    assert g._CAPI_EncodedBlocks(seeds, ptr, rows, good, good_ptr, None, None) is not None
+    sub, _, names = g._CAPI_EncodedPickedRows(seeds, ptr, rows, good, good_ptr)
+    assert torch.equal(names, rows[good])
+
+    cut, _ = g._CAPI_BatchColSlicing(seeds, ptr, True)
+    ids, _ = cut._CAPI_BatchGetRows()
+    want = cut._CAPI_BatchGraphRelabel(seeds, ids)
+    edge_rows = cut._CAPI_GetCOORows()
+    kept = edge_rows[3].item()
+    for wrong in (-1, ids.numel(), 2**40):
+        edge_rows[3] = wrong
+        for call in (cut._CAPI_BatchGraphRelabel, cut._CAPI_BatchGetValidNodes, cut._CAPI_BatchBlocks):
+            with pytest.raises(RuntimeError, match="row of an edge lies outside"):
+                call(seeds, ids.clone())
+    edge_rows[3] = kept
+    with pytest.raises(RuntimeError, match="row of an edge lies outside"):
+        cut._CAPI_BatchGraphRelabel(seeds, ids[:-1].contiguous())  # (every row has an edge)
+    for a, b in zip(cut._CAPI_BatchGraphRelabel(seeds, ids.clone()), want):
+        assert a is b is None or torch.equal(a, b)
 
 
 @pytest.mark.parametrize("order", ["blocks", "nodes first", "edge list first", "rows written"])
