@@ -267,9 +267,9 @@ constexpr int kEdgeLabelTile = kBlock * kEdgeLabelItems;
 __global__ __launch_bounds__(kBlock) void batch_list_edges_kernel(
     const int64_t* __restrict__ row, const int64_t* __restrict__ col, int64_t nnz,
     const int64_t* __restrict__ edge_ptr, const int64_t* __restrict__ list_ptr,
-    int64_t num_batches, const int64_t* __restrict__ list_label,
-    const int64_t* __restrict__ seed_label, int64_t* __restrict__ out_row,
-    int64_t* __restrict__ out_col, int* __restrict__ refused) {
+    int64_t num_batches, int64_t num_ids, int64_t num_seeds,
+    const int64_t* __restrict__ list_label, const int64_t* __restrict__ seed_label,
+    int64_t* __restrict__ out_row, int64_t* __restrict__ out_col, int* __restrict__ refused) {
   const int64_t e0 = (int64_t)blockIdx.x * kEdgeLabelTile;
   const int64_t last = e0 + kEdgeLabelTile <= nnz ? e0 + kEdgeLabelTile - 1 : nnz - 1;
   const SegmentSpan span = segment_span(edge_ptr, num_batches, e0, last);
@@ -292,8 +292,11 @@ __global__ __launch_bounds__(kBlock) void batch_list_edges_kernel(
       const int64_t b = span.segment_at(edge_ptr, e);
       outside |= r[j] < list_ptr[b] || r[j] >= list_ptr[b + 1];
     }
-    out_row[e] = list_label[r[j]];
-    out_col[e] = seed_label[c[j]];
+    // (rows and columns may be the caller's: none is read past the lists)
+    const bool row_in = (uint64_t)r[j] < (uint64_t)num_ids, col_in = (uint64_t)c[j] < (uint64_t)num_seeds;
+    outside |= !row_in || !col_in;
+    out_row[e] = list_label[row_in ? r[j] : 0];
+    out_col[e] = seed_label[col_in ? c[j] : 0];
   }
   if (__any(outside) && lane_id() == 0) *refused = 1;
 }
@@ -448,8 +451,8 @@ extern "C" int gs_batch_list_labels(
     GS_LAUNCH("list_edges", s,
               batch_list_edges_kernel<<<dim3((unsigned)ceil_div(nnz, kEdgeLabelTile)),
                                         dim3(kBlock), 0, s>>>(
-                  row, col, nnz, edge_ptr, list_ptr, num_batches, out_list_label, out_seed_label,
-                  out_row, out_col, refused));
+                  row, col, nnz, edge_ptr, list_ptr, num_batches, num_ids, num_seeds,
+                  out_list_label, out_seed_label, out_row, out_col, refused));
   GS_LAUNCH("list_publish", s,
             batch_list_publish_kernel<<<dim3(1), dim3(kBlock), 0, s>>>(unique_ptr, num_batches,
                                                                        refused, unique_ptr_mirror));

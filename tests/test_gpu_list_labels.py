@@ -194,6 +194,31 @@ def test_batched_labels_by_way_of_the_list(sizes, picks, mode):
                 assert np.array_equal(col[e], want[3])
 
 
+def test_batched_labels_of_rows_that_the_caller_wrote():
+    """A row in another batch's segment goes by the general path; one outside the list is read
+    by nobody and refused."""
+    rng = np.random.default_rng(9)
+    indptr, indices = random_csc(rng, 2500, 1500, 3000)
+    g = gs.Graph(1500, 2500)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    seeds, ptr = T(rng.permutation(2500)[:60]), T([0, 40, 60])
+    sub, _ = g._CAPI_BatchColSlicing(seeds, ptr, True)
+    ids, row_ptr = sub._CAPI_BatchGetRows()
+    picked, picked_ptr = T(np.concatenate([np.arange(90), int(row_ptr[1]) + np.arange(50)])), T([0, 90, 140])
+    part, _ = sub._CAPI_BatchRowSlicing(picked, picked_ptr)
+    assert part._CAPI_GetNumEdges() >= 8 * 200
+    edge_rows = part._CAPI_GetCOORows()
+    for wrong in (-1, -2**62, 140, 2**40):
+        kept = edge_rows[7].item()
+        edge_rows[7] = wrong
+        with pytest.raises(RuntimeError, match="row of an edge lies outside"):
+            part._CAPI_BatchGraphRelabel(seeds, ids[picked])
+        edge_rows[7] = 139  # of the other batch
+        frontier, uptr, row, _, _, _ = part._CAPI_BatchGraphRelabel(seeds, ids[picked])
+        assert frontier[row[7]] == ids[picked][139] and row[7] < uptr[1]
+        edge_rows[7] = kept
+
+
 @pytest.mark.parametrize("sizes,picks", [
     ([64] * 8, [512] * 8),             # 4096 listed ids, the most that the list pass holds in LDS
     ([20] * 17, [241] * 17),           # 4097, few edges: by way of the list all the same
