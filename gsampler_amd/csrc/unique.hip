@@ -1129,10 +1129,16 @@ constexpr uint32_t kFewListed = 2048;  // keys of a bin that are found again wit
 // first[position] of a call that went this way carries a mark where the position is itself
 // a first occurrence.  (Positions are below 2^31 - 1.)
 constexpr uint32_t kFirstMark = 0x80000000u;
-// Bin of a key: a hash of 32 bits, for every work-group hashes every key of its batch.
+constexpr uint32_t kFewOpen = 0xFFFFFFFFu;  // no position, marked or not
+// Bin of a key: a hash of 32 bits, for every work-group hashes every key of its batch.  A
+// multiplication alone puts ids in steps of some sizes into one bin (by 2^32 over the golden
+// ratio 4096 ids, each 10 946 after the one before: all of them, and 1.1 ms instead of 11 us).
+// With a shift in front of it 2 to 96 bins of 512 keys on average get at most 661 for any of
+// 6000 steps, powers of two and Fibonacci numbers among them, and for runs of ids in steps; a
+// second multiplication spreads no better and takes 1 of 22 us on 48 K keys.
 __device__ __forceinline__ uint32_t few_bin(uint64_t key, uint32_t bins) {
   const uint32_t x = (uint32_t)key + (uint32_t)(key >> 32) * 33u;
-  return __umulhi(x * 0x9E3779B1u, bins);
+  return __umulhi((x ^ (x >> 8)) * 0x846CA68Bu, bins);
 }
 
 __global__ __launch_bounds__(kFewThreads) void unique_few_kernel(
@@ -1263,12 +1269,37 @@ __global__ __launch_bounds__(kFewThreads) void unique_few_kernel(
   }
   __syncthreads();
   if (overflow) {
-    // keys made to meet in one bin: every one looks for itself among those before it
-    each_key([&](uint64_t key, uint32_t p) {
-      uint32_t q = 0;
-      while (key_of(q) != key) ++q;
-      store(p, q);
-    });
+    // Keys made to meet in one bin: rounds, each with as many of those that are left as the
+    // table takes (a thread has the same positions in all of them).  N keys take N / 1536
+    // rounds over the batch at most; 48 K distinct ids in one bin 12 ms.
+    each_key([&](uint64_t, uint32_t p) { first_b[p] = kFewOpen; });
+    auto each_open = [&](auto&& f) {
+      each_key([&](uint64_t key, uint32_t p) {
+        if (first_b[p] == kFewOpen) f(key, p);
+      });
+    };
+    do {
+      __syncthreads();  // (`overflow` and the slots have been read)
+      for (uint32_t i = t; i <= kFewSlots; i += kFewThreads) {
+        if (i < kFewSlots) keys[i] = kEmptySlot;
+        mins[i] = 0xFFFFFFFFu;
+      }
+      if (t == 0) claimed = overflow = 0;
+      __syncthreads();
+      each_open([&](uint64_t key, uint32_t) { slot_of(key, true); });
+      __syncthreads();
+      each_open([&](uint64_t key, uint32_t p) {
+        const uint32_t s = slot_of(key, false);
+        if (s <= kFewSlots && mins[s] > p) atomicMin(&mins[s], p);
+      });
+      __syncthreads();
+      each_open([&](uint64_t key, uint32_t p) {
+        const uint32_t s = slot_of(key, false);
+        if (s <= kFewSlots) store(p, mins[s]);
+        else overflow = 1;  // every writer stores the same value
+      });
+      __syncthreads();
+    } while (overflow);
   } else if (all_listed) {
 #pragma unroll
     for (int j = 0; j < kMine; ++j) {

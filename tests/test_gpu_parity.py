@@ -206,7 +206,37 @@ def test_unique_relabel_with_many_batches_in_a_group_of_positions(B, most):
 
 def _bin_of(ids, bins):
     """Bin of an id below 2^32 among those that a call of few keys is cut into."""
-    return ((ids * 0x9E3779B1 & 0xFFFFFFFF) * bins) >> 32
+    x = np.asarray(ids, dtype=np.uint64)
+    x = (x ^ (x >> np.uint64(8))) * np.uint64(0x846CA68B) & np.uint64(0xFFFFFFFF)
+    return ((x * np.uint64(bins)) >> np.uint64(32)).astype(np.int64)
+
+
+@pytest.mark.parametrize("n", [4096, 8192, 49_152])
+@pytest.mark.parametrize("step", [1, 8, 4096, 6765, 10_946, 17_711, 28_657, 65_537])
+def test_unique_of_few_ids_in_equal_steps(n, step):
+    """Ids a Fibonacci number or a power of two apart do not meet in one bin."""
+    ids = np.arange(n, dtype=np.int64) * step
+    assert np.bincount(_bin_of(ids, n // 512)).max() < 700      # of 512 on average
+    ids = np.random.default_rng(step).permutation(ids)
+    assert_same(capi.unique_relabel(T(ids[:n // 4]), T(ids[n // 8:]))[:3],
+                orc.unique_relabel(ids[:n // 4], ids[n // 8:])[:3])
+
+
+@pytest.mark.parametrize("n", [1537, 2048, 2049, 3100, 20_000, 49_152])
+def test_unique_of_few_ids_that_meet_in_one_bin(n):
+    """A bin with more distinct ids than its table takes at once, up to all of a call, half of
+    them repeated, with the one that marks empty slots among the others."""
+    bins = -(-n // 512)
+    pool = np.arange(n * bins * 2, dtype=np.int64)
+    pool = pool[_bin_of(pool, bins) == bins - 1]
+    rng = np.random.default_rng(n)
+    for keys in (rng.permutation(pool)[:n], rng.choice(pool[:n // 2], size=n)):
+        keys = keys[:n]
+        keys[len(keys) // 2] = -1
+        S = n // 3
+        edge_col = rng.integers(0, S, size=len(keys) - S)
+        assert_same(capi.unique_relabel(T(keys[:S]), T(keys[S:]), edge_col=T(edge_col)),
+                    orc.unique_relabel(keys[:S], keys[S:], edge_col=edge_col))
 
 
 @pytest.mark.parametrize("kind", ["mixed", "distinct", "one bin", "hub", "any int64"])
@@ -221,7 +251,7 @@ def test_unique_relabel_of_few_keys(n, kind):
     if kind == "distinct":
         keys = rng.permutation(4 * n)[:n]
     elif kind == "one bin":
-        few = min(n, 4097)  # (each then looks through those before it)
+        few = min(n, 4097)
         of = -(-n // 512)
         pool = np.arange(few * of * 2, dtype=np.int64)
         pool = pool[_bin_of(pool, of) == 0][:few]
