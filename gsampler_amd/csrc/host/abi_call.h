@@ -290,6 +290,10 @@ class OffsetMirror {
     e->stream = (hipStream_t)cur_stream();
     e->pending = true;
   }
+  // For an array that a kernel on its way writes, with values that the host knows already.
+  static void known(const torch::Tensor& offsets, std::vector<int64_t> values) {
+    fresh_entry(offsets).host = std::move(values);
+  }
   static const std::vector<int64_t>& values(const torch::Tensor& offsets) {
     Entry& e = entry_for(offsets);
     if (e.pending) {
@@ -321,22 +325,29 @@ class OffsetMirror {
     static thread_local Entry* e = nullptr;
     return e;
   }
-  static Entry& entry_for(const torch::Tensor& offsets, bool copy = true) {
-    static thread_local std::vector<Entry> ring(kEntries);
+  static std::vector<Entry>& ring() {
+    static thread_local std::vector<Entry> r(kEntries);
+    return r;
+  }
+  static Entry& fresh_entry(const torch::Tensor& offsets) {
     static thread_local size_t next = 0;
-    TORCH_CHECK(offsets.defined() && offsets.scalar_type() == torch::kInt64,
-                "batch offsets must be an int64 tensor");
-    for (Entry& e : ring)
-      if (e.tensor.defined() && e.tensor.is_same(offsets) &&
-          e.version == (int64_t)offsets._version() && e.epoch == cache_epoch())
-        return e;
-    Entry& e = ring[next++ % kEntries];
+    Entry& e = ring()[next++ % kEntries];
     if (e.pending) await_words(e.pinned, e.count, e.stream);  // its copy must not land later
     e.tensor = offsets;
     e.version = offsets._version();
     e.epoch = cache_epoch();
     e.count = (size_t)offsets.numel();
     e.pending = false;
+    return e;
+  }
+  static Entry& entry_for(const torch::Tensor& offsets, bool copy = true) {
+    TORCH_CHECK(offsets.defined() && offsets.scalar_type() == torch::kInt64,
+                "batch offsets must be an int64 tensor");
+    for (Entry& e : ring())
+      if (e.tensor.defined() && e.tensor.is_same(offsets) &&
+          e.version == (int64_t)offsets._version() && e.epoch == cache_epoch())
+        return e;
+    Entry& e = fresh_entry(offsets);
     if (!offsets.is_cuda() && copy) {
       torch::Tensor c = offsets.contiguous();
       e.host.assign(c.data_ptr<int64_t>(), c.data_ptr<int64_t>() + e.count);

@@ -557,6 +557,16 @@ static c10::intrusive_ptr<BlockBatch> blocks_of(const HandedOn& edges, const tor
   return out;
 }
 
+// Whether the keys of every batch fit the one work-group that labels them: known before
+// anything is queued (a batch that does not would be refused behind the whole slice).
+static bool batches_fit_labels(const torch::Tensor& col_bptr, const torch::Tensor& row_bptr) {
+  const std::vector<int64_t> cols = OffsetMirror::values(col_bptr);
+  const std::vector<int64_t>& rows = OffsetMirror::values(row_bptr);
+  for (size_t b = 0; b + 1 < cols.size(); ++b)
+    if (cols[b + 1] - cols[b] + rows[b + 1] - rows[b] > GS_LIST_LABELS_MAX_KEYS) return false;
+  return true;
+}
+
 // (every kept edge's row lies in its batch's segment of the list: both are moved by the batch)
 c10::optional<std::tuple<c10::intrusive_ptr<BlockBatch>, c10::optional<torch::Tensor>>>
 Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
@@ -568,7 +578,7 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   rows = ids(rows, "rows");
   const int64_t R = row_ids.numel(), S = seeds.numel(), B = col_bptr.numel() - 1;
   if (!m.indices.is_cuda() || R == 0 || S == 0 || R + S > B * (GS_LIST_LABELS_MAX_KEYS / 2) ||
-      !values_in_passing(m, values, row_divisor, R))
+      !values_in_passing(m, values, row_divisor, R) || !batches_fit_labels(col_bptr, row_bptr))
     return {};
   const std::shared_ptr<SliceOffsets> so = slice_offsets_for(seeds);
   const int64_t nnz = so->nnz;
@@ -608,7 +618,7 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   edges.finish(k, indptr, sums);
   c10::intrusive_ptr<BlockBatch> out = blocks_of(edges, indptr, col_bptr, seeds);
   const int64_t total = OffsetMirror::values(unique_ptr).back();
-  if (total < 0 || (k == 0 && values.has_value())) return {};  // (a batch of too many keys)
+  if (k == 0 && values.has_value()) return {};  // (the operators say what the values of no edges are)
   BatchOffsets::trust(unique_ptr);
   out->frontier_ptr = unique_ptr;
   out->frontier = frontier.narrow(0, 0, total);

@@ -210,13 +210,16 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
   auto picks_of = [&](int64_t size) {
     return replace ? (size > 0 ? num_picks : 0) : std::min(size, num_picks);
   };
-  int64_t total = 0;
+  std::vector<int64_t> picks_ptr{0};
   if (range.defined()) {
     const std::vector<int64_t>& p = OffsetMirror::values(range);
-    for (size_t b = 0; b + 1 < p.size(); ++b) total += picks_of(p[b + 1] - p[b]);
+    picks_ptr.reserve(p.size());
+    for (size_t b = 0; b + 1 < p.size(); ++b)
+      picks_ptr.push_back(picks_ptr.back() + picks_of(p[b + 1] - p[b]));
   } else {
-    total = picks_of(n);
+    picks_ptr.push_back(picks_of(n));
   }
+  const int64_t total = picks_ptr.back();
   torch::Tensor out = new_ids(total, probs);
   if (values) *values = torch::empty({total}, probs.options().requires_grad(false));
   const RandomState& rs = random_state();
@@ -225,6 +228,7 @@ static std::tuple<torch::Tensor, torch::Tensor> list_weighted(
       rs.seed, next_call_id(), mptr(out_range), total, mptr(out),
       values ? values->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), cur_stream()));
   BatchOffsets::trust(out_range, total);
+  if (range.defined()) OffsetMirror::known(out_range, std::move(picks_ptr));
   return {out, out_range};
 }
 

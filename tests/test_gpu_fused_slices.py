@@ -729,10 +729,16 @@ def test_encoded_row_slice_that_is_only_handed_on(seeds, picks, values):
     row_ids, row_ptr = T(np.concatenate(chosen)), T(np.concatenate([[0], np.cumsum([len(c) for c in chosen])]))
     by = torch.as_tensor((2.0 ** rng.integers(-2, 3, size=row_ids.numel())).astype(np.float32), device=DEV)
     extra = (w, by) if values else (None, None)
+    capi.profile_reset()
+    capi.profile_enable(True)
     got = g._CAPI_EncodedBlocks(seeds, ptr, rows, row_ids, row_ptr, *extra)
+    capi.profile_enable(False)
+    launched = capi.profile_totals()
     assert (got is None) == refused
     if refused:
+        assert not any(n.startswith(("member", "list")) for n in launched)  # before the slice is cut
         return
+    assert "member_label" in launched
     sub, index, names = g._CAPI_EncodedPickedRows(seeds, ptr, rows, row_ids, row_ptr)
     same_blocks(got[0], sub._CAPI_BatchBlocks(seeds, names))
     assert torch.equal(got[1], sub._CAPI_NormaliseColumns(w, index, by)) if values else got[1] is None

@@ -361,6 +361,20 @@ def test_picks_come_with_their_weights(n, k, replace):
     assert torch.equal(with_grad.grad, torch.bincount(picks, minlength=n).float())
 
 
+@pytest.mark.parametrize("replace", [False, True])
+@pytest.mark.parametrize("k", [0, 1, 40, 5000])
+def test_offsets_of_picks_are_known_to_the_host(k, replace):
+    """What a split of the picks goes by is what the device has: short and empty segments."""
+    ranges = T(np.concatenate([[0], np.cumsum([3, 0, 90, 40, 4500, 0])]))
+    probs = F(np.random.default_rng(k).random(int(ranges[-1])).astype(np.float32))
+    ops = torch.ops.gs_ops
+    picks, offsets = ops._CAPI_BatchListSamplingWithProbs(probs, k, replace, ranges)
+    parts = ops._CAPI_BatchSplitByOffset(picks, offsets)
+    assert [p.numel() for p in parts] == torch.diff(offsets).tolist()
+    for p, lo, hi in zip(parts, ranges[:-1].tolist(), ranges[1:].tolist()):
+        assert ((p >= lo) & (p < hi)).all()
+
+
 def picks(A, seeds, K, probs):
     sub = A[:, seeds]
     picked, index = sub.collective_sampling(K, probs, False)
