@@ -400,8 +400,8 @@ class Graph : public torch::CustomClassHolder {
                     bool replace, const torch::Tensor& cdf, uint64_t call_id, bool labels,
                     const std::function<void()>& idle);
   // Workspace of the small layers, kept between calls (one per matrix, at most
-  // 2^19 positions, 14 to 18 MB): its table is empty whenever a call has been
-  // queued, so the next call on the same stream starts without clearing it.  A call
+  // 2^19 positions, 22 MiB, 18 of weighted layers): its tables, two or one, are empty
+  // whenever a call has been queued, so the next call on the same stream starts without clearing it.  A call
   // takes it out and puts it back; one that finds none (another thread has it, or it
   // belongs to another stream) makes its own.
   struct LayerWorkspace {

@@ -230,7 +230,7 @@ std::vector<Graph::Layer> Graph::sample_layers(const torch::Tensor& seeds,
           cptr(ptr), B, K, replace ? 1 : 0, rs.seed, first_call + i, base, base + q.at_ptr,
           base + q.at_row, base + q.at_col, base + q.at_edge_ptr,
           blocks ? base + q.at_indptr : nullptr, mirrors + words * i, lw.positions, lw.ws.data_ptr(),
-          (size_t)lw.ws.numel(), (int)(i & 1)};
+          (size_t)lw.ws.numel(), weighted ? 0 : (int)(i & 1)};
       GS_CALL(gs_sample_layer_next(unlabelled.columns ? &unlabelled : nullptr, &next, cur_stream()));
       unlabelled = next;
       // the next layer's columns, as far as they are known

@@ -87,9 +87,10 @@ static LayerWs carve_layer(void* ws, int64_t positions, int weighted) {
   const int64_t n = positions > 0 ? positions : 1;
   w.slots = layer_table_slots(n);
   w.tiles = ceil_div(n, kLayerTile);
-  // (first, so that their places do not depend on the rest)
+  // (first, so that their places do not depend on the rest; weighted layers, which never run
+  // beside another's labels, have the first alone)
   w.table[0] = c.take<uint64_t>((size_t)w.slots);
-  w.table[1] = c.take<uint64_t>((size_t)w.slots);
+  w.table[1] = weighted ? nullptr : c.take<uint64_t>((size_t)w.slots);
   w.wide = c.take<int32_t>(1);
   w.slot = c.take<uint32_t>((size_t)n);
   w.first = c.take<uint32_t>((size_t)n);
@@ -625,7 +626,10 @@ __global__ __launch_bounds__(kBlock) void layer_clear_kernel(uint64_t* table0, u
                                                              int64_t slots, int32_t* wide) {
   int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i == 0) *wide = 0;
-  for (; i < slots; i += (int64_t)gridDim.x * kBlock) table0[i] = table1[i] = kEmptySlot;
+  for (; i < slots; i += (int64_t)gridDim.x * kBlock) {
+    table0[i] = kEmptySlot;
+    if (table1) table1[i] = kEmptySlot;
+  }
 }
 
 // weighted.hip: draws of a weighted layer into fanout places per column, the number
@@ -696,8 +700,9 @@ static int check_layer(const gs_layer& l) {
                  l.max_positions <= gs_layer_max_positions(),
              "sample_layer: %lld positions", (long long)(l.num_columns * (l.fanout + 1)));
   GS_REQUIRE(l.indptr && l.columns && l.out_frontier && l.out_frontier_ptr && l.out_row &&
-                 l.out_col && l.out_edge_ptr && l.mirror && (l.table == 0 || l.table == 1),
+                 l.out_col && l.out_edge_ptr && l.mirror,
              "sample_layer: null pointer");
+  GS_REQUIRE(l.table == 0 || (l.table == 1 && !l.cdf), "sample_layer: table %d", l.table);
   const LayerWs w = carve_layer(l.workspace, l.max_positions, l.cdf != nullptr);
   if (l.workspace == nullptr || l.workspace_bytes < w.total) {
     set_error("layer workspace too small: %zu < %zu", l.workspace_bytes, w.total);

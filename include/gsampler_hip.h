@@ -474,7 +474,8 @@ int gs_sample_layer(const int64_t* indptr, int64_t num_cols, const int64_t* indi
  * Every layer is given twice, first as `layer`, then as `before`, on one stream; where the
  * columns of `layer` are the frontier of `before` (its outputs as columns and col_ptr, the
  * same workspace and table != before->table) and neither is weighted the two run beside
- * each other.  `table`: 0 or 1, which of the workspace's two tables the layer hashes into;
+ * each other.  `table`: 0 or 1, which of the workspace's two tables the layer hashes into
+ * (a workspace for weighted layers has one: 0);
  * one that an unfinished layer has is not to be used. */
 typedef struct gs_layer {
   const int64_t* indptr;

@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import gsampler_amd as gs
+from gsampler_amd import capi
 from gsampler_amd.utils.block import Block, BlockList
 from tests.conftest import random_csc
 
@@ -171,6 +172,41 @@ def test_nodes_of_a_super_batch(rng, cuts, fanouts, replace, weighted):
     want = compiled.gm(run_time, [bm._graph], [[bm.row_ndata, bm.col_ndata, bm.edata]])
     for a, b in zip((*got[:2], *got[2]), (*want[:2], *want[2])):
         assert torch.equal(a, b)
+
+
+def test_workspaces_have_a_second_table_where_picks_run_beside_labels():
+    size, most = capi.lib().gs_layer_workspace_bytes, 1 << 19
+    table, drawn = 8 << 20, 8 * most
+    unweighted, weighted = size(most, 0) - table, size(most, 1) - drawn
+    assert 0 <= unweighted - weighted <= 256            # (the place of one draw, aligned)
+    assert size(most, 1) < 19 << 20 and size(most, 0) < 23 << 20
+
+
+@pytest.mark.parametrize("count,fanout,replace,weighted", [(1, 1, False, False), (73, 63, True, False),
+                                                           (1100, 10, False, True), (4000, 25, False, False)])
+def test_one_layer_by_the_call_of_its_own(rng, count, fanout, replace, weighted):
+    """gs_sample_layer, picks and labels in one call, against the chained form."""
+    m = matrix(rng, 3000, 40, 700, weighted)
+    seeds = torch.from_numpy(rng.integers(0, 3000, size=count)).to(DEV)
+    gs.manual_seed(5)
+    w = m.edata["w"] if weighted else None
+    want = m._graph._CAPI_SampleLayers(seeds, [fanout], replace, w)
+    l, P = capi.lib(), lambda t: t.data_ptr()
+    indptr, indices = m._graph._CAPI_GetCSCIndptr(), m._graph._CAPI_GetCSCIndices()
+    cdf = capi.weight_cdf(indptr, w, indices, 3000) if weighted else None
+    most = count * (fanout + 1)
+    ws = torch.empty(l.gs_layer_workspace_bytes(most, int(weighted)), dtype=torch.uint8, device=DEV)
+    capi.check(l.gs_layer_begin(most, int(weighted), P(ws), ws.numel(), None))
+    ids = [torch.empty(n, dtype=torch.int64, device=DEV) for n in (most, 2, most, most, 2)]
+    mirror = torch.empty(6, dtype=torch.int64).pin_memory()
+    for call in range(2):  # (the first leaves the table as it found it)
+        capi.check(l.gs_sample_layer(P(indptr), 3000, P(indices), None, P(cdf) if weighted else None, 3000,
+                                     P(seeds), count, None, 1, fanout, int(replace), 5, 0,
+                                     *(P(t) for t in ids), None, P(mirror), most, P(ws), ws.numel(), None))
+        torch.cuda.synchronize()
+        sizes = (int(mirror[1]), int(mirror[3]), int(mirror[3]))
+        for got, n, expect in zip((ids[0], ids[2], ids[3]), sizes, want):
+            assert torch.equal(got[:n], expect)
 
 
 def test_seeds_outside_the_matrix_take_the_other_path(rng):
