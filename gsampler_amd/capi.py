@@ -117,6 +117,7 @@ SIGNATURES = {
     "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
                                             _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),
+    "gs_col_row_slice_first_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_col_row_slice_labels": (_int, [_p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p, _p,
                                        _p, _sz, _p]),
     "gs_col_row_slice_fill": (_int, [_p, _p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
@@ -787,7 +788,9 @@ def col_row_slice(indptr, indices, cols, rows, key_offset=None, with_major=True,
     sub_indptr = col_count(indptr, cols, -1, False)
     nnz = int(sub_indptr[-1].item())
     l = lib()
-    ws = _workspace(l.gs_minor_slice_workspace_bytes(nnz, nrow), dev)
+    size = (l.gs_minor_slice_workspace_bytes if out_first is None
+            else l.gs_col_row_slice_first_workspace_bytes)
+    ws = _workspace(size(nnz, nrow), dev)
     out_indptr = torch.empty(ncol + 1, dtype=torch.int64, device=dev)
     total = torch.empty(1, dtype=torch.int64, device=dev)
     check(l.gs_col_row_slice_count_first(

@@ -155,7 +155,6 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
                                  torch::Tensor* zeros = nullptr) {
   const int64_t n = cols.numel(), np = picked.numel();
   MajorResult r;
-  torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, np), m.indptr);
   r.indptr = new_ids(n + 1, m.indptr);
   // the number of kept edges goes straight to pinned host memory; the fill pass
   // is queued into buffers sized by the bound (every edge kept) and runs while
@@ -165,6 +164,8 @@ static MajorResult col_row_slice(const Compressed& m, const torch::Tensor& cols,
   // (the relabel of a slice with far fewer rows than edges goes by its rows' first edges)
   // (and its edges' values are often divided by sums over their columns: cleared in passing)
   const bool tells = firsts && nnz >= 8 * np && gs_col_row_slice_tells_first(nnz, np);
+  torch::Tensor ws = new_workspace(tells ? gs_col_row_slice_first_workspace_bytes(nnz, np)
+                                         : gs_minor_slice_workspace_bytes(nnz, np), m.indptr);
   if (zeros) {
     const torch::Tensor buffer = new_ids((tells ? np : 0) + n, m.indptr);
     *zeros = piece_of(buffer, 0, n, false);
@@ -285,7 +286,7 @@ Graph::RelabelledRows(torch::Tensor cols, torch::Tensor rows, c10::optional<torc
   const int64_t nnz = so->nnz;
   if (nnz < 8 * (R + S) || nnz > kBoundLimit || !gs_col_row_slice_tells_first(nnz, R)) return {};
   const torch::Tensor narrow = narrow_for_slice(m, nnz, S);
-  torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, R), m.indptr);
+  torch::Tensor ws = new_workspace(gs_col_row_slice_first_workspace_bytes(nnz, R), m.indptr);
   torch::Tensor indptr = new_ids(S + 1, m.indptr);
   // first edges and labels of the rows, labels of the columns and their sums
   torch::Tensor small = new_ids(2 * R + 2 * S, m.indptr);
@@ -589,7 +590,7 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   GS_CALL(gs_pick_batch_ids(cptr(rows), rows.numel(), cptr(row_ids), cptr(row_bptr), B, R, num_rows_,
                             mptr(names), mptr(picked), nullptr, refused.word(), cur_stream()));
   const torch::Tensor narrow = narrow_for_slice(m, nnz, S);
-  torch::Tensor ws = new_workspace(gs_minor_slice_workspace_bytes(nnz, R), m.indptr);
+  torch::Tensor ws = new_workspace(gs_col_row_slice_first_workspace_bytes(nnz, R), m.indptr);
   torch::Tensor indptr = new_ids(S + 1, m.indptr), unique_ptr = new_ids(B + 1, m.indptr);
   torch::Tensor frontier = new_ids(R + S, m.indptr);
   // first edges and labels of the rows, labels of the columns and their sums, scratch

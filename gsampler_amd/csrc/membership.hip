@@ -129,7 +129,8 @@ static uint64_t member_table_slots(int64_t num_picked) {
   return (uint64_t)((num_picked <= kMemberRoomyIds ? 4 : 2) * num_picked + 2);
 }
 
-static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
+// firsts: with room for first edges, behind the rest, which lies where it does without.
+static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked, bool firsts = false) {
   Carver c(ws);
   MemberWs w;
   w.chunks = ceil_div(nnz > 0 ? nnz : 1, kBlock);
@@ -141,10 +142,11 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked) {
       c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
   w.wide = c.take<int>(1);
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
-  w.first_groups = member_in_lds(num_picked) ? std::min(w.chunks, kMemberMostGroups) : 0;
-  w.firsts = c.take<uint32_t>((size_t)(w.first_groups * num_picked));
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
+  w.first_groups =
+      firsts && member_in_lds(num_picked) ? std::min(w.chunks, kMemberMostGroups) : 0;
+  w.firsts = c.take<uint32_t>((size_t)(w.first_groups * num_picked));
   w.total = c.total();
   return w;
 }
@@ -499,7 +501,8 @@ void member_flag_kernel(
   if (kInLds) {
     static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
     for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
-    for (int i = threadIdx.x; i < kMemberLdsIds; i += kThreads) sh.first[i] = UINT32_MAX;
+    if (firsts)
+      for (uint32_t i = threadIdx.x; i < num_picked; i += kThreads) sh.first[i] = UINT32_MAX;
     wide = buckets.template stage<kThreads>(
         picked, num_picked, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
           const uint32_t h = Filter::hash(key);
@@ -1077,6 +1080,11 @@ size_t gs_minor_slice_workspace_bytes(int64_t nnz, int64_t num_picked) {
   return gs::carve_member(nullptr, nnz, num_picked).total;
 }
 
+size_t gs_col_row_slice_first_workspace_bytes(int64_t slice_nnz, int64_t num_rows_picked) {
+  if (slice_nnz < 0 || num_rows_picked < 0) return 0;
+  return gs::carve_member(nullptr, slice_nnz, num_rows_picked, true).total;
+}
+
 static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int64_t nnz,
                                   const int64_t* picked,
                                   int64_t num_picked, const int64_t* indptr,
@@ -1101,7 +1109,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   // per id) is addressed with 32-bit arithmetic
   GS_REQUIRE(num_picked < (int64_t(1) << 30),
              "minor_slice_count: at most 2^30 - 1 picked ids, got %lld", (long long)num_picked);
-  MemberWs w = carve_member(workspace, nnz, num_picked);
+  MemberWs w = carve_member(workspace, nnz, num_picked, out_first != nullptr);
   if (workspace == nullptr || workspace_bytes < w.total) {
     set_error("minor_slice workspace too small: %zu < %zu", workspace_bytes, w.total);
     return GS_ERR_WORKSPACE;

@@ -723,8 +723,8 @@ int gs_minor_slice_fill(const int64_t* ids, int64_t nnz, int64_t num_picked,
  *  fill: out_minor[kept] = position in `rows`, out_select[kept] = position of the
  *    edge in the PARENT's indices, out_major[kept] (nullable) = position of its
  *    column in `cols`.
- * Workspace: gs_minor_slice_workspace_bytes(slice_nnz, num_rows_picked), the
- * same buffer for both calls.  Stands in for CSCColRowSlicingCUDA and
+ * Workspace: gs_minor_slice_workspace_bytes(slice_nnz, num_rows_picked), with
+ * out_first gs_col_row_slice_first_workspace_bytes of them, the same buffer for both calls.  Stands in for CSCColRowSlicingCUDA and
  * BatchCSCColRowSlicingCUDA (src/cuda/fusion/column_row_slicing.cu:213-217,
  * 356-362; kernels :102-146, :220-264), whose select index addresses the
  * intermediate slice instead of the parent.
@@ -745,6 +745,7 @@ int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
                                  double* col_zeros, void* workspace, size_t workspace_bytes,
                                  gs_stream_t stream);
 int gs_col_row_slice_tells_first(int64_t slice_nnz, int64_t num_rows_picked);
+size_t gs_col_row_slice_first_workspace_bytes(int64_t slice_nnz, int64_t num_rows_picked);
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,
                           int64_t num_cols_picked, const int64_t* sub_indptr,
                           int64_t slice_nnz, int64_t num_rows_picked, int64_t* out_major,

@@ -92,6 +92,27 @@ def test_col_row_slice_tells_the_first_edge_of_every_row(nnz, nrow):
         assert np.array_equal(got[2].cpu().numpy(), order[found[hit]])
 
 
+def test_scratch_for_first_edges_where_they_are_asked_for():
+    """1024 work-groups' lists of 2047 ids are 8 MB: in the workspace of the calls that tell
+    first edges, in no other's, and refused where it is missing."""
+    l, nnz, nrow = capi.lib(), 1 << 23, 2047
+    plain = l.gs_minor_slice_workspace_bytes(nnz, nrow)
+    told = l.gs_col_row_slice_first_workspace_bytes(nnz, nrow)
+    assert told - plain == 4 * 1024 * nrow
+    assert l.gs_col_row_slice_first_workspace_bytes(nnz, 2049) == l.gs_minor_slice_workspace_bytes(nnz, 2049)
+    rng = np.random.default_rng(2)
+    indptr, ids = T([0, 5000]), T(rng.integers(0, 90, size=5000))
+    cols, sub, out = T([0]), T([0, 5000]), torch.empty(2, dtype=torch.int64, device=DEV)
+    rows, first = T(np.arange(70)), torch.full((70,), -7, dtype=torch.int64, device=DEV)
+    ws = torch.empty(l.gs_minor_slice_workspace_bytes(5000, 70), dtype=torch.uint8, device=DEV)
+    P = lambda t: t.data_ptr()
+    args = (P(indptr), P(ids), None, P(cols), None, 1, P(sub), 5000, P(rows), 70, P(out), None)
+    assert l.gs_col_row_slice_count_first(*args, P(first), None, P(ws), ws.numel(), None) != 0
+    assert l.gs_col_row_slice_count_first(*args, None, None, P(ws), ws.numel(), None) == 0
+    torch.cuda.synchronize()
+    assert (first == -7).all() and out[1].item() == int((ids < 70).sum())
+
+
 def test_col_row_slice_of_long_columns():
     """Columns far longer than a work-group's run of edges (the layer-wise
     sampler's case), columns without edges in between, a column id outside the
