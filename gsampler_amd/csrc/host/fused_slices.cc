@@ -433,7 +433,7 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
 
 // What a layer-wise sampler asks an encoded slice (BatchColSlicing with encoding) for:
 // its rows with where every batch's begin, and the sums of its squared edge values on
-// them.  The slice is not written; the picked rows' edges come from EncodedRowSlicing.
+// them.  The slice is not written; the picked rows' edges come from EncodedPickedRows.
 // Nothing where the slice has to be written after all: values that are no plain float32
 // edge data, or keys too many or too few for the pass.
 c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> Graph::EncodedSquareSums(
@@ -515,15 +515,6 @@ static void check_encoded(torch::Tensor& seeds, torch::Tensor& col_bptr, torch::
 static void check_picks(const HostFlag& refused, const torch::Tensor& rows) {
   TORCH_CHECK(!refused.raised(), "BatchRowSlicing: a picked row lies outside the ", rows.numel(),
               " rows of the slice");
-}
-
-GraphAndIndex Graph::EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr,
-                                       torch::Tensor rows, torch::Tensor row_ids,
-                                       torch::Tensor row_bptr) {
-  check_encoded(seeds, col_bptr, row_ids, row_bptr);
-  torch::Tensor picked =
-      encoded_ids(rows.index_select(0, row_ids), row_bptr, row_ids.numel(), num_rows_);
-  return encoded_row_slice(seeds, col_bptr, picked, row_ids, row_bptr);
 }
 
 std::tuple<GraphPtr, torch::Tensor, torch::Tensor> Graph::EncodedPickedRows(

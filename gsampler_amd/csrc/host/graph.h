@@ -340,9 +340,7 @@ class Graph : public torch::CustomClassHolder {
                                 bool encoding);
   c10::optional<std::tuple<torch::Tensor, torch::Tensor, torch::Tensor>> EncodedSquareSums(
       torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor efeat);
-  GraphAndIndex EncodedRowSlicing(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows,
-                                  torch::Tensor row_ids, torch::Tensor row_bptr);
-  // The same for row_ids known to lie in `rows` (a sampler's picks of them); and rows[row_ids].
+  // BatchRowSlicing of that slice by row_ids, positions in its `rows`; and rows[row_ids].
   std::tuple<GraphPtr, torch::Tensor, torch::Tensor> EncodedPickedRows(
       torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor rows, torch::Tensor row_ids,
       torch::Tensor row_bptr);

@@ -125,8 +125,7 @@ TORCH_LIBRARY(gs_classes, m) {
       .def("_CAPI_SubgraphBlocks", &Graph::SubgraphBlocks)
       .def("_CAPI_NormaliseColumns", &Graph::NormaliseColumns)
       .def("_CAPI_EncodedSquareSums", &Graph::EncodedSquareSums)
-      .def("_CAPI_EncodedPickedRows", &Graph::EncodedPickedRows)
-      .def("_CAPI_EncodedRowSlicing", &Graph::EncodedRowSlicing);
+      .def("_CAPI_EncodedPickedRows", &Graph::EncodedPickedRows);
 }
 
 TORCH_LIBRARY(gs_ops, m) {

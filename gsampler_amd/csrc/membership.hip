@@ -48,7 +48,12 @@ constexpr int kMemberThreads = 1024;  // 16 waves share one table
 // where two now take 64 and 43).
 constexpr int kMemberWavesPerSimd = 8;
 constexpr int kMemberLdsSlots = 4096;  // of a table in LDS (32 KB)
-constexpr int kMemberLdsIds = kMemberLdsSlots / 2;  // picked sets of up to so many ids have theirs in LDS
+// Picked sets of up to so many ids have theirs in LDS: half of its slots.  Count passes that
+// tell no first edges, us, at the bound and one id past it, with the launches that make a table
+// in L2: 28 M edges 51 and 59, 8 M 49 and 42, 1 M 26 and 21.  On the shorter lists the table in
+// L2 is ahead from about 1500 ids on, but first edges, and with them slices that are only
+// handed on, need the one in LDS.
+constexpr int kMemberLdsIds = kMemberLdsSlots / 2;
 constexpr int64_t kMemberSmallEdges = int64_t(1) << 23;  // below: work-groups of kBlock threads
 // Work-groups of a launch that stages its table in LDS, at most: what is resident on 256
 // compute units is 512 large ones or 768 small ones.
