@@ -31,7 +31,8 @@ __global__ __launch_bounds__(kBlock) void encode_batch_ids_kernel(
 // The same for ids picked from a list: id = ids[index[i]] (without index: ids[i]), which goes
 // out as it is, moved by its batch, and the move alone, whatever of the three is wanted: one
 // launch where a gather and up to two of the above were.  A place outside the list reads no id
-// and raises `refused`.
+// and raises `refused`.  An id that is no row is moved past the rows of all batches, where
+// nothing meets it: moved by its batch it would be another batch's row.
 __global__ __launch_bounds__(kBlock) void pick_batch_ids_kernel(
     const int64_t* __restrict__ ids, int64_t num_ids, const int64_t* __restrict__ index,
     const int64_t* __restrict__ batch_ptr, int64_t num_batches, int64_t n, int64_t stride,
@@ -47,7 +48,8 @@ __global__ __launch_bounds__(kBlock) void pick_batch_ids_kernel(
   if (!listed && refused) store_for_host(refused, 1);
   const int64_t offset = span.segment_at(batch_ptr, i) * stride;
   if (out_id) out_id[i] = id;
-  if (out_moved) out_moved[i] = id + offset;
+  if (out_moved)
+    out_moved[i] = (uint64_t)id < (uint64_t)stride ? id + offset : num_batches * stride;
   if (out_offset) out_offset[i] = offset;
 }
 

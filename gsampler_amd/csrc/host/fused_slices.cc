@@ -338,12 +338,10 @@ torch::Tensor Graph::take_column_zeros() {
   return zeros;
 }
 
-// The ids `of` (undefined: zeros) of every batch moved by batch * stride.
-static torch::Tensor encoded_ids(const torch::Tensor& of, const torch::Tensor& bptr, int64_t n,
-                                 int64_t stride) {
+// batch * stride for everything that the batches hold.
+static torch::Tensor moves_by_batch(const torch::Tensor& bptr, int64_t n, int64_t stride) {
   torch::Tensor e = new_ids(n, bptr);
-  GS_CALL(gs_encode_batch_ids(cptr(of), cptr(bptr), bptr.numel() - 1, n, stride, mptr(e),
-                              cur_stream()));
+  GS_CALL(gs_encode_batch_ids(nullptr, cptr(bptr), bptr.numel() - 1, n, stride, mptr(e), cur_stream()));
   return e;
 }
 
@@ -363,7 +361,7 @@ void Graph::SliceOffsets::keep_key_offset(const torch::Tensor& bptr, const torch
 torch::Tensor Graph::key_offsets_for(SliceOffsets& so, const torch::Tensor& col_bptr) {
   torch::Tensor offset = so.kept_key_offset(col_bptr);
   if (!offset.defined()) {
-    offset = encoded_ids(torch::Tensor(), col_bptr, so.cols.numel(), num_rows_);
+    offset = moves_by_batch(col_bptr, so.cols.numel(), num_rows_);
     so.keep_key_offset(col_bptr, offset);
   }
   return offset;
@@ -396,8 +394,11 @@ GraphAndIndex Graph::BatchColRowSlcing(torch::Tensor col, torch::Tensor col_bptr
                               row.numel(), stride, nullptr, mptr(picked), mptr(key_offset),
                               nullptr, cur_stream()));
   } else {
-    key_offset = encoded_ids(torch::Tensor(), col_bptr, col.numel(), stride);
-    picked = encoded_ids(row, row_bptr, row.numel(), stride);
+    key_offset = moves_by_batch(col_bptr, col.numel(), stride);
+    picked = new_ids(row.numel(), row_bptr);
+    GS_CALL(gs_pick_batch_ids(cptr(row), row.numel(), nullptr, cptr(row_bptr), row_bptr.numel() - 1,
+                              row.numel(), stride, nullptr, mptr(picked), nullptr, nullptr,
+                              cur_stream()));
   }
   const std::shared_ptr<SliceOffsets> shared = slice_offsets_for(col);
   SliceOffsets& so = *shared;

@@ -875,7 +875,8 @@ int gs_batch_seeds_distinct(const int64_t* frontier, const int64_t* frontier_ptr
                             int64_t num_batches, int64_t* out_distinct,
                             gs_stream_t stream);
 /* gs_pick_batch_ids: with id = ids[index[i]] (index nullable: ids[i]) for item i of batch b,
- * out_id[i] = id, out_moved[i] = id + b * stride and out_offset[i] = b * stride, each
+ * out_id[i] = id, out_moved[i] = id + b * stride (num_batches * stride, which no id of a
+ * batch becomes, where id lies outside [0, stride)) and out_offset[i] = b * stride, each
  * nullable.  A place outside [0, num_ids) counts as id 0.
  * gs_local_ids: out[e] = table[rows[e]], its remainder by stride where stride > 0; a row
  * outside [0, num_ids) reads table[0].

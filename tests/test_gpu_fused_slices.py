@@ -765,6 +765,34 @@ def test_encoded_row_slice_that_is_only_handed_on(seeds, picks, values):
     assert torch.equal(got[1], sub._CAPI_NormaliseColumns(w, index, by)) if values else got[1] is None
 
 
+@pytest.mark.parametrize("blocks", [False, True])
+@pytest.mark.parametrize("square", [False, True])
+def test_batches_whose_lists_have_ids_that_are_no_rows(square, blocks):
+    """A matrix of fewer rows than columns: an id past its rows has no edges in any batch, in
+    its own or in the one whose rows it would be taken for when moved by its batch."""
+    rng = np.random.default_rng(6)
+    num_rows, num_cols = 60, 100
+    indptr, indices = columns_of(rng.integers(5, 40, num_cols), rng, num_rows)
+    g = gs.Graph(num_rows, num_cols)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    lists = [rng.permutation(num_cols)[:k] for k in (30, 0, 50, 41, 100, 7)]
+    ptr = T(np.concatenate([[0], np.cumsum([len(x) for x in lists])]))
+    nodes = T(np.concatenate(lists))
+    rows = nodes if square else nodes.clone()
+    if blocks and square:
+        batch = g._CAPI_SubgraphBlocks(nodes, ptr)
+    else:
+        sub, _ = g._CAPI_BatchColRowSlcing(nodes, ptr, rows, ptr)
+        batch = sub._CAPI_BatchBlocks(nodes, rows)
+    frontier, fptr, eptr = (x().tolist() for x in (batch.frontier, batch.frontier_ptr, batch.edge_ptr))
+    row, col = batch.row().cpu().numpy(), batch.col().cpu().numpy()
+    for b, ids in enumerate(lists):
+        assert frontier[fptr[b]:fptr[b + 1]] == ids.tolist()
+        want = [(r, c) for c in ids for r in indices[indptr[c]:indptr[c + 1]] if r in ids]
+        edges = slice(eptr[b], eptr[b + 1])
+        assert [(ids[r], ids[c]) for r, c in zip(row[edges], col[edges])] == want
+
+
 @pytest.mark.parametrize("sizes", [[40], [64, 0, 300, 1], [3] * 70, [3000, 20_000]])
 def test_subgraphs_that_are_only_handed_on(sizes):
     rng = np.random.default_rng(len(sizes))
