@@ -14,15 +14,15 @@
 //            start), the batch of every tile, bucket, group of positions and
 //            tile of edges (so that a work-group finds its work with two
 //            dependent loads instead of a binary search); zero the counters
-//   scatter  per tile: order the tile by bucket in LDS, reserve a run in every
+//   scatter  per tile: keep one position, the smallest, of a key that repeats inside
+//            the tile; order the tile by bucket in LDS, reserve a run in every
 //            bucket with one atomic on the bucket's cursor, write
 //            key << 32 | local.  A bucket owns a region of fixed capacity (as
 //            many entries as the batch has keys, at most kBucketCap, five times
 //            the average bucket), so where a run goes is known without
 //            counting the keys per bucket first: the keys are read once here,
-//            not twice.  What does not fit a region (a key that repeats more
-//            than kBucketCap times in one batch) goes to the batch's overflow
-//            list together with its bucket
+//            not twice.  What does not fit a region (very many keys that meet in
+//            one bucket) goes to the batch's overflow list together with its bucket
 //   dedup    per bucket: LDS table with "smallest position wins" (64-bit
 //            atomicMin on the packed entry), then every entry writes the first
 //            position of its key into first[position]
@@ -37,8 +37,8 @@
 //            (80 KB per batch of 330 K keys), which a die's L2 holds
 // The result does not depend on the order in which entries land in a bucket, so
 // the atomics above leave it deterministic.  A bucket with more entries than the
-// LDS table is sure to hold (a hub that repeats thousands of times, a batch too
-// large for kMaxBuckets buckets) is deduplicated by the same work-group in a
+// LDS table is sure to hold (a batch too large for kMaxBuckets buckets, a wide key
+// that repeats thousands of times) is deduplicated by the same work-group in a
 // table in global memory that is private to the bucket; a bucket whose region
 // ran over first collects its entries from the batch's overflow list.
 //
@@ -64,14 +64,15 @@ constexpr int kLdsMaxEntries = kLdsSlots * 3 / 4; // bucket sizes the LDS table 
 constexpr int64_t kBucketCap = 8192;              // entries a bucket's region holds at most
 static_assert(kBucketCap >= kLdsMaxEntries, "the short dedup path reads a bucket from its region alone");
 
-// Average entries per bucket and whether work-groups are laid out per die: the
-// best of a sweep on 21M keys in 64 batches (bucket sizes 512..3072, with and
-// without the per-die layout).
+// Keys per bucket (a fifth of them repeats that never get there) and whether work-groups
+// are laid out per die: the best of a sweep on 21M keys in 64 batches (dedup pass of
+// 1536 keys 83 us, 1792 78, 2048 78; before repeats stayed behind 512..3072, with and without
+// the per-die layout).
 struct UniqueTuning {
   int64_t bucket_keys;
   int remap;
 };
-static UniqueTuning tuning() { return UniqueTuning{1536, 1}; }
+static UniqueTuning tuning() { return UniqueTuning{1792, 1}; }
 
 // Work-group index -> unit of work (tile or bucket).  Consecutive work-groups
 // go to consecutive dies, so die x is given the x-th eighth of the units, in
@@ -115,6 +116,8 @@ struct alignas(16) RankWord {
   uint32_t before;
   uint32_t unused;
 };
+
+constexpr uint32_t kFirstMark = 0x80000000u;  // (positions are below 2^31 - 1)
 
 struct UniqueWs {
   BatchInfo* batch;       // [B]
@@ -425,11 +428,14 @@ __device__ __forceinline__ uint32_t key_tag(uint64_t key) {
 // overflow list instead (the cursor still counts them, which is how the dedup
 // pass knows).  The tile is first ordered by bucket in LDS so that every run
 // leaves as one contiguous write instead of one line per entry.
-// 48 KB of LDS per work-group lets three share a compute unit: with 512 threads
+// 48 KB of LDS per work-group (the words of repeats lie where the tile is ordered later) lets three share a compute unit: with 512 threads
 // each they fill three quarters of its wavefront slots (256 threads: 11 % slower
 // on 21 M keys; 1024, two work-groups per unit: 45 % slower).
 constexpr int kScatterThreads = 512;
 constexpr int kScatterItems = kPartTile / kScatterThreads;
+constexpr int kTileBits = 12;
+static_assert(kPartTile == 1 << kTileBits, "a position inside a tile takes kTileBits bits");
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;  // of a position that has no part in this
 __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
     Keys k, const int32_t* __restrict__ tile_batch,
     const BatchInfo* __restrict__ batch, int64_t* bucket_cur, int64_t* ovf_cur,
@@ -440,6 +446,7 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
   __shared__ uint32_t run_at[kMaxBuckets]; // where the tile's run starts in the bucket
   __shared__ uint64_t stage[kPartTile];
   __shared__ uint32_t scan_smem[kScatterThreads / kWave + 1];
+  uint32_t* const kept = (uint32_t*)stage;  // (until the tile is ordered there)
   const int64_t tile = unit_of_block(max_tiles, remap);
   if (tile >= max_tiles) return;
   TileInfo t;
@@ -475,24 +482,55 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
     const uint32_t bin = threadIdx.x + r * kScatterThreads;
     if (bin < buckets) hist[bin] = 0;
   }
-  __syncthreads();
+  // One position of a key, its smallest, stands for all that the tile holds of it: the others
+  // are told now, and marked, to take what that one will be told.  Ids of a power law repeat
+  // within 4096 keys a fifth of the time (within a batch of 330 K half), and hubs always do:
+  // their buckets, thousands of repeats each, took the dedup pass 40 of 125 us on 21M keys and
+  // now 82, this pass 92 and now 86, the labels' further look-up 114 and now 120.
+  // A key has one word to meet in, told by the upper bits of a product that loses nothing of
+  // it; of several keys the last to write has the word, more likely so the more often it is
+  // there, and the others' repeats are sent as they are.  (A key of 2^32 - 1 or more stays out:
+  // it is not known by its tag.)
   bool wide = false;
+  uint32_t slot[kScatterItems], word[kScatterItems];  // word: rest of the product, place in the tile
+  auto same_key = [](uint32_t a, uint32_t b) { return (a ^ b) < (uint32_t)kPartTile; };
+#pragma unroll
+  for (int i = 0; i < kScatterItems; ++i) {
+    const uint32_t l = i * kScatterThreads + threadIdx.x;
+    wide |= full[i] > kMaxPackedKey;
+    key[i] = key_tag(full[i]);
+    const uint32_t h = key[i] * 0x9E3779B1u;
+    slot[i] = h >> (32 - kTileBits);
+    word[i] = h << kTileBits | l;
+    if (t.begin + l >= t.end || full[i] > kMaxPackedKey) slot[i] = kNoSlot;
+    if (slot[i] != kNoSlot) kept[slot[i]] = word[i] | (uint32_t)(kPartTile - 1);
+  }
+  if (wide) *wide_keys = 1;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kScatterItems; ++i) {
+    const uint32_t w = slot[i] != kNoSlot ? kept[slot[i]] : 0u;
+    if (w > word[i] && same_key(w, word[i])) atomicMin(&kept[slot[i]], word[i]);
+  }
+  __syncthreads();
+  bool sent[kScatterItems];
 #pragma unroll
   for (int i = 0; i < kScatterItems; ++i) {
     const int64_t l = t.begin + i * kScatterThreads + threadIdx.x;
-    wide |= full[i] > kMaxPackedKey;
-    key[i] = key_tag(full[i]);
-    // every position starts as its own first occurrence; the dedup pass only
-    // writes the positions that are not (half as many scattered stores)
-    if (l < t.end) first[t.b.fb + l] = (uint32_t)l;
+    const uint32_t w = slot[i] != kNoSlot ? kept[slot[i]] : word[i];
+    const bool repeat = w < word[i] && same_key(w, word[i]);
+    sent[i] = l < t.end && !repeat;
+    // every position that is sent starts as its own first occurrence; the dedup pass only
+    // writes those that are not (half as many scattered stores)
+    if (l < t.end)
+      first[t.b.fb + l] =
+          repeat ? ((uint32_t)t.begin + w % (uint32_t)kPartTile) | kFirstMark : (uint32_t)l;
   }
-  if (wide) *wide_keys = 1;
 #pragma unroll
   for (int i = 0; i < kScatterItems; ++i)
-    if (t.begin + i * kScatterThreads + threadIdx.x < t.end)
-      place[i] = atomicAdd(&hist[bucket_of(key[i], buckets)], 1u);
+    if (sent[i]) place[i] = atomicAdd(&hist[bucket_of(key[i], buckets)], 1u);
   __syncthreads();
-  const uint32_t count = (uint32_t)(t.end - t.begin);
+  uint32_t count;
   {
     const uint32_t bin0 = threadIdx.x * kBins;
     uint32_t c[kBins], sum = 0;
@@ -501,8 +539,7 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
       c[j] = bin0 + j < buckets ? hist[bin0 + j] : 0u;
       sum += c[j];
     }
-    uint32_t total;
-    uint32_t run = block_exclusive_sum<uint32_t, kScatterThreads>(sum, scan_smem, &total);
+    uint32_t run = block_exclusive_sum<uint32_t, kScatterThreads>(sum, scan_smem, &count);
 #pragma unroll
     for (int j = 0; j < kBins; ++j) {
       if (bin0 + j < buckets) hist[bin0 + j] = run;
@@ -529,7 +566,7 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
 #pragma unroll
   for (int i = 0; i < kScatterItems; ++i) {
     const int64_t l = t.begin + i * kScatterThreads + threadIdx.x;
-    if (l < t.end)
+    if (sent[i])
       stage[hist[bucket_of(key[i], buckets)] + place[i]] =
           ((uint64_t)key[i] << 32) | (uint64_t)l;
   }
@@ -1126,9 +1163,8 @@ constexpr int kFewBinKeys = 512;
 constexpr uint32_t kFewSlots = 2048;  // of a bin's table: four times the keys it gets on average
 constexpr uint32_t kFewClaims = kFewSlots * 3 / 4;
 constexpr uint32_t kFewListed = 2048;  // keys of a bin that are found again without a second look
-// first[position] of a call that went this way carries a mark where the position is itself
-// a first occurrence.  (Positions are below 2^31 - 1.)
-constexpr uint32_t kFirstMark = 0x80000000u;
+// first[position] of a call that went this way carries kFirstMark where the position is itself
+// a first occurrence.
 constexpr uint32_t kFewOpen = 0xFFFFFFFFu;  // no position, marked or not
 // Bin of a key: a hash of 32 bits, for every work-group hashes every key of its batch.  A
 // multiplication alone puts ids in steps of some sizes into one bin (by 2^32 over the golden
@@ -1541,7 +1577,17 @@ struct LabelArgs {
   int64_t* out_col;
   int remap;
   int col_prefilled;  // out_col holds every column's place inside its batch already
+  bool chase;         // a mark in first[] means that what it says has to be looked up in turn
 };
+
+// What first[] says of a position, when it said f: a marked position is a repeat inside a
+// partition tile and takes what the one it names was told.
+__device__ __forceinline__ uint32_t first_of(const uint32_t* __restrict__ first_b, uint32_t f,
+                                             bool chase) {
+  if (!(f & kFirstMark)) return f;
+  f &= ~kFirstMark;
+  return chase ? first_b[f] : f;
+}
 
 template <bool kByIndptr>
 __device__ __forceinline__ void relabel_tile(
@@ -1550,7 +1596,7 @@ __device__ __forceinline__ void relabel_tile(
     const RankWord* __restrict__ words, const int64_t* __restrict__ group_off,
     const int64_t* __restrict__ unique_ptr, const int64_t* __restrict__ edge_col,
     const int64_t* __restrict__ col_indptr, int64_t* __restrict__ out_row,
-    int64_t* __restrict__ out_col_or_null, int remap, int col_prefilled) {
+    int64_t* __restrict__ out_col_or_null, int remap, int col_prefilled, bool chase) {
   const int64_t num_tiles = ceil_div_dev(k.E, kRelabelTile);
   const int64_t tile = unit_of_block(num_tiles, remap);
   if (tile >= num_tiles) return;
@@ -1588,8 +1634,17 @@ __device__ __forceinline__ void relabel_tile(
     if (!one_batch) info = batch[batch_in_span(k.rows_ptr, span, e)];
     // row key e of batch b sits at flat position
     //   fb + (seeds of b) + (e - rows_ptr[b])  =  e + seeds_ptr[b + 1]
-    if (out_row) row_first[i] = first[e + info.s_lo + info.ns] & ~kFirstMark;
+    if (out_row) row_first[i] = first[e + info.s_lo + info.ns];
     if (out_col && !kByIndptr) col[i] = edge_col[e];
+  }
+  if (out_row) {
+#pragma unroll
+    for (int i = 0; i < kRelabelItems; ++i) {
+      const int64_t e = edge_of(i);
+      if (e >= k.E) break;
+      if (!one_batch) info = batch[batch_in_span(k.rows_ptr, span, e)];
+      row_first[i] = first_of(first + info.fb, row_first[i], chase);
+    }
   }
   if (kByIndptr && out_col) {
     // (after the loads above have been issued: they travel during the search)
@@ -1628,8 +1683,8 @@ __device__ __forceinline__ void relabel_tile(
         col_label.v[j] =
             seeds_distinct
                 ? col[i + j] - info.s_lo
-                : rank_of(info.fb + (first[col[i + j] + info.r_lo] & ~kFirstMark), words, group_off) -
-                      rank0;
+                : rank_of(info.fb + first_of(first + info.fb, first[col[i + j] + info.r_lo], chase),
+                          words, group_off) - rank0;
     }
     const int64_t e = edge_of(i);
     if (e + 1 < k.E && wide_stores) {
@@ -1652,7 +1707,7 @@ __global__ __launch_bounds__(kBlock) void unique_relabel_kernel(
     const RankWord* __restrict__ words, const int64_t* __restrict__ group_off) {
   relabel_tile<kByIndptr>(k, l.etile_batch, batch, l.first, words, group_off, l.unique_ptr,
                           l.edge_col, l.col_indptr, l.out_row, l.out_col, l.remap,
-                          l.col_prefilled);
+                          l.col_prefilled, l.chase);
 }
 
 // Both of the above in one launch: the first `label_blocks` work-groups label
@@ -1667,7 +1722,7 @@ __global__ __launch_bounds__(kBlock) void unique_fill_relabel_kernel(
   if (blockIdx.x < label_blocks)
     relabel_tile<kByIndptr>(k, l.etile_batch, batch, l.first, words, group_off, l.unique_ptr,
                             l.edge_col, l.col_indptr, l.out_row, l.out_col, l.remap,
-                            l.col_prefilled);
+                            l.col_prefilled, l.chase);
   else
     fill_group(blockIdx.x - label_blocks, k, f.flat_ptr, f.group_batch, batch, f.N, words,
                group_off, f.out_unique);
@@ -1682,6 +1737,10 @@ __global__ __launch_bounds__(kBlock) void unique_empty_kernel(
   if (distinct_mirror && i < n - 1) store_for_host(distinct_mirror + i, 1);
   unique_ptr[i] = 0;
   if (unique_ptr_mirror) store_for_host(unique_ptr_mirror + i, 0);
+}
+
+static bool is_few(int64_t N, int64_t B) {
+  return N <= (B == 1 ? kFewOfOneBatch : kFewKeys) && B <= kFewBatches;
 }
 
 static int check_unique_args(const int64_t* seeds, const int64_t* seeds_ptr,
@@ -1756,7 +1815,7 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
     return GS_OK;
   }
   const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
-  if (N <= (B == 1 ? kFewOfOneBatch : kFewKeys) && B <= kFewBatches) {
+  if (is_few(N, B)) {
     GS_LAUNCH("unique_few", s,
               unique_few_kernel<<<dim3((unsigned)(N / kFewBinKeys + B)), dim3(kFewThreads), 0, s>>>(
                   k, N, w.batch, w.flat_ptr, w.group_batch, w.groups, w.etile_batch, w.etiles,
@@ -1823,7 +1882,7 @@ static int launch_fill_relabel(const gs::Keys& k, const gs::UniqueWs& w, int64_t
   const FillArgs f{w.flat_ptr, w.group_batch, N, out_unique};
   const LabelArgs l{w.etile_batch, w.first, w.unique_ptr, by_indptr ? nullptr : edge_col,
                     by_indptr ? col_indptr : nullptr, out_row, out_col, tn.remap,
-                    col_prefilled && by_indptr ? 1 : 0};
+                    col_prefilled && by_indptr ? 1 : 0, !is_few(N, k.B)};
   const unsigned label_blocks =
       label ? (unsigned)grid_for_units(ceil_div(k.E, kRelabelTile), tn.remap) : 0u;
   if (fill && label) {

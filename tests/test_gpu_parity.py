@@ -453,6 +453,54 @@ def test_unique_relabel_many_tiny_batches(B):
                 orc.unique_relabel(seeds, rows, sp, rp))
 
 
+@pytest.mark.parametrize("kind", ["one id", "runs", "a tile apart", "hubs", "equal tags"])
+@pytest.mark.parametrize("B,n", [(1, 65_537), (1, 69_632), (1, 69_631), (3, 80_001), (20, 120_000)])
+def test_unique_relabel_of_repeats_inside_a_tile(B, n, kind):
+    """Ids that repeat inside a tile of 4096 keys, all of it, next to each other, across the
+    tile's border, or with others that share their low 32 bits; seeds among the repeats, so that
+    column labels go by them too.  Tiles that are full, that hold one key, that end a batch."""
+    rng = np.random.default_rng(n + len(kind))
+    keys = rng.integers(0, n, size=n)
+    if kind == "one id":
+        keys[:] = 2**32 - 2
+    elif kind == "runs":
+        keys = np.repeat(rng.integers(0, n, size=n // 7 + 1), 7)[:n]
+    elif kind == "a tile apart":
+        keys = np.tile(rng.permutation(n)[:4096], n // 4096 + 1)[:n]
+    elif kind == "hubs":
+        hub = rng.random(n) < 0.3
+        keys[hub] = rng.integers(0, 20, size=int(hub.sum()))
+    else:
+        keys = rng.integers(0, 300, size=n) + 2**32 * rng.integers(0, 3, size=n) * (rng.random(n) < 0.1)
+    S = 700 * B
+    seeds, rows = keys[:S], keys[S:]
+    sp = np.arange(B + 1) * 700
+    rp = np.concatenate([[0], np.sort(rng.integers(0, n - S + 1, size=B - 1)), [n - S]])
+    col = np.concatenate([rng.integers(sp[b], sp[b + 1], size=rp[b + 1] - rp[b]) for b in range(B)])
+    col = np.sort(col)
+    indptr = np.searchsorted(col, np.arange(S + 1))
+    batches = (T(sp), T(rp)) if B > 1 else (None, None)
+    want = orc.unique_relabel(seeds, rows, *((sp, rp) if B > 1 else (None, None)), col)
+    assert_same(capi.unique_relabel(T(seeds), T(rows), *batches, T(col)), want)
+    assert_same(capi.unique_relabel(T(seeds), T(rows), *batches, col_indptr=T(indptr), fused=False), want)
+
+
+@pytest.mark.parametrize("n,meet", [(70_000, 2900), (70_000, 8193), (100_000, 30_000)])
+def test_unique_relabel_of_ids_that_meet_in_one_bucket(n, meet):
+    """Distinct ids, and a few thousand repeats far apart, whose hash puts them in one bucket:
+    more than its table is sure to hold, and more than its region."""
+    rng = np.random.default_rng(meet)
+    pool = np.arange(100 * meet, dtype=np.uint64)
+    pool = pool[(pool * np.uint64(0x9E3779B97F4A7C15) >> np.uint64(32)) & np.uint64(0xFFFFFFFF) < 2**26]
+    keys = rng.permutation(10**7)[:n]
+    at = rng.permutation(n)[:meet]
+    keys[at] = np.resize(pool[:max(1000, pool.size)].astype(np.int64), meet)
+    S = 500
+    col = rng.integers(0, S, size=n - S)
+    assert_same(capi.unique_relabel(T(keys[:S]), T(keys[S:]), edge_col=T(col)),
+                orc.unique_relabel(keys[:S], keys[S:], edge_col=col))
+
+
 def test_unique_relabel_one_huge_batch():
     """More keys in one batch than its buckets can take at the usual size: every
     bucket is deduplicated in global memory."""
