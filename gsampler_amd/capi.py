@@ -55,6 +55,8 @@ SIGNATURES = {
     "gs_csc_col_sample_uniform_fill_i32": (_int, [_p, _i64, _p, _p, _i64, _i64, _int,
                                                   _int, _u64, _u64, _p, _p, _p, _p, _p,
                                                   _p, _i64, _p]),
+    "gs_csc_col_sample_uniform_fill_rows32": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _int, _u64,
+                                                     _u64, _p, _p, _p, _p, _p, _i64, _p]),
     "gs_unique_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "gs_unique_count": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _sz, _p]),
     "gs_unique_fill": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _sz, _p]),
@@ -73,6 +75,11 @@ SIGNATURES = {
     "gs_batch_seeds_distinct": (_int, [_p, _p, _p, _p, _i64, _p, _p]),
     "gs_unique_count_distinct": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _sz,
                                         _p]),
+    "gs_unique_count_distinct_rows32": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p,
+                                               _sz, _p]),
+    "gs_unique_fill_rows32": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _sz, _p]),
+    "gs_unique_fill_relabel_rows32": (_int, [_p, _p, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _p,
+                                             _p, _int, _p, _sz, _p]),
     "gs_layer_max_positions": (_i64, []),
     "gs_layer_workspace_bytes": (_sz, [_i64, _int]),
     "gs_layer_begin": (_int, [_i64, _int, _p, _sz, _p]),
@@ -137,6 +144,8 @@ SIGNATURES = {
                                        _p]),
     "gs_weight_cdf_workspace_bytes": (_sz, [_i64, _i64]),
     "gs_weight_cdf_build": (_int, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _sz, _p]),
+    "gs_csc_col_sample_weighted_fill_rows32": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _int, _u64,
+                                                      _u64, _p, _p, _p, _p, _p, _i64, _p]),
     "gs_csc_col_sample_weighted_fill": (_int, [_p, _i64, _p, _p, _p, _p, _i64, _i64, _int, _u64,
                                                _u64, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "gs_weighted_key_probe": (_int, [_u64, _u64, _u64, _u64, C.c_float, _u64, _p, _p]),
@@ -382,7 +391,7 @@ def col_slice_values(indptr, column_ids, sub_indptr, values):
 
 def sample_uniform(indptr, indices, column_ids, fanout, replace=False,
                    algo=ALGO_AUTO, seed=7777, call_id=0, with_coo=True, col_batch_ptr=None,
-                   spans=True):
+                   spans=True, rows32=False):
     """Uniform per-column sampling, fused with the slice when column_ids is given.
 
     `indices` may be the matrix's int32 copy of the row ids (same outputs).
@@ -390,8 +399,9 @@ def sample_uniform(indptr, indices, column_ids, fanout, replace=False,
     every column's place inside its batch instead of its place in the call.
     `spans`: the count pass leaves every column's start and degree for the fill
     pass, which then does not look the column pointer up again (same outputs).
+    `rows32`: sub_indices are int32 and there is no select_index.
 
-    -> (sub_indptr, coo_col | None, sub_indices, select_index)
+    -> (sub_indptr, coo_col | None, sub_indices, select_index | None)
     """
     indptr = _i64t(indptr, "indptr")
     fill = lib().gs_csc_col_sample_uniform_fill
@@ -413,9 +423,23 @@ def sample_uniform(indptr, indices, column_ids, fanout, replace=False,
     sub_indptr = col_count(indptr, column_ids, fanout, replace, n, count, col_span)
     bound = n * fanout                       # no column yields more than fanout edges
     size = bound if bound <= _BOUND_LIMIT else count.get()
+    out_col = torch.empty(size, dtype=torch.int64, device=dev) if with_coo else None
+    if rows32:
+        if algo != ALGO_AUTO:
+            raise ValueError("sample_uniform: rows32 goes with ALGO_AUTO")
+        out_idx = torch.empty(size, dtype=torch.int32, device=dev)
+        wide = _ptr(indices) if indices.dtype == torch.int64 else None
+        narrow = _ptr(indices) if indices.dtype == torch.int32 else None
+        if size > 0:
+            check(lib().gs_csc_col_sample_uniform_fill_rows32(
+                _ptr(indptr), num_cols, wide, narrow, _ptr(column_ids), n, fanout, int(replace),
+                seed, call_id, sub_indptr.data_ptr(), _ptr(col_span), _ptr(out_col),
+                out_idx.data_ptr(), _ptr(col_batch_ptr),
+                col_batch_ptr.numel() - 1 if col_batch_ptr is not None else 0, _stream()))
+        nnz = count.get()
+        return sub_indptr, out_col[:nnz] if with_coo else None, out_idx[:nnz], None
     out_idx = torch.empty(size, dtype=torch.int64, device=dev)
     out_sel = torch.empty(size, dtype=torch.int64, device=dev)
-    out_col = torch.empty(size, dtype=torch.int64, device=dev) if with_coo else None
     if size > 0:
         check(fill(
             _ptr(indptr), num_cols, _ptr(indices), _ptr(column_ids), n, fanout,
@@ -429,6 +453,7 @@ def sample_uniform(indptr, indices, column_ids, fanout, replace=False,
 def unique_relabel(seeds, rows, seeds_ptr=None, rows_ptr=None, edge_col=None,
                    want_row=True, want_col=True, col_indptr=None, fused=True, out_col=None):
     """First-occurrence unique of seeds_b ++ rows_b per batch, plus relabel.
+    `rows` may be int32, as a sampler left them (rows32).
 
     The column of an edge comes from `edge_col` (a position into `seeds` per
     edge) or, for edges grouped by column, from `col_indptr` (len(seeds) + 1).
@@ -440,7 +465,9 @@ def unique_relabel(seeds, rows, seeds_ptr=None, rows_ptr=None, edge_col=None,
 
     -> (unique, unique_ptr, out_row | None, out_col | None)
     """
-    seeds, rows = _i64t(seeds, "seeds"), _i64t(rows, "rows")
+    seeds = _i64t(seeds, "seeds")
+    rows32 = rows.dtype == torch.int32 and rows.is_cuda
+    rows = rows.contiguous() if rows32 else _i64t(rows, "rows")
     dev = seeds.device
     S, E = seeds.numel(), rows.numel()
     if seeds_ptr is not None:
@@ -454,9 +481,14 @@ def unique_relabel(seeds, rows, seeds_ptr=None, rows_ptr=None, edge_col=None,
     sp = seeds_ptr.data_ptr() if seeds_ptr is not None else None
     rp = rows_ptr.data_ptr() if rows_ptr is not None else None
     count = _Count(B + 1) if B + 1 <= _Count._WIDTH else None
-    check(l.gs_unique_count(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
-                            unique_ptr.data_ptr(), count.mirror() if count else None,
-                            ws.data_ptr(), ws.numel(), _stream()))
+    mirror = count.mirror() if count else None
+    if rows32:
+        check(l.gs_unique_count_distinct_rows32(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
+                                                unique_ptr.data_ptr(), mirror, None,
+                                                ws.data_ptr(), ws.numel(), _stream()))
+    else:
+        check(l.gs_unique_count(_ptr(seeds), sp, S, _ptr(rows), rp, E, B, unique_ptr.data_ptr(),
+                                mirror, ws.data_ptr(), ws.numel(), _stream()))
     count = count.arm() if count else _Fetched(unique_ptr)
     size = S + E if S + E <= _BOUND_LIMIT else count.get()   # U <= S + E
     unique = torch.empty(size, dtype=torch.int64, device=dev)
@@ -482,14 +514,15 @@ def unique_relabel(seeds, rows, seeds_ptr=None, rows_ptr=None, edge_col=None,
             raise ValueError(f"unique_relabel: col_indptr has {col_indptr.numel()} entries "
                              f"for {S} seeds")
     if (want_row or want_col) and fused:
-        check(l.gs_unique_fill_relabel(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
-                                       unique_ptr.data_ptr(), _ptr(unique), _ptr(edge_col),
-                                       _ptr(col_indptr), _ptr(out_row), _ptr(out_col), prefilled,
-                                       ws.data_ptr(), ws.numel(), _stream()))
+        fill_relabel = l.gs_unique_fill_relabel_rows32 if rows32 else l.gs_unique_fill_relabel
+        check(fill_relabel(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
+                           unique_ptr.data_ptr(), _ptr(unique), _ptr(edge_col),
+                           _ptr(col_indptr), _ptr(out_row), _ptr(out_col), prefilled,
+                           ws.data_ptr(), ws.numel(), _stream()))
     else:
-        check(l.gs_unique_fill(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
-                               unique_ptr.data_ptr(), _ptr(unique), ws.data_ptr(),
-                               ws.numel(), _stream()))
+        fill = l.gs_unique_fill_rows32 if rows32 else l.gs_unique_fill
+        check(fill(_ptr(seeds), sp, S, _ptr(rows), rp, E, B, unique_ptr.data_ptr(), _ptr(unique),
+                   ws.data_ptr(), ws.numel(), _stream()))
         if want_row or want_col:
             check(l.gs_unique_relabel(_ptr(seeds), sp, S, _ptr(rows), rp, E, B,
                                       _ptr(edge_col), _ptr(col_indptr), _ptr(out_row),
@@ -936,7 +969,7 @@ def sample_weighted(indptr, indices, probs, column_ids, fanout, replace=False, s
 
 
 def _sample_weighted_cdf(indptr, indices, cdf, column_ids, fanout, replace, seed, call_id,
-                         with_coo, col_batch_ptr=None, spans=True):
+                         with_coo, col_batch_ptr=None, spans=True, rows32=False):
     num_cols = indptr.numel() - 1
     dev = indptr.device
     if column_ids is not None:
@@ -949,7 +982,17 @@ def _sample_weighted_cdf(indptr, indices, cdf, column_ids, fanout, replace, seed
     sub_indptr = col_count(indptr, column_ids, fanout, replace, n, count, col_span)
     bound = n * fanout
     size = bound if bound <= _BOUND_LIMIT else count.get()
-    out_idx = torch.empty(size, dtype=torch.int64, device=dev)
+    out_idx = torch.empty(size, dtype=torch.int32 if rows32 else torch.int64, device=dev)
+    if rows32:
+        out_col = torch.empty(size, dtype=torch.int64, device=dev) if with_coo else None
+        if size > 0:
+            check(lib().gs_csc_col_sample_weighted_fill_rows32(
+                _ptr(indptr), num_cols, _ptr(indices), cdf.data_ptr(), _ptr(column_ids), n, fanout,
+                int(replace), seed, call_id, sub_indptr.data_ptr(), _ptr(col_span), _ptr(out_col),
+                out_idx.data_ptr(), _ptr(col_batch_ptr),
+                col_batch_ptr.numel() - 1 if col_batch_ptr is not None else 0, _stream()))
+        nnz = count.get()
+        return sub_indptr, out_col[:nnz] if with_coo else None, out_idx[:nnz], None
     out_sel = torch.empty(size, dtype=torch.int64, device=dev)
     out_col = torch.empty(size, dtype=torch.int64, device=dev) if with_coo else None
     if size > 0:

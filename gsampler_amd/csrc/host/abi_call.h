@@ -105,6 +105,10 @@ inline torch::Tensor new_ids(int64_t n, const torch::Tensor& like) {
   return torch::empty({n}, device_options(like).dtype(torch::kInt64));
 }
 
+inline torch::Tensor new_ids32(int64_t n, const torch::Tensor& like) {
+  return torch::empty({n}, device_options(like).dtype(torch::kInt32));
+}
+
 inline torch::Tensor new_workspace(size_t bytes, const torch::Tensor& like) {
   return torch::empty({(int64_t)(bytes > 0 ? bytes : 1)},
                       device_options(like).dtype(torch::kUInt8));
@@ -396,7 +400,8 @@ class EdgeCount {
     // batch, which is the column's label in the batch's block while the batch's
     // seeds are distinct (the relabel pass then has nothing to do on that side)
     torch::Tensor col_labels;
-    bool no_select = false;  // set by a caller that has no use for the edges' positions
+    bool no_select = false;  // set by a caller that has no use for the edges' positions,
+    // and that takes row ids of 32 bits where the matrix and the call allow them
   };
   static Hint& hint() {
     static thread_local Hint h;

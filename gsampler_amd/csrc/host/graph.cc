@@ -297,10 +297,11 @@ MajorResult major_sample_uniform(const Compressed& m,
   count.arm(r.indptr);
   const int64_t bound = n * fanout;
   const int64_t size = bound <= kBoundLimit ? bound : count.get();
-  r.minor_ids = new_ids(size, m.indptr);
   // (the reservoir algorithm keeps its slots in the array of positions)
   const RandomState& rs = random_state();
   const bool no_select = EdgeCount::hint().no_select && fanout <= 64 && (replace || rs.algo != GS_ALGO_RESERVOIR);
+  const bool rows32 = no_select && !with_coo && m.minor_ids_fit_32();
+  r.minor_ids = rows32 ? new_ids32(size, m.indptr) : new_ids(size, m.indptr);
   if (!no_select) r.select = new_ids(size, m.indptr);
   if (with_coo) r.major_ids = new_ids(size, m.indptr);
   // a super-batched caller that asked for no coordinate form gets the columns'
@@ -313,7 +314,13 @@ MajorResult major_sample_uniform(const Compressed& m,
   const int64_t col_batches = label_cols ? hint.col_bptr.numel() - 1 : 0;
   const torch::Tensor narrow = m.narrow_indices();
   const uint64_t call = call_id.has_value() ? *call_id : next_call_id();
-  if (narrow.defined()) {
+  if (rows32) {
+    GS_CALL(gs_csc_col_sample_uniform_fill_rows32(
+        cptr(m.indptr), num_major, cptr(m.indices),
+        narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr, fused ? cptr(picked) : nullptr, n,
+        fanout, replace ? 1 : 0, rs.seed, call, cptr(r.indptr), cptr(col_span), out_col,
+        r.minor_ids.data_ptr<int32_t>(), col_batch_ptr, col_batches, cur_stream()));
+  } else if (narrow.defined()) {
     GS_CALL(gs_csc_col_sample_uniform_fill_i32(
         cptr(m.indptr), num_major, narrow.data_ptr<int32_t>(),
         fused ? cptr(picked) : nullptr, n, fanout, replace ? 1 : 0, (int)rs.algo,

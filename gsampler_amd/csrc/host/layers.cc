@@ -7,7 +7,8 @@
 // once, at the end, for all offsets.  A layer whose bound has grown too large for
 // that waits for the one before it first; large layers run on the count / fill /
 // unique kernels, with the edges' positions in the matrix left out (nobody asked
-// for them) and the columns' labels left by the sampler.
+// for them), the columns' labels left by the sampler, and the row ids, which end with
+// the layer, 32 bits wide where the matrix's are.
 #include "abi_call.h"
 #include "graph.h"
 
@@ -56,32 +57,39 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
   l.edge_ptr = EdgeCount::hint().edge_bptr;
   if (!l.edge_ptr.defined()) l.edge_ptr = r.indptr.index_select(0, col_bptr);
   const torch::Tensor& rows = r.minor_ids;
+  const bool rows32 = rows.scalar_type() == torch::kInt32;
   const int64_t E = rows.numel();
   const torch::Tensor labels = EdgeCount::hint().col_labels;
   const bool prefilled = labels_wanted && labels.defined() && labels.numel() == E && E > 0;
   if (labels_wanted) {
-    l.row = new_ids(E, rows);
-    l.col = prefilled ? labels : new_ids(E, rows);
+    l.row = new_ids(E, cols);
+    l.col = prefilled ? labels : new_ids(E, cols);
   }
-  torch::Tensor ws = new_workspace(gs_unique_workspace_bytes(S, E, B), rows);
-  l.frontier_ptr = new_ids(B + 1, rows);
+  torch::Tensor ws = new_workspace(gs_unique_workspace_bytes(S, E, B), cols);
+  l.frontier_ptr = new_ids(B + 1, cols);
   int64_t* distinct = PinnedWords::take((size_t)B);
   int64_t* mirror = OffsetMirror::reserve(l.frontier_ptr);
-  GS_CALL(gs_unique_count_distinct(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E,
-                                   B, mptr(l.frontier_ptr), mirror, distinct, ws.data_ptr(),
-                                   ws.numel(), cur_stream()));
-  OffsetMirror::arm(l.frontier_ptr);
-  const int64_t bound = S + E <= kBoundLimit ? S + E : OffsetMirror::values(l.frontier_ptr).back();
-  torch::Tensor frontier = new_ids(bound, rows);
-  if (labels_wanted)
-    GS_CALL(gs_unique_fill_relabel(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E,
-                                   B, cptr(l.frontier_ptr), mptr(frontier), nullptr,
-                                   cptr(r.indptr), mptr(l.row), mptr(l.col), prefilled ? 1 : 0,
-                                   ws.data_ptr(), ws.numel(), cur_stream()));
-  else
-    GS_CALL(gs_unique_fill(cptr(cols), cptr(col_bptr), S, cptr(rows), cptr(l.edge_ptr), E, B,
-                           cptr(l.frontier_ptr), mptr(frontier), ws.data_ptr(), ws.numel(),
+  // the same calls for either width of the row ids
+  auto calls = [&](auto* row_ids, auto count, auto fill, auto fill_relabel) {
+    GS_CALL(count(cptr(cols), cptr(col_bptr), S, row_ids, cptr(l.edge_ptr), E, B,
+                  mptr(l.frontier_ptr), mirror, distinct, ws.data_ptr(), ws.numel(), cur_stream()));
+    OffsetMirror::arm(l.frontier_ptr);
+    const int64_t bound = S + E <= kBoundLimit ? S + E : OffsetMirror::values(l.frontier_ptr).back();
+    l.frontier = new_ids(bound, cols);
+    if (labels_wanted)
+      GS_CALL(fill_relabel(cptr(cols), cptr(col_bptr), S, row_ids, cptr(l.edge_ptr), E, B,
+                           cptr(l.frontier_ptr), mptr(l.frontier), nullptr, cptr(r.indptr),
+                           mptr(l.row), mptr(l.col), prefilled ? 1 : 0, ws.data_ptr(), ws.numel(),
                            cur_stream()));
+    else
+      GS_CALL(fill(cptr(cols), cptr(col_bptr), S, row_ids, cptr(l.edge_ptr), E, B,
+                   cptr(l.frontier_ptr), mptr(l.frontier), ws.data_ptr(), ws.numel(), cur_stream()));
+  };
+  if (rows32)
+    calls(E > 0 ? rows.data_ptr<int32_t>() : nullptr, gs_unique_count_distinct_rows32,
+          gs_unique_fill_rows32, gs_unique_fill_relabel_rows32);
+  else
+    calls(cptr(rows), gs_unique_count_distinct, gs_unique_fill, gs_unique_fill_relabel);
   idle();
   l.e_off = OffsetMirror::values(l.edge_ptr);
   l.f_off = OffsetMirror::values(l.frontier_ptr);
@@ -89,7 +97,7 @@ Graph::Layer Graph::large_layer(const torch::Tensor& cols, const torch::Tensor& 
   PinnedWords::arrived();
   l.distinct.assign((size_t)B, 1);
   for (int64_t b = 0; b < B; ++b) l.distinct[(size_t)b] = distinct[b] != 0;
-  l.frontier = frontier.narrow(0, 0, l.f_off.back());
+  l.frontier = l.frontier.narrow(0, 0, l.f_off.back());
   return l;
 }
 

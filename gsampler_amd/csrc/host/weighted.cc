@@ -104,9 +104,10 @@ MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
   count.arm(r.indptr);
   const int64_t bound = n * fanout;
   const int64_t size = bound <= kBoundLimit ? bound : count.get();
-  r.minor_ids = new_ids(size, m.indptr);
   EdgeCount::Hint& hint = EdgeCount::hint();
   const bool no_select = hint.no_select;
+  const bool rows32 = no_select && !with_coo && m.minor_ids_fit_32();
+  r.minor_ids = rows32 ? new_ids32(size, m.indptr) : new_ids(size, m.indptr);
   if (!no_select) r.select = new_ids(size, m.indptr);
   if (with_coo) r.major_ids = new_ids(size, m.indptr);
   // (as in the uniform sampler: a super-batched caller without a coordinate form
@@ -114,14 +115,20 @@ MajorResult major_sample_weighted(const Compressed& m, const torch::Tensor& cdf,
   const bool label_cols = !with_coo && hint.col_bptr.defined();
   torch::Tensor col_labels = label_cols ? new_ids(size, m.indptr) : torch::Tensor();
   const RandomState& rs = random_state();
-  GS_CALL(gs_csc_col_sample_weighted_fill(
-      cptr(m.indptr), num_major, cptr(m.indices), nullptr, cptr(cdf), cptr(picked), n,
-      fanout, replace ? 1 : 0, rs.seed, call_id.has_value() ? *call_id : next_call_id(),
-      cptr(r.indptr), cptr(col_span),
-      nullptr, nullptr,
-      with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr,
-      mptr(r.minor_ids), mptr(r.select), label_cols ? cptr(hint.col_bptr) : nullptr,
-      label_cols ? hint.col_bptr.numel() - 1 : 0, cur_stream()));
+  const uint64_t call = call_id.has_value() ? *call_id : next_call_id();
+  int64_t* out_col = with_coo ? mptr(r.major_ids) : label_cols ? mptr(col_labels) : nullptr;
+  const int64_t* col_batch_ptr = label_cols ? cptr(hint.col_bptr) : nullptr;
+  const int64_t col_batches = label_cols ? hint.col_bptr.numel() - 1 : 0;
+  if (rows32)
+    GS_CALL(gs_csc_col_sample_weighted_fill_rows32(
+        cptr(m.indptr), num_major, cptr(m.indices), cptr(cdf), cptr(picked), n, fanout,
+        replace ? 1 : 0, rs.seed, call, cptr(r.indptr), cptr(col_span), out_col,
+        r.minor_ids.data_ptr<int32_t>(), col_batch_ptr, col_batches, cur_stream()));
+  else
+    GS_CALL(gs_csc_col_sample_weighted_fill(
+        cptr(m.indptr), num_major, cptr(m.indices), nullptr, cptr(cdf), cptr(picked), n, fanout,
+        replace ? 1 : 0, rs.seed, call, cptr(r.indptr), cptr(col_span), nullptr, nullptr, out_col,
+        mptr(r.minor_ids), mptr(r.select), col_batch_ptr, col_batches, cur_stream()));
   const int64_t nnz = count.get();
   if (label_cols) hint.col_labels = col_labels.narrow(0, 0, nnz);
   r.minor_ids = r.minor_ids.narrow(0, 0, nnz);

@@ -87,13 +87,13 @@ __device__ __forceinline__ void sample_column_generic(
 // 32 nothing is stored.
 constexpr int kProbeHash = 1, kProbeNoExchange = 2, kProbeNoIndptr = 4, kProbeNoIndices = 8,
               kProbeOneStore = 16, kProbeNoStore = 32;
-template <typename IdxT, int kProbe = 0>
+template <typename IdxT, typename OutT, int kProbe = 0>
 __global__ __launch_bounds__(kBlock) void sample_uniform_packed_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols,
     const IdxT* __restrict__ indices, const int64_t* __restrict__ column_ids,
     int64_t num_items, int fanout, int cols_per_wave, int replace, PhiloxKey key,
     const int64_t* __restrict__ sub_indptr, int64_t* __restrict__ out_coo_col,
-    int64_t* __restrict__ out_indices, int64_t* __restrict__ out_select,
+    OutT* __restrict__ out_indices, int64_t* __restrict__ out_select,
     ColumnLabels labels, const int64_t* __restrict__ col_span, int64_t probe_degree = 0) {
   const int wave_lane = threadIdx.x & (kWave - 1);
   const int group = wave_lane / fanout;
@@ -142,10 +142,10 @@ __global__ __launch_bounds__(kBlock) void sample_uniform_packed_kernel(
   const int64_t v = (indices && !(kProbe & kProbeNoIndices)) ? (int64_t)indices[p] : p;
   if (kProbe & kProbeNoStore) {
     // keep the pick (and the row id behind it) live without a store that happens
-    if (v == -7777) out_indices[0] = p;  // ids are not negative; the compiler cannot know
+    if (v == -7777) out_indices[0] = (OutT)p;  // ids are not negative; the compiler cannot know
     return;
   }
-  out_indices[out_start + lane] = v;
+  out_indices[out_start + lane] = (OutT)v;
   if (kProbe & kProbeOneStore) return;
   if (out_select) out_select[out_start + lane] = p;
   if (out_coo_col) out_coo_col[out_start + lane] = col_label;
@@ -192,12 +192,12 @@ static int launch_sample_strided(const int64_t* indptr, int64_t num_cols, const 
 }  // namespace gs
 
 namespace gs {
-template <typename IdxT>
+template <typename IdxT, typename OutT>
 static int sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const IdxT* indices,
                                const int64_t* column_ids, int64_t num_items, int64_t fanout,
                                int replace, int algo, uint64_t seed, uint64_t call_id,
                                const int64_t* sub_indptr, const int64_t* col_span,
-                               int64_t* out_coo_col, int64_t* out_indices,
+                               int64_t* out_coo_col, OutT* out_indices,
                                int64_t* out_select, const int64_t* col_batch_ptr,
                                int64_t num_col_batches, gs_stream_t stream) {
   GS_REQUIRE(num_items >= 0 && num_cols >= 0, "sample_uniform: negative size");
@@ -226,13 +226,18 @@ static int sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const Id
     const int cols_per_wave = kWave / (int)fanout;
     const int64_t waves = ceil_div(num_items, cols_per_wave);
     GS_LAUNCH("sample_uniform", s,
-              sample_uniform_packed_kernel<IdxT><<<dim3((unsigned)(ceil_div(ceil_div(waves * kWave, kBlock), 8) * 8)),
-                                                   dim3(kBlock), 0, s>>>(
+              (sample_uniform_packed_kernel<IdxT, OutT>)
+              <<<dim3((unsigned)(ceil_div(ceil_div(waves * kWave, kBlock), 8) * 8)), dim3(kBlock), 0, s>>>(
                   indptr, num_cols, indices, column_ids, num_items, (int)fanout, cols_per_wave,
                   replace, key, sub_indptr, out_coo_col, out_indices, out_select, labels,
                   col_span));
     return GS_OK;
   }
+  if constexpr (sizeof(OutT) != sizeof(int64_t)) {
+    set_error("sample_uniform: 32-bit row ids need a fanout of at most %d, got %lld", kWave,
+              (long long)fanout);
+    return GS_ERR_INVALID;
+  } else {
   // (the reservoir keeps its slots there)
   GS_REQUIRE(out_select, "sample_uniform: this algorithm and fanout need out_select");
 #define GS_SAMPLE_ARGS                                                          \
@@ -243,6 +248,7 @@ static int sample_uniform_fill(const int64_t* indptr, int64_t num_cols, const Id
   if (fanout <= 32) return launch_sample_strided<32, IdxT>(GS_SAMPLE_ARGS);
   return launch_sample_strided<64, IdxT>(GS_SAMPLE_ARGS);
 #undef GS_SAMPLE_ARGS
+  }
 }
 }  // namespace gs
 
@@ -252,7 +258,7 @@ extern "C" int gs_csc_col_sample_uniform_fill(
     int algo, uint64_t seed, uint64_t call_id, const int64_t* sub_indptr,
     const int64_t* col_span, int64_t* out_coo_col, int64_t* out_indices, int64_t* out_select,
     const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream) {
-  return gs::sample_uniform_fill<int64_t>(indptr, num_cols, indices, column_ids, num_items,
+  return gs::sample_uniform_fill<int64_t, int64_t>(indptr, num_cols, indices, column_ids, num_items,
                                           fanout, replace, algo, seed, call_id, sub_indptr,
                                           col_span, out_coo_col, out_indices, out_select, col_batch_ptr,
                                           num_col_batches, stream);
@@ -265,10 +271,29 @@ extern "C" int gs_csc_col_sample_uniform_fill_i32(
     const int64_t* col_span, int64_t* out_coo_col, int64_t* out_indices, int64_t* out_select,
     const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream) {
   GS_REQUIRE(indices32 != nullptr, "sample_uniform_i32: null indices");
-  return gs::sample_uniform_fill<int32_t>(indptr, num_cols, indices32, column_ids, num_items,
+  return gs::sample_uniform_fill<int32_t, int64_t>(indptr, num_cols, indices32, column_ids, num_items,
                                           fanout, replace, algo, seed, call_id, sub_indptr,
                                           col_span, out_coo_col, out_indices, out_select, col_batch_ptr,
                                           num_col_batches, stream);
+}
+
+extern "C" int gs_csc_col_sample_uniform_fill_rows32(
+    const int64_t* indptr, int64_t num_cols, const int64_t* indices, const int32_t* indices32,
+    const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace,
+    uint64_t seed, uint64_t call_id, const int64_t* sub_indptr, const int64_t* col_span,
+    int64_t* out_coo_col, int32_t* out_rows, const int64_t* col_batch_ptr,
+    int64_t num_col_batches, gs_stream_t stream) {
+  GS_REQUIRE(indices || indices32, "sample_uniform_rows32: null indices");
+  GS_REQUIRE(fanout <= gs::kWave, "sample_uniform_rows32: fanout %lld is above 64", (long long)fanout);
+  if (indices32)
+    return gs::sample_uniform_fill<int32_t, int32_t>(
+        indptr, num_cols, indices32, column_ids, num_items, fanout, replace, GS_ALGO_AUTO, seed,
+        call_id, sub_indptr, col_span, out_coo_col, out_rows, nullptr, col_batch_ptr,
+        num_col_batches, stream);
+  return gs::sample_uniform_fill<int64_t, int32_t>(
+      indptr, num_cols, indices, column_ids, num_items, fanout, replace, GS_ALGO_AUTO, seed,
+      call_id, sub_indptr, col_span, out_coo_col, out_rows, nullptr, col_batch_ptr,
+      num_col_batches, stream);
 }
 
 // One launch of the packed sampler with parts switched off (`variant` = a sum of
@@ -296,7 +321,7 @@ extern "C" int gs_probe_sample_uniform(
 #define GS_PROBE_CASE(V)                                                                      \
   case V:                                                                                     \
     GS_LAUNCH("probe_sample_uniform", s,                                                      \
-              (sample_uniform_packed_kernel<int32_t, V>)<<<grid, dim3(kBlock), 0, s>>>(       \
+              (sample_uniform_packed_kernel<int32_t, int64_t, V>)<<<grid, dim3(kBlock), 0, s>>>(       \
                   indptr, num_cols, indices32, column_ids, num_items, (int)fanout,            \
                   cols_per_wave, 0, key, sub_indptr, out_coo_col, out_indices, out_select,    \
                   ColumnLabels{nullptr, 0}, col_span, probe_degree));                         \

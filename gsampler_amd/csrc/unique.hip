@@ -192,29 +192,76 @@ static UniqueWs carve_unique(void* ws, int64_t S, int64_t E, int64_t B) {
   return w;
 }
 
-// The caller's view of the keys.
-struct Keys {
-  const int64_t* seeds;
+// The caller's view of the keys: where the batches begin, and the keys themselves.  Row ids
+// that a sampler of this library has just written may be 32 bits wide.
+struct KeyPtrs {
   const int64_t* seeds_ptr;  // null: one batch
   int64_t S;
-  const int64_t* rows;
   const int64_t* rows_ptr;   // null: one batch
   int64_t E;
   int64_t B;
 };
+template <typename Row>
+struct Keys : KeyPtrs {
+  const int64_t* seeds;
+  const Row* rows;
+};
 
-__device__ __forceinline__ int64_t seeds_lo(const Keys& k, int64_t b) {
+__device__ __forceinline__ int64_t seeds_lo(const KeyPtrs& k, int64_t b) {
   return k.seeds_ptr ? k.seeds_ptr[b] : (b == 0 ? 0 : k.S);
 }
-__device__ __forceinline__ int64_t rows_lo(const Keys& k, int64_t b) {
+__device__ __forceinline__ int64_t rows_lo(const KeyPtrs& k, int64_t b) {
   return k.rows_ptr ? k.rows_ptr[b] : (b == 0 ? 0 : k.E);
 }
 
 // Key at position `local` of batch b (whose seeds are [s_lo, s_lo + ns)).
-__device__ __forceinline__ uint64_t key_at(const Keys& k, int64_t s_lo,
+template <typename Row>
+__device__ __forceinline__ uint64_t key_at(const Keys<Row>& k, int64_t s_lo,
                                            int64_t ns, int64_t r_lo,
                                            int64_t local) {
-  return (uint64_t)(local < ns ? k.seeds[s_lo + local] : k.rows[r_lo + local - ns]);
+  return (uint64_t)(local < ns ? k.seeds[s_lo + local] : (int64_t)k.rows[r_lo + local - ns]);
+}
+
+// Keys at `count` positions first + stride i of a batch, none at `end` or beyond (a position
+// there reads the key before `end`), all asked for before the first is looked at.  The
+// positions of a work-group or wavefront, `from` to `end`, are mostly rows alone or seeds
+// alone: where two arrays of different widths would need a branch around each load, and a
+// wait in it, that is asked once.
+template <int kCount, typename Row>
+__device__ __forceinline__ void keys_at(const Keys<Row>& k, int64_t s_lo, int64_t ns, int64_t r_lo,
+                                        int64_t from, int64_t end, int64_t first, int stride,
+                                        uint64_t* key) {
+  auto clamped = [&](int i) {
+    const int64_t l = first + (int64_t)i * stride;
+    return l < end ? l : end - 1;
+  };
+  if constexpr (sizeof(Row) == sizeof(int64_t)) {
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) {
+      const int64_t l = clamped(i);
+      key[i] = (uint64_t)*(l < ns ? k.seeds + (s_lo + l) : k.rows + (r_lo + l - ns));
+    }
+  } else if (from >= ns) {
+    Row r[kCount];
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) r[i] = k.rows[r_lo + clamped(i) - ns];
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) key[i] = (uint64_t)(int64_t)r[i];
+  } else if (end <= ns) {
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) key[i] = (uint64_t)k.seeds[s_lo + clamped(i)];
+  } else {  // both: from < ns < end
+    Row r[kCount];
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) {
+      const int64_t l = clamped(i);
+      key[i] = (uint64_t)k.seeds[s_lo + (l < ns ? l : ns - 1)];
+      r[i] = k.rows[r_lo + (l < ns ? 0 : l - ns)];
+    }
+#pragma unroll
+    for (int i = 0; i < kCount; ++i)
+      if (clamped(i) >= ns) key[i] = (uint64_t)(int64_t)r[i];
+  }
 }
 
 // Bucket of a key among the `buckets` of its batch: the high bits of the hash.
@@ -230,7 +277,7 @@ __device__ __forceinline__ uint32_t slot_hash(uint64_t key) {
 // The walk over the batches: where the keys, tiles and buckets of every batch
 // start.  Run by one whole work-group; the three offset arrays may live in LDS
 // or in global memory, `batch` (the records) may be null.
-__device__ __forceinline__ void walk_batches(const Keys& k, int64_t bucket_keys,
+__device__ __forceinline__ void walk_batches(const KeyPtrs& k, int64_t bucket_keys,
                                              BatchInfo* batch, int64_t* flat_ptr,
                                              int64_t* tile_ptr, int64_t* bucket_ptr,
                                              int64_t* region_ptr, int64_t* smem) {
@@ -284,7 +331,7 @@ struct UnitTables {
     return max_tiles + max_buckets + groups + 1 + etiles + 1;
   }
 };
-__device__ __forceinline__ void assign_unit(int64_t i, const Keys& k, int64_t N,
+__device__ __forceinline__ void assign_unit(int64_t i, const KeyPtrs& k, int64_t N,
                                             const int64_t* flat_ptr,
                                             const int64_t* tile_ptr,
                                             const int64_t* bucket_ptr,
@@ -344,7 +391,7 @@ __device__ __forceinline__ void zero_counters(int64_t* bucket_cur, int64_t max_b
 // leaves the records and offset arrays in global memory.
 constexpr int kPlanMaxBatches = 1024;
 __global__ __launch_bounds__(kBlock) void unique_plan_kernel(
-    Keys k, int64_t N, int64_t bucket_keys, BatchInfo* __restrict__ batch,
+    KeyPtrs k, int64_t N, int64_t bucket_keys, BatchInfo* __restrict__ batch,
     int64_t* __restrict__ flat_ptr, int64_t* __restrict__ tile_ptr,
     int64_t* __restrict__ bucket_ptr, int64_t* __restrict__ region_ptr,
     int64_t* __restrict__ bucket_cur, int64_t* __restrict__ ovf_cur,
@@ -371,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void unique_plan_kernel(
 
 // More batches than that: the walk by one work-group into global memory ...
 __global__ __launch_bounds__(kBlock) void unique_prep_kernel(
-    Keys k, int64_t bucket_keys, BatchInfo* __restrict__ batch,
+    KeyPtrs k, int64_t bucket_keys, BatchInfo* __restrict__ batch,
     int64_t* __restrict__ flat_ptr, int64_t* __restrict__ tile_ptr,
     int64_t* __restrict__ bucket_ptr, int64_t* __restrict__ region_ptr,
     int64_t* __restrict__ bucket_cur, int64_t max_buckets, int64_t* __restrict__ ovf_cur,
@@ -384,7 +431,7 @@ __global__ __launch_bounds__(kBlock) void unique_prep_kernel(
 
 // ... and the units from there in a launch of their own.
 __global__ __launch_bounds__(kBlock) void unique_units_kernel(
-    Keys k, int64_t N, const int64_t* __restrict__ flat_ptr,
+    KeyPtrs k, int64_t N, const int64_t* __restrict__ flat_ptr,
     const int64_t* __restrict__ tile_ptr, const int64_t* __restrict__ bucket_ptr,
     const int64_t* __restrict__ region_ptr, UnitTables u) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -409,7 +456,8 @@ __device__ __forceinline__ bool tile_info(int64_t tile,
   return true;
 }
 
-__device__ __forceinline__ uint64_t key_at(const Keys& k, const BatchInfo& b,
+template <typename Row>
+__device__ __forceinline__ uint64_t key_at(const Keys<Row>& k, const BatchInfo& b,
                                            int64_t local) {
   return key_at(k, b.s_lo, b.ns, b.r_lo, local);
 }
@@ -436,8 +484,9 @@ constexpr int kScatterItems = kPartTile / kScatterThreads;
 constexpr int kTileBits = 12;
 static_assert(kPartTile == 1 << kTileBits, "a position inside a tile takes kTileBits bits");
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;  // of a position that has no part in this
+template <typename Row>
 __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
-    Keys k, const int32_t* __restrict__ tile_batch,
+    Keys<Row> k, const int32_t* __restrict__ tile_batch,
     const BatchInfo* __restrict__ batch, int64_t* bucket_cur, int64_t* ovf_cur,
     uint64_t* __restrict__ packed, uint64_t* __restrict__ ovf_entry,
     int32_t* __restrict__ ovf_bucket, uint32_t* __restrict__ first, int64_t max_tiles,
@@ -467,15 +516,10 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
   }
   uint64_t full[kScatterItems];
   uint32_t key[kScatterItems], place[kScatterItems];
-#pragma unroll
-  for (int i = 0; i < kScatterItems; ++i) {
-    // All loads in flight before anything else: a position past the end reads
-    // the tile's last key instead of branching around the load (the compiler
-    // otherwise moves the first use of the key into that branch and waits
-    // there, one load at a time).
-    const int64_t l = t.begin + i * kScatterThreads + threadIdx.x;
-    full[i] = key_at(k, t.b, l < t.end ? l : t.end - 1);
-  }
+  // (no branch around a load: the compiler moves the first use of the key into that branch
+  // and waits there, one load at a time)
+  keys_at<kScatterItems>(k, t.b.s_lo, t.b.ns, t.b.r_lo, t.begin, t.end, t.begin + threadIdx.x,
+                         kScatterThreads, full);
   constexpr int kBins = kMaxBuckets / kScatterThreads;
 #pragma unroll
   for (int r = 0; r < kBins; ++r) {
@@ -603,9 +647,9 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
 // Whether two entries with the same upper half stand for the same key: always
 // when every key of the call fits that half; otherwise the keys themselves are
 // read back through the entries' positions and compared.
-template <bool kWide>
+template <bool kWide, typename Row>
 struct SameKey {
-  const Keys* k;
+  const Keys<Row>* k;
   const BatchInfo* b;
   __device__ __forceinline__ bool operator()(uint64_t a, uint64_t c) const {
     if (!kWide) return true;
@@ -737,15 +781,15 @@ struct BucketEntries {
   }
 };
 
-template <int kThreads, bool kWide>
+template <int kThreads, bool kWide, typename Row>
 __device__ __forceinline__ void dedup_bucket(
-    const Keys& k, const BatchInfo& info, int64_t n, const BucketEntries& entries,
+    const Keys<Row>& k, const BatchInfo& info, int64_t n, const BucketEntries& entries,
     uint64_t* spill, unsigned long long* pool_cur, uint32_t* __restrict__ first,
     uint64_t* tab, uint32_t* distinct_ptr, uint32_t* overflow_ptr,
     unsigned long long* pool_at) {
   uint32_t& distinct = *distinct_ptr;
   uint32_t& overflow = *overflow_ptr;
-  const SameKey<kWide> same{&k, &info};
+  const SameKey<kWide, Row> same{&k, &info};
   uint32_t* first_b = first + info.fb;
   // table of two slots per entry, a power of two, at most kLdsSlots
   uint32_t slots = 256;
@@ -842,9 +886,9 @@ __device__ __forceinline__ void dedup_bucket(
 // Everything else (oversize buckets, wide keys) goes through dedup_bucket.
 constexpr uint32_t kNoTag = 0xFFFFFFFFu;  // never a tag, see key_tag
 
-template <int kThreads>
-__global__ __launch_bounds__(kThreads) void unique_dedup_kernel(
-    Keys k, const int* __restrict__ wide_keys,
+template <int kThreads, typename Row>
+__global__ __launch_bounds__(kThreads, 8) void unique_dedup_kernel(
+    Keys<Row> k, const int* __restrict__ wide_keys,
     const int32_t* __restrict__ bucket_batch, const BatchInfo* __restrict__ batch,
     const int64_t* __restrict__ bucket_cur, const int64_t* __restrict__ bucket_base,
     const int32_t* __restrict__ bucket_cap, const int64_t* __restrict__ ovf_cur,
@@ -1177,8 +1221,9 @@ __device__ __forceinline__ uint32_t few_bin(uint64_t key, uint32_t bins) {
   return __umulhi((x ^ (x >> 8)) * 0x846CA68Bu, bins);
 }
 
+template <typename Row>
 __global__ __launch_bounds__(kFewThreads) void unique_few_kernel(
-    Keys k, int64_t N, BatchInfo* __restrict__ batch, int64_t* __restrict__ flat_ptr,
+    Keys<Row> k, int64_t N, BatchInfo* __restrict__ batch, int64_t* __restrict__ flat_ptr,
     int32_t* __restrict__ group_batch, int64_t groups, int32_t* __restrict__ etile_batch,
     int64_t etiles, uint32_t* __restrict__ first) {
   __shared__ uint64_t keys[kFewSlots];
@@ -1235,9 +1280,13 @@ __global__ __launch_bounds__(kFewThreads) void unique_few_kernel(
   ns = l_flat[b + 1] - l_rows[b + 1] - s_lo;
   uint32_t* first_b = first + fb;
   const uint32_t n32 = (uint32_t)n, ns32 = (uint32_t)ns;
-  const int64_t *seeds_b = k.seeds + s_lo, *rows_b = k.rows + (r_lo - ns);
-  auto key_of = [&](uint32_t p) {  // (one load from either array: no branch between the loads of a round)
-    return (uint64_t)(p < ns32 ? seeds_b : rows_b)[p];
+  const int64_t* const seeds_b = k.seeds + s_lo;
+  const Row* const rows_b = k.rows + (r_lo - ns);
+  auto key_of = [&](uint32_t p) {
+    if constexpr (sizeof(Row) == sizeof(int64_t))  // (one load from either array: no branch between the loads of a round)
+      return (uint64_t)(p < ns32 ? seeds_b : rows_b)[p];
+    else
+      return (uint64_t)(p < ns32 ? seeds_b[p] : (int64_t)rows_b[p]);
   };
   auto store = [&](uint32_t p, uint32_t f) { first_b[p] = f == p ? f | kFirstMark : f; };
   // the slot of a key: kFewSlots for the key that marks empty ones, more if there is none
@@ -1422,8 +1471,9 @@ struct FillArgs {
   int64_t* out_unique;
 };
 
+template <typename Row>
 __device__ __forceinline__ void fill_group(
-    int64_t group, const Keys& k, const int64_t* __restrict__ flat_ptr,
+    int64_t group, const Keys<Row>& k, const int64_t* __restrict__ flat_ptr,
     const int32_t* __restrict__ group_batch, const BatchInfo* __restrict__ batch,
     int64_t N, const RankWord* __restrict__ words,
     const int64_t* __restrict__ group_off, int64_t* __restrict__ out_unique) {
@@ -1457,7 +1507,10 @@ __device__ __forceinline__ void fill_group(
         const int64_t r = (int64_t)__shfl((long long)rows_before, i, kWave);
         const int64_t s = (int64_t)__shfl((long long)seeds_to, i, kWave);
         // a flat position: place among the seeds + rows before, or among the rows + seeds so far
-        key[j] = (uint64_t)*(p < r + s ? k.seeds + (p - r) : k.rows + (p - s));
+        if constexpr (sizeof(Row) == sizeof(int64_t))
+          key[j] = (uint64_t)*(p < r + s ? k.seeds + (p - r) : k.rows + (p - s));
+        else
+          key[j] = (uint64_t)(p < r + s ? k.seeds[p - r] : (int64_t)k.rows[p - s]);
       }
 #pragma unroll
       for (int j = 0; j < LaneBatches::kRows; ++j) store(j0 + j, key[j]);
@@ -1465,21 +1518,28 @@ __device__ __forceinline__ void fill_group(
     return;
   }
   uint64_t key[kWordsPerWave];
+  if (one_batch) {
+    const int64_t from = word0 * kWave - info.fb;
+    const int64_t to = from + kWordsPerWave * kWave < info.n ? from + kWordsPerWave * kWave : info.n;
+    keys_at<kWordsPerWave>(k, info.s_lo, info.ns, info.r_lo, from, to, from + lane, kWave, key);
+  } else {
 #pragma unroll
-  for (int j = 0; j < kWordsPerWave; ++j) {
-    const int64_t p = (word0 + j) * kWave + lane;
-    key[j] = 0;
-    if (p < N) {
-      if (!one_batch) info = batch[batch_in_span(flat_ptr, span, p)];
-      key[j] = key_at(k, info, p - info.fb);
+    for (int j = 0; j < kWordsPerWave; ++j) {
+      const int64_t p = (word0 + j) * kWave + lane;
+      key[j] = 0;
+      if (p < N) {
+        info = batch[batch_in_span(flat_ptr, span, p)];
+        key[j] = key_at(k, info, p - info.fb);
+      }
     }
   }
 #pragma unroll
   for (int j = 0; j < kWordsPerWave; ++j) store(j, key[j]);
 }
 
+template <typename Row>
 __global__ __launch_bounds__(kBlock) void unique_fill_kernel(
-    Keys k, FillArgs f, const BatchInfo* __restrict__ batch,
+    Keys<Row> k, FillArgs f, const BatchInfo* __restrict__ batch,
     const RankWord* __restrict__ words, const int64_t* __restrict__ group_off) {
   fill_group(blockIdx.x, k, f.flat_ptr, f.group_batch, batch, f.N, words, group_off,
              f.out_unique);
@@ -1591,7 +1651,7 @@ __device__ __forceinline__ uint32_t first_of(const uint32_t* __restrict__ first_
 
 template <bool kByIndptr>
 __device__ __forceinline__ void relabel_tile(
-    const Keys& k, const int32_t* __restrict__ etile_batch,
+    const KeyPtrs& k, const int32_t* __restrict__ etile_batch,
     const BatchInfo* __restrict__ batch, const uint32_t* __restrict__ first,
     const RankWord* __restrict__ words, const int64_t* __restrict__ group_off,
     const int64_t* __restrict__ unique_ptr, const int64_t* __restrict__ edge_col,
@@ -1703,7 +1763,7 @@ __device__ __forceinline__ void relabel_tile(
 
 template <bool kByIndptr>
 __global__ __launch_bounds__(kBlock) void unique_relabel_kernel(
-    Keys k, LabelArgs l, const BatchInfo* __restrict__ batch,
+    KeyPtrs k, LabelArgs l, const BatchInfo* __restrict__ batch,
     const RankWord* __restrict__ words, const int64_t* __restrict__ group_off) {
   relabel_tile<kByIndptr>(k, l.etile_batch, batch, l.first, words, group_off, l.unique_ptr,
                           l.edge_col, l.col_indptr, l.out_row, l.out_col, l.remap,
@@ -1714,9 +1774,9 @@ __global__ __launch_bounds__(kBlock) void unique_relabel_kernel(
 // tiles of edges, the rest write the frontier.  Neither reads what the other
 // writes; the short frontier work-groups fill the machine while the last
 // labelling ones drain.
-template <bool kByIndptr>
+template <bool kByIndptr, typename Row>
 __global__ __launch_bounds__(kBlock) void unique_fill_relabel_kernel(
-    Keys k, FillArgs f, LabelArgs l, unsigned label_blocks,
+    Keys<Row> k, FillArgs f, LabelArgs l, unsigned label_blocks,
     const BatchInfo* __restrict__ batch, const RankWord* __restrict__ words,
     const int64_t* __restrict__ group_off) {
   if (blockIdx.x < label_blocks)
@@ -1744,7 +1804,7 @@ static bool is_few(int64_t N, int64_t B) {
 }
 
 static int check_unique_args(const int64_t* seeds, const int64_t* seeds_ptr,
-                             int64_t S, const int64_t* rows,
+                             int64_t S, const void* rows,
                              const int64_t* rows_ptr, int64_t E, int64_t B) {
   GS_REQUIRE(S >= 0 && E >= 0, "unique: negative size");
   GS_REQUIRE(B >= 1, "unique: num_batches must be >= 1, got %lld", (long long)B);
@@ -1771,32 +1831,15 @@ static int check_workspace(const UniqueWs& w, const void* workspace,
 
 }  // namespace gs
 
-extern "C" {
+namespace gs {
 
-size_t gs_unique_workspace_bytes(int64_t num_seeds, int64_t num_rows_keys,
-                                 int64_t num_batches) {
-  if (num_seeds < 0 || num_rows_keys < 0 || num_batches < 1) return 0;
-  return gs::carve_unique(nullptr, num_seeds, num_rows_keys, num_batches).total;
-}
-
-int gs_unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
-                    int64_t num_seeds, const int64_t* rows,
-                    const int64_t* rows_ptr, int64_t num_rows_keys,
-                    int64_t num_batches, int64_t* unique_ptr,
-                    int64_t* unique_ptr_mirror, void* workspace,
-                    size_t workspace_bytes, gs_stream_t stream) {
-  return gs_unique_count_distinct(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
-                                  num_batches, unique_ptr, unique_ptr_mirror, nullptr, workspace,
-                                  workspace_bytes, stream);
-}
-
-int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
-                             int64_t num_seeds, const int64_t* rows,
+template <typename Row>
+static int unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
+                             int64_t num_seeds, const Row* rows,
                              const int64_t* rows_ptr, int64_t num_rows_keys,
                              int64_t num_batches, int64_t* unique_ptr,
                              int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
                              void* workspace, size_t workspace_bytes, gs_stream_t stream) {
-  using namespace gs;
   const int64_t S = num_seeds, E = num_rows_keys, B = num_batches;
   int rc = check_unique_args(seeds, seeds_ptr, S, rows, rows_ptr, E, B);
   if (rc != GS_OK) return rc;
@@ -1814,10 +1857,10 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
                                                           B + 1));
     return GS_OK;
   }
-  const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
+  const Keys<Row> k{{seeds_ptr, S, rows_ptr, E, B}, seeds, rows};
   if (is_few(N, B)) {
     GS_LAUNCH("unique_few", s,
-              unique_few_kernel<<<dim3((unsigned)(N / kFewBinKeys + B)), dim3(kFewThreads), 0, s>>>(
+              unique_few_kernel<Row><<<dim3((unsigned)(N / kFewBinKeys + B)), dim3(kFewThreads), 0, s>>>(
                   k, N, w.batch, w.flat_ptr, w.group_batch, w.groups, w.etile_batch, w.etiles,
                   w.first));
     GS_LAUNCH("unique_few_offsets", s,
@@ -1849,11 +1892,11 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
   }
   const dim3 tile_grid((unsigned)grid_for_units(w.max_tiles, tn.remap));
   GS_LAUNCH("unique_scatter", s,
-            unique_scatter_kernel<<<tile_grid, dim3(kScatterThreads), 0, s>>>(
+            unique_scatter_kernel<Row><<<tile_grid, dim3(kScatterThreads), 0, s>>>(
                 k, w.tile_batch, w.batch, w.bucket_cur, w.ovf_cur, w.packed, w.ovf_entry,
                 w.ovf_bucket, w.first, w.max_tiles, tn.remap, w.wide_keys));
   GS_LAUNCH("unique_dedup", s,
-            unique_dedup_kernel<512><<<dim3((unsigned)grid_for_units(w.max_buckets, tn.remap)),
+            (unique_dedup_kernel<512, Row>)<<<dim3((unsigned)grid_for_units(w.max_buckets, tn.remap)),
                                        dim3(512), 0, s>>>(
                 k, w.wide_keys, w.bucket_batch, w.batch, w.bucket_cur, w.bucket_base,
                 w.bucket_cap, w.ovf_cur, w.packed, w.ovf_entry, w.ovf_bucket, w.spill,
@@ -1869,11 +1912,11 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
 }
 
 // The launches behind gs_unique_fill, gs_unique_relabel and gs_unique_fill_relabel.
-static int launch_fill_relabel(const gs::Keys& k, const gs::UniqueWs& w, int64_t* out_unique,
+template <typename Row>
+static int launch_fill_relabel(const Keys<Row>& k, const UniqueWs& w, int64_t* out_unique,
                                const int64_t* edge_col, const int64_t* col_indptr,
                                int64_t* out_row, int64_t* out_col, int col_prefilled,
                                hipStream_t s) {
-  using namespace gs;
   const UniqueTuning tn = tuning();
   const int64_t N = k.S + k.E;
   const bool fill = out_unique != nullptr && N > 0;
@@ -1889,15 +1932,15 @@ static int launch_fill_relabel(const gs::Keys& k, const gs::UniqueWs& w, int64_t
     const dim3 grid(label_blocks + (unsigned)w.groups);
     if (by_indptr)
       GS_LAUNCH("unique_fill_relabel", s,
-                unique_fill_relabel_kernel<true><<<grid, dim3(kBlock), 0, s>>>(
+                (unique_fill_relabel_kernel<true, Row>)<<<grid, dim3(kBlock), 0, s>>>(
                     k, f, l, label_blocks, w.batch, w.words, w.group_off));
     else
       GS_LAUNCH("unique_fill_relabel", s,
-                unique_fill_relabel_kernel<false><<<grid, dim3(kBlock), 0, s>>>(
+                (unique_fill_relabel_kernel<false, Row>)<<<grid, dim3(kBlock), 0, s>>>(
                     k, f, l, label_blocks, w.batch, w.words, w.group_off));
   } else if (fill) {
     GS_LAUNCH("unique_fill", s,
-              unique_fill_kernel<<<dim3((unsigned)w.groups), dim3(kBlock), 0, s>>>(
+              unique_fill_kernel<Row><<<dim3((unsigned)w.groups), dim3(kBlock), 0, s>>>(
                   k, f, w.batch, w.words, w.group_off));
   } else if (label) {
     if (by_indptr)
@@ -1912,13 +1955,13 @@ static int launch_fill_relabel(const gs::Keys& k, const gs::UniqueWs& w, int64_t
   return GS_OK;
 }
 
-int gs_unique_fill(const int64_t* seeds, const int64_t* seeds_ptr,
-                   int64_t num_seeds, const int64_t* rows,
+template <typename Row>
+static int unique_fill(const int64_t* seeds, const int64_t* seeds_ptr,
+                   int64_t num_seeds, const Row* rows,
                    const int64_t* rows_ptr, int64_t num_rows_keys,
                    int64_t num_batches, const int64_t* unique_ptr,
                    int64_t* out_unique, void* workspace, size_t workspace_bytes,
                    gs_stream_t stream) {
-  using namespace gs;
   const int64_t S = num_seeds, E = num_rows_keys, B = num_batches;
   int rc = check_unique_args(seeds, seeds_ptr, S, rows, rows_ptr, E, B);
   if (rc != GS_OK) return rc;
@@ -1927,7 +1970,7 @@ int gs_unique_fill(const int64_t* seeds, const int64_t* seeds_ptr,
   if ((rc = check_workspace(w, workspace, workspace_bytes)) != GS_OK) return rc;
   if (S + E == 0) return GS_OK;
   GS_REQUIRE(out_unique, "unique_fill: null out_unique");
-  const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
+  const Keys<Row> k{{seeds_ptr, S, rows_ptr, E, B}, seeds, rows};
   return launch_fill_relabel(k, w, out_unique, nullptr, nullptr, nullptr, nullptr, 0,
                              as_stream(stream));
 }
@@ -1939,6 +1982,70 @@ static int check_label_args(int64_t S, int64_t E, const int64_t* edge_col,
   GS_REQUIRE(col_indptr == nullptr || E == 0 || S > 0,
              "unique_relabel: %lld edges grouped by column but no seeds", (long long)E);
   return GS_OK;
+}
+
+template <typename Row>
+static int unique_fill_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
+                           int64_t num_seeds, const Row* rows,
+                           const int64_t* rows_ptr, int64_t num_rows_keys,
+                           int64_t num_batches, const int64_t* unique_ptr,
+                           int64_t* out_unique, const int64_t* edge_col,
+                           const int64_t* col_indptr, int64_t* out_row, int64_t* out_col,
+                           int out_col_prefilled, void* workspace, size_t workspace_bytes,
+                           gs_stream_t stream) {
+  const int64_t S = num_seeds, E = num_rows_keys, B = num_batches;
+  int rc = check_unique_args(seeds, seeds_ptr, S, rows, rows_ptr, E, B);
+  if (rc != GS_OK) return rc;
+  GS_REQUIRE(unique_ptr, "unique_fill_relabel: null unique_ptr");
+  if ((rc = check_label_args(S, E, edge_col, col_indptr, out_col)) != GS_OK) return rc;
+  UniqueWs w = carve_unique(workspace, S, E, B);
+  if ((rc = check_workspace(w, workspace, workspace_bytes)) != GS_OK) return rc;
+  GS_REQUIRE(S + E == 0 || out_unique, "unique_fill_relabel: null out_unique");
+  const Keys<Row> k{{seeds_ptr, S, rows_ptr, E, B}, seeds, rows};
+  return launch_fill_relabel(k, w, out_unique, edge_col, col_indptr, out_row, out_col,
+                             out_col_prefilled, as_stream(stream));
+}
+
+}  // namespace gs
+
+extern "C" {
+
+size_t gs_unique_workspace_bytes(int64_t num_seeds, int64_t num_rows_keys,
+                                 int64_t num_batches) {
+  if (num_seeds < 0 || num_rows_keys < 0 || num_batches < 1) return 0;
+  return gs::carve_unique(nullptr, num_seeds, num_rows_keys, num_batches).total;
+}
+
+int gs_unique_count(const int64_t* seeds, const int64_t* seeds_ptr,
+                    int64_t num_seeds, const int64_t* rows,
+                    const int64_t* rows_ptr, int64_t num_rows_keys,
+                    int64_t num_batches, int64_t* unique_ptr,
+                    int64_t* unique_ptr_mirror, void* workspace,
+                    size_t workspace_bytes, gs_stream_t stream) {
+  return gs_unique_count_distinct(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+                                  num_batches, unique_ptr, unique_ptr_mirror, nullptr, workspace,
+                                  workspace_bytes, stream);
+}
+
+int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr,
+                             int64_t num_seeds, const int64_t* rows,
+                             const int64_t* rows_ptr, int64_t num_rows_keys,
+                             int64_t num_batches, int64_t* unique_ptr,
+                             int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+                             void* workspace, size_t workspace_bytes, gs_stream_t stream) {
+  return gs::unique_count(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+      num_batches, unique_ptr, unique_ptr_mirror, distinct_mirror, workspace, workspace_bytes,
+      stream);
+}
+
+int gs_unique_fill(const int64_t* seeds, const int64_t* seeds_ptr,
+                   int64_t num_seeds, const int64_t* rows,
+                   const int64_t* rows_ptr, int64_t num_rows_keys,
+                   int64_t num_batches, const int64_t* unique_ptr,
+                   int64_t* out_unique, void* workspace, size_t workspace_bytes,
+                   gs_stream_t stream) {
+  return gs::unique_fill(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys, num_batches,
+      unique_ptr, out_unique, workspace, workspace_bytes, stream);
 }
 
 int gs_unique_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
@@ -1955,7 +2062,7 @@ int gs_unique_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
   if ((rc = check_label_args(S, E, edge_col, col_indptr, out_col)) != GS_OK) return rc;
   UniqueWs w = carve_unique(workspace, S, E, B);
   if ((rc = check_workspace(w, workspace, workspace_bytes)) != GS_OK) return rc;
-  const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
+  const Keys<int64_t> k{{seeds_ptr, S, rows_ptr, E, B}, seeds, rows};
   return launch_fill_relabel(k, w, nullptr, edge_col, col_indptr, out_row, out_col,
                              out_col_prefilled, as_stream(stream));
 }
@@ -1968,18 +2075,40 @@ int gs_unique_fill_relabel(const int64_t* seeds, const int64_t* seeds_ptr,
                            const int64_t* col_indptr, int64_t* out_row, int64_t* out_col,
                            int out_col_prefilled, void* workspace, size_t workspace_bytes,
                            gs_stream_t stream) {
-  using namespace gs;
-  const int64_t S = num_seeds, E = num_rows_keys, B = num_batches;
-  int rc = check_unique_args(seeds, seeds_ptr, S, rows, rows_ptr, E, B);
-  if (rc != GS_OK) return rc;
-  GS_REQUIRE(unique_ptr, "unique_fill_relabel: null unique_ptr");
-  if ((rc = check_label_args(S, E, edge_col, col_indptr, out_col)) != GS_OK) return rc;
-  UniqueWs w = carve_unique(workspace, S, E, B);
-  if ((rc = check_workspace(w, workspace, workspace_bytes)) != GS_OK) return rc;
-  GS_REQUIRE(S + E == 0 || out_unique, "unique_fill_relabel: null out_unique");
-  const Keys k{seeds, seeds_ptr, S, rows, rows_ptr, E, B};
-  return launch_fill_relabel(k, w, out_unique, edge_col, col_indptr, out_row, out_col,
-                             out_col_prefilled, as_stream(stream));
+  return gs::unique_fill_relabel(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+      num_batches, unique_ptr, out_unique, edge_col, col_indptr, out_row, out_col,
+      out_col_prefilled, workspace, workspace_bytes, stream);
+}
+
+int gs_unique_count_distinct_rows32(const int64_t* seeds, const int64_t* seeds_ptr,
+                                    int64_t num_seeds, const int32_t* rows,
+                                    const int64_t* rows_ptr, int64_t num_rows_keys,
+                                    int64_t num_batches, int64_t* unique_ptr,
+                                    int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+                                    void* workspace, size_t workspace_bytes, gs_stream_t stream) {
+  return gs::unique_count(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+      num_batches, unique_ptr, unique_ptr_mirror, distinct_mirror, workspace, workspace_bytes,
+      stream);
+}
+
+int gs_unique_fill_rows32(const int64_t* seeds, const int64_t* seeds_ptr, int64_t num_seeds,
+                          const int32_t* rows, const int64_t* rows_ptr, int64_t num_rows_keys,
+                          int64_t num_batches, const int64_t* unique_ptr, int64_t* out_unique,
+                          void* workspace, size_t workspace_bytes, gs_stream_t stream) {
+  return gs::unique_fill(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys, num_batches,
+      unique_ptr, out_unique, workspace, workspace_bytes, stream);
+}
+
+int gs_unique_fill_relabel_rows32(const int64_t* seeds, const int64_t* seeds_ptr,
+                                  int64_t num_seeds, const int32_t* rows, const int64_t* rows_ptr,
+                                  int64_t num_rows_keys, int64_t num_batches,
+                                  const int64_t* unique_ptr, int64_t* out_unique,
+                                  const int64_t* edge_col, const int64_t* col_indptr,
+                                  int64_t* out_row, int64_t* out_col, int out_col_prefilled,
+                                  void* workspace, size_t workspace_bytes, gs_stream_t stream) {
+  return gs::unique_fill_relabel(seeds, seeds_ptr, num_seeds, rows, rows_ptr, num_rows_keys,
+      num_batches, unique_ptr, out_unique, edge_col, col_indptr, out_row, out_col,
+      out_col_prefilled, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

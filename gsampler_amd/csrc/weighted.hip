@@ -629,13 +629,13 @@ constexpr int kMaxCdfFanout = 64;
 template <int KMAX>
 constexpr int kCdfThreads = KMAX <= 16 ? kBlock : kWave;
 
-template <int KMAX>
+template <int KMAX, typename Row>
 __global__ __launch_bounds__(kCdfThreads<KMAX>, KMAX <= 10 ? 4 : 1) void sample_weighted_cdf_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols,
     const int64_t* __restrict__ indices, const uint64_t* __restrict__ cdf,
     const int64_t* __restrict__ column_ids, int64_t num_items, int fanout,
     int replace, PhiloxKey key, const int64_t* __restrict__ sub_indptr,
-    int64_t* __restrict__ out_coo_col, int64_t* __restrict__ out_indices,
+    int64_t* __restrict__ out_coo_col, Row* __restrict__ out_indices,
     int64_t* __restrict__ out_select, ColumnLabels labels,
     const int64_t* __restrict__ col_span, const int64_t* __restrict__ num_dev) {
   constexpr int kThreads = kCdfThreads<KMAX>;
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(kCdfThreads<KMAX>, KMAX <= 10 ? 4 : 1) void sample_
     }
     const int64_t p = in_start + off;
     out_indices[out_start + slot] =
-        row_bits ? (int64_t)(entry & row_mask) : indices ? indices[p] : p;
+        (Row)(row_bits ? (int64_t)(entry & row_mask) : indices ? indices[p] : p);
     if (out_select) out_select[out_start + slot] = p;
     if (out_coo_col) out_coo_col[out_start + slot] = col_label;
   };
@@ -761,23 +761,23 @@ __global__ __launch_bounds__(kCdfThreads<KMAX>, KMAX <= 10 ? 4 : 1) void sample_
     const int64_t p = __shfl(in_start, owner, kWave) + pick.x;
     const int64_t label = __shfl(col_label, owner, kWave);
     if (!mine) continue;
-    out_indices[to] = row_bits ? (int64_t)pick.y : indices ? indices[p] : p;
+    out_indices[to] = (Row)(row_bits ? (int64_t)pick.y : indices ? indices[p] : p);
     if (out_select) out_select[to] = p;
     if (out_coo_col) out_coo_col[to] = label;
   }
 }
 
-template <int KMAX>
+template <int KMAX, typename Row>
 static int launch_weighted_cdf(const int64_t* indptr, int64_t num_cols,
                                const int64_t* indices, const int64_t* cdf,
                                const int64_t* column_ids, int64_t num_items,
                                int fanout, int replace, PhiloxKey key,
                                const int64_t* sub_indptr, int64_t* out_coo_col,
-                               int64_t* out_indices, int64_t* out_select,
+                               Row* out_indices, int64_t* out_select,
                                ColumnLabels labels, const int64_t* col_span,
                                const int64_t* num_dev, hipStream_t s) {
   GS_LAUNCH("sample_weighted_cdf", s,
-            sample_weighted_cdf_kernel<KMAX>
+            (sample_weighted_cdf_kernel<KMAX, Row>)
                 <<<dim3((unsigned)ceil_div(num_items, kCdfThreads<KMAX>)),
                    dim3(kCdfThreads<KMAX>), 0, s>>>(
                 indptr, num_cols, indices, (const uint64_t*)cdf, column_ids, num_items,
@@ -788,27 +788,28 @@ static int launch_weighted_cdf(const int64_t* indptr, int64_t num_cols,
 
 // (every slot of the register arrays costs instructions in every draw whether it is
 // used or not: the common fan-outs get arrays of their own size)
+template <typename Row>
 static int launch_weighted_cdf_any(const int64_t* indptr, int64_t num_cols,
                                    const int64_t* indices, const int64_t* cdf,
                                    const int64_t* column_ids, int64_t num_items, int fanout,
                                    int replace, PhiloxKey key, const int64_t* sub_indptr,
-                                   int64_t* out_coo_col, int64_t* out_indices,
+                                   int64_t* out_coo_col, Row* out_indices,
                                    int64_t* out_select, ColumnLabels labels,
                                    const int64_t* col_span, const int64_t* num_dev,
                                    hipStream_t s) {
 #define GS_CDF_ARGS                                                              \
   indptr, num_cols, indices, cdf, column_ids, num_items, fanout, replace, key, sub_indptr, \
       out_coo_col, out_indices, out_select, labels, col_span, num_dev, s
-  if (fanout <= 4) return launch_weighted_cdf<4>(GS_CDF_ARGS);
-  if (fanout == 5) return launch_weighted_cdf<5>(GS_CDF_ARGS);
-  if (fanout <= 8) return launch_weighted_cdf<8>(GS_CDF_ARGS);
-  if (fanout <= 10) return launch_weighted_cdf<10>(GS_CDF_ARGS);
-  if (fanout <= 12) return launch_weighted_cdf<12>(GS_CDF_ARGS);
-  if (fanout <= 15) return launch_weighted_cdf<15>(GS_CDF_ARGS);
-  if (fanout <= 16) return launch_weighted_cdf<16>(GS_CDF_ARGS);
-  if (fanout <= 24) return launch_weighted_cdf<24>(GS_CDF_ARGS);
-  if (fanout <= 32) return launch_weighted_cdf<32>(GS_CDF_ARGS);
-  return launch_weighted_cdf<64>(GS_CDF_ARGS);
+  if (fanout <= 4) return launch_weighted_cdf<4, Row>(GS_CDF_ARGS);
+  if (fanout == 5) return launch_weighted_cdf<5, Row>(GS_CDF_ARGS);
+  if (fanout <= 8) return launch_weighted_cdf<8, Row>(GS_CDF_ARGS);
+  if (fanout <= 10) return launch_weighted_cdf<10, Row>(GS_CDF_ARGS);
+  if (fanout <= 12) return launch_weighted_cdf<12, Row>(GS_CDF_ARGS);
+  if (fanout <= 15) return launch_weighted_cdf<15, Row>(GS_CDF_ARGS);
+  if (fanout <= 16) return launch_weighted_cdf<16, Row>(GS_CDF_ARGS);
+  if (fanout <= 24) return launch_weighted_cdf<24, Row>(GS_CDF_ARGS);
+  if (fanout <= 32) return launch_weighted_cdf<32, Row>(GS_CDF_ARGS);
+  return launch_weighted_cdf<64, Row>(GS_CDF_ARGS);
 #undef GS_CDF_ARGS
 }
 
@@ -819,6 +820,36 @@ int launch_weighted_places(const int64_t* indptr, int64_t num_cols, const int64_
   return launch_weighted_cdf_any(indptr, num_cols, indices, cdf, column_ids, bound, (int)fanout,
                                  replace, key, nullptr, nullptr, out_rows, nullptr,
                                  ColumnLabels{nullptr, 0}, nullptr, num_dev, s);
+}
+
+// Weighted picks of columns through the CDF, row ids of either width.
+template <typename Row>
+static int sample_weighted_by_cdf(const int64_t* indptr, int64_t num_cols, const int64_t* indices,
+                                  const int64_t* cdf, const int64_t* column_ids, int64_t num_items,
+                                  int64_t fanout, int replace, uint64_t seed, uint64_t call_id,
+                                  const int64_t* sub_indptr, const int64_t* col_span,
+                                  int64_t* out_coo_col, Row* out_indices, int64_t* out_select,
+                                  const int64_t* col_batch_ptr, int64_t num_col_batches,
+                                  gs_stream_t stream) {
+  GS_REQUIRE(num_items >= 0 && num_cols >= 0, "sample_weighted: negative size");
+  GS_REQUIRE(col_batch_ptr == nullptr || num_col_batches >= 1,
+             "sample_weighted: col_batch_ptr given but num_col_batches = %lld",
+             (long long)num_col_batches);
+  GS_REQUIRE(fanout >= 0, "sample_weighted: negative fanout %lld", (long long)fanout);
+  if (num_items == 0 || fanout == 0) return GS_OK;
+  GS_REQUIRE(indptr && cdf && sub_indptr && out_indices, "sample_weighted: null pointer");
+  GS_REQUIRE(column_ids != nullptr || num_items <= num_cols,
+             "sample_weighted: %lld items but the matrix has %lld columns",
+             (long long)num_items, (long long)num_cols);
+  GS_REQUIRE(replace || fanout <= kMaxCdfFanout,
+             "sample_weighted: fanout %lld > %d is not supported without replacement",
+             (long long)fanout, kMaxCdfFanout);
+  GS_REQUIRE(fanout <= INT32_MAX, "sample_weighted: fanout too large");
+  return launch_weighted_cdf_any(indptr, num_cols, indices, cdf, column_ids, num_items, (int)fanout,
+                                 replace, make_key(seed, call_id), sub_indptr, out_coo_col,
+                                 out_indices, out_select,
+                                 ColumnLabels{col_batch_ptr, num_col_batches}, col_span, nullptr,
+                                 as_stream(stream));
 }
 
 // ------------------------------------------------------------ list sampling
@@ -1463,6 +1494,11 @@ int gs_csc_col_sample_weighted_fill(
     int64_t* out_coo_col, int64_t* out_indices, int64_t* out_select,
     const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream) {
   using namespace gs;
+  if (cdf != nullptr)
+    return sample_weighted_by_cdf<int64_t>(indptr, num_cols, indices, cdf, column_ids, num_items,
+                                           fanout, replace, seed, call_id, sub_indptr, col_span,
+                                           out_coo_col, out_indices, out_select, col_batch_ptr,
+                                           num_col_batches, stream);
   GS_REQUIRE(num_items >= 0 && num_cols >= 0, "sample_weighted: negative size");
   GS_REQUIRE(col_batch_ptr == nullptr || num_col_batches >= 1,
              "sample_weighted: col_batch_ptr given but num_col_batches = %lld",
@@ -1470,22 +1506,13 @@ int gs_csc_col_sample_weighted_fill(
   const ColumnLabels labels{col_batch_ptr, num_col_batches};
   GS_REQUIRE(fanout >= 0, "sample_weighted: negative fanout %lld", (long long)fanout);
   if (num_items == 0 || fanout == 0) return GS_OK;
-  GS_REQUIRE(indptr && (probs || cdf) && sub_indptr && out_indices && (out_select || cdf),
+  GS_REQUIRE(indptr && probs && sub_indptr && out_indices && out_select,
              "sample_weighted: null pointer");
   GS_REQUIRE(column_ids != nullptr || num_items <= num_cols,
              "sample_weighted: %lld items but the matrix has %lld columns",
              (long long)num_items, (long long)num_cols);
   const PhiloxKey key = make_key(seed, call_id);
   hipStream_t s = as_stream(stream);
-  if (cdf != nullptr) {
-    GS_REQUIRE(replace || fanout <= kMaxCdfFanout,
-               "sample_weighted: fanout %lld > %d is not supported without replacement",
-               (long long)fanout, kMaxCdfFanout);
-    GS_REQUIRE(fanout <= INT32_MAX, "sample_weighted: fanout too large");
-    return launch_weighted_cdf_any(indptr, num_cols, indices, cdf, column_ids, num_items,
-                                   (int)fanout, replace, key, sub_indptr, out_coo_col, out_indices,
-                                   out_select, labels, col_span, nullptr, s);
-  }
   if (replace) {
     GS_REQUIRE(cdf_scratch, "sample_weighted: sampling with replacement needs the CDF scratch");
     GS_REQUIRE(column_ids == nullptr || cdf_offsets != nullptr,
@@ -1516,6 +1543,17 @@ int gs_csc_col_sample_weighted_fill(
                 (int)fanout, key, sub_indptr, out_coo_col, out_indices,
                 out_select, labels));
   return GS_OK;
+}
+
+int gs_csc_col_sample_weighted_fill_rows32(
+    const int64_t* indptr, int64_t num_cols, const int64_t* indices, const int64_t* cdf,
+    const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace, uint64_t seed,
+    uint64_t call_id, const int64_t* sub_indptr, const int64_t* col_span, int64_t* out_coo_col,
+    int32_t* out_rows, const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream) {
+  return gs::sample_weighted_by_cdf<int32_t>(indptr, num_cols, indices, cdf, column_ids, num_items,
+                                             fanout, replace, seed, call_id, sub_indptr, col_span,
+                                             out_coo_col, out_rows, nullptr, col_batch_ptr,
+                                             num_col_batches, stream);
 }
 
 size_t gs_list_sample_workspace_bytes(int64_t n, int64_t num_segments) {

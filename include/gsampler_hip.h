@@ -236,6 +236,17 @@ int gs_csc_col_sample_uniform_fill_i32(const int64_t* indptr, int64_t num_cols,
                                        int64_t num_col_batches,
                                        gs_stream_t stream);
 
+/* That again with the row ids (all of them below 2^31) written 32 bits wide and no edge
+ * positions, for a caller whose next step reads the ids once more and nobody else does
+ * (gs_unique_*_rows32).  Ids are read from indices32, or from `indices` when that is NULL.
+ * fanout <= 64; the picks of GS_ALGO_AUTO. */
+int gs_csc_col_sample_uniform_fill_rows32(
+    const int64_t* indptr, int64_t num_cols, const int64_t* indices, const int32_t* indices32,
+    const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace, uint64_t seed,
+    uint64_t call_id, const int64_t* sub_indptr, const int64_t* col_span, int64_t* out_coo_col,
+    int32_t* out_rows, const int64_t* col_batch_ptr, int64_t num_col_batches,
+    gs_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * Weighted per-column sampling (fill phase; counts come from
  * gs_csc_col_count).  probs[nnz] (fp32) is aligned with `indices`; indices may
@@ -294,6 +305,15 @@ int gs_csc_col_sample_weighted_fill(
     const int64_t* sub_indptr, const int64_t* col_span, const int64_t* cdf_offsets,
     void* cdf_scratch, int64_t* out_coo_col, int64_t* out_indices, int64_t* out_select,
     const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream);
+
+/* The CDF form with the row ids (all of them below 2^31) written 32 bits wide and no edge
+ * positions, as gs_csc_col_sample_uniform_fill_rows32. */
+int gs_csc_col_sample_weighted_fill_rows32(
+    const int64_t* indptr, int64_t num_cols, const int64_t* indices, const int64_t* cdf,
+    const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace, uint64_t seed,
+    uint64_t call_id, const int64_t* sub_indptr, const int64_t* col_span, int64_t* out_coo_col,
+    int32_t* out_rows, const int64_t* col_batch_ptr, int64_t num_col_batches,
+    gs_stream_t stream);
 
 /* Evaluates the key arithmetic on the device: out2[0] = -log2((r64>>12)+1)/2^52),
  * out2[1] = key of weight w at stream (seed, call_id, pos, draw).  Test hook. */
@@ -431,6 +451,26 @@ int gs_unique_count_distinct(const int64_t* seeds, const int64_t* seeds_ptr, int
                              int64_t num_rows_keys, int64_t num_batches, int64_t* unique_ptr,
                              int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
                              void* workspace, size_t workspace_bytes, gs_stream_t stream);
+
+/* gs_unique_count_distinct, gs_unique_fill and gs_unique_fill_relabel for row keys that are
+ * 32 bits wide (the samplers' _rows32 forms leave them so); everything else is the same. */
+int gs_unique_count_distinct_rows32(const int64_t* seeds, const int64_t* seeds_ptr,
+                                    int64_t num_seeds, const int32_t* rows,
+                                    const int64_t* rows_ptr, int64_t num_rows_keys,
+                                    int64_t num_batches, int64_t* unique_ptr,
+                                    int64_t* unique_ptr_mirror, int64_t* distinct_mirror,
+                                    void* workspace, size_t workspace_bytes, gs_stream_t stream);
+int gs_unique_fill_rows32(const int64_t* seeds, const int64_t* seeds_ptr, int64_t num_seeds,
+                          const int32_t* rows, const int64_t* rows_ptr, int64_t num_rows_keys,
+                          int64_t num_batches, const int64_t* unique_ptr, int64_t* out_unique,
+                          void* workspace, size_t workspace_bytes, gs_stream_t stream);
+int gs_unique_fill_relabel_rows32(const int64_t* seeds, const int64_t* seeds_ptr,
+                                  int64_t num_seeds, const int32_t* rows, const int64_t* rows_ptr,
+                                  int64_t num_rows_keys, int64_t num_batches,
+                                  const int64_t* unique_ptr, int64_t* out_unique,
+                                  const int64_t* edge_col, const int64_t* col_indptr,
+                                  int64_t* out_row, int64_t* out_col, int out_col_prefilled,
+                                  void* workspace, size_t workspace_bytes, gs_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * One whole layer of node-wise sampling in three launches, for small layers:

@@ -501,6 +501,56 @@ def test_unique_relabel_of_ids_that_meet_in_one_bucket(n, meet):
                 orc.unique_relabel(keys[:S], keys[S:], edge_col=col))
 
 
+@pytest.mark.parametrize("fanout", [1, 5, 15, 64])
+def test_row_ids_of_32_bits_from_the_samplers(fanout):
+    """The same picks and column labels as with row ids of 64 bits, from either array of ids,
+    uniform and by weight, with and without replacement; empty columns and ids of none."""
+    rng = np.random.default_rng(fanout)
+    indptr, indices = random_csc(rng, 3000, 2**31 - 1, 60, hub_deg=5000)
+    cols = rng.integers(-2, 3003, size=2500)
+    ptr = T([0, 100, 100, 1700, 2500])
+    ip, ix, c = T(indptr), T(indices), T(cols)
+    cdf = capi.weight_cdf(ip, torch.as_tensor(rng.random(indices.size, dtype=np.float32), device=DEV),
+                          ix, 2**31 - 1)
+    for replace in (False, True):
+        want = capi.sample_uniform(ip, ix, c, fanout, replace, col_batch_ptr=ptr)
+        for ids in (ix, ix.to(torch.int32)):
+            got = capi.sample_uniform(ip, ids, c, fanout, replace, col_batch_ptr=ptr, rows32=True)
+            assert got[2].dtype == torch.int32 and got[3] is None
+            assert_same((got[0], got[1], got[2].long()), [N(t) for t in want[:3]])
+        wide, narrow = (capi._sample_weighted_cdf(ip, ix, cdf, c, fanout, replace, 7, 3, True, ptr,
+                                                  rows32=narrow) for narrow in (False, True))
+        assert_same((narrow[0], narrow[1], narrow[2].long()), [N(t) for t in wide[:3]])
+    with pytest.raises(capi.GsError, match="above 64"):
+        capi.sample_uniform(ip, ix, c, 65, rows32=True)
+
+
+@pytest.mark.parametrize("shape", ["one batch", "few keys", "tiny batches", "seeds of tiles", "wide seeds"])
+def test_unique_relabel_of_row_ids_of_32_bits(shape):
+    """Row keys of 32 bits beside seeds of 64: tiles and groups of positions that hold seeds
+    alone, rows alone and both; batches of a few keys; seeds that no 32 bits hold, and rows that
+    share their low bits; negative rows."""
+    rng = np.random.default_rng(len(shape))
+    B, s_size, r_size, ids = {"one batch": (1, 5000, 90_000, 10**5), "few keys": (3, 40, 900, 2000),
+                              "tiny batches": (2000, 9, 60, 300), "seeds of tiles": (3, 9000, 30_000, 10**5),
+                              "wide seeds": (4, 5000, 20_000, 3000)}[shape]
+    seeds = rng.integers(0, ids, size=B * s_size)
+    rows = rng.integers(-3 if shape == "wide seeds" else 0, ids, size=B * r_size)
+    rows[::7] = 2**31 - 1
+    if shape == "wide seeds":
+        seeds[::3] += 2**32 * rng.integers(1, 3, size=seeds[::3].size)
+        seeds[1::50] = -2
+    sp, rp = np.arange(B + 1) * s_size, np.arange(B + 1) * r_size
+    col = np.sort(np.concatenate([rng.integers(sp[b], sp[b + 1], size=r_size) for b in range(B)]))
+    want = orc.unique_relabel(seeds, rows, sp, rp, col)
+    rows = T(rows).to(torch.int32)
+    assert_same(capi.unique_relabel(T(seeds), rows, T(sp), T(rp), T(col)), want)
+    indptr = T(np.searchsorted(col, np.arange(B * s_size + 1)))
+    assert_same(capi.unique_relabel(T(seeds), rows, T(sp), T(rp), col_indptr=indptr), want)
+    got = capi.unique_relabel(T(seeds), rows, T(sp), T(rp), want_row=False, want_col=False)
+    assert_same(got[:2], want[:2])
+
+
 def test_unique_relabel_one_huge_batch():
     """More keys in one batch than its buckets can take at the usual size: every
     bucket is deduplicated in global memory."""
