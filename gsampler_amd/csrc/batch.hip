@@ -87,6 +87,11 @@ __global__ __launch_bounds__(kBlock) void local_ids_kernel(
 // the tile's first and last element are looked up once per work-group (the
 // position is the same in every lane: scalar loads) and an element searches
 // only between them -- not at all when one piece covers the tile.
+// No more pieces than a wavefront has lanes, as most calls have: a lane holds where its piece
+// begins and what it begins with, and the piece of an element is told by comparing with those,
+// so that two trips to memory lie in front of the stores, not one per step of a search.  64
+// batches of 65 K, 592 K and 3.5 M columns in all, us: 7.7, 10.0 and 18.1 with the search, now
+// 4.6, 4.6 and 12.9.
 constexpr int kSplitItems = 4;
 constexpr int kSplitTile = kBlock * kSplitItems;
 
@@ -108,6 +113,34 @@ __device__ __forceinline__ void split_tile(
   const int64_t p0 = tile * kSplitTile;
   if (p0 >= out_len) return;
   const int64_t p_last = p0 + kSplitTile - 1 < out_len ? p0 + kSplitTile - 1 : out_len - 1;
+  if (num_batches <= kWave) {
+    const int lane = lane_id();
+    const int64_t begin = offset[lane < num_batches ? lane : num_batches - 1];
+    const int64_t first = wave_uniform_first(begin);
+    const int64_t start = lane < num_batches ? begin - first + lane : INT64_MAX;
+    const int b_lo = __popcll(__ballot(start <= p0)) - 1;
+    const int b_hi = __popcll(__ballot(start <= p_last)) - 1;
+    const int64_t base = indptr[begin];
+    int piece[kSplitItems];
+    int64_t v[kSplitItems];
+#pragma unroll
+    for (int i = 0; i < kSplitItems; ++i) {
+      int64_t p = p0 + i * kBlock + threadIdx.x;
+      if (p > p_last) p = p_last;
+      int b = b_lo;
+      for (int k = b_lo + 1; k <= b_hi; ++k)
+        if (p >= (int64_t)__shfl((long long)start, k, kWave)) b = k;
+      piece[i] = b;
+      v[i] = indptr[p + first - b];
+    }
+#pragma unroll
+    for (int i = 0; i < kSplitItems; ++i) {
+      const int64_t p = p0 + i * kBlock + threadIdx.x;
+      const int64_t from = (int64_t)__shfl((long long)base, piece[i], kWave);
+      if (p <= p_last) out[p] = v[i] - from;
+    }
+    return;
+  }
   const int64_t first = offset[0];
   const int64_t b_lo = piece_of(offset, first, 0, num_batches, p0);
   const int64_t b_hi = piece_of(offset, first, b_lo, num_batches, p_last);

@@ -588,6 +588,21 @@ def test_block_offsets_and_flags_in_one_launch(sizes):
     assert torch.equal(flags, kept)  # the host copy is not the only one
 
 
+@pytest.mark.parametrize("B", [1, 2, 63, 64, 65])
+@pytest.mark.parametrize("total", [0, 1, 1022, 1023, 1024, 5000])
+def test_split_indptr_of_as_many_batches_as_a_wavefront_has_lanes(B, total):
+    """Offsets of up to, and of more, batches than a wavefront has lanes: pieces that end at a
+    tile's border, empty ones, tiles inside one piece and over all, offsets that begin past 0."""
+    rng = np.random.default_rng(B + total)
+    indptr = np.concatenate([[0], np.cumsum(rng.integers(0, 9, size=total + 7))])
+    offset = 3 + np.concatenate([[0], np.sort(rng.integers(0, total + 1, size=B - 1)), [total]])
+    out = torch.full((total + B,), -7, dtype=torch.int64, device=DEV)
+    ip, off = T(indptr), T(offset)
+    capi.check(capi.lib().gs_split_indptr(ip.data_ptr(), off.data_ptr(), B, total + B, out.data_ptr(), None))
+    want = [indptr[offset[b]:offset[b + 1] + 1] - indptr[offset[b]] for b in range(B)]
+    assert np.array_equal(N(out), np.concatenate(want))
+
+
 def test_graphsage_layers_end_to_end():
     """Three fused slice+sample + unique/relabel layers on an R-MAT graph, super-batch
     of 8, compared with the oracle layer by layer."""
