@@ -124,6 +124,37 @@ struct LayerColumns {
   }
 };
 
+// The batches' offsets, one a lane, where a wavefront has lanes for all of them: asked for
+// once, beside a kernel's first loads, and compared with from then on, where a search takes a
+// trip to the cache a step, and the ends of a batch two more.  All lanes call these together.
+struct HeldBatches {
+  int64_t at;  // ptr[lane], INT64_MAX past the last
+  int B;
+  bool held;
+  __device__ __forceinline__ explicit HeldBatches(const LayerColumns& cols)
+      : at(0), B((int)cols.B), held(cols.ptr && cols.B < kWave) {
+    if (held) {
+      at = cols.ptr[lane_id() <= B ? lane_id() : B];
+      if (lane_id() > B) at = INT64_MAX;
+    }
+  }
+  __device__ __forceinline__ int64_t ptr(int b) const { return __shfl((long long)at, b, kWave); }
+  __device__ __forceinline__ int64_t num(const LayerColumns& cols) const {
+    return held ? wave_uniform_first(ptr(B)) : cols.num();
+  }
+  // batch of column x / width, x the same in every lane and below the last batch's end
+  __device__ __forceinline__ int of_uniform(int64_t x, int width) const {
+    return __popcll(__ballot(lane_id() < B && at * width <= x)) - 1;
+  }
+  // batch of column x / width, which lies in one of lo to hi
+  __device__ __forceinline__ int of(int64_t x, int width, int lo, int hi) const {
+    int b = lo;
+    for (int k = lo + 1; k <= hi; ++k)
+      if (ptr(k) * width <= x) b = k;
+    return b;
+  }
+};
+
 // The slot of a key in the global table after (key, position) went in; `cur` is what its
 // first slot was seen to hold.
 __device__ __forceinline__ uint32_t layer_insert(uint64_t* table, uint32_t mask, uint32_t key,
@@ -251,13 +282,24 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
   const PickLane l(blockIdx.x, fanout, cols_per_wave);
   // one round trip for the number of columns and the id, of a place that may be no column's
   const int64_t id = cols.ids[cols.place(l.c, 1)];
-  const int64_t n = cols.num();
+  const HeldBatches batches(cols);
+  const int64_t n = batches.num(cols);
   if (l.first_col >= n) return;  // uniform per work-group
   sh.clear();
+  int64_t held_b = 0, held_lo = 0, held_hi = 0;
+  if (batches.held) {
+    const int64_t last_col = l.first_col + kPickThreads / kWave * cols_per_wave - 1;
+    const int b = batches.of(l.c, 1, batches.of_uniform(l.first_col, 1),
+                             batches.of_uniform(last_col < n ? last_col : n - 1, 1));
+    held_b = b;
+    held_lo = batches.ptr(b);
+    held_hi = batches.ptr(b + 1);
+  }
   pick_columns(
       l, l.in_group && l.c < n,
       [&](int64_t* start, int64_t* deg) {
         *deg = column_degree(indptr, num_cols, id, start);
+        if (batches.held) return PickColumn{id, held_b, held_lo, held_hi - held_lo};
         const int64_t b0 =
             cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(l.first_col)) : 0;
         const int64_t b = cols.batch_of(l.c, b0);
@@ -275,9 +317,10 @@ struct TileBatches {
     return b;
   }
 };
-__device__ __forceinline__ TileBatches tile_batches(const LayerColumns& cols, int width,
-                                                    int64_t p0, int64_t p_last) {
+__device__ __forceinline__ TileBatches tile_batches(const LayerColumns& cols, const HeldBatches& held,
+                                                    int width, int64_t p0, int64_t p_last) {
   if (!cols.ptr) return TileBatches{0, 0};
+  if (held.held) return TileBatches{held.of_uniform(p0, width), held.of_uniform(p_last, width)};
   return TileBatches{segment_of(cols.ptr, cols.B, wave_uniform_first(p0 / width)),
                      segment_of(cols.ptr, cols.B, wave_uniform_first(p_last / width))};
 }
@@ -296,7 +339,8 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
 #pragma unroll
   for (int j = 0; j < kLayerWordsPerWave; ++j)
     s[j] = slot_of[cols.place(wave_p0 + j * kWave + lane, width)];
-  const int64_t N = cols.num() * width;
+  const HeldBatches held(cols);
+  const int64_t N = held.num(cols) * width;
   if (p0 >= N) return;
 #pragma unroll
   for (int j = 0; j < kLayerWordsPerWave; ++j) {
@@ -304,20 +348,29 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
     e[j] = s[j] != kNoSlot ? table[s[j]] : 0ull;
   }
   const TileBatches batches =
-      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
+      tile_batches(cols, held, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
   LayerWord mine{0ull, 0ull, 0u, 0u, 0ull};
   uint32_t firsts = 0, edges = 0;
 #pragma unroll
   for (int j = 0; j < kLayerWordsPerWave; ++j) {
     const int64_t p = wave_p0 + j * kWave + lane;
     bool is_first = false, is_edge = false;
+    int64_t s_lo = 0, s_hi = 0;
+    if (held.held) {
+      const int b = held.of(p, width, (int)batches.b_lo, (int)batches.b_hi);
+      s_lo = held.ptr(b);
+      s_hi = held.ptr(b + 1);
+    }
     if (s[j] != kNoSlot) {
       const uint32_t f = (uint32_t)e[j];
       first[p] = f;
       is_first = f == (uint32_t)p;
-      const int64_t b = batches.of(cols, width, p);
-      const int64_t s_lo = cols.lo(b);
-      is_edge = p - s_lo * width >= cols.hi(b) - s_lo;
+      if (!held.held) {
+        const int64_t b = batches.of(cols, width, p);
+        s_lo = cols.lo(b);
+        s_hi = cols.hi(b);
+      }
+      is_edge = p - s_lo * width >= s_hi - s_lo;
     }
     const uint64_t fw = __ballot(is_first), ew = __ballot(is_edge);
     if (lane == j) mine = LayerWord{fw, ew, firsts, edges, 0ull};
@@ -416,11 +469,12 @@ __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned bl
 #pragma unroll
   for (int j = 0; j < kPer; ++j)
     cnt[j] = tile_cnt[(int64_t)threadIdx.x * kPer + j < blocks ? threadIdx.x * kPer + j : 0];
-  const int64_t n = cols.num(), N = n * width;
+  const HeldBatches held(cols);
+  const int64_t n = held.num(cols), N = n * width;
   const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
   if (block != 0 && (int64_t)block >= tiles) return empty_table();
   const TileBatches batches =
-      tile_batches(cols, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
+      tile_batches(cols, held, width, p0, p0 + kLayerTile - 1 < N ? p0 + kLayerTile - 1 : N - 1);
   LayerWord first_word[kItems];
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
@@ -430,8 +484,22 @@ __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned bl
     if (!edge) first_of[i] = 0;
     first_word[i] = words[first_of[i] / kWave];
   }
-  int64_t b = batches.b_lo;
-  int64_t s_lo = cols.lo(b), ns = cols.hi(b) - s_lo, fb = s_lo * width;
+  int64_t b = batches.b_lo, b_of[kItems];
+  int64_t s_lo, ns;
+  if (held.held) {
+    s_lo = wave_uniform_first(held.ptr((int)b));
+    ns = wave_uniform_first(held.ptr((int)b + 1)) - s_lo;
+  } else {
+    s_lo = cols.lo(b);
+    ns = cols.hi(b) - s_lo;
+  }
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    const int64_t p = p0 + i * kThreads + threadIdx.x;
+    if (held.held) b_of[i] = held.of(p, width, (int)batches.b_lo, (int)batches.b_hi);
+    else b_of[i] = p < N ? batches.of(cols, width, p) : b;
+  }
+  int64_t fb = s_lo * width;
   LayerWord word_b = words[cols.place(fb, width) / kWave];
   LayerWord word_q = words[cols.place(fb + (ns > 0 ? ns - 1 : 0), width) / kWave];
   uint64_t sum = 0;
@@ -517,9 +585,8 @@ __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned bl
   for (int i = 0; i < kItems; ++i) {
     const int64_t p = p0 + i * kThreads + threadIdx.x;
     if (p >= N) break;
-    const int64_t b_now = batches.of(cols, width, p);
-    if (b_now != b) {
-      b = b_now;
+    if (b_of[i] != b) {
+      b = b_of[i];
       s_lo = cols.lo(b);
       ns = cols.hi(b) - s_lo;
       fb = s_lo * width;

@@ -139,6 +139,12 @@ def test_chains_of_short_layers_around_the_most_batches(rng, batches, replace):
             assert torch.equal(getattr(layer.batch, name)(), getattr(other.batch, name)()), name
 
 
+@pytest.mark.parametrize("batches", [2, 62, 63, 64, 65])
+def test_chains_of_short_layers_around_a_wavefront_of_batches(rng, batches):
+    """As many batches as have their offsets held by the lanes of a wavefront, and more."""
+    test_chains_of_short_layers_around_the_most_batches(rng, batches, False)
+
+
 @pytest.mark.parametrize("cuts,fanouts,replace,weighted", [
     ([0, 8], [3, 2], False, False),
     ([0, 0, 30, 30, 64], [10, 5], False, False),         # batches without seeds
