@@ -767,6 +767,154 @@ __global__ __launch_bounds__(kCdfThreads<KMAX>, KMAX <= 10 ? 4 : 1) void sample_
   }
 }
 
+// The same picks where there are few columns: a column on sixteen neighbouring lanes.  A lane
+// that owns its column goes through a chain of dependent loads for every draw, and where the
+// device has no other wavefronts to run meanwhile, that chain is the time: 3 to 4.5 us a draw.
+// Here the column's entries (of a longer one, kHeld of them at equal distances) are in LDS
+// before the first draw, and a step of a search is one comparison by all lanes of a column and a
+// count of those that hold.
+//   draws      lane j's random number is draw j's
+//   intervals  lane i holds the i-th of those taken, in the order of their starts: where it
+//              starts in the mass that was left (`from`) and what it and those before it come
+//              to (`sum`).  A point r of the mass that is left lies past as many of them as
+//              have from <= r, and the new one is put in behind those
+//   search     which of sixteen pieces of the held entries, which entry of that; in a column
+//              of more than kHeld, sixteen entries a step from there on
+constexpr int kTeam = 16;   // lanes of a column, and the most draws
+constexpr int kHeld = 128;  // entries of a column in LDS
+static_assert(kHeld % kTeam == 0 && kHeld / kTeam <= kTeam, "a lane for every entry of a piece");
+// Columns per draw up to which a call goes this way.  A column costs a wavefront sixteen times
+// the instructions, and of a long one up to kHeld lines are read however few the draws: with
+// columns met by their degree (the frontiers of layers) in a graph of 2.45 M nodes and hubs of
+// millions, us, a lane a column and this: fanout 5, 64 columns 17 and 11, 4096 20 and 19, 8192
+// 20 and 24; fanout 10, 64 33 and 18, 8192 39 and 35, 16384 48 and 42, 32768 49 and 77; fanout
+// 15, 64 63 and 23, 16384 84 and 55, 32768 83 and 99.  Columns met evenly gain up to four times as
+// many.  (Windows of sixteen entries from a guess in place of the held ones of a long column:
+// fanout 15, 64 columns 30, 32768 80.)
+constexpr int64_t kTeamColumns = 1024;
+
+template <typename Row>
+__global__ __launch_bounds__(kBlock) void sample_weighted_team_kernel(
+    const int64_t* __restrict__ indptr, int64_t num_cols,
+    const int64_t* __restrict__ indices, const uint64_t* __restrict__ cdf,
+    const int64_t* __restrict__ column_ids, int64_t num_items, int fanout, PhiloxKey key,
+    const int64_t* __restrict__ sub_indptr, int64_t* __restrict__ out_coo_col,
+    Row* __restrict__ out_indices, int64_t* __restrict__ out_select, ColumnLabels labels,
+    const int64_t* __restrict__ col_span, const int64_t* __restrict__ num_dev) {
+  constexpr int kPiece = kHeld / kTeam;
+  __shared__ uint64_t s_held[kBlock / kTeam][kHeld];
+  const int lane = lane_id(), t = lane % kTeam, team0 = lane - t;
+  uint64_t* const held = s_held[threadIdx.x / kTeam];
+  const int64_t item = (int64_t)blockIdx.x * (kBlock / kTeam) + threadIdx.x / kTeam;
+  const int row_bits = (int)cdf[0];
+  const uint64_t row_mask = row_bits ? (~0ull >> (64 - row_bits)) : 0ull;
+  const int64_t id = column_ids ? column_ids[item < num_items ? item : num_items - 1] : item;
+  if (item >= (num_dev ? *num_dev : num_items)) return;  // whole teams leave together
+  int64_t col_label = item, in_start = 0;
+  if (out_coo_col) col_label = labels.of_near(item, item - (threadIdx.x % kWave) / kTeam);
+  const int64_t deg = col_span ? column_span(col_span, column_ids, indptr, num_cols, item, &in_start)
+                               : column_degree(indptr, num_cols, id, &in_start);
+  const int64_t out_start = sub_indptr ? sub_indptr[item] : item * fanout;
+  const uint64_t* const col = cdf + in_start;  // col[j], 1 <= j <= deg: entry of item j - 1
+  auto store = [&](int64_t slot, int64_t off, uint64_t entry) {
+    const int64_t p = in_start + off;
+    out_indices[out_start + slot] =
+        (Row)(row_bits ? (int64_t)(entry & row_mask) : indices ? indices[p] : p);
+    if (out_select) out_select[out_start + slot] = p;
+    if (out_coo_col) out_coo_col[out_start + slot] = col_label;
+  };
+  if (deg <= fanout) {  // whole column, original order, zero weights included
+    if (t < deg) store(t, t, col[t + 1]);
+    return;
+  }
+  // lanes of this team for which it holds, counted
+  auto count = [&](bool holds) {
+    return (int)__popc((uint32_t)(__ballot(holds) >> team0) & ((1u << kTeam) - 1u));
+  };
+  // held[i]: the entry that ends stretch i of `step` entries
+  const int64_t step = (deg + kHeld - 1) / kHeld;
+  const int stretches = (int)((deg + step - 1) / step);
+  uint64_t entry[kPiece];
+#pragma unroll
+  for (int i = 0; i < kPiece; ++i) {
+    const int64_t end = (int64_t)(i * kTeam + t + 1) * step;
+    entry[i] = col[end < deg ? end : deg];
+  }
+  const Words4 words = philox(key, (uint64_t)item, (uint64_t)t);
+  const uint64_t random = ((uint64_t)words.y << 32) | words.x;
+#pragma unroll
+  for (int i = 0; i < kPiece; ++i) held[i * kTeam + t] = entry[i];
+  // (by this wavefront's lanes only)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const uint64_t pivot = held[t * kPiece + kPiece - 1];
+  const int cb = 64 - row_bits < 62 ? 64 - row_bits : 62;
+  const uint64_t full = (1ull << cb) - 1ull;
+  // (a column without mass has share 0 throughout)
+  const bool mass = (held[stretches - 1] >> row_bits) != 0;
+  uint64_t from = 0, sum = 0, removed = 0, my_entry = 0;
+  int64_t my_off = 0;
+  int taken = 0;
+  while (mass && taken < fanout && removed < full) {
+    const uint64_t r = __umul64hi(
+        (uint64_t)__shfl((unsigned long long)random, team0 + taken, kWave), full - removed);
+    const int before = count(t < taken && from <= r);
+    const uint64_t skipped = before ? (uint64_t)__shfl((unsigned long long)sum, team0 + before - 1, kWave) : 0ull;
+    // the first entry that starts after x ends the item that holds it
+    const uint64_t beyond = (r + skipped + 1) << row_bits;
+    const int piece = count(pivot < beyond);
+    const uint64_t mine = held[(piece < kTeam ? piece : kTeam - 1) * kPiece + t % kPiece];
+    const int at = piece * kPiece + count(t < kPiece && mine < beyond);
+    int64_t off = at;
+    uint64_t e_lo, e_hi;
+    if (step == 1) {
+      e_lo = at ? held[at - 1] : 0ull;
+      e_hi = held[at];
+    } else {
+      int64_t lo = (int64_t)at * step;  // among entries lo + 1 to lo + len
+      int64_t len = lo + step < deg ? step : deg - lo;
+      while (len >= kTeam) {
+        const int64_t part = (len + kTeam - 1) / kTeam;
+        const int64_t end = (int64_t)(t + 1) * part < len ? (int64_t)(t + 1) * part : len;
+        const int64_t passed = part * count(col[lo + end] < beyond);
+        lo += passed;
+        len = part < len - passed ? part : len - passed;
+      }
+      const uint64_t e = lo + t == 0 ? 0ull : col[lo + (t <= len ? t : len)];
+      const int c = count(t >= 1 && t <= len && e < beyond);
+      off = lo + c;
+      e_lo = (uint64_t)__shfl((unsigned long long)e, team0 + c, kWave);
+      e_hi = (uint64_t)__shfl((unsigned long long)e, team0 + c + 1, kWave);
+    }
+    const uint64_t start = e_lo >> row_bits, length = (e_hi >> row_bits) - start;
+    const uint64_t from_up = (uint64_t)__shfl_up((unsigned long long)from, 1, kTeam);
+    const uint64_t sum_up = (uint64_t)__shfl_up((unsigned long long)sum, 1, kTeam);
+    if (t > before) {
+      from = from_up - length;
+      sum = sum_up + length;
+    } else if (t == before) {
+      from = start - skipped;
+      sum = skipped + length;
+    }
+    if (t == taken) {
+      my_off = off;
+      my_entry = e_hi;
+    }
+    removed += length;
+    ++taken;
+  }
+  if (t < taken) store(t, my_off, my_entry);
+  // fewer than fanout items have positive weight: zero-weight items in order
+  for (int64_t o = t; taken < fanout && o - t < deg; o += kTeam) {
+    const uint64_t e = col[o < deg ? o + 1 : deg], prev = o == 0 ? 0ull : col[o < deg ? o : deg];
+    const bool zero = o < deg && (e >> row_bits) == (prev >> row_bits);
+    const uint32_t zeros = (uint32_t)(__ballot(zero) >> team0) & ((1u << kTeam) - 1u);
+    const int slot = taken + (int)__popc(zeros & ((1u << t) - 1u));
+    if (zero && slot < fanout) store(slot, o, e);
+    taken += (int)__popc(zeros);
+  }
+}
+
 template <int KMAX, typename Row>
 static int launch_weighted_cdf(const int64_t* indptr, int64_t num_cols,
                                const int64_t* indices, const int64_t* cdf,
@@ -797,6 +945,15 @@ static int launch_weighted_cdf_any(const int64_t* indptr, int64_t num_cols,
                                    int64_t* out_select, ColumnLabels labels,
                                    const int64_t* col_span, const int64_t* num_dev,
                                    hipStream_t s) {
+  if (!replace && fanout <= kTeam && num_items <= kTeamColumns * fanout) {
+    GS_LAUNCH("sample_weighted_team", s,
+              sample_weighted_team_kernel<Row>
+                  <<<dim3((unsigned)ceil_div(num_items, kBlock / kTeam)), dim3(kBlock), 0, s>>>(
+                      indptr, num_cols, indices, (const uint64_t*)cdf, column_ids, num_items, fanout,
+                      key, sub_indptr, out_coo_col, out_indices, out_select, labels, col_span,
+                      num_dev));
+    return GS_OK;
+  }
 #define GS_CDF_ARGS                                                              \
   indptr, num_cols, indices, cdf, column_ids, num_items, fanout, replace, key, sub_indptr, \
       out_coo_col, out_indices, out_select, labels, col_span, num_dev, s

@@ -187,6 +187,46 @@ def test_cdf_columns_of_every_short_length(fanout):
                                      cdf=cdf))
 
 
+@pytest.mark.parametrize("fanout", [1, 2, 5, 15, 16, 17])
+def test_cdf_sampling_around_the_most_columns_of_a_team(fanout):
+    """As many columns as go sixteen lanes each, and one more; columns of every length around
+    what the lanes hold and around one and several steps of the search behind it, hubs; weights
+    that leave fewer items with a share than picks, none at all, and one with all but nothing."""
+    rng = np.random.default_rng(fanout)
+    lengths = np.concatenate([np.arange(0, 34), [63, 64, 65, 126, 127, 128, 129, 130, 255, 256, 257, 500],
+                              128 * np.array([15, 16, 17, 31, 32, 255, 256, 257]) + 1, [70_001, 300_000]])
+    kinds = ["even", "zeros", "few", "none", "one"]
+    lengths = np.repeat(lengths, len(kinds))
+    indptr = np.concatenate([[0], np.cumsum(lengths)])
+    indices = rng.integers(0, 2_450_000, size=indptr[-1])
+    probs = rng.lognormal(0, 1, size=indices.size).astype(np.float32)
+    for c, n in enumerate(lengths):
+        w = probs[indptr[c]:indptr[c + 1]]
+        kind = kinds[c % len(kinds)]
+        if kind == "zeros":
+            w[rng.random(n) < 0.6] = 0.0
+        elif kind in ("few", "none"):
+            w[:] = 0.0
+            if kind == "few" and n:
+                w[rng.integers(0, n, size=max(1, fanout // 2))] = 1.0
+        elif kind == "one" and n:
+            w[:] *= 1e-7
+            w[rng.integers(0, n)] = 1.0
+    cdfs = [(orc.weight_cdf(indptr, probs, ids), capi.weight_cdf(T(indptr), F(probs), T(ids) if ids is not None else None))
+            for ids in (indices, None)]
+    most = 1024 * fanout
+    for count in (1, most, most + 1):
+        cols = np.resize(np.concatenate([np.arange(lengths.size), [-1, lengths.size]]), count)
+        ptr = np.array([0, count // 3, count // 3, count])
+        for host, device in cdfs:
+            same(capi.sample_weighted(T(indptr), T(indices), None, T(cols), fanout, call_id=5, cdf=device),
+                 orc.sample_weighted(indptr, indices, None, cols, fanout, call_id=5, cdf=host))
+            a, b = (capi._sample_weighted_cdf(T(indptr), T(indices), device, T(cols), fanout, False, 7, 5, True,
+                                              T(ptr), spans=spans) for spans in (False, True))
+            for x, y in zip(a, b):
+                assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("n,k", [(10, 20), (1000, 64), (233000, 512), (5000, 5000)])
 def test_list_sampling_parity(n, k):
     rng = np.random.default_rng(n)
