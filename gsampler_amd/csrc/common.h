@@ -179,6 +179,12 @@ __device__ __forceinline__ int64_t wave_uniform_first(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// Between a wave's writes to its own part of LDS and its reads of other lanes' words.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Inclusive scan across the 64 lanes of a wavefront.
 template <typename T>
 __device__ __forceinline__ T wave_inclusive_sum(T v) {

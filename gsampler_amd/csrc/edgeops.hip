@@ -628,9 +628,7 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_sum_kernel(
 // The end of a LADIES layer, out[e] = q[e] / (sum of q over e's column) with q[e] =
 // values[select[e]] / row_divisor[row[e]], in two passes over the edges: the first writes
 // q and adds it up, the second divides.  7.3 M edges in 1024 columns: gather, division,
-// sums and division took 40 + 28 + 41 + 23 us, each a launch of its own; 55 + 17 now, 3.8
-// and 5.1 TB/s.
-// A tile inside one column -- columns worth normalising are long -- adds up in registers.
+// sums and division took 40 + 28 + 41 + 23 us, each a launch of its own.
 // Sums are of 64 bits, rounded once.
 struct ColumnTile {
   int64_t first, end, c0, c1;
@@ -639,10 +637,10 @@ struct ColumnTile {
 
 // The columns of a tile of kSumTile edges, with where they begin in the tile in LDS where
 // they fit.
-__device__ __forceinline__ ColumnTile column_tile(const int64_t* __restrict__ indptr,
+__device__ __forceinline__ ColumnTile column_tile(int64_t tile0, const int64_t* __restrict__ indptr,
                                                   int64_t num_cols, int64_t nnz, int32_t* begins) {
   ColumnTile t;
-  t.first = (int64_t)blockIdx.x * kSumTile;
+  t.first = tile0;
   t.end = t.first + kSumTile < nnz ? t.first + kSumTile : nnz;
   const SegmentSpan span = segment_span(indptr, num_cols, t.first, t.end - 1);
   t.c0 = span.lo;
@@ -674,100 +672,157 @@ __global__ __launch_bounds__(kBlock) void normalise_clear_kernel(double* sums, i
   if (i < n) sums[i] = 0.0;
 }
 
-template <bool kSelect, bool kDivide>
-__global__ __launch_bounds__(kBlock) void normalise_sum_kernel(
+// A wavefront adds up a run of kItems * 64 edges.  The look-up of its columns (two or three
+// loads, one behind the other) is on its way with the values; where columns meet the run goes
+// to LDS and is read back column by column, the short ones a lane each.  What bounds it is the
+// adds to one sum, 30 ns each: a column of a power law's hub has a sixth of all edges, and with
+// an add for every 2048 edges of it 7.1 M edges of 512 columns (28 MB) took 32 us.  So the
+// wavefronts of a work-group that are inside one column add once: 13 us.  37 K edges of as many
+// columns: 9.8 and 5.8 us, 10.7 with every column the whole wavefront's.
+// kItems: eight, which is eight million edges in the work-groups that are resident together,
+// or 32 beyond that (and on as few as four million, for fewer adds).
+constexpr int kRunItems = 8, kLongRunItems = 32;
+constexpr int64_t kLongRuns = int64_t(1) << 22;
+constexpr int kRunThreads = 512;
+template <bool kSelect, bool kDivide, int kItems>
+__global__ __launch_bounds__(kRunThreads) void normalise_sum_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols, const int64_t* __restrict__ rows,
     int64_t nnz, const float* __restrict__ values, int64_t num_values,
     const int64_t* __restrict__ select, const float* __restrict__ row_divisor,
     double* __restrict__ sums, float* __restrict__ out) {
-  __shared__ double acc[kSumSegs];
-  __shared__ int32_t begins[kSumSegs];
-  const int64_t tile0 = (int64_t)blockIdx.x * kSumTile;
-  float v[kSumItems];
-  int64_t at[kSumItems], row[kSumItems];
+  constexpr int kWaves = kRunThreads / kWave;
+  __shared__ float held[kWaves][kItems * kWave];
+  __shared__ double wave_sum[kWaves];
+  __shared__ int64_t wave_column[kWaves];  // -1: there is no such sum
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  float* const run = held[wave];
+  if (lane == 0) wave_column[wave] = -1;
+  const int64_t first =
+      wave_uniform_first(((int64_t)blockIdx.x * kWaves + wave) * (kItems * kWave));
+  if (first < nnz) {
+    const int64_t end = first + kItems * kWave < nnz ? first + kItems * kWave : nnz;
+    float v[kItems];
+    if (kSelect || kDivide) {
+      int64_t at[kItems], row[kItems];
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i) {
-    const int64_t e0 = tile0 + i * kBlock + threadIdx.x, e = e0 < nnz ? e0 : nnz - 1;
-    at[i] = kSelect ? select[e] : e;
-    row[i] = kDivide ? rows[e] : 0;
-  }
+      for (int i = 0; i < kItems; ++i) {
+        const int64_t e0 = first + i * kWave + lane, e = e0 < end ? e0 : end - 1;
+        at[i] = kSelect ? select[e] : e;
+        row[i] = kDivide ? rows[e] : 0;
+      }
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i)
-    v[i] = values[!kSelect || (uint64_t)at[i] < (uint64_t)num_values ? at[i] : 0];
-  if (kSelect) {  // (edge data may be shorter than the edges that `select` names)
+      for (int i = 0; i < kItems; ++i)
+        v[i] = values[!kSelect || (uint64_t)at[i] < (uint64_t)num_values ? at[i] : 0];
+      if (kSelect) {  // (edge data may be shorter than the edges that `select` names)
 #pragma unroll
-    for (int i = 0; i < kSumItems; ++i)
-      if ((uint64_t)at[i] >= (uint64_t)num_values) v[i] = 0.f;
-  }
-  if (kDivide) {
+        for (int i = 0; i < kItems; ++i)
+          if ((uint64_t)at[i] >= (uint64_t)num_values) v[i] = 0.f;
+      }
+      if (kDivide) {
 #pragma unroll
-    for (int i = 0; i < kSumItems; ++i) v[i] /= row_divisor[row[i]];
-  }
-  const ColumnTile t = column_tile(indptr, num_cols, nnz, begins);
+        for (int i = 0; i < kItems; ++i) v[i] /= row_divisor[row[i]];
+      }
+    } else if (end - first == kItems * kWave) {
+      const float* const from = values + first;
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i) {
-    const int64_t e = tile0 + i * kBlock + threadIdx.x;
-    if (e < t.end) {
-      if (kSelect || kDivide) out[e] = v[i];
+      for (int i = 0; i < kItems; ++i) v[i] = from[i * kWave + lane];
     } else {
-      v[i] = 0.f;
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int64_t e = first + i * kWave + lane;
+        v[i] = values[e < end ? e : end - 1];
+      }
+    }
+    const SegmentSpan span = segment_span(indptr, num_cols, first, end - 1);
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const int64_t e = first + i * kWave + lane;
+      if (e < end) {
+        if (kSelect || kDivide) out[e] = v[i];
+      } else {
+        v[i] = 0.f;
+      }
+    }
+    auto together = [](double mine) {  // the lanes' sum, in lane 0
+#pragma unroll
+      for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
+      return mine;
+    };
+    if (span.lo == span.hi) {
+      double mine = 0.0;
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) mine += (double)v[i];
+      mine = together(mine);
+      if (lane == 0) {
+        wave_sum[wave] = mine;
+        wave_column[wave] = span.lo;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) run[i * kWave + lane] = v[i];
+      wave_lds_fence();
+      // Few columns: sixteen lanes each, the long ones the wavefront; many: a lane or the wavefront.
+      constexpr int kFew = 16, kTeam = 16, kTeamLongest = 16 * kTeam;
+      const bool few = span.hi - span.lo < kFew;
+      const int longest = few ? kTeamLongest : kWave;  // of those that are not the wavefront's
+      for (int64_t c0 = span.lo; c0 <= span.hi; c0 += kWave) {
+        const int64_t c = c0 + lane <= span.hi ? c0 + lane : span.hi;
+        const int64_t s = indptr[c] > first ? indptr[c] : first;
+        const int64_t t = indptr[c + 1] < end ? indptr[c + 1] : end;
+        const int begin = (int)(s - first), n = c0 + lane <= span.hi && t > s ? (int)(t - s) : 0;
+        if (few) {
+          for (int c1 = 0; c1 <= span.hi - span.lo; c1 += kWave / kTeam) {
+            const int from = __shfl(begin, c1 + lane / kTeam, kWave);
+            const int many = __shfl(n, c1 + lane / kTeam, kWave);
+            if (many > longest) continue;  // (the same in all of a team)
+            double mine = 0.0;
+            for (int i = lane % kTeam; i < many; i += kTeam) mine += (double)run[from + i];
+#pragma unroll
+            for (int d = kTeam / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kTeam);
+            if (lane % kTeam == 0 && many > 0) unsafeAtomicAdd(sums + c0 + c1 + lane / kTeam, mine);
+          }
+        } else if (n > 0 && n <= longest) {
+          double mine = 0.0;
+          for (int i = 0; i < n; ++i) mine += (double)run[begin + i];
+          unsafeAtomicAdd(sums + c, mine);
+        }
+        for (uint64_t left = __ballot(n > longest); left; left &= left - 1) {
+          const int l = __builtin_ctzll(left);
+          const int from = __shfl(begin, l, kWave), many = __shfl(n, l, kWave);
+          double mine = 0.0;
+          for (int i = lane; i < many; i += kWave) mine += (double)run[from + i];
+          mine = together(mine);
+          if (lane == 0) unsafeAtomicAdd(sums + c0 + l, mine);
+        }
+      }
     }
   }
-  if (t.c0 == t.c1) {
-    double mine = 0.0;
-#pragma unroll
-    for (int i = 0; i < kSumItems; ++i) mine += (double)v[i];
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
-    if (lane_id() == 0) acc[threadIdx.x / kWave] = mine;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double sum = acc[0];
-#pragma unroll
-      for (int w = 1; w < kBlock / kWave; ++w) sum += acc[w];
-      unsafeAtomicAdd(sums + t.c0, sum);
-    }
-    return;
-  }
-  const int64_t n = t.c1 - t.c0 + 1;
-  if (t.in_lds)
-    for (int64_t j = threadIdx.x; j < n; j += kBlock) acc[j] = 0.0;
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kSumItems; ++i) {
-    const int64_t e = tile0 + i * kBlock + threadIdx.x;
-    const bool active = e < t.end;
-    const int c = active ? column_in_tile(t, indptr, begins, e) : -1;
-    const int first = __builtin_amdgcn_readfirstlane(c);
-    double sum = (double)v[i];
-    const bool together = __all(c == first) && first >= 0;  // one add a wavefront
-    if (together) {
-#pragma unroll
-      for (int d = kWave / 2; d > 0; d >>= 1) sum += __shfl_down(sum, d, kWave);
-    }
-    if (together ? lane_id() == 0 : active) {
-      if (t.in_lds) atomicAdd(&acc[c], sum);
-      else unsafeAtomicAdd(sums + t.c0 + c, sum);
-    }
-  }
-  if (!t.in_lds) return;
-  __syncthreads();
-  for (int64_t j = threadIdx.x; j < n; j += kBlock)
-    if (acc[j] != 0.0) unsafeAtomicAdd(sums + t.c0 + j, acc[j]);
+  if (threadIdx.x >= kWaves) return;
+  const int64_t c = wave_column[threadIdx.x];
+  if (c < 0 || (threadIdx.x > 0 && wave_column[threadIdx.x - 1] == c)) return;
+  double sum = wave_sum[threadIdx.x];
+  for (int w = threadIdx.x + 1; w < kWaves && wave_column[w] == c; ++w) sum += wave_sum[w];
+  unsafeAtomicAdd(sums + c, sum);
 }
 
+// group: so many tiles in a row were one work-group's of the sums, whose die has their values
+// (7.1 M edges: 17.2 us with the dies' tiles in turn, 15.4 so).
 __global__ __launch_bounds__(kBlock) void normalise_divide_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols, int64_t nnz,
-    const double* __restrict__ sums, const float* values, float* out) {
+    const double* __restrict__ sums, const float* values, float* out, unsigned group) {
   __shared__ int32_t begins[kSumSegs];
-  const int64_t tile0 = (int64_t)blockIdx.x * kSumTile;
+  const unsigned nth = blockIdx.x / kDies;  // of its die
+  const int64_t tile0 =
+      ((int64_t)(nth / group * kDies + blockIdx.x % kDies) * group + nth % group) * kSumTile;
+  if (tile0 >= nnz) return;
   float v[kSumItems];
 #pragma unroll
   for (int i = 0; i < kSumItems; ++i) {
     const int64_t e = tile0 + i * kBlock + threadIdx.x;
     v[i] = values[e < nnz ? e : nnz - 1];
   }
-  const ColumnTile t = column_tile(indptr, num_cols, nnz, begins);
+  const ColumnTile t = column_tile(tile0, indptr, num_cols, nnz, begins);
   const bool one = t.c0 == t.c1;
   float s = 0.f;
   if (one) s = (float)sums[t.c0];
@@ -1724,19 +1779,24 @@ int gs_normalise_columns_cleared(const int64_t* indptr, int64_t num_cols, const 
   GS_REQUIRE(num_values >= 1 && (select || num_values >= nnz), "normalise_columns: %lld values",
              (long long)num_values);
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)ceil_div(nnz, (int64_t)kSumTile));
-#define GS_NORMALISE_SUM(SELECT, DIVIDE)                                                     \
-  GS_LAUNCH("normalise_sum", s,                                                              \
-            (normalise_sum_kernel<SELECT, DIVIDE>)<<<grid, dim3(kBlock), 0, s>>>(            \
+  const bool moved = select || row_divisor, long_runs = !moved && nnz > kLongRuns;
+  const unsigned run = kRunThreads * (long_runs ? kLongRunItems : kRunItems);
+  const dim3 grid((unsigned)ceil_div(nnz, (int64_t)run));
+#define GS_NORMALISE_SUM(SELECT, DIVIDE, ITEMS)                                               \
+  GS_LAUNCH("normalise_sum", s,                                                               \
+            (normalise_sum_kernel<SELECT, DIVIDE, ITEMS>)<<<grid, dim3(kRunThreads), 0, s>>>( \
                 indptr, num_cols, rows, nnz, values, num_values, select, row_divisor, sums, out))
-  if (select && row_divisor) GS_NORMALISE_SUM(true, true);
-  else if (select) GS_NORMALISE_SUM(true, false);
-  else if (row_divisor) GS_NORMALISE_SUM(false, true);
-  else GS_NORMALISE_SUM(false, false);
+  if (select && row_divisor) GS_NORMALISE_SUM(true, true, kRunItems);
+  else if (select) GS_NORMALISE_SUM(true, false, kRunItems);
+  else if (row_divisor) GS_NORMALISE_SUM(false, true, kRunItems);
+  else if (!long_runs) GS_NORMALISE_SUM(false, false, kRunItems);
+  else GS_NORMALISE_SUM(false, false, kLongRunItems);
 #undef GS_NORMALISE_SUM
+  const unsigned group = run / kSumTile;
   GS_LAUNCH("normalise_divide", s,
-            normalise_divide_kernel<<<grid, dim3(kBlock), 0, s>>>(
-                indptr, num_cols, nnz, sums, select || row_divisor ? out : values, out));
+            normalise_divide_kernel<<<dim3((unsigned)ceil_div(grid.x, kDies) * kDies * group),
+                                      dim3(kBlock), 0, s>>>(
+                indptr, num_cols, nnz, sums, moved ? out : values, out, group));
   return GS_OK;
 }
 

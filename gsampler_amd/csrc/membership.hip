@@ -449,12 +449,6 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t set, uint32_t base) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)set, base));
 }
-// Between a wave's writes to its own part of LDS and its reads of other lanes' words.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // What the ids of a run are tested with: the table in LDS and a filter of all its ids
 // in front of it, or the table in L2 and the filter that the insert pass left.
 template <bool kInLds, int kThreads>

@@ -442,3 +442,11 @@ def test_normalised_columns_against_64_bits(degrees, select, divide):
     sums = torch.zeros(deg.numel(), dtype=torch.float64, device=DEV).index_add_(0, column, q)
     # the sum and the quotient are rounded once each
     torch.testing.assert_close(got.double(), q / sums[column], rtol=2.5 * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("degrees", [[2_500_000, 65, 1, 0, 64, 2_000_000, 17], [40] * 110_000,
+                                     [2048, 2047, 2, 63, 64, 65] * 1000 + [0, 1], [300, 0, 2, 2] * 14_500])
+def test_normalised_columns_of_long_runs(degrees):
+    """More edges than the short runs take on: runs of one column, of a few, and of hundreds."""
+    test_normalised_columns_against_64_bits(degrees, False, False)
