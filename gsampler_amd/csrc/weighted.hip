@@ -1789,7 +1789,9 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
   if (list_selects(n, num_segments, num_picks, replace)) {
     // few items per thread while that still fills the device, else sixteen (fewer
     // work-groups meet at the same histogram bins), eight where there are copies of those
-    const int items = n < (int64_t(1) << 20) ? 4 : w.copies > 1 ? 8 : 16;
+    // or sixteen would leave less than four work-groups a compute unit (eight segments of
+    // 233 K: bounds 25 us with sixteen and 16 with eight, emit 13 and 14)
+    const int items = n < (int64_t(1) << 20) ? 4 : w.copies > 1 || n < (int64_t(1) << 22) ? 8 : 16;
     // bins half a power of two wide, an eighth where many picks make candidates dear
     // (they are compared with one another): 233 K items 24 and 27 us with 400 picks, 69
     // and 58 with 2048

@@ -477,3 +477,14 @@ def test_operators_through_the_api():
     w_idx, w_ptr = orc.list_sample_weighted(np.ones(400, dtype=np.float32), 20, range_=ranges,
                                             seed=99, call_id=4)
     assert np.array_equal(idx.cpu().numpy(), w_idx)
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 1, 1 << 20, (1 << 22) - 1, 1 << 22])
+def test_batched_list_selection_where_the_items_a_thread_takes_change(n):
+    """Nine segments, whose borders are no tile's, with one histogram each."""
+    rng = np.random.default_rng(n)
+    ranges = np.sort(np.concatenate([[0, n], rng.integers(n // 9, n // 9 * 8, size=8)]))
+    probs = rng.random(n).astype(np.float32)
+    for k in (1, 256):
+        same(capi.list_sample_weighted(F(probs), k, range_=T(ranges), call_id=3),
+             orc.list_sample_weighted(probs, k, range_=ranges, call_id=3))
