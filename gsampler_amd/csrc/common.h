@@ -354,15 +354,21 @@ struct SliceView {
   };
   // Every lane of the wavefront must call this, with the same arguments.
   __device__ __forceinline__ Run run(int64_t first, int64_t last) const {
-    Run r;
     // the column of the first edge by a search; the last edge is nearly always
     // in the same column, which one more look at the pointer tells
     const int64_t first_u = wave_uniform_first(first), last_u = wave_uniform_first(last);
+    SegmentSpan span;
+    span.lo = wave_segment_of(sub_indptr, n, first_u);
+    span.hi = span.lo;
+    if (sub_indptr[span.lo + 1] <= last_u)
+      span.hi = span.lo + wave_segment_of(sub_indptr + span.lo, n - span.lo, last_u);
+    return run(first_u, span);
+  }
+  // The same where the columns of the run's first and last edge are known.
+  __device__ __forceinline__ Run run(int64_t first_u, SegmentSpan span) const {
+    Run r;
     r.first = first_u;
-    r.span.lo = wave_segment_of(sub_indptr, n, first_u);
-    r.span.hi = r.span.lo;
-    if (sub_indptr[r.span.lo + 1] <= last_u)
-      r.span.hi = r.span.lo + wave_segment_of(sub_indptr + r.span.lo, n - r.span.lo, last_u);
+    r.span = span;
     r.split = INT64_MAX;
     r.shift[0] = r.shift[1] = r.offset[0] = r.offset[1] = 0;
     r.count = 0;

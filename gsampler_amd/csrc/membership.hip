@@ -19,6 +19,7 @@
 // flag, and every match of the 32-bit halves is then confirmed against the
 // picked id itself.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "hashtable.h"
@@ -86,15 +87,28 @@ struct IdFilter {
     for (int i = 0; i < kBits; ++i) b |= 1u << ((h >> (13 - 5 * i)) & 31u);
     return b;
   }
-  __device__ __forceinline__ static bool passes(const uint32_t* words, uint32_t key) {
-    const uint32_t h = hash(key), w = words[word(h)];
+  // 1 or 0, by the word of the hash
+  __device__ __forceinline__ static uint32_t passes(uint32_t w, uint32_t, uint32_t h) {
     uint32_t all = 1u;
 #pragma unroll
     for (int i = 0; i < kBits; ++i) all &= w >> ((h >> (13 - 5 * i)) & 31u);
-    return all != 0u;
+    return all;
   }
 };
 using L2Filter = IdFilter<kFilterWords, kFilterBits>;
+
+// The same for a few ids, one bit each: the key's low bits say which, of the word that a product
+// of 24 bits names (one of 32 takes the time of four other instructions).
+template <int kWords>
+struct FewIdFilter {
+  static_assert((kWords & (kWords - 1)) == 0, "the top bits of a product are a word");
+  __device__ __forceinline__ static uint32_t hash(uint32_t key) { return __umul24(key, 0x9E3779u); }
+  __device__ __forceinline__ static uint32_t word(uint32_t h) { return h >> (32 - __builtin_ctz(kWords)); }
+  __device__ __forceinline__ static uint32_t bits(uint32_t key) { return 1u << (key & 31u); }
+  __device__ __forceinline__ static uint32_t passes(uint32_t w, uint32_t key, uint32_t) {
+    return (w >> (key & 31u)) & 1u;
+  }
+};
 
 // Up to this many chunks the offsets of chunks and columns take one launch
 // (member_offsets_kernel), in which a work-group adds up the counts of all chunks before
@@ -391,26 +405,33 @@ struct BucketTable {
 #pragma unroll
     for (int j = 0; j < kShare; ++j) {
       const uint32_t i = j * kThreads + threadIdx.x;
-      if (i >= num_picked) continue;
-      const uint32_t first = find(member_tag(id[j]));
-      if (first != slot[j]) atomicMin(&lds_values[first], i);
+      if ((uint32_t)(j * kThreads) >= num_picked) break;
+      const uint32_t first = find(i < num_picked ? member_tag(id[j]) : kNoKey);
+      if (i < num_picked && first != slot[j]) atomicMin(&lds_values[first], i);
     }
     __syncthreads();
     return false;
   }
 
-  // Where a key sits, kMemberLdsSlots when it is absent (or kNoKey).
+  // Where a key sits, kMemberLdsSlots when it is absent (or kNoKey).  Every lane of the
+  // wavefront calls this.  The first bucket is read whole, in one instruction and without a
+  // branch: compares that end early were four reads one behind the other.
   __device__ __forceinline__ uint32_t find(uint32_t key) const {
     uint32_t b = home(key);
-    if (key == kNoKey) return kMemberLdsSlots;
-    for (int rounds = 0; rounds < kMemberBuckets; ++rounds) {
-      const uint4 k = keys[b];
-      const uint32_t hit = place_in(k, key);
-      if (hit < 4u) return b * 4 + hit;
-      if (k.w == kNoKey) break;  // a bucket with room would hold the key
+    uint4 k = keys[b];
+    asm volatile("" : "+v"(k.x), "+v"(k.y), "+v"(k.z), "+v"(k.w));
+    uint32_t hit = place_in(k, key);
+    uint32_t slot = hit < 4u && key != kNoKey ? b * 4 + hit : (uint32_t)kMemberLdsSlots;
+    bool on = hit == 4u && k.w != kNoKey && key != kNoKey;  // (a bucket with room would hold the key)
+    for (int rounds = 1; rounds < kMemberBuckets && __any(on); ++rounds) {
+      if (!on) continue;
       b = (b + 1) & (kMemberBuckets - 1);
+      k = keys[b];
+      hit = place_in(k, key);
+      if (hit < 4u) slot = b * 4 + hit;
+      on = hit == 4u && k.w != kNoKey;
     }
-    return kMemberLdsSlots;
+    return slot;
   }
 
   // The smallest position of an id among ids that may not fit 32 bits, kNoKey when it is
@@ -449,33 +470,146 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t set, uint32_t base) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)set, base));
 }
+// An index of a slice's pointer in LDS: every entry of it up to kEntries, and some of them
+// beyond that.
+template <int kThreads>
+struct PointerIndex {
+  static constexpr int kShare = kMemberWords, kEntries = kThreads * kShare;
+  uint32_t entries, step;  // none: 0
+  uint32_t own[kShare];    // entries j * kThreads + threadIdx.x
+  __device__ __forceinline__ void request(const int64_t* __restrict__ ptr, int64_t n, int64_t nnz) {
+    const bool fits = n > 0 && nnz <= (int64_t)UINT32_MAX && n <= (int64_t)UINT32_MAX / 2;
+    step = fits ? (uint32_t)((n + kEntries - 1) / kEntries) : 0u;
+    entries = fits ? (uint32_t)((n + step - 1) / step) : 0u;
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const uint32_t i = j * kThreads + threadIdx.x;
+      own[j] = i < entries ? (uint32_t)ptr[(int64_t)i * step] : 0u;
+    }
+  }
+  __device__ __forceinline__ void place(uint32_t* lds) const {
+#pragma unroll
+    for (int j = 0; j < kShare; ++j) {
+      const uint32_t i = j * kThreads + threadIdx.x;
+      if (i < entries) lds[i] = own[j];
+    }
+  }
+};
+// Where runs of kRunEdges edges lie in the columns of a slice that is read in place, by their
+// numbers among a work-group's.
+template <int kRuns, int kRunEdges>
+struct RunColumns {
+  int64_t shift[2][kRuns];  // of the first two columns
+  uint32_t lo[kRuns], more[kRuns];  // the first edge's column; how many further on the last one's is
+  uint32_t split[kRuns];    // edges before the second column
+  // A thread looks up one run.
+  template <typename Index>
+  __device__ __forceinline__ void find(const SliceView& view, int64_t nnz, int64_t run, int number,
+                                       const uint32_t* lds, const Index& index) {
+    const int64_t first = run * kRunEdges;
+    const int64_t last = (first + kRunEdges < nnz ? first + kRunEdges : nnz) - 1;
+    // the last columns that begin at or before the two edges
+    int64_t c[2] = {0, 0}, end[2] = {view.n, view.n};
+    if (lds && index.entries > 0) {
+      uint32_t at[2] = {0, 0};
+      for (uint32_t step = 1u << (31 - __builtin_clz(index.entries)); step > 0; step >>= 1) {
+        uint32_t probe[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          probe[k] = at[k] + step < index.entries ? lds[at[k] + step] : UINT32_MAX;
+        at[0] = at[0] + step < index.entries && (int64_t)probe[0] <= first ? at[0] + step : at[0];
+        at[1] = at[1] + step < index.entries && (int64_t)probe[1] <= last ? at[1] + step : at[1];
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        c[k] = (int64_t)at[k] * index.step;
+        if (c[k] + index.step < view.n) end[k] = c[k] + index.step;
+      }
+    }
+    while (end[0] - c[0] > 1 || end[1] - c[1] > 1) {
+      int64_t mid[2], begins[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        mid[k] = (c[k] + end[k]) >> 1;  // (c[k] itself where it is found)
+        begins[k] = view.sub_indptr[mid[k]];
+      }
+      if (begins[0] <= first) c[0] = mid[0];
+      else end[0] = mid[0];
+      if (begins[1] <= last) c[1] = mid[1];
+      else end[1] = mid[1];
+    }
+    int64_t start[2], id[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      start[k] = view.sub_indptr[c[k]];
+      id[k] = view.cols[c[k]];
+    }
+    // (an id outside the matrix is an empty column: neither edge lies in one)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) shift[k][number] = view.indptr[id[k]] - start[k];
+    lo[number] = (uint32_t)c[0];
+    more[number] = (uint32_t)(c[1] - c[0]);
+    split[number] = (uint32_t)(start[1] - first);
+  }
+  __device__ __forceinline__ SliceView::Run run(const SliceView& view, int64_t first, int number) const {
+    auto of = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+    SegmentSpan span;
+    span.lo = of(lo[number]);
+    span.hi = span.lo + of(more[number]);
+    if (span.hi - span.lo > 1) return view.run(first, span);
+    SliceView::Run r{};
+    r.first = first;
+    r.span = span;
+    r.split = span.hi != span.lo ? first + of(split[number]) : INT64_MAX;
+    r.shift[0] = wave_uniform_first(shift[0][number]);
+    r.shift[1] = wave_uniform_first(shift[1][number]);
+    if (view.key_offset) {
+      r.offset[0] = view.key_offset[span.lo];
+      r.offset[1] = view.key_offset[span.hi];
+    }
+    return r;
+  }
+};
+
 // What the ids of a run are tested with: the table in LDS and a filter of all its ids
 // in front of it, or the table in L2 and the filter that the insert pass left.
-template <bool kInLds, int kThreads>
+// kRunEdges: of the runs whose columns are looked up for a work-group; none: 0.
+template <bool kInLds, int kThreads, int kRunEdges>
 struct MemberShared {
-  static constexpr int kWords = !kInLds ? kFilterWords : kThreads == kMemberThreads ? 4096 : 2048;
-  using Filter = IdFilter<kWords, kInLds ? 2 : kFilterBits>;
+  static constexpr int kWords = !kInLds ? kFilterWords : kThreads == kMemberThreads ? 2048 : 1024;
+  static constexpr int kRuns = kThreads / (kInLds ? 4 : 8);  // looked up at a time
+  using Filter = std::conditional_t<kInLds, FewIdFilter<kInLds ? kWords : 1>, L2Filter>;
+  // (the queues lie within the reach of an instruction's offset)
+  uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
+  uint8_t queue_place[kThreads * kMemberWords];
   __align__(16) uint32_t keys[kInLds ? kMemberLdsSlots : 4];
   uint32_t values[kInLds ? kMemberLdsSlots : 4];
   uint32_t first[kInLds ? kMemberLdsIds : 4];  // first edge kept by each picked id
   __align__(16) uint32_t filter[kWords];
-  uint32_t queue_key[kThreads * kMemberWords];   // a chunk's worth per wave
-  uint8_t queue_place[kThreads * kMemberWords];
+  RunColumns<(kRunEdges > 0 ? kRuns : 1), kRunEdges> columns;
+  uint32_t next_run;  // of the work-group's, for the next wavefront that is done with its own
 };
 // Work-groups that a compute unit holds, with 160 KB of LDS and 2048 threads: two of 1024
 // threads, of kBlock threads three with the table in LDS and two with the filter.
 template <bool kInLds, int kThreads>
-constexpr int kMemberResident = std::min(160 * 1024 / (int)sizeof(MemberShared<kInLds, kThreads>),
-                                         2048 / kThreads);
+constexpr int kMemberResident =
+    std::min(160 * 1024 / (int)sizeof(MemberShared<kInLds, kThreads, 1>), 2048 / kThreads);
+static_assert(kMemberResident<true, kMemberThreads> == 2 && kMemberResident<false, kMemberThreads> == 2 &&
+                  kMemberResident<true, kBlock> == 3,
+              "what the figures were measured with");
 
 // Whether a row of 64 edges holds picked ids is told by the filter, a word of LDS and
 // eight instructions an edge; the edges that pass are packed into the wave's queue, and
 // only they, 64 at a time, go through a look-up and are written out.  Most edges of a
-// slice are not kept, and the pass is bound by the instructions it issues: with a look-up
-// for every row 78 vector and 38 scalar instructions a row and 91 us on 31 M edges of which
-// a quarter is kept (two thirds of it the vector units), 66 on 19 M with one kept in
-// twenty-five; now 42 and 30, 64 us and 43 (reading the ids and writing what is kept take 33
-// and 17 at the rate of a copy).  Behind the filter, table in L2: 83 -> 52 on 18.5 M edges.
+// slice are not kept, and the pass is bound by the instructions it issues, which keep the
+// vector units busy for two thirds of it: with a look-up for every row 91 us on 31 M edges of
+// which a quarter is kept and 66 on 20 M with one kept in twenty-five, with the queue 67 and 36,
+// with the columns of runs told beforehand, runs that the wavefronts take one by one and the
+// words of the filter read together 51 and 34 (reading the ids and writing what is kept take 33
+// and 17 at the rate of a copy; the table, the filter and the columns 6).  Ids of the next run
+// asked for ahead, for registers that then spill, were slower: 58 and 38.  Behind the filter,
+// table in L2: 83 -> 52 on 18.5 M edges, and where columns are short, 8.4 M edges of 19 K
+// columns, 43 -> 38 (a run of two columns waited for its loads one by one).
 // kThreads: work-group size.  A large one shares a staged table among more
 // edges; a small one spreads a short edge list over all compute units.
 // kRun: chunks per wave and run, whose ids are in flight together.
@@ -490,13 +624,18 @@ void member_flag_kernel(
     int64_t* __restrict__ chunk_count, uint16_t* __restrict__ chunk_kept,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
     const uint32_t* __restrict__ filter, uint32_t* __restrict__ firsts, SliceView view) {
-  using Shared = MemberShared<kInLds, kThreads>;
+  constexpr int kRunEdges = kRun * kBlock;
+  // (small ones have about a run a wavefront, which looks it up for itself: 4 us less on 0.3 M edges)
+  constexpr bool kTold = kView && kThreads == kMemberThreads;  // the columns of runs, by RunColumns
+  using Shared = MemberShared<kInLds, kThreads, kTold ? kRunEdges : 0>;
   using Filter = typename Shared::Filter;
   __shared__ Shared sh;
   const bool filtered = kInLds || filter != nullptr;
   const MemberTable table{global_table, cap};
   BucketTable buckets;
   bool wide;  // the same for every thread of the launch
+  PointerIndex<kThreads> index;
+  if (kTold) index.request(view.sub_indptr, view.n, nnz);
   if (kInLds) {
     static_assert(sizeof(sh.queue_key) >= kMemberBuckets * sizeof(uint32_t), "counters lie there");
     for (int i = threadIdx.x; i < Shared::kWords; i += kThreads) sh.filter[i] = 0u;
@@ -504,8 +643,8 @@ void member_flag_kernel(
       for (uint32_t i = threadIdx.x; i < num_picked; i += kThreads) sh.first[i] = UINT32_MAX;
     wide = buckets.template stage<kThreads>(
         picked, num_picked, sh.keys, sh.values, sh.queue_key, [&](uint32_t key) {
-          const uint32_t h = Filter::hash(key);
-          return (~atomicOr(&sh.filter[Filter::word(h)], Filter::bits(h)) & Filter::bits(h)) == 0u;
+          const uint32_t h = Filter::hash(key), bit = Filter::bits(key);
+          return (~atomicOr(&sh.filter[Filter::word(h)], bit) & bit) == 0u;
         });
   } else {
     wide = *wide_flag != 0;
@@ -529,60 +668,60 @@ void member_flag_kernel(
   const int lane = lane_id();
   const int wave = threadIdx.x / kWave;
   const uint32_t queue0 = wave_uniform_first(wave * kBlock);  // where this wave's queue starts
-  // A wave takes runs of kRun chunks, the waves of the launch striding over them (a launch
-  // with fewer waves than runs stages its tables once per work-group, not once per run).
-  // The short columns of a slice are often neighbours, and a wave that took neighbouring
-  // runs would be at them when all others have ended (126 us where this takes 69).
-  constexpr int kRunEdges = kRun * kBlock;
+  // A work-group takes runs of kRun chunks, the work-groups of the launch striding over them
+  // (a launch with fewer work-groups than would have a run a wavefront stages its tables once
+  // for many; neighbouring runs are the short columns' in one and long ones' in another: 126 us
+  // where strides took 69).  Its wavefronts take them from it one by one: with as many for each
+  // the last ended at 55 us where half were done at 40 (31 M edges), and at 37 for 25 (19 M).
   const int64_t num_runs = ceil_div_dev(num_chunks, kRun);
-  const int64_t waves = (int64_t)gridDim.x * (kThreads / kWave);
-  const int64_t self = wave_uniform_first((int64_t)blockIdx.x * (kThreads / kWave) + wave);
 
-  int kept = 0;  // of the chunk at hand; the same in every lane
-  // writes the lanes' edges that were found behind the chunk's others
-  auto keep = [&](int64_t chunk, bool found, uint32_t value, uint32_t place) {
+  // What is kept of the chunks at hand, the same in every lane; the first of two counts alone.
+  int kept = 0, kept_first = 0;
+  // writes the lanes' edges that were found behind the others; `second`: of the chunk behind
+  // the first of two, which all lanes of that follow
+  auto keep = [&](int64_t chunk, bool found, bool second, uint32_t value, uint32_t place) {
     const uint64_t peers = __ballot(found);
+    kept_first += __popcll(peers & ~__ballot(second));
     if (found) {
-      const uint32_t at = lanes_below(peers, kept);
+      const uint32_t at = lanes_below(peers, kept) + (second ? kBlock - kept_first : 0);
       (staged + chunk * kBlock)[at] = value;
       (staged_pos + chunk * kBlock)[at] = (uint8_t)place;
       if (kInLds && firsts) {
-        const uint32_t e = (uint32_t)(chunk * kBlock) + place;
+        const uint32_t e = (uint32_t)(chunk * kBlock) + place + (second ? kBlock : 0);
         if (sh.first[value] > e) atomicMin(&sh.first[value], e);
       }
     }
     kept += __popcll(peers);
   };
-  auto finish_chunk = [&](int64_t chunk) {
-    if (lane == 0) {
-      if (chunk_kept) {
-        chunk_kept[chunk] = (uint16_t)kept;
-      } else {
-        chunk_count[chunk] = kept;
-        if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
-      }
+  auto finish_chunk = [&](int64_t chunk, int count) {
+    if (chunk_kept) {
+      chunk_kept[chunk] = (uint16_t)count;
+    } else {
+      chunk_count[chunk] = count;
+      if (chunk == num_chunks - 1) chunk_count[num_chunks] = 0;
     }
-    kept = 0;
   };
-  auto flag_chunk = [&](int64_t chunk, const uint32_t (&key)[kMemberWords]) {
-    uint32_t end = queue0;
-#pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      const bool may = !filtered || Filter::passes(sh.filter, key[j]);
-      const uint64_t peers = __ballot(may);
-      if (may) {
-        const uint32_t at = lanes_below(peers, end);
-        sh.queue_key[at] = key[j];
-        sh.queue_place[at] = (uint8_t)(j * kWave + lane);
-      }
-      end += __popcll(peers);
+  // The edges of a chunk that the filter lets through are queued and looked up, 64 at a time;
+  // those of two chunks together where the queue holds them: of one chunk few pass, or a few
+  // more than one look-up takes.
+  uint32_t end = queue0, second0 = ~0u;  // of the queue; where the second chunk's begin in it
+  auto enqueue = [&](bool may, uint32_t key, int row) {
+    const uint64_t peers = __ballot(may);
+    if (may) {
+      const uint32_t at = lanes_below(peers, end);
+      sh.queue_key[at] = key;
+      sh.queue_place[at] = (uint8_t)(row * kWave + lane);
     }
+    end += __popcll(peers);
+  };
+  auto look_up = [&](int64_t chunk) {
     wave_lds_fence();
     if (kInLds) {
       for (uint32_t q0 = queue0; q0 < end; q0 += kWave) {
         const uint32_t q = q0 + lane < end ? q0 + lane : end - 1;
         const uint32_t slot = buckets.find(q0 + lane < end ? sh.queue_key[q] : kNoKey);
-        keep(chunk, slot < kMemberLdsSlots, sh.values[slot & (kMemberLdsSlots - 1)], sh.queue_place[q]);
+        keep(chunk, slot < kMemberLdsSlots, q >= second0,
+             sh.values[slot & (kMemberLdsSlots - 1)], sh.queue_place[q]);
       }
     } else {
       // a table in L2 answers after a round trip: two edges a lane go through their
@@ -599,11 +738,52 @@ void member_flag_kernel(
         }
         table.find_many(k, slot, value);
 #pragma unroll
-        for (int i = 0; i < kN; ++i) keep(chunk, slot[i] < cap, value[i], place[i]);
+        for (int i = 0; i < kN; ++i)
+          keep(chunk, slot[i] < cap, q0 + i * kWave + lane >= second0, value[i], place[i]);
       }
     }
-    wave_lds_fence();  // the next chunk's queue overwrites this one's
-    finish_chunk(chunk);
+    wave_lds_fence();  // the next queue overwrites this one
+    if (lane == 0) {
+      finish_chunk(chunk, kept_first);
+      if (second0 != ~0u) finish_chunk(chunk + 1, kept - kept_first);
+    }
+    kept = kept_first = 0;
+    end = queue0;
+    second0 = ~0u;
+  };
+  // Not 0 where the filter lets a key through.  (The words are read together: a queue's writes
+  // behind each would be waited for by the next.)
+  auto test = [&](const auto& key, auto& may) {
+    constexpr int kKeys = sizeof(key) / sizeof(uint32_t);
+    const uint32_t(&k)[kKeys] = reinterpret_cast<const uint32_t(&)[kKeys]>(key);
+    uint32_t(&m)[kKeys] = reinterpret_cast<uint32_t(&)[kKeys]>(may);
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j) m[j] = filtered ? sh.filter[Filter::word(Filter::hash(k[j]))] : 1u;
+    if (!filtered) return;
+#pragma unroll
+    for (int j = 0; j < kKeys; ++j) m[j] = Filter::passes(m[j], k[j], Filter::hash(k[j]));
+  };
+  auto flag_chunk = [&](int64_t chunk, const uint32_t (&key)[kMemberWords]) {
+    uint32_t may[kMemberWords];
+    test(key, may);
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) enqueue(may[j] != 0u, key[j], j);
+    look_up(chunk);
+  };
+  auto flag_two_chunks = [&](int64_t chunk, const uint32_t (&key)[2][kMemberWords]) {
+    uint32_t may[2][kMemberWords];
+    test(key, may);
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) enqueue(may[0][j] != 0u, key[0][j], j);
+    uint32_t after = end;
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) after += __popcll(__ballot(may[1][j] != 0u));
+    const bool together = after - queue0 <= kBlock;
+    if (together) second0 = end;
+    else look_up(chunk);
+#pragma unroll
+    for (int j = 0; j < kMemberWords; ++j) enqueue(may[1][j] != 0u, key[1][j], j);
+    look_up(together ? chunk : chunk + 1);
   };
 
   // A run over several columns, or of a call with wide ids.
@@ -638,7 +818,8 @@ void member_flag_kernel(
         for (int j = 0; j < kMemberWords; ++j) {
           bool in;
           const uint64_t id = id_of(chunk * kBlock + j * kWave, &in);
-          const bool may = in && (!filtered || Filter::passes(sh.filter, member_tag(id)));
+          const uint32_t h = Filter::hash(member_tag(id));
+          const bool may = in && (!filtered || Filter::passes(sh.filter[Filter::word(h)], member_tag(id), h) != 0u);
           uint32_t value = kNoKey;
           if (may && kInLds) {
             value = buckets.find_confirmed(id, picked);
@@ -646,22 +827,56 @@ void member_flag_kernel(
             const uint32_t slot = table.find_confirmed(id, picked);
             if (slot < cap) value = table.value_at(slot);
           }
-          keep(chunk, value != kNoKey, value, j * kWave + lane);
+          keep(chunk, value != kNoKey, false, value, j * kWave + lane);
         }
-        finish_chunk(chunk);
+        if (lane == 0) finish_chunk(chunk, kept);
+        kept = kept_first = 0;
       }
     }
   };
 
-  for (int64_t run = self; run < num_runs; run += waves) {
+  // Of a slice that is read in place the columns of kRuns runs are told at once, a thread a
+  // run: six loads one behind the other for each run as it came, which eight wavefronts a SIMD
+  // hid in part (31 M edges: 66 us, 57 with the look-ups ahead).
+  const int64_t own_runs =
+      num_runs > blockIdx.x ? (num_runs - 1 - blockIdx.x) / gridDim.x + 1 : 0;
+  int64_t run0 = 0;  // of those looked up
+  auto prepare_runs = [&](const uint32_t* lds) {
+    if (threadIdx.x == 0) sh.next_run = 0;
+    if (kTold && threadIdx.x < Shared::kRuns && run0 + threadIdx.x < own_runs)
+      sh.columns.find(view, nnz, blockIdx.x + (run0 + threadIdx.x) * gridDim.x, threadIdx.x, lds, index);
+    __syncthreads();
+  };
+  if (kTold) {
+    index.place(sh.queue_key);
+    __syncthreads();
+  }
+  prepare_runs(sh.queue_key);
+  for (;;) {
+    // (the compiler must not join what lane 0 alone does here and at the end of a run: it has
+    // made a loop of the other lanes, in which the number is always 0)
+    __builtin_amdgcn_wave_barrier();
+    uint32_t number = 0;
+    if (lane == 0) number = atomicAdd(&sh.next_run, 1u);
+    __builtin_amdgcn_wave_barrier();
+    number = __builtin_amdgcn_readfirstlane(number);
+    if (kTold && number >= (uint32_t)Shared::kRuns) {  // every wavefront comes here, or none
+      if (run0 + Shared::kRuns >= own_runs) break;
+      __syncthreads();
+      run0 += Shared::kRuns;
+      prepare_runs(nullptr);
+      continue;
+    }
+    if (run0 + number >= own_runs) break;
+    const int64_t run = blockIdx.x + (run0 + number) * gridDim.x;
     const int64_t chunk0 = run * kRun, e_first = run * kRunEdges;
     const bool whole = e_first + kRunEdges <= nnz;
-    // With a view the edges are those of a column slice that was never written:
-    // the run's columns are looked up once, and an edge's id
-    // is read from the parent's array.
+    // With a view the edges are those of a column slice that was never written, and an
+    // edge's id is read from the parent's array.
     SliceView::Run vrun{};
     vrun.split = INT64_MAX;  // no view: every edge at distance 0, offset 0
-    if (kView) vrun = view.run(e_first, (whole ? e_first + kRunEdges : nnz) - 1);
+    if constexpr (kTold) vrun = sh.columns.run(view, e_first, (int)number);
+    else if (kView) vrun = view.run(e_first, (whole ? e_first + kRunEdges : nnz) - 1);
     if (wide || (kView && !vrun.near())) {
       slow_run(run, vrun);
       continue;
@@ -690,19 +905,21 @@ void member_flag_kernel(
       for (int c = 0; c < kRun; ++c)
 #pragma unroll
         for (int j = 0; j < kMemberWords; ++j) {
-          const int64_t e = (chunk0 + c) * kBlock + j * kWave + lane;
-          if (kView) {
-            keys[c][j] = e >= nnz ? kNoKey
-                                  : member_key((uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e)));
-          } else {  // (a lane past the end reads the last edge: a branch would wait for the load in it)
-            const uint32_t key = member_key((uint64_t)(int64_t)ids[e < nnz ? e : nnz - 1]);
-            keys[c][j] = e < nnz ? key : kNoKey;
-          }
+          // (a lane past the end reads the last edge: a branch would wait for the load in it)
+          const int64_t at = (chunk0 + c) * kBlock + j * kWave + lane, e = at < nnz ? at : nnz - 1;
+          const uint32_t key = member_key(
+              kView ? (uint64_t)((int64_t)ids[vrun.place(e)] + vrun.id_offset(e)) : (uint64_t)(int64_t)ids[e]);
+          keys[c][j] = at < nnz ? key : kNoKey;
         }
     }
-#pragma unroll
-    for (int c = 0; c < kRun; ++c)
-      if (chunk0 + c < num_chunks) flag_chunk(chunk0 + c, keys[c]);
+    static_assert(kRun <= 2, "two chunks meet in the queue");
+    if constexpr (kRun == 2) {
+      if (chunk0 + 1 < num_chunks) {
+        flag_two_chunks(chunk0, keys);
+        continue;
+      }
+    }
+    flag_chunk(chunk0, keys[0]);
   }
   if (kInLds && firsts) {
     __syncthreads();

@@ -978,3 +978,32 @@ def handed_on_by_operators(compiled):
     other = copy.copy(compiled)
     other._run = None  # the operator graph itself
     return other
+
+
+@pytest.mark.parametrize("lengths,picks", [([4_000_000], 300), ([4_000_000, 0, 700_001], 2048), ([1, 300, 0, 513, 2000, 90], 300),
+                                           ([4_000_000, 3], 4000), ([700, 0, 255, 40], 4000)])
+@pytest.mark.parametrize("narrow", [False, True])
+def test_row_slices_whose_work_groups_look_up_their_runs_in_several_rounds(lengths, picks, narrow):
+    """More than 67 M edges between picked columns that repeat: of a few long columns and of
+    many that meet in a run, with the table in LDS and in L2, by ids of both widths."""
+    g = torch.Generator(device=DEV).manual_seed(picks + len(lengths))
+    deg = torch.tensor(lengths, device=DEV)
+    indptr = torch.zeros(deg.numel() + 1, dtype=torch.int64, device=DEV)
+    torch.cumsum(deg, 0, out=indptr[1:])
+    indices = torch.randint(0, 100_000, (int(indptr[-1]),), generator=g, device=DEV)
+    rows = torch.randint(0, 100_000, (picks,), generator=g, device=DEV)
+    cols = torch.arange(len(lengths), device=DEV).repeat(70_000_000 // int(indptr[-1]) + 1)
+    got = capi.col_row_slice(indptr, indices, cols, rows, with_major=False,
+                             indices32=indices.to(torch.int32) if narrow else None)
+    place = torch.full((100_000,), picks, dtype=torch.int64, device=DEV)
+    place.scatter_reduce_(0, rows, torch.arange(picks, device=DEV), "amin")
+    kept = torch.nonzero(place[indices] < picks).flatten()
+    kept_ptr = torch.searchsorted(kept, indptr)
+    count = (kept_ptr[1:] - kept_ptr[:-1])[cols]
+    want_ptr = torch.zeros(cols.numel() + 1, dtype=torch.int64, device=DEV)
+    torch.cumsum(count, 0, out=want_ptr[1:])
+    assert torch.equal(got[0], want_ptr)
+    select = kept[torch.arange(int(want_ptr[-1]), device=DEV)
+                  + torch.repeat_interleave(kept_ptr[cols] - want_ptr[:-1], count)]
+    assert torch.equal(got[3], select)
+    assert torch.equal(got[2], place[indices[select]])
