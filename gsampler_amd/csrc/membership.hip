@@ -116,12 +116,14 @@ struct FewIdFilter {
 // at the bound, where three launches that read every count once take 15.2).
 constexpr int64_t kOffsetsMaxChunks = int64_t(1) << 17;
 
+constexpr int kRecordWords = 4;  // of a RunRecord, 64 bits each
 struct MemberWs {
   uint64_t* table;     // [member_table_slots(num_picked)], a table in L2
   uint32_t* staged;    // [chunks * kBlock]: per chunk, the new ids of its kept edges, in order
   uint8_t* staged_pos;  // [chunks * kBlock]: and their places in the chunk
   int64_t* chunk_off;  // [chunks + 1]
   uint16_t* chunk_kept;  // [chunks] kept edges of a chunk, for lists of up to kOffsetsMaxChunks
+  struct RunRecord* records;  // [chunks / kMemberLongRun] of a long slice that is read in place
   int* wide;           // [1] set when a picked id does not fit the upper half of a slot
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
   uint32_t* firsts;    // [first_groups * num_picked] per work-group of the flag pass, the first edge it kept by each id
@@ -148,6 +150,12 @@ static uint64_t member_table_slots(int64_t num_picked) {
   return (uint64_t)((num_picked <= kMemberRoomyIds ? 4 : 2) * num_picked + 2);
 }
 
+// Whether the flag pass leaves a RunRecord of every run.  (Their columns are 32 bits wide.)
+static bool member_columns_fit(const SliceView& view) { return view.n <= (int64_t)UINT32_MAX; }
+static bool member_told(int64_t nnz, const SliceView& view) {
+  return view.sub_indptr != nullptr && nnz >= kMemberSmallEdges && member_columns_fit(view);
+}
+
 // firsts: with room for first edges, behind the rest, which lies where it does without.
 static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked, bool firsts = false) {
   Carver c(ws);
@@ -159,6 +167,8 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked, bool fir
   w.chunk_off = c.take<int64_t>((size_t)w.chunks + 1);
   w.chunk_kept =
       c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
+  w.records = (RunRecord*)c.take<uint64_t>(
+      nnz >= kMemberSmallEdges ? (size_t)ceil_div(w.chunks, kMemberLongRun) * kRecordWords : 0);
   w.wide = c.take<int>(1);
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
@@ -495,8 +505,35 @@ struct PointerIndex {
     }
   }
 };
-// Where runs of kRunEdges edges lie in the columns of a slice that is read in place, by their
-// numbers among a work-group's.
+// Where a run of edges lies in the columns of a slice that is read in place.  The flag pass of a
+// long slice looks them up and leaves them for the passes over what it kept.
+struct __align__(16) RunRecord {
+  int64_t shift[2];   // of the first two columns
+  uint32_t lo, more;  // the first edge's column; how many further on the last one's is
+  uint32_t split;     // edges before the second column
+  uint32_t unused;
+  // The same record for every lane of the wavefront.
+  __device__ __forceinline__ SliceView::Run run(const SliceView& view, int64_t first) const {
+    auto of = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+    SegmentSpan span;
+    span.lo = of(lo);
+    span.hi = span.lo + of(more);
+    if (span.hi - span.lo > 1) return view.run(first, span);
+    SliceView::Run r{};
+    r.first = first;
+    r.span = span;
+    r.split = span.hi != span.lo ? first + of(split) : INT64_MAX;
+    r.shift[0] = wave_uniform_first(shift[0]);
+    r.shift[1] = wave_uniform_first(shift[1]);
+    if (view.key_offset) {
+      r.offset[0] = view.key_offset[span.lo];
+      r.offset[1] = view.key_offset[span.hi];
+    }
+    return r;
+  }
+};
+static_assert(sizeof(RunRecord) == kRecordWords * sizeof(uint64_t), "the workspace holds them");
+// Those of a work-group's runs of kRunEdges edges, by their numbers.
 template <int kRuns, int kRunEdges>
 struct RunColumns {
   int64_t shift[2][kRuns];  // of the first two columns
@@ -505,7 +542,8 @@ struct RunColumns {
   // A thread looks up one run.
   template <typename Index>
   __device__ __forceinline__ void find(const SliceView& view, int64_t nnz, int64_t run, int number,
-                                       const uint32_t* lds, const Index& index) {
+                                       const uint32_t* lds, const Index& index,
+                                       RunRecord* __restrict__ records) {
     const int64_t first = run * kRunEdges;
     const int64_t last = (first + kRunEdges < nnz ? first + kRunEdges : nnz) - 1;
     // the last columns that begin at or before the two edges
@@ -545,29 +583,18 @@ struct RunColumns {
       id[k] = view.cols[c[k]];
     }
     // (an id outside the matrix is an empty column: neither edge lies in one)
-#pragma unroll
-    for (int k = 0; k < 2; ++k) shift[k][number] = view.indptr[id[k]] - start[k];
-    lo[number] = (uint32_t)c[0];
-    more[number] = (uint32_t)(c[1] - c[0]);
-    split[number] = (uint32_t)(start[1] - first);
+    const RunRecord r{{view.indptr[id[0]] - start[0], view.indptr[id[1]] - start[1]},
+                      (uint32_t)c[0], (uint32_t)(c[1] - c[0]), (uint32_t)(start[1] - first), 0u};
+    shift[0][number] = r.shift[0];
+    shift[1][number] = r.shift[1];
+    lo[number] = r.lo;
+    more[number] = r.more;
+    split[number] = r.split;
+    records[run] = r;
   }
   __device__ __forceinline__ SliceView::Run run(const SliceView& view, int64_t first, int number) const {
-    auto of = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
-    SegmentSpan span;
-    span.lo = of(lo[number]);
-    span.hi = span.lo + of(more[number]);
-    if (span.hi - span.lo > 1) return view.run(first, span);
-    SliceView::Run r{};
-    r.first = first;
-    r.span = span;
-    r.split = span.hi != span.lo ? first + of(split[number]) : INT64_MAX;
-    r.shift[0] = wave_uniform_first(shift[0][number]);
-    r.shift[1] = wave_uniform_first(shift[1][number]);
-    if (view.key_offset) {
-      r.offset[0] = view.key_offset[span.lo];
-      r.offset[1] = view.key_offset[span.hi];
-    }
-    return r;
+    return RunRecord{{shift[0][number], shift[1][number]}, lo[number], more[number], split[number], 0u}
+        .run(view, first);
   }
 };
 
@@ -623,7 +650,8 @@ void member_flag_kernel(
     const int64_t* __restrict__ picked, uint32_t num_picked, const int* __restrict__ wide_flag,
     int64_t* __restrict__ chunk_count, uint16_t* __restrict__ chunk_kept,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
-    const uint32_t* __restrict__ filter, uint32_t* __restrict__ firsts, SliceView view) {
+    const uint32_t* __restrict__ filter, uint32_t* __restrict__ firsts,
+    RunRecord* __restrict__ records, SliceView view) {
   constexpr int kRunEdges = kRun * kBlock;
   // (small ones have about a run a wavefront, which looks it up for itself: 4 us less on 0.3 M edges)
   constexpr bool kTold = kView && kThreads == kMemberThreads;  // the columns of runs, by RunColumns
@@ -844,7 +872,8 @@ void member_flag_kernel(
   auto prepare_runs = [&](const uint32_t* lds) {
     if (threadIdx.x == 0) sh.next_run = 0;
     if (kTold && threadIdx.x < Shared::kRuns && run0 + threadIdx.x < own_runs)
-      sh.columns.find(view, nnz, blockIdx.x + (run0 + threadIdx.x) * gridDim.x, threadIdx.x, lds, index);
+      sh.columns.find(view, nnz, blockIdx.x + (run0 + threadIdx.x) * gridDim.x, threadIdx.x, lds, index,
+                      records);
     __syncthreads();
   };
   if (kTold) {
@@ -1094,13 +1123,62 @@ __global__ __launch_bounds__(kBlock) void member_indptr_kernel(
   out_indptr[c] = r;
 }
 
-// A wave writes the kept edges of kRun consecutive chunks: how many each has comes
-// from the chunk offsets, the columns of the wave's first and last edge take a
-// search each (one column covers the whole span unless columns
-// are short), and the staged ids and places of all chunks are requested together
-// before anything is stored.  The work goes with the kept edges, not with all of
+// The kept edges of kRun consecutive chunks, which a wavefront writes: they are one piece of the
+// output, and a lane takes one of them whichever chunk it is of.  Of two chunks with one edge in
+// four kept two or three rows of 64 are written where a row for every 64 places of either took
+// four, each behind a branch of its own in which the one before was waited for (7.1 M of 31 M
+// edges with values 86 us so and 73 now, 0.8 M of 20 M without 20 and 18; 95 and 23 with a look-up
+// of the columns by every wavefront in front of it).
+template <int kRun>
+struct KeptEdges {
+  int64_t first, out0;  // edge of the slice; place of the first kept one
+  int kept;
+  int before[kRun];     // kept edges of the chunks before each
+  const uint32_t* staged;
+  const uint8_t* places;
+  __device__ __forceinline__ KeptEdges(int64_t first_chunk, int64_t num_chunks,
+                                       const int64_t* __restrict__ chunk_off,
+                                       const uint32_t* __restrict__ all_staged,
+                                       const uint8_t* __restrict__ all_places) {
+    const int lane = lane_id();
+    const int64_t lane_chunk = first_chunk + (lane < kRun ? lane : kRun);
+    const int64_t off = chunk_off[lane_chunk < num_chunks ? lane_chunk : num_chunks];
+    first = first_chunk * kBlock;
+    out0 = wave_uniform_first(off);
+#pragma unroll
+    for (int c = 0; c < kRun; ++c) before[c] = (int)(wave_uniform_first(__shfl((long long)off, c, kWave)) - out0);
+    kept = (int)(wave_uniform_first(__shfl((long long)off, kRun, kWave)) - out0);
+    staged = all_staged + first;
+    places = all_places + first;
+  }
+  // Picked id's place and edge of the slice for kept edge i, or the last one.
+  __device__ __forceinline__ void get(int i, uint32_t* minor, int* edge) const {
+    const int k = i < kept ? i : kept - 1;
+    int at = k, chunk = 0;
+#pragma unroll
+    for (int c = 1; c < kRun; ++c)
+      if (k >= before[c]) {
+        at = k + c * kBlock - before[c];
+        chunk = c * kBlock;
+      }
+    *minor = staged[at];
+    *edge = chunk + (int)places[at];
+  }
+  // write(N as an integral_constant, i0): kept edges i0 to i0 + 64 N - 1, as far as there are.
+  template <typename Write>
+  __device__ __forceinline__ void in_rows(Write write) const {
+    int i0 = 0;
+    for (; kept - i0 > 2 * kWave; i0 += 4 * kWave) write(std::integral_constant<int, 4>(), i0);
+    if (kept - i0 > kWave) write(std::integral_constant<int, 2>(), i0);
+    else if (kept - i0 > 0) write(std::integral_constant<int, 1>(), i0);
+  }
+};
+
+// A wave writes the kept edges of kRun consecutive chunks: the columns of the wave's first and
+// last edge take a search each where the flag pass has not left them (one column covers the
+// whole span unless columns are short).  The work goes with the kept edges, not with all of
 // them: a lane per edge that looked its flag up took 88 us on 19 M edges of which
-// one in twenty-five is kept, and 84 on 29 M with one in four; this takes 32 and 59.
+// one in twenty-five is kept, and 84 on 29 M with one in four; this took 32 and 59.
 // kEdgeMajor: the id on the other axis comes from edge_major (an edge list)
 // instead of the compressed pointer.
 // kView: the edges are those of a column slice read in place (without it none of
@@ -1110,71 +1188,64 @@ __global__ __launch_bounds__(kBlock) void member_fill_kernel(
     int64_t nnz, const int64_t* __restrict__ chunk_off, const uint32_t* __restrict__ staged,
     const uint8_t* __restrict__ staged_pos, const int64_t* __restrict__ indptr, int64_t num_major,
     const int64_t* __restrict__ edge_major, int64_t* __restrict__ out_major,
-    int64_t* __restrict__ out_minor, int64_t* __restrict__ out_select, SliceView view) {
+    int64_t* __restrict__ out_minor, int64_t* __restrict__ out_select,
+    const RunRecord* __restrict__ records, SliceView view) {
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
-  const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  const int lane = lane_id();
+  const int64_t wave =
+      wave_uniform_first((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave);
   const int64_t first_chunk = wave * kRun;
   if (first_chunk >= num_chunks) return;
-  const int64_t lane_chunk = first_chunk + (lane < kRun ? lane : kRun);
-  const int64_t lane_off = chunk_off[lane_chunk < num_chunks ? lane_chunk : num_chunks];
-  const int64_t e_first = first_chunk * kBlock;
-  const int64_t e_end = e_first + kRun * kBlock < nnz ? e_first + kRun * kBlock : nnz;
-  int kept[kRun];  // the same in every lane
-#pragma unroll
-  for (int c = 0; c < kRun; ++c)
-    kept[c] = (int)wave_uniform_first(__shfl((long long)lane_off, c + 1, kWave) -
-                                      __shfl((long long)lane_off, c, kWave));
-  uint32_t minor[kRun][kMemberWords];
-  int at[kRun][kMemberWords];
-#pragma unroll
-  for (int c = 0; c < kRun; ++c)
-#pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      minor[c][j] = 0;
-      at[c][j] = 0;
-      if (j * kWave < kept[c]) {
-        const int k = j * kWave + lane < kept[c] ? j * kWave + lane : kept[c] - 1;
-        minor[c][j] = staged[(first_chunk + c) * kBlock + k];
-        at[c][j] = staged_pos[(first_chunk + c) * kBlock + k];
-      }
-    }
+  const bool told = kRun == kMemberLongRun && records != nullptr;
+  const RunRecord record = told ? records[wave] : RunRecord{};
+  const KeptEdges<kRun> edges(first_chunk, num_chunks, chunk_off, staged, staged_pos);
+  if (edges.kept == 0) return;
+  const int64_t e_end = edges.first + kRun * kBlock < nnz ? edges.first + kRun * kBlock : nnz;
   SegmentSpan span{0, 0};
   SliceView::Run vrun{};
   if (kView) {  // indptr is the view's column pointer: one look-up serves both
-    vrun = view.run(e_first, e_end - 1);
-    span = vrun.span;
+    vrun = told ? record.run(view, edges.first) : view.run(edges.first, e_end - 1);
   } else if (out_major && !kEdgeMajor) {
-    span = segment_span(indptr, num_major, e_first, e_end - 1);
+    span = segment_span(indptr, num_major, edges.first, e_end - 1);
   }
+  edges.in_rows([&](auto rows, int i0) {
+    constexpr int kRows = decltype(rows)::value;
+    uint32_t minor[kRows];
+    int64_t e[kRows], parent_pos[kRows], major[kRows];
 #pragma unroll
-  for (int c = 0; c < kRun; ++c) {
-    const int64_t out0 = __shfl((long long)lane_off, c, kWave);
-#pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      if (j * kWave >= kept[c]) break;  // the whole wave
-      const int64_t e = (first_chunk + c) * kBlock + at[c][j];
-      // with a view: the edge's place in the parent and its column in the slice
-      // (on a scattered run the look-up shuffles: all lanes take it, the ones past
-      // the last kept edge with that edge)
-      int64_t parent_pos = e, major = 0;
-      if (kView) {
-        if (vrun.near()) {
-          parent_pos = vrun.place(e);
-          major = vrun.column(e);
-        } else {
-          int64_t offset;
-          parent_pos = view.position(vrun, e, &major, &offset);
-        }
-      }
-      if (j * kWave + lane >= kept[c]) continue;
-      const int64_t pos = out0 + j * kWave + lane;
-      out_minor[pos] = (int64_t)minor[c][j];
-      out_select[pos] = parent_pos;
-      if (out_major)
-        out_major[pos] = kView ? major : kEdgeMajor ? edge_major[e] : span.segment_at(indptr, e);
+    for (int j = 0; j < kRows; ++j) {
+      int at;
+      edges.get(i0 + j * kWave + lane_id(), &minor[j], &at);
+      e[j] = edges.first + at;
     }
-  }
+    // with a view: the edge's place in the parent and its column in the slice
+    // (on a scattered run the look-up shuffles: all lanes take it, the ones past
+    // the last kept edge with that edge)
+    if (kView && !vrun.near()) {
+#pragma unroll
+      for (int j = 0; j < kRows; ++j) {
+        int64_t offset;
+        parent_pos[j] = view.position(vrun, e[j], &major[j], &offset);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < kRows; ++j) {
+        parent_pos[j] = kView ? vrun.place(e[j]) : e[j];
+        major[j] = kView ? vrun.column(e[j]) : 0;
+      }
+    }
+    if (!kView && out_major)
+#pragma unroll
+      for (int j = 0; j < kRows; ++j)
+        major[j] = kEdgeMajor ? edge_major[e[j]] : span.segment_at(indptr, e[j]);
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int i = i0 + j * kWave + lane_id();
+      if (i >= edges.kept) continue;
+      out_minor[edges.out0 + i] = (int64_t)minor[j];
+      out_select[edges.out0 + i] = parent_pos[j];
+      if (out_major) out_major[edges.out0 + i] = major[j];
+    }
+  });
 }
 
 // The same for a slice whose edges are only wanted with the labels of their ends, and with
@@ -1199,92 +1270,79 @@ struct LabelledEdges {
 template <bool kValues, int kRun>
 __global__ __launch_bounds__(kBlock) void member_label_kernel(
     int64_t nnz, const int64_t* __restrict__ chunk_off, const uint32_t* __restrict__ staged,
-    const uint8_t* __restrict__ staged_pos, LabelledEdges edges, SliceView view) {
+    const uint8_t* __restrict__ staged_pos, LabelledEdges labels,
+    const RunRecord* __restrict__ records, SliceView view) {
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
-  const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  const int lane = lane_id();
+  const int64_t wave =
+      wave_uniform_first((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave);
   const int64_t first_chunk = wave * kRun;
   if (first_chunk >= num_chunks) return;
-  const int64_t lane_chunk = first_chunk + (lane < kRun ? lane : kRun);
-  const int64_t lane_off = chunk_off[lane_chunk < num_chunks ? lane_chunk : num_chunks];
-  const int64_t e_first = first_chunk * kBlock;
-  const int64_t e_end = e_first + kRun * kBlock < nnz ? e_first + kRun * kBlock : nnz;
-  int kept[kRun];  // the same in every lane
+  const bool told = kRun == kMemberLongRun && records != nullptr;
+  const RunRecord record = told ? records[wave] : RunRecord{};
+  const KeptEdges<kRun> edges(first_chunk, num_chunks, chunk_off, staged, staged_pos);
+  if (edges.kept == 0) return;
+  const int64_t e_end = edges.first + kRun * kBlock < nnz ? edges.first + kRun * kBlock : nnz;
+  const SliceView::Run run = told ? record.run(view, edges.first) : view.run(edges.first, e_end - 1);
+  edges.in_rows([&](auto rows, int i0) {
+    constexpr int kRows = decltype(rows)::value;
+    uint32_t minor[kRows];
+    int at[kRows];
 #pragma unroll
-  for (int c = 0; c < kRun; ++c)
-    kept[c] = (int)wave_uniform_first(__shfl((long long)lane_off, c + 1, kWave) -
-                                      __shfl((long long)lane_off, c, kWave));
-  uint32_t minor[kRun][kMemberWords];
-  int at[kRun][kMemberWords];
-#pragma unroll
-  for (int c = 0; c < kRun; ++c)
-#pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      minor[c][j] = 0;
-      at[c][j] = 0;
-      if (j * kWave < kept[c]) {
-        const int k = j * kWave + lane < kept[c] ? j * kWave + lane : kept[c] - 1;
-        minor[c][j] = staged[(first_chunk + c) * kBlock + k];
-        at[c][j] = staged_pos[(first_chunk + c) * kBlock + k];
-      }
-    }
-  const SliceView::Run run = view.run(e_first, e_end - 1);
-  // (all loads before the first store, which they might alias for all the compiler knows)
-  float v[kRun][kMemberWords], by[kRun][kMemberWords];
-  uint32_t row[kRun][kMemberWords], col[kRun][kMemberWords];
-#pragma unroll
-  for (int c = 0; c < kRun; ++c) {
-    int64_t place[kMemberWords], column[kMemberWords];
-    // (on a scattered run the look-up shuffles: all lanes take it)
+    for (int j = 0; j < kRows; ++j) edges.get(i0 + j * kWave + lane_id(), &minor[j], &at[j]);
+    int64_t place[kRows], column[kRows];
     if (run.near()) {
 #pragma unroll
-      for (int j = 0; j < kMemberWords; ++j) {
-        const int64_t e = (first_chunk + c) * kBlock + at[c][j];
-        place[j] = run.place(e);
-        column[j] = run.column(e);
+      for (int j = 0; j < kRows; ++j) {
+        place[j] = run.place(edges.first + at[j]);
+        column[j] = run.column(edges.first + at[j]);
       }
-    } else {
+    } else {  // (the look-up shuffles: all lanes take it)
 #pragma unroll
-      for (int j = 0; j < kMemberWords; ++j) {
-        place[j] = column[j] = 0;
-        if (j * kWave >= kept[c]) continue;  // the whole wave
+      for (int j = 0; j < kRows; ++j) {
         int64_t offset;
-        place[j] = view.position(run, (first_chunk + c) * kBlock + at[c][j], &column[j], &offset);
+        place[j] = view.position(run, edges.first + at[j], &column[j], &offset);
       }
     }
+    // (all loads before the first store, which they might alias for all the compiler knows)
+    float v[kRows], by[kRows];
+    uint32_t row[kRows], col[kRows];
 #pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      v[c][j] = 0.f;
-      by[c][j] = 1.f;
-      row[c][j] = col[c][j] = 0;
-      if (j * kWave >= kept[c]) continue;
-      // (edge data may be shorter than the matrix has edges)
-      if (kValues && (uint64_t)place[j] < (uint64_t)edges.num_values)
-        v[c][j] = edges.values[place[j]];
-      row[c][j] = (uint32_t)edges.row_label[minor[c][j]];
-      col[c][j] = (uint32_t)edges.col_label[column[j]];
-      if (kValues && edges.row_divisor) by[c][j] = edges.row_divisor[minor[c][j]];
+    for (int j = 0; j < kRows; ++j) {
+      row[j] = (uint32_t)labels.row_label[minor[j]];
+      col[j] = (uint32_t)labels.col_label[column[j]];
+      v[j] = 0.f;
     }
-  }
+    if (kValues && labels.num_values > 0) {
 #pragma unroll
-  for (int c = 0; c < kRun; ++c) {
-    const int64_t out0 = __shfl((long long)lane_off, c, kWave);
+      for (int j = 0; j < kRows; ++j)  // (edge data may be shorter than the matrix has edges)
+        v[j] = labels.values[(uint64_t)place[j] < (uint64_t)labels.num_values ? place[j] : 0];
 #pragma unroll
-    for (int j = 0; j < kMemberWords; ++j) {
-      if (j * kWave + lane >= kept[c]) continue;
-      const int64_t pos = out0 + j * kWave + lane;
+      for (int j = 0; j < kRows; ++j)
+        if ((uint64_t)place[j] >= (uint64_t)labels.num_values) v[j] = 0.f;
+    }
+    if (kValues && labels.row_divisor) {
+#pragma unroll
+      for (int j = 0; j < kRows; ++j) by[j] = labels.row_divisor[minor[j]];
+#pragma unroll
+      for (int j = 0; j < kRows; ++j) v[j] /= by[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int i = i0 + j * kWave + lane_id();
+      if (i >= edges.kept) continue;
+      const int64_t pos = edges.out0 + i;
       // (past L2 where the list is long: the passes over the values behind this one find more
       // there, LADIES 577 -> 569 us; what a short list leaves may be read from it)
       if (kRun > 1) {
-        __builtin_nontemporal_store((int64_t)row[c][j], edges.row + pos);
-        __builtin_nontemporal_store((int64_t)col[c][j], edges.col + pos);
+        __builtin_nontemporal_store((int64_t)row[j], labels.row + pos);
+        __builtin_nontemporal_store((int64_t)col[j], labels.col + pos);
       } else {
-        edges.row[pos] = (int64_t)row[c][j];
-        edges.col[pos] = (int64_t)col[c][j];
+        labels.row[pos] = (int64_t)row[j];
+        labels.col[pos] = (int64_t)col[j];
       }
-      if (kValues) edges.out[pos] = edges.row_divisor ? v[c][j] / by[c][j] : v[c][j];
+      if (kValues) labels.out[pos] = v[j];
     }
-  }
+  });
 }
 
 }  // namespace gs
@@ -1345,7 +1403,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   }
   uint16_t* kept = w.chunks <= kOffsetsMaxChunks ? w.chunk_kept : nullptr;
   if (nnz > 0) {
-    const bool small = nnz < kMemberSmallEdges;
+    const bool small = nnz < kMemberSmallEdges || !member_columns_fit(view);
     const int threads = small ? kBlock : kMemberThreads;
     const int run = w.chunks <= kMemberShortChunks ? 1 : kMemberLongRun;
     // a large list, or work-groups that stage a table or a filter: as many of them as are
@@ -1365,7 +1423,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
                 IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, kept,   \
-                w.staged, w.staged_pos, filter, firsts, view))
+                w.staged, w.staged_pos, filter, firsts, w.records, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
@@ -1437,7 +1495,7 @@ static int minor_slice_fill_impl(const int64_t* ids, int64_t nnz, int64_t num_pi
   GS_LAUNCH("member_fill", s,                                                          \
             (member_fill_kernel<MAJOR, VIEW, RUN>)<<<grid, dim3(kBlock), 0, s>>>(      \
                 nnz, w.chunk_off, w.staged, w.staged_pos, indptr, num_major, edge_major, \
-                out_major, out_minor, out_select, view))
+                out_major, out_minor, out_select, member_told(nnz, view) ? w.records : nullptr, view))
 #define GS_MEMBER_FILL(MAJOR, VIEW)                                                    \
   do {                                                                                 \
     if (run == 1) GS_MEMBER_FILL_RUN(MAJOR, VIEW, 1);                                  \
@@ -1567,7 +1625,8 @@ int gs_col_row_slice_labels(const int64_t* indptr, const int64_t* cols, int64_t 
 #define GS_MEMBER_LABEL(VALUES, RUN)                                             \
   GS_LAUNCH("member_label", s,                                                   \
             (member_label_kernel<VALUES, RUN>)<<<grid, dim3(kBlock), 0, s>>>(    \
-                slice_nnz, w.chunk_off, w.staged, w.staged_pos, edges, view))
+                slice_nnz, w.chunk_off, w.staged, w.staged_pos, edges,           \
+                member_told(slice_nnz, view) ? w.records : nullptr, view))
   if (values && run == 1) GS_MEMBER_LABEL(true, 1);
   else if (values) GS_MEMBER_LABEL(true, kMemberLongRun);
   else if (run == 1) GS_MEMBER_LABEL(false, 1);
