@@ -843,3 +843,19 @@ def test_a_column_too_long_for_a_span_is_looked_up():
     got = capi.sample_uniform(d_indptr, T(indices), d_cols, 5, False, 0, 7, 1, spans=True)
     want = orc.sample_uniform(indptr, indices, cols, 5, False, 0, 7, 1)
     assert_same(got, want)
+
+
+@pytest.mark.parametrize("keys", [[511 * 4096], [511 * 4096 + 1], [5000, 511 * 4096, 3, 0, 9000, 511 * 4096 + 7],
+                                  [1023, 1024, 1025, 4096, 40_000, 1]])
+def test_row_labels_of_batches_around_the_longest_whose_groups_are_in_lds(keys):
+    """Rows' labels alone, of tiles inside a batch and over several, of batches whose groups of
+    positions begin inside another's; a third of the keys repeat inside a tile."""
+    rng = np.random.default_rng(sum(keys))
+    ns = [min(n // 7, 300) for n in keys]
+    seeds = np.concatenate([rng.permutation(10**6)[:n] for n in ns])
+    rows = rng.integers(0, 10**6, size=sum(keys) - sum(ns))
+    rows[rng.random(rows.size) < 0.35] %= 50
+    sp = np.concatenate([[0], np.cumsum(ns)])
+    rp = np.concatenate([[0], np.cumsum(np.array(keys) - ns)])
+    got = capi.unique_relabel(T(seeds), T(rows), T(sp), T(rp))
+    assert_same(got[:3], orc.unique_relabel(seeds, rows, sp, rp)[:3])
