@@ -9,6 +9,8 @@
 // 1 = edge, 2 = dst ("v").  All kernels are memory bound; features are scalar
 // in every sampler that uses them, so the fast paths are the feature-length-1
 // ones and the general-length paths favour simplicity.
+#include <type_traits>
+
 #include "common.h"
 #include "scan.h"
 #include "sums.h"
@@ -630,46 +632,42 @@ __global__ __launch_bounds__(kBlock) void spmm_csc_sum_kernel(
 // q and adds it up, the second divides.  7.3 M edges in 1024 columns: gather, division,
 // sums and division took 40 + 28 + 41 + 23 us, each a launch of its own.
 // Sums are of 64 bits, rounded once.
-struct ColumnTile {
-  int64_t first, end, c0, c1;
-  bool in_lds;
-};
-
-// The columns of a tile of kSumTile edges, with where they begin in the tile in LDS where
-// they fit.
-__device__ __forceinline__ ColumnTile column_tile(int64_t tile0, const int64_t* __restrict__ indptr,
-                                                  int64_t num_cols, int64_t nnz, int32_t* begins) {
-  ColumnTile t;
-  t.first = tile0;
-  t.end = t.first + kSumTile < nnz ? t.first + kSumTile : nnz;
-  const SegmentSpan span = segment_span(indptr, num_cols, t.first, t.end - 1);
-  t.c0 = span.lo;
-  t.c1 = span.hi;
-  t.in_lds = t.c1 - t.c0 < kSumSegs;
-  if (t.c0 != t.c1 && t.in_lds)
-    for (int64_t j = threadIdx.x; j <= t.c1 - t.c0; j += kBlock)
-      begins[j] = (int32_t)(indptr[t.c0 + j] - t.first < 0 ? -1 : indptr[t.c0 + j] - t.first);
-  return t;
-}
-// The last of them that begins at or before edge e, which is in it.
-__device__ __forceinline__ int column_in_tile(const ColumnTile& t,
-                                              const int64_t* __restrict__ indptr,
-                                              const int32_t* begins, int64_t e) {
-  const int n = (int)(t.c1 - t.c0) + 1;
-  if (!t.in_lds) return (int)segment_of(indptr + t.c0, n, e);
-  const int32_t x = (int32_t)(e - t.first);
-  int lo = 0, hi = n;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (begins[mid] <= x) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
-
 __global__ __launch_bounds__(kBlock) void normalise_clear_kernel(double* sums, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) sums[i] = 0.0;
+}
+
+// The columns of a run of edges [first, end) that a wavefront has, each for a team of lanes:
+// sixteen where they are few, one where they are many, the wavefront for a long one.
+// part(team as an integral_constant, column, where it begins in the run, how many of its edges
+// are there); none of a team leaves it before the others.
+template <typename Part>
+__device__ __forceinline__ void columns_of_run(const int64_t* __restrict__ indptr, SegmentSpan span,
+                                               int64_t first, int64_t end, Part part) {
+  constexpr int kFew = 16, kTeam = 16;
+  const int lane = lane_id();
+  const bool few = span.hi - span.lo < kFew;
+  const int longest = few ? 16 * kTeam : kWave;  // of the columns that are not the wavefront's
+  for (int64_t c0 = span.lo; c0 <= span.hi; c0 += kWave) {
+    const int64_t c = c0 + lane <= span.hi ? c0 + lane : span.hi;
+    const int64_t s = indptr[c] > first ? indptr[c] : first;
+    const int64_t t = indptr[c + 1] < end ? indptr[c + 1] : end;
+    const int begin = (int)(s - first), n = c0 + lane <= span.hi && t > s ? (int)(t - s) : 0;
+    if (few) {
+      for (int c1 = 0; c1 <= span.hi - span.lo; c1 += kWave / kTeam) {
+        const int from = __shfl(begin, c1 + lane / kTeam, kWave);
+        const int many = __shfl(n, c1 + lane / kTeam, kWave);
+        if (many <= longest)
+          part(std::integral_constant<int, kTeam>(), c0 + c1 + lane / kTeam, from, many);
+      }
+    } else if (n <= longest) {
+      part(std::integral_constant<int, 1>(), c, begin, n);
+    }
+    for (uint64_t left = __ballot(n > longest); left; left &= left - 1) {
+      const int l = __builtin_ctzll(left);
+      part(std::integral_constant<int, kWave>(), c0 + l, __shfl(begin, l, kWave), __shfl(n, l, kWave));
+    }
+  }
 }
 
 // A wavefront adds up a run of kItems * 64 edges.  The look-up of its columns (two or three
@@ -743,16 +741,12 @@ __global__ __launch_bounds__(kRunThreads) void normalise_sum_kernel(
         v[i] = 0.f;
       }
     }
-    auto together = [](double mine) {  // the lanes' sum, in lane 0
-#pragma unroll
-      for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
-      return mine;
-    };
     if (span.lo == span.hi) {
       double mine = 0.0;
 #pragma unroll
       for (int i = 0; i < kItems; ++i) mine += (double)v[i];
-      mine = together(mine);
+#pragma unroll
+      for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
       if (lane == 0) {
         wave_sum[wave] = mine;
         wave_column[wave] = span.lo;
@@ -761,40 +755,14 @@ __global__ __launch_bounds__(kRunThreads) void normalise_sum_kernel(
 #pragma unroll
       for (int i = 0; i < kItems; ++i) run[i * kWave + lane] = v[i];
       wave_lds_fence();
-      // Few columns: sixteen lanes each, the long ones the wavefront; many: a lane or the wavefront.
-      constexpr int kFew = 16, kTeam = 16, kTeamLongest = 16 * kTeam;
-      const bool few = span.hi - span.lo < kFew;
-      const int longest = few ? kTeamLongest : kWave;  // of those that are not the wavefront's
-      for (int64_t c0 = span.lo; c0 <= span.hi; c0 += kWave) {
-        const int64_t c = c0 + lane <= span.hi ? c0 + lane : span.hi;
-        const int64_t s = indptr[c] > first ? indptr[c] : first;
-        const int64_t t = indptr[c + 1] < end ? indptr[c + 1] : end;
-        const int begin = (int)(s - first), n = c0 + lane <= span.hi && t > s ? (int)(t - s) : 0;
-        if (few) {
-          for (int c1 = 0; c1 <= span.hi - span.lo; c1 += kWave / kTeam) {
-            const int from = __shfl(begin, c1 + lane / kTeam, kWave);
-            const int many = __shfl(n, c1 + lane / kTeam, kWave);
-            if (many > longest) continue;  // (the same in all of a team)
-            double mine = 0.0;
-            for (int i = lane % kTeam; i < many; i += kTeam) mine += (double)run[from + i];
+      columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
+        constexpr int kTeam = decltype(team)::value;
+        double mine = 0.0;
+        for (int i = lane % kTeam; i < n; i += kTeam) mine += (double)run[begin + i];
 #pragma unroll
-            for (int d = kTeam / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kTeam);
-            if (lane % kTeam == 0 && many > 0) unsafeAtomicAdd(sums + c0 + c1 + lane / kTeam, mine);
-          }
-        } else if (n > 0 && n <= longest) {
-          double mine = 0.0;
-          for (int i = 0; i < n; ++i) mine += (double)run[begin + i];
-          unsafeAtomicAdd(sums + c, mine);
-        }
-        for (uint64_t left = __ballot(n > longest); left; left &= left - 1) {
-          const int l = __builtin_ctzll(left);
-          const int from = __shfl(begin, l, kWave), many = __shfl(n, l, kWave);
-          double mine = 0.0;
-          for (int i = lane; i < many; i += kWave) mine += (double)run[from + i];
-          mine = together(mine);
-          if (lane == 0) unsafeAtomicAdd(sums + c0 + l, mine);
-        }
-      }
+        for (int d = kTeam / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kTeam);
+        if (lane % kTeam == 0 && n > 0) unsafeAtomicAdd(sums + c, mine);
+      });
     }
   }
   __syncthreads();
@@ -807,32 +775,47 @@ __global__ __launch_bounds__(kRunThreads) void normalise_sum_kernel(
 }
 
 // group: so many tiles in a row were one work-group's of the sums, whose die has their values
-// (7.1 M edges: 17.2 us with the dies' tiles in turn, 15.4 so).
-__global__ __launch_bounds__(kBlock) void normalise_divide_kernel(
+// (7.1 M edges: 17.2 us with the dies' tiles in turn, 15.4 so).  A wavefront for itself, as above,
+// and where columns meet their sums go to the places of their edges in LDS (work-groups that
+// of 2048 edges that searched a column for each took 15.4 and 7.8 us on 7.1 M and 37 K edges of
+// 512 columns, 22.8 on two layers of 8 batches; this 12.9, 5.0 and 14.6).
+__global__ __launch_bounds__(kRunThreads) void normalise_divide_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols, int64_t nnz,
     const double* __restrict__ sums, const float* values, float* out, unsigned group) {
-  __shared__ int32_t begins[kSumSegs];
+  constexpr int kWaves = kRunThreads / kWave;
+  __shared__ float divisors[kWaves][kRunItems * kWave];
   const unsigned nth = blockIdx.x / kDies;  // of its die
-  const int64_t tile0 =
-      ((int64_t)(nth / group * kDies + blockIdx.x % kDies) * group + nth % group) * kSumTile;
-  if (tile0 >= nnz) return;
-  float v[kSumItems];
+  const int64_t tile = (int64_t)(nth / group * kDies + blockIdx.x % kDies) * group + nth % group;
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t first = wave_uniform_first((tile * kWaves + wave) * (kRunItems * kWave));
+  if (first >= nnz) return;
+  const int64_t end = first + kRunItems * kWave < nnz ? first + kRunItems * kWave : nnz;
+  float v[kRunItems], by[kRunItems];
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i) {
-    const int64_t e = tile0 + i * kBlock + threadIdx.x;
-    v[i] = values[e < nnz ? e : nnz - 1];
+  for (int i = 0; i < kRunItems; ++i) {
+    const int64_t e = first + i * kWave + lane;
+    v[i] = values[e < end ? e : end - 1];
   }
-  const ColumnTile t = column_tile(tile0, indptr, num_cols, nnz, begins);
-  const bool one = t.c0 == t.c1;
-  float s = 0.f;
-  if (one) s = (float)sums[t.c0];
-  else __syncthreads();
+  const SegmentSpan span = segment_span(indptr, num_cols, first, end - 1);
+  if (span.lo == span.hi) {
+    const float s = (float)sums[span.lo];
 #pragma unroll
-  for (int i = 0; i < kSumItems; ++i) {
-    const int64_t e = tile0 + i * kBlock + threadIdx.x;
-    if (e >= t.end) continue;
-    if (!one) s = (float)sums[t.c0 + column_in_tile(t, indptr, begins, e)];
-    out[e] = v[i] / s;
+    for (int i = 0; i < kRunItems; ++i) by[i] = s;
+  } else {
+    float* const run = divisors[wave];
+    columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
+      constexpr int kTeam = decltype(team)::value;
+      const float s = n > 0 ? (float)sums[c] : 0.f;
+      for (int i = lane % kTeam; i < n; i += kTeam) run[begin + i] = s;
+    });
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < kRunItems; ++i) by[i] = run[i * kWave + lane];
+  }
+#pragma unroll
+  for (int i = 0; i < kRunItems; ++i) {
+    const int64_t e = first + i * kWave + lane;
+    if (e < end) out[e] = v[i] / by[i];
   }
 }
 
@@ -1792,10 +1775,10 @@ int gs_normalise_columns_cleared(const int64_t* indptr, int64_t num_cols, const 
   else if (!long_runs) GS_NORMALISE_SUM(false, false, kRunItems);
   else GS_NORMALISE_SUM(false, false, kLongRunItems);
 #undef GS_NORMALISE_SUM
-  const unsigned group = run / kSumTile;
+  const unsigned group = run / (kRunThreads * kRunItems);
   GS_LAUNCH("normalise_divide", s,
             normalise_divide_kernel<<<dim3((unsigned)ceil_div(grid.x, kDies) * kDies * group),
-                                      dim3(kBlock), 0, s>>>(
+                                      dim3(kRunThreads), 0, s>>>(
                 indptr, num_cols, nnz, sums, moved ? out : values, out, group));
   return GS_OK;
 }
