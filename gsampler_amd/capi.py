@@ -121,6 +121,8 @@ SIGNATURES = {
     "gs_minor_slice_fill": (_int, [_p, _i64, _i64, _p, _i64, _p, _p, _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_count": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p, _p,
                                       _sz, _p]),
+    "gs_col_row_slice_count_labels": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, *([_p] * 9),
+                                             _sz, _p]),
     "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
                                             _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),

@@ -294,16 +294,14 @@ Graph::RelabelledRows(torch::Tensor cols, torch::Tensor rows, c10::optional<torc
   int64_t* const row_label = first + R;
   int64_t* const col_label = row_label + R;
   double* const sums = (double*)(col_label + S);
-  AsyncCount kept = AsyncCount::mirrored();
-  GS_CALL(gs_col_row_slice_count_first(
-      cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
-      cptr(cols), nullptr, S, cptr(so->sub_indptr), nnz, cptr(rows), R, mptr(indptr),
-      kept.mirror(), first, sums, ws.data_ptr(), ws.numel(), cur_stream()));
-  kept.arm();
   torch::Tensor frontier = new_ids(R + S, m.indptr);
-  AsyncCount nodes = AsyncCount::mirrored();
-  GS_CALL(gs_list_labels(cptr(cols), S, cptr(rows), first, R, mptr(frontier), nullptr,
-                         nodes.mirror(), row_label, col_label, cur_stream()));
+  AsyncCount kept = AsyncCount::mirrored(), nodes = AsyncCount::mirrored();
+  GS_CALL(gs_col_row_slice_count_labels(
+      cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
+      cptr(cols), S, cptr(so->sub_indptr), nnz, cptr(rows), R, mptr(indptr), kept.mirror(), first,
+      sums, mptr(frontier), nodes.mirror(), row_label, col_label, ws.data_ptr(), ws.numel(),
+      cur_stream()));
+  kept.arm();
   nodes.arm();
   HandedOn edges;
   edges.queue(m, cols, so->sub_indptr, nnz, R, row_label, col_label, values, row_divisor, ws);

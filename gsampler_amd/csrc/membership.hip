@@ -23,6 +23,7 @@
 
 #include "common.h"
 #include "hashtable.h"
+#include "listlabels.h"
 #include "scan.h"
 
 namespace gs {
@@ -128,6 +129,7 @@ struct MemberWs {
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
   uint32_t* firsts;    // [first_groups * num_picked] per work-group of the flag pass, the first edge it kept by each id
   int64_t first_groups;
+  uint32_t* first_parts;  // [1] behind `wide`: how many parts of the first edges are told (ListLabels)
   void* scan_ws;
   size_t scan_ws_bytes;
   int64_t chunks;
@@ -169,7 +171,8 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked, bool fir
       c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
   w.records = (RunRecord*)c.take<uint64_t>(
       nnz >= kMemberSmallEdges ? (size_t)ceil_div(w.chunks, kMemberLongRun) * kRecordWords : 0);
-  w.wide = c.take<int>(1);
+  w.wide = c.take<int>(2);
+  w.first_parts = w.wide ? (uint32_t*)(w.wide + 1) : nullptr;
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
@@ -651,7 +654,7 @@ void member_flag_kernel(
     int64_t* __restrict__ chunk_count, uint16_t* __restrict__ chunk_kept,
     uint32_t* __restrict__ staged, uint8_t* __restrict__ staged_pos,
     const uint32_t* __restrict__ filter, uint32_t* __restrict__ firsts,
-    RunRecord* __restrict__ records, SliceView view) {
+    uint32_t* __restrict__ first_parts, RunRecord* __restrict__ records, SliceView view) {
   constexpr int kRunEdges = kRun * kBlock;
   // (small ones have about a run a wavefront, which looks it up for itself: 4 us less on 0.3 M edges)
   constexpr bool kTold = kView && kThreads == kMemberThreads;  // the columns of runs, by RunColumns
@@ -659,6 +662,7 @@ void member_flag_kernel(
   using Filter = typename Shared::Filter;
   __shared__ Shared sh;
   const bool filtered = kInLds || filter != nullptr;
+  if (kInLds && firsts && blockIdx.x == 0 && threadIdx.x == 0) *first_parts = 0u;
   const MemberTable table{global_table, cap};
   BucketTable buckets;
   bool wide;  // the same for every thread of the launch
@@ -986,7 +990,10 @@ __device__ __forceinline__ void member_first(int64_t part, const uint32_t* __res
   if (wave > 0 || i >= num_picked) return;
 #pragma unroll
   for (int w = 1; w < kWaves; ++w) m = least[w][lane] < m ? least[w][lane] : m;
-  out_first[i] = m == UINT32_MAX ? INT64_MAX : (int64_t)m;
+  // (seen by other dies as soon as it is stored: a fence for the whole device would have them
+  // write their L2 back, 5 us)
+  __hip_atomic_store(out_first + i, m == UINT32_MAX ? INT64_MAX : (int64_t)m, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 }
 __global__ __launch_bounds__(1024) void member_first_kernel(
     const uint32_t* __restrict__ firsts, int64_t groups, int64_t num_picked,
@@ -1026,25 +1033,57 @@ __device__ __forceinline__ int member_below(int64_t e, int kept,
 // in three launches took 15 us behind the flag pass on 8 to 29 M edges, this takes 9 to 10
 // (tiles of 2048 chunks 11, and 16 where 19 K columns are short and meet in few tiles).
 constexpr int kOffsetsThreads = 1024;
-static_assert(kOffsetsThreads == 1024, "member_first() runs in these work-groups too");
+static_assert(kOffsetsThreads == 1024 && kOffsetsThreads == kLabelThreads,
+              "member_first() and list_labels_of() run in these work-groups too");
 constexpr int kOffsetsTile = 512;
+// Labels of the picked rows and of the columns (list_labels_of).  They wait for the first edges
+// alone: the work-group that tells the last part of those goes on with them while others are at
+// the offsets (31 M edges and 512 picks, 20 M and 400: 21 us in two launches, now 16; 37 K and
+// 10 K edges 20 and 18, now 15 and 12).
+struct ListLabels {
+  const int64_t* seeds;  // null: none are wanted
+  const int64_t* list_ids;
+  int num_seeds;
+  uint32_t* parts_told;  // 0 before the launch
+  int64_t *frontier, *count_mirror, *list_label, *seed_label;
+};
+
+template <bool kLabels>
 __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
     const uint8_t* __restrict__ staged_pos, const uint16_t* __restrict__ chunk_kept,
     int64_t nnz, int64_t* __restrict__ chunk_off, int64_t* __restrict__ out_indptr,
     int64_t* __restrict__ out_total, unsigned tiles, const uint32_t* __restrict__ firsts,
     int64_t first_groups, int64_t num_picked, int64_t* __restrict__ out_first,
-    double* __restrict__ col_zeros) {
-  if (blockIdx.x >= tiles) {  // (there are such only where out_first is asked for)
-    member_first(blockIdx.x - tiles, firsts, first_groups, num_picked, out_first);
+    double* __restrict__ col_zeros, ListLabels labels) {
+  // (the first work-groups tell the first edges where out_first is asked for: those that go on
+  // with the labels are under way when the others begin)
+  const unsigned parts = gridDim.x - tiles;
+  if (blockIdx.x < parts) {
+    member_first(blockIdx.x, firsts, first_groups, num_picked, out_first);
+    if constexpr (kLabels) {
+      __shared__ uint32_t told;
+      if (threadIdx.x < kWave) {  // (which has stored this part)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (threadIdx.x == 0)
+          told = __hip_atomic_fetch_add(labels.parts_told, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (told + 1 != parts) return;
+      const int total = list_labels_of<true>(labels.seeds, labels.num_seeds, labels.list_ids, 0, out_first,
+                                       (int)num_picked, labels.frontier, labels.list_label,
+                                       labels.seed_label);
+      if (threadIdx.x == 0) store_for_host(labels.count_mirror, total);
+    }
     return;
   }
+  const unsigned tile = blockIdx.x - parts;
   __shared__ uint32_t smem[kOffsetsThreads / kWave + 1];
   __shared__ uint32_t before[kOffsetsTile + 1];  // kept edges of the tile before each chunk
   __shared__ int64_t col_range[2];
   const int64_t num_chunks = ceil_div_dev(nnz, kBlock);
-  const int64_t chunk0 = (int64_t)blockIdx.x * kOffsetsTile;
-  const bool last_tile = blockIdx.x + 1 == tiles;
+  const int64_t chunk0 = (int64_t)tile * kOffsetsTile;
+  const bool last_tile = tile + 1 == tiles;
   const int t = threadIdx.x, wave = t / kWave;
   const bool owns = t < kOffsetsTile && chunk0 + t < num_chunks;
   const uint32_t own = owns ? chunk_kept[chunk0 + t] : 0u;
@@ -1054,7 +1093,7 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
     if (indptr) {
       const int64_t e = wave_uniform_first((chunk0 + (wave ? kOffsetsTile : 0)) * kBlock);
       int64_t c;
-      if (wave ? last_tile : blockIdx.x == 0) c = wave ? num_major + 1 : 0;
+      if (wave ? last_tile : tile == 0) c = wave ? num_major + 1 : 0;
       else c = indptr[0] >= e ? 0 : wave_segment_of(indptr, num_major + 1, e - 1) + 1;
       if (lane_id() == 0) col_range[wave] = c;
     }
@@ -1366,7 +1405,8 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
                                   int64_t* out_total, void* workspace,
                                   size_t workspace_bytes, gs_stream_t stream,
                                   gs::SliceView view, int64_t* out_first = nullptr,
-                                  double* col_zeros = nullptr) {
+                                  double* col_zeros = nullptr,
+                                  gs::ListLabels labels = gs::ListLabels{}) {
   using namespace gs;
   GS_REQUIRE(nnz >= 0 && num_picked >= 0 && num_major >= 0,
              "minor_slice_count: negative size");
@@ -1423,7 +1463,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
   GS_LAUNCH("member_flag", s,                                                                 \
             (member_flag_kernel<LDS, THREADS, RUN, IDT, VIEW>)<<<grid, dim3(THREADS), 0, s>>>( \
                 IDS, nnz, w.table, cap, picked, (uint32_t)num_picked, w.wide, w.chunk_off, kept,   \
-                w.staged, w.staged_pos, filter, firsts, w.records, view))
+                w.staged, w.staged_pos, filter, firsts, w.first_parts, w.records, view))
 #define GS_MEMBER_FLAG_IDS(LDS, THREADS, RUN)                                                 \
   do {                                                                                        \
     const bool in_place = view.sub_indptr != nullptr;                                         \
@@ -1446,16 +1486,28 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
     const unsigned first_parts = out_first ? (unsigned)ceil_div(num_picked, kWave) : 0u;
     if (kept) {
       const unsigned tiles = (unsigned)ceil_div(w.chunks, kOffsetsTile);
-      GS_LAUNCH("member_offsets", s,
-                member_offsets_kernel<<<dim3(tiles + first_parts), dim3(kOffsetsThreads), 0, s>>>(
-                    indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,
-                    out_total, tiles, firsts, blocks, num_picked, out_first, col_zeros));
+      labels.parts_told = w.first_parts;
+#define GS_MEMBER_OFFSETS(LABELS)                                                             \
+  GS_LAUNCH("member_offsets", s,                                                              \
+            (member_offsets_kernel<LABELS>)<<<dim3(tiles + first_parts),                      \
+                                              dim3(kOffsetsThreads), 0, s>>>(                 \
+                indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,          \
+                out_total, tiles, firsts, blocks, num_picked, out_first, col_zeros, labels))
+      if (labels.seeds) GS_MEMBER_OFFSETS(true);
+      else GS_MEMBER_OFFSETS(false);
+#undef GS_MEMBER_OFFSETS
       return GS_OK;
     }
     if (out_first)
       GS_LAUNCH("member_first", s,
                 member_first_kernel<<<dim3(first_parts), dim3(1024), 0, s>>>(firsts, blocks,
                                                                              num_picked, out_first));
+    if (labels.seeds) {
+      const int rc = gs_list_labels(labels.seeds, labels.num_seeds, labels.list_ids, out_first, num_picked,
+                                    labels.frontier, nullptr, labels.count_mirror, labels.list_label,
+                                    labels.seed_label, stream);
+      if (rc != GS_OK) return rc;
+    }
     int rc = exclusive_scan_i64(w.chunk_off, w.chunk_off, w.chunks + 1, w.scan_ws,
                                 w.scan_ws_bytes, s);
     if (rc != GS_OK) return rc;
@@ -1580,6 +1632,32 @@ int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
   return minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
                                 num_cols_picked, out_indptr, out_total, workspace,
                                 workspace_bytes, stream, view, out_first, col_zeros);
+}
+
+int gs_col_row_slice_count_labels(const int64_t* indptr, const int64_t* indices,
+                                  const int32_t* indices32, const int64_t* cols,
+                                  int64_t num_cols_picked, const int64_t* sub_indptr,
+                                  int64_t slice_nnz, const int64_t* rows, int64_t num_rows_picked,
+                                  int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
+                                  double* col_zeros, int64_t* out_frontier,
+                                  int64_t* out_count_mirror, int64_t* out_row_label,
+                                  int64_t* out_col_label, void* workspace, size_t workspace_bytes,
+                                  gs_stream_t stream) {
+  int rc = check_slice_view(indptr, indices, cols, num_cols_picked, sub_indptr, slice_nnz,
+                            "col_row_slice_count");
+  if (rc != GS_OK) return rc;
+  GS_REQUIRE(gs_col_row_slice_tells_first(slice_nnz, num_rows_picked) && out_first && rows && cols &&
+                 num_rows_picked + num_cols_picked <= GS_LIST_LABELS_MAX_KEYS,
+             "col_row_slice_count_labels: no labels of %lld rows and %lld columns",
+             (long long)num_rows_picked, (long long)num_cols_picked);
+  GS_REQUIRE(out_frontier && out_count_mirror && out_row_label && out_col_label,
+             "col_row_slice_count_labels: null pointer");
+  const gs::SliceView view{sub_indptr, cols, indptr, nullptr, num_cols_picked};
+  const gs::ListLabels labels{cols, rows, (int)num_cols_picked, nullptr, out_frontier,
+                              out_count_mirror, out_row_label, out_col_label};
+  return minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
+                                num_cols_picked, out_indptr, out_total, workspace,
+                                workspace_bytes, stream, view, out_first, col_zeros, labels);
 }
 
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,

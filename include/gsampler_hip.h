@@ -776,6 +776,17 @@ int gs_col_row_slice_count(const int64_t* indptr, const int64_t* indices,
                            const int64_t* rows, int64_t num_rows_picked,
                            int64_t* out_indptr, int64_t* out_total, void* workspace,
                            size_t workspace_bytes, gs_stream_t stream);
+/* gs_col_row_slice_count_first, without moves, and gs_list_labels of (cols, rows, out_first) in
+ * one call: the labels beside the offsets.  out_count_mirror as there. */
+int gs_col_row_slice_count_labels(const int64_t* indptr, const int64_t* indices,
+                                  const int32_t* indices32, const int64_t* cols,
+                                  int64_t num_cols_picked, const int64_t* sub_indptr,
+                                  int64_t slice_nnz, const int64_t* rows, int64_t num_rows_picked,
+                                  int64_t* out_indptr, int64_t* out_total, int64_t* out_first,
+                                  double* col_zeros, int64_t* out_frontier,
+                                  int64_t* out_count_mirror, int64_t* out_row_label,
+                                  int64_t* out_col_label, void* workspace, size_t workspace_bytes,
+                                  gs_stream_t stream);
 int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
                                  const int32_t* indices32, const int64_t* cols,
                                  const int64_t* key_offset, int64_t num_cols_picked,

@@ -1007,3 +1007,21 @@ def test_row_slices_whose_work_groups_look_up_their_runs_in_several_rounds(lengt
                   + torch.repeat_interleave(kept_ptr[cols] - want_ptr[:-1], count)]
     assert torch.equal(got[3], select)
     assert torch.equal(got[2], place[indices[select]])
+
+
+@pytest.mark.parametrize("R", [1, 63, 64, 65, 512, 1500, 2000])
+@pytest.mark.parametrize("edges", [20_000, 700_000, 9_000_000])
+def test_labels_beside_the_offsets(R, edges):
+    """One part of the first edges and up to 32, of few and of all work-groups' lists, told by
+    the last that ends; again and again on the same scratch memory."""
+    rng = np.random.default_rng(R + edges)
+    indptr, indices = columns_of(rng.multinomial(edges, np.ones(30) / 30), rng, 3000)
+    g = gs.Graph(3100, 30)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    for _ in range(5):
+        cols, rows = T(rng.permutation(30)), T(rng.integers(0, 3100, size=R))
+        got = g._CAPI_RelabelledRows(cols, rows, None, None)
+        sub, _ = g._CAPI_ColRowSlicing(cols, rows, gs.format._CSC, gs.format._CSC | gs.format._COO)
+        assert (got is None) == (edges < 8 * (R + 30))
+        for a, b in zip(got[:3] if got else (), sub._CAPI_GraphRelabel(cols, rows)):
+            assert torch.equal(a, b)
