@@ -123,6 +123,8 @@ SIGNATURES = {
                                       _sz, _p]),
     "gs_col_row_slice_count_labels": (_int, [_p, _p, _p, _p, _i64, _p, _i64, _p, _i64, *([_p] * 9),
                                              _sz, _p]),
+    "gs_col_row_slice_count_batch_labels": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64,
+                                                   *([_p] * 7), _i64, _i64, *([_p] * 7), _sz, _p]),
     "gs_col_row_slice_count_first": (_int, [_p, _p, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p, _p,
                                             _p, _p, _p, _sz, _p]),
     "gs_col_row_slice_tells_first": (_int, [_i64, _i64]),

@@ -591,16 +591,14 @@ Graph::EncodedBlocks(torch::Tensor seeds, torch::Tensor col_bptr, torch::Tensor 
   double* const sums = (double*)(col_label + S);
   int64_t* const scratch = col_label + 2 * S;
   AsyncCount kept = AsyncCount::mirrored();
-  GS_CALL(gs_col_row_slice_count_first(
+  int64_t* mirror = OffsetMirror::reserve(unique_ptr);
+  GS_CALL(gs_col_row_slice_count_batch_labels(
       cptr(m.indptr), cptr(m.indices), narrow.defined() ? narrow.data_ptr<int32_t>() : nullptr,
       cptr(seeds), cptr(key_offset), S, cptr(so->sub_indptr), nnz, cptr(picked), R, mptr(indptr),
-      kept.mirror(), first, sums, ws.data_ptr(), ws.numel(), cur_stream()));
+      kept.mirror(), first, sums, cptr(col_bptr), cptr(names), cptr(row_bptr), num_rows_, B,
+      mptr(frontier), mptr(unique_ptr), mirror, row_label, col_label, scratch, ws.data_ptr(),
+      ws.numel(), cur_stream()));
   kept.arm();
-  int64_t* mirror = OffsetMirror::reserve(unique_ptr);
-  GS_CALL(gs_batch_list_labels(cptr(seeds), cptr(col_bptr), S, cptr(names), cptr(row_bptr), R,
-                               num_rows_, B, nullptr, nullptr, nullptr, 0, first, mptr(frontier),
-                               mptr(unique_ptr), mirror, row_label, col_label, nullptr, nullptr,
-                               scratch, cur_stream()));
   OffsetMirror::arm(unique_ptr);
   HandedOn edges;
   edges.queue(m, seeds, so->sub_indptr, nnz, R, row_label, col_label, values, row_divisor, ws);

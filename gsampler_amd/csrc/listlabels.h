@@ -187,6 +187,12 @@ __device__ __forceinline__ int list_labels_of(
   return total;
 }
 
+// The frontiers of batches, each at the place of its bound, moved together; the batch pointer, its
+// last entry -1 where a batch's count is, for the host too.
+int batch_list_frontier(const int64_t* seeds_ptr, const int64_t* list_ptr, const int64_t* counts,
+                        int64_t num_batches, const int64_t* bound_frontier, int64_t* out_frontier,
+                        int64_t* unique_ptr, int64_t* mirror, hipStream_t s);
+
 }  // namespace gs
 
 #endif  // GSAMPLER_CSRC_LISTLABELS_H_

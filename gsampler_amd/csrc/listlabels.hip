@@ -56,12 +56,14 @@ __global__ __launch_bounds__(kLabelThreads) void batch_list_labels_kernel(
 }
 
 // A work-group per batch: its frontier to its place behind those of the batches
-// before it.  The first one also clears or raises the flag of a refused batch.
+// before it.  The first one also clears or raises the flag of a refused batch.  mirror: no pass
+// over edges can refuse any more, and the batch pointer is the host's too (in a launch of its own,
+// which is for those that can, 3 us and the gap in front of it).
 __global__ __launch_bounds__(kBlock) void batch_list_frontier_kernel(
     const int64_t* __restrict__ seeds_ptr, const int64_t* __restrict__ list_ptr,
     const int64_t* __restrict__ counts, int64_t num_batches,
     const int64_t* __restrict__ bound_frontier, int64_t* __restrict__ out_frontier,
-    int64_t* __restrict__ unique_ptr, int* __restrict__ refused) {
+    int64_t* __restrict__ unique_ptr, int* __restrict__ refused, int64_t* mirror) {
   __shared__ int64_t smem[kBlock / kWave + 1];
   __shared__ int any_refused;
   const int64_t b = blockIdx.x;
@@ -77,8 +79,13 @@ __global__ __launch_bounds__(kBlock) void batch_list_frontier_kernel(
   const int64_t n = counts[b] > 0 ? counts[b] : 0;
   if (threadIdx.x == 0) {
     unique_ptr[b] = base;
-    if (b == num_batches - 1) unique_ptr[num_batches] = base + n;
-    if (b == 0) *refused = any_refused;
+    if (mirror) store_for_host(mirror + b, base);
+    if (b == num_batches - 1) {
+      const int64_t total = mirror && any_refused ? -1 : base + n;
+      unique_ptr[num_batches] = total;
+      if (mirror) store_for_host(mirror + num_batches, total);
+    }
+    if (b == 0 && refused) *refused = any_refused;
   }
   if (n == 0) return;
   const int64_t* from = bound_frontier + seeds_ptr[b] + list_ptr[b];
@@ -187,6 +194,16 @@ __global__ __launch_bounds__(kBlock) void batch_list_publish_kernel(
   }
 }
 
+int batch_list_frontier(const int64_t* seeds_ptr, const int64_t* list_ptr, const int64_t* counts,
+                        int64_t num_batches, const int64_t* bound_frontier, int64_t* out_frontier,
+                        int64_t* unique_ptr, int64_t* mirror, hipStream_t s) {
+  GS_LAUNCH("list_frontier", s,
+            batch_list_frontier_kernel<<<dim3((unsigned)num_batches), dim3(kBlock), 0, s>>>(
+                seeds_ptr, list_ptr, counts, num_batches, bound_frontier, out_frontier, unique_ptr,
+                nullptr, mirror));
+  return GS_OK;
+}
+
 }  // namespace gs
 
 extern "C" int gs_list_labels(const int64_t* seeds, int64_t num_seeds, const int64_t* list_ids,
@@ -266,12 +283,14 @@ extern "C" int gs_batch_list_labels(
             batch_list_labels_kernel<<<batches, dim3(kLabelThreads), 0, s>>>(
                 seeds, seeds_ptr, list_ids, list_ptr, num_ids, id_stride, first_pos, bound, counts,
                 out_list_label, out_seed_label));
+  if (nnz == 0)
+    return batch_list_frontier(seeds_ptr, list_ptr, counts, num_batches, bound, out_frontier,
+                               unique_ptr, unique_ptr_mirror, s);
   GS_LAUNCH("list_frontier", s,
             batch_list_frontier_kernel<<<batches, dim3(kBlock), 0, s>>>(
                 seeds_ptr, list_ptr, counts, num_batches, bound, out_frontier, unique_ptr,
-                refused));
-  if (nnz > 0)
-    GS_LAUNCH("list_edges", s,
+                refused, nullptr));
+  GS_LAUNCH("list_edges", s,
               batch_list_edges_kernel<<<dim3((unsigned)ceil_div(nnz, kEdgeLabelTile)),
                                         dim3(kBlock), 0, s>>>(
                   row, col, nnz, edge_ptr, list_ptr, num_batches, num_ids, num_seeds,

@@ -117,6 +117,7 @@ struct FewIdFilter {
 // at the bound, where three launches that read every count once take 15.2).
 constexpr int64_t kOffsetsMaxChunks = int64_t(1) << 17;
 
+constexpr int kMostLabelBatches = 32;  // whose labels are made beside the offsets
 constexpr int kRecordWords = 4;  // of a RunRecord, 64 bits each
 struct MemberWs {
   uint64_t* table;     // [member_table_slots(num_picked)], a table in L2
@@ -129,7 +130,7 @@ struct MemberWs {
   uint32_t* filter;    // [kFilterWords] which ids may be in the table (member_filtered)
   uint32_t* firsts;    // [first_groups * num_picked] per work-group of the flag pass, the first edge it kept by each id
   int64_t first_groups;
-  uint32_t* first_parts;  // [1] behind `wide`: how many parts of the first edges are told (ListLabels)
+  uint32_t* first_parts;  // [kMostLabelBatches] behind `wide`: how many parts of the first edges are told (ListLabels)
   void* scan_ws;
   size_t scan_ws_bytes;
   int64_t chunks;
@@ -171,7 +172,7 @@ static MemberWs carve_member(void* ws, int64_t nnz, int64_t num_picked, bool fir
       c.take<uint16_t>(w.chunks <= kOffsetsMaxChunks ? (size_t)ceil_div(w.chunks, 8) * 8 : 0);
   w.records = (RunRecord*)c.take<uint64_t>(
       nnz >= kMemberSmallEdges ? (size_t)ceil_div(w.chunks, kMemberLongRun) * kRecordWords : 0);
-  w.wide = c.take<int>(2);
+  w.wide = c.take<int>(1 + kMostLabelBatches);
   w.first_parts = w.wide ? (uint32_t*)(w.wide + 1) : nullptr;
   w.filter = c.take<uint32_t>(member_filtered(num_picked) ? (size_t)kFilterWords : 0);
   w.scan_ws_bytes = scan_workspace_bytes(w.chunks + 1);
@@ -662,7 +663,7 @@ void member_flag_kernel(
   using Filter = typename Shared::Filter;
   __shared__ Shared sh;
   const bool filtered = kInLds || filter != nullptr;
-  if (kInLds && firsts && blockIdx.x == 0 && threadIdx.x == 0) *first_parts = 0u;
+  if (kInLds && firsts && blockIdx.x == 0 && threadIdx.x < kMostLabelBatches) first_parts[threadIdx.x] = 0u;
   const MemberTable table{global_table, cap};
   BucketTable buckets;
   bool wide;  // the same for every thread of the launch
@@ -1039,16 +1040,64 @@ constexpr int kOffsetsTile = 512;
 // Labels of the picked rows and of the columns (list_labels_of).  They wait for the first edges
 // alone: the work-group that tells the last part of those goes on with them while others are at
 // the offsets (31 M edges and 512 picks, 20 M and 400: 21 us in two launches, now 16; 37 K and
-// 10 K edges 20 and 18, now 15 and 12).
+// 10 K edges 20 and 18, now 15 and 12; of 8 batches of 384 keys 20 us, of which the labels 11 in a
+// launch of their own, now 17).
 struct ListLabels {
   const int64_t* seeds;  // null: none are wanted
   const int64_t* list_ids;
   int num_seeds;
-  uint32_t* parts_told;  // 0 before the launch
+  uint32_t* parts_told;  // [kMostLabelBatches], 0 before the launch
   int64_t *frontier, *count_mirror, *list_label, *seed_label;
+  // of batches (null: there is one), as gs_batch_list_labels says; `frontier` is that of the bounds
+  const int64_t *seeds_ptr, *list_ptr;
+  int64_t id_stride;
+  int num_batches;
+  int64_t* counts;
 };
 
-template <bool kLabels>
+// The labels of the batches whose first edges the work-group of this part is the last to tell.
+// Lane b looks at batch b, whose rows lie in a part or in several (without rows: in one).
+__device__ __forceinline__ void member_batch_labels(unsigned part, unsigned parts, int64_t num_picked,
+                                                    const int64_t* __restrict__ first,
+                                                    const ListLabels& labels) {
+  static_assert(kMostLabelBatches <= kWave, "a lane a batch");
+  __shared__ uint32_t told[kMostLabelBatches];
+  const int lane = lane_id(), b = lane < labels.num_batches ? lane : 0;
+  const int64_t s0 = labels.seeds_ptr[b], s1 = labels.seeds_ptr[b + 1];
+  const int64_t l0 = labels.list_ptr[b], l1 = labels.list_ptr[b + 1];
+  const bool fits = s0 >= 0 && s1 >= s0 && s1 <= labels.num_seeds && l0 >= 0 && l1 >= l0 &&
+                    l1 <= num_picked && (s1 - s0) + (l1 - l0) <= kLabelMaxKeys;
+  unsigned p0 = fits ? (unsigned)(l0 / kWave) : 0u;
+  if (p0 >= parts) p0 = parts - 1;
+  const unsigned p1 = fits && l1 > l0 ? (unsigned)((l1 - 1) / kWave) : p0;
+  const bool mine = lane < labels.num_batches && p0 <= part && part <= p1;
+  if (threadIdx.x < kWave) {  // (which has stored this part)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (mine)
+      told[b] = __hip_atomic_fetch_add(labels.parts_told + b, 1u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const uint64_t fitting = __ballot(fits);
+  uint64_t left = __ballot(mine && told[b] == p1 - p0);
+  for (; left; left &= left - 1) {
+    const int i = __builtin_ctzll(left);
+    int total = -1;
+    if ((fitting >> i) & 1) {
+      const int64_t seed0 = labels.seeds_ptr[i], id0 = labels.list_ptr[i];
+      total = list_labels_of<true>(labels.seeds + seed0, (int)(labels.seeds_ptr[i + 1] - seed0),
+                                   labels.list_ids + id0, labels.id_stride, first + id0,
+                                   (int)(labels.list_ptr[i + 1] - id0),
+                                   labels.frontier + seed0 + id0, labels.list_label + id0,
+                                   labels.seed_label + seed0);
+    }
+    if (threadIdx.x == 0) labels.counts[i] = total;
+    __syncthreads();
+  }
+}
+
+enum { kNoLabels, kOneList, kBatchLists };
+template <int kLabels>
 __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
     const int64_t* __restrict__ indptr, int64_t num_major,
     const uint8_t* __restrict__ staged_pos, const uint16_t* __restrict__ chunk_kept,
@@ -1061,7 +1110,9 @@ __global__ __launch_bounds__(kOffsetsThreads) void member_offsets_kernel(
   const unsigned parts = gridDim.x - tiles;
   if (blockIdx.x < parts) {
     member_first(blockIdx.x, firsts, first_groups, num_picked, out_first);
-    if constexpr (kLabels) {
+    if constexpr (kLabels == kBatchLists) {
+      member_batch_labels(blockIdx.x, parts, num_picked, out_first, labels);
+    } else if constexpr (kLabels == kOneList) {
       __shared__ uint32_t told;
       if (threadIdx.x < kWave) {  // (which has stored this part)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1493,8 +1544,9 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
                                               dim3(kOffsetsThreads), 0, s>>>(                 \
                 indptr, num_major, w.staged_pos, kept, nnz, w.chunk_off, out_indptr,          \
                 out_total, tiles, firsts, blocks, num_picked, out_first, col_zeros, labels))
-      if (labels.seeds) GS_MEMBER_OFFSETS(true);
-      else GS_MEMBER_OFFSETS(false);
+      if (labels.list_ptr) GS_MEMBER_OFFSETS(kBatchLists);
+      else if (labels.seeds) GS_MEMBER_OFFSETS(kOneList);
+      else GS_MEMBER_OFFSETS(kNoLabels);
 #undef GS_MEMBER_OFFSETS
       return GS_OK;
     }
@@ -1502,7 +1554,7 @@ static int minor_slice_count_impl(const int64_t* ids, const int32_t* ids32, int6
       GS_LAUNCH("member_first", s,
                 member_first_kernel<<<dim3(first_parts), dim3(1024), 0, s>>>(firsts, blocks,
                                                                              num_picked, out_first));
-    if (labels.seeds) {
+    if (labels.seeds && !labels.list_ptr) {
       const int rc = gs_list_labels(labels.seeds, labels.num_seeds, labels.list_ids, out_first, num_picked,
                                     labels.frontier, nullptr, labels.count_mirror, labels.list_label,
                                     labels.seed_label, stream);
@@ -1658,6 +1710,50 @@ int gs_col_row_slice_count_labels(const int64_t* indptr, const int64_t* indices,
   return minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
                                 num_cols_picked, out_indptr, out_total, workspace,
                                 workspace_bytes, stream, view, out_first, col_zeros, labels);
+}
+
+int gs_col_row_slice_count_batch_labels(
+    const int64_t* indptr, const int64_t* indices, const int32_t* indices32, const int64_t* cols,
+    const int64_t* key_offset, int64_t num_cols_picked, const int64_t* sub_indptr,
+    int64_t slice_nnz, const int64_t* rows, int64_t num_rows_picked, int64_t* out_indptr,
+    int64_t* out_total, int64_t* out_first, double* col_zeros, const int64_t* cols_ptr,
+    const int64_t* list_ids, const int64_t* list_ptr, int64_t id_stride, int64_t num_batches,
+    int64_t* out_frontier, int64_t* unique_ptr, int64_t* unique_ptr_mirror, int64_t* out_row_label,
+    int64_t* out_col_label, int64_t* scratch, void* workspace, size_t workspace_bytes,
+    gs_stream_t stream) {
+  using namespace gs;
+  int rc = check_slice_view(indptr, indices, cols, num_cols_picked, sub_indptr, slice_nnz,
+                            "col_row_slice_count");
+  if (rc != GS_OK) return rc;
+  GS_REQUIRE(gs_col_row_slice_tells_first(slice_nnz, num_rows_picked) && out_first && rows && cols &&
+                 num_batches >= 1,
+             "col_row_slice_count_batch_labels: no labels of %lld rows of %lld batches",
+             (long long)num_rows_picked, (long long)num_batches);
+  GS_REQUIRE(cols_ptr && list_ids && list_ptr && out_frontier && unique_ptr && unique_ptr_mirror &&
+                 out_row_label && out_col_label && scratch,
+             "col_row_slice_count_batch_labels: null pointer");
+  const SliceView view{sub_indptr, cols, indptr, key_offset, num_cols_picked};
+  int64_t* const counts = scratch + num_cols_picked + num_rows_picked;
+  // (few batches: a work-group may have to label several that share its part)
+  const bool beside = num_batches <= kMostLabelBatches && num_batches * kWave <= num_rows_picked &&
+                      num_cols_picked <= INT32_MAX &&
+                      ceil_div(slice_nnz, kBlock) <= kOffsetsMaxChunks;
+  ListLabels labels{};
+  if (beside)
+    labels = ListLabels{cols, list_ids, (int)num_cols_picked, nullptr, scratch, nullptr,
+                        out_row_label, out_col_label, cols_ptr, list_ptr, id_stride,
+                        (int)num_batches, counts};
+  rc = minor_slice_count_impl(indices, indices32, slice_nnz, rows, num_rows_picked, sub_indptr,
+                              num_cols_picked, out_indptr, out_total, workspace, workspace_bytes,
+                              stream, view, out_first, col_zeros, labels);
+  if (rc != GS_OK) return rc;
+  if (!beside)
+    return gs_batch_list_labels(cols, cols_ptr, num_cols_picked, list_ids, list_ptr,
+                                num_rows_picked, id_stride, num_batches, nullptr, nullptr, nullptr,
+                                0, out_first, out_frontier, unique_ptr, unique_ptr_mirror,
+                                out_row_label, out_col_label, nullptr, nullptr, scratch, stream);
+  return batch_list_frontier(cols_ptr, list_ptr, counts, num_batches, scratch, out_frontier,
+                             unique_ptr, unique_ptr_mirror, as_stream(stream));
 }
 
 int gs_col_row_slice_fill(const int64_t* indptr, const int64_t* indices, const int64_t* cols,

@@ -787,6 +787,17 @@ int gs_col_row_slice_count_labels(const int64_t* indptr, const int64_t* indices,
                                   int64_t* out_count_mirror, int64_t* out_row_label,
                                   int64_t* out_col_label, void* workspace, size_t workspace_bytes,
                                   gs_stream_t stream);
+/* gs_col_row_slice_count_first and gs_batch_list_labels of (cols, list_ids, out_first) without
+ * edges, in one call; list_ids[num_rows_picked] names the rows, whose keys carry their batch. */
+int gs_col_row_slice_count_batch_labels(
+    const int64_t* indptr, const int64_t* indices, const int32_t* indices32, const int64_t* cols,
+    const int64_t* key_offset, int64_t num_cols_picked, const int64_t* sub_indptr,
+    int64_t slice_nnz, const int64_t* rows, int64_t num_rows_picked, int64_t* out_indptr,
+    int64_t* out_total, int64_t* out_first, double* col_zeros, const int64_t* cols_ptr,
+    const int64_t* list_ids, const int64_t* list_ptr, int64_t id_stride, int64_t num_batches,
+    int64_t* out_frontier, int64_t* unique_ptr, int64_t* unique_ptr_mirror, int64_t* out_row_label,
+    int64_t* out_col_label, int64_t* scratch, void* workspace, size_t workspace_bytes,
+    gs_stream_t stream);
 int gs_col_row_slice_count_first(const int64_t* indptr, const int64_t* indices,
                                  const int32_t* indices32, const int64_t* cols,
                                  const int64_t* key_offset, int64_t num_cols_picked,
