@@ -765,13 +765,13 @@ def test_encoded_row_slice_that_is_only_handed_on(seeds, picks, values):
     assert torch.equal(got[1], sub._CAPI_NormaliseColumns(w, index, by)) if values else got[1] is None
 
 
-@pytest.mark.parametrize("batches,picks", [(32, 64), (31, 65), (33, 61), (2, 1000), (8, 255), (16, 65)])
+@pytest.mark.parametrize("batches,picks", [(32, 64), (31, 65), (33, 61), (2, 900), (8, 255), (16, 65)])
 def test_labels_of_batches_beside_the_offsets(batches, picks):
     """Parts of the first edges that are a batch's, or of two, or a batch's of many; one batch
     more than are labelled there.  Again and again on the same scratch memory."""
     uneven = [picks + (-1) ** b * min(b, 40) for b in range(batches)] if batches != 32 else [picks] * batches
     for _ in range(3):
-        test_encoded_row_slice_that_is_only_handed_on([20] * batches, uneven, True)
+        test_encoded_row_slice_that_is_only_handed_on([60] * batches, uneven, True)
     empty = [0] + [picks + picks // (batches - 1)] * (batches - 2) + [0]
     test_encoded_row_slice_that_is_only_handed_on([50] * batches, empty if batches > 2 else [0, picks], False)
 
