@@ -1163,7 +1163,7 @@ __global__ __launch_bounds__(kBlock) void table_fill_kernel32(uint32_t* __restri
 // if enough of them lie before it (100 K items, 300 of them positive, 400 picks: 710 us
 // without that).
 // 2.45 M items, 400 picks, us: keys 25, two levels of histograms 10 and 11 and finish 7
-// when all keys were made; now bounds 13, emit 9, finish 5.
+// when all keys were made; now bounds 13, emit 8, finish 6.
 constexpr int kSelBins = 2048;
 // Long segments: neighbouring work-groups add to one of eight histograms, and half as many
 // items a work-group, twice as many of them, fill the device better than the adds to the same
@@ -1271,6 +1271,34 @@ __device__ __forceinline__ SelSegment sel_segment(const int64_t* __restrict__ ra
                                                   int64_t seg) {
   return range ? SelSegment{range[seg], range[seg + 1]} : SelSegment{0, n};
 }
+// A segment's candidates lie in kSelLists lists: neighbouring tiles share one, which begins where
+// their items do and so has room for all of them.  Work-groups that append wait for one another
+// by the counter's line, some 10 ns each: with one list a segment, its counters side by side, emit
+// took 9.6 us on 2.45 M items and 400 picks, 14.3 on eight segments of 233 K and 256, 6.4 on one of
+// 233 K and 512; with eight, a line each, 8.3, 10.4 and 5.7.
+constexpr int kSelLists = 8;
+constexpr int kSelCountStride = 32;  // words, a line of the L2
+struct SelLists {
+  int64_t lo;
+  int tile_shift;             // items of a tile
+  uint32_t first_tile, tiles;  // of the segment; of a list
+  __device__ __forceinline__ SelLists(SelSegment sg, int shift)
+      : lo(sg.lo), tile_shift(shift), first_tile((uint32_t)(sg.lo >> shift)) {
+    tiles = ((uint32_t)((sg.hi - 1) >> shift) - first_tile + kSelLists) / kSelLists;
+  }
+  __device__ __forceinline__ int of_tile(uint32_t t) const {
+    int list = 0;
+#pragma unroll
+    for (int c = 1; c < kSelLists; ++c) list += t - first_tile >= c * tiles;
+    return list;
+  }
+  __device__ __forceinline__ int64_t begin(int list) const {
+    return list == 0 ? lo : (int64_t)(first_tile + list * tiles) << tile_shift;
+  }
+  static __device__ __forceinline__ int64_t counter(int64_t seg, int list) {
+    return (seg * kSelLists + list) * kSelCountStride;
+  }
+};
 __device__ __forceinline__ SegmentSpan sel_span(const int64_t* __restrict__ range, int64_t nseg,
                                                 int64_t i0, int64_t i_last) {
   return range ? segment_span(range, nseg, i0, i_last) : SegmentSpan{0, 0};
@@ -1371,18 +1399,21 @@ __global__ __launch_bounds__(kBlock) void list_emit_kernel(
     }
     uint32_t cands;
     uint32_t at = block_exclusive_sum((uint32_t)__popc(is_cand), smem, &cands);
-    if (threadIdx.x == 0) base = cands ? atomicAdd(&counts[seg], cands) : 0u;
+    const SelLists lists(sg, __builtin_ctz(kBlock * kSelItems));
+    const int list = lists.of_tile(blockIdx.x);
+    if (threadIdx.x == 0) base = cands ? atomicAdd(&counts[SelLists::counter(seg, list)], cands) : 0u;
     __syncthreads();
+    const int64_t room = lists.begin(list);
     at += base;
     while (is_cand) {
       const int j = __ffs((int)is_cand) - 1;
       is_cand &= is_cand - 1;
       const int64_t i = i0 + j * kBlock + threadIdx.x;
-      if ((int64_t)at < sg.hi - sg.lo) {  // always
+      if (room + at < sg.hi) {  // always
         // non-negative doubles (and +inf) order like their bit patterns
-        cand_key[sg.lo + at] =
+        cand_key[room + at] =
             (uint64_t)__double_as_longlong(weighted_key(key, (uint64_t)i, 0, probs[i]));
-        cand_idx[sg.lo + at] = i;
+        cand_idx[room + at] = i;
       }
       ++at;
     }
@@ -1396,7 +1427,7 @@ __device__ __forceinline__ unsigned __int128 sel_composite(uint64_t k, int64_t i
 }
 
 __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
-    const int64_t* __restrict__ range, int64_t n, int64_t num_picks,
+    const int64_t* __restrict__ range, int64_t n, int64_t num_picks, int tile_shift,
     const uint32_t* __restrict__ counts, const uint64_t* __restrict__ cand_key,
     const int64_t* __restrict__ cand_idx, const int64_t* __restrict__ out_range,
     int64_t* __restrict__ out_index, const float* __restrict__ probs,
@@ -1413,21 +1444,40 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
   const int64_t seg = blockIdx.x;
   const SelSegment sg = sel_segment(range, n, seg);
   const int64_t nb = sg.hi - sg.lo, out0 = out_range[seg];
+  uint32_t many[kSelLists];
+#pragma unroll
+  for (int c = 0; c < kSelLists; ++c) many[c] = counts[SelLists::counter(seg, c)];
   if (nb <= num_picks) {  // taken whole, in the original order
     if (blockIdx.y == 0)
       for (int64_t k = threadIdx.x; k < nb; k += kFinishThreads) pick(out0 + k, sg.lo + k);
     return;
   }
   // (no list is longer than its segment; restated here because indices follow from it)
-  uint32_t M = counts[seg];
-  if ((int64_t)M > nb) M = (uint32_t)nb;
-  const uint64_t* ck = cand_key + sg.lo;
-  const int64_t* ci = cand_idx + sg.lo;
+  const SelLists lists(sg, tile_shift);
+  uint32_t M = 0, list_end[kSelLists];
+#pragma unroll
+  for (int c = 0; c < kSelLists; ++c) {
+    const int64_t room = sg.hi - lists.begin(c);
+    M += room <= 0 ? 0u : (int64_t)many[c] < room ? many[c] : (uint32_t)room;
+    list_end[c] = M;
+  }
+  auto place = [&](uint32_t t) {
+    int list = 0;
+    uint32_t before = 0;
+#pragma unroll
+    for (int c = 0; c + 1 < kSelLists; ++c)
+      if (t >= list_end[c]) {
+        list = c + 1;
+        before = list_end[c];
+      }
+    return lists.begin(list) + (t - before);
+  };
   uint32_t total = M;
   if (total <= (uint32_t)kFinishSlots) {
     for (uint32_t t = threadIdx.x; t < M; t += kFinishThreads) {
-      sk[t] = ck[t];
-      si[t] = ci[t];
+      const int64_t at = place(t);
+      sk[t] = cand_key[at];
+      si[t] = cand_idx[at];
     }
   } else {
     // the `want` smallest of the M candidates: fix the composite of the last
@@ -1439,7 +1489,8 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
       for (int b = threadIdx.x; b < 256; b += kFinishThreads) hist[b] = 0;
       __syncthreads();
       for (uint32_t t = threadIdx.x; t < M; t += kFinishThreads) {
-        const unsigned __int128 c = sel_composite(ck[t], ci[t]);
+        const int64_t at = place(t);
+        const unsigned __int128 c = sel_composite(cand_key[at], cand_idx[at]);
         if ((c >> (shift + 8)) == (fixed >> (shift + 8)))
           atomicAdd(&hist[(uint32_t)(c >> shift) & 255u], 1u);
       }
@@ -1458,8 +1509,9 @@ __global__ __launch_bounds__(kFinishThreads) void list_finish_kernel(
     if (threadIdx.x == 0) appended = 0;
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < M; t += kFinishThreads) {
-      const uint64_t k = ck[t];
-      const int64_t i = ci[t];
+      const int64_t from = place(t);
+      const uint64_t k = cand_key[from];
+      const int64_t i = cand_idx[from];
       if (sel_composite(k, i) <= fixed) {
         const uint32_t at = atomicAdd(&appended, 1u);
         if (at < (uint32_t)kFinishSlots) {
@@ -1564,7 +1616,7 @@ static ListWs carve_list(void* ws, int64_t n, int64_t nseg) {
   w.scan_ws = c.take<char>(w.scan_ws_bytes);
   const size_t segs = list_can_select(n, nseg) ? (size_t)nseg : 0;
   w.copies = nseg > 0 && n / nseg >= kSelLongSegment ? kSelCopies : 1;
-  w.sel_words = segs * ((size_t)w.copies * kSelBins + 1);
+  w.sel_words = segs * ((size_t)w.copies * kSelBins + kSelLists * kSelCountStride);
   w.sel_block = c.take<uint32_t>(w.sel_words);
   w.hist = w.sel_block;
   w.counts = w.hist ? w.hist + segs * w.copies * kSelBins : nullptr;
@@ -1816,7 +1868,7 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
 #undef GS_SEL_LAUNCH
     GS_LAUNCH("list_finish", s,
               list_finish_kernel<<<dim3((unsigned)num_segments, kFinishSplit), dim3(kFinishThreads), 0, s>>>(
-                  range, n, num_picks, w.counts, w.keys_out, w.vals_out,
+                  range, n, num_picks, __builtin_ctz(kBlock * items), w.counts, w.keys_out, w.vals_out,
                   out_range, out_index, probs, out_value));
     return GS_OK;
   }

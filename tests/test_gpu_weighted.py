@@ -488,3 +488,22 @@ def test_batched_list_selection_where_the_items_a_thread_takes_change(n):
     for k in (1, 256):
         same(capi.list_sample_weighted(F(probs), k, range_=T(ranges), call_id=3),
              orc.list_sample_weighted(probs, k, range_=ranges, call_id=3))
+
+
+@pytest.mark.parametrize("n", [4096, 5000, 8192, 9217, 600_000, (1 << 20) + 3])
+@pytest.mark.parametrize("where", ["first", "last", "few", "all"])
+def test_list_selection_of_candidates_that_lie_together(n, where):
+    """All candidates in a segment's first or last tiles, in one list of them; weights of zero in
+    the others; fewer tiles than lists; all of one weight, which narrows them in the end."""
+    probs = np.full(n, 1e-6, dtype=np.float32)
+    if where == "few":
+        probs[:] = 0
+    probs[{"first": slice(0, 900), "last": slice(n - 900, n), "few": slice(n // 2, n // 2 + 90),
+           "all": slice(0, n)}[where]] = 1.0
+    for ranges in (None, np.array([0, n // 2 + 77, n])):
+        if ranges is not None and n < 9000:
+            continue  # (segments too short to be selected from)
+        for k in (1, 400, 2048):
+            args = {} if ranges is None else {"range_": T(ranges)}
+            same(capi.list_sample_weighted(F(probs), k, call_id=3, **args),
+                 orc.list_sample_weighted(probs, k, range_=ranges, call_id=3))
