@@ -127,12 +127,15 @@ struct LayerColumns {
 // The batches' offsets, one a lane, where a wavefront has lanes for all of them: asked for
 // once, beside a kernel's first loads, and compared with from then on, where a search takes a
 // trip to the cache a step, and the ends of a batch two more.  All lanes call these together.
+// kMany: of kernels for more batches than one; those for one have no code for any of it
+// (two layers of 1024 seeds 39.2 us of kernels with it and 37.7 without, 47.9 and 46.2 a call).
+template <bool kMany>
 struct HeldBatches {
   int64_t at;  // ptr[lane], INT64_MAX past the last
   int B;
   bool held;
   __device__ __forceinline__ explicit HeldBatches(const LayerColumns& cols)
-      : at(0), B((int)cols.B), held(cols.ptr && cols.B < kWave) {
+      : at(0), B((int)cols.B), held(kMany && cols.ptr && cols.B < kWave) {
     if (held) {
       at = cols.ptr[lane_id() <= B ? lane_id() : B];
       if (lane_id() > B) at = INT64_MAX;
@@ -272,7 +275,7 @@ __device__ __forceinline__ void pick_columns(const PickLane& l, bool live, Colum
   if (live) slot_of[position] = my_key != kNoSlot ? sh.global_slot[at] : kNoSlot;
 }
 
-template <typename IdT>
+template <typename IdT, bool kMany>
 __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
     const int64_t* __restrict__ indptr, int64_t num_cols, const IdT* __restrict__ indices,
     LayerColumns cols, int fanout, int cols_per_wave, int replace, PhiloxKey key, uint32_t stride,
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
   const PickLane l(blockIdx.x, fanout, cols_per_wave);
   // one round trip for the number of columns and the id, of a place that may be no column's
   const int64_t id = cols.ids[cols.place(l.c, 1)];
-  const HeldBatches batches(cols);
+  const HeldBatches<kMany> batches(cols);
   const int64_t n = batches.num(cols);
   if (l.first_col >= n) return;  // uniform per work-group
   sh.clear();
@@ -301,8 +304,8 @@ __global__ __launch_bounds__(kPickThreads) void layer_pick_kernel(
         *deg = column_degree(indptr, num_cols, id, start);
         if (batches.held) return PickColumn{id, held_b, held_lo, held_hi - held_lo};
         const int64_t b0 =
-            cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(l.first_col)) : 0;
-        const int64_t b = cols.batch_of(l.c, b0);
+            kMany && cols.ptr ? segment_of(cols.ptr, cols.B, wave_uniform_first(l.first_col)) : 0;
+        const int64_t b = kMany ? cols.batch_of(l.c, b0) : 0;
         return PickColumn{id, b, cols.lo(b), cols.hi(b) - cols.lo(b)};
       },
       indices, fanout, replace, key, stride, picked, table, mask, slot_of, wide, sh);
@@ -317,14 +320,16 @@ struct TileBatches {
     return b;
   }
 };
-__device__ __forceinline__ TileBatches tile_batches(const LayerColumns& cols, const HeldBatches& held,
+template <bool kMany>
+__device__ __forceinline__ TileBatches tile_batches(const LayerColumns& cols, const HeldBatches<kMany>& held,
                                                     int width, int64_t p0, int64_t p_last) {
-  if (!cols.ptr) return TileBatches{0, 0};
+  if (!kMany || !cols.ptr) return TileBatches{0, 0};
   if (held.held) return TileBatches{held.of_uniform(p0, width), held.of_uniform(p_last, width)};
   return TileBatches{segment_of(cols.ptr, cols.B, wave_uniform_first(p0 / width)),
                      segment_of(cols.ptr, cols.B, wave_uniform_first(p_last / width))};
 }
 
+template <bool kMany>
 __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
     LayerColumns cols, int fanout, const uint64_t* __restrict__ table,
     const uint32_t* __restrict__ slot_of, uint32_t* __restrict__ first,
@@ -339,7 +344,7 @@ __global__ __launch_bounds__(kBlock) void layer_flag_kernel(
 #pragma unroll
   for (int j = 0; j < kLayerWordsPerWave; ++j)
     s[j] = slot_of[cols.place(wave_p0 + j * kWave + lane, width)];
-  const HeldBatches held(cols);
+  const HeldBatches<kMany> held(cols);
   const int64_t N = held.num(cols) * width;
   if (p0 >= N) return;
 #pragma unroll
@@ -430,7 +435,7 @@ struct LabelShared {
 
 // Work-group `block` of `blocks`.  kThreads: of the launch (alone 11.6 us with 256 and 12.8
 // with 512 on 150 K positions).
-template <int kThreads>
+template <int kThreads, bool kMany>
 __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned block,
                                            unsigned blocks, LabelShared& sh) {
   const LayerColumns& cols = layer.cols;
@@ -469,7 +474,7 @@ __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned bl
 #pragma unroll
   for (int j = 0; j < kPer; ++j)
     cnt[j] = tile_cnt[(int64_t)threadIdx.x * kPer + j < blocks ? threadIdx.x * kPer + j : 0];
-  const HeldBatches held(cols);
+  const HeldBatches<kMany> held(cols);
   const int64_t n = held.num(cols), N = n * width;
   const int64_t tiles = (N + kLayerTile - 1) / kLayerTile;
   if (block != 0 && (int64_t)block >= tiles) return empty_table();
@@ -611,21 +616,22 @@ __device__ __forceinline__ void label_tile(const LayerLabels& layer, unsigned bl
   empty_table();
 }
 
+template <bool kMany>
 __global__ __launch_bounds__(kBlock) void layer_label_kernel(LayerLabels layer) {
   __shared__ LabelShared sh;
-  label_tile<kBlock>(layer, blockIdx.x, gridDim.x, sh);
+  label_tile<kBlock, kMany>(layer, blockIdx.x, gridDim.x, sh);
 }
 
 // Labels of a layer and picks of the one whose columns are its frontier: the first
 // `pick_blocks` work-groups pick.
-template <typename IdT>
+template <typename IdT, bool kMany>
 __global__ __launch_bounds__(kPickThreads) void layer_label_pick_kernel(
     LayerLabels before, unsigned pick_blocks, const int64_t* __restrict__ indptr, int64_t num_cols,
     const IdT* __restrict__ indices, int fanout, int cols_per_wave, int replace, PhiloxKey key,
     uint64_t* table, uint32_t mask, uint32_t* __restrict__ slot_of, int32_t* wide) {
   if (blockIdx.x >= pick_blocks) {
     __shared__ LabelShared label;
-    label_tile<kPickThreads>(before, blockIdx.x - pick_blocks, gridDim.x - pick_blocks, label);
+    label_tile<kPickThreads, kMany>(before, blockIdx.x - pick_blocks, gridDim.x - pick_blocks, label);
     return;
   }
   __shared__ PickShared sh;
@@ -680,7 +686,7 @@ __global__ __launch_bounds__(kPickThreads) void layer_label_pick_kernel(
           else hi = mid;
         }
         const uint32_t found = before.keys[(int64_t)lo * kLayerTile + (c - tile_first[lo])];
-        const uint32_t b = found / before.stride;
+        const uint32_t b = kMany ? found / before.stride : 0u;
         const int64_t id = (int64_t)(found - b * before.stride);
         *deg = column_degree(indptr, num_cols, id, start);
         return PickColumn{id, b, batch_first[b], batch_first[b + 1] - batch_first[b]};
@@ -808,7 +814,9 @@ int gs_sample_layer_next(const gs_layer* before, const gs_layer* layer, gs_strea
                       layer->num_batches <= kLayerMaxBatches;
   if (before && !beside)
     GS_LAUNCH("layer_label", s,
-              layer_label_kernel<<<dim3(label_grid), dim3(kBlock), 0, s>>>(labels));
+              if (before->num_batches > 1)
+                layer_label_kernel<true><<<dim3(label_grid), dim3(kBlock), 0, s>>>(labels);
+              else layer_label_kernel<false><<<dim3(label_grid), dim3(kBlock), 0, s>>>(labels));
   if (!layer) return GS_OK;
   const gs_layer& l = *layer;
   const LayerWs w = carve_layer(l.workspace, l.max_positions, l.cdf != nullptr);
@@ -826,28 +834,35 @@ int gs_sample_layer_next(const gs_layer* before, const gs_layer* layer, gs_strea
                                 l.fanout, l.replace, key, w.picked, s);
     if (rc != GS_OK) return rc;
   }
-#define GS_PICK(T, IDS)                                                                       \
+#define GS_PICK(T, MANY, IDS)                                                                       \
   do {                                                                                        \
     if (beside)                                                                               \
       GS_LAUNCH("layer_label_pick", s,                                                        \
-                layer_label_pick_kernel<T><<<dim3(pick_grid + label_grid), dim3(kPickThreads), 0, \
+                (layer_label_pick_kernel<T, MANY>)<<<dim3(pick_grid + label_grid), dim3(kPickThreads), 0, \
                                              s>>>(                                            \
                     labels, pick_grid, l.indptr, l.num_cols, IDS, (int)l.fanout, cols_per_wave, \
                     l.replace, key, table, (uint32_t)(slots - 1), w.slot, w.wide));           \
     else                                                                                      \
       GS_LAUNCH("layer_pick", s,                                                              \
-                layer_pick_kernel<T><<<dim3(pick_grid), dim3(kPickThreads), 0, s>>>(          \
+                (layer_pick_kernel<T, MANY>)<<<dim3(pick_grid), dim3(kPickThreads), 0, s>>>(  \
                     l.indptr, l.num_cols, IDS, cols, (int)l.fanout, cols_per_wave, l.replace, \
                     key, (uint32_t)l.id_stride, l.cdf ? w.picked : nullptr, table,            \
                     (uint32_t)(slots - 1), w.slot, w.wide));                                  \
   } while (0)
-  if (l.indices32) GS_PICK(int32_t, l.indices32);
-  else GS_PICK(int64_t, l.indices);
+#define GS_PICK_AND_FLAG(MANY)                                                                \
+  do {                                                                                        \
+    if (l.indices32) GS_PICK(int32_t, MANY, l.indices32);                                     \
+    else GS_PICK(int64_t, MANY, l.indices);                                                   \
+    GS_LAUNCH("layer_flag", s,                                                                \
+              layer_flag_kernel<MANY><<<dim3((unsigned)ceil_div(positions, kLayerTile)),      \
+                                        dim3(kBlock), 0, s>>>(cols, (int)l.fanout, table,     \
+                                                              w.slot, w.first, w.key, w.words, \
+                                                              w.tile_cnt));                   \
+  } while (0)
+  if (l.num_batches > 1) GS_PICK_AND_FLAG(true);
+  else GS_PICK_AND_FLAG(false);
+#undef GS_PICK_AND_FLAG
 #undef GS_PICK
-  GS_LAUNCH("layer_flag", s,
-            layer_flag_kernel<<<dim3((unsigned)ceil_div(positions, kLayerTile)), dim3(kBlock), 0,
-                                s>>>(cols, (int)l.fanout, table, w.slot, w.first, w.key, w.words,
-                                     w.tile_cnt));
   return GS_OK;
 }
 
