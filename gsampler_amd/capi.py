@@ -134,6 +134,7 @@ SIGNATURES = {
     "gs_col_row_slice_fill": (_int, [_p, _p, _p, _i64, _p, _i64, _i64, _p, _p, _p, _p, _sz, _p]),
     "gs_probe_stream_copy": (_int, [_p, _p, _i64, _p]),
     "gs_probe_line_gather": (_int, [_p, _i64, _i64, _u64, _int, _p, _p]),
+    "gs_probe_few_id_filter": (_i64, [_p, _i64, _p, _i64, _int]),
     "gs_probe_sample_uniform": (_int, [_p, _i64, _p, _p, _i64, _i64, _int, _i64, _u64, _u64, _p,
                                        _p, _p, _p, _p, _p]),
     "gs_encoded_square_sums_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -1088,10 +1088,15 @@ int gs_e_div_u_sum(int format, const int64_t* a, const int64_t* b,
  *    long, outputs sized num_items * fanout), 8 (row ids not read), 16 (only
  *    the row id stored), 32 (nothing stored).  Built: 0, 1, 2, 4, 8, 24, 16,
  *    32, 40.  col_span (nullable) as for the sampler fills.
+ *  gs_probe_few_id_filter: how many of `ids` the filter in front of a row slice's table in
+ *    LDS lets through with `picked` in it, that of small work-groups or of large ones; host
+ *    arrays, evaluated on the host.  -1: bad arguments.
  * ---------------------------------------------------------------------- */
 int gs_probe_stream_copy(const void* src, void* dst, int64_t bytes, gs_stream_t stream);
 int gs_probe_line_gather(const void* table, int64_t table_bytes, int64_t num_picks,
                          uint64_t salt, int ordered, void* out, gs_stream_t stream);
+int64_t gs_probe_few_id_filter(const int32_t* picked, int64_t num_picked, const int32_t* ids,
+                               int64_t num_ids, int small);
 int gs_probe_sample_uniform(
     const int64_t* indptr, int64_t num_cols, const int32_t* indices32,
     const int64_t* column_ids, int64_t num_items, int64_t fanout, int variant,
