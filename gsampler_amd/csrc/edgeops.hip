@@ -670,6 +670,48 @@ __device__ __forceinline__ void columns_of_run(const int64_t* __restrict__ indpt
   }
 }
 
+// The same edge by edge, for a run most of whose columns are empty: part(column, place in the
+// run, whether there is such an edge), by all lanes, for 64 neighbouring edges at a time.  The
+// columns of 256 edges are searched for together, a step for twice as many columns, where going
+// through the columns takes a step for 64 more of them (with eight rows of 64 in place of four
+// the registers leave fewer wavefronts resident).  Sums and division, us, by columns and so:
+// 5000 edges of 10 K columns 34 and 36, of 16 K 48 and 32, of 100 K 213 and 42, of 1 M 1634 and
+// 69; 1 M edges of 4 M columns 75 and 66.
+constexpr int64_t kSparseColumns = 2;  // an edge, from where on
+__device__ __forceinline__ bool is_sparse(SegmentSpan span, int64_t edges) {
+  return span.hi - span.lo >= kSparseColumns * edges;
+}
+template <typename Part>
+__device__ __forceinline__ void edges_of_run(const int64_t* __restrict__ indptr, SegmentSpan span,
+                                             int64_t first, int64_t end, Part part) {
+  constexpr int kRows = 4;
+  const int n = (int)(end - first);
+  const int64_t most = span.hi - span.lo;
+  const int64_t* const begins = indptr + span.lo;
+  for (int i0 = 0; i0 < n; i0 += kRows * kWave) {
+    int64_t e[kRows], c[kRows];  // c: the last column known to begin at or before the edge
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int at = i0 + j * kWave + lane_id();
+      e[j] = first + (at < n ? at : n - 1);
+      c[j] = 0;
+    }
+    for (int64_t step = int64_t(1) << (63 - __builtin_clzll((uint64_t)most)); step > 0; step >>= 1) {
+      int64_t begin[kRows];
+#pragma unroll
+      for (int j = 0; j < kRows; ++j) begin[j] = begins[c[j] + step <= most ? c[j] + step : most];
+#pragma unroll
+      for (int j = 0; j < kRows; ++j)
+        if (c[j] + step <= most && begin[j] <= e[j]) c[j] += step;
+    }
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int at = i0 + j * kWave + lane_id();
+      part(span.lo + c[j], at, at < n);
+    }
+  }
+}
+
 // A wavefront adds up a run of kItems * 64 edges.  The look-up of its columns (two or three
 // loads, one behind the other) is on its way with the values; where columns meet the run goes
 // to LDS and is read back column by column, the short ones a lane each.  What bounds it is the
@@ -677,8 +719,9 @@ __device__ __forceinline__ void columns_of_run(const int64_t* __restrict__ indpt
 // an add for every 2048 edges of it 7.1 M edges of 512 columns (28 MB) took 32 us.  So the
 // wavefronts of a work-group that are inside one column add once: 13 us.  37 K edges of as many
 // columns: 9.8 and 5.8 us, 10.7 with every column the whole wavefront's.
-// kItems: eight, which is eight million edges in the work-groups that are resident together,
-// or 32 beyond that (and on as few as four million, for fewer adds).
+// kItems: eight, which is 4.2 million edges in the work-groups that are resident together (four
+// a compute unit), or 32 beyond that.  Values that are gathered or divided on the way always go
+// by eight (the indexes of 32 would be 128 registers).
 constexpr int kRunItems = 8, kLongRunItems = 32;
 constexpr int64_t kLongRuns = int64_t(1) << 22;
 constexpr int kRunThreads = 512;
@@ -755,7 +798,18 @@ __global__ __launch_bounds__(kRunThreads) void normalise_sum_kernel(
 #pragma unroll
       for (int i = 0; i < kItems; ++i) run[i * kWave + lane] = v[i];
       wave_lds_fence();
-      columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
+      if (is_sparse(span, end - first))
+        edges_of_run(indptr, span, first, end, [&](int64_t c, int at, bool live) {
+          // (each column's edges in these 64 are neighbours: their sum at the first of them)
+          double mine = live ? (double)run[at] : 0.0;
+          for (int d = 1; d < kWave; d <<= 1) {
+            const double other = __shfl_down(mine, d, kWave);
+            if ((int64_t)__shfl_down((long long)c, d, kWave) == c && lane + d < kWave) mine += other;
+          }
+          const bool begins = (int64_t)__shfl_up((long long)c, 1, kWave) != c || lane == 0;
+          if (live && begins) unsafeAtomicAdd(sums + c, mine);
+        });
+      else columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
         constexpr int kTeam = decltype(team)::value;
         double mine = 0.0;
         for (int i = lane % kTeam; i < n; i += kTeam) mine += (double)run[begin + i];
@@ -803,7 +857,11 @@ __global__ __launch_bounds__(kRunThreads) void normalise_divide_kernel(
     for (int i = 0; i < kRunItems; ++i) by[i] = s;
   } else {
     float* const run = divisors[wave];
-    columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
+    if (is_sparse(span, end - first))
+      edges_of_run(indptr, span, first, end, [&](int64_t c, int at, bool live) {
+        if (live) run[at] = (float)sums[c];
+      });
+    else columns_of_run(indptr, span, first, end, [&](auto team, int64_t c, int begin, int n) {
       constexpr int kTeam = decltype(team)::value;
       const float s = n > 0 ? (float)sums[c] : 0.f;
       for (int i = lane % kTeam; i < n; i += kTeam) run[begin + i] = s;

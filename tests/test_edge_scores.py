@@ -450,3 +450,32 @@ def test_normalised_columns_against_64_bits(degrees, select, divide):
 def test_normalised_columns_of_long_runs(degrees):
     """More edges than the short runs take on: runs of one column, of a few, and of hundreds."""
     test_normalised_columns_against_64_bits(degrees, False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("degrees", [[1, 0, 0, 0] * 700, [0] * 999 + [300] + [0, 0, 3] * 100 + [700] + [0] * 5000 + [1],
+                                     [1] + [0] * 1023 + [511], [1] + [0] * 1022 + [511], [64, 0, 0] * 40 + [65] + [0] * 9000 + [1],
+                                     ([0] * 70_000 + [40]) * 30])
+def test_normalised_columns_of_which_most_are_empty(degrees):
+    """Runs around two columns an edge, columns longer than a row of 64 among them."""
+    for select in (False, True):
+        test_normalised_columns_against_64_bits(degrees, select, select)
+
+
+@pytest.mark.gpu
+def test_normalised_columns_of_few_edges_take_no_time_by_the_column():
+    """400 edges in two million columns: 0.05 ms, and 17 where a wavefront goes through the
+    columns between them."""
+    n = 2_000_000
+    indptr = torch.arange(n + 1, device=DEV) // 5000
+    graph = gs.Graph(500, n)
+    graph._CAPI_LoadCSC(indptr, torch.zeros(400, dtype=torch.int64, device=DEV))
+    values = torch.ones(400, device=DEV)
+    call = lambda: fused_op._normalised(graph, values, None, None, (gs._COO, gs._CSC, gs._COO))
+    assert torch.equal(call(), values)
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record()
+    call()
+    end.record()
+    end.synchronize()
+    assert start.elapsed_time(end) < 3.0
