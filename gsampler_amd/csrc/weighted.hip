@@ -1762,6 +1762,8 @@ int gs_csc_col_sample_weighted_fill_rows32(
     const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace, uint64_t seed,
     uint64_t call_id, const int64_t* sub_indptr, const int64_t* col_span, int64_t* out_coo_col,
     int32_t* out_rows, const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream) {
+  // (without row ids the kernels hand on positions of edges, which have no such bound)
+  GS_REQUIRE(indices, "sample_weighted_rows32: null indices");
   return gs::sample_weighted_by_cdf<int32_t>(indptr, num_cols, indices, cdf, column_ids, num_items,
                                              fanout, replace, seed, call_id, sub_indptr, col_span,
                                              out_coo_col, out_rows, nullptr, col_batch_ptr,

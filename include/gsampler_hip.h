@@ -307,7 +307,7 @@ int gs_csc_col_sample_weighted_fill(
     const int64_t* col_batch_ptr, int64_t num_col_batches, gs_stream_t stream);
 
 /* The CDF form with the row ids (all of them below 2^31) written 32 bits wide and no edge
- * positions, as gs_csc_col_sample_uniform_fill_rows32. */
+ * positions, as gs_csc_col_sample_uniform_fill_rows32; `indices` may not be NULL. */
 int gs_csc_col_sample_weighted_fill_rows32(
     const int64_t* indptr, int64_t num_cols, const int64_t* indices, const int64_t* cdf,
     const int64_t* column_ids, int64_t num_items, int64_t fanout, int replace, uint64_t seed,

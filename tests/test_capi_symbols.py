@@ -46,3 +46,8 @@ def test_argument_errors_are_reported_without_a_gpu():
     assert rc == 1 and b"Floyd" in l.gs_last_error()
     rc = l.gs_unique_count(None, None, 0, None, None, 0, 0, None, None, None, 0, None)
     assert rc == 1
+    # row ids of 32 bits need row ids: edge positions have no bound
+    for fill, args in ((l.gs_csc_col_sample_uniform_fill_rows32, (None, 0, None, None, None)),
+                       (l.gs_csc_col_sample_weighted_fill_rows32, (None, 0, None, None, None))):
+        rc = fill(*args, 0, 5, 0, 0, 0, None, None, None, None, None, 0, None)
+        assert rc == 1 and b"null indices" in l.gs_last_error()
