@@ -76,8 +76,10 @@ struct Compressed {
   // gains less tells how many ids it is about to read, and makes the copy once the reads
   // so told come to as many as the matrix has edges.
   torch::Tensor narrow_indices(int64_t reads = -1) const;
-  // The ids on the other axis are known to be below 2^31.
-  bool minor_ids_fit_32() const { return num_minor >= 0 && num_minor < (int64_t(1) << 31); }
+  // There are ids on the other axis, known to be below 2^31.
+  bool minor_ids_fit_32() const {
+    return indices.numel() > 0 && num_minor >= 0 && num_minor < (int64_t(1) << 31);
+  }
   // Where the column behind every edge lies (gs_hop_table), for walks over a
   // square matrix; made at the second walk over the same matrix.
   torch::Tensor hop_table() const;

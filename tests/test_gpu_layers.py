@@ -87,6 +87,20 @@ def test_one_batch(rng, nodes, count, fanouts, replace, weighted):
         same(x, y)
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("count", [7, 0])
+def test_large_layer_of_a_matrix_without_edges(count, weighted):
+    m = gs.Matrix(gs.Graph(50, 50))
+    m._graph._CAPI_LoadCSC(torch.zeros(51, dtype=torch.int64, device=DEV),
+                           torch.zeros(0, dtype=torch.int64, device=DEV))
+    if weighted:
+        m.edata["w"] = torch.zeros(0, device=DEV)
+    seeds = torch.arange(count, device=DEV) * 3
+    nodes, blocks = both(single, m, (seeds, [64], False), 1)[0]
+    assert torch.equal(nodes, seeds)
+    assert blocks[0].row.numel() == 0 and blocks[0].num_dst == count
+
+
 @pytest.mark.parametrize("cuts,fanouts,replace,weighted", [
     ([0, 64], [5], False, False),
     ([0, 0, 7, 7, 1000, 1001], [15, 10, 5], False, False),       # empty batches, one of one seed
