@@ -1036,3 +1036,47 @@ def test_labels_beside_the_offsets(R, edges):
         assert (got is None) == (edges < 8 * (R + 30))
         for a, b in zip(got[:3] if got else (), sub._CAPI_GraphRelabel(cols, rows)):
             assert torch.equal(a, b)
+
+
+def test_labels_of_the_longest_slices():
+    """More chunks of edges than have their offsets in one launch: labels, first edges and
+    offsets in launches of their own.  (Values and so their sums are exact.)"""
+    rng = np.random.default_rng(12)
+    indptr, indices = columns_of(rng.integers(50_000, 150_000, 20), rng, 30_000)
+    g = gs.Graph(30_000, 20)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+    cols = T(np.concatenate([rng.permutation(20) for _ in range(34_000_000 // indices.size + 1)]))
+    rows = T(rng.integers(0, 30_000, size=100))
+    by = torch.as_tensor((2.0 ** rng.integers(-2, 3, size=100)).astype(np.float32), device=DEV)
+    capi.profile_reset()
+    capi.profile_enable(True)
+    got = g._CAPI_RelabelledRows(cols, rows, w, by)
+    capi.profile_enable(False)
+    assert "member_first" in capi.profile_totals() and "list_labels" in capi.profile_totals()
+    sub, index = g._CAPI_ColRowSlicing(cols, rows, gs.format._CSC, gs.format._CSC | gs.format._COO)
+    for a, b in zip(got[:3], sub._CAPI_GraphRelabel(cols, rows)):
+        assert torch.equal(a, b)
+    assert torch.equal(got[3], sub._CAPI_NormaliseColumns(w, index, by))
+
+
+def test_labels_of_batches_of_the_longest_slices():
+    rng = np.random.default_rng(13)
+    indptr, indices = columns_of(rng.integers(10_000, 15_000, 2500), rng, 2500)
+    g = gs.Graph(2500, 2500)
+    g._CAPI_LoadCSC(T(indptr), T(indices))
+    w = torch.as_tensor(rng.integers(1, 9, size=indices.size).astype(np.float32), device=DEV)
+    seeds, ptr = batches_of(rng, 2500, [250] * 12)
+    rows, rows_ptr, _ = g._CAPI_EncodedSquareSums(seeds, ptr, w)
+    counts, starts = torch.diff(rows_ptr).tolist(), rows_ptr.tolist()
+    row_ids = T(np.concatenate([a + rng.choice(n, size=70, replace=False) for a, n in zip(starts, counts)]))
+    row_ptr = torch.arange(13, device=DEV) * 70
+    by = torch.as_tensor((2.0 ** rng.integers(-2, 3, size=row_ids.numel())).astype(np.float32), device=DEV)
+    capi.profile_reset()
+    capi.profile_enable(True)
+    got = g._CAPI_EncodedBlocks(seeds, ptr, rows, row_ids, row_ptr, w, by)
+    capi.profile_enable(False)
+    assert "member_first" in capi.profile_totals() and "list_labels" in capi.profile_totals()
+    sub, index, names = g._CAPI_EncodedPickedRows(seeds, ptr, rows, row_ids, row_ptr)
+    same_blocks(got[0], sub._CAPI_BatchBlocks(seeds, names))
+    assert torch.equal(got[1], sub._CAPI_NormaliseColumns(w, index, by))
