@@ -240,7 +240,7 @@ static bool values_in_passing(const Compressed& m, const c10::optional<torch::Te
 // What the kept edges of a row slice are handed on as.  Passes of compiled samplers, us, with
 // the slice written first and handed on, when that came: LADIES of 512 seeds 631, 571; of 8
 // batches of 128 seeds 693, 643; FastGCN of 1024 seeds 284, 228; subgraphs of 8.4 M edges between
-// 19 K nodes 240, 218.  (Now 487, 588, 183 and 203.)
+// 19 K nodes 240, 218.
 struct HandedOn {
   torch::Tensor row, col, values;
   // Behind the count pass; the arrays are sized by the slice's edges until trimmed.

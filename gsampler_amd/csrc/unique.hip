@@ -117,7 +117,10 @@ struct alignas(16) RankWord {
   uint32_t unused;
 };
 
-constexpr uint32_t kFirstMark = 0x80000000u;  // (positions are below 2^31 - 1)
+// The top bit of first[position] (positions are below 2^31 - 1), by the path of the call:
+constexpr uint32_t kFirstMark = 0x80000000u;   // few keys: the position is itself a first occurrence
+constexpr uint32_t kRepeatMark = 0x80000000u;  // partition: a repeat inside a tile, whose first
+                                               // occurrence is that of the position named
 
 struct UniqueWs {
   BatchInfo* batch;       // [B]
@@ -476,9 +479,10 @@ __device__ __forceinline__ uint32_t key_tag(uint64_t key) {
 // overflow list instead (the cursor still counts them, which is how the dedup
 // pass knows).  The tile is first ordered by bucket in LDS so that every run
 // leaves as one contiguous write instead of one line per entry.
-// 48 KB of LDS per work-group (the words of repeats lie where the tile is ordered later) lets three share a compute unit: with 512 threads
-// each they fill three quarters of its wavefront slots (256 threads: 11 % slower
-// on 21 M keys; 1024, two work-groups per unit: 45 % slower).
+// 48 KB of LDS per work-group (the words of repeats lie where the tile is ordered
+// later) lets three share a compute unit: with 512 threads each they fill three
+// quarters of its wavefront slots (256 threads: 11 % slower on 21 M keys; 1024, two
+// work-groups per unit: 45 % slower).
 constexpr int kScatterThreads = 512;
 constexpr int kScatterItems = kPartTile / kScatterThreads;
 constexpr int kTileBits = 12;
@@ -568,7 +572,7 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
     // writes those that are not (half as many scattered stores)
     if (l < t.end)
       first[t.b.fb + l] =
-          repeat ? ((uint32_t)t.begin + w % (uint32_t)kPartTile) | kFirstMark : (uint32_t)l;
+          repeat ? ((uint32_t)t.begin + w % (uint32_t)kPartTile) | kRepeatMark : (uint32_t)l;
   }
 #pragma unroll
   for (int i = 0; i < kScatterItems; ++i)
@@ -819,8 +823,9 @@ __device__ __forceinline__ void dedup_bucket(
       }
     return;
   }
-  // Many entries: fine for the LDS table while few of them are distinct (a hub
-  // that repeats thousands of times), so try, and count.  Entries are read
+  // Many entries: fine for the LDS table while few of them are distinct, so try, and
+  // count.  (A wide key may be here thousands of times, a narrow one about once for
+  // every partition tile of its batch.)  Entries are read
   // kDeep at a time per thread so that a long bucket streams at memory speed;
   // the overflow flag is read before every insert, which bounds the slots
   // claimed after it rises to one per thread.
@@ -1207,8 +1212,6 @@ constexpr int kFewBinKeys = 512;
 constexpr uint32_t kFewSlots = 2048;  // of a bin's table: four times the keys it gets on average
 constexpr uint32_t kFewClaims = kFewSlots * 3 / 4;
 constexpr uint32_t kFewListed = 2048;  // keys of a bin that are found again without a second look
-// first[position] of a call that went this way carries kFirstMark where the position is itself
-// a first occurrence.
 constexpr uint32_t kFewOpen = 0xFFFFFFFFu;  // no position, marked or not
 // Bin of a key: a hash of 32 bits, for every work-group hashes every key of its batch.  A
 // multiplication alone puts ids in steps of some sizes into one bin (by 2^32 over the golden
@@ -1637,15 +1640,15 @@ struct LabelArgs {
   int64_t* out_col;
   int remap;
   int col_prefilled;  // out_col holds every column's place inside its batch already
-  bool chase;         // a mark in first[] means that what it says has to be looked up in turn
+  bool chase;         // the mark in first[] is kRepeatMark, not kFirstMark
 };
 
-// What first[] says of a position, when it said f: a marked position is a repeat inside a
-// partition tile and takes what the one it names was told.
+// The first occurrence of a position of which first[] said f: behind kRepeatMark that of the
+// position named, behind kFirstMark (without `chase`) the position named.
 __device__ __forceinline__ uint32_t first_of(const uint32_t* __restrict__ first_b, uint32_t f,
                                              bool chase) {
-  if (!(f & kFirstMark)) return f;
-  f &= ~kFirstMark;
+  if (!(f & kRepeatMark)) return f;
+  f &= ~kRepeatMark;
   return chase ? first_b[f] : f;
 }
 
@@ -1677,9 +1680,9 @@ __device__ __forceinline__ void relabel_rows(const BatchInfo& b, const uint32_t*
     uint32_t told[kRelabelItems];
 #pragma unroll
     for (int i = 0; i < kRelabelItems; ++i)
-      told[i] = first_b[f[i] & kFirstMark ? f[i] & ~kFirstMark : 0u];
+      told[i] = first_b[f[i] & kRepeatMark ? f[i] & ~kRepeatMark : 0u];
 #pragma unroll
-    for (int i = 0; i < kRelabelItems; ++i) f[i] = f[i] & kFirstMark ? told[i] : f[i];
+    for (int i = 0; i < kRelabelItems; ++i) f[i] = f[i] & kRepeatMark ? told[i] : f[i];
   } else {
 #pragma unroll
     for (int i = 0; i < kRelabelItems; ++i) f[i] &= ~kFirstMark;

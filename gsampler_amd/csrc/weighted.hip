@@ -1846,8 +1846,10 @@ static int list_fill(const float* probs, const int64_t* range, int64_t n, int64_
   if (list_selects(n, num_segments, num_picks, replace)) {
     // few items per thread while that still fills the device, else sixteen (fewer
     // work-groups meet at the same histogram bins), eight where there are copies of those
-    // or sixteen would leave less than four work-groups a compute unit (eight segments of
-    // 233 K: bounds 25 us with sixteen and 16 with eight, emit 13 and 14)
+    // or sixteen would leave less than four work-groups a compute unit (256 picks of 1.05 M
+    // items, kernels of a call in us with sixteen and with eight: in 8 segments 54 and 47, in 64
+    // 64 and 57; of 2.45 M 57 and 50, 66 and 60; of 4.19 M 69 and 63, 75 and 71; with 1024 picks
+    // of 3.5 M in 8 segments, the worst of 64 to 1024 picks, 69 and 70)
     const int items = n < (int64_t(1) << 20) ? 4 : w.copies > 1 || n < (int64_t(1) << 22) ? 8 : 16;
     // bins half a power of two wide, an eighth where many picks make candidates dear
     // (they are compared with one another): 233 K items 24 and 27 us with 400 picks, 69
