@@ -282,20 +282,23 @@ def test_unique_relabel_of_few_keys(n, kind):
                     orc.unique_relabel(seeds, rows, sp, rp, col))
 
 
+@pytest.mark.parametrize("base", [0, 2**33])
 @pytest.mark.parametrize("B", [1, 3])
-def test_unique_relabel_buckets_beyond_their_regions(B):
+def test_unique_relabel_buckets_beyond_their_regions(B, base):
     """The partition pass gives every bucket a region of at most 8192 entries.  Ids
     that repeat 9000 to 150000 times in one batch run over it (several buckets of
-    one batch at once), next to a million ordinary keys; a last batch is all one id."""
+    one batch at once), next to a million ordinary keys; a last batch is all one id.
+    (Ids of 32 bits that repeat inside a tile are sent once; wider ones all are.)"""
     rng = np.random.default_rng(40 + B)
     n_r = 1_200_000
     rows = rng.integers(0, 10**6, size=n_r)
     for hub, times in [(3, 9000), (77777, 30000), (999_999, 150000), (5, 8193), (123, 8192)]:
         rows[rng.choice(n_r, size=times, replace=False)] = hub
-    seeds = rng.integers(0, 10**6, size=500 * B)
+    seeds = base + rng.integers(0, 10**6, size=500 * B)
+    rows += base
     sp = rp = None
     if B > 1:
-        rows = np.concatenate([rows, np.full(20000, 42), rng.integers(0, 300, size=100000)])
+        rows = np.concatenate([rows, np.full(20000, base + 42), base + rng.integers(0, 300, size=100000)])
         sp = np.arange(B + 1) * 500
         rp = np.array([0, n_r, n_r + 20000, rows.size])
         edge_col = np.concatenate([rng.integers(sp[b], sp[b + 1], size=rp[b + 1] - rp[b])
