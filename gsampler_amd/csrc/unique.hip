@@ -66,7 +66,7 @@ static_assert(kBucketCap >= kLdsMaxEntries, "the short dedup path reads a bucket
 
 // Keys per bucket (a fifth of them repeats that never get there) and whether work-groups
 // are laid out per die: the best of a sweep on 21M keys in 64 batches (dedup pass of
-// 1536 keys 83 us, 1792 78, 2048 78; before repeats stayed behind 512..3072, with and without
+// 1536 keys 70 us, 1792 68, 2048 68; before repeats stayed behind 512..3072, with and without
 // the per-die layout).
 struct UniqueTuning {
   int64_t bucket_keys;
@@ -533,8 +533,8 @@ __global__ __launch_bounds__(kScatterThreads) void unique_scatter_kernel(
   // One position of a key, its smallest, stands for all that the tile holds of it: the others
   // are told now, and marked, to take what that one will be told.  Ids of a power law repeat
   // within 4096 keys a fifth of the time (within a batch of 330 K half), and hubs always do:
-  // their buckets, thousands of repeats each, took the dedup pass 40 of 125 us on 21M keys and
-  // now 82, this pass 92 and now 86, the labels' further look-up 114 and now 120.
+  // their buckets, thousands of repeats each, took the dedup pass 40 of 122 us on 21M keys.
+  // It takes 68 now, and this pass, which stores as many entries less, 79 where it took 83.
   // A key has one word to meet in, told by the upper bits of a product that loses nothing of
   // it; of several keys the last to write has the word, more likely so the more often it is
   // there, and the others' repeats are sent as they are.  (A key of 2^32 - 1 or more stays out:
