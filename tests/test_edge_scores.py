@@ -473,9 +473,12 @@ def test_normalised_columns_of_few_edges_take_no_time_by_the_column():
     values = torch.ones(400, device=DEV)
     call = lambda: fused_op._normalised(graph, values, None, None, (gs._COO, gs._CSC, gs._COO))
     assert torch.equal(call(), values)
-    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-    start.record()
-    call()
-    end.record()
-    end.synchronize()
-    assert start.elapsed_time(end) < 3.0
+    took = []
+    for _ in range(5):  # (the host may pause inside one)
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        call()
+        end.record()
+        end.synchronize()
+        took.append(start.elapsed_time(end))
+    assert min(took) < 3.0
